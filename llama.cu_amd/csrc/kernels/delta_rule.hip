@@ -13,9 +13,15 @@
 //           of its lanes from the request's first token of the step to its last);
 //   out   (parallel): o of each head divided by its root mean square, times a weight, times
 //           sigmoid(gate).
-// A token's result depends on the tokens before it in its request only, in an order of
-// operations that does not depend on how the request was cut into steps.
+// A request that feeds DELTA_LONG tokens or more in a step goes through chunks on the matrix cores instead of the scan
+// (delta_chunks.h, heads of up to 128 key channels) if its outputs are rounded to bfloat16: the chunks' 32-bit results are 4e-7 of
+// their size off the recurrence in 64 bits, the scan's 1e-7 to 8e-7 (the smaller the faster a state decays; over 640 to 1,000 tokens).
+// A token's result depends on the tokens before it in its request only; portions below DELTA_LONG tokens are folded in in an
+// order of operations that does not depend on how the request was cut into them, longer ones change roundings.
+#include <limits.h>
 #include "common.h"
+#include "lane_moves.h"
+#include "delta_chunks.h"
 
 constexpr int MAX_RANK = 512;
 constexpr float DECAY_SCALE = 0.6065306597126334f;      // exp(-1/2)
@@ -25,34 +31,55 @@ __device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + expf
 // proj: [n, row_stride] rows that hold r, k, a_lin (dk per head each) and the low-rank
 // projection l (rank) at the given column offsets.  w2t: [rank, heads * dk], the decay's second matrix
 // transposed.  prep: [n, heads, 5, dk] 32-bit.
-template <class T>
-__global__ void delta_prep_kernel(const T *__restrict__ proj, int row_stride, int off_r, int off_k, int off_a, int off_l,
-                                  const float *__restrict__ w2t, const float *__restrict__ w0,
-                                  const float *__restrict__ a_bias, float *__restrict__ prep, int heads, int dk, int rank) {
-    __shared__ float th[MAX_RANK];
-    __shared__ float scratch[16];
-    const int t = blockIdx.x, h = blockIdx.y;
-    const T *row = proj + (size_t)t * row_stride;
-    for (int i = threadIdx.x; i < rank; i += blockDim.x) th[i] = tanhf(to_f32(row[off_l + i]));
-    float ss = 0.f;
-    for (int i = threadIdx.x; i < dk; i += blockDim.x) {
-        const float kk = to_f32(row[off_k + h * dk + i]);
-        ss += kk * kk;
+// A workgroup per (TB tokens, head, 64 key channels), a wave per quarter of the rank: a value of w2t serves TB tokens.  (A workgroup
+// per token and head read 4 dk rank bytes of w2t for it: 57 us for 2,048 tokens of 16 heads of 128 with a rank of 64.)  The
+// sum over the rank is made of the quarters' four, whatever TB is.
+template <class T, int TB>
+__global__ void __launch_bounds__(256)
+delta_prep_kernel(const T *__restrict__ proj, int row_stride, int off_r, int off_k, int off_a, int off_l,
+                  const float *__restrict__ w2t, const float *__restrict__ w0,
+                  const float *__restrict__ a_bias, float *__restrict__ prep, int n, int heads, int dk, int rank) {
+    __shared__ __attribute__((aligned(16))) float th[MAX_RANK * TB];
+    __shared__ float part[4][TB][WAVE], inv[TB];
+    const int t0 = blockIdx.x * TB, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nt = min(TB, n - t0), i = blockIdx.z * WAVE + lane, c = h * dk + min(i, dk - 1);
+    for (int x = threadIdx.x; x < rank * TB; x += 256) {
+        const int t = x / rank, j = x % rank;
+        th[j * TB + t] = t < nt ? tanhf(to_f32(proj[(size_t)(t0 + t) * row_stride + off_l + j])) : 0.f;
     }
-    ss = block_sum(ss, scratch);                 // (its barriers also make th visible)
-    const float inv = 1.0f / sqrtf(ss + 1e-6f);
-    float *out = prep + ((size_t)t * heads + h) * 5 * dk;
-    for (int i = threadIdx.x; i < dk; i += blockDim.x) {
-        const int c = h * dk + i;
-        float z = w0[c];
+    for (int t = wave; t < nt; t += 4) {
+        const T *row = proj + (size_t)(t0 + t) * row_stride + off_k + h * dk;
+        float ss = 0.f;
+        for (int x = lane; x < dk; x += WAVE) {
+            const float kk = to_f32(row[x]);
+            ss += kk * kk;
+        }
+        ss = wave_sum_in_place(ss);
+        if (lane == 0) inv[t] = 1.0f / sqrtf(ss + 1e-6f);
+    }
+    __syncthreads();
+    const int quarter = (rank + 3) / 4, j0 = wave * quarter, j1 = min(rank, j0 + quarter);
+    float z[TB];
+#pragma unroll
+    for (int t = 0; t < TB; ++t) z[t] = 0.f;
+    const float *w = w2t + c;                                 // (neighbouring lanes, neighbouring addresses)
 #pragma unroll 8
-        for (int j = 0; j < rank; ++j) z += w2t[(size_t)j * heads * dk + c] * th[j];      // (neighbouring lanes, neighbouring addresses)
-        const float w = expf(-DECAY_SCALE * sigmoidf_(z));
-        const float a = sigmoidf_(to_f32(row[off_a + c]) + a_bias[c]);
-        const float kk = to_f32(row[off_k + c]);
-        const float u = kk * inv;
-        out[i] = w;
-        out[dk + i] = a * u;
+    for (int j = j0; j < j1; ++j) {
+        const float v = w[(size_t)j * heads * dk];
+#pragma unroll
+        for (int t = 0; t < TB; ++t) z[t] += v * th[j * TB + t];
+    }
+#pragma unroll
+    for (int t = 0; t < TB; ++t) part[wave][t][lane] = z[t];
+    __syncthreads();
+    if (i >= dk) return;
+    for (int t = wave; t < nt; t += 4) {
+        const T *row = proj + (size_t)(t0 + t) * row_stride;
+        const float sum = (part[0][t][lane] + part[1][t][lane]) + (part[2][t][lane] + part[3][t][lane]);
+        const float kk = to_f32(row[off_k + c]), u = kk * inv[t];
+        float *out = prep + ((size_t)(t0 + t) * heads + h) * 5 * dk;
+        out[i] = expf(-DECAY_SCALE * sigmoidf_(w0[c] + sum));
+        out[dk + i] = sigmoidf_(to_f32(row[off_a + c]) + a_bias[c]) * u;
         out[2 * dk + i] = u;
         out[3 * dk + i] = kk;
         out[4 * dk + i] = to_f32(row[off_r + c]);
@@ -87,14 +114,15 @@ constexpr int scan_groups() { return DK > 0 && DK % 32 == 0 ? 8 : 4; }
 
 // GATED: the gated rule, whose decay g and rate beta are one number each per token and head and whose key is its unit
 // key: S <- g S + u (v - (beta g) (u^T S)) with v the value times beta already.  A token then brings two vectors (u, r) and
-// two numbers (g, beta g) instead of five vectors: prep rows are [u | r | g, beta g, 0, 0], 2 dk + 4 floats.
+// two numbers (g, beta g) instead of five vectors: prep rows are [u | r | g, beta g, log g, 0], 2 dk + 4 floats.
 template <class T, int DK, bool GATED>
 __global__ void __launch_bounds__(64)
 delta_scan_kernel(const T *__restrict__ proj, int row_stride, int off_v, const float *__restrict__ vf, const float *__restrict__ prep,
                   float *__restrict__ state, size_t slot_stride, float *__restrict__ o, const int *__restrict__ q_start,
-                  const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int heads, int dk_rt, int dv) {
+                  const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int heads, int dk_rt, int dv, int below) {
     const int r = blockIdx.x, h = blockIdx.y;
     const int t0 = q_start[r], t1 = q_start[r + 1];
+    if (t1 - t0 >= below) return;                             // a request for the chunks
     const bool fresh = ctx_len[r] - (t1 - t0) == 0;          // the request's first token: the state starts at zero
     if constexpr (DK > 0) {
         constexpr int SCAN_GROUPS = scan_groups<T, DK>(), SCAN_COLS = WAVE / SCAN_GROUPS;
@@ -232,12 +260,25 @@ delta_out_kernel(const float *__restrict__ o, const T *__restrict__ proj, int ro
     }
 }
 
-// The scan over the step's tokens for every head size it is compiled for.  vf: null, or the values as 32-bit rows.
+// The recurrence over the step's tokens: the scan for every head size it is compiled for, and the chunks where a request may feed
+// enough tokens (`work`: delta_chunk_floats floats; null: everything is scanned).  vf: null, or the values as 32-bit rows.
 template <class T, bool GATED = false>
-static int delta_scan_launch(const T *proj, int row_stride, int off_v, const float *vf, const float *prep, float *state,
+static int delta_scan_launch(const T *proj, int row_stride, int off_v, const float *vf, const float *prep, float *work, float *state,
                              size_t slot_stride, float *o, const int *q_start, const int *ctx_len, const int *state_slot,
-                             int n_req, int heads, int dk, int dv, hipStream_t stream) {
-#define SCAN(DK) delta_scan_kernel<T, DK, GATED><<<dim3(n_req, heads, (dv + (DK ? 64 / scan_groups<T, DK>() : 64) - 1) / (DK ? 64 / scan_groups<T, DK>() : 64)), dim3(64), 0, stream>>>(proj, row_stride, off_v, vf, prep, state, slot_stride, o, q_start, ctx_len, state_slot, heads, dk, dv)
+                             int n, int n_req, int heads, int dk, int dv, hipStream_t stream) {
+    int below = INT_MAX;
+    if (work && delta_chunks_possible(n, n_req, dk)) {
+        DeltaChunkArgs c = {};
+        c.prep = prep; c.proj = proj; c.row_stride = row_stride; c.off_v = off_v; c.vf = vf;
+        c.state = state; c.slot_stride = slot_stride; c.o = o;
+        c.q_start = q_start; c.ctx_len = ctx_len; c.state_slot = state_slot;
+        c.n_req = n_req; c.heads = heads; c.dk = dk; c.dv = dv;
+        const int rc = delta_chunks_launch<T, GATED>(c, work, n, stream);
+        if (rc != LCU_OK) return rc;
+        if (n_req == 1) return LCU_OK;                        // (its one request is long: n >= DELTA_LONG)
+        below = DELTA_LONG;
+    }
+#define SCAN(DK) delta_scan_kernel<T, DK, GATED><<<dim3(n_req, heads, (dv + (DK ? 64 / scan_groups<T, DK>() : 64) - 1) / (DK ? 64 / scan_groups<T, DK>() : 64)), dim3(64), 0, stream>>>(proj, row_stride, off_v, vf, prep, state, slot_stride, o, q_start, ctx_len, state_slot, heads, dk, dv, below)
     switch (dk) {
     case 16: SCAN(16); break;
     case 32: SCAN(32); break;
@@ -258,15 +299,17 @@ static int delta_scan_launch(const T *proj, int row_stride, int off_v, const flo
 
 template <class T>
 static int delta_rule_t(const T *proj, int row_stride, int off_r, int off_k, int off_v, int off_g, int off_a, int off_l,
-                        const float *w2, const float *w0, const float *a_bias, const float *weight, float *prep,
+                        const float *w2, const float *w0, const float *a_bias, const float *weight, float *prep, float *work,
                         float *o, float *state, T *out, const int *q_start, const int *ctx_len, const int *state_slot,
                         int n, int n_req, int heads, int dk, int dv, int rank, float eps, hipStream_t stream) {
-    int threads = ((dk > rank ? dk : rank) + 63) / 64 * 64;
-    if (threads > 256) threads = 256;
-    delta_prep_kernel<T><<<dim3(n, heads), dim3(threads), 0, stream>>>(proj, row_stride, off_r, off_k, off_a, off_l, w2, w0, a_bias, prep, heads, dk, rank);
+    // eight tokens a workgroup where that still gives every compute unit some
+#define PREP(TB) delta_prep_kernel<T, TB><<<dim3((n + TB - 1) / TB, heads, (dk + WAVE - 1) / WAVE), dim3(256), 0, stream>>>(proj, row_stride, off_r, off_k, off_a, off_l, w2, w0, a_bias, prep, n, heads, dk, rank)
+    if ((long long)n * heads >= 8 * 512) PREP(8);
+    else PREP(1);
+#undef PREP
     LCU_LAUNCH_CHECK();
-    const int rc = delta_scan_launch<T>(proj, row_stride, off_v, nullptr, prep, state, (size_t)heads * dk * dv, o, q_start, ctx_len,
-                                        state_slot, n_req, heads, dk, dv, stream);
+    const int rc = delta_scan_launch<T>(proj, row_stride, off_v, nullptr, prep, work, state, (size_t)heads * dk * dv, o, q_start, ctx_len,
+                                        state_slot, n, n_req, heads, dk, dv, stream);
     if (rc != LCU_OK) return rc;
     delta_out_kernel<T><<<dim3(n, heads), dim3(64), 0, stream>>>(o, proj, row_stride, off_g, weight, out, heads, dv, eps);
     LCU_LAUNCH_CHECK();
@@ -274,19 +317,24 @@ static int delta_rule_t(const T *proj, int row_stride, int off_r, int off_k, int
 }
 
 // proj: [n, row_stride] of `type`; the offsets are columns.  w2: [rank, heads * dk] (transposed), w0, a_bias: [heads * dk],
-// weight: [heads * dv], all 32-bit.  prep: scratch [n, heads, 5, dk], o: scratch [n, heads * dv], both 32-bit.
+// weight: [heads * dv], all 32-bit.  prep: scratch [n, heads, 5, dk], o: scratch [n, heads * dv], work: scratch of
+// lcu_delta_work_floats floats (null: every request is scanned token by token), all 32-bit.
 // state: [slots, heads, dk, dv] 32-bit.  out: [n, heads * dv] of `type`.
+LCU_API long long lcu_delta_work_floats(int n, int n_req, int heads, int dk, int dv) {
+    return n > 0 && n_req > 0 && heads > 0 && dk > 0 && dv > 0 ? (long long)delta_chunk_floats(n, n_req, heads, dk, dv) : 0;
+}
+
 LCU_API int lcu_delta_rule(const void *proj, int type, int row_stride, int off_r, int off_k, int off_v, int off_g,
                            int off_a, int off_l, const float *w2, const float *w0, const float *a_bias,
-                           const float *weight, float *prep, float *o, float *state, void *out, const int *q_start,
+                           const float *weight, float *prep, float *work, float *o, float *state, void *out, const int *q_start,
                            const int *ctx_len, const int *state_slot, int n, int n_req, int heads, int dk, int dv,
                            int rank, float eps, hipStream_t stream) {
     if (n <= 0 || n_req <= 0) return LCU_OK;
     if (heads <= 0 || heads > 65535 || dk <= 0 || dv <= 0 || rank <= 0 || rank > MAX_RANK || dv > 8 * 65535) return LCU_BAD_ARGUMENT;
     if (type == LCU_F32)
-        return delta_rule_t<float>((const float *)proj, row_stride, off_r, off_k, off_v, off_g, off_a, off_l, w2, w0, a_bias, weight, prep, o, state, (float *)out, q_start, ctx_len, state_slot, n, n_req, heads, dk, dv, rank, eps, stream);
+        return delta_rule_t<float>((const float *)proj, row_stride, off_r, off_k, off_v, off_g, off_a, off_l, w2, w0, a_bias, weight, prep, work, o, state, (float *)out, q_start, ctx_len, state_slot, n, n_req, heads, dk, dv, rank, eps, stream);
     if (type == LCU_BF16)
-        return delta_rule_t<bf16_t>((const bf16_t *)proj, row_stride, off_r, off_k, off_v, off_g, off_a, off_l, w2, w0, a_bias, weight, prep, o, state, (bf16_t *)out, q_start, ctx_len, state_slot, n, n_req, heads, dk, dv, rank, eps, stream);
+        return delta_rule_t<bf16_t>((const bf16_t *)proj, row_stride, off_r, off_k, off_v, off_g, off_a, off_l, w2, w0, a_bias, weight, prep, work, o, state, (bf16_t *)out, q_start, ctx_len, state_slot, n, n_req, heads, dk, dv, rank, eps, stream);
     return LCU_BAD_ARGUMENT;
 }
 
@@ -303,32 +351,35 @@ LCU_API int lcu_delta_rule(const void *proj, int type, int row_stride, int off_r
 // off_a and off_b, and the gate's heads * dv columns at off_g.
 __device__ __forceinline__ float softplus_(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 
-__global__ void gated_delta_prep_kernel(const float *__restrict__ qkv, const float *__restrict__ rows, int row_stride, int off_a,
-                                        int off_b, const float *__restrict__ a_log, const float *__restrict__ dt_bias,
-                                        float *__restrict__ prep, float *__restrict__ vb, int heads, int group, int dk, int dv) {
-    __shared__ float scratch[16];
-    const int t = blockIdx.x, h = blockIdx.y, qh = h / group, qk_heads = heads / group;
+// One wave per (token, value head), four a workgroup.
+__global__ void __launch_bounds__(256)
+gated_delta_prep_kernel(const float *__restrict__ qkv, const float *__restrict__ rows, int row_stride, int off_a,
+                        int off_b, const float *__restrict__ a_log, const float *__restrict__ dt_bias,
+                        float *__restrict__ prep, float *__restrict__ vb, int n, int heads, int group, int dk, int dv) {
+    const int item = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (item >= n * heads) return;
+    const int t = item / heads, h = item % heads, qh = h / group, qk_heads = heads / group;
     const int width = 2 * qk_heads * dk + heads * dv;
     const float *q = qkv + (size_t)t * width + qh * dk, *k = q + qk_heads * dk;
     const float *v = qkv + (size_t)t * width + 2 * qk_heads * dk + h * dv;
+    const float *row = rows + (size_t)t * row_stride;
+    const float beta = sigmoidf_(row[off_b + h]);
+    const float lg = -expf(a_log[h]) * softplus_(row[off_a + h] + dt_bias[h]), g = expf(lg);
     float sq = 0.f, sk = 0.f;
-    for (int i = threadIdx.x; i < dk; i += blockDim.x) {
+    for (int i = lane; i < dk; i += 64) {
         sq += q[i] * q[i];
         sk += k[i] * k[i];
     }
-    sq = block_sum(sq, scratch);
-    sk = block_sum(sk, scratch);
+    sq = wave_sum_in_place(sq);
+    sk = wave_sum_in_place(sk);
     const float qf = 1.0f / sqrtf(sq + 1e-6f) / sqrtf((float)dk), kf = 1.0f / sqrtf(sk + 1e-6f);
-    const float *row = rows + (size_t)t * row_stride;
-    const float beta = sigmoidf_(row[off_b + h]);
-    const float g = expf(-expf(a_log[h]) * softplus_(row[off_a + h] + dt_bias[h]));
-    float *out = prep + ((size_t)t * heads + h) * (2 * dk + 4);
-    for (int i = threadIdx.x; i < dk; i += blockDim.x) {
+    float *out = prep + (size_t)item * (2 * dk + 4);
+    for (int i = lane; i < dk; i += 64) {
         out[i] = k[i] * kf;
         out[dk + i] = q[i] * qf;
     }
-    if (threadIdx.x < 4) out[2 * dk + threadIdx.x] = threadIdx.x == 0 ? g : (threadIdx.x == 1 ? beta * g : 0.f);
-    for (int j = threadIdx.x; j < dv; j += blockDim.x) vb[((size_t)t * heads + h) * dv + j] = beta * v[j];
+    if (lane < 4) out[2 * dk + lane] = lane == 0 ? g : lane == 1 ? beta * g : lane == 2 ? lg : 0.f;
+    for (int j = lane; j < dv; j += 64) vb[(size_t)item * dv + j] = beta * v[j];
 }
 
 // One wave per (token, head): out = o / rms(o) * weight * silu(gate); weight: [dv], shared by the heads.
@@ -347,10 +398,10 @@ gated_delta_out_kernel(const float *__restrict__ o, const float *__restrict__ ro
     }
 }
 
-// a_log, dt_bias: [heads]; weight: [dv], 32-bit.  prep: scratch [n, heads, 2 * dk + 4]; vb, o: scratch [n, heads * dv], 32-bit.
+// a_log, dt_bias: [heads]; weight: [dv], 32-bit.  prep: scratch [n, heads, 2 * dk + 4]; vb, o: scratch [n, heads * dv], work: as above, 32-bit.
 // state: slot s at state + s * slot_stride, [heads, dk, dv] 32-bit.  out: [n, heads * dv] of out_type.
 LCU_API int lcu_gated_delta_rule(const float *qkv, const float *rows, int row_stride, int off_a, int off_b, int off_g,
-                                 const float *a_log, const float *dt_bias, const float *weight, float *prep, float *vb, float *o,
+                                 const float *a_log, const float *dt_bias, const float *weight, float *prep, float *vb, float *work, float *o,
                                  float *state, long long slot_stride, void *out, int out_type, const int *q_start,
                                  const int *ctx_len, const int *state_slot, int n, int n_req, int heads, int qk_heads, int dk,
                                  int dv, float eps, hipStream_t stream) {
@@ -358,12 +409,11 @@ LCU_API int lcu_gated_delta_rule(const float *qkv, const float *rows, int row_st
     if (heads <= 0 || heads > 65535 || qk_heads <= 0 || heads % qk_heads || dk <= 0 || dv <= 0 || dv > 8 * 65535 ||
         (out_type != LCU_F32 && out_type != LCU_BF16))
         return LCU_BAD_ARGUMENT;
-    int threads = ((dk > dv ? dk : dv) + 63) / 64 * 64;
-    if (threads > 256) threads = 256;
-    gated_delta_prep_kernel<<<dim3(n, heads), dim3(threads), 0, stream>>>(qkv, rows, row_stride, off_a, off_b, a_log, dt_bias, prep, vb,
-                                                                           heads, heads / qk_heads, dk, dv);
+    if ((long long)n * heads > INT_MAX - 4) return LCU_BAD_ARGUMENT;
+    gated_delta_prep_kernel<<<dim3((n * heads + 3) / 4), dim3(256), 0, stream>>>(qkv, rows, row_stride, off_a, off_b, a_log, dt_bias, prep, vb,
+                                                                                n, heads, heads / qk_heads, dk, dv);
     LCU_LAUNCH_CHECK();
-    const int rc = delta_scan_launch<float, true>(nullptr, 0, 0, vb, prep, state, (size_t)slot_stride, o, q_start, ctx_len, state_slot, n_req,
+    const int rc = delta_scan_launch<float, true>(nullptr, 0, 0, vb, prep, work, state, (size_t)slot_stride, o, q_start, ctx_len, state_slot, n, n_req,
                                             heads, dk, dv, stream);
     if (rc != LCU_OK) return rc;
     if (out_type == LCU_F32)

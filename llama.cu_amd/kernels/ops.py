@@ -1278,6 +1278,17 @@ def qk_norm_store(qkv: torch.Tensor, positions: torch.Tensor, n_heads: int, n_kv
 # ------------------------------------------------------------------ the generalised delta rule
 
 
+def _delta_work(lib, n: int, n_req: int, heads: int, key_dim: int, value_dim: int, out: torch.Tensor) -> Optional[torch.Tensor]:
+    """Scratch memory for the delta rules' chunks.  None: everything is scanned token by token, because the step holds no
+    request that feeds enough tokens for chunks, or because the outputs are 32-bit (a chunk's are 4e-7 of their size off the
+    exact ones, where the scan's may be only 1e-7 off; rounded to bfloat16 both are the same)."""
+    if out.dtype == torch.float32:
+        return None
+    lib.lcu_delta_work_floats.restype = ctypes.c_longlong
+    floats = lib.lcu_delta_work_floats(n, n_req, heads, key_dim, value_dim)
+    return torch.empty(floats, dtype=torch.float32, device=out.device) if floats else None
+
+
 def delta_rule(proj: torch.Tensor, offsets: Dict[str, int], w2_t: torch.Tensor, w0: torch.Tensor, a_bias: torch.Tensor,
                weight: torch.Tensor, state: torch.Tensor, step, heads: int, key_dim: int, value_dim: int, eps: float,
                out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -1313,9 +1324,10 @@ def delta_rule(proj: torch.Tensor, offsets: Dict[str, int], w2_t: torch.Tensor, 
     prep = torch.empty((n, heads, 5, key_dim), dtype=torch.float32, device=proj.device)
     o = torch.empty((n, hv), dtype=torch.float32, device=proj.device)
     lib = build.load("delta_rule")
+    work = _delta_work(lib, n, step.n_req, heads, key_dim, value_dim, out)
     _check(lib.lcu_delta_rule(_ptr(proj), _type(proj, "delta projections"), proj.stride(0), offsets["r"], offsets["k"], offsets["v"],
                               offsets["g"], offsets["a"], offsets["l"], _ptr(w2_t), _ptr(w0), _ptr(a_bias), _ptr(weight), _ptr(prep),
-                              _ptr(o), _ptr(state), _ptr(out), _ptr(step.q_start), _ptr(step.ctx_len), _ptr(step.state_slot), n,
+                              _ptr(work), _ptr(o), _ptr(state), _ptr(out), _ptr(step.q_start), _ptr(step.ctx_len), _ptr(step.state_slot), n,
                               step.n_req, heads, key_dim, value_dim, rank, ctypes.c_float(eps), _stream()), "delta_rule")
     return out
 
@@ -2007,13 +2019,14 @@ def gated_delta_rule(qkv: torch.Tensor, rows: torch.Tensor, off_a: int, off_b: i
     if n != step.n:
         raise KernelError("gated_delta_rule: the rows are not the step's")
     slot_stride = _slot_state(state, (heads, key_dim, value_dim), "gated_delta_rule", step)
-    prep = torch.empty((n, heads, 2 * key_dim + 4), dtype=torch.float32, device=qkv.device)     # per token and head: unit key, query, g, beta g
+    prep = torch.empty((n, heads, 2 * key_dim + 4), dtype=torch.float32, device=qkv.device)     # per token and head: unit key, query, g, beta g, log g
     vb = torch.empty((n, hv), dtype=torch.float32, device=qkv.device)
     o = torch.empty((n, hv), dtype=torch.float32, device=qkv.device)
     out = torch.empty((n, hv), dtype=out_dtype, device=qkv.device)
     lib = build.load("delta_rule")
+    work = _delta_work(lib, n, step.n_req, heads, key_dim, value_dim, out)
     _check(lib.lcu_gated_delta_rule(_ptr(qkv), _ptr(rows), rows.stride(0), int(off_a), int(off_b), int(off_g), _ptr(a_log), _ptr(dt_bias),
-                                    _ptr(weight), _ptr(prep), _ptr(vb), _ptr(o), _ptr(state), ctypes.c_longlong(slot_stride), _ptr(out),
+                                    _ptr(weight), _ptr(prep), _ptr(vb), _ptr(work), _ptr(o), _ptr(state), ctypes.c_longlong(slot_stride), _ptr(out),
                                     _type(out, "gated delta out"), _ptr(step.q_start), _ptr(step.ctx_len), _ptr(step.state_slot), n,
                                     step.n_req, heads, qk_heads, key_dim, value_dim, ctypes.c_float(eps), _stream()), "gated_delta_rule")
     return out

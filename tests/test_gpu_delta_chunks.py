@@ -1,0 +1,110 @@
+"""The delta rules' chunks (csrc/kernels/delta_chunks.h) against the recurrences in 64 bits, beside the token-by-token scan:
+at the chunks' edges, from states of earlier portions, and where decays are as small as they can be."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from divasun_common import assert_close
+from test_gpu_divasun import hand_step, rnd
+
+pytestmark = pytest.mark.gpu
+F64 = torch.float64
+EPS = 1e-5
+
+
+def unit_rms(x):
+    return x / torch.sqrt((x * x).mean(-1, keepdim=True) + EPS)
+
+
+def walk(w, al, u, k, v, r):
+    """o [T, heads, dv] and the last state of S <- diag(w) S - al (u^T S) + k v^T from zeros; all [T, heads, .]."""
+    S = torch.zeros(w.shape[1], w.shape[2], v.shape[2], dtype=F64)
+    outs = []
+    for t in range(w.shape[0]):
+        seen = u[t][:, None, :] @ S
+        S = w[t][:, :, None] * S - al[t][:, :, None] * seen + k[t][:, :, None] * v[t][:, None, :]
+        outs.append((r[t][:, None, :] @ S)[:, 0])
+    return torch.stack(outs), S
+
+
+def general(T, heads, dim, rank, decay, seed):
+    """(arguments of ops.delta_rule, a row maker, the expected outputs and state); ``decay``: added to w0."""
+    hd = heads * dim
+    off = {"r": 0, "k": hd, "v": 2 * hd, "g": 3 * hd, "a": 4 * hd, "l": 5 * hd}
+    proj = rnd(T, 5 * hd + rank, seed=seed).bfloat16()
+    w2, w0, ab, nw = rnd(hd, rank, seed=3), rnd(hd, seed=4) + decay, rnd(hd, seed=5), rnd(hd, seed=6) * 0.1 + 1
+    x = proj.to(F64)
+    r, k, v, g, a = (x[:, off[c]:off[c] + hd].view(T, heads, dim) for c in "rkvga")
+    w = torch.exp(-math.exp(-0.5) * torch.sigmoid(torch.tanh(x[:, 5 * hd:]) @ w2.to(F64).T + w0.to(F64))).view(T, heads, dim)
+    u = k / torch.sqrt((k * k).sum(-1, keepdim=True) + 1e-6)
+    o, S = walk(w, torch.sigmoid(a + ab.to(F64).view(heads, dim)) * u, u, k, v, r)
+    want = unit_rms(o).reshape(T, hd) * nw.to(F64) * torch.sigmoid(g.reshape(T, hd))
+    return (off, w2.t().contiguous().cuda(), w0.cuda(), ab.cuda(), nw.cuda()), proj, want, S
+
+
+def run_general(args, proj, heads, dim, portions):
+    """Outputs and last state of the rows in portions, from a slot that holds other values; a short request walks beside."""
+    from llama_cu_amd.kernels import ops
+    state = torch.full((3, heads, dim, dim), 7.0, device="cuda")
+    outs, at = [], 0
+    for n in portions:
+        rows = torch.cat([proj[:2], proj[at:at + n]]).cuda()
+        outs.append(ops.delta_rule(rows, *args, state, hand_step([2, n], [2, at + n], [0, 2]), heads, dim, dim, EPS)[2:].clone())
+        at += n
+    assert (state[1] == 7.0).all()
+    return torch.cat(outs), state[2]
+
+
+@pytest.mark.parametrize("heads,dim,portions,decay", [
+    (2, 128, [64], 0.0), (1, 128, [65, 63, 64], 0.0), (2, 128, [129], 9.0), (2, 64, [127, 1, 66], -3.0),
+    (3, 20, [200, 129], 0.0), (1, 72, [128, 128], 9.0), (2, 16, [191], -9.0), (1, 112, [100, 70], 0.0)])
+def test_the_generalised_rule_in_chunks(heads, dim, portions, decay):
+    """``decay`` 9: every decay is as small as the rule allows (0.545 a token); -9: close to 1."""
+    args, proj, want, S = general(sum(portions), heads, dim, 3, decay, seed=11)
+    got, state = run_general(args, proj, heads, dim, portions)
+    # the state: sums of some hundred 32-bit products of either sign, 2e-7 to 17e-7 of the largest value off as measured (the
+    # scan's 2e-7 to 18e-7); the outputs are rounded to 8 bits: half a unit of the last is up to 2^-8 of the value, and what
+    # the 32-bit value is off adds to it
+    assert_close(state, S, 5e-6, "state")
+    assert_close(got, want, 2.0 ** -8 + 1e-5, "outputs")
+
+
+def gated(T, heads, qk_heads, dk, dv, gate, seed):
+    width, hv = 2 * qk_heads * dk + heads * dv, heads * dv
+    qkv = rnd(T, width, seed=seed)
+    rows = rnd(T, 2 * heads + hv, seed=seed + 1)                        # a, b, gate
+    a_log, bias, weight = rnd(heads, seed=7), rnd(heads, seed=8) + gate, rnd(dv, seed=9) * 0.1 + 1
+    x, y = qkv.to(F64), rows.to(F64)
+    rep = heads // qk_heads
+    q, k = (x[:, i * qk_heads * dk:(i + 1) * qk_heads * dk].view(T, qk_heads, dk) for i in (0, 1))
+    q, k = ((z / torch.sqrt((z * z).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(rep, 1) for z in (q, k))
+    v = x[:, 2 * qk_heads * dk:].view(T, heads, dv)
+    g = torch.exp(-torch.exp(a_log.to(F64)) * torch.nn.functional.softplus(y[:, :heads] + bias.to(F64)))[..., None]
+    beta = torch.sigmoid(y[:, heads:2 * heads])[..., None]
+    o, S = walk(g.expand(T, heads, dk), beta * g * k, k, k, beta * v, q * dk ** -0.5)
+    z = y[:, 2 * heads:].view(T, heads, dv)
+    want = (unit_rms(o) * weight.to(F64) * (z * torch.sigmoid(z))).reshape(T, hv)
+    return (a_log.cuda(), bias.cuda(), weight.cuda()), qkv, rows, want, S
+
+
+@pytest.mark.parametrize("heads,qk_heads,dk,dv,portions,gate", [
+    (2, 1, 128, 128, [64], 0.0), (2, 2, 128, 128, [65, 63, 130], -4.0), (4, 2, 64, 20, [127, 1, 66], 0.0), (1, 1, 24, 40, [200], 80.0),
+    (3, 1, 72, 136, [128, 65], 3.0), (2, 2, 16, 16, [191], -9.0), (1, 1, 128, 272, [100], 0.0)])
+def test_the_gated_rule_in_chunks(heads, qk_heads, dk, dv, portions, gate):
+    """``gate`` 80: a token's decay is 0 in 32 bits; -9: it is 1 but for the fourth digit."""
+    from llama_cu_amd.kernels import ops
+    T = sum(portions)
+    args, qkv, rows, want, S = gated(T, heads, qk_heads, dk, dv, gate, seed=21)
+    state = torch.full((3, heads, dk, dv), 7.0, device="cuda")
+    outs, at = [], 0
+    for n in portions:
+        pick = torch.cat([torch.arange(at, at + n), torch.arange(3)])
+        outs.append(ops.gated_delta_rule(qkv[pick].cuda(), rows[pick].cuda(), 0, heads, 2 * heads, *args, state,
+                                         hand_step([n, 3], [at + n, 3], [1, 2]), heads, qk_heads, dk, dv, EPS, torch.bfloat16)[:n].clone())
+        at += n
+    assert (state[0] == 7.0).all()
+    assert_close(state[1], S, 5e-6, "state")
+    assert_close(torch.cat(outs), want, 2.0 ** -8 + 1e-5, "outputs")
