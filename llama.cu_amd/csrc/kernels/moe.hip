@@ -6,8 +6,9 @@
 //            over all experts, the choice by s + a correction per expert, and the chosen scores divided by their sum (or as
 //            they are) times a factor as weights; the choice may be limited to the experts of the best groups; rows of the router's matrix behind the experts' are gates: sigmoid of their logit goes out per
 //            token; the last experts may be identity experts, which have no matrices and return their input;
-//   group:   the (token, choice) pairs sorted by expert and cut into tiles of up to 16 or 64 rows of
-//            one expert, on the device (nothing comes back to the host);
+//   group:   the (token, choice) pairs sorted by expert and cut into tiles of up to 64 rows of one expert, on the
+//            device (nothing comes back to the host); where experts have few pairs a product's workgroups look for theirs
+//            themselves instead;
 //   up:      act = gelu(W_up[e] (weight * h))    the weight scales what goes INTO the expert; or, gated:
 //            act = silu(W_gate[e] h) * (W_up[e] h) (or the limited form, gate_act.h), and the weight scales what comes OUT of the expert
 //   down:    y = W_down[e] act, added to the token's output row (32-bit), in the gated form times the weight
@@ -20,7 +21,7 @@
 #include "gate_act.h"
 
 constexpr int MOE_MAX_EXPERTS = 1024;
-constexpr int MOE_TILE_ROWS = 64;        // rows of a tile of the kernel for many rows; the kernel for few rows takes 16
+constexpr int MOE_TILE_ROWS = 64;        // rows of a tile of the kernel for many rows
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
@@ -234,19 +235,21 @@ template <> struct Mma<float> {
 
 __device__ __forceinline__ float gelu_erf(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 
+template <class T> struct alignas(4 * sizeof(T)) Quad { T v[4]; };
+
 enum { MOE_UP = 0, MOE_DOWN = 1, MOE_UP_GATED = 2 };
 
-// Both kernels below multiply the rows of a tile (sorted rows of one expert) with that expert's matrix
-// w[e] ([N, K], row-major) on the matrix cores.  The weight is the instruction's first operand (16
+// Both kernels below multiply rows of one expert with that expert's matrix w[e] ([N, K], as it is or PACKED, see Unit) on the
+// matrix cores.  The weight is the instruction's first operand (16
 // features x k), the rows the second (k x 16 rows): a lane then holds four neighbouring features of
 // one row.  Rows and features beyond the tile's or the matrix's end are computed from clamped
 // addresses and never stored.  K is a multiple of the elements in 16 bytes.
 //   MOE_UP:   x = h [n, K], a row is the token of its pair, scaled by the pair's weight; out_t = act
-//             [total, N] at the sorted row, gelu applied.
-//   MOE_DOWN: x = act [total, K] at the sorted row; out_f [total or n, N] 32-bit at the flat pair
+//             [total, N] at the pair's row (few rows: the flat pair's; many: the sorted one's), gelu applied.
+//   MOE_DOWN: x = act [total, K] at the pair's row; out_f [total or n, N] 32-bit at the flat pair
 //             (add == 0: stored) or at the pair's token (add == 1: added; only with top == 1).
 //   MOE_UP_GATED: x = h [n, K], not scaled; w[e] holds N = 2 * features rows, in turns 16 rows of the gate matrix and the
-//             16 rows of the up matrix that meet them; out_t = act [total, N / 2] at the sorted row,
+//             16 rows of the up matrix that meet them; out_t = act [total, N / 2] at the pair's row,
 //             silu(gate) * up, or with limit > 0 the limited form with alpha and limit.
 template <class T, int MODE>
 __device__ __forceinline__ void moe_store(const f32x4 &acc, int dst, int col0, int N, T *__restrict__ out_t,
@@ -264,77 +267,128 @@ __device__ __forceinline__ void moe_store(const f32x4 &acc, int dst, int col0, i
     }
 }
 
-// Few rows an expert (decoding): tiles of up to 16 rows; a block of four waves takes a tile and 64
-// features, a wave 16 of them, and streams its 16 rows of the weight once, eight steps of loads in flight.
-template <class T, int MODE>
-__global__ void __launch_bounds__(256)
+// Where a lane's part of the matrix lies: lane (g, l16) of unit (16 rows, KSTEP of k) takes row l16, PER_LANE elements from k = g *
+// PER_LANE on.  PACKED: w[e] is [ceil(N / 16)][ceil(K / KSTEP)][64 lanes][PER_LANE], zeros beyond N and K: a wave's load is one piece
+// of 1 KB.  Otherwise it is [N][K], and a load takes half a line of each of 16 rows.
+template <class T, bool PACKED> struct Unit {
+    typedef Mma<T> M;
+    const T *p;
+    int k_left;                                      // elements of k from this lane's first one on (not PACKED)
+    __device__ __forceinline__ Unit(const T *w, int tile, int N, int K, int steps, int lane) {
+        if (PACKED) {
+            const int tiles = (N + 15) / 16;
+            p = w + ((size_t)(tile < tiles ? tile : tiles - 1) * steps * WAVE + lane) * M::PER_LANE;
+        } else {
+            const int row = tile * 16 + lane % 16;
+            p = w + (size_t)(row < N ? row : N - 1) * K + lane / 16 * M::PER_LANE;
+            k_left = K - lane / 16 * M::PER_LANE;
+        }
+    }
+    // read once: past the caches' lines that other data lives in, where a load takes whole lines
+    __device__ __forceinline__ typename M::frag load(int step) const {
+        if (PACKED) return __builtin_nontemporal_load((const typename M::frag *)(p + (size_t)step * WAVE * M::PER_LANE));
+        return step * M::KSTEP < k_left ? M::load(p + step * M::KSTEP) : M::zero();
+    }
+};
+
+// Both kernels sum K in four parts of so many steps (an even number: 128 bytes a row), one after the other, and add the parts up in
+// turn: the kernel for few rows gives each of its waves a part, and a row has the same bits whichever kernel its step goes to.
+__device__ __forceinline__ int quarter_steps(int steps) { return (steps + 7) / 8 * 2; }
+
+// Few rows an expert (decoding).  A workgroup per expert and 32 of its matrix's rows looks through the step's pairs for the expert's
+// (a list in LDS, in any order: a row's result does not depend on its place), and multiplies them 16 at a time; its four waves take a
+// quarter of K each, four steps of loads always on their way, and add up through LDS in a fixed order.
+// What bounds it is the experts' matrices out of memory, once.  One wave for 16 features and all of K left 3 to 4 waves a compute
+// unit, which waited for eight loads and then issued the next eight: 2.8 (gated first product) and 3.2 TB/s (second) for 14 of 16
+// experts of 2 x 1024 x 2048 and 2048 x 1024, 42 and 18 us; now 24 and 14 us, and 16 experts of 2 x 1408 x 2048 52 -> 34.5 us, 5.3 TB/s.
+// (Eight steps on their way and half as many waves: 25 and 37.5.)  The list costs a scan of n * top numbers, but no kernel in front.
+constexpr int MOE_LIST = 2048;
+template <class T, int MODE, bool PACKED>
+__global__ void __launch_bounds__(256, 4)
 moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__ w, size_t w_expert_stride, int N, int K,
-                    const int *__restrict__ sorted_to_flat, const float *__restrict__ wts,
-                    const int *__restrict__ tile_expert, const int *__restrict__ tile_begin,
-                    const int *__restrict__ tile_rows, const int *__restrict__ n_tiles, int /* max_tiles */, T *__restrict__ out_t,
+                    const int *__restrict__ ids, int total, const float *__restrict__ wts, T *__restrict__ out_t,
                     float *__restrict__ out_f, int out_stride, int top, int add, float alpha, float limit) {
     typedef Mma<T> M;
     typedef typename M::frag frag;
-    const int tile = blockIdx.x;
-    if (tile >= n_tiles[0]) return;
-    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, g = lane / 16, l16 = lane % 16;
     constexpr bool GATED = MODE == MOE_UP_GATED, UP = MODE != MOE_DOWN;
-    const int NF = GATED ? N / 2 : N;                // output features
-    const int f0 = blockIdx.y * 64 + wave * 16;
-    if (f0 >= NF) return;
-    const int e = tile_expert[tile], row0 = tile_begin[tile], rows = tile_rows[tile];
-    const int f = f0 + l16 < NF ? f0 + l16 : NF - 1;
-    const int wr = GATED ? (f / 16) * 32 + f % 16 : f;       // the gate's row; the up row that meets it lies 16 further
-    const T *wrow = w + (size_t)e * w_expert_stride + (size_t)wr * K + g * M::PER_LANE;
-    const bool valid = l16 < rows;
-    const int srow = row0 + (valid ? l16 : 0);
-    const int flat = sorted_to_flat[srow];
-    const T *xrow = (UP ? x + (size_t)(flat / top) * x_stride : x + (size_t)srow * x_stride) + g * M::PER_LANE;
-    const float sc = MODE == MOE_UP ? wts[flat] : 1.f;
-    const int dst = UP ? srow : (add ? flat / top : flat);
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f}, acc2 = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int kfull = K / M::KSTEP * M::KSTEP;
-    int k0 = 0;
-    constexpr int AHEAD = 8;                         // steps of loads in flight: a wave's own arithmetic is short
-    for (; k0 + AHEAD * M::KSTEP <= kfull; k0 += AHEAD * M::KSTEP) {
-        frag a[AHEAD], b[AHEAD], a2[GATED ? AHEAD : 1];
+    constexpr int AHEAD = 4;
+    __shared__ int list[MOE_LIST], found;
+    __shared__ f32x4 red[4][2][WAVE];
+    const int e = blockIdx.y, tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, g = lane / 16, l16 = lane % 16;
+    const int tile0 = 2 * blockIdx.x, steps = (K + M::KSTEP - 1) / M::KSTEP, per = quarter_steps(steps);
+    const int s0 = wave * per, s1 = min(steps, s0 + per);
+    const Unit<T, PACKED> w0(w + (size_t)e * w_expert_stride, tile0, N, K, steps, lane), w1(w + (size_t)e * w_expert_stride, tile0 + 1, N, K, steps, lane);
+    for (int first = 0; first < total; first += MOE_LIST) {
+        __syncthreads();                             // the list of before has been read
+        if (tid == 0) found = 0;
+        __syncthreads();
+        for (int p = first + tid; p < min(total, first + MOE_LIST); p += 256)
+            if (ids[p] == e) list[atomicAdd(&found, 1)] = p;
+        __syncthreads();
+        const int count = found;
+        for (int r0 = 0; r0 < count; r0 += 16) {
+            const bool valid = r0 + l16 < count;
+            const int flat = list[valid ? r0 + l16 : r0];
+            const T *xrow = x + (size_t)(UP ? flat / top : flat) * x_stride + g * M::PER_LANE;
+            const float sc = MODE == MOE_UP ? wts[flat] : 1.f;
+            const int x_left = K - g * M::PER_LANE;
+            f32x4 acc0 = f32x4{0.f, 0.f, 0.f, 0.f}, acc1 = f32x4{0.f, 0.f, 0.f, 0.f};
+            frag a0[AHEAD], a1[AHEAD], b[AHEAD];
+            auto fetch = [&](int u, int s) {
+                a0[u] = w0.load(s);
+                a1[u] = w1.load(s);
+                b[u] = s * M::KSTEP < x_left ? M::load(xrow + s * M::KSTEP) : M::zero();
+            };
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u) a[u] = M::load(wrow + k0 + u * M::KSTEP);    // (through the caches: a load takes half of each line, the next one the other half)
-        if (GATED) {
+            for (int u = 0; u < AHEAD; ++u)
+                if (s0 + u < s1) fetch(u, s0 + u);
+            for (int s = s0; s < s1; s += AHEAD) {
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u) a2[GATED ? u : 0] = M::load(wrow + (size_t)16 * K + k0 + u * M::KSTEP);
+                for (int u = 0; u < AHEAD; ++u) {
+                    if (s + u >= s1) break;
+                    const frag bb = MODE == MOE_UP ? M::scaled(b[u], sc) : b[u];
+                    acc0 = M::mma(a0[u], bb, acc0);
+                    acc1 = M::mma(a1[u], bb, acc1);
+                    if (s + u + AHEAD < s1) fetch(u, s + u + AHEAD);
+                }
+            }
+            if (r0) __syncthreads();                 // the sums of the rows before have been read
+            red[wave][0][lane] = acc0;
+            red[wave][1][lane] = acc1;
+            __syncthreads();
+            // the first wave stores (with two products' sums the first two, one each): four neighbouring features of a row a lane
+            if (wave < (GATED ? 1 : 2)) {
+                const f32x4 v = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
+                const int dst = !UP && add ? flat / top : flat;
+                if constexpr (GATED) {
+                    const f32x4 up = ((red[0][1][lane] + red[1][1][lane]) + red[2][1][lane]) + red[3][1][lane];
+                    Quad<T> q;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gate_up_of(v[i], up[i], alpha, limit));
+                    if (valid && tile0 * 16 < N) *(Quad<T> *)(out_t + (size_t)dst * out_stride + tile0 * 8 + 4 * g) = q;
+                } else {
+                    const int col = (tile0 + wave) * 16 + 4 * g;         // (N is a multiple of 4)
+                    if (valid && col < N) {
+                        if constexpr (MODE == MOE_UP) {
+                            Quad<T> q;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gelu_erf(v[i]));
+                            *(Quad<T> *)(out_t + (size_t)dst * out_stride + col) = q;
+                        } else {
+                            f32x4 *o = (f32x4 *)(out_f + (size_t)dst * out_stride + col);
+                            *o = add ? *o + v : v;
+                        }
+                    }
+                }
+            }
         }
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) b[u] = M::load(xrow + k0 + u * M::KSTEP);
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-            acc = M::mma(a[u], MODE == MOE_UP ? M::scaled(b[u], sc) : b[u], acc);
-            if (GATED) acc2 = M::mma(a2[GATED ? u : 0], b[u], acc2);
-        }
-    }
-    for (; k0 < K; k0 += M::KSTEP) {                 // the steps that are left, the last one perhaps in part
-        const bool in = k0 + g * M::PER_LANE < K;
-        const frag a = in ? M::load(wrow + k0) : M::zero();
-        const frag b = in ? M::load(xrow + k0) : M::zero();
-        acc = M::mma(a, MODE == MOE_UP ? M::scaled(b, sc) : b, acc);
-        if (GATED) acc2 = M::mma(in ? M::load(wrow + (size_t)16 * K + k0) : M::zero(), b, acc2);
-    }
-    if (!valid) return;
-    if (GATED) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int col = f0 + 4 * g + i;
-            if (col < NF) out_t[(size_t)dst * out_stride + col] = from_f32<T>(gate_up_of(acc[i], acc2[i], alpha, limit));
-        }
-    } else {
-        moe_store<T, MODE>(acc, dst, f0 + 4 * g, N, out_t, out_f, out_stride, add);
     }
 }
 
 // Many rows an expert (prompts): tiles of up to 64 rows; a block of four waves takes a tile and 128
 // features.  Rows and weights go through LDS in steps of 128 bytes of k, the next step's loads on their
 // way while one is multiplied; a wave multiplies 32 features with all 64 rows (eight sums).
-template <class T, int MODE>
+template <class T, int MODE, bool PACKED>
 __global__ void __launch_bounds__(256)
 moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__ w, size_t w_expert_stride, int N, int K,
                      const int *__restrict__ sorted_to_flat, const float *__restrict__ wts,
@@ -374,29 +428,43 @@ moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict_
             xsc[i] = 1.f;
         }
     }
+    // the weight's piece i of this thread: row wr[i] of the tile, 16 bytes of k from element wk on
+    constexpr int SS = KS / M::KSTEP;               // units of k a step
+    const int steps = (K + M::KSTEP - 1) / M::KSTEP;
     const T *wptr[4];
+    int wr[4], wk;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int fr = n0 + tid / CH + 32 * i;
-        wptr[i] = w + (size_t)e * w_expert_stride + (size_t)(fr < N ? fr : N - 1) * K + ch * PL;
+        if (PACKED) {                               // a wave takes whole units: pieces tid + 256 i of [8 tiles of rows][SS][64 lanes]
+            const int unit = wave + 4 * i, rt = unit / SS, tiles = (N + 15) / 16, t = n0 / 16 + rt;
+            wr[i] = 16 * rt + l16;
+            wk = unit % SS * M::KSTEP + g * PL;     // (4 units are whole rows of units: the same for every i)
+            wptr[i] = w + (size_t)e * w_expert_stride + (((size_t)(t < tiles ? t : tiles - 1) * steps + unit % SS) * WAVE + lane) * PL;
+        } else {
+            const int fr = n0 + tid / CH + 32 * i;
+            wr[i] = tid / CH + 32 * i;
+            wk = ch * PL;
+            wptr[i] = w + (size_t)e * w_expert_stride + (size_t)(fr < N ? fr : N - 1) * K + ch * PL;
+        }
     }
     frag xreg[2], wreg[4];
     auto from_memory = [&](int k0) {
-        const bool in = k0 + ch * PL < K;
+        const bool in = k0 + ch * PL < K, w_in = PACKED ? k0 + wk / M::KSTEP * M::KSTEP < K : in;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) wreg[i] = in ? M::load(wptr[i] + k0) : M::zero();
+        for (int i = 0; i < 4; ++i) wreg[i] = w_in ? M::load(wptr[i] + (PACKED ? (size_t)(k0 / M::KSTEP) * WAVE * PL : k0)) : M::zero();
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             xreg[i] = in ? M::load(xptr[i] + k0) : M::zero();
             if (MODE == MOE_UP) xreg[i] = M::scaled(xreg[i], xsc[i]);
         }
     };
-    f32x4 acc[2][4];
+    f32x4 acc[2][4], sum[2][4];
 #pragma unroll
     for (int ft = 0; ft < 2; ++ft)
 #pragma unroll
-        for (int m = 0; m < 4; ++m) acc[ft][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int m = 0; m < 4; ++m) acc[ft][m] = sum[ft][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     from_memory(0);
+    int left = quarter_steps(steps) / SS;           // steps of this part that are left
     // (one buffer and two barriers a step: with two buffers in turn and one barrier the kernel was a quarter slower, its
     // workgroups being fewer on a compute unit)
     for (int k0 = 0; k0 < K; k0 += KS) {
@@ -404,8 +472,19 @@ moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict_
 #pragma unroll
         for (int i = 0; i < 2; ++i) *(frag *)(xs + (tid / CH + 32 * i) * LD + ch * PL) = xreg[i];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *(frag *)(ws + (tid / CH + 32 * i) * LD + ch * PL) = wreg[i];
+        for (int i = 0; i < 4; ++i) *(frag *)(ws + wr[i] * LD + wk) = wreg[i];
         __syncthreads();
+        if (left == 0) {
+            left = quarter_steps(steps) / SS;
+#pragma unroll
+            for (int ft = 0; ft < 2; ++ft)
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    sum[ft][m] += acc[ft][m];
+                    acc[ft][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+        --left;
         if (k0 + KS < K) from_memory(k0 + KS);
 #pragma unroll
         for (int ks = 0; ks < KS / M::KSTEP; ++ks) {
@@ -423,6 +502,10 @@ moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict_
             }
         }
     }
+#pragma unroll
+    for (int ft = 0; ft < 2; ++ft)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc[ft][m] = sum[ft][m] + acc[ft][m];
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         const int r = 16 * m + l16;
@@ -468,9 +551,9 @@ __global__ void moe_combine_kernel(float *__restrict__ out, const float *__restr
     }
 }
 
-// Rows of a tile for n * top pairs over so many experts: 16 (the kernel for few rows) while an expert has 16 rows
-// or fewer on average, else 64.  The caller sizes its scratch with it: max_tiles = min(total, total / rows + experts).
-LCU_API int lcu_moe_tile_rows(int total, int experts) { return (long long)total <= 16ll * experts ? 16 : MOE_TILE_ROWS; }
+// Rows of a tile for n * top pairs over so many experts: 0 (the kernel for few rows, which has no tiles) while an expert has 16 rows
+// or fewer on average, else 64.  The caller sizes its scratch with it: max_tiles = min(total, total / rows + experts), or 0.
+LCU_API int lcu_moe_tile_rows(int total, int experts) { return (long long)total <= 16ll * experts ? 0 : MOE_TILE_ROWS; }
 
 // h: [n, d] of `type`; router: [experts, d] 32-bit; ids, wts: [n * top].
 // bias: null or [experts] 32-bit; mode 0: sigmoid weights, 1: softmax over the chosen; extra, gates: see the kernel
@@ -494,8 +577,8 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
 }
 
 // ints: scratch of total + 3 * max_tiles + 1 entries, laid out as sorted_to_flat, tile_expert, tile_begin,
-// tile_rows, n_tiles.
-// w_up: [experts, ff, d], w_down: [experts, d, ff] of `type`.  act: scratch [total, ff] of `type`; y: scratch
+// tile_rows, n_tiles (null where lcu_moe_tile_rows says 0).
+// w_up: [experts, ff, d], w_down: [experts, d, ff] of `type`; packed_up, packed_down: in the order of Unit.  act: scratch [total, ff] of `type`; y: scratch
 // [total, d] 32-bit (only read and written when top > 1 or gated).  out: [n, d] 32-bit, added to.
 // gated: w_up is [experts, 2 * ff, d], in turns 16 rows of the gate matrix and the 16 rows of the up matrix that meet
 // them (ff a multiple of 16); act = silu(gate h) * (up h), and the weight scales what comes out; fresh: out is written
@@ -503,46 +586,60 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
 // token's input.  shared (null or
 // [n, d] of `type`) with shared_gate (null or [n] 32-bit): rows that are added beside the experts', times the gate.
 LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float *wts, int *ints, int max_tiles,
-                            const void *w_up, const void *w_down, void *act, float *y, float *out, int n, int d, int ff,
+                            const void *w_up, int packed_up, const void *w_down, int packed_down, void *act, float *y, float *out, int n, int d, int ff,
                             int experts, int top, int gated, const void *shared, const float *shared_gate, int fresh,
                             int identity, float alpha, float limit, hipStream_t stream) {
     if (n <= 0) return LCU_OK;
     const int per = type == LCU_BF16 ? 8 : 4;
-    if (d <= 0 || ff <= 0 || d % per || ff % per || experts <= 0 || experts > MOE_MAX_EXPERTS || top <= 0 || max_tiles <= 0 ||
+    if (d <= 0 || ff <= 0 || d % per || ff % per || experts <= 0 || experts > MOE_MAX_EXPERTS || top <= 0 ||
         (type != LCU_F32 && type != LCU_BF16) || (gated && ff % 16) || (shared && !gated) || (fresh && !gated) || identity < 0 ||
         (identity && !gated) || experts + identity > MOE_MAX_EXPERTS)
         return LCU_BAD_ARGUMENT;
     const int total = n * top;
-    const int tile_rows = lcu_moe_tile_rows(total, experts);
-    int *sorted = ints, *t_exp = ints + total, *t_beg = t_exp + max_tiles, *t_rows = t_beg + max_tiles, *n_tiles = t_rows + max_tiles;
-    moe_group_kernel<<<dim3(1), dim3(1024), 0, stream>>>(ids, total, experts + identity, sorted, t_exp, t_beg, t_rows, n_tiles, max_tiles, tile_rows, experts);
-    LCU_LAUNCH_CHECK();
+    const bool few = lcu_moe_tile_rows(total, experts) == 0;
     const int add = top == 1 && !gated;
     float *down_to = add ? out : y;
     if (!add && !y) return LCU_BAD_ARGUMENT;
-    const int per_block = tile_rows == 16 ? 64 : 128;         // features a block takes
-    dim3 block(256), gu(max_tiles, (ff + per_block - 1) / per_block), gd(max_tiles, (d + per_block - 1) / per_block);
     const int up_rows = gated ? 2 * ff : ff;                  // rows of an expert's first matrix
-    if (tile_rows != 16) {                                    // a flat grid: the kernel shares it out over the dies itself
-        gu = dim3(8 * max_tiles * (((up_rows + 127) / 128 + 7) / 8));
-        gd = dim3(8 * max_tiles * (((d + 127) / 128 + 7) / 8));
-    }
-#define GO(KERNEL, T)                                                                                                              \
-    if (gated)                                                                                                                     \
-        KERNEL<T, MOE_UP_GATED><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, (size_t)up_rows * d, up_rows, d, sorted, wts, \
-                                                      t_exp, t_beg, t_rows, n_tiles, max_tiles, (T *)act, nullptr, ff, top, 0, alpha, limit);       \
-    else                                                                                                                           \
-        KERNEL<T, MOE_UP><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, (size_t)ff * d, ff, d, sorted, wts, t_exp, t_beg, \
-                                                t_rows, n_tiles, max_tiles, (T *)act, nullptr, ff, top, 0, 0.f, 0.f);                         \
-    KERNEL<T, MOE_DOWN><<<gd, block, 0, stream>>>((const T *)act, ff, (const T *)w_down, (size_t)ff * d, d, ff, sorted, wts, t_exp, \
-                                                  t_beg, t_rows, n_tiles, max_tiles, nullptr, down_to, d, top, add, 0.f, 0.f)
-    if (type == LCU_BF16) {
-        if (tile_rows == 16) { GO(moe_gemm_few_kernel, bf16_t); } else { GO(moe_gemm_many_kernel, bf16_t); }
+    const int kstep = type == LCU_BF16 ? 32 : 16;             // elements an expert's matrix takes
+    auto elems = [&](int rows, int k, int packed) { return packed ? (size_t)((rows + 15) / 16 * 16) * ((k + kstep - 1) / kstep * kstep) : (size_t)rows * k; };
+    const size_t up_stride = elems(up_rows, d, packed_up), down_stride = elems(d, ff, packed_down);
+#define TYPED(GO, ...)                                                                                             \
+    if (type == LCU_BF16) { if (packed) GO(bf16_t, true, __VA_ARGS__); else GO(bf16_t, false, __VA_ARGS__); }       \
+    else { if (packed) GO(float, true, __VA_ARGS__); else GO(float, false, __VA_ARGS__); }                          \
+    LCU_LAUNCH_CHECK()
+    if (few) {
+        if (!ids) return LCU_BAD_ARGUMENT;
+        const dim3 block(256), gu((up_rows + 31) / 32, experts), gd((d + 31) / 32, experts);
+#define UP(T, PACKED, MODE) moe_gemm_few_kernel<T, MODE, PACKED><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \
+                                                ids, total, wts, (T *)act, nullptr, ff, top, 0, alpha, limit)
+#define DOWN(T, PACKED, MODE) moe_gemm_few_kernel<T, MODE, PACKED><<<gd, block, 0, stream>>>((const T *)act, ff, (const T *)w_down, down_stride, d, ff, \
+                                                ids, total, wts, nullptr, down_to, d, top, add, 0.f, 0.f)
+        int packed = packed_up;
+        if (gated) { TYPED(UP, MOE_UP_GATED); } else { TYPED(UP, MOE_UP); }
+        packed = packed_down;
+        TYPED(DOWN, MOE_DOWN);
+#undef UP
+#undef DOWN
     } else {
-        if (tile_rows == 16) { GO(moe_gemm_few_kernel, float); } else { GO(moe_gemm_many_kernel, float); }
+        if (!ints || max_tiles <= 0) return LCU_BAD_ARGUMENT;
+        int *sorted = ints, *t_exp = ints + total, *t_beg = t_exp + max_tiles, *t_rows = t_beg + max_tiles, *n_tiles = t_rows + max_tiles;
+        moe_group_kernel<<<dim3(1), dim3(1024), 0, stream>>>(ids, total, experts + identity, sorted, t_exp, t_beg, t_rows, n_tiles, max_tiles, MOE_TILE_ROWS, experts);
+        LCU_LAUNCH_CHECK();
+        // flat grids: the kernel shares them out over the dies itself
+        const dim3 block(256), gu(8 * max_tiles * (((up_rows + 127) / 128 + 7) / 8)), gd(8 * max_tiles * (((d + 127) / 128 + 7) / 8));
+#define UP(T, PACKED, MODE) moe_gemm_many_kernel<T, MODE, PACKED><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \
+                                                sorted, wts, t_exp, t_beg, t_rows, n_tiles, max_tiles, (T *)act, nullptr, ff, top, 0, alpha, limit)
+#define DOWN(T, PACKED, MODE) moe_gemm_many_kernel<T, MODE, PACKED><<<gd, block, 0, stream>>>((const T *)act, ff, (const T *)w_down, down_stride, d, ff, \
+                                                sorted, wts, t_exp, t_beg, t_rows, n_tiles, max_tiles, nullptr, down_to, d, top, add, 0.f, 0.f)
+        int packed = packed_up;
+        if (gated) { TYPED(UP, MOE_UP_GATED); } else { TYPED(UP, MOE_UP); }
+        packed = packed_down;
+        TYPED(DOWN, MOE_DOWN);
+#undef UP
+#undef DOWN
     }
-#undef GO
-    LCU_LAUNCH_CHECK();
+#undef TYPED
     if (!add) {
         const dim3 gc((d + 255) / 256, n < 65535 ? n : 65535);
         const int *idp = identity ? ids : nullptr;

@@ -8,7 +8,8 @@ CPU path: a tensor that is not on the GPU is an error.
 from __future__ import annotations
 
 import ctypes
-from typing import Dict, Optional
+from dataclasses import dataclass
+from typing import Dict, Optional, Tuple
 
 import torch
 
@@ -1377,17 +1378,18 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
     weight scales what goes INTO the expert, not what comes out).  ``w_up [experts, ff, d]``, ``w_down [experts, d, ff]`` in ``h``'s type,
     ``out`` float32 ``[n, d]``.  ``gated``: ``out[t] += sum_e weight * w_down[e] @ (silu(gate[e] @ h[t]) * (up[e] @ h[t]))``
     with ``w_up [experts, 2 * ff, d]`` holding in turns 16 rows of the gate matrix and the 16 up rows that meet them
-    (``gated_rows`` lays them out so); ``shared [n, d]`` (with ``shared_gate [n]`` float32, or ones) is added beside;
+    (``gated_rows`` lays them out so); either matrix may be given as ``pack_experts`` makes it; ``shared [n, d]`` (with ``shared_gate [n]`` float32, or ones) is added beside;
     ``fresh``: ``out`` is written, not added to (it need not hold anything).  ``identity``: ``ids`` may name ``experts +
     identity`` experts, of which the last ``identity`` have no matrices: their output is ``weight * h[t]`` (gated form only).
     ``act_limit`` > 0: the limited activation (``swiglu``) with ``act_alpha`` instead of silu."""
-    _gpu(h, ids, wts, w_up, w_down, out, shared, shared_gate)
+    up, down = (w.data if isinstance(w, PackedExperts) else w for w in (w_up, w_down))
+    _gpu(h, ids, wts, up, down, out, shared, shared_gate)
     _rows(h, "moe input")
-    for t, what in ((h, "moe input"), (ids, "moe ids"), (wts, "moe weights"), (w_up, "moe up"), (w_down, "moe down"), (out, "moe out")):
+    for t, what in ((h, "moe input"), (ids, "moe ids"), (wts, "moe weights"), (up, "moe up"), (down, "moe down"), (out, "moe out")):
         _contig(t, what)
     n, d = h.shape
-    experts, ff = w_down.shape[0], w_down.shape[2] if w_down.dim() == 3 else 0
-    if w_up.dim() != 3 or w_down.dim() != 3 or w_up.shape != (experts, (2 if gated else 1) * ff, d) or w_down.shape[1] != d \
+    experts, ff = w_down.shape[0], w_down.shape[2] if len(w_down.shape) == 3 else 0
+    if len(w_up.shape) != 3 or len(w_down.shape) != 3 or w_up.shape != (experts, (2 if gated else 1) * ff, d) or w_down.shape[1] != d \
             or w_up.dtype != h.dtype or w_down.dtype != h.dtype:
         raise KernelError(f"moe_experts: up {tuple(w_up.shape)} {w_up.dtype} and down {tuple(w_down.shape)} {w_down.dtype} do not fit rows of {d} {h.dtype}")
     top = ids.shape[1] if ids.dim() == 2 else 0
@@ -1414,15 +1416,40 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
     lib = build.load("moe")
     total = n * top
     tile = lib.lcu_moe_tile_rows(total, experts)
-    max_tiles = min(total, total // tile + experts)
-    ints = torch.empty(total + 3 * max_tiles + 1, dtype=torch.int32, device=h.device)
+    max_tiles = min(total, total // tile + experts) if tile else 0
+    ints = torch.empty(total + 3 * max_tiles + 1, dtype=torch.int32, device=h.device) if tile else None
     act = torch.empty((total, ff), dtype=h.dtype, device=h.device)
     y = torch.empty((total, d), dtype=torch.float32, device=h.device) if (top > 1 or gated) else None
-    _check(lib.lcu_moe_experts(_ptr(h), _type(h, "moe input"), _ptr(ids), _ptr(wts), _ptr(ints), max_tiles, _ptr(w_up),
-                               _ptr(w_down), _ptr(act), _ptr(y), _ptr(out), n, d, ff, experts, top, int(bool(gated)),
+    _check(lib.lcu_moe_experts(_ptr(h), _type(h, "moe input"), _ptr(ids), _ptr(wts), _ptr(ints), max_tiles, _ptr(up),
+                               int(up is not w_up), _ptr(down), int(down is not w_down), _ptr(act), _ptr(y), _ptr(out), n, d, ff, experts, top, int(bool(gated)),
                                _ptr(shared), _ptr(shared_gate if shared is not None else None), int(bool(fresh)), identity, ctypes.c_float(act_alpha),
                                ctypes.c_float(act_limit), _stream()), "moe_experts")
     return out
+
+
+@dataclass(frozen=True)
+class PackedExperts:
+    """Experts' matrices ``[experts, rows, k]`` in the order in which the experts' kernels load them (``pack_experts``)."""
+    data: torch.Tensor
+    shape: Tuple[int, int, int]
+
+    @property
+    def dtype(self):
+        return self.data.dtype
+
+
+def pack_experts(w: torch.Tensor) -> PackedExperts:
+    """``w [experts, rows, k]`` (bfloat16 or float32) as units of 16 rows times 64 bytes of k, one after the other along k, then
+    along the rows; in a unit the 16 rows' first 16 bytes stand first, then their second, and so on.  Rows and columns of
+    zeros fill the last units."""
+    e, n, k = w.shape
+    per = 8 if w.dtype == torch.bfloat16 else 4
+    if w.dtype not in (torch.bfloat16, torch.float32):
+        raise KernelError(f"pack_experts: {w.dtype} is not supported")
+    if n % 16 or k % (4 * per):
+        w = torch.nn.functional.pad(w, (0, -k % (4 * per), 0, -n % 16))
+    units = w.reshape(e, w.shape[1] // 16, 16, w.shape[2] // (4 * per), 4, per)
+    return PackedExperts(units.permute(0, 1, 3, 4, 2, 5).contiguous(), (e, n, k))
 
 
 def gated_rows(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:

@@ -62,6 +62,8 @@ class SigmoidMoE(Part):
             pad = 8 - ff % 8
             self.w_up = torch.cat([self.w_up, self.w_up.new_zeros(n, pad, d)], dim=1).contiguous()
             self.w_down = torch.cat([self.w_down, self.w_down.new_zeros(n, d, pad)], dim=2).contiguous()
+        if build.pack_weights:
+            self.w_up, self.w_down = ops.pack_experts(self.w_up), ops.pack_experts(self.w_down)
         self.dtype = build.dtype
 
     def forward(self, h, add_to: Optional[torch.Tensor] = None):
@@ -191,6 +193,8 @@ class GatedMoE(Part):
             gate, up, self.router = fill(gate, (0, self.pad_width)), fill(up, (0, self.pad_width)), fill(self.router, (0, self.pad_width)).contiguous()
             self.w_down = fill(self.w_down, (0, 0, 0, self.pad_width)).contiguous()
         self.w_gate_up = ops.gated_rows(gate.contiguous(), up.contiguous())
+        if build.pack_weights:
+            self.w_gate_up, self.w_down = ops.pack_experts(self.w_gate_up), ops.pack_experts(self.w_down)
         if self.shared is not None:
             self.shared.load(tensors, build)
         self.dtype = build.dtype

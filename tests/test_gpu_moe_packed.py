@@ -1,0 +1,64 @@
+"""Experts' matrices in the kernels' own order (``ops.pack_experts``) against the matrices as they are, and the kernel for few rows
+an expert at the edges of its lists, tiles and quarters of K."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+import plain_divasun as P
+from divasun_common import assert_close
+from test_gpu_divasun import F64, TYPES, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+# one pair; an expert with 17 rows (two tiles) and K of less than a step; K that ends within a step, and rows that end within a tile;
+# more pairs than a list holds; the kernel for many rows; every quarter of K of another length
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("experts,top,d,ff,n", [(4, 1, 72, 24, 1), (2, 1, 16, 8, 31), (5, 2, 200, 88, 33), (160, 8, 72, 16, 300), (4, 2, 264, 136, 300),
+                                                (8, 3, 1032, 40, 40)])
+def test_packed_experts(dtype, experts, top, d, ff, n):
+    from llama_cu_amd.kernels import ops
+    tdt = TYPES[dtype]
+    h, router = rnd(n, d, seed=1).to(tdt).cuda(), rnd(experts, d, seed=2, std=0.5).cuda()
+    up, down = rnd(experts, ff, d, seed=3, std=d ** -0.5).to(tdt).cuda(), rnd(experts, d, ff, seed=4, std=ff ** -0.5).to(tdt).cuda()
+    base = rnd(n, d, seed=5)
+    ids, wts = ops.moe_route(h, router, top)
+    outs = []
+    for u, w in ((up, down), (ops.pack_experts(up), ops.pack_experts(down)), (up, ops.pack_experts(down))):
+        out = base.clone().cuda()
+        ops.moe_experts(h, ids, wts, u, w, out)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    plain = {"router": router.cpu().to(F64)}
+    for e in range(experts):
+        plain[f"e{e}.up"], plain[f"e{e}.down"] = up[e].cpu().to(F64), down[e].cpu().to(F64)
+    want = base.to(F64) + P.moe(h.cpu().to(F64), plain, experts, top)
+    assert_close(outs[0], want, 1e-4 if dtype == "float32" else 3e-2, "output")      # (the bounds of the unpacked experts' test)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("n,ff", [(1, 16), (20, 48), (200, 112)])
+def test_packed_gated_experts(dtype, n, ff):
+    from llama_cu_amd.kernels import ops
+    experts, top, d, tdt = 6, 2, 104, TYPES[dtype]
+    h, router = rnd(n, d, seed=1).to(tdt).cuda(), rnd(experts + 1, d, seed=2).cuda()
+    gate, up = (rnd(experts, ff, d, seed=k, std=d ** -0.5).to(tdt).cuda() for k in (3, 4))
+    down = rnd(experts, d, ff, seed=5, std=ff ** -0.5).to(tdt).cuda()
+    ids, wts = ops.moe_route(h, router, top, softmax_chosen=True)        # (the last of the router's rows is an identity expert)
+    rows, outs = ops.gated_rows(gate, up), []
+    for u, w in ((rows, down), (ops.pack_experts(rows), ops.pack_experts(down))):
+        out = torch.empty(n, d, device="cuda")
+        ops.moe_experts(h, ids, wts, u, w, out, gated=True, fresh=True, identity=1, act_alpha=1.702, act_limit=2.0)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    x, want = h.cpu().to(F64), torch.zeros(n, d, dtype=F64)
+    for t in range(n):
+        for e, w in zip(ids[t].tolist(), wts[t].cpu().to(F64)):
+            if e == experts:
+                want[t] += w * x[t]
+                continue
+            g = torch.clamp(gate[e].cpu().to(F64) @ x[t], max=2.0)
+            v = torch.clamp(up[e].cpu().to(F64) @ x[t], -2.0, 2.0)
+            want[t] += w * (down[e].cpu().to(F64) @ (g * torch.sigmoid(1.702 * g) * (v + 1.0)))
+    assert_close(outs[0], want, 1e-4 if dtype == "float32" else 3e-2, "output")
