@@ -33,3 +33,16 @@ __device__ __forceinline__ float wave_sum_in_place(float v) {
     const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);     // (lower half twice, upper half twice)
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
+
+// The largest of a wave's values (NaN is passed over), in all lanes.
+__device__ __forceinline__ float wave_max_in_place(float v) {
+    v = fmaxf(v, lane_xor1(v));
+    v = fmaxf(v, lane_xor2(v));
+    v = fmaxf(v, lane_mirror8(v));
+    v = fmaxf(v, lane_mirror16(v));
+    const unsigned u = __float_as_uint(v);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned w = __float_as_uint(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+    const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}

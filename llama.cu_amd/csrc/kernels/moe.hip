@@ -19,6 +19,7 @@
 // the batch.
 #include "common.h"
 #include "gate_act.h"
+#include "lane_moves.h"
 
 constexpr int MOE_MAX_EXPERTS = 1024;
 constexpr int MOE_TILE_ROWS = 64;        // rows of a tile of the kernel for many rows
@@ -65,21 +66,39 @@ moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, cons
                 for (int e = 0; e < 8; ++e) x[k][e] = to_f32(in.v[e]);
             }
         }
-        for (int e = wave; e < experts; e += THREADS / WAVE) {
-            const float *w = router + (size_t)e * d;
-            float acc = 0.f;
+        // two rows of the router at a time, so that 17 rows on 16 waves (16 experts and a gate) are not two trips to memory
+        for (int e = wave; e < experts; e += 2 * (THREADS / WAVE)) {
+            const int e2 = e + THREADS / WAVE;
+            const float *w = router + (size_t)e * d, *v = router + (size_t)(e2 < experts ? e2 : e) * d;
+            float acc = 0.f, acc2 = 0.f;
+            if (e2 < experts) {
 #pragma unroll
-            for (int k = 0; k < ROUTE_CHUNKS; ++k) {
-                const int c = k * 512 + lane * 8;
-                if (c < d) {
-                    const f32x4 w0 = *(const f32x4 *)(w + c), w1 = *(const f32x4 *)(w + c + 4);
+                for (int k = 0; k < ROUTE_CHUNKS; ++k) {
+                    const int c = k * 512 + lane * 8;
+                    if (c < d) {
+                        const f32x4 w0 = *(const f32x4 *)(w + c), w1 = *(const f32x4 *)(w + c + 4), v0 = *(const f32x4 *)(v + c), v1 = *(const f32x4 *)(v + c + 4);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) acc += x[k][i] * w0[i];
+                        for (int i = 0; i < 4; ++i) { acc += x[k][i] * w0[i]; acc2 += x[k][i] * v0[i]; }
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) acc += x[k][4 + i] * w1[i];
+                        for (int i = 0; i < 4; ++i) { acc += x[k][4 + i] * w1[i]; acc2 += x[k][4 + i] * v1[i]; }
+                    }
+                }
+                acc2 = wave_sum_in_place(acc2);
+                if (lane == 0) z[e2] = acc2 + (logit_bias && e2 < n_experts ? logit_bias[e2] : 0.f);
+            } else {
+#pragma unroll
+                for (int k = 0; k < ROUTE_CHUNKS; ++k) {
+                    const int c = k * 512 + lane * 8;
+                    if (c < d) {
+                        const f32x4 w0 = *(const f32x4 *)(w + c), w1 = *(const f32x4 *)(w + c + 4);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc += x[k][i] * w0[i];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc += x[k][4 + i] * w1[i];
+                    }
                 }
             }
-            acc = wave_sum(acc);
+            acc = wave_sum_in_place(acc);
             if (lane == 0) z[e] = acc + (logit_bias && e < n_experts ? logit_bias[e] : 0.f);
         }
     } else {
@@ -87,49 +106,59 @@ moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, cons
             const float *w = router + (size_t)e * d;
             float acc = 0.f;
             for (int c = lane; c < d; c += WAVE) acc += to_f32(row[c]) * w[c];
-            acc = wave_sum(acc);
+            acc = wave_sum_in_place(acc);
             if (lane == 0) z[e] = acc + (logit_bias && e < n_experts ? logit_bias[e] : 0.f);
         }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < extra; e += THREADS) gates[(size_t)t * extra + e] = 1.0f / (1.0f + expf(-z[n_experts + e]));
+    // the first wave does the rest alone
+    if (wave != 0) return;
+    for (int e = lane; e < extra; e += WAVE) gates[(size_t)t * extra + e] = 1.0f / (1.0f + expf(-z[n_experts + e]));
+    const bool one_each = n_experts <= WAVE;         // an expert a lane: the choice stays in registers
     if (mode == 2) {                                 // scores over all experts; z becomes what the choice goes by
-        if (wave == 0) {
-            float m = -INFINITY;
-            for (int e = lane; e < n_experts; e += WAVE) m = fmaxf(m, z[e]);
-            m = wave_max(m);
-            float part = 0.f;
-            for (int e = lane; e < n_experts; e += WAVE) part += expf(z[e] - m);
-            const float sum = wave_sum(part);
-            for (int e = lane; e < n_experts; e += WAVE) {
-                const float s = expf(z[e] - m) / sum;
-                sc[e] = s;
-                z[e] = s + (bias ? bias[e] : 0.f);
-            }
+        float m = -INFINITY;
+        for (int e = lane; e < n_experts; e += WAVE) m = fmaxf(m, z[e]);
+        m = wave_max_in_place(m);
+        float part = 0.f;
+        for (int e = lane; e < n_experts; e += WAVE) part += expf(z[e] - m);
+        const float sum = wave_sum_in_place(part);
+        for (int e = lane; e < n_experts; e += WAVE) {
+            const float s = expf(z[e] - m) / sum;
+            sc[e] = s;
+            z[e] = s + (bias ? bias[e] : 0.f);
         }
-        __syncthreads();
+        __threadfence_block();
         if (groups > 1) {
             // every group's best (in zc), then every group's place among them; the experts of a group behind the kept ones are out
             const int per = n_experts / groups;
-            for (int g = threadIdx.x; g < groups; g += THREADS) {
+            for (int g = lane; g < groups; g += WAVE) {
                 float best = z[g * per];
                 for (int e = 1; e < per; ++e) best = fmaxf(best, z[g * per + e]);
                 zc[g] = best;
             }
-            __syncthreads();
-            for (int g = threadIdx.x; g < groups; g += THREADS) {
+            __threadfence_block();
+            for (int g = lane; g < groups; g += WAVE) {
                 int before = 0;
                 for (int o = 0; o < groups; ++o) before += zc[o] > zc[g] || (zc[o] == zc[g] && o < g);
                 if (before >= keep)
                     for (int e = 0; e < per; ++e) z[g * per + e] = -INFINITY;
             }
-            __syncthreads();
+            __threadfence_block();
         }
     }
-    for (int k = 0; k < top; ++k) {                  // the first wave chooses; the others only keep the barriers
-        if (wave == 0) {
+    float mine = lane < n_experts ? z[lane] : -INFINITY;
+    for (int k = 0; k < top; ++k) {
+        int arg;
+        float value;                                 // what the weight is made of
+        if (one_each) {
+            const float best = wave_max_in_place(mine);
+            const unsigned long long who = __ballot(lane < n_experts && mine == best);
+            arg = who ? __ffsll((long long)who) - 1 : 0;     // the lowest of equals; every logit NaN: any expert
+            value = mode == 2 ? sc[arg] : z[arg];
+            if (lane == arg) mine = -INFINITY;
+        } else {
             float best = -INFINITY;
-            int arg = 0x7fffffff;
+            arg = 0x7fffffff;
             for (int e = lane; e < n_experts; e += WAVE) {
                 const float v = z[e];
                 if (v > best || (v == best && e < arg)) { best = v; arg = e; }
@@ -140,27 +169,30 @@ moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, cons
                 const int oa = __shfl_xor(arg, off, WAVE);
                 if (ob > best || (ob == best && oa < arg)) { best = ob; arg = oa; }
             }
-            if (arg >= n_experts) arg = 0;               // every logit NaN: any expert
-            if (lane == 0) {
-                ids[(size_t)t * top + k] = arg;
-                zc[k] = mode == 2 ? sc[arg] : z[arg];
-                if (mode == 0) wts[(size_t)t * top + k] = 1.0f / (1.0f + expf(-z[arg]));
-                z[arg] = -INFINITY;
-            }
+            if (arg >= n_experts) arg = 0;
+            value = mode == 2 ? sc[arg] : z[arg];
+            __threadfence_block();
+            if (lane == 0) z[arg] = -INFINITY;
+            __threadfence_block();
         }
-        __syncthreads();
+        if (lane == 0) {
+            ids[(size_t)t * top + k] = arg;
+            zc[k] = value;
+            if (mode == 0) wts[(size_t)t * top + k] = 1.0f / (1.0f + expf(-value));
+        }
     }
-    if (mode == 2 && wave == 0) {                    // the chosen scores, made to add up to one
+    __threadfence_block();
+    if (mode == 2) {                                 // the chosen scores, made to add up to one
         float part = 0.f;
         for (int k = lane; k < top; k += WAVE) part += zc[k];
-        const float sum = renorm ? wave_sum(part) + 1e-20f : 1.f;
+        const float sum = renorm ? wave_sum_in_place(part) + 1e-20f : 1.f;
         for (int k = lane; k < top; k += WAVE) wts[(size_t)t * top + k] = zc[k] / sum * scale;
     }
-    if (mode == 1 && wave == 0) {                    // the softmax over the chosen logits (the first is the largest)
+    if (mode == 1) {                                 // the softmax over the chosen logits (the first is the largest)
         const float z0 = zc[0];
         float part = 0.f;
         for (int k = lane; k < top; k += WAVE) part += expf(zc[k] - z0);
-        const float sum = wave_sum(part);
+        const float sum = wave_sum_in_place(part);
         for (int k = lane; k < top; k += WAVE) wts[(size_t)t * top + k] = expf(zc[k] - z0) / sum;
     }
 }
@@ -301,13 +333,17 @@ __device__ __forceinline__ int quarter_steps(int steps) { return (steps + 7) / 8
 // What bounds it is the experts' matrices out of memory, once.  One wave for 16 features and all of K left 3 to 4 waves a compute
 // unit, which waited for eight loads and then issued the next eight: 2.8 (gated first product) and 3.2 TB/s (second) for 14 of 16
 // experts of 2 x 1024 x 2048 and 2048 x 1024, 42 and 18 us; now 24 and 14 us, and 16 experts of 2 x 1408 x 2048 52 -> 34.5 us, 5.3 TB/s.
+// A shared expert that every token uses rides along as one more expert (sw: its matrix, packed alike, of s_n rows and s_k columns; only
+// while the tokens are few, as each 16 of them read it once): beside the others it costs its bytes, in kernels of its own it took
+// 11 and 5 us.
 // (Eight steps on their way and half as many waves: 25 and 37.5.)  The list costs a scan of n * top numbers, but no kernel in front.
 constexpr int MOE_LIST = 2048;
 template <class T, int MODE, bool PACKED>
 __global__ void __launch_bounds__(256, 4)
 moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__ w, size_t w_expert_stride, int N, int K,
                     const int *__restrict__ ids, int total, const float *__restrict__ wts, T *__restrict__ out_t,
-                    float *__restrict__ out_f, int out_stride, int top, int add, float alpha, float limit) {
+                    float *__restrict__ out_f, int out_stride, int top, int add, float alpha, float limit, int experts,
+                    const T *__restrict__ sx, const T *__restrict__ sw, int s_n, int s_k, T *__restrict__ s_out_t, float *__restrict__ s_out_f) {
     typedef Mma<T> M;
     typedef typename M::frag frag;
     constexpr bool GATED = MODE == MOE_UP_GATED, UP = MODE != MOE_DOWN;
@@ -315,15 +351,32 @@ moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__
     __shared__ int list[MOE_LIST], found;
     __shared__ f32x4 red[4][2][WAVE];
     const int e = blockIdx.y, tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, g = lane / 16, l16 = lane % 16;
+    const bool shared = e == experts;
+    const T *we = w + (size_t)e * w_expert_stride;
+    if (shared) {                                    // every token's rows [n, s_k] and a matrix of its own size
+        total /= top;
+        top = 1;
+        x = sx;
+        we = sw;
+        N = s_n;
+        K = s_k;
+        x_stride = GATED ? x_stride : s_k;
+        out_t = s_out_t;
+        out_f = s_out_f;
+        out_stride = GATED ? s_n / 2 : out_stride;
+        alpha = 1.f;
+        limit = 0.f;
+    }
+    if ((int)blockIdx.x * 32 >= N) return;
     const int tile0 = 2 * blockIdx.x, steps = (K + M::KSTEP - 1) / M::KSTEP, per = quarter_steps(steps);
     const int s0 = wave * per, s1 = min(steps, s0 + per);
-    const Unit<T, PACKED> w0(w + (size_t)e * w_expert_stride, tile0, N, K, steps, lane), w1(w + (size_t)e * w_expert_stride, tile0 + 1, N, K, steps, lane);
+    const Unit<T, PACKED> w0(we, tile0, N, K, steps, lane), w1(we, tile0 + 1, N, K, steps, lane);
     for (int first = 0; first < total; first += MOE_LIST) {
         __syncthreads();                             // the list of before has been read
         if (tid == 0) found = 0;
         __syncthreads();
         for (int p = first + tid; p < min(total, first + MOE_LIST); p += 256)
-            if (ids[p] == e) list[atomicAdd(&found, 1)] = p;
+            if (shared || ids[p] == e) list[atomicAdd(&found, 1)] = p;
         __syncthreads();
         const int count = found;
         for (int r0 = 0; r0 < count; r0 += 16) {
@@ -530,24 +583,32 @@ moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict_
     }
 }
 
-// out[t, c] (+)= sum_k wts[t, k] * y[t * top + k, c]  (in the order of k; wts null: ones)  + gate[t] * shared[t, c]  (shared null: nothing)
+// out[t, c] (+)= sum_k wts[t, k] * y[t * top + k, c]  (in the order of k; wts null: ones)  + gate[t] * shared[t, c]  (shared null: nothing;
+// shared32: the same rows in 32 bits)
 // fresh: out is written, not added to (what it held is not read).  ids (null: none), real, h: a pair whose expert is
-// `real` or beyond is an identity expert, whose output is the token's input row h[t] itself.
+// `real` or beyond is an identity expert, whose output is the token's input row h[t] itself.  Four columns a thread; d is a multiple of 4.
 template <class T>
-__global__ void moe_combine_kernel(float *__restrict__ out, const float *__restrict__ y, const float *__restrict__ wts,
-                                   const T *__restrict__ shared, const float *__restrict__ gate, int n, int d, int top, int fresh,
-                                   const int *__restrict__ ids, int real, const T *__restrict__ h) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256)
+moe_combine_kernel(float *__restrict__ out, const float *__restrict__ y, const float *__restrict__ wts,
+                   const T *__restrict__ shared, const float *__restrict__ shared32, const float *__restrict__ gate, int n, int d, int top,
+                   int fresh, const int *__restrict__ ids, int real, const T *__restrict__ h) {
+    const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (c >= d) return;
+    auto four = [](const T *p) {
+        const Quad<T> q = *(const Quad<T> *)p;
+        return f32x4{to_f32(q.v[0]), to_f32(q.v[1]), to_f32(q.v[2]), to_f32(q.v[3])};
+    };
     for (size_t t = blockIdx.y; t < (size_t)n; t += gridDim.y) {
-        float acc = fresh ? 0.f : out[t * d + c];
+        f32x4 acc = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *(const f32x4 *)(out + t * d + c);
         for (int k = 0; k < top; ++k) {
             const float w = wts ? wts[t * top + k] : 1.f;
-            if (ids && ids[t * top + k] >= real) acc += w * to_f32(h[t * d + c]);
-            else acc += w * y[(t * top + k) * d + c];
+            if (ids && ids[t * top + k] >= real) acc += w * four(h + t * d + c);
+            else acc += w * *(const f32x4 *)(y + (t * top + k) * d + c);
         }
-        if (shared) acc += (gate ? gate[t] : 1.f) * to_f32(shared[t * d + c]);
-        out[t * d + c] = acc;
+        const float g = gate ? gate[t] : 1.f;
+        if (shared) acc += g * four(shared + t * d + c);
+        if (shared32) acc += g * *(const f32x4 *)(shared32 + t * d + c);
+        *(f32x4 *)(out + t * d + c) = acc;
     }
 }
 
@@ -584,11 +645,13 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
 // them (ff a multiple of 16); act = silu(gate h) * (up h), and the weight scales what comes out; fresh: out is written
 // and not added to; limit > 0: the limited activation (gate_act.h) with alpha and limit instead of silu.  identity: ids may name experts + identity experts; the last `identity` have no matrices and return the
 // token's input.  shared (null or
-// [n, d] of `type`) with shared_gate (null or [n] 32-bit): rows that are added beside the experts', times the gate.
+// [n, d] of `type`) with shared_gate (null or [n] 32-bit): rows that are added beside the experts', times the gate.  shared_up,
+// shared_down (null, or the matrices [2 * shared_ff, d] and [d, shared_ff] of a shared expert that is computed here, with silu, in the order of Unit
+// like w_up and w_down; only where lcu_moe_tile_rows says 0): act then holds n * shared_ff elements more and y n rows more.
 LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float *wts, int *ints, int max_tiles,
                             const void *w_up, int packed_up, const void *w_down, int packed_down, void *act, float *y, float *out, int n, int d, int ff,
-                            int experts, int top, int gated, const void *shared, const float *shared_gate, int fresh,
-                            int identity, float alpha, float limit, hipStream_t stream) {
+                            int experts, int top, int gated, const void *shared, const float *shared_gate, const void *shared_up,
+                            const void *shared_down, int shared_ff, int fresh, int identity, float alpha, float limit, hipStream_t stream) {
     if (n <= 0) return LCU_OK;
     const int per = type == LCU_BF16 ? 8 : 4;
     if (d <= 0 || ff <= 0 || d % per || ff % per || experts <= 0 || experts > MOE_MAX_EXPERTS || top <= 0 ||
@@ -597,6 +660,7 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
         return LCU_BAD_ARGUMENT;
     const int total = n * top;
     const bool few = lcu_moe_tile_rows(total, experts) == 0;
+    if (shared_up && (!shared_down || shared || !gated || !few || !packed_up || !packed_down || shared_ff <= 0 || shared_ff % 16)) return LCU_BAD_ARGUMENT;
     const int add = top == 1 && !gated;
     float *down_to = add ? out : y;
     if (!add && !y) return LCU_BAD_ARGUMENT;
@@ -610,11 +674,16 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
     LCU_LAUNCH_CHECK()
     if (few) {
         if (!ids) return LCU_BAD_ARGUMENT;
-        const dim3 block(256), gu((up_rows + 31) / 32, experts), gd((d + 31) / 32, experts);
+        // one more expert, the shared one: its activations lie behind the pairs' (act [total, ff], then [n, shared_ff]), its outputs too
+        const int with = experts + (shared_up ? 1 : 0), s_rows = 2 * shared_ff, wider = shared_up && s_rows > up_rows ? s_rows : up_rows;
+        const size_t act_end = (size_t)total * ff;
+        const dim3 block(256), gu((wider + 31) / 32, with), gd((d + 31) / 32, with);
 #define UP(T, PACKED, MODE) moe_gemm_few_kernel<T, MODE, PACKED><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \
-                                                ids, total, wts, (T *)act, nullptr, ff, top, 0, alpha, limit)
+                                                ids, total, wts, (T *)act, nullptr, ff, top, 0, alpha, limit, experts, \
+                                                (const T *)h, (const T *)shared_up, s_rows, d, (T *)act + act_end, nullptr)
 #define DOWN(T, PACKED, MODE) moe_gemm_few_kernel<T, MODE, PACKED><<<gd, block, 0, stream>>>((const T *)act, ff, (const T *)w_down, down_stride, d, ff, \
-                                                ids, total, wts, nullptr, down_to, d, top, add, 0.f, 0.f)
+                                                ids, total, wts, nullptr, down_to, d, top, add, 0.f, 0.f, experts, \
+                                                (const T *)act + act_end, (const T *)shared_down, d, shared_ff, nullptr, y + (size_t)total * d)
         int packed = packed_up;
         if (gated) { TYPED(UP, MOE_UP_GATED); } else { TYPED(UP, MOE_UP); }
         packed = packed_down;
@@ -641,10 +710,13 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
     }
 #undef TYPED
     if (!add) {
-        const dim3 gc((d + 255) / 256, n < 65535 ? n : 65535);
+        const dim3 gc((d + 1023) / 1024, n < 65535 ? n : 65535);
         const int *idp = identity ? ids : nullptr;
-        if (type == LCU_BF16) moe_combine_kernel<bf16_t><<<gc, dim3(256), 0, stream>>>(out, y, gated ? wts : nullptr, (const bf16_t *)shared, shared_gate, n, d, top, fresh, idp, experts, (const bf16_t *)h);
-        else moe_combine_kernel<float><<<gc, dim3(256), 0, stream>>>(out, y, gated ? wts : nullptr, (const float *)shared, shared_gate, n, d, top, fresh, idp, experts, (const float *)h);
+        const float *shared32 = shared_up ? y + (size_t)total * d : nullptr;
+#define COMBINE(T) moe_combine_kernel<T><<<gc, dim3(256), 0, stream>>>(out, y, gated ? wts : nullptr, (const T *)shared, shared32, shared_gate, n, d, top, fresh, idp, experts, (const T *)h)
+        if (type == LCU_BF16) COMBINE(bf16_t);
+        else COMBINE(float);
+#undef COMBINE
         LCU_LAUNCH_CHECK();
     }
     return LCU_OK;

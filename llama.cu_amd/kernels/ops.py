@@ -1373,7 +1373,7 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, top: int, bias: Optional[to
 def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
                 out: torch.Tensor, gated: bool = False, shared: Optional[torch.Tensor] = None,
                 shared_gate: Optional[torch.Tensor] = None, fresh: bool = False, identity: int = 0,
-                act_alpha: float = 1.0, act_limit: float = 0.0) -> torch.Tensor:
+                act_alpha: float = 1.0, act_limit: float = 0.0, shared_expert: Optional[tuple] = None) -> torch.Tensor:
     """``out[t] += sum over t's experts e of  w_down[e] @ gelu(w_up[e] @ (weight * h[t]))`` (the exact gelu; the
     weight scales what goes INTO the expert, not what comes out).  ``w_up [experts, ff, d]``, ``w_down [experts, d, ff]`` in ``h``'s type,
     ``out`` float32 ``[n, d]``.  ``gated``: ``out[t] += sum_e weight * w_down[e] @ (silu(gate[e] @ h[t]) * (up[e] @ h[t]))``
@@ -1381,7 +1381,9 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
     (``gated_rows`` lays them out so); either matrix may be given as ``pack_experts`` makes it; ``shared [n, d]`` (with ``shared_gate [n]`` float32, or ones) is added beside;
     ``fresh``: ``out`` is written, not added to (it need not hold anything).  ``identity``: ``ids`` may name ``experts +
     identity`` experts, of which the last ``identity`` have no matrices: their output is ``weight * h[t]`` (gated form only).
-    ``act_limit`` > 0: the limited activation (``swiglu``) with ``act_alpha`` instead of silu."""
+    ``act_limit`` > 0: the limited activation (``swiglu``) with ``act_alpha`` instead of silu.  ``shared_expert``: in the place of
+    ``shared`` the matrices (``[1, 2 * sff, d]`` as ``gated_rows`` lays them out and ``[1, d, sff]``, both packed) of an expert with
+    silu that every token uses, computed beside the others; where ``moe_shared_beside`` says so."""
     up, down = (w.data if isinstance(w, PackedExperts) else w for w in (w_up, w_down))
     _gpu(h, ids, wts, up, down, out, shared, shared_gate)
     _rows(h, "moe input")
@@ -1413,18 +1415,41 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
             raise KernelError("moe_experts: shared rows go with gated experts and must be [n, d] of the input's type")
         if shared_gate is not None and (shared_gate.dtype != torch.float32 or shared_gate.numel() != n or not shared_gate.is_contiguous()):
             raise KernelError("moe_experts: the shared rows' gate must be contiguous float32 [n]")
+    shared_up = shared_down = None
+    sff = 0
+    if shared_expert is not None:
+        shared_up, shared_down = shared_expert
+        sff = shared_down.shape[2]
+        if not gated or shared is not None or not moe_shared_beside(n, top, experts, w_up, w_down) or sff % 16 \
+                or not isinstance(shared_up, PackedExperts) or not isinstance(shared_down, PackedExperts) \
+                or shared_up.shape != (1, 2 * sff, d) or shared_down.shape != (1, d, sff) or shared_up.dtype != h.dtype or shared_down.dtype != h.dtype:
+            raise KernelError("moe_experts: the shared expert's matrices do not fit, or the step has too many tokens for it")
+        if shared_gate is not None and (shared_gate.dtype != torch.float32 or shared_gate.numel() != n or not shared_gate.is_contiguous()):
+            raise KernelError("moe_experts: the shared rows' gate must be contiguous float32 [n]")
+        _gpu(h, shared_up.data, shared_down.data, shared_gate)
+        _contig(shared_up.data, "shared up"); _contig(shared_down.data, "shared down")
     lib = build.load("moe")
     total = n * top
     tile = lib.lcu_moe_tile_rows(total, experts)
     max_tiles = min(total, total // tile + experts) if tile else 0
     ints = torch.empty(total + 3 * max_tiles + 1, dtype=torch.int32, device=h.device) if tile else None
-    act = torch.empty((total, ff), dtype=h.dtype, device=h.device)
-    y = torch.empty((total, d), dtype=torch.float32, device=h.device) if (top > 1 or gated) else None
+    act = torch.empty(total * ff + n * sff, dtype=h.dtype, device=h.device)
+    y = torch.empty((total + (n if sff else 0), d), dtype=torch.float32, device=h.device) if (top > 1 or gated) else None
     _check(lib.lcu_moe_experts(_ptr(h), _type(h, "moe input"), _ptr(ids), _ptr(wts), _ptr(ints), max_tiles, _ptr(up),
                                int(up is not w_up), _ptr(down), int(down is not w_down), _ptr(act), _ptr(y), _ptr(out), n, d, ff, experts, top, int(bool(gated)),
-                               _ptr(shared), _ptr(shared_gate if shared is not None else None), int(bool(fresh)), identity, ctypes.c_float(act_alpha),
+                               _ptr(shared), _ptr(shared_gate if shared is not None or sff else None), _ptr(shared_up.data if sff else None),
+                               _ptr(shared_down.data if sff else None), sff, int(bool(fresh)), identity, ctypes.c_float(act_alpha),
                                ctypes.c_float(act_limit), _stream()), "moe_experts")
     return out
+
+
+MOE_SHARED_ROWS = 32        # tokens up to which a shared expert is computed beside the others (each 16 read its matrices once)
+
+
+def moe_shared_beside(n: int, top: int, experts: int, w_up, w_down) -> bool:
+    """Whether ``moe_experts`` computes a shared expert beside the others for ``n`` tokens."""
+    return n <= MOE_SHARED_ROWS and isinstance(w_up, PackedExperts) and isinstance(w_down, PackedExperts) \
+        and build.load("moe").lcu_moe_tile_rows(n * top, experts) == 0
 
 
 @dataclass(frozen=True)

@@ -195,8 +195,13 @@ class GatedMoE(Part):
         self.w_gate_up = ops.gated_rows(gate.contiguous(), up.contiguous())
         if build.pack_weights:
             self.w_gate_up, self.w_down = ops.pack_experts(self.w_gate_up), ops.pack_experts(self.w_down)
+        self.shared_expert = None
         if self.shared is not None:
             self.shared.load(tensors, build)
+            sg, su, sd = (tensors[nm[k]] for k in ("shared_gate", "shared_up", "shared_down"))
+            if build.pack_weights and sg.shape[0] % 16 == 0 and sg.dtype == su.dtype == sd.dtype == self.w_down.dtype:
+                # steps of few tokens compute it beside the experts, from a copy in their order
+                self.shared_expert = (ops.pack_experts(ops.gated_rows(sg[None].contiguous(), su[None].contiguous())), ops.pack_experts(sd[None].contiguous()))
         self.dtype = build.dtype
 
     def forward(self, h, add_to: Optional[torch.Tensor] = None):
@@ -214,8 +219,9 @@ class GatedMoE(Part):
         fresh = add_to is None
         out = add_to if not fresh else torch.empty((h.shape[0], h.shape[1]), dtype=torch.float32, device=h.device)
         if self.shared is not None:
-            ops.moe_experts(h, ids, wts, self.w_gate_up, self.w_down, out, gated=True, shared=self.shared.forward(h),
-                            shared_gate=routed[2] if self.gates else None, fresh=fresh, identity=self.identity, **self.act)
+            beside = self.shared_expert is not None and ops.moe_shared_beside(h.shape[0], ids.shape[1], self.experts, self.w_gate_up, self.w_down)
+            ops.moe_experts(h, ids, wts, self.w_gate_up, self.w_down, out, gated=True, shared=None if beside else self.shared.forward(h),
+                            shared_expert=self.shared_expert if beside else None, shared_gate=routed[2] if self.gates else None, fresh=fresh, identity=self.identity, **self.act)
         else:
             ops.moe_experts(h, ids, wts, self.w_gate_up, self.w_down, out, gated=True, fresh=fresh, identity=self.identity, **self.act)
         return out

@@ -62,3 +62,33 @@ def test_packed_gated_experts(dtype, n, ff):
             v = torch.clamp(up[e].cpu().to(F64) @ x[t], -2.0, 2.0)
             want[t] += w * (down[e].cpu().to(F64) @ (g * torch.sigmoid(1.702 * g) * (v + 1.0)))
     assert_close(outs[0], want, 1e-4 if dtype == "float32" else 3e-2, "output")
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("n,ff,sff,gate", [(1, 16, 48, True), (17, 112, 16, False), (32, 32, 208, True)])
+def test_a_shared_expert_beside_the_others(dtype, n, ff, sff, gate):
+    """The shared expert smaller and larger than the others, at one and two tiles of rows, against the sum in 64 bits."""
+    from llama_cu_amd.kernels import ops
+    experts, top, d, tdt = 5, 2, 88, TYPES[dtype]
+    pack = ops.pack_experts
+    h, router = rnd(n, d, seed=1).to(tdt).cuda(), rnd(experts + 1, d, seed=2).cuda()
+    gates, ups = (rnd(experts, ff, d, seed=k, std=d ** -0.5).to(tdt).cuda() for k in (3, 4))
+    down = rnd(experts, d, ff, seed=5, std=ff ** -0.5).to(tdt).cuda()
+    sg, su = (rnd(1, sff, d, seed=k, std=d ** -0.5).to(tdt).cuda() for k in (6, 7))
+    sd = rnd(1, d, sff, seed=8, std=sff ** -0.5).to(tdt).cuda()
+    up_p, down_p = pack(ops.gated_rows(gates, ups)), pack(down)
+    assert ops.moe_shared_beside(n, top, experts, up_p, down_p) == (n * top <= 16 * experts)
+    ids, wts, g = ops.moe_route(h, router, top, softmax_chosen=True, extra=1)
+    out = torch.full((n, d), 3.0, device="cuda")
+    ops.moe_experts(h, ids, wts, up_p, down_p, out, gated=True, shared_expert=(pack(ops.gated_rows(sg, su)), pack(sd)),
+                    shared_gate=g if gate else None, act_alpha=1.702, act_limit=2.0)
+    x, want = h.cpu().to(F64), torch.full((n, d), 3.0, dtype=F64)
+    f = lambda t: t.cpu().to(F64)
+    z = f(sg[0]) @ x.T
+    shared = (f(sd[0]) @ (z * torch.sigmoid(z) * (f(su[0]) @ x.T))).T
+    want += shared * (torch.sigmoid(x @ f(router[experts]))[:, None] if gate else 1.0)
+    for t in range(n):
+        for e, w in zip(ids[t].tolist(), f(wts[t])):
+            a, b = torch.clamp(f(gates[e]) @ x[t], max=2.0), torch.clamp(f(ups[e]) @ x[t], -2.0, 2.0)
+            want[t] += w * (f(down[e]) @ (a * torch.sigmoid(1.702 * a) * (b + 1.0)))
+    assert_close(out, want, 1e-4 if dtype == "float32" else 3e-2, "output")
