@@ -10,6 +10,7 @@
 // where rows before the request's first row of this step come from the request's state (the
 // last T - 1 rows of earlier steps) and rows before position 0 are zeros.
 #include "common.h"
+#include "lane_moves.h"
 
 constexpr int NC_THREADS = 256;
 constexpr int MAX_TAPS = 16;
@@ -47,47 +48,113 @@ layernorm_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes
     }
 }
 
-// The same for rows of up to NC_THREADS * PT elements: the row stays in registers between its one read and
-// its writes (a step of few rows is a chain of dependent trips to memory, and this kernel has one, not three).
-template <class TD, class TO, int PT>
-__global__ void __launch_bounds__(NC_THREADS)
+// V neighbouring elements as one access.
+template <class T, int V> struct alignas(V * sizeof(T)) Pack { T v[V]; };
+template <class T, int V> __device__ __forceinline__ void load_as_f32(const T *p, float *out) {
+    const Pack<T, V> in = *(const Pack<T, V> *)p;
+#pragma unroll
+    for (int e = 0; e < V; ++e) out[e] = to_f32(in.v[e]);
+}
+template <class T, int V> __device__ __forceinline__ void store_f32(T *p, const float *in) {
+    Pack<T, V> out;
+#pragma unroll
+    for (int e = 0; e < V; ++e) out.v[e] = from_f32<T>(in[e]);
+    *(Pack<T, V> *)p = out;
+}
+
+// The sum over a workgroup of up to 16 waves; `scratch` (16 floats) is not in use by an earlier call.
+__device__ __forceinline__ float row_sum(float v, float *scratch) {
+    v = wave_sum_in_place(v);
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+    __syncthreads();
+    float t = 0.f;
+    for (int i = 0; i < (int)blockDim.x / WAVE; ++i) t += scratch[i];
+    return t;
+}
+
+// A row's elements in one thread's registers: PT pieces of V neighbours, ROW_THREADS pieces apart.  The row takes in the planes
+// of delta, is written back, and its mean and the inverse of its deviation come out.  A step of few rows is a chain of dependent
+// trips to memory and through the barriers: one trip, two barriers.
+constexpr int ROW_THREADS = 512;
+template <class TD, int V, int PT>
+__device__ __forceinline__ void take_row(float *xr, const TD *delta, int planes, size_t plane_stride, size_t row_at, int d, float eps,
+                                         float (&v)[PT][V], float &mean, float &rstd, float (*scratch)[16]) {
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+        const int c = (threadIdx.x + ROW_THREADS * i) * V;
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[i][e] = 0.f;
+        if (c < d) {
+            load_as_f32<float, V>(xr + c, v[i]);
+            if (delta) {
+                for (int p = 0; p < planes; ++p) {
+                    float more[V];
+                    load_as_f32<TD, V>(delta + p * plane_stride + row_at + c, more);
+#pragma unroll
+                    for (int e = 0; e < V; ++e) v[i][e] += more[e];
+                }
+                store_f32<float, V>(xr + c, v[i]);
+            }
+#pragma unroll
+            for (int e = 0; e < V; ++e) sum += v[i][e];
+        }
+    }
+    mean = row_sum(sum, scratch[0]) / (float)d;
+    float sq = 0.f;
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            const float dev = v[i][e] - mean;
+            if ((threadIdx.x + ROW_THREADS * i) * V < d) sq += dev * dev;
+        }
+    rstd = rsqrtf(row_sum(sq, scratch[1]) / (float)d + eps);
+}
+
+// The same for rows of up to ROW_THREADS * V * PT elements: the row stays in registers between its one read and its writes.  V is 4
+// where d is a multiple of 4 and every pointer is aligned for it (2,048 rows of 2,048 with two 32-bit outputs 21.8 -> 14.2 us, one
+// row 5.5 -> 2.3), else 1.
+template <class TD, class TO, int V, int PT>
+__global__ void __launch_bounds__(ROW_THREADS)
 layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes, size_t plane_stride,
                      const float *__restrict__ w1, const float *__restrict__ b1, TO *__restrict__ out1,
                      const float *__restrict__ w2, const float *__restrict__ b2, TO *__restrict__ out2, int d, float eps) {
-    __shared__ float scratch[16];
-    float *xr = x + (size_t)blockIdx.x * d;
-    float v[PT], sum = 0.f;
+    __shared__ float scratch[2][16];
+    const size_t row_at = (size_t)blockIdx.x * d;
+    float v[PT][V], w[2][PT][V], b[2][PT][V], mean, rstd;
+    // (the weights are on their way while the sums are made)
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-        const int c = threadIdx.x + NC_THREADS * i;
-        v[i] = 0.f;
+        const int c = (threadIdx.x + ROW_THREADS * i) * V;
         if (c < d) {
-            v[i] = xr[c];
-            if (delta) {
-                for (int p = 0; p < planes; ++p) v[i] += to_f32(delta[p * plane_stride + (size_t)blockIdx.x * d + c]);
-                xr[c] = v[i];
+            load_as_f32<float, V>(w1 + c, w[0][i]);
+            load_as_f32<float, V>(b1 + c, b[0][i]);
+            if (w2) {
+                load_as_f32<float, V>(w2 + c, w[1][i]);
+                load_as_f32<float, V>(b2 + c, b[1][i]);
             }
-            sum += v[i];
         }
     }
-    const float mean = block_sum(sum, scratch) / (float)d;
-    float sq = 0.f;
+    take_row<TD, V, PT>(x + row_at, delta, planes, plane_stride, row_at, d, eps, v, mean, rstd, scratch);
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-        const float dev = v[i] - mean;
-        if (threadIdx.x + NC_THREADS * i < d) sq += dev * dev;
-    }
-    const float rstd = rsqrtf(block_sum(sq, scratch) / (float)d + eps);
+        const int c = (threadIdx.x + ROW_THREADS * i) * V;
+        if (c >= d) continue;
+        float y[V];
 #pragma unroll
-    for (int i = 0; i < PT; ++i) {
-        const int c = threadIdx.x + NC_THREADS * i;
-        if (c < d) {
-            const float z = (v[i] - mean) * rstd;
-            out1[(size_t)blockIdx.x * d + c] = from_f32<TO>(z * w1[c] + b1[c]);
-            if (w2) out2[(size_t)blockIdx.x * d + c] = from_f32<TO>(z * w2[c] + b2[c]);
+        for (int e = 0; e < V; ++e) y[e] = (v[i][e] - mean) * rstd * w[0][i][e] + b[0][i][e];
+        store_f32<TO, V>(out1 + row_at + c, y);
+        if (w2) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) y[e] = (v[i][e] - mean) * rstd * w[1][i][e] + b[1][i][e];
+            store_f32<TO, V>(out2 + row_at + c, y);
         }
     }
 }
+
+// Whether four elements at a time may be read and written at p (null: nothing is).
+static bool four_ok(const void *p, int type) { return ((uintptr_t)p & (type == LCU_BF16 ? 7 : 15)) == 0; }
 
 // delta_type: -1 none, LCU_F32 or LCU_BF16.  out_type: LCU_F32 or LCU_BF16.
 LCU_API int lcu_layernorm(float *x, const void *delta, int delta_type, int planes, const float *w1, const float *b1,
@@ -97,15 +164,19 @@ LCU_API int lcu_layernorm(float *x, const void *delta, int delta_type, int plane
     if (d <= 0 || !w1 || !b1 || !out1 || (w2 && (!b2 || !out2)) || (delta && planes <= 0)) return LCU_BAD_ARGUMENT;
     const size_t stride = (size_t)n * d;
     dim3 grid(n), block(NC_THREADS);
-#define ROW(TD, TO, PT) layernorm_row_kernel<TD, TO, PT><<<grid, block, 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
+    const int dt = delta ? delta_type : LCU_F32;
+    const bool four = d % 4 == 0 && four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) && four_ok(out1, out_type) &&
+                      four_ok(w2, LCU_F32) && four_ok(b2, LCU_F32) && four_ok(out2, out_type);
+#define ROW(TD, TO, V, PT) layernorm_row_kernel<TD, TO, V, PT><<<grid, dim3(ROW_THREADS), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
 #define GO(TD, TO)                                                                                                           \
     do {                                                                                                                     \
-        if (d <= 4 * NC_THREADS) ROW(TD, TO, 4);                                                                             \
-        else if (d <= 16 * NC_THREADS) ROW(TD, TO, 16);                                                                      \
+        if (four && d <= 4 * ROW_THREADS) ROW(TD, TO, 4, 1);                                                                 \
+        else if (four && d <= 8 * ROW_THREADS) ROW(TD, TO, 4, 2);                                                            \
+        else if (d <= 2 * ROW_THREADS) ROW(TD, TO, 1, 2);                                                                    \
+        else if (d <= 8 * ROW_THREADS) ROW(TD, TO, 1, 8);                                                                    \
         else layernorm_kernel<TD, TO><<<grid, block, 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1,  \
                                                                   w2, b2, (TO *)out2, d, eps);                               \
     } while (0)
-    const int dt = delta ? delta_type : LCU_F32;
     if (dt == LCU_F32 && out_type == LCU_F32) GO(float, float);
     else if (dt == LCU_F32 && out_type == LCU_BF16) GO(float, bf16_t);
     else if (dt == LCU_BF16 && out_type == LCU_F32) GO(bf16_t, float);
@@ -218,76 +289,70 @@ LCU_API int lcu_short_conv(const void *h, int h_type, long long set_stride_h, co
 // convolutions from the requests' states, and the states' update, with the row in registers throughout.  A block
 // is the only reader and writer of its request's state, and a thread of its channels'.
 // out: [sets][n, d] of TO; state: [slots, sets, taps - 1, d]; cw: [sets][d, taps] 32-bit.
-template <class TD, class TO, int PT>
-__global__ void __launch_bounds__(NC_THREADS)
+// Everything that is read is read before the row's sums are made: one trip to memory.  V as above, and 4 for four taps only (element
+// e's taps are then the numbers 4 e .. of a thread's sixteen); up to FUSED_TAPS taps.  With 256 threads, single numbers and the two sets
+// one after the other four rows of 2,048 with four taps took 13.8 us, now 5.0.
+constexpr int FUSED_TAPS = 8;
+template <class TD, class TO, int V, int PT>
+__global__ void __launch_bounds__(ROW_THREADS)
 norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes, size_t plane_stride,
                         const float *__restrict__ w1, const float *__restrict__ b1, const float *__restrict__ w2,
                         const float *__restrict__ b2, const float *__restrict__ cw, float *__restrict__ st,
                         TO *__restrict__ out, size_t set_stride_out, const int *__restrict__ ctx_len,
-                        const int *__restrict__ state_slot, int d, int taps, int sets, float eps) {
-    __shared__ float scratch[16];
+                        const int *__restrict__ state_slot, int d, int taps_rt, int sets, float eps) {
+    __shared__ float scratch[2][16];
+    const int taps = V == 4 ? 4 : taps_rt;
     const int r = blockIdx.x;
     const int pos = ctx_len[r] - 1;                  // the token's position
-    float *xr = x + (size_t)r * d;
-    float v[PT], sum = 0.f;
+    float *slot = st + (size_t)state_slot[r] * sets * (taps - 1) * d;
+    float v[PT][V], mean, rstd;
+    float old[2][PT][FUSED_TAPS - 1][V], k[2][PT][V * FUSED_TAPS], wv[2][PT][V], bv[2][PT][V];
 #pragma unroll
-    for (int i = 0; i < PT; ++i) {
-        const int c = threadIdx.x + NC_THREADS * i;
-        v[i] = 0.f;
-        if (c < d) {
-            v[i] = xr[c];
-            if (delta) {
-                for (int p = 0; p < planes; ++p) v[i] += to_f32(delta[p * plane_stride + (size_t)r * d + c]);
-                xr[c] = v[i];
+    for (int s = 0; s < 2; ++s) {
+        if (s >= sets) break;
+        const float *w = s ? w2 : w1, *b = s ? b2 : b1, *state = slot + (size_t)s * (taps - 1) * d;
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+            const int c = (threadIdx.x + ROW_THREADS * i) * V;
+            if (c >= d) continue;
+            load_as_f32<float, V>(w + c, wv[s][i]);
+            load_as_f32<float, V>(b + c, bv[s][i]);
+            const float *kc = cw + ((size_t)s * d + c) * taps;             // V * taps numbers: taps pieces of V
+#pragma unroll
+            for (int j = 0; j < FUSED_TAPS; ++j)
+                if (j < taps) load_as_f32<float, V>(kc + j * V, k[s][i] + j * V);
+#pragma unroll
+            for (int j = 0; j < FUSED_TAPS - 1; ++j) {                     // row j of the state lies taps - 1 - j positions before the token
+#pragma unroll
+                for (int e = 0; e < V; ++e) old[s][i][j][e] = 0.f;
+                if (j < taps - 1 && pos - (taps - 1 - j) >= 0) load_as_f32<float, V>(state + (size_t)j * d + c, old[s][i][j]);
             }
-            sum += v[i];
         }
     }
-    const float mean = block_sum(sum, scratch) / (float)d;
-    float sq = 0.f;
+    take_row<TD, V, PT>(x + (size_t)r * d, delta, planes, plane_stride, (size_t)r * d, d, eps, v, mean, rstd, scratch);
 #pragma unroll
-    for (int i = 0; i < PT; ++i) {
-        const float dev = v[i] - mean;
-        if (threadIdx.x + NC_THREADS * i < d) sq += dev * dev;
-    }
-    const float rstd = rsqrtf(block_sum(sq, scratch) / (float)d + eps);
-    constexpr int FUSED_TAPS = 8;                    // the most taps this kernel takes
-    for (int s = 0; s < sets; ++s) {
-        const float *w = s ? w2 : w1, *b = s ? b2 : b1;
-        float *state = st + ((size_t)state_slot[r] * sets + s) * (taps - 1) * d;
-        // everything is read before anything is written: the state's new rows are its old ones, and loads that had to
-        // wait for the stores before them would be a chain of trips to memory
-        float old[PT][FUSED_TAPS - 1], k[PT][FUSED_TAPS], wv[PT], bv[PT];
+    for (int s = 0; s < 2; ++s) {
+        if (s >= sets) break;
+        float *state = slot + (size_t)s * (taps - 1) * d;
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
-            const int c = threadIdx.x + NC_THREADS * i;
+            const int c = (threadIdx.x + ROW_THREADS * i) * V;
             if (c >= d) continue;
-            wv[i] = w[c];
-            bv[i] = b[c];
+            float h[V], acc[V];
 #pragma unroll
-            for (int j = 0; j < FUSED_TAPS; ++j)
-                if (j < taps) k[i][j] = cw[((size_t)s * d + c) * taps + j];
+            for (int e = 0; e < V; ++e) acc[e] = h[e] = (v[i][e] - mean) * rstd * wv[s][i][e] + bv[s][i][e];
+            // (the order of short_conv_kernel's additions)
 #pragma unroll
-            for (int j = 0; j < FUSED_TAPS - 1; ++j)      // row j of the state lies taps - 1 - j positions before the token
-                if (j < taps - 1) old[i][j] = pos - (taps - 1 - j) >= 0 ? state[(size_t)j * d + c] : 0.f;
-        }
+            for (int j = 0; j < FUSED_TAPS; ++j) {
+                if (j >= taps) break;
 #pragma unroll
-        for (int i = 0; i < PT; ++i) {
-            const int c = threadIdx.x + NC_THREADS * i;
-            if (c >= d) continue;
-            const float h = (v[i] - mean) * rstd * wv[i] + bv[i];
-            float acc = h;                            // (the order of short_conv_kernel's additions)
-#pragma unroll
-            for (int j = 0; j < FUSED_TAPS - 1; ++j)
-                if (j < taps - 1) {
-                    acc += k[i][j] * old[i][j];
-                    if (j > 0) state[(size_t)(j - 1) * d + c] = old[i][j];     // row j becomes row j - 1
+                for (int e = 0; e < V; ++e) {
+                    acc[e] += k[s][i][V == 4 ? e * 4 + j : j] * (j == taps - 1 ? h[e] : old[s][i][j < FUSED_TAPS - 1 ? j : 0][e]);
                 }
-#pragma unroll
-            for (int j = 0; j < FUSED_TAPS; ++j)
-                if (j == taps - 1) acc += k[i][j] * h;
-            if (taps > 1) state[(size_t)(taps - 2) * d + c] = h;
-            out[s * set_stride_out + (size_t)r * d + c] = from_f32<TO>(acc);
+                if (j > 0 && j < taps - 1) store_f32<float, V>(state + (size_t)(j - 1) * d + c, old[s][i][j < FUSED_TAPS - 1 ? j : 0]);     // row j becomes row j - 1
+            }
+            if (taps > 1) store_f32<float, V>(state + (size_t)(taps - 2) * d + c, h);
+            store_f32<TO, V>(out + s * set_stride_out + (size_t)r * d + c, acc);
         }
     }
 }
@@ -297,18 +362,20 @@ LCU_API int lcu_norm_conv_single(float *x, const void *delta, int delta_type, in
                                  const int *ctx_len, const int *state_slot, int n, int d, int taps, int sets, float eps,
                                  hipStream_t stream) {
     if (n <= 0) return LCU_OK;
-    if (d <= 0 || d > 8 * NC_THREADS || taps < 1 || taps > 8 || sets < 1 || sets > 2 || !w1 || !b1 || (sets == 2 && (!w2 || !b2)) ||
+    if (d <= 0 || d > 4 * ROW_THREADS || taps < 1 || taps > 8 || sets < 1 || sets > 2 || !w1 || !b1 || (sets == 2 && (!w2 || !b2)) ||
         !cw || (taps > 1 && !state) || (delta && planes <= 0))
         return LCU_BAD_ARGUMENT;
     const size_t stride = (size_t)n * d;
-    dim3 grid(n), block(NC_THREADS);
-#define ROW(TD, TO, PT) norm_conv_single_kernel<TD, TO, PT><<<grid, block, 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, w2, b2, cw, state, (TO *)out, stride, ctx_len, state_slot, d, taps, sets, eps)
+    dim3 grid(n);
+    const int dt = delta ? delta_type : LCU_F32;
+    const bool four = d % 4 == 0 && taps == 4 && four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) &&
+                      four_ok(w2, LCU_F32) && four_ok(b2, LCU_F32) && four_ok(cw, LCU_F32) && four_ok(state, LCU_F32) && four_ok(out, out_type);
+#define ROW(TD, TO, V, PT) norm_conv_single_kernel<TD, TO, V, PT><<<grid, dim3(ROW_THREADS), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, w2, b2, cw, state, (TO *)out, stride, ctx_len, state_slot, d, taps, sets, eps)
 #define GO(TD, TO)                                   \
     do {                                             \
-        if (d <= 4 * NC_THREADS) ROW(TD, TO, 4);     \
-        else ROW(TD, TO, 8);                         \
+        if (four) ROW(TD, TO, 4, 1);                 \
+        else ROW(TD, TO, 1, 4);                      \
     } while (0)
-    const int dt = delta ? delta_type : LCU_F32;
     if (dt == LCU_F32 && out_type == LCU_F32) GO(float, float);
     else if (dt == LCU_F32 && out_type == LCU_BF16) GO(float, bf16_t);
     else if (dt == LCU_BF16 && out_type == LCU_F32) GO(bf16_t, float);
