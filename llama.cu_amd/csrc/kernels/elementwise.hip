@@ -3,6 +3,7 @@
 // 32-bit whatever the storage type.
 #include "common.h"
 #include "gate_act.h"
+#include "lane_moves.h"
 
 // ---------------------------------------------------------------- embedding gather
 // out[i, k, :] = table[ids[i], :] * scale for k < copies (the product in 32-bit).  An id outside the table writes NaN into the row
@@ -125,34 +126,35 @@ __global__ void rmsnorm_kernel(TX *__restrict__ x, const TD *__restrict__ delta,
 }
 
 // The same for rows of up to 8192 elements whose width is a multiple of 4: one read of
-// the row (four elements per load), the row kept in registers between the sum and the
-// scaling.  The row is dealt to 1024 virtual threads, two loads each; a block has 1024
+// the row (four elements per load), the row and the weight kept in registers between the sum and the
+// scaling.  The row is dealt to VT virtual threads (512 for rows of up to 2048 elements, else 1024), one or two loads each; a block has VT
 // threads (few rows leave most of the chip idle: what counts then is how many loads a row has
-// in flight) or 256 that play four virtual threads each (many rows: fewer, longer-lived waves
-// stream faster).  The sums are added as the 1024 threads would add them, wave by wave, so
+// in flight) or 256 that play several virtual threads each (many rows: fewer, longer-lived waves
+// stream faster).  The sums are added as the VT threads would add them, wave by wave, so
 // the result does not depend on the block's size, only on d.  The planes are loaded four at
-// a time.
-constexpr int NORM_VTHREADS = 1024, NORM_ITEMS = 2;
-
+// a time.  (With 1024 virtual threads for every width, the weight loaded behind the sum and the sum by shuffles one row of 2,048 took
+// 2.1 us, now 1.8; 16 rows 3.1, now 2.8; 2,048 rows 9.1, now 8.3.)
 template <class T> struct alignas(4 * sizeof(T)) Vec4 { T v[4]; };
 
-template <int THREADS, class TX, class TD, class TW, class TO>
+template <int VT, int ITEMS, int THREADS, class TX, class TD, class TW, class TO>
 __global__ void __launch_bounds__(THREADS)
 rmsnorm_fast_kernel(TX *__restrict__ x, const TD *__restrict__ delta, const TW *__restrict__ w, TO *__restrict__ out,
                     int d, float eps, int write_back, int planes, size_t plane_stride, float delta_scale) {
-    constexpr int PLAY = NORM_VTHREADS / THREADS;           // virtual threads per thread
-    __shared__ float scratch[NORM_VTHREADS / WAVE];
+    constexpr int PLAY = VT / THREADS;           // virtual threads per thread
+    __shared__ float scratch[VT / WAVE];
     TX *xr = x + (size_t)blockIdx.x * d;
     const TD *dr = delta ? delta + (size_t)blockIdx.x * d : nullptr;
-    float v[PLAY][NORM_ITEMS][4];
+    float v[PLAY][ITEMS][4];
+    Vec4<TW> wv[PLAY][ITEMS];
 #pragma unroll
     for (int j = 0; j < PLAY; ++j) {
         float acc = 0.f;
 #pragma unroll
-        for (int i = 0; i < NORM_ITEMS; ++i) {
-            const int c = (i * NORM_VTHREADS + j * THREADS + threadIdx.x) * 4;
+        for (int i = 0; i < ITEMS; ++i) {
+            const int c = (i * VT + j * THREADS + threadIdx.x) * 4;
             if (c < d) {
                 const Vec4<TX> xv = *(const Vec4<TX> *)(xr + c);
+                wv[j][i] = *(const Vec4<TW> *)(w + c);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[j][i][e] = to_f32(xv.v[e]);
                 if (dr) {
@@ -177,25 +179,24 @@ rmsnorm_fast_kernel(TX *__restrict__ x, const TD *__restrict__ delta, const TW *
             }
         }
         // the wave of the 1024 threads that these virtual threads are
-        acc = wave_sum(acc);
+        acc = wave_sum_in_place(acc);
         if ((threadIdx.x & (WAVE - 1)) == 0) scratch[j * (THREADS / WAVE) + threadIdx.x / WAVE] = acc;
     }
     __syncthreads();
     float total = 0.f;
 #pragma unroll
-    for (int k = 0; k < NORM_VTHREADS / WAVE; ++k) total += scratch[k];
+    for (int k = 0; k < VT / WAVE; ++k) total += scratch[k];
     const float rms = rsqrtf(total / (float)d + eps);
     TO *o = out + (size_t)blockIdx.x * d;
 #pragma unroll
     for (int j = 0; j < PLAY; ++j)
 #pragma unroll
-        for (int i = 0; i < NORM_ITEMS; ++i) {
-            const int c = (i * NORM_VTHREADS + j * THREADS + threadIdx.x) * 4;
+        for (int i = 0; i < ITEMS; ++i) {
+            const int c = (i * VT + j * THREADS + threadIdx.x) * 4;
             if (c < d) {
-                const Vec4<TW> wv = *(const Vec4<TW> *)(w + c);
                 Vec4<TO> ov;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) ov.v[e] = from_f32<TO>(rms * v[j][i][e] * to_f32(wv.v[e]));
+                for (int e = 0; e < 4; ++e) ov.v[e] = from_f32<TO>(rms * v[j][i][e] * to_f32(wv[j][i].v[e]));
                 *(Vec4<TO> *)(o + c) = ov;
             }
         }
@@ -205,17 +206,24 @@ template <class TX, class TD, class TO>
 static int rmsnorm_w(void *x, const void *delta, const void *w, int w_type, void *out, int n, int d, float eps,
                      int write_back, float delta_scale, hipStream_t stream, int planes = 1, size_t plane_stride = 0) {
     dim3 grid(n), block(d >= 2048 ? 512 : 256);
-    if (d % 4 == 0 && d <= NORM_VTHREADS * NORM_ITEMS * 4) {
-#define FAST(T_, TW_) rmsnorm_fast_kernel<T_, TX, TD, TW_, TO><<<grid, dim3(T_), 0, stream>>>((TX *)x, (const TD *)delta, (const TW_ *)w, (TO *)out, d, eps, write_back, planes, plane_stride, delta_scale)
+    if (d % 4 == 0 && d <= 8192) {
+#define SIZED(VT_, I_, T_, TW_) rmsnorm_fast_kernel<VT_, I_, T_, TX, TD, TW_, TO><<<grid, dim3(T_), 0, stream>>>((TX *)x, (const TD *)delta, (const TW_ *)w, (TO *)out, d, eps, write_back, planes, plane_stride, delta_scale)
+#define FAST(FEW_, TW_)                                                         \
+    do {                                                                         \
+        if (d <= 2048) SIZED(512, 1, (FEW_ ? 512 : 256), TW_);                   \
+        else if (d <= 4096) SIZED(1024, 1, (FEW_ ? 1024 : 256), TW_);            \
+        else SIZED(1024, 2, (FEW_ ? 1024 : 256), TW_);                           \
+    } while (0)
         const bool few = n <= 192;        // (measured with four planes: steps of 160 and 192 rows 2 % faster with 1024 threads, of 256 rows 1 % slower)
         if (w_type == LCU_F32) {
-            if (few) FAST(1024, float); else FAST(256, float);
+            if (few) FAST(true, float); else FAST(false, float);
         } else if (w_type == LCU_BF16) {
-            if (few) FAST(1024, bf16_t); else FAST(256, bf16_t);
+            if (few) FAST(true, bf16_t); else FAST(false, bf16_t);
         } else {
             return LCU_BAD_ARGUMENT;
         }
 #undef FAST
+#undef SIZED
         LCU_LAUNCH_CHECK();
         return LCU_OK;
     }

@@ -10,7 +10,7 @@
 // where rows before the request's first row of this step come from the request's state (the
 // last T - 1 rows of earlier steps) and rows before position 0 are zeros.
 #include "common.h"
-#include "lane_moves.h"
+#include "rows.h"
 
 constexpr int NC_THREADS = 256;
 constexpr int MAX_TAPS = 16;
@@ -46,30 +46,6 @@ layernorm_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes
         out1[(size_t)blockIdx.x * d + c] = from_f32<TO>(z * w1[c] + b1[c]);
         if (w2) out2[(size_t)blockIdx.x * d + c] = from_f32<TO>(z * w2[c] + b2[c]);
     }
-}
-
-// V neighbouring elements as one access.
-template <class T, int V> struct alignas(V * sizeof(T)) Pack { T v[V]; };
-template <class T, int V> __device__ __forceinline__ void load_as_f32(const T *p, float *out) {
-    const Pack<T, V> in = *(const Pack<T, V> *)p;
-#pragma unroll
-    for (int e = 0; e < V; ++e) out[e] = to_f32(in.v[e]);
-}
-template <class T, int V> __device__ __forceinline__ void store_f32(T *p, const float *in) {
-    Pack<T, V> out;
-#pragma unroll
-    for (int e = 0; e < V; ++e) out.v[e] = from_f32<T>(in[e]);
-    *(Pack<T, V> *)p = out;
-}
-
-// The sum over a workgroup of up to 16 waves; `scratch` (16 floats) is not in use by an earlier call.
-__device__ __forceinline__ float row_sum(float v, float *scratch) {
-    v = wave_sum_in_place(v);
-    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float t = 0.f;
-    for (int i = 0; i < (int)blockDim.x / WAVE; ++i) t += scratch[i];
-    return t;
 }
 
 // A row's elements in one thread's registers: PT pieces of V neighbours, ROW_THREADS pieces apart.  The row takes in the planes
@@ -152,9 +128,6 @@ layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int pl
         }
     }
 }
-
-// Whether four elements at a time may be read and written at p (null: nothing is).
-static bool four_ok(const void *p, int type) { return ((uintptr_t)p & (type == LCU_BF16 ? 7 : 15)) == 0; }
 
 // delta_type: -1 none, LCU_F32 or LCU_BF16.  out_type: LCU_F32 or LCU_BF16.
 LCU_API int lcu_layernorm(float *x, const void *delta, int delta_type, int planes, const float *w1, const float *b1,

@@ -8,7 +8,7 @@
 // ones: the sum of the streams, behind the last sublayer).  y may be float32 planes of partial sums, added one after the other.
 // One block per row; all of it is 32-bit with one rounding where h is stored.  Several streams are several times the bytes of one:
 // the kernel reads and writes each once, V neighbouring columns of all streams a thread, and keeps u in registers for the norm.
-#include "common.h"
+#include "rows.h"
 
 template <class T, int V> struct alignas(V * sizeof(T)) StVec { T v[V]; };
 
@@ -26,6 +26,7 @@ streams_norm_kernel(float *__restrict__ x, int streams, const TY *__restrict__ y
     float *xr = x + (size_t)blockIdx.x * S * d;
     const TY *yr = y ? y + (size_t)blockIdx.x * d : nullptr;
     float u[ITEMS][V];
+    StVec<float, V> wv[ITEMS];                 // (on its way while the sums are made)
     float acc = 0.f;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
@@ -33,6 +34,7 @@ streams_norm_kernel(float *__restrict__ x, int streams, const TY *__restrict__ y
 #pragma unroll
         for (int e = 0; e < V; ++e) u[k][e] = 0.f;
         if (c >= d) continue;
+        wv[k] = *(const StVec<float, V> *)(w + c);
         StVec<float, V> xs[SMAX];
 #pragma unroll
         for (int s = 0; s < SMAX; ++s)
@@ -79,16 +81,15 @@ streams_norm_kernel(float *__restrict__ x, int streams, const TY *__restrict__ y
 #pragma unroll
         for (int e = 0; e < V; ++e) acc += u[k][e] * u[k][e];
     }
-    const float f = rsqrtf(block_sum(acc, scratch) / (float)d + eps);
+    const float f = rsqrtf(row_sum(acc, scratch) / (float)d + eps);
     TO *o = h + (size_t)blockIdx.x * d;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         const int c = (k * threads + threadIdx.x) * V;
         if (c >= d) continue;
-        const StVec<float, V> wv = *(const StVec<float, V> *)(w + c);
         StVec<TO, V> ov;
 #pragma unroll
-        for (int e = 0; e < V; ++e) ov.v[e] = from_f32<TO>(u[k][e] * f * wv.v[e]);
+        for (int e = 0; e < V; ++e) ov.v[e] = from_f32<TO>(u[k][e] * f * wv[k].v[e]);
         *(StVec<TO, V> *)(o + c) = ov;
     }
 }

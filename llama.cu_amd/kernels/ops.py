@@ -1477,6 +1477,21 @@ def pack_experts(w: torch.Tensor) -> PackedExperts:
     return PackedExperts(units.permute(0, 1, 3, 4, 2, 5).contiguous(), (e, n, k))
 
 
+def pack_gated_experts(gate: torch.Tensor, up: torch.Tensor) -> PackedExperts:
+    """``pack_experts(gated_rows(gate, up))`` in one pass: a unit of 16 gate rows and the unit of the up rows that meet them in turns."""
+    e, ff, k = gate.shape
+    per = 8 if gate.dtype == torch.bfloat16 else 4
+    if up.shape != gate.shape or up.dtype != gate.dtype or gate.dtype not in (torch.bfloat16, torch.float32) or ff % 16:
+        raise KernelError(f"pack_gated_experts: gate {gate.dtype} {tuple(gate.shape)} and up {up.dtype} {tuple(up.shape)} must agree, with a multiple of 16 rows")
+    if k % (4 * per):
+        gate, up = (torch.nn.functional.pad(t, (0, -k % (4 * per))) for t in (gate, up))
+    steps = gate.shape[2] // (4 * per)
+    data = torch.empty((e, ff // 16, 2, steps, 4, 16, per), dtype=gate.dtype, device=gate.device)
+    for i, t in enumerate((gate, up)):
+        data[:, :, i] = t.reshape(e, ff // 16, 16, steps, 4, per).permute(0, 1, 3, 4, 2, 5)
+    return PackedExperts(data.view(e, ff // 8, steps, 4, 16, per), (e, 2 * ff, k))
+
+
 def gated_rows(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """``gate, up [experts, ff, d]`` (ff a multiple of 16) as the gated experts' first matrix ``[experts, 2 * ff, d]``: in
     turns 16 rows of the gate matrix and the 16 rows of the up matrix that meet them."""

@@ -192,16 +192,17 @@ class GatedMoE(Part):
             fill = lambda t, dims: torch.nn.functional.pad(t, dims)
             gate, up, self.router = fill(gate, (0, self.pad_width)), fill(up, (0, self.pad_width)), fill(self.router, (0, self.pad_width)).contiguous()
             self.w_down = fill(self.w_down, (0, 0, 0, self.pad_width)).contiguous()
-        self.w_gate_up = ops.gated_rows(gate.contiguous(), up.contiguous())
         if build.pack_weights:
-            self.w_gate_up, self.w_down = ops.pack_experts(self.w_gate_up), ops.pack_experts(self.w_down)
+            self.w_gate_up, self.w_down = ops.pack_gated_experts(gate, up), ops.pack_experts(self.w_down)
+        else:
+            self.w_gate_up = ops.gated_rows(gate.contiguous(), up.contiguous())
         self.shared_expert = None
         if self.shared is not None:
             self.shared.load(tensors, build)
             sg, su, sd = (tensors[nm[k]] for k in ("shared_gate", "shared_up", "shared_down"))
             if build.pack_weights and sg.shape[0] % 16 == 0 and sg.dtype == su.dtype == sd.dtype == self.w_down.dtype:
                 # steps of few tokens compute it beside the experts, from a copy in their order
-                self.shared_expert = (ops.pack_experts(ops.gated_rows(sg[None].contiguous(), su[None].contiguous())), ops.pack_experts(sd[None].contiguous()))
+                self.shared_expert = (ops.pack_gated_experts(sg[None], su[None]), ops.pack_experts(sd[None]))
         self.dtype = build.dtype
 
     def forward(self, h, add_to: Optional[torch.Tensor] = None):

@@ -47,6 +47,7 @@ def test_packed_gated_experts(dtype, n, ff):
     down = rnd(experts, d, ff, seed=5, std=ff ** -0.5).to(tdt).cuda()
     ids, wts = ops.moe_route(h, router, top, softmax_chosen=True)        # (the last of the router's rows is an identity expert)
     rows, outs = ops.gated_rows(gate, up), []
+    assert torch.equal(ops.pack_gated_experts(gate, up).data, ops.pack_experts(rows).data)
     for u, w in ((rows, down), (ops.pack_experts(rows), ops.pack_experts(down))):
         out = torch.empty(n, d, device="cuda")
         ops.moe_experts(h, ids, wts, u, w, out, gated=True, fresh=True, identity=1, act_alpha=1.702, act_limit=2.0)
