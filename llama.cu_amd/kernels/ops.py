@@ -865,6 +865,66 @@ def mid_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
             and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+WAVEK_MAX_ROWS = 64       # what gemm_wavek takes
+
+
+def wavek_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_wavek`` takes these rows with a packed weight of ``w``'s shape: up to 64 bfloat16 rows, K a multiple of 128."""
+    return (x.is_cuda and w.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() in (2, 3) and w.dim() == 2
+            and 0 < x.shape[-2] <= WAVEK_MAX_ROWS and x.shape[-1] == w.shape[1] and packable(w) and x.stride(-1) == 1
+            and x.stride(-2) % 8 == 0 and (x.dim() == 2 or x.stride(0) % 8 == 0) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def wavek_preferred(m: int, n: int, k: int, swiglu: bool = False) -> bool:
+    """Whether ``gemm_wavek`` is the fastest choice for ``m`` rows and a packed ``[n, k]`` weight (``TUNING``'s numbers)."""
+    t = TUNING
+    if k > t.wavek_max_k or n > 32 * t.compute_units:                    # (more workgroups of 32 features than compute units: a second round)
+        return False
+    if swiglu:
+        return m <= WAVEK_MAX_ROWS
+    if m <= t.wavek_few_rows:
+        return n >= t.wavek_wide_features
+    return m <= t.wavek_rows or (m <= WAVEK_MAX_ROWS and k <= t.wavek_short_k) or (m <= t.wavek_more_rows and n >= t.wavek_more_features)
+
+
+def gemm_wavek(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None,
+               swiglu: bool = False, gate: Optional[torch.Tensor] = None, row_sumsq: Optional[torch.Tensor] = None, norm_width: int = 0,
+               eps: float = 0.0, act_alpha: float = 1.0, act_limit: float = 0.0) -> torch.Tensor:
+    """``x @ w.T`` for up to 64 bfloat16 rows, ``w [n, k]`` the result of ``pack_weight``, K shared out over the waves of a workgroup.
+    ``out [m, n]`` bfloat16 or float32; ``swiglu``: ``w`` holds gate rows, then up rows, ``out [m, n / 2]`` bfloat16 (the limited
+    activation with ``act_limit`` > 0); ``x [groups, m, k]``: group ``g`` multiplies ``w``'s rows ``g * n / groups ..``;
+    ``gate [m, n]``: the bfloat16 result is multiplied by ``sigmoid(gate)``; ``row_sumsq [m, parts]``: the rows wait for their
+    normalisation, as in ``gemm_skinny``."""
+    _gpu(x, w, out, gate, row_sumsq)
+    if not wavek_supported(x, w) or not w.is_contiguous():
+        raise KernelError(f"gemm_wavek: x {tuple(x.shape)} {x.dtype} with w {tuple(w.shape)} {w.dtype} is not supported "
+                          f"(at most {WAVEK_MAX_ROWS} bfloat16 rows, a packed weight)")
+    groups, m, k = (x.shape[0] if x.dim() == 3 else 1), x.shape[-2], x.shape[-1]
+    n = w.shape[0]
+    if n % (16 * groups) or (swiglu and (n % 32 or x.dim() == 3 or gate is not None)):
+        raise KernelError(f"gemm_wavek: {n} features do not go with {groups} groups{' and SwiGLU' if swiglu else ''}")
+    dtype = out.dtype if out is not None else (out_dtype or torch.bfloat16)
+    cols = n // 2 if swiglu else n
+    if out is None:
+        out = torch.empty((m, cols), dtype=dtype, device=x.device)
+    if dtype not in (torch.bfloat16, torch.float32) or (dtype != torch.bfloat16 and (swiglu or gate is not None)) or out.shape != (m, cols) \
+            or out.stride(1) != 1 or out.stride(0) % 4 or out.data_ptr() % 16:
+        raise KernelError(f"gemm_wavek out: {out.dtype} {tuple(out.shape)} with strides {out.stride()} is not supported")
+    if gate is not None and (gate.dtype != torch.bfloat16 or gate.shape != (m, n) or gate.stride(1) != 1 or gate.stride(0) % 4 or gate.data_ptr() % 8):
+        raise KernelError(f"gemm_wavek gate: {gate.dtype} {tuple(gate.shape)} is not supported")
+    if row_sumsq is not None:
+        _contig(row_sumsq, "row sums")
+        if row_sumsq.dtype != torch.float32 or row_sumsq.dim() != 2 or row_sumsq.shape[0] != m or norm_width <= 0 or groups != 1:
+            raise KernelError(f"gemm_wavek: row sums {row_sumsq.dtype} {tuple(row_sumsq.shape)} do not go with {m} rows")
+    epi = 2 if swiglu else 3 if gate is not None else 1 if dtype == torch.float32 else 0
+    lib = build.load("gemm_wavek")
+    _check(lib.lcu_gemm_wavek(_ptr(x), x.stride(-2), ctypes.c_longlong(x.stride(0) if x.dim() == 3 else 0), groups, _ptr(w), _ptr(out), out.stride(0),
+                              _ptr(gate), gate.stride(0) if gate is not None else 0, m, n, k, epi, int(n >= TUNING.wavek_wide_features),
+                              _ptr(row_sumsq), row_sumsq.shape[1] if row_sumsq is not None else 0, int(norm_width), ctypes.c_float(eps),
+                              ctypes.c_float(act_alpha), ctypes.c_float(act_limit), _stream()), "gemm_wavek")
+    return out
+
+
 def mid_planes(k: int, slices: int) -> int:
     """The number of planes ``gemm_mid(..., slices=)`` writes for a weight with ``k`` columns."""
     steps = k // 128

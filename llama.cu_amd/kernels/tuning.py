@@ -59,6 +59,16 @@ class Tuning:
                                         # nothing at 25 to 32)
     mid_min_slice_steps: int = 4        # a slice of K keeps at least this many macro-steps of 128
     mid_max_slices: int = 8
+    # ---- the product whose waves share out K (gemm_wavek.hip, up to 64 rows)
+    # (its numbers stand in gemm_wavek.hip; measured with widths of 1024 and 2048)
+    wavek_wide_features: int = 4096     # 32 features a workgroup instead of 16 from this many on
+    wavek_max_k: int = 3072             # with a longer K the weight-streaming kernel is faster (K = 4096: 8.0 us against 9.9 at 8 rows)
+    wavek_few_rows: int = 4             # up to here a plain product goes to it from wavek_wide_features features on only (below the
+                                        # two are equal)
+    wavek_rows: int = 32                # up to here every plain product does,
+    wavek_short_k: int = 1024           # ... up to 64 rows with a K up to this (2048 x 768: 5.7 us against the library's 7.2 at 64 rows),
+    wavek_more_rows: int = 48           # ... and up to here from so many features on (3072 x 2048: 9.2 us against 10.2 to 10.6; at 64 rows
+    wavek_more_features: int = 3072     # 11.1 against 10.9, with 2048 features 9.0 against 8.3 at 48)
     # ---- the library's product of many rows (parts/linear.library_friendly_rows)
     library_rows: int = -1              # rows of zeros behind each half of a plain gate/up matrix: -1 times the library once per
                                         # shape at load and fills up where that is 15 % faster (the outcome can differ from box

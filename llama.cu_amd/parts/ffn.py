@@ -16,7 +16,7 @@ from ..kernels import ops
 from .base import BuildContext, Part, ScaledRows, TensorSpec, register_part
 from ..weights.loader import fused_rows
 from .linear import (Weight, end_in_norm, library_friendly_rows, linear, linear_planes, linear_swiglu,
-                     linear_swiglu_mid, mid_swiglu_takes, mid_takes, skinny_row_limit, skinny_takes)
+                     linear_swiglu_mid, mid_swiglu_takes, mid_takes, skinny_row_limit, skinny_takes, wavek_swiglu_takes)
 
 
 class SwiGLU(Part):
@@ -115,6 +115,8 @@ class SwiGLU(Part):
         elif self.dtype == torch.bfloat16 and mid_swiglu_takes(h.shape[0], self.w_gate_up) and ops.mid_supported(h, self.w_gate_up.plain):
             # 15 to 192 rows (mid_swiglu_max_rows): the rows shared through LDS, the activation in the product's epilogue
             act = linear_swiglu_mid(h, self.w_gate_up, **self.act)
+        elif self.dtype == torch.bfloat16 and wavek_swiglu_takes(h, self.w_gate_up):
+            act = linear_swiglu(h, self.w_gate_up, **self.act)
         elif (self.dtype == torch.bfloat16 and h.shape[0] <= skinny_row_limit(self.w_gate_up)
               and ops.skinny_supported(h, self.w_gate_up.plain, self.dtype)):
             # few rows: one pass over the weights, the activation in the product's epilogue

@@ -57,6 +57,15 @@ def _split(weight):
     return weight, None
 
 
+def wavek_takes(x: torch.Tensor, packed: Optional[torch.Tensor], swiglu: bool = False) -> bool:
+    """Whether the product whose waves share out K is the choice for these rows and this packed matrix."""
+    return packed is not None and ops.wavek_preferred(x.shape[-2], packed.shape[0], packed.shape[1], swiglu) and ops.wavek_supported(x, packed)
+
+
+def _plain_rows(out: torch.Tensor) -> bool:
+    return out.dtype in (torch.bfloat16, torch.float32) and out.dim() == 2 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0
+
+
 def linear(x: torch.Tensor, weight: Union[torch.Tensor, Weight], out_dtype: Optional[torch.dtype] = None,
            out: Optional[torch.Tensor] = None, accumulate: bool = False) -> torch.Tensor:
     """``out (+)= x @ weight.T``.  ``accumulate`` adds into a float32 ``out`` in 32-bit."""
@@ -65,6 +74,9 @@ def linear(x: torch.Tensor, weight: Union[torch.Tensor, Weight], out_dtype: Opti
     weight, packed = _split(weight)
     out_dtype = out.dtype if out is not None else (out_dtype or x.dtype)
     all_bf16 = x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+    if (all_bf16 and packed is not None and packed.shape == weight.shape and not accumulate and x.dim() == 2 and wavek_takes(x, packed)
+            and out_dtype in (torch.bfloat16, torch.float32) and (out is None or _plain_rows(out))):
+        return ops.gemm_wavek(x, packed, out=out, out_dtype=out_dtype)
     if all_bf16 and ops.skinny_supported(x, weight, out_dtype) and (
             accumulate or ops.skinny_preferred(x.shape[0], weight.shape[0], weight.shape[1], out_dtype, packed is not None)):
         if packed is not None:
@@ -89,15 +101,25 @@ def linear_swiglu(h, weight: Union[torch.Tensor, Weight], row_sumsq=None, norm_w
     the limited activation."""
     weight, packed = _split(weight)
     kw = dict(act, row_sumsq=row_sumsq, norm_width=norm_width, eps=eps) if row_sumsq is not None else act
+    if packed is not None and packed.shape[0] % 32 == 0 and wavek_takes(h, packed, swiglu=True):
+        return ops.gemm_wavek(h, packed, swiglu=True, **kw)
     if packed is not None:
         return ops.gemm_skinny(h, packed, swiglu=True, packed=True, **kw)
     return ops.gemm_skinny(h, weight, swiglu=True, **kw)
+
+
+def wavek_swiglu_takes(h: torch.Tensor, weight: Union[torch.Tensor, Weight]) -> bool:
+    """Whether ``linear_swiglu`` sends these rows to the product whose waves share out K (up to 64 of them)."""
+    packed = _split(weight)[1]
+    return packed is not None and packed.shape[0] % 32 == 0 and h.dtype == torch.bfloat16 and h.dim() == 2 and wavek_takes(h, packed, swiglu=True)
 
 
 def linear_scaled(rows, weight: Union[torch.Tensor, Weight], out_dtype: Optional[torch.dtype] = None):
     """``rows.rows @ weight.T`` with the rows' normalisation applied in the epilogue (``rows``: ScaledRows)."""
     weight, packed = _split(weight)
     kw = dict(row_sumsq=rows.sumsq, norm_width=rows.width, eps=rows.eps, out_dtype=out_dtype)
+    if packed is not None and wavek_takes(rows.rows, packed):
+        return ops.gemm_wavek(rows.rows, packed, **kw)
     if packed is not None:
         return ops.gemm_skinny(rows.rows, packed, packed=True, **kw)
     return ops.gemm_skinny(rows.rows, weight, **kw)
@@ -360,6 +382,9 @@ def linear_groups(x: torch.Tensor, weight: GroupWeight, out: torch.Tensor, gate:
     g, m, _ = x.shape
     if x.dtype == torch.bfloat16 and weight.each.dtype == torch.bfloat16:
         packed = weight.stacked.packed
+        if packed is not None and weight.rows % 16 == 0 and out.dtype == torch.bfloat16 and _plain_rows(out) and wavek_takes(x, packed) \
+                and (gate is None or (gate.dtype == torch.bfloat16 and gate.stride(1) == 1 and gate.stride(0) % 4 == 0 and gate.data_ptr() % 8 == 0)):
+            return ops.gemm_wavek(x, packed, out=out, gate=gate)
         if m <= ops.skinny_max_rows(packed is not None) and ops.skinny_grouped_supported(x, weight.stacked.plain, g):
             return ops.gemm_skinny_grouped(x, weight.stacked.plain if packed is None else packed, out, packed=packed is not None, gate=gate)
         if out.dtype == torch.bfloat16:
