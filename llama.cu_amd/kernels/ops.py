@@ -878,7 +878,7 @@ def wavek_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
 def wavek_preferred(m: int, n: int, k: int, swiglu: bool = False) -> bool:
     """Whether ``gemm_wavek`` is the fastest choice for ``m`` rows and a packed ``[n, k]`` weight (``TUNING``'s numbers)."""
     t = TUNING
-    if k > t.wavek_max_k or n > 32 * t.compute_units:                    # (more workgroups of 32 features than compute units: a second round)
+    if min(n, k) < t.wavek_least or k > t.wavek_max_k or n > 32 * t.compute_units:                    # (more workgroups of 32 features than compute units: a second round)
         return False
     if swiglu:
         return m <= WAVEK_MAX_ROWS

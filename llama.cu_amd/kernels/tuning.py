@@ -63,6 +63,7 @@ class Tuning:
     # (its numbers stand in gemm_wavek.hip; measured with widths of 1024 and 2048)
     wavek_wide_features: int = 4096     # 32 features a workgroup instead of 16 from this many on
     wavek_max_k: int = 3072             # with a longer K the weight-streaming kernel is faster (K = 4096: 8.0 us against 9.9 at 8 rows)
+    wavek_least: int = 512              # features and K from which on it was measured: below either, the general path
     wavek_few_rows: int = 4             # up to here a plain product goes to it from wavek_wide_features features on only (below the
                                         # two are equal)
     wavek_rows: int = 32                # up to here every plain product does,

@@ -65,7 +65,7 @@ def test_groups(m, n, k, groups):
 
 
 @pytest.mark.parametrize("m", [4, 5, 32, 33, 48, 49, 64, 65])
-@pytest.mark.parametrize("n,k", [(1024, 1024), (2048, 2048), (3072, 2048), (8192, 256), (8224, 256)])
+@pytest.mark.parametrize("n,k", [(1024, 1024), (2048, 2048), (3072, 2048), (8192, 512), (8224, 512), (496, 512), (512, 384)])
 def test_the_rule_against_the_general_path(m, n, k):
     """A product on both sides of the rule's lines, the rows as they are and where they cannot be loaded 16 bytes at a time."""
     from llama_cu_amd.parts.linear import Weight, linear
