@@ -29,6 +29,7 @@
 // (group g reads X + g * x_group_stride): one product per head, or several projections of differently mixed rows, in
 // one launch.  Their outputs may be multiplied by the sigmoid of a gate [M, N] on the way out.
 #include "common.h"
+#include "lane_moves.h"
 #include "gate_act.h"
 #include "kv_layout.h"
 
@@ -609,11 +610,28 @@ LCU_API int lcu_gemm_skinny_bf16_qkv_rope(const void *X, int ldx, const void *W,
 // ============================================================================ float32
 // The same weight-streaming layout for float32 operands, with v_mfma_f32_16x16x4_f32: a true
 // 32-bit matrix product (32-bit multiplies and adds; no reduced-precision mode).  A lane's
-// 16-byte load holds four k of its row, one per instruction.  K goes in macro-steps of 64; the
+// 16-byte load holds four k of its row, one per instruction, and the four lane groups' loads of a row lie side by side.  K goes in
+// macro-steps of 64; the
 // waves of a workgroup take macro-steps in turn and their sums are added in a fixed order, so
 // a token's result depends on K and the number of waves only: not on M, not on which tile of
-// 64 tokens (grid.y) it is in, not on the other tokens.
+// 16 or 64 tokens (grid.y) it is in, not on the other tokens.
+//
+// The products that begin and end a branch of a 32-bit model do more, so that no norm or activation kernel runs between them: the
+// rows may wait for their normalisation (sumsq_in), the result may go into the residual stream, with the next norm's weight on its
+// way out (norm_w), and gate and up rows may meet in SwiGLU (PAIR: the matrix tile's sixteen rows are eight gate rows and the eight up rows
+// that meet them, so that there are as many workgroups as without).  What
+// bounds it at few tokens is latency (a launch, one round of loads, 0.9 us of matrix instructions), not the matrix: us at 2 tokens, 1024 x 1024
+// 5.5, with the rows' factor 5.9, with residual and norm weight 6.2, SwiGLU of 2816 x 1024 6.5 (and 3.3 and 3.5 for the kernels that ran
+// between); 32000 x 1024 32.5 (4.0 TB/s).
 constexpr int F32_WAVES = 8;
+
+struct F32Extra {
+    int accumulate;
+    float scale;                                             // of the product before it is added (accumulate, norm_w)
+    const float *sumsq_in; int n_in, norm_width; float eps;  // null, or [M, n_in] shares of the rows' sums of squares
+    const float *norm_w; float *h_out; int ldh; float *sumsq_out;      // null, or: Y += ..., h_out = Y * norm_w, sumsq_out [M, N / 16 rounded up]
+    float act_alpha, act_limit;
+};
 
 template <int MT>
 struct FragF32 {
@@ -624,28 +642,38 @@ struct FragF32 {
 template <int MT>
 __device__ __forceinline__ void load_frag_f32(FragF32<MT> &f, const float *wrow, const float *const (&xrow)[MT],
                                               const bool (&xvalid)[MT], int s, int grp, int K) {
-    const int kb = 64 * s + 16 * grp;
     const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const bool in = kb + 4 * j + 4 <= K;                // K is a multiple of 4
-        f.w[j] = in ? *(const f32x4 *)(wrow + kb + 4 * j) : zero;
+        const int kb = 64 * s + 16 * j + 4 * grp;
+        const bool in = kb + 4 <= K;                        // K is a multiple of 4
+        f.w[j] = in ? *(const f32x4 *)(wrow + kb) : zero;
 #pragma unroll
-        for (int m = 0; m < MT; ++m) f.x[m][j] = (in && xvalid[m]) ? *(const f32x4 *)(xrow[m] + kb + 4 * j) : zero;
+        for (int m = 0; m < MT; ++m) f.x[m][j] = (in && xvalid[m]) ? *(const f32x4 *)(xrow[m] + kb) : zero;
     }
 }
 
 template <int MT>
+__device__ __forceinline__ void mul_frag_f32(const FragF32<MT> &f, f32x4 (&acc)[MT]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[j][e], f.x[m][j][e], acc[m], 0, 0, 0);
+}
+
+template <int MT, bool PAIR>
 __global__ void __launch_bounds__(F32_WAVES *WAVE)
 gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W, int ldw, float *__restrict__ Y,
-                       int ldy, int M, int N, int K, int accumulate) {
-    __shared__ float red[F32_WAVES][MT * 4][WAVE];
+                       int ldy, int M, int N, int K, F32Extra ex) {
+    __shared__ f32x4 red[F32_WAVES][MT][WAVE];
+    __shared__ float factor[16 * MT];
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     const int l16 = lane & 15, grp = lane >> 4;
-    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16 * MT;
-    int row = n0 + l16;
-    row = row < N ? row : N - 1;                            // a row beyond the end is read, not stored
-    const float *wrow = W + (size_t)row * ldw;
+    const int n0 = blockIdx.x * (PAIR ? 8 : 16), m0 = blockIdx.y * 16 * MT;
+    // (a row beyond the end is read, not stored)
+    const float *wrow = W + (size_t)(PAIR ? min(n0 + (l16 & 7), N - 1) + (l16 < 8 ? 0 : N) : min(n0 + l16, N - 1)) * ldw;
     const float *xrow[MT];
     bool xvalid[MT];
 #pragma unroll
@@ -660,62 +688,98 @@ gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__rest
     FragF32<MT> fa, fb;
     int s = wave;
     if (s < nsteps) load_frag_f32<MT>(fa, wrow, xrow, xvalid, s, grp, K);
-    for (; s < nsteps; s += 2 * F32_WAVES) {
-        const bool has_b = s + F32_WAVES < nsteps;
-        if (has_b) load_frag_f32<MT>(fb, wrow, xrow, xvalid, s + F32_WAVES, grp, K);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa.w[j][e], fa.x[m][j][e], acc[m], 0, 0, 0);
-        if (s + 2 * F32_WAVES < nsteps) load_frag_f32<MT>(fa, wrow, xrow, xvalid, s + 2 * F32_WAVES, grp, K);
-        if (has_b) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb.w[j][e], fb.x[m][j][e], acc[m], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) red[wave][m * 4 + r][lane] = acc[m][r];
-    __syncthreads();
-    if (wave != 0) return;
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int tok = m0 + 16 * m + l16;
+    if (s + F32_WAVES < nsteps) load_frag_f32<MT>(fb, wrow, xrow, xvalid, s + F32_WAVES, grp, K);
+    // a wave stores sixteen tokens in the end; what it adds to, and the norm's weights, are on their way meanwhile
+    const int tok = m0 + 16 * wave + l16;
+    const bool adds = !PAIR && (ex.accumulate || ex.norm_w) && wave < MT;
+    float old[4] = {}, nw[4] = {};
+    if (adds) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            float sum = red[0][m * 4 + r][lane];
-#pragma unroll
-            for (int w = 1; w < F32_WAVES; ++w) sum += red[w][m * 4 + r][lane];
             const int n = n0 + 4 * grp + r;
             if (tok < M && n < N) {
-                float *y = Y + (size_t)tok * ldy + n;
-                *y = accumulate ? *y + sum : sum;
+                old[r] = Y[(size_t)tok * ldy + n];
+                if (ex.norm_w) nw[r] = ex.norm_w[n];
             }
         }
     }
+    if (ex.sumsq_in) {
+        for (int r = wave; r < 16 * MT && m0 + r < M; r += F32_WAVES) {
+            float t = 0.f;
+            for (int i = lane; i < ex.n_in; i += WAVE) t += ex.sumsq_in[(size_t)(m0 + r) * ex.n_in + i];
+            t = wave_sum_in_place(t);
+            if (lane == 0) factor[r] = rsqrtf(t / (float)ex.norm_width + ex.eps);
+        }
+    }
+    for (; s < nsteps; s += 2 * F32_WAVES) {
+        mul_frag_f32<MT>(fa, acc);
+        if (s + 2 * F32_WAVES < nsteps) load_frag_f32<MT>(fa, wrow, xrow, xvalid, s + 2 * F32_WAVES, grp, K);
+        if (s + F32_WAVES < nsteps) mul_frag_f32<MT>(fb, acc);
+        if (s + 3 * F32_WAVES < nsteps) load_frag_f32<MT>(fb, wrow, xrow, xvalid, s + 3 * F32_WAVES, grp, K);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) red[wave][m][lane] = acc[m];
+    __syncthreads();
+    if (wave >= MT) return;
+    f32x4 sum = red[0][wave][lane];
+#pragma unroll
+    for (int w = 1; w < F32_WAVES; ++w) sum += red[w][wave][lane];
+    if (ex.sumsq_in) sum *= factor[16 * wave + l16];
+    if constexpr (PAIR) {                                    // the up rows' sums are 32 lanes further
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const unsigned u = __float_as_uint(sum[r]);
+            const float up = __uint_as_float(__builtin_amdgcn_permlane32_swap(u, u, false, false)[1]);
+            const int n = n0 + 4 * grp + r;
+            if (grp < 2 && tok < M && n < N) Y[(size_t)tok * ldy + n] = gate_up_of(sum[r], up, ex.act_alpha, ex.act_limit);
+        }
+        return;
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int n = n0 + 4 * grp + r;
+        if (tok >= M || n >= N) continue;
+        const float v = adds ? old[r] + ex.scale * sum[r] : sum[r];
+        Y[(size_t)tok * ldy + n] = v;
+        if (ex.norm_w) {
+            ex.h_out[(size_t)tok * ex.ldh + n] = v * nw[r];
+            ss += v * v;
+        }
+    }
+    if (ex.norm_w) {                                         // every lane takes part: the others bring zero
+        ss += __shfl_xor(ss, 16, WAVE);
+        ss += __shfl_xor(ss, 32, WAVE);
+        if (grp == 0 && tok < M) ex.sumsq_out[(size_t)tok * gridDim.x + blockIdx.x] = ss;
+    }
 }
 
-// X: [M, K] float32, W: [N, K] float32, Y: [M, N] float32 (accumulate: Y += X W^T).  Any M
-// (tiles of 64 tokens; W is read once per tile); K, ldx, ldw multiples of 4.
+// X: [M, K] float32, W: [N, K] float32, Y: [M, N] float32 (accumulate: Y += scale X W^T).  Any M
+// (tiles of 16 or 64 tokens; W is read once per tile); K, ldx, ldw multiples of 4, X and W 16-byte aligned.
+// swiglu: W holds N gate rows, then N up rows.  sumsq_in: null, or [M, n_in] shares of the rows' sums of squares: the product's rows are
+// multiplied by rsqrt(sum / norm_width + eps).  norm_w: null, or [N]: Y += scale X W^T, h_out [M, ldh] = Y norm_w, sumsq_out [M, ceil(N / 16)] the
+// shares of the new rows' sums of squares.
 LCU_API int lcu_gemm_skinny_f32(const float *X, int ldx, const float *W, int ldw, float *Y, int ldy, int M, int N,
-                                int K, int accumulate, hipStream_t stream) {
+                                int K, int accumulate, float scale, int swiglu, const float *sumsq_in, int n_in, int norm_width, float eps,
+                                const float *norm_w, float *h_out, int ldh, float *sumsq_out, float act_alpha, float act_limit, hipStream_t stream) {
     if (M <= 0 || N <= 0) return LCU_OK;
     if (K <= 0 || K % 4 || ldx % 4 || ldw % 4 || ldx < K || ldw < K || ldy < N) return LCU_BAD_ARGUMENT;
-    const dim3 block(F32_WAVES * WAVE);
-    if (M <= 16) {
-        gemm_skinny_f32_kernel<1><<<dim3((N + 15) / 16, 1), block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, accumulate);
-    } else {
-        const int tiles = (M + 63) / 64;
-        if (tiles > 65535) return LCU_BAD_ARGUMENT;
-        gemm_skinny_f32_kernel<4><<<dim3((N + 15) / 16, tiles), block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, accumulate);
-    }
+    if ((sumsq_in && (n_in <= 0 || norm_width <= 0)) || (norm_w && (!h_out || !sumsq_out || ldh < N || swiglu)) || (swiglu && accumulate))
+        return LCU_BAD_ARGUMENT;
+    F32Extra ex = {accumulate, scale, sumsq_in, n_in, norm_width, eps, norm_w, h_out, ldh, sumsq_out, act_alpha, act_limit};
+    // 16 tokens a workgroup, each of which reads its rows of W (from the L2 caches, but for the first), while the matrix instructions are
+    // what takes the time: up to 32 tokens, and up to three workgroups a compute unit.  One MI355X, us with 16 / 64 tokens a
+    // workgroup: 1024 x 1024 at 62 tokens 6.8 / 14.6, at 128 10.5 / 15.0, at 250 (1,024 workgroups) 18.2 / 15.0; 2816 x 1024 at 62 (704) 15.0 / 16.1;
+    // 32000 x 1024 at 62 127 / 117, at 32 70 (77 with 32 tokens a workgroup).
+    const int rows = M <= 32 || ((N + 15) / 16) * ((M + 15) / 16) <= 768 ? 16 : 64;
+    const int tiles = (M + rows - 1) / rows;
+    if (tiles > 65535) return LCU_BAD_ARGUMENT;
+    const dim3 grid(swiglu ? (N + 7) / 8 : (N + 15) / 16, tiles), block(F32_WAVES * WAVE);
+#define GO(MT, PAIR) gemm_skinny_f32_kernel<MT, PAIR><<<grid, block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, ex)
+    if (rows == 16) { if (swiglu) GO(1, true); else GO(1, false); }
+    else if (swiglu) GO(4, true);
+    else GO(4, false);
+#undef GO
     LCU_LAUNCH_CHECK();
     return LCU_OK;
 }

@@ -1180,14 +1180,35 @@ def skinny_f32_supported(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtyp
 
 
 def gemm_skinny_f32(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
-                    accumulate: bool = False) -> torch.Tensor:
+                    accumulate: bool = False, swiglu: bool = False, row_sumsq: Optional[torch.Tensor] = None, norm_width: int = 0,
+                    eps: float = 0.0, act_alpha: float = 1.0, act_limit: float = 0.0) -> torch.Tensor:
     """``out (+)= x @ w.T`` in true 32-bit on the matrix cores (v_mfma_f32_16x16x4_f32), any
-    number of rows; a row's result does not depend on the other rows."""
-    _gpu(x, w, out)
+    number of rows; a row's result does not depend on the other rows.  ``swiglu``: ``w`` holds gate rows, then up rows, ``out [m, n / 2]``
+    (the limited activation with ``act_limit`` > 0); ``row_sumsq``: the rows wait for their normalisation, as in ``gemm_skinny``."""
+    return _skinny_f32(x, w, out, accumulate=accumulate, swiglu=swiglu, row_sumsq=row_sumsq, norm_width=norm_width, eps=eps,
+                       act_alpha=act_alpha, act_limit=act_limit)
+
+
+def gemm_skinny_f32_add_norm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, norm_weight: torch.Tensor, scale: float = 1.0):
+    """``gemm_skinny_add_norm`` in 32 bits, any number of rows: ``residual += scale * (x @ w.T)``; returns ``(h, sumsq)`` with
+    ``h = residual * norm_weight`` and the shares of the rows' sums of squares.  A row's result does not depend on the other rows."""
+    _gpu(residual, norm_weight)
+    n = w.shape[0]
+    if norm_weight.dtype != torch.float32 or norm_weight.shape != (n,) or not norm_weight.is_contiguous():
+        raise KernelError(f"gemm_skinny_f32_add_norm: the norm's weight must be contiguous float32 [{n}]")
+    h = torch.empty((x.shape[0], n), dtype=torch.float32, device=x.device)
+    sumsq = torch.empty((x.shape[0], -(-n // 16)), dtype=torch.float32, device=x.device)
+    _skinny_f32(x, w, residual, scale=scale, norm_weight=norm_weight, h=h, sumsq=sumsq)
+    return h, sumsq
+
+
+def _skinny_f32(x, w, out, accumulate=False, scale=1.0, swiglu=False, row_sumsq=None, norm_width=0, eps=0.0, norm_weight=None, h=None, sumsq=None,
+                act_alpha=1.0, act_limit=0.0):
+    _gpu(x, w, out, row_sumsq)
     _rows(x, "skinny x"); _rows(w, "skinny w")
     m, k = x.shape
-    n = w.shape[0]
-    if w.shape[1] != k or not skinny_f32_supported(x, w, torch.float32):
+    n = w.shape[0] // 2 if swiglu else w.shape[0]
+    if w.shape[1] != k or not skinny_f32_supported(x, w, torch.float32) or (swiglu and (w.shape[0] % 2 or accumulate)):
         raise KernelError(f"gemm_skinny_f32: x {tuple(x.shape)} {x.dtype} with w {tuple(w.shape)} {w.dtype} is not supported")
     if out is None:
         if accumulate:
@@ -1196,9 +1217,15 @@ def gemm_skinny_f32(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor
     _rows(out, "skinny out")
     if out.shape != (m, n) or out.dtype != torch.float32:
         raise KernelError("gemm_skinny_f32 out: wrong shape or type")
+    if row_sumsq is not None and (row_sumsq.dtype != torch.float32 or row_sumsq.dim() != 2 or row_sumsq.shape[0] != m
+                                  or not row_sumsq.is_contiguous() or norm_width <= 0):
+        raise KernelError("gemm_skinny_f32: row_sumsq must be a contiguous float32 [rows, parts] tensor, with the norm's width")
     lib = build.load("gemm_skinny")
     _check(lib.lcu_gemm_skinny_f32(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), m, n, k,
-                                   int(bool(accumulate)), _stream()), "gemm_skinny_f32")
+                                   int(bool(accumulate)), ctypes.c_float(scale), int(bool(swiglu)),
+                                   _ptr(row_sumsq), row_sumsq.shape[1] if row_sumsq is not None else 0, int(norm_width), ctypes.c_float(eps),
+                                   _ptr(norm_weight), _ptr(h), n, _ptr(sumsq), ctypes.c_float(act_alpha), ctypes.c_float(act_limit), _stream()),
+           "gemm_skinny_f32")
     return out
 
 

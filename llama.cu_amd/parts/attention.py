@@ -15,7 +15,7 @@ import torch
 
 from ..kernels import ops
 from .base import BuildContext, PagedKV, Part, PartSpec, ScaledRows, TensorSpec, make_part, register_part
-from .linear import (Weight, end_in_norm, linear, linear_planes, linear_qkv_rope, linear_scaled, mid_qkv_takes, mid_takes,
+from .linear import (Weight, end_in_norm, f32_takes_scaled_rows, linear, linear_planes, linear_qkv_rope, linear_scaled, mid_qkv_takes, mid_takes,
                      project, skinny_takes)
 from ..weights.loader import fused_rows
 
@@ -319,6 +319,8 @@ class Attention(Part):
         if self.general:
             return (self.dtype == torch.bfloat16 and n_rows <= ops.ADD_NORM_MAX_ROWS
                     and skinny_takes(n_rows, self.w_in, preferred=True))
+        if self.dtype == torch.float32:          # any number of rows
+            return f32_takes_scaled_rows(self.w_qkv)
         return self.dtype == torch.bfloat16 and n_rows <= ops.ADD_NORM_MAX_ROWS and skinny_takes(n_rows, self.w_qkv, preferred=True)
 
     def forward(self, h, step, cache, into=None, planes_ok=False, out_dtype=None, bias_later=False):

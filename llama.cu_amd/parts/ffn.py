@@ -15,7 +15,7 @@ import torch
 from ..kernels import ops
 from .base import BuildContext, Part, ScaledRows, TensorSpec, register_part
 from ..weights.loader import fused_rows
-from .linear import (Weight, end_in_norm, library_friendly_rows, linear, linear_planes, linear_swiglu,
+from .linear import (Weight, end_in_norm, f32_takes_scaled_rows, library_friendly_rows, linear, linear_planes, linear_swiglu,
                      linear_swiglu_mid, mid_swiglu_takes, mid_takes, skinny_row_limit, skinny_takes, wavek_swiglu_takes)
 
 
@@ -79,6 +79,8 @@ class SwiGLU(Part):
     def takes_scaled_rows(self, n_rows: int) -> bool:
         """Whether ``forward`` could be given ScaledRows of ``n_rows`` rows in the place of
         plain rows: the factor then goes into the first product's epilogue."""
+        if self.fused_activation and self.dtype == torch.float32:          # any number of rows
+            return f32_takes_scaled_rows(self.w_gate_up)
         if self.dtype != torch.bfloat16 or not self.fused_activation:
             return False
         if n_rows <= min(ops.ADD_NORM_MAX_ROWS, skinny_row_limit(self.w_gate_up)) and skinny_takes(n_rows, self.w_gate_up):
@@ -108,6 +110,9 @@ class SwiGLU(Part):
             act = ops.swiglu(linear(h, self.w_gate_up, out_dtype=self.dtype), activation=self.activation)
         elif isinstance(h, ScaledRows) and mid_swiglu_takes(h.rows.shape[0], self.w_gate_up) and ops.mid_supported(h.rows, self.w_gate_up.plain):
             act = linear_swiglu_mid(h, self.w_gate_up, **self.act)
+        elif self.dtype == torch.float32 and (isinstance(h, ScaledRows) or ops.skinny_f32_supported(h, self.w_gate_up.plain, self.dtype)):
+            act = (linear_swiglu(h.rows, self.w_gate_up, row_sumsq=h.sumsq, norm_width=h.width, eps=h.eps, **self.act)
+                   if isinstance(h, ScaledRows) else linear_swiglu(h, self.w_gate_up, **self.act))
         elif isinstance(h, ScaledRows):
             if not ops.skinny_supported(h.rows, self.w_gate_up.plain, self.dtype):
                 raise ops.KernelError("feed-forward: rows that wait for their normalisation need the kernel for few rows")
@@ -132,8 +137,8 @@ class SwiGLU(Part):
             # from 12 rows on the product cut over K and the norm kernel that adds its planes are faster
             # than the weight-streaming product with that norm in its epilogue (30 against 35 us)
             return linear_planes(act, self.w_down)
-        if into is not None and act.dtype == torch.bfloat16 and skinny_takes(act.shape[0], self.w_down, preferred=True):
-            # only where the kernel for few rows is the faster one for this product anyway
+        if into is not None and (act.dtype == torch.float32 or skinny_takes(act.shape[0], self.w_down, preferred=True)):
+            # (bfloat16:) only where the kernel for few rows is the faster one for this product anyway
             fused = end_in_norm(act, self.w_down, into)
             if fused is not None:
                 return fused

@@ -101,6 +101,8 @@ def linear_swiglu(h, weight: Union[torch.Tensor, Weight], row_sumsq=None, norm_w
     the limited activation."""
     weight, packed = _split(weight)
     kw = dict(act, row_sumsq=row_sumsq, norm_width=norm_width, eps=eps) if row_sumsq is not None else act
+    if h.dtype == torch.float32:
+        return ops.gemm_skinny_f32(h, weight, swiglu=True, **kw)
     if packed is not None and packed.shape[0] % 32 == 0 and wavek_takes(h, packed, swiglu=True):
         return ops.gemm_wavek(h, packed, swiglu=True, **kw)
     if packed is not None:
@@ -114,10 +116,21 @@ def wavek_swiglu_takes(h: torch.Tensor, weight: Union[torch.Tensor, Weight]) -> 
     return packed is not None and packed.shape[0] % 32 == 0 and h.dtype == torch.bfloat16 and h.dim() == 2 and wavek_takes(h, packed, swiglu=True)
 
 
+def f32_takes_scaled_rows(weight: Union[torch.Tensor, Weight]) -> bool:
+    """Whether the 32-bit product takes this matrix with rows that wait for their normalisation.  It asks nothing of the number of rows:
+    a 32-bit model computes the same for a token however many are with it."""
+    w = _split(weight)[0]
+    return (w.dtype == torch.float32 and w.is_cuda and w.dim() == 2 and w.shape[1] % 4 == 0 and w.stride(1) == 1 and w.stride(0) % 4 == 0
+            and w.data_ptr() % 16 == 0)
+
+
 def linear_scaled(rows, weight: Union[torch.Tensor, Weight], out_dtype: Optional[torch.dtype] = None):
     """``rows.rows @ weight.T`` with the rows' normalisation applied in the epilogue (``rows``: ScaledRows)."""
     weight, packed = _split(weight)
     kw = dict(row_sumsq=rows.sumsq, norm_width=rows.width, eps=rows.eps, out_dtype=out_dtype)
+    if rows.rows.dtype == torch.float32:
+        del kw["out_dtype"]
+        return ops.gemm_skinny_f32(rows.rows, weight, **kw)
     if packed is not None and wavek_takes(rows.rows, packed):
         return ops.gemm_wavek(rows.rows, packed, **kw)
     if packed is not None:
@@ -265,6 +278,11 @@ def linear_into_norm(a: torch.Tensor, weight: Union[torch.Tensor, Weight], resid
     not take these operands (then nothing has been done)."""
     whole = weight
     weight, packed = _split(weight)
+    if a.dtype == torch.float32:
+        if not (f32_takes_scaled_rows(weight) and ops.skinny_f32_supported(a, weight, torch.float32) and residual.dtype == torch.float32
+                and residual.stride(1) == 1 and norm_weight.dtype == torch.float32):
+            return None
+        return ops.gemm_skinny_f32_add_norm(a, weight, residual, norm_weight, scale=scale)
     if not (a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and residual.dtype == torch.float32
             and norm_weight.dtype in (torch.bfloat16, torch.float32)):
         return None
