@@ -142,8 +142,8 @@ struct KVFrag {
 // stream_load), so that they do not displace the weights' neighbours and the rows in the caches.
 constexpr int DEC_STREAM = 2;
 
-// The numbers of the two pages that hold the keys k0 .. k0+15 and k0+16 .. k0+31 (k0 the same in
-// all lanes: the table is read through the scalar unit).
+// The numbers of the two pages that hold the keys k0 .. k0+15 and k0+16 .. k0+31 (where k0 is a scalar, the table is read through the
+// scalar unit).
 __device__ __forceinline__ void kv_pages(int (&pid)[2], const int *__restrict__ bt, int max_pages, int page, int k0) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -183,18 +183,15 @@ __device__ __forceinline__ void load_kv(KVFrag<DH> &f, const bf16_t *__restrict_
     }
 }
 
-// The same loads with a full address in every lane (the block table is read by the lanes too).
+// The same loads with a full address in every lane (pid: the two pages, read by the lanes too).
 template <int DH>
-__device__ __forceinline__ void load_kv_flat(KVFrag<DH> &f, const bf16_t *__restrict__ cache, const int *__restrict__ bt,
-                                             int max_pages, int page, size_t page_elems, int nkvh, int kvh, int k0, int l16,
+__device__ __forceinline__ void load_kv_flat(KVFrag<DH> &f, const bf16_t *__restrict__ cache, const int (&pid)[2], int page, size_t page_elems, int nkvh, int kvh, int k0, int l16,
                                              int grp) {
     const size_t v_off = (size_t)nkvh * DH * page + (size_t)kvh * DH * page + 4 * grp;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const int j = k0 + 16 * t;
-        int pi = j / page;
-        pi = pi < max_pages ? pi : max_pages - 1;       // a tile beyond the context is masked; keep the read in bounds
-        const bf16_t *pg = cache + (size_t)bt[pi] * page_elems;
+        const bf16_t *pg = cache + (size_t)pid[t] * page_elems;
         const int tok0 = j % page;
         const bf16_t *kp = pg + ((size_t)kvh * (DH / 8) * page + tok0 + l16) * 8;
 #pragma unroll
@@ -360,7 +357,9 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
                         const int *__restrict__ q_start, const int *__restrict__ ctx_len,
                         const int *__restrict__ req_list, int nh, int nkvh, int page, float scale_log2, int window,
                         int n_splits, float *__restrict__ part_o, float *__restrict__ part_ml SCORE_KPARAMS) {
-    extern __shared__ float lds[];                 // [waves][16][DH] outputs, then [waves][16][2] (m, l)
+    // [waves][16][DH + 4] outputs, then [waves][16][2] (m, l).  The four words more a row spread the sixteen rows over the banks
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    constexpr int PITCH = DH + 4;
     const int g = nh / nkvh;
     const int chunks = (g + 15) / 16;
     const int ri = blockIdx.x / (nkvh * chunks);
@@ -373,6 +372,10 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     const int lane = threadIdx.x & (WAVE - 1), wave = FLAT ? threadIdx.x / WAVE : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int l16 = lane & 15, grp = lane >> 4;
     const int rows = (g - 16 * chunk) < 16 ? (g - 16 * chunk) : 16;
+    const int *bt = block_table + (size_t)r * max_pages;
+    int pid[2];
+    // without a window a request's one part begins with its first key: its pages are asked for together with its length
+    if (FLAT && window == 0) kv_pages(pid, bt, max_pages, page, wave * 32);
     const int token = q_start[r];
     const int p = ctx_len[r] - 1;
     const int lo = first_key(p, window);
@@ -390,7 +393,6 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     st.cap_out = cap_out;
 #endif
     const int p_row[1] = {p}, lo_row[1] = {lo};
-    const int *bt = block_table + (size_t)r * max_pages;
     const size_t page_elems = kv_page_elems(nkvh, DH, page);
 
     // this split's share of the 32-key steps, the waves in turn
@@ -401,12 +403,19 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     KVFrag<DH> fa, fb;
     if (FLAT) {
         int blk = b0 + wave;
-        if (blk < b1) load_kv_flat<DH>(fa, cache, bt, max_pages, page, page_elems, nkvh, kvh, blk * 32, l16, grp);
+        if (window != 0) kv_pages(pid, bt, max_pages, page, blk * 32);
+        if (blk < b1) load_kv_flat<DH>(fa, cache, pid, page, page_elems, nkvh, kvh, blk * 32, l16, grp);
         for (; blk < b1; blk += 2 * DEC_WAVES) {
             const int nb = blk + DEC_WAVES, nb2 = blk + 2 * DEC_WAVES;
-            if (nb < b1) load_kv_flat<DH>(fb, cache, bt, max_pages, page, page_elems, nkvh, kvh, nb * 32, l16, grp);
+            if (nb < b1) {
+                kv_pages(pid, bt, max_pages, page, nb * 32);
+                load_kv_flat<DH>(fb, cache, pid, page, page_elems, nkvh, kvh, nb * 32, l16, grp);
+            }
             attn_block<DH, 1>(fa, blk * 32, blk * 32 + 31 > p || blk * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
-            if (nb2 < b1) load_kv_flat<DH>(fa, cache, bt, max_pages, page, page_elems, nkvh, kvh, nb2 * 32, l16, grp);
+            if (nb2 < b1) {
+                kv_pages(pid, bt, max_pages, page, nb2 * 32);
+                load_kv_flat<DH>(fa, cache, pid, page, page_elems, nkvh, kvh, nb2 * 32, l16, grp);
+            }
             if (nb < b1)
                 attn_block<DH, 1>(fb, nb * 32, nb * 32 + 31 > p || nb * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
         }
@@ -431,46 +440,59 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
                 attn_block<DH, 1>(fb, nb * 32, nb * 32 + 31 > p || nb * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
         }
     }
-    // ---- merge the waves
+    // ---- merge the waves (rows that are no head are not looked at).  What bounds the kernel over few keys is the way from one load to the
+    // next and this merge: one MI355X, inside a step, 16 requests of 64 to 206 keys, 16 heads of 128 over 4: 9.6 us with a word a lane and
+    // store and sixteen rows in the same bank, the pages asked for after the length; 7.9 us now (32 requests of 20 to 116 keys: 10.3, 7.9).
     float l_all = st.l[0];
     l_all += __shfl_xor(l_all, 16, WAVE);
     l_all += __shfl_xor(l_all, 32, WAVE);
     float *lds_o = lds;
-    float *lds_ml = lds + DEC_WAVES * 16 * DH;
+    float *lds_ml = lds + DEC_WAVES * 16 * PITCH;
+    if (l16 < rows) {
 #pragma unroll
-    for (int dt = 0; dt < DH / 16; ++dt)
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) lds_o[((size_t)wave * 16 + l16) * DH + 16 * dt + 4 * grp + rr] = st.o[0][dt][rr];
-    if (grp == 0) {
-        lds_ml[(wave * 16 + l16) * 2 + 0] = st.m[0];
-        lds_ml[(wave * 16 + l16) * 2 + 1] = l_all;
+        for (int dt = 0; dt < DH / 16; ++dt) *(f32x4 *)(lds_o + (wave * 16 + l16) * PITCH + 16 * dt + 4 * grp) = st.o[0][dt];
+        if (grp == 0) {
+            lds_ml[(wave * 16 + l16) * 2 + 0] = st.m[0];
+            lds_ml[(wave * 16 + l16) * 2 + 1] = l_all;
+        }
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < rows * DH; idx += DEC_WAVES * WAVE) {
-        const int row = idx / DH, d = idx % DH;
+    const bool four = ((uintptr_t)out & 7) == 0;       // (out_stride is a multiple of four)
+    for (int idx = threadIdx.x; idx < rows * (DH / 4); idx += DEC_WAVES * WAVE) {
+        const int row = idx / (DH / 4), d = idx % (DH / 4) * 4;
         float M = -INFINITY;
 #pragma unroll
         for (int w = 0; w < DEC_WAVES; ++w) M = fmaxf(M, lds_ml[(w * 16 + row) * 2]);
         const float M_safe = M == -INFINITY ? 0.f : M;
-        float L = 0.f, val = 0.f;
+        float L = 0.f;
+        f32x4 val = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < DEC_WAVES; ++w) {
             const float f = exp2f(lds_ml[(w * 16 + row) * 2] - M_safe);
             L += lds_ml[(w * 16 + row) * 2 + 1] * f;
-            val += lds_o[((size_t)w * 16 + row) * DH + d] * f;
+            val += *(const f32x4 *)(lds_o + (w * 16 + row) * PITCH + d) * f;
         }
         const int head = head0 + row;
         if (n_splits == 1) {
+            bf16_t *to = out + (size_t)token * out_stride + (size_t)head * DH + d;
+            f32x4 o;
 #ifdef LCU_SCORE_BIAS
-            if (sinks) {
-                out[(size_t)token * out_stride + (size_t)head * DH + d] = from_f32<bf16_t>(val * sink_share(M_safe, L, sinks[head]));
-                continue;
-            }
+            const float share = sinks ? sink_share(M_safe, L, sinks[head]) : 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = sinks ? val[e] * share : val[e] / L;
+#else
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = val[e] / L;
 #endif
-            out[(size_t)token * out_stride + (size_t)head * DH + d] = from_f32<bf16_t>(val / L);
+            if (four) {
+                *(u32x2 *)to = u32x2{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) to[e] = from_f32<bf16_t>(o[e]);
+            }
         } else {
             const size_t slot = ((size_t)ri * nh + head) * n_splits + split;
-            part_o[slot * DH + d] = val;
+            *(f32x4 *)(part_o + slot * DH + d) = val;
             if (d == 0) { part_ml[slot * 2] = M; part_ml[slot * 2 + 1] = L; }
         }
     }
@@ -535,7 +557,7 @@ static int launch_decode(const void *q, int q_stride, void *out, int out_stride,
                          int n_splits, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
     const int g = nh / nkvh, chunks = (g + 15) / 16;
     const float scale_log2 = SCORE_LOG2(scale);
-    const size_t lds_bytes = (size_t)DEC_WAVES * 16 * (DH + 2) * sizeof(float);
+    const size_t lds_bytes = (size_t)DEC_WAVES * 16 * (DH + 4 + 2) * sizeof(float);
     dim3 grid(n_req * nkvh * chunks, n_splits), block(DEC_WAVES * WAVE);
     // Two ways to address the pages (the same arithmetic, the same results).  FLAT: every lane holds
     // full addresses and reads the block table itself.  Not FLAT: the wave's number and with it the

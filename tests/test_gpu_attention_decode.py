@@ -1,0 +1,33 @@
+"""The decode kernel's merge of its waves: outputs that cannot be stored four at a time are the same bits as those that can, and both are
+the generic kernel's numbers up to rounding, with and without a window (whose first keys lie anywhere)."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from divasun_common import assert_close
+from test_gpu_divasun import rnd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nh,nkv,dh", [(4, 4, 32), (16, 4, 128), (20, 1, 64), (34, 2, 96)])
+@pytest.mark.parametrize("window,splits", [(0, 1), (0, 3), (50, 1)])
+def test_stores(nh, nkv, dh, window, splits):
+    from llama_cu_amd.kernels import ops
+    ctx, page = [1, 31, 33, 128, 129, 290], 16
+    n, most = len(ctx), -(-max(ctx) // page)
+    cache = rnd(n * most + 1, 2, nkv * dh * page, seed=1).bfloat16().cuda()
+    table = (torch.randperm(n * most, generator=torch.Generator().manual_seed(2)) + 1).to(torch.int32).view(n, most).contiguous().cuda()
+    q = rnd(n, nh * dh, seed=3).bfloat16().cuda()
+    starts, of, lens = torch.arange(n + 1, dtype=torch.int32).cuda(), torch.arange(n, dtype=torch.int32).cuda(), torch.tensor(ctx, dtype=torch.int32).cuda()
+    scale = dh ** -0.5
+    even, odd = torch.empty(n, nh * dh, dtype=torch.bfloat16, device="cuda"), torch.zeros(n, nh * dh + 4, dtype=torch.bfloat16, device="cuda")
+    wanted = torch.empty_like(even)
+    ops.paged_attention_generic(q, wanted, cache, table, starts, lens, of, nh, nkv, dh, page, scale, window)
+    ops.attention_decode(q, even, cache, table, starts, lens, n, nh, nkv, dh, page, scale, window, splits)
+    assert_close(even, wanted, 3 * 2.0 ** -8, "against the generic kernel")        # the weights and both outputs rounded to bfloat16
+    if splits == 1:                                                                # (the kernel that adds parts stores four at a time only)
+        ops.attention_decode(q, odd[:, 2:2 + nh * dh], cache, table, starts, lens, n, nh, nkv, dh, page, scale, window, splits)
+        assert torch.equal(odd[:, 2:2 + nh * dh], even)
+        assert (odd[:, :2] == 0).all() and (odd[:, 2 + nh * dh:] == 0).all()
