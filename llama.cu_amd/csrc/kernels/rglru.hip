@@ -49,15 +49,43 @@ __device__ __forceinline__ float conv_at(const TI *__restrict__ rows, int row_st
     return acc;
 }
 
+// The same for up to four taps, without a loop: the loads of all taps, and of the elements that a thread makes one after the other, are on
+// their way together.
+template <class TI>
+__device__ __forceinline__ float conv_few(const TI *__restrict__ rows, int row_stride, int x_off, const float *__restrict__ bias,
+                                          const float *__restrict__ conv_w, const float *__restrict__ conv_b,
+                                          const float *__restrict__ st, int t, int t0, int first_pos, int c, int width, int taps) {
+    float here[4], before[4], w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int back = max(taps - 1 - j, 0), m = t0 - (t - back);
+        here[j] = to_f32(rows[(size_t)(m <= 0 ? t - back : t) * row_stride + x_off + c]);
+        before[j] = st[(size_t)(m > 0 && first_pos - m >= 0 ? taps - 1 - m : 0) * width + c];
+        w[j] = conv_w[(size_t)c * taps + min(j, taps - 1)];
+    }
+    const float bx = bias ? bias[x_off + c] : 0.f;
+    float acc = conv_b ? conv_b[c] : 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int back = taps - 1 - j, m = t0 - (t - back);
+        const float x = m <= 0 ? here[j] + bx : first_pos - m >= 0 ? before[j] : 0.f;
+        acc = j < taps ? acc + w[j] * x : acc;
+    }
+    return acc;
+}
+
 constexpr int RG_TOK = 8;          // tokens a workgroup of the gates kernel takes
 constexpr int RG_OUT = 32;         // output channels a workgroup takes
 constexpr int RG_SLICES = 8;       // parts into which the sum over a block's input channels is cut (one per 32 threads)
+constexpr int RG_AHEAD = 16;       // rows of the two matrices whose loads are on their way together
 constexpr int RG_MAX_BS = 1024;    // channels of a block (LDS holds RG_TOK rows of them)
 
 // The convolution and the gates.  A workgroup takes RG_TOK tokens, one block of channels and RG_OUT of its outputs: it
 // makes u for all the block's channels of its tokens (in LDS; workgroups of the same block make the same u), then each
 // of its eight groups of 32 threads sums over an eighth of the input channels, and the eight partial sums are added in
-// a fixed order.  So a decoding step, with few tokens, still has blocks x (bs / 32) workgroups.
+// a fixed order.  So a decoding step, with few tokens, still has blocks x (bs / 32) workgroups.  Latency bounds it: the matrices' rows are asked
+// for before u is made, sixteen at a time, the next sixteen during the sums of these (one MI355X, 8 tokens, width 2048 in 16 blocks, 4 taps: 12.5 us with a loop over
+// the taps and the gates' own vectors asked for at the end, 8.1 us).
 template <class TI>
 __global__ void __launch_bounds__(RG_OUT * RG_SLICES)
 rglru_gates_kernel(const TI *__restrict__ rows, int row_stride, int x_off, const float *__restrict__ bias,
@@ -72,47 +100,67 @@ rglru_gates_kernel(const TI *__restrict__ rows, int row_stride, int x_off, const
     __shared__ float part[RG_SLICES][RG_TOK][2][RG_OUT];
     const int b = blockIdx.y, tok0 = blockIdx.x * RG_TOK, o0 = blockIdx.z * RG_OUT;
     const int nt = min(RG_TOK, n - tok0);
-#pragma unroll 4
-    for (int w = threadIdx.x; w < RG_TOK * bs; w += blockDim.x) {
-        const int tt = w / bs, i = w % bs;
-        float u = 0.f;
-        if (tt < nt) {
-            const int t = tok0 + tt, r = req_of_token[t], t0 = q_start[r];
-            const int first_pos = ctx_len[r] - (q_start[r + 1] - t0);
-            u = conv_at(rows, row_stride, x_off, bias, conv_w, conv_b, state + (size_t)state_slot[r] * taps * width, t, t0,
-                        first_pos, b * bs + i, width, taps);
-        }
-        us[tt][i] = u;
-    }
-    __syncthreads();
     const int og = threadIdx.x % RG_OUT, slice = threadIdx.x / RG_OUT, o = o0 + og;
     const int per = (bs + RG_SLICES - 1) / RG_SLICES;
     const int i0 = slice * per, i1 = min(bs, i0 + per);
+    const float *wa = wa_t + (size_t)b * bs * bs + min(o, bs - 1), *wi = wi_t + (size_t)b * bs * bs + min(o, bs - 1);
+    const bool fours = per % 4 == 0 && bs % 4 == 0;
+    float a[2][RG_AHEAD], g[2][RG_AHEAD];
+    auto fetch = [&](int u, int i) {                 // (a row beyond the end is the last one, and is not used)
+#pragma unroll
+        for (int e = 0; e < RG_AHEAD; ++e) {
+            a[u][e] = wa[(size_t)min(i + e, bs - 1) * bs];
+            g[u][e] = wi[(size_t)min(i + e, bs - 1) * bs];
+        }
+    };
+    if (fours) fetch(0, i0);                         // on their way while u is made
+    // what a thread needs in the end for its token (its slice's number) and channel
+    const int c = b * bs + min(o, bs - 1);
+    const size_t y_at = (size_t)(tok0 + min(slice, nt - 1)) * row_stride + y_off + c;
+    const float l = lam[c], ba_c = ba[c], bi_c = bi[c], y_in = to_f32(rows[y_at]) + (bias ? bias[y_off + c] : 0.f);
+    // (a token beyond the end is the last one, made once more and not used)
+    auto make = [&](int w, auto conv) {
+        const int t = tok0 + min(w / bs, nt - 1), r = req_of_token[t], t0 = q_start[r];
+        const int first_pos = ctx_len[r] - (q_start[r + 1] - t0);
+        us[w / bs][w % bs] = conv(rows, row_stride, x_off, bias, conv_w, conv_b, state + (size_t)state_slot[r] * taps * width, t, t0,
+                                  first_pos, b * bs + w % bs, width, taps);
+    };
+    if (taps <= 4) {
+#pragma unroll 4
+        for (int w = threadIdx.x; w < RG_TOK * bs; w += RG_OUT * RG_SLICES) make(w, conv_few<TI>);
+    } else {
+        for (int w = threadIdx.x; w < RG_TOK * bs; w += RG_OUT * RG_SLICES) make(w, conv_at<TI>);
+    }
+    __syncthreads();
     float ra[RG_TOK], ri[RG_TOK];
 #pragma unroll
     for (int tt = 0; tt < RG_TOK; ++tt) ra[tt] = ri[tt] = 0.f;
-    if (o < bs) {
-        const float *wa = wa_t + (size_t)b * bs * bs + o, *wi = wi_t + (size_t)b * bs * bs + o;
-        int i = i0;
-        if (per % 4 == 0 && bs % 4 == 0) {
-            for (; i + 4 <= i1; i += 4) {
-                float a[4], g[4];
+    if (fours) {
+        for (int i = i0; i < i1; i += 2 * RG_AHEAD) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { a[e] = wa[(size_t)(i + e) * bs]; g[e] = wi[(size_t)(i + e) * bs]; }
+            for (int u = 0; u < 2; ++u) {
+                const int j = i + u * RG_AHEAD;
+                if (j >= i1) break;
+                if (j + RG_AHEAD < i1) fetch(u ^ 1, j + RG_AHEAD);
 #pragma unroll
-                for (int tt = 0; tt < RG_TOK; ++tt) {
-                    const float4 u = *(const float4 *)&us[tt][i];
-                    ra[tt] += a[0] * u.x; ra[tt] += a[1] * u.y; ra[tt] += a[2] * u.z; ra[tt] += a[3] * u.w;
-                    ri[tt] += g[0] * u.x; ri[tt] += g[1] * u.y; ri[tt] += g[2] * u.z; ri[tt] += g[3] * u.w;
+                for (int q = 0; q < RG_AHEAD; q += 4) {
+                    if (j + q >= i1) break;
+#pragma unroll
+                    for (int tt = 0; tt < RG_TOK; ++tt) {
+                        const float4 x = *(const float4 *)&us[tt][j + q];
+                        ra[tt] += a[u][q] * x.x; ra[tt] += a[u][q + 1] * x.y; ra[tt] += a[u][q + 2] * x.z; ra[tt] += a[u][q + 3] * x.w;
+                        ri[tt] += g[u][q] * x.x; ri[tt] += g[u][q + 1] * x.y; ri[tt] += g[u][q + 2] * x.z; ri[tt] += g[u][q + 3] * x.w;
+                    }
                 }
             }
         }
-        for (; i < i1; ++i) {
-            const float a = wa[(size_t)i * bs], g = wi[(size_t)i * bs];
+    } else {
+        for (int i = i0; i < i1; ++i) {
+            const float wa1 = wa[(size_t)i * bs], wi1 = wi[(size_t)i * bs];
 #pragma unroll
             for (int tt = 0; tt < RG_TOK; ++tt) {
-                ra[tt] += a * us[tt][i];
-                ri[tt] += g * us[tt][i];
+                ra[tt] += wa1 * us[tt][i];
+                ri[tt] += wi1 * us[tt][i];
             }
         }
     }
@@ -130,16 +178,14 @@ rglru_gates_kernel(const TI *__restrict__ rows, int row_stride, int x_off, const
         sa += part[k][tt][0][og];
         si += part[k][tt][1][og];
     }
-    const int c = b * bs + o;
-    const float l = lam[c];
     const float sp = l > 20.f ? l : log1pf(expf(l));          // softplus
-    const float r = 1.0f / (1.0f + expf(-(sa + ba[c])));
-    const float gate = 1.0f / (1.0f + expf(-(si + bi[c])));
+    const float r = 1.0f / (1.0f + expf(-(sa + ba_c)));
+    const float gate = 1.0f / (1.0f + expf(-(si + bi_c)));
     const float log_a = -c_exp * r * sp;
     const float mult = sqrtf(-expm1f(2.0f * log_a));
     a_out[tile_index(tok0 + tt, c, n)] = expf(log_a);
     gx_out[tile_index(tok0 + tt, c, n)] = mult * gate * us[tt][o];
-    y_out[tile_index(tok0 + tt, c, n)] = gelu_tanh(to_f32(rows[(size_t)(tok0 + tt) * row_stride + y_off + c]) + (bias ? bias[y_off + c] : 0.f));
+    y_out[tile_index(tok0 + tt, c, n)] = gelu_tanh(y_in);
 }
 
 constexpr int RG_BATCH = 16;       // tokens whose loads the scan has in flight at a time
