@@ -83,9 +83,10 @@ constexpr int RG_MAX_BS = 1024;    // channels of a block (LDS holds RG_TOK rows
 // The convolution and the gates.  A workgroup takes RG_TOK tokens, one block of channels and RG_OUT of its outputs: it
 // makes u for all the block's channels of its tokens (in LDS; workgroups of the same block make the same u), then each
 // of its eight groups of 32 threads sums over an eighth of the input channels, and the eight partial sums are added in
-// a fixed order.  So a decoding step, with few tokens, still has blocks x (bs / 32) workgroups.  Latency bounds it: the matrices' rows are asked
-// for before u is made, sixteen at a time, the next sixteen during the sums of these (one MI355X, 8 tokens, width 2048 in 16 blocks, 4 taps: 12.5 us with a loop over
-// the taps and the gates' own vectors asked for at the end, 8.1 us).
+// a fixed order.  So a decoding step, with few tokens, still has blocks x (bs / 32) workgroups.  Latency bounds it: the
+// matrices' rows are asked for before u is made, sixteen at a time, the next sixteen during the sums of these (one MI355X,
+// 8 tokens, width 2048 in 16 blocks, 4 taps: 12.5 us with a loop over the taps and the gates' own vectors asked for at the
+// end, 8.1 us now).
 template <class TI>
 __global__ void __launch_bounds__(RG_OUT * RG_SLICES)
 rglru_gates_kernel(const TI *__restrict__ rows, int row_stride, int x_off, const float *__restrict__ bias,
