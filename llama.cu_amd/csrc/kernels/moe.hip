@@ -154,7 +154,9 @@ moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, cons
             const float best = wave_max_in_place(mine);
             const unsigned long long who = __ballot(lane < n_experts && mine == best);
             arg = who ? __ffsll((long long)who) - 1 : 0;     // the lowest of equals; every logit NaN: any expert
-            value = mode == 2 ? sc[arg] : z[arg];
+            // where fewer logits are finite than experts are chosen, what is left may be an expert that was chosen already: it comes with
+            // the -inf that stands in its place now, and so with no weight
+            value = mode == 2 ? sc[arg] : who ? best : z[arg];
             if (lane == arg) mine = -INFINITY;
         } else {
             float best = -INFINITY;

@@ -208,6 +208,26 @@ def test_router_ties_go_to_the_lower_index_and_the_weight_multiplies_the_input()
     assert abs(out[0, 0].item() - want) < 1e-5
 
 
+@pytest.mark.parametrize("experts,top,open_", [(4, 2, 1), (4, 4, 2), (64, 5, 3), (65, 5, 3), (64, 64, 7), (4, 2, 0)])
+def test_experts_that_a_bias_shuts_off_have_no_weight(experts, top, open_):
+    """A bias of -inf on all but ``open_`` experts, fewer than are chosen: each open one has its weight once, the others none."""
+    from llama_cu_amd.kernels import ops
+    h, router = rnd(3, 16, seed=1), rnd(experts, 16, seed=2)
+    which = torch.cat([torch.zeros(1, dtype=torch.long), torch.randperm(experts - 1, generator=torch.Generator().manual_seed(3)) + 1])[:open_]
+    bias = torch.full((experts,), -math.inf)
+    bias[which] = rnd(open_, seed=4)
+    z = (h.to(F64) @ router.to(F64).T)[:, which] + bias[which].to(F64)
+    for softmax, want in ((False, torch.sigmoid(z)), (True, torch.softmax(z, 1))):
+        if softmax and not open_:
+            continue                                   # (a softmax over nothing)
+        ids, wts = ops.moe_route(h.cuda(), router.cuda(), top, bias=bias.cuda(), softmax_chosen=softmax)
+        assert int(ids.min()) >= 0 and int(ids.max()) < experts
+        total = torch.zeros(3, experts, dtype=F64).scatter_add_(1, ids.long().cpu(), wts.to(F64).cpu())
+        full = torch.zeros(3, experts, dtype=F64)
+        full[:, which] = want
+        assert float((total - full).abs().max()) < 1e-5
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("nh,nkv,dh,dv,page", [(6, 2, 24, 16, 8), (4, 1, 64, 64, 16), (2, 2, 16, 40, 16)])
 def test_attention_norm_temperature_bias_and_values_of_their_own_size(dtype, nh, nkv, dh, dv, page):
