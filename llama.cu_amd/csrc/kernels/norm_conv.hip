@@ -51,8 +51,11 @@ layernorm_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes
 // A row's elements in one thread's registers: PT pieces of V neighbours, ROW_THREADS pieces apart.  The row takes in the planes
 // of delta, is written back, and its mean and the inverse of its deviation come out.  A step of few rows is a chain of dependent
 // trips to memory and through the barriers: one trip, two barriers.
+// V is 4 where d is a multiple of 4, else 1, and the number of threads is fixed: which elements a thread adds, and so a row's bits, depend on d
+// alone.  (A 32-bit model gives a token the same bits in a portion, whose norm and convolution are kernels of their own, and alone.)  WIDE:
+// every address lets four elements be read at once.
 constexpr int ROW_THREADS = 512;
-template <class TD, int V, int PT>
+template <class TD, int V, int PT, bool WIDE>
 __device__ __forceinline__ void take_row(float *xr, const TD *delta, int planes, size_t plane_stride, size_t row_at, int d, float eps,
                                          float (&v)[PT][V], float &mean, float &rstd, float (*scratch)[16]) {
     float sum = 0.f;
@@ -62,15 +65,15 @@ __device__ __forceinline__ void take_row(float *xr, const TD *delta, int planes,
 #pragma unroll
         for (int e = 0; e < V; ++e) v[i][e] = 0.f;
         if (c < d) {
-            load_as_f32<float, V>(xr + c, v[i]);
+            load_some<float, V, WIDE>(xr + c, v[i]);
             if (delta) {
                 for (int p = 0; p < planes; ++p) {
                     float more[V];
-                    load_as_f32<TD, V>(delta + p * plane_stride + row_at + c, more);
+                    load_some<TD, V, WIDE>(delta + p * plane_stride + row_at + c, more);
 #pragma unroll
                     for (int e = 0; e < V; ++e) v[i][e] += more[e];
                 }
-                store_f32<float, V>(xr + c, v[i]);
+                store_some<float, V, WIDE>(xr + c, v[i]);
             }
 #pragma unroll
             for (int e = 0; e < V; ++e) sum += v[i][e];
@@ -88,10 +91,9 @@ __device__ __forceinline__ void take_row(float *xr, const TD *delta, int planes,
     rstd = rsqrtf(row_sum(sq, scratch[1]) / (float)d + eps);
 }
 
-// The same for rows of up to ROW_THREADS * V * PT elements: the row stays in registers between its one read and its writes.  V is 4
-// where d is a multiple of 4 and every pointer is aligned for it (2,048 rows of 2,048 with two 32-bit outputs 21.8 -> 14.2 us, one
-// row 5.5 -> 2.3), else 1.
-template <class TD, class TO, int V, int PT>
+// The same for rows of up to ROW_THREADS * V * PT elements: the row stays in registers between its one read and its writes.  With 256
+// threads and single elements 2,048 rows of 2,048 with two 32-bit outputs took 21.8 us, now 14.2, one row 5.5, now 2.3.
+template <class TD, class TO, int V, int PT, bool WIDE>
 __global__ void __launch_bounds__(ROW_THREADS)
 layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes, size_t plane_stride,
                      const float *__restrict__ w1, const float *__restrict__ b1, TO *__restrict__ out1,
@@ -104,15 +106,15 @@ layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int pl
     for (int i = 0; i < PT; ++i) {
         const int c = (threadIdx.x + ROW_THREADS * i) * V;
         if (c < d) {
-            load_as_f32<float, V>(w1 + c, w[0][i]);
-            load_as_f32<float, V>(b1 + c, b[0][i]);
+            load_some<float, V, WIDE>(w1 + c, w[0][i]);
+            load_some<float, V, WIDE>(b1 + c, b[0][i]);
             if (w2) {
-                load_as_f32<float, V>(w2 + c, w[1][i]);
-                load_as_f32<float, V>(b2 + c, b[1][i]);
+                load_some<float, V, WIDE>(w2 + c, w[1][i]);
+                load_some<float, V, WIDE>(b2 + c, b[1][i]);
             }
         }
     }
-    take_row<TD, V, PT>(x + row_at, delta, planes, plane_stride, row_at, d, eps, v, mean, rstd, scratch);
+    take_row<TD, V, PT, WIDE>(x + row_at, delta, planes, plane_stride, row_at, d, eps, v, mean, rstd, scratch);
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
         const int c = (threadIdx.x + ROW_THREADS * i) * V;
@@ -120,11 +122,11 @@ layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int pl
         float y[V];
 #pragma unroll
         for (int e = 0; e < V; ++e) y[e] = (v[i][e] - mean) * rstd * w[0][i][e] + b[0][i][e];
-        store_f32<TO, V>(out1 + row_at + c, y);
+        store_some<TO, V, WIDE>(out1 + row_at + c, y);
         if (w2) {
 #pragma unroll
             for (int e = 0; e < V; ++e) y[e] = (v[i][e] - mean) * rstd * w[1][i][e] + b[1][i][e];
-            store_f32<TO, V>(out2 + row_at + c, y);
+            store_some<TO, V, WIDE>(out2 + row_at + c, y);
         }
     }
 }
@@ -138,15 +140,16 @@ LCU_API int lcu_layernorm(float *x, const void *delta, int delta_type, int plane
     const size_t stride = (size_t)n * d;
     dim3 grid(n), block(NC_THREADS);
     const int dt = delta ? delta_type : LCU_F32;
-    const bool four = d % 4 == 0 && four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) && four_ok(out1, out_type) &&
+    const bool four = d % 4 == 0;
+    const bool wide = four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) && four_ok(out1, out_type) &&
                       four_ok(w2, LCU_F32) && four_ok(b2, LCU_F32) && four_ok(out2, out_type);
-#define ROW(TD, TO, V, PT) layernorm_row_kernel<TD, TO, V, PT><<<grid, dim3(ROW_THREADS), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
+#define ROW(TD, TO, V, PT, WIDE) layernorm_row_kernel<TD, TO, V, PT, WIDE><<<grid, dim3(ROW_THREADS), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
 #define GO(TD, TO)                                                                                                           \
     do {                                                                                                                     \
-        if (four && d <= 4 * ROW_THREADS) ROW(TD, TO, 4, 1);                                                                 \
-        else if (four && d <= 8 * ROW_THREADS) ROW(TD, TO, 4, 2);                                                            \
-        else if (d <= 2 * ROW_THREADS) ROW(TD, TO, 1, 2);                                                                    \
-        else if (d <= 8 * ROW_THREADS) ROW(TD, TO, 1, 8);                                                                    \
+        if (four && d <= 4 * ROW_THREADS) { if (wide) ROW(TD, TO, 4, 1, true); else ROW(TD, TO, 4, 1, false); }              \
+        else if (four && d <= 8 * ROW_THREADS) { if (wide) ROW(TD, TO, 4, 2, true); else ROW(TD, TO, 4, 2, false); }         \
+        else if (d <= 2 * ROW_THREADS) ROW(TD, TO, 1, 2, false);                                                             \
+        else if (d <= 8 * ROW_THREADS) ROW(TD, TO, 1, 8, false);                                                             \
         else layernorm_kernel<TD, TO><<<grid, block, 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1,  \
                                                                   w2, b2, (TO *)out2, d, eps);                               \
     } while (0)
@@ -262,11 +265,11 @@ LCU_API int lcu_short_conv(const void *h, int h_type, long long set_stride_h, co
 // convolutions from the requests' states, and the states' update, with the row in registers throughout.  A block
 // is the only reader and writer of its request's state, and a thread of its channels'.
 // out: [sets][n, d] of TO; state: [slots, sets, taps - 1, d]; cw: [sets][d, taps] 32-bit.
-// Everything that is read is read before the row's sums are made: one trip to memory.  V as above, and 4 for four taps only (element
-// e's taps are then the numbers 4 e .. of a thread's sixteen); up to FUSED_TAPS taps.  With 256 threads, single numbers and the two sets
-// one after the other four rows of 2,048 with four taps took 13.8 us, now 5.0.
+// Everything that is read is read before the row's sums are made: one trip to memory.  V and WIDE as above; TAPS: the number
+// of taps where a thread reads its 4 TAPS weights in pieces of four, or 0 (one by one, up to FUSED_TAPS).  With 256 threads,
+// single numbers and the two sets one after the other four rows of 2,048 with four taps took 13.8 us, now 5.0.
 constexpr int FUSED_TAPS = 8;
-template <class TD, class TO, int V, int PT>
+template <class TD, class TO, int V, int PT, bool WIDE, int TAPS>
 __global__ void __launch_bounds__(ROW_THREADS)
 norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes, size_t plane_stride,
                         const float *__restrict__ w1, const float *__restrict__ b1, const float *__restrict__ w2,
@@ -274,12 +277,13 @@ norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int
                         TO *__restrict__ out, size_t set_stride_out, const int *__restrict__ ctx_len,
                         const int *__restrict__ state_slot, int d, int taps_rt, int sets, float eps) {
     __shared__ float scratch[2][16];
-    const int taps = V == 4 ? 4 : taps_rt;
+    const int taps = TAPS ? TAPS : taps_rt;
+    constexpr int MOST = TAPS ? TAPS : FUSED_TAPS;
     const int r = blockIdx.x;
     const int pos = ctx_len[r] - 1;                  // the token's position
     float *slot = st + (size_t)state_slot[r] * sets * (taps - 1) * d;
     float v[PT][V], mean, rstd;
-    float old[2][PT][FUSED_TAPS - 1][V], k[2][PT][V * FUSED_TAPS], wv[2][PT][V], bv[2][PT][V];
+    float old[2][PT][MOST > 1 ? MOST - 1 : 1][V], k[2][PT][V][MOST], wv[2][PT][V], bv[2][PT][V];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         if (s >= sets) break;
@@ -288,21 +292,33 @@ norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int
         for (int i = 0; i < PT; ++i) {
             const int c = (threadIdx.x + ROW_THREADS * i) * V;
             if (c >= d) continue;
-            load_as_f32<float, V>(w + c, wv[s][i]);
-            load_as_f32<float, V>(b + c, bv[s][i]);
-            const float *kc = cw + ((size_t)s * d + c) * taps;             // V * taps numbers: taps pieces of V
+            load_some<float, V, WIDE>(w + c, wv[s][i]);
+            load_some<float, V, WIDE>(b + c, bv[s][i]);
+            const float *kc = cw + ((size_t)s * d + c) * taps;
+            if constexpr (WIDE && TAPS > 0) {                              // V * TAPS numbers in a row: TAPS pieces of four
 #pragma unroll
-            for (int j = 0; j < FUSED_TAPS; ++j)
-                if (j < taps) load_as_f32<float, V>(kc + j * V, k[s][i] + j * V);
+                for (int q = 0; q < TAPS; ++q) {
+                    float piece[4];
+                    load_as_f32<float, 4>(kc + 4 * q, piece);
 #pragma unroll
-            for (int j = 0; j < FUSED_TAPS - 1; ++j) {                     // row j of the state lies taps - 1 - j positions before the token
+                    for (int u = 0; u < 4; ++u) k[s][i][(4 * q + u) / TAPS][(4 * q + u) % TAPS] = piece[u];
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < V; ++e)
+#pragma unroll
+                    for (int j = 0; j < MOST; ++j)
+                        if (j < taps) k[s][i][e][j] = kc[e * taps + j];
+            }
+#pragma unroll
+            for (int j = 0; j < MOST - 1; ++j) {                     // row j of the state lies taps - 1 - j positions before the token
 #pragma unroll
                 for (int e = 0; e < V; ++e) old[s][i][j][e] = 0.f;
-                if (j < taps - 1 && pos - (taps - 1 - j) >= 0) load_as_f32<float, V>(state + (size_t)j * d + c, old[s][i][j]);
+                if (j < taps - 1 && pos - (taps - 1 - j) >= 0) load_some<float, V, WIDE>(state + (size_t)j * d + c, old[s][i][j]);
             }
         }
     }
-    take_row<TD, V, PT>(x + (size_t)r * d, delta, planes, plane_stride, (size_t)r * d, d, eps, v, mean, rstd, scratch);
+    take_row<TD, V, PT, WIDE>(x + (size_t)r * d, delta, planes, plane_stride, (size_t)r * d, d, eps, v, mean, rstd, scratch);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         if (s >= sets) break;
@@ -316,16 +332,14 @@ norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int
             for (int e = 0; e < V; ++e) acc[e] = h[e] = (v[i][e] - mean) * rstd * wv[s][i][e] + bv[s][i][e];
             // (the order of short_conv_kernel's additions)
 #pragma unroll
-            for (int j = 0; j < FUSED_TAPS; ++j) {
+            for (int j = 0; j < MOST; ++j) {
                 if (j >= taps) break;
 #pragma unroll
-                for (int e = 0; e < V; ++e) {
-                    acc[e] += k[s][i][V == 4 ? e * 4 + j : j] * (j == taps - 1 ? h[e] : old[s][i][j < FUSED_TAPS - 1 ? j : 0][e]);
-                }
-                if (j > 0 && j < taps - 1) store_f32<float, V>(state + (size_t)(j - 1) * d + c, old[s][i][j < FUSED_TAPS - 1 ? j : 0]);     // row j becomes row j - 1
+                for (int e = 0; e < V; ++e) acc[e] += k[s][i][e][j] * (j == taps - 1 ? h[e] : old[s][i][j < MOST - 1 ? j : 0][e]);
+                if (j > 0 && j < taps - 1) store_some<float, V, WIDE>(state + (size_t)(j - 1) * d + c, old[s][i][j < MOST - 1 ? j : 0]);     // row j becomes row j - 1
             }
-            if (taps > 1) store_f32<float, V>(state + (size_t)(taps - 2) * d + c, h);
-            store_f32<TO, V>(out + s * set_stride_out + (size_t)r * d + c, acc);
+            if (taps > 1) store_some<float, V, WIDE>(state + (size_t)(taps - 2) * d + c, h);
+            store_some<TO, V, WIDE>(out + s * set_stride_out + (size_t)r * d + c, acc);
         }
     }
 }
@@ -341,13 +355,21 @@ LCU_API int lcu_norm_conv_single(float *x, const void *delta, int delta_type, in
     const size_t stride = (size_t)n * d;
     dim3 grid(n);
     const int dt = delta ? delta_type : LCU_F32;
-    const bool four = d % 4 == 0 && taps == 4 && four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) &&
+    const bool wide = four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) &&
                       four_ok(w2, LCU_F32) && four_ok(b2, LCU_F32) && four_ok(cw, LCU_F32) && four_ok(state, LCU_F32) && four_ok(out, out_type);
-#define ROW(TD, TO, V, PT) norm_conv_single_kernel<TD, TO, V, PT><<<grid, dim3(ROW_THREADS), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, w2, b2, cw, state, (TO *)out, stride, ctx_len, state_slot, d, taps, sets, eps)
+#define ROW(TD, TO, V, PT, WIDE, TAPS) norm_conv_single_kernel<TD, TO, V, PT, WIDE, TAPS><<<grid, dim3(ROW_THREADS), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, w2, b2, cw, state, (TO *)out, stride, ctx_len, state_slot, d, taps, sets, eps)
 #define GO(TD, TO)                                   \
     do {                                             \
-        if (four) ROW(TD, TO, 4, 1);                 \
-        else ROW(TD, TO, 1, 4);                      \
+        if (d % 4) ROW(TD, TO, 1, 4, false, 0);                     \
+        else if (!wide) ROW(TD, TO, 4, 1, false, 0);                \
+        else if (taps == 1) ROW(TD, TO, 4, 1, true, 1);             \
+        else if (taps == 2) ROW(TD, TO, 4, 1, true, 2);             \
+        else if (taps == 3) ROW(TD, TO, 4, 1, true, 3);             \
+        else if (taps == 4) ROW(TD, TO, 4, 1, true, 4);             \
+        else if (taps == 5) ROW(TD, TO, 4, 1, true, 5);             \
+        else if (taps == 6) ROW(TD, TO, 4, 1, true, 6);             \
+        else if (taps == 7) ROW(TD, TO, 4, 1, true, 7);             \
+        else ROW(TD, TO, 4, 1, true, 8);                            \
     } while (0)
     if (dt == LCU_F32 && out_type == LCU_F32) GO(float, float);
     else if (dt == LCU_F32 && out_type == LCU_BF16) GO(float, bf16_t);

@@ -17,6 +17,24 @@ template <class T, int V> __device__ __forceinline__ void store_f32(T *p, const 
     *(Pack<T, V> *)p = out;
 }
 
+// The same where the address may lie at any element: V accesses unless WIDE.
+template <class T, int V, bool WIDE> __device__ __forceinline__ void load_some(const T *p, float *out) {
+    if constexpr (WIDE) {
+        load_as_f32<T, V>(p, out);
+    } else {
+#pragma unroll
+        for (int e = 0; e < V; ++e) out[e] = to_f32(p[e]);
+    }
+}
+template <class T, int V, bool WIDE> __device__ __forceinline__ void store_some(T *p, const float *in) {
+    if constexpr (WIDE) {
+        store_f32<T, V>(p, in);
+    } else {
+#pragma unroll
+        for (int e = 0; e < V; ++e) p[e] = from_f32<T>(in[e]);
+    }
+}
+
 // The sum over a workgroup of up to 16 waves; `scratch` (16 floats) is not in use by an earlier call.
 __device__ __forceinline__ float row_sum(float v, float *scratch) {
     v = wave_sum_in_place(v);

@@ -475,6 +475,20 @@ def test_logits_do_not_depend_on_the_cut_or_the_batch_bit_for_bit_in_32_bit():
     assert torch.equal(torch.cat([p1[:17], p2]), alone)
 
 
+@pytest.mark.parametrize("taps", [2, 3, 4, 5, 8])
+def test_single_tokens_have_a_portions_bits_in_32_bit(taps):
+    """Steps in which every request feeds one token, the norms and convolutions of which are a kernel of their own."""
+    cfg = dict(CFG_B, canon={"taps": taps})
+    folder = make_folder(cfg, random_weights(cfg, RANKS_B, 2))
+    a, b = tokens_of(cfg["vocab"], 24, 22), tokens_of(cfg["vocab"], 24, 23)
+    r = runner_for(folder, "float32")
+    alone = r.step([0], [a], [list(range(24))]).clone()
+    r.step([1], [b[:9]], [[]])
+    r.step([2], [a[:9]], [[]])
+    for t in range(9, 24):
+        assert torch.equal(r.step([1, 2], [[b[t]], [a[t]]])[1], alone[t]), f"token {t}"
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_greedy_generation_through_the_engine_and_its_scheduler(dtype):
     """The framework's entry point: prompts of unequal lengths, more than run at a time, prefilled in portions; the

@@ -54,3 +54,25 @@ def test_norm_and_convolution_of_single_tokens(d, taps, by):
         for s in range(2):
             h = P.layer_norm(rows[r].to(F64), w[s].cpu().to(F64), b[s].cpu().to(F64), 1e-5)
             assert_close(got[:, s, r], P.short_conv(h, cw[s].to(F64)), 1e-5, f"request {r}, set {s}")
+
+
+@pytest.mark.parametrize("d", [8, 100, 513, 1026, 2044, 2048])
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5, 8])
+def test_a_token_alone_has_the_bits_of_the_token_in_a_portion(d, taps):
+    """32-bit: the fused kernel for single tokens against the norm and the convolution of whole portions, which are kernels of their own."""
+    from llama_cu_amd.kernels import ops
+    T, planes = 9, 2
+    x, delta = rnd(T, d, seed=1) + 2.0, rnd(planes, T, d, seed=2)
+    w, b = [rnd(d, seed=k).cuda() for k in (3, 4)], [rnd(d, seed=k).cuda() for k in (5, 6)]
+    cw = rnd(2, d, taps, seed=7, std=0.5).cuda()
+    h = torch.empty(2, T, d, device="cuda")
+    ops.layernorm(x.cuda(), w[0], b[0], 1e-5, h[0], delta=delta.cuda(), weight2=w[1], bias2=b[1], out2=h[1])
+    whole_state = torch.full((1, 2, taps - 1, d), 9.0, device="cuda")
+    whole = ops.short_conv(h, cw, whole_state, torch.empty_like(h), hand_step([T], [T], [0]))
+    for by in (0, 1):                                        # (rows at any address: the bits do not depend on it)
+        state = torch.full((1, 2, taps - 1, d), 9.0, device="cuda")
+        for t in range(T):
+            out = torch.empty(2, 1, d, device="cuda")
+            ops.norm_conv_single(shifted(x[t:t + 1], by), delta[:, t:t + 1].contiguous().cuda(), w, b, 1e-5, cw, state, out, hand_step([1], [t + 1], [0]))
+            assert torch.equal(out[:, 0], whole[:, t]), f"token {t}, shifted by {by}"
+        assert torch.equal(state, whole_state)
