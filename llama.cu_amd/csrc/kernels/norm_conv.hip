@@ -48,36 +48,43 @@ layernorm_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes
     }
 }
 
-// A row's elements in one thread's registers: PT pieces of V neighbours, ROW_THREADS pieces apart.  The row takes in the planes
+// A row's elements in one thread's registers: PT pieces of V neighbours, T pieces apart.  The row takes in the planes
 // of delta, is written back, and its mean and the inverse of its deviation come out.  A step of few rows is a chain of dependent
 // trips to memory and through the barriers: one trip, two barriers.
-// V is 4 where d is a multiple of 4, else 1, and the number of threads is fixed: which elements a thread adds, and so a row's bits, depend on d
-// alone.  (A 32-bit model gives a token the same bits in a portion, whose norm and convolution are kernels of their own, and alone.)  WIDE:
-// every address lets four elements be read at once.
-constexpr int ROW_THREADS = 512;
-template <class TD, int V, int PT, bool WIDE>
+// V is 4 where d is a multiple of 4, else 1, and T, the number of threads, 256 where that makes one piece a thread, else 512: which elements a
+// thread adds, and so a row's bits, depend on d alone.  (A 32-bit model gives a token the same bits in a portion, whose norm and
+// convolution are kernels of their own, and alone.)  2,048 rows of 64 or 100: 4.9 and 5.6 us with 512 threads, 3.6 and 4.0 with 256; one odd row of
+// 513: 2.7 us with 512, 3.4 with 256 (2,048 of them 7.5 and 6.3).  WIDE: every address lets four elements be read at once.
+template <class TD, int T, int V, int PT, bool WIDE>
 __device__ __forceinline__ void take_row(float *xr, const TD *delta, int planes, size_t plane_stride, size_t row_at, int d, float eps,
                                          float (&v)[PT][V], float &mean, float &rstd, float (*scratch)[16]) {
-    float sum = 0.f;
+    float sum = 0.f, first[PT][V];                   // (the row and the first plane are on their way before anything is added or written)
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-        const int c = (threadIdx.x + ROW_THREADS * i) * V;
+        const int c = (threadIdx.x + T * i) * V;
 #pragma unroll
-        for (int e = 0; e < V; ++e) v[i][e] = 0.f;
+        for (int e = 0; e < V; ++e) v[i][e] = first[i][e] = 0.f;
         if (c < d) {
             load_some<float, V, WIDE>(xr + c, v[i]);
-            if (delta) {
-                for (int p = 0; p < planes; ++p) {
-                    float more[V];
-                    load_some<TD, V, WIDE>(delta + p * plane_stride + row_at + c, more);
-#pragma unroll
-                    for (int e = 0; e < V; ++e) v[i][e] += more[e];
-                }
-                store_some<float, V, WIDE>(xr + c, v[i]);
-            }
-#pragma unroll
-            for (int e = 0; e < V; ++e) sum += v[i][e];
+            if (delta) load_some<TD, V, WIDE>(delta + row_at + c, first[i]);
         }
+    }
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+        const int c = (threadIdx.x + T * i) * V;
+        if (delta && c < d) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) v[i][e] += first[i][e];
+            for (int p = 1; p < planes; ++p) {
+                float more[V];
+                load_some<TD, V, WIDE>(delta + p * plane_stride + row_at + c, more);
+#pragma unroll
+                for (int e = 0; e < V; ++e) v[i][e] += more[e];
+            }
+            store_some<float, V, WIDE>(xr + c, v[i]);
+        }
+#pragma unroll
+        for (int e = 0; e < V; ++e) sum += v[i][e];
     }
     mean = row_sum(sum, scratch[0]) / (float)d;
     float sq = 0.f;
@@ -86,15 +93,15 @@ __device__ __forceinline__ void take_row(float *xr, const TD *delta, int planes,
 #pragma unroll
         for (int e = 0; e < V; ++e) {
             const float dev = v[i][e] - mean;
-            if ((threadIdx.x + ROW_THREADS * i) * V < d) sq += dev * dev;
+            if ((threadIdx.x + T * i) * V < d) sq += dev * dev;
         }
     rstd = rsqrtf(row_sum(sq, scratch[1]) / (float)d + eps);
 }
 
-// The same for rows of up to ROW_THREADS * V * PT elements: the row stays in registers between its one read and its writes.  With 256
+// The same for rows of up to T * V * PT elements: the row stays in registers between its one read and its writes.  With 256
 // threads and single elements 2,048 rows of 2,048 with two 32-bit outputs took 21.8 us, now 14.2, one row 5.5, now 2.3.
-template <class TD, class TO, int V, int PT, bool WIDE>
-__global__ void __launch_bounds__(ROW_THREADS)
+template <class TD, class TO, int T, int V, int PT, bool WIDE>
+__global__ void __launch_bounds__(T)
 layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes, size_t plane_stride,
                      const float *__restrict__ w1, const float *__restrict__ b1, TO *__restrict__ out1,
                      const float *__restrict__ w2, const float *__restrict__ b2, TO *__restrict__ out2, int d, float eps) {
@@ -104,7 +111,7 @@ layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int pl
     // (the weights are on their way while the sums are made)
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-        const int c = (threadIdx.x + ROW_THREADS * i) * V;
+        const int c = (threadIdx.x + T * i) * V;
         if (c < d) {
             load_some<float, V, WIDE>(w1 + c, w[0][i]);
             load_some<float, V, WIDE>(b1 + c, b[0][i]);
@@ -114,10 +121,10 @@ layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int pl
             }
         }
     }
-    take_row<TD, V, PT, WIDE>(x + row_at, delta, planes, plane_stride, row_at, d, eps, v, mean, rstd, scratch);
+    take_row<TD, T, V, PT, WIDE>(x + row_at, delta, planes, plane_stride, row_at, d, eps, v, mean, rstd, scratch);
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-        const int c = (threadIdx.x + ROW_THREADS * i) * V;
+        const int c = (threadIdx.x + T * i) * V;
         if (c >= d) continue;
         float y[V];
 #pragma unroll
@@ -143,13 +150,15 @@ LCU_API int lcu_layernorm(float *x, const void *delta, int delta_type, int plane
     const bool four = d % 4 == 0;
     const bool wide = four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) && four_ok(out1, out_type) &&
                       four_ok(w2, LCU_F32) && four_ok(b2, LCU_F32) && four_ok(out2, out_type);
-#define ROW(TD, TO, V, PT, WIDE) layernorm_row_kernel<TD, TO, V, PT, WIDE><<<grid, dim3(ROW_THREADS), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
+#define ROW(TD, TO, T, V, PT, WIDE) layernorm_row_kernel<TD, TO, T, V, PT, WIDE><<<grid, dim3(T), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
 #define GO(TD, TO)                                                                                                           \
     do {                                                                                                                     \
-        if (four && d <= 4 * ROW_THREADS) { if (wide) ROW(TD, TO, 4, 1, true); else ROW(TD, TO, 4, 1, false); }              \
-        else if (four && d <= 8 * ROW_THREADS) { if (wide) ROW(TD, TO, 4, 2, true); else ROW(TD, TO, 4, 2, false); }         \
-        else if (d <= 2 * ROW_THREADS) ROW(TD, TO, 1, 2, false);                                                             \
-        else if (d <= 8 * ROW_THREADS) ROW(TD, TO, 1, 8, false);                                                             \
+        if (four && d <= 1024) { if (wide) ROW(TD, TO, 256, 4, 1, true); else ROW(TD, TO, 256, 4, 1, false); }               \
+        else if (four && d <= 2048) { if (wide) ROW(TD, TO, 512, 4, 1, true); else ROW(TD, TO, 512, 4, 1, false); }          \
+        else if (four && d <= 4096) { if (wide) ROW(TD, TO, 512, 4, 2, true); else ROW(TD, TO, 512, 4, 2, false); }          \
+        else if (d <= 256) ROW(TD, TO, 256, 1, 1, false);                                                                    \
+        else if (d <= 1024) ROW(TD, TO, 512, 1, 2, false);                                                                   \
+        else if (d <= 4096) ROW(TD, TO, 512, 1, 8, false);                                                                   \
         else layernorm_kernel<TD, TO><<<grid, block, 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1,  \
                                                                   w2, b2, (TO *)out2, d, eps);                               \
     } while (0)
@@ -269,8 +278,8 @@ LCU_API int lcu_short_conv(const void *h, int h_type, long long set_stride_h, co
 // of taps where a thread reads its 4 TAPS weights in pieces of four, or 0 (one by one, up to FUSED_TAPS).  With 256 threads,
 // single numbers and the two sets one after the other four rows of 2,048 with four taps took 13.8 us, now 5.0.
 constexpr int FUSED_TAPS = 8;
-template <class TD, class TO, int V, int PT, bool WIDE, int TAPS>
-__global__ void __launch_bounds__(ROW_THREADS)
+template <class TD, class TO, int T, int V, int PT, bool WIDE, int TAPS>
+__global__ void __launch_bounds__(T)
 norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes, size_t plane_stride,
                         const float *__restrict__ w1, const float *__restrict__ b1, const float *__restrict__ w2,
                         const float *__restrict__ b2, const float *__restrict__ cw, float *__restrict__ st,
@@ -290,7 +299,7 @@ norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int
         const float *w = s ? w2 : w1, *b = s ? b2 : b1, *state = slot + (size_t)s * (taps - 1) * d;
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
-            const int c = (threadIdx.x + ROW_THREADS * i) * V;
+            const int c = (threadIdx.x + T * i) * V;
             if (c >= d) continue;
             load_some<float, V, WIDE>(w + c, wv[s][i]);
             load_some<float, V, WIDE>(b + c, bv[s][i]);
@@ -318,14 +327,14 @@ norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int
             }
         }
     }
-    take_row<TD, V, PT, WIDE>(x + (size_t)r * d, delta, planes, plane_stride, (size_t)r * d, d, eps, v, mean, rstd, scratch);
+    take_row<TD, T, V, PT, WIDE>(x + (size_t)r * d, delta, planes, plane_stride, (size_t)r * d, d, eps, v, mean, rstd, scratch);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         if (s >= sets) break;
         float *state = slot + (size_t)s * (taps - 1) * d;
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
-            const int c = (threadIdx.x + ROW_THREADS * i) * V;
+            const int c = (threadIdx.x + T * i) * V;
             if (c >= d) continue;
             float h[V], acc[V];
 #pragma unroll
@@ -349,7 +358,7 @@ LCU_API int lcu_norm_conv_single(float *x, const void *delta, int delta_type, in
                                  const int *ctx_len, const int *state_slot, int n, int d, int taps, int sets, float eps,
                                  hipStream_t stream) {
     if (n <= 0) return LCU_OK;
-    if (d <= 0 || d > 4 * ROW_THREADS || taps < 1 || taps > 8 || sets < 1 || sets > 2 || !w1 || !b1 || (sets == 2 && (!w2 || !b2)) ||
+    if (d <= 0 || d > 2048 || taps < 1 || taps > 8 || sets < 1 || sets > 2 || !w1 || !b1 || (sets == 2 && (!w2 || !b2)) ||
         !cw || (taps > 1 && !state) || (delta && planes <= 0))
         return LCU_BAD_ARGUMENT;
     const size_t stride = (size_t)n * d;
@@ -357,25 +366,29 @@ LCU_API int lcu_norm_conv_single(float *x, const void *delta, int delta_type, in
     const int dt = delta ? delta_type : LCU_F32;
     const bool wide = four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) &&
                       four_ok(w2, LCU_F32) && four_ok(b2, LCU_F32) && four_ok(cw, LCU_F32) && four_ok(state, LCU_F32) && four_ok(out, out_type);
-#define ROW(TD, TO, V, PT, WIDE, TAPS) norm_conv_single_kernel<TD, TO, V, PT, WIDE, TAPS><<<grid, dim3(ROW_THREADS), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, w2, b2, cw, state, (TO *)out, stride, ctx_len, state_slot, d, taps, sets, eps)
-#define GO(TD, TO)                                   \
-    do {                                             \
-        if (d % 4) ROW(TD, TO, 1, 4, false, 0);                     \
-        else if (!wide) ROW(TD, TO, 4, 1, false, 0);                \
-        else if (taps == 1) ROW(TD, TO, 4, 1, true, 1);             \
-        else if (taps == 2) ROW(TD, TO, 4, 1, true, 2);             \
-        else if (taps == 3) ROW(TD, TO, 4, 1, true, 3);             \
-        else if (taps == 4) ROW(TD, TO, 4, 1, true, 4);             \
-        else if (taps == 5) ROW(TD, TO, 4, 1, true, 5);             \
-        else if (taps == 6) ROW(TD, TO, 4, 1, true, 6);             \
-        else if (taps == 7) ROW(TD, TO, 4, 1, true, 7);             \
-        else ROW(TD, TO, 4, 1, true, 8);                            \
+#define ROW(TD, TO, T, V, PT, WIDE, TAPS) norm_conv_single_kernel<TD, TO, T, V, PT, WIDE, TAPS><<<grid, dim3(T), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, w2, b2, cw, state, (TO *)out, stride, ctx_len, state_slot, d, taps, sets, eps)
+#define SIZED(TD, TO, V, PT, WIDE, TAPS) do { if (d <= 1024) ROW(TD, TO, 256, V, PT, WIDE, TAPS); else ROW(TD, TO, 512, V, PT, WIDE, TAPS); } while (0)
+#define GO(TD, TO)                                                      \
+    do {                                                                \
+        if (d % 4 && d <= 256) ROW(TD, TO, 256, 1, 1, false, 0);        \
+        else if (d % 4 && d <= 1024) ROW(TD, TO, 512, 1, 2, false, 0);  \
+        else if (d % 4) ROW(TD, TO, 512, 1, 4, false, 0);               \
+        else if (!wide) SIZED(TD, TO, 4, 1, false, 0);                  \
+        else if (taps == 1) SIZED(TD, TO, 4, 1, true, 1);               \
+        else if (taps == 2) SIZED(TD, TO, 4, 1, true, 2);               \
+        else if (taps == 3) SIZED(TD, TO, 4, 1, true, 3);               \
+        else if (taps == 4) SIZED(TD, TO, 4, 1, true, 4);               \
+        else if (taps == 5) SIZED(TD, TO, 4, 1, true, 5);               \
+        else if (taps == 6) SIZED(TD, TO, 4, 1, true, 6);               \
+        else if (taps == 7) SIZED(TD, TO, 4, 1, true, 7);               \
+        else SIZED(TD, TO, 4, 1, true, 8);                              \
     } while (0)
     if (dt == LCU_F32 && out_type == LCU_F32) GO(float, float);
     else if (dt == LCU_F32 && out_type == LCU_BF16) GO(float, bf16_t);
     else if (dt == LCU_BF16 && out_type == LCU_F32) GO(bf16_t, float);
     else if (dt == LCU_BF16 && out_type == LCU_BF16) GO(bf16_t, bf16_t);
     else return LCU_BAD_ARGUMENT;
+#undef SIZED
 #undef ROW
 #undef GO
     LCU_LAUNCH_CHECK();
