@@ -43,3 +43,23 @@ def test_norm_factor_and_store(nh, nkv, dh, dv, page, by, kind):
         assert_close(ks[at, tok], keys[t], rel, f"keys of row {t}")
         assert torch.equal(vs[at, tok], rows[t, nq + nk:])
     assert (ks[~held] == 0).all() and (vs[~held] == 0).all()
+
+
+@pytest.mark.parametrize("kind", ["float32", "bfloat16"])
+@pytest.mark.parametrize("nh,nkv,dh,dv", [(1, 1, 8, 3), (16, 4, 128, 128), (33, 5, 120, 20), (80, 40, 128, 8)])
+def test_a_rows_bits_do_not_depend_on_the_number_of_rows(nh, nkv, dh, dv, kind):
+    """On both sides of the line between a workgroup a part and one for all three; one to forty stretches of a sum."""
+    from llama_cu_amd.kernels import ops
+    tdt, page, n = TYPES[kind], 16, 300
+    qkv = rnd(n, nh * dh + nkv * (dh + dv), seed=1).to(tdt).cuda()
+    qw, kw = rnd(nh * dh, seed=2).cuda(), rnd(nkv * dh, seed=3).cuda()
+    positions, slots = torch.arange(n, dtype=torch.int32).cuda(), torch.randperm(n, generator=torch.Generator().manual_seed(4)).to(torch.int32).cuda()
+    outs = []
+    for cut in (n, 128, 7):
+        rows, cache = qkv.clone(), torch.zeros(-(-n // page), 1, nkv * (dh + dv) * page, dtype=tdt, device="cuda")
+        for a in range(0, n, cut):
+            b = min(n, a + cut)
+            ops.qk_norm_store(rows[a:b], positions[a:b].contiguous(), nh, nkv, dh, dv, qw, kw, 1e-5, 0.3, 5, cache, slots[a:b].contiguous(), page)
+        outs.append((rows, cache))
+    for rows, cache in outs[1:]:
+        assert torch.equal(rows, outs[0][0]) and torch.equal(cache, outs[0][1])
