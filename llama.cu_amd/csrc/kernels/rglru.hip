@@ -49,15 +49,15 @@ __device__ __forceinline__ float conv_at(const TI *__restrict__ rows, int row_st
     return acc;
 }
 
-// The same for up to four taps, without a loop: the loads of all taps, and of the elements that a thread makes one after the other, are on
+// The same for up to MOST taps, without a loop: the loads of all taps, and of the elements that a thread makes one after the other, are on
 // their way together.
-template <class TI>
+template <int MOST, class TI>
 __device__ __forceinline__ float conv_few(const TI *__restrict__ rows, int row_stride, int x_off, const float *__restrict__ bias,
                                           const float *__restrict__ conv_w, const float *__restrict__ conv_b,
                                           const float *__restrict__ st, int t, int t0, int first_pos, int c, int width, int taps) {
-    float here[4], before[4], w[4];
+    float here[MOST], before[MOST], w[MOST];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < MOST; ++j) {
         const int back = max(taps - 1 - j, 0), m = t0 - (t - back);
         here[j] = to_f32(rows[(size_t)(m <= 0 ? t - back : t) * row_stride + x_off + c]);
         before[j] = st[(size_t)(m > 0 && first_pos - m >= 0 ? taps - 1 - m : 0) * width + c];
@@ -66,7 +66,7 @@ __device__ __forceinline__ float conv_few(const TI *__restrict__ rows, int row_s
     const float bx = bias ? bias[x_off + c] : 0.f;
     float acc = conv_b ? conv_b[c] : 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < MOST; ++j) {
         const int back = taps - 1 - j, m = t0 - (t - back);
         const float x = m <= 0 ? here[j] + bx : first_pos - m >= 0 ? before[j] : 0.f;
         acc = j < taps ? acc + w[j] * x : acc;
@@ -119,19 +119,26 @@ rglru_gates_kernel(const TI *__restrict__ rows, int row_stride, int x_off, const
     const int c = b * bs + min(o, bs - 1);
     const size_t y_at = (size_t)(tok0 + min(slice, nt - 1)) * row_stride + y_off + c;
     const float l = lam[c], ba_c = ba[c], bi_c = bi[c], y_in = to_f32(rows[y_at]) + (bias ? bias[y_off + c] : 0.f);
-    // (a token beyond the end is the last one, made once more and not used)
     auto make = [&](int w, auto conv) {
-        const int t = tok0 + min(w / bs, nt - 1), r = req_of_token[t], t0 = q_start[r];
+        const int t = tok0 + w / bs, r = req_of_token[t], t0 = q_start[r];
         const int first_pos = ctx_len[r] - (q_start[r + 1] - t0);
         us[w / bs][w % bs] = conv(rows, row_stride, x_off, bias, conv_w, conv_b, state + (size_t)state_slot[r] * taps * width, t, t0,
                                   first_pos, b * bs + w % bs, width, taps);
     };
-    if (taps <= 4) {
+    // (the tokens that there are: the rows of us beyond them hold zeros, whose sums are not used)
+    if (taps == 1) {
 #pragma unroll 4
-        for (int w = threadIdx.x; w < RG_TOK * bs; w += RG_OUT * RG_SLICES) make(w, conv_few<TI>);
+        for (int w = threadIdx.x; w < nt * bs; w += RG_OUT * RG_SLICES) make(w, conv_few<1, TI>);
+    } else if (taps == 2) {
+#pragma unroll 4
+        for (int w = threadIdx.x; w < nt * bs; w += RG_OUT * RG_SLICES) make(w, conv_few<2, TI>);
+    } else if (taps <= 4) {
+#pragma unroll 4
+        for (int w = threadIdx.x; w < nt * bs; w += RG_OUT * RG_SLICES) make(w, conv_few<4, TI>);
     } else {
-        for (int w = threadIdx.x; w < RG_TOK * bs; w += RG_OUT * RG_SLICES) make(w, conv_at<TI>);
+        for (int w = threadIdx.x; w < nt * bs; w += RG_OUT * RG_SLICES) make(w, conv_at<TI>);
     }
+    for (int w = nt * bs + threadIdx.x; w < RG_TOK * bs; w += RG_OUT * RG_SLICES) us[w / bs][w % bs] = 0.f;
     __syncthreads();
     float ra[RG_TOK], ri[RG_TOK];
 #pragma unroll
