@@ -204,29 +204,38 @@ moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, cons
 // sorted_to_flat [total] (the pairs sorted by expert), and the tiles of up to rows_per_tile rows:
 // tile_expert, tile_begin (first sorted row), tile_rows, each [max_tiles], and n_tiles [1].  Only the first `tiled`
 // experts get tiles: the ones behind them have no matrices (identity experts), and their pairs are only sorted.
+// A thread an expert: the pairs and tiles before its own by a sum over the threads (one thread that walked 1,024 experts took 40 us).
+static_assert(MOE_MAX_EXPERTS <= 1024, "a thread an expert");
 __global__ void __launch_bounds__(1024)
 moe_group_kernel(const int *__restrict__ ids, int total, int experts, int *__restrict__ sorted_to_flat,
                  int *__restrict__ tile_expert, int *__restrict__ tile_begin, int *__restrict__ tile_rows,
                  int *__restrict__ n_tiles, int max_tiles, int rows_per_tile, int tiled) {
     __shared__ int count[MOE_MAX_EXPERTS];
     __shared__ int cursor[MOE_MAX_EXPERTS];
-    for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;
+    __shared__ int ends[2][1024 / WAVE];
+    const int e = threadIdx.x, lane = e % WAVE, wave = e / WAVE;
+    if (e < experts) count[e] = 0;
     __syncthreads();
     for (int i = threadIdx.x; i < total; i += blockDim.x) atomicAdd(&count[ids[i]], 1);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int at = 0, tiles = 0;
-        for (int e = 0; e < experts; ++e) {
-            cursor[e] = at;
-            for (int r = 0; e < tiled && r < count[e] && tiles < max_tiles; r += rows_per_tile) {
-                tile_expert[tiles] = e;
-                tile_begin[tiles] = at + r;
-                tile_rows[tiles] = count[e] - r < rows_per_tile ? count[e] - r : rows_per_tile;
-                ++tiles;
-            }
-            at += count[e];
-        }
-        n_tiles[0] = tiles;
+    const int pairs = e < experts ? count[e] : 0, tiles = e < tiled ? (pairs + rows_per_tile - 1) / rows_per_tile : 0;
+    int at = pairs, tile = tiles;                   // up to and with this expert, first within the wave
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+        const int a = __shfl_up(at, off, WAVE), b = __shfl_up(tile, off, WAVE);
+        if (lane >= off) { at += a; tile += b; }
+    }
+    if (lane == WAVE - 1) { ends[0][wave] = at; ends[1][wave] = tile; }
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) { at += ends[0][w]; tile += ends[1][w]; }
+    if (e == 1023) n_tiles[0] = min(tile, max_tiles);
+    at -= pairs;
+    tile -= tiles;
+    if (e < experts) cursor[e] = at;
+    for (int k = 0; k < tiles && tile + k < max_tiles; ++k) {
+        tile_expert[tile + k] = e;
+        tile_begin[tile + k] = at + k * rows_per_tile;
+        tile_rows[tile + k] = min(pairs - k * rows_per_tile, rows_per_tile);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < total; i += blockDim.x) sorted_to_flat[atomicAdd(&cursor[ids[i]], 1)] = i;
@@ -329,31 +338,39 @@ template <class T, bool PACKED> struct Unit {
 // turn: the kernel for few rows gives each of its waves a part, and a row has the same bits whichever kernel its step goes to.
 __device__ __forceinline__ int quarter_steps(int steps) { return (steps + 7) / 8 * 2; }
 
-// Few rows an expert (decoding).  A workgroup per expert and 32 of its matrix's rows looks through the step's pairs for the expert's
-// (a list in LDS, in any order: a row's result does not depend on its place), and multiplies them 16 at a time; its four waves take a
-// quarter of K each, four steps of loads always on their way, and add up through LDS in a fixed order.
+// Few rows an expert (decoding).  A workgroup takes 32 rows of an expert's matrix and the expert's rows, 16 at a time, or 48 where there are
+// more of them; its four waves take a quarter of K each, steps of loads always on their way, and add up through LDS in a fixed order.
+// Up to MOE_LIST pairs a step (MOE_LIST_F32 in 32 bits), a workgroup an expert looks through the step's pairs for the expert's (a list in LDS, in any order: a
+// row's result does not depend on its place): no kernel in front.  Beyond, the pairs come sorted and in tiles of 16 rows (moe_group_kernel),
+// a workgroup a tile: each looking through thousands of numbers took longer than the kernel in front (1,024 experts, 1,024 tokens of eight:
+// 552 us, now 143), and an expert that most tokens name was one workgroup's, 16 rows at a time (64 experts, all of 512 tokens
+// on one: 120 us, now 24; of 128 tokens 38, now 28).
 // What bounds it is the experts' matrices out of memory, once.  One wave for 16 features and all of K left 3 to 4 waves a compute
 // unit, which waited for eight loads and then issued the next eight: 2.8 (gated first product) and 3.2 TB/s (second) for 14 of 16
 // experts of 2 x 1024 x 2048 and 2048 x 1024, 42 and 18 us; now 24 and 14 us, and 16 experts of 2 x 1408 x 2048 52 -> 34.5 us, 5.3 TB/s.
 // A shared expert that every token uses rides along as one more expert (sw: its matrix, packed alike, of s_n rows and s_k columns; only
 // while the tokens are few, as each 16 of them read it once): beside the others it costs its bytes, in kernels of its own it took
 // 11 and 5 us.
-// (Eight steps on their way and half as many waves: 25 and 37.5.)  The list costs a scan of n * top numbers, but no kernel in front.
-constexpr int MOE_LIST = 2048;
+// (Eight steps on their way and half as many waves: 25 and 37.5.)
+constexpr int MOE_LIST = 128, MOE_LIST_F32 = 64;      // (in 32 bits the matrix instructions of a workgroup's rows take longer)
+template <int N> struct Int { static constexpr int value = N; };
 template <class T, int MODE, bool PACKED>
 __global__ void __launch_bounds__(256, 4)
 moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__ w, size_t w_expert_stride, int N, int K,
                     const int *__restrict__ ids, int total, const float *__restrict__ wts, T *__restrict__ out_t,
                     float *__restrict__ out_f, int out_stride, int top, int add, float alpha, float limit, int experts,
-                    const T *__restrict__ sx, const T *__restrict__ sw, int s_n, int s_k, T *__restrict__ s_out_t, float *__restrict__ s_out_f) {
+                    const T *__restrict__ sx, const T *__restrict__ sw, int s_n, int s_k, T *__restrict__ s_out_t, float *__restrict__ s_out_f,
+                    const int *__restrict__ sorted, const int *__restrict__ tile_expert, const int *__restrict__ tile_begin,
+                    const int *__restrict__ tile_rows, const int *__restrict__ n_tiles, int max_tiles) {
     typedef Mma<T> M;
     typedef typename M::frag frag;
     constexpr bool GATED = MODE == MOE_UP_GATED, UP = MODE != MOE_DOWN;
-    constexpr int AHEAD = 4;
     __shared__ int list[MOE_LIST], found;
     __shared__ f32x4 red[4][2][WAVE];
-    const int e = blockIdx.y, tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, g = lane / 16, l16 = lane % 16;
-    const bool shared = e == experts;
+    const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, g = lane / 16, l16 = lane % 16;
+    const bool shared = (int)blockIdx.y == (sorted ? max_tiles : experts);
+    if (sorted && !shared && (int)blockIdx.y >= n_tiles[0]) return;
+    const int e = sorted && !shared ? tile_expert[blockIdx.y] : (int)blockIdx.y;
     const T *we = w + (size_t)e * w_expert_stride;
     if (shared) {                                    // every token's rows [n, s_k] and a matrix of its own size
         total /= top;
@@ -373,48 +390,72 @@ moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__
     const int tile0 = 2 * blockIdx.x, steps = (K + M::KSTEP - 1) / M::KSTEP, per = quarter_steps(steps);
     const int s0 = wave * per, s1 = min(steps, s0 + per);
     const Unit<T, PACKED> w0(we, tile0, N, K, steps, lane), w1(we, tile0 + 1, N, K, steps, lane);
-    for (int first = 0; first < total; first += MOE_LIST) {
-        __syncthreads();                             // the list of before has been read
+    const int *rows = list;                          // the pairs of this workgroup's rows (null: row r is token r)
+    int count = total;
+    if (shared) {
+        rows = nullptr;
+    } else if (sorted) {
+        rows = sorted + tile_begin[blockIdx.y];
+        count = tile_rows[blockIdx.y];
+    } else {
         if (tid == 0) found = 0;
         __syncthreads();
-        for (int p = first + tid; p < min(total, first + MOE_LIST); p += 256)
-            if (shared || ids[p] == e) list[atomicAdd(&found, 1)] = p;
+        if (tid < total && ids[tid] == e) list[atomicAdd(&found, 1)] = tid;      // (total is at most MOE_LIST, a thread a pair)
         __syncthreads();
-        const int count = found;
-        for (int r0 = 0; r0 < count; r0 += 16) {
-            const bool valid = r0 + l16 < count;
-            const int flat = list[valid ? r0 + l16 : r0];
-            const T *xrow = x + (size_t)(UP ? flat / top : flat) * x_stride + g * M::PER_LANE;
-            const float sc = MODE == MOE_UP ? wts[flat] : 1.f;
-            const int x_left = K - g * M::PER_LANE;
-            f32x4 acc0 = f32x4{0.f, 0.f, 0.f, 0.f}, acc1 = f32x4{0.f, 0.f, 0.f, 0.f};
-            frag a0[AHEAD], a1[AHEAD], b[AHEAD];
-            auto fetch = [&](int u, int s) {
-                a0[u] = w0.load(s);
-                a1[u] = w1.load(s);
-                b[u] = s * M::KSTEP < x_left ? M::load(xrow + s * M::KSTEP) : M::zero();
-            };
+        count = found;
+    }
+    // rows r0 .. of RT tiles of 16
+    auto pass = [&](auto rt, auto ahead, int r0) {
+        constexpr int RT = decltype(rt)::value, AHEAD = decltype(ahead)::value;
+        int flat[RT];
+        unsigned xat[RT];                            // (few rows: their elements are less than 2^32)
+        float sc[RT];
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u)
-                if (s0 + u < s1) fetch(u, s0 + u);
-            for (int s = s0; s < s1; s += AHEAD) {
+        for (int m = 0; m < RT; ++m) {
+            const int r = min(r0 + 16 * m + l16, count - 1);
+            flat[m] = rows ? rows[r] : r;
+            xat[m] = (unsigned)(UP ? flat[m] / top : flat[m]) * x_stride + g * M::PER_LANE;
+            if (MODE == MOE_UP) sc[m] = wts[flat[m]];
+        }
+        const int x_left = K - g * M::PER_LANE;
+        f32x4 acc[RT][2];
 #pragma unroll
-                for (int u = 0; u < AHEAD; ++u) {
-                    if (s + u >= s1) break;
-                    const frag bb = MODE == MOE_UP ? M::scaled(b[u], sc) : b[u];
-                    acc0 = M::mma(a0[u], bb, acc0);
-                    acc1 = M::mma(a1[u], bb, acc1);
-                    if (s + u + AHEAD < s1) fetch(u, s + u + AHEAD);
+        for (int m = 0; m < RT; ++m) acc[m][0] = acc[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        frag a0[AHEAD], a1[AHEAD], b[AHEAD][RT];
+        auto fetch = [&](int u, int s) {
+            a0[u] = w0.load(s);
+            a1[u] = w1.load(s);
+#pragma unroll
+            for (int m = 0; m < RT; ++m) b[u][m] = s * M::KSTEP < x_left ? M::load(x + xat[m] + s * M::KSTEP) : M::zero();
+        };
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (s0 + u < s1) fetch(u, s0 + u);
+        for (int s = s0; s < s1; s += AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                if (s + u >= s1) break;
+#pragma unroll
+                for (int m = 0; m < RT; ++m) {
+                    const frag bb = MODE == MOE_UP ? M::scaled(b[u][m], sc[m]) : b[u][m];
+                    acc[m][0] = M::mma(a0[u], bb, acc[m][0]);
+                    acc[m][1] = M::mma(a1[u], bb, acc[m][1]);
                 }
+                if (s + u + AHEAD < s1) fetch(u, s + u + AHEAD);
             }
-            if (r0) __syncthreads();                 // the sums of the rows before have been read
-            red[wave][0][lane] = acc0;
-            red[wave][1][lane] = acc1;
+        }
+#pragma unroll
+        for (int m = 0; m < RT; ++m) {
+            if (m > 0 && r0 + 16 * m >= count) break;
+            if (r0 + m) __syncthreads();             // the sums of the rows before have been read
+            red[wave][0][lane] = acc[m][0];
+            red[wave][1][lane] = acc[m][1];
             __syncthreads();
             // the first wave stores (with two products' sums the first two, one each): four neighbouring features of a row a lane
             if (wave < (GATED ? 1 : 2)) {
+                const bool valid = r0 + 16 * m + l16 < count;
                 const f32x4 v = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
-                const int dst = !UP && add ? flat / top : flat;
+                const int dst = !UP && add ? flat[m] / top : flat[m];
                 if constexpr (GATED) {
                     const f32x4 up = ((red[0][1][lane] + red[1][1][lane]) + red[2][1][lane]) + red[3][1][lane];
                     Quad<T> q;
@@ -437,6 +478,11 @@ moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__
                 }
             }
         }
+    };
+    if (count <= 16) {
+        if (count > 0) pass(Int<1>(), Int<4>(), 0);
+    } else {
+        for (int r0 = 0; r0 < count; r0 += 48) pass(Int<3>(), Int<2>(), r0);
     }
 }
 
@@ -614,9 +660,12 @@ moe_combine_kernel(float *__restrict__ out, const float *__restrict__ y, const f
     }
 }
 
-// Rows of a tile for n * top pairs over so many experts: 0 (the kernel for few rows, which has no tiles) while an expert has 16 rows
-// or fewer on average, else 64.  The caller sizes its scratch with it: max_tiles = min(total, total / rows + experts), or 0.
-LCU_API int lcu_moe_tile_rows(int total, int experts) { return (long long)total <= 16ll * experts ? 0 : MOE_TILE_ROWS; }
+// Rows of a tile for n * top pairs over so many experts: while an expert has 16 rows or fewer on average the kernel for few rows, with no
+// tiles up to MOE_LIST pairs (0; MOE_LIST_F32 in 32 bits) and tiles of 16 beyond; else 64.  The caller sizes its scratch with it: max_tiles = min(total,
+// total / rows + experts), or 0.
+LCU_API int lcu_moe_tile_rows(int type, int total, int experts) {
+    return (long long)total > 16ll * experts ? MOE_TILE_ROWS : total > (type == LCU_F32 ? MOE_LIST_F32 : MOE_LIST) ? 16 : 0;
+}
 
 // h: [n, d] of `type`; router: [experts, d] 32-bit; ids, wts: [n * top].
 // bias: null or [experts] 32-bit; mode 0: sigmoid weights, 1: softmax over the chosen; extra, gates: see the kernel
@@ -649,7 +698,7 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
 // token's input.  shared (null or
 // [n, d] of `type`) with shared_gate (null or [n] 32-bit): rows that are added beside the experts', times the gate.  shared_up,
 // shared_down (null, or the matrices [2 * shared_ff, d] and [d, shared_ff] of a shared expert that is computed here, with silu, in the order of Unit
-// like w_up and w_down; only where lcu_moe_tile_rows says 0): act then holds n * shared_ff elements more and y n rows more.
+// like w_up and w_down; only where lcu_moe_tile_rows does not say 64): act then holds n * shared_ff elements more and y n rows more.
 LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float *wts, int *ints, int max_tiles,
                             const void *w_up, int packed_up, const void *w_down, int packed_down, void *act, float *y, float *out, int n, int d, int ff,
                             int experts, int top, int gated, const void *shared, const float *shared_gate, const void *shared_up,
@@ -661,7 +710,8 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
         (identity && !gated) || experts + identity > MOE_MAX_EXPERTS)
         return LCU_BAD_ARGUMENT;
     const int total = n * top;
-    const bool few = lcu_moe_tile_rows(total, experts) == 0;
+    const int tile_rows = lcu_moe_tile_rows(type, total, experts);
+    const bool few = tile_rows < MOE_TILE_ROWS;
     if (shared_up && (!shared_down || shared || !gated || !few || !packed_up || !packed_down || shared_ff <= 0 || shared_ff % 16)) return LCU_BAD_ARGUMENT;
     const int add = top == 1 && !gated;
     float *down_to = add ? out : y;
@@ -674,18 +724,29 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
     if (type == LCU_BF16) { if (packed) GO(bf16_t, true, __VA_ARGS__); else GO(bf16_t, false, __VA_ARGS__); }       \
     else { if (packed) GO(float, true, __VA_ARGS__); else GO(float, false, __VA_ARGS__); }                          \
     LCU_LAUNCH_CHECK()
+    int *sorted = nullptr, *t_exp = nullptr, *t_beg = nullptr, *t_rows = nullptr, *n_tiles = nullptr;
+    if (!ids) return LCU_BAD_ARGUMENT;
+    if (tile_rows) {
+        if (!ints || max_tiles <= 0) return LCU_BAD_ARGUMENT;
+        sorted = ints;
+        t_exp = ints + total;
+        t_beg = t_exp + max_tiles;
+        t_rows = t_beg + max_tiles;
+        n_tiles = t_rows + max_tiles;
+        moe_group_kernel<<<dim3(1), dim3(1024), 0, stream>>>(ids, total, experts + identity, sorted, t_exp, t_beg, t_rows, n_tiles, max_tiles, tile_rows, experts);
+        LCU_LAUNCH_CHECK();
+    }
     if (few) {
-        if (!ids) return LCU_BAD_ARGUMENT;
         // one more expert, the shared one: its activations lie behind the pairs' (act [total, ff], then [n, shared_ff]), its outputs too
-        const int with = experts + (shared_up ? 1 : 0), s_rows = 2 * shared_ff, wider = shared_up && s_rows > up_rows ? s_rows : up_rows;
+        const int with = (tile_rows ? max_tiles : experts) + (shared_up ? 1 : 0), s_rows = 2 * shared_ff, wider = shared_up && s_rows > up_rows ? s_rows : up_rows;
         const size_t act_end = (size_t)total * ff;
         const dim3 block(256), gu((wider + 31) / 32, with), gd((d + 31) / 32, with);
 #define UP(T, PACKED, MODE) moe_gemm_few_kernel<T, MODE, PACKED><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \
                                                 ids, total, wts, (T *)act, nullptr, ff, top, 0, alpha, limit, experts, \
-                                                (const T *)h, (const T *)shared_up, s_rows, d, (T *)act + act_end, nullptr)
+                                                (const T *)h, (const T *)shared_up, s_rows, d, (T *)act + act_end, nullptr, sorted, t_exp, t_beg, t_rows, n_tiles, max_tiles)
 #define DOWN(T, PACKED, MODE) moe_gemm_few_kernel<T, MODE, PACKED><<<gd, block, 0, stream>>>((const T *)act, ff, (const T *)w_down, down_stride, d, ff, \
                                                 ids, total, wts, nullptr, down_to, d, top, add, 0.f, 0.f, experts, \
-                                                (const T *)act + act_end, (const T *)shared_down, d, shared_ff, nullptr, y + (size_t)total * d)
+                                                (const T *)act + act_end, (const T *)shared_down, d, shared_ff, nullptr, y + (size_t)total * d, sorted, t_exp, t_beg, t_rows, n_tiles, max_tiles)
         int packed = packed_up;
         if (gated) { TYPED(UP, MOE_UP_GATED); } else { TYPED(UP, MOE_UP); }
         packed = packed_down;
@@ -693,10 +754,6 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
 #undef UP
 #undef DOWN
     } else {
-        if (!ints || max_tiles <= 0) return LCU_BAD_ARGUMENT;
-        int *sorted = ints, *t_exp = ints + total, *t_beg = t_exp + max_tiles, *t_rows = t_beg + max_tiles, *n_tiles = t_rows + max_tiles;
-        moe_group_kernel<<<dim3(1), dim3(1024), 0, stream>>>(ids, total, experts + identity, sorted, t_exp, t_beg, t_rows, n_tiles, max_tiles, MOE_TILE_ROWS, experts);
-        LCU_LAUNCH_CHECK();
         // flat grids: the kernel shares them out over the dies itself
         const dim3 block(256), gu(8 * max_tiles * (((up_rows + 127) / 128 + 7) / 8)), gd(8 * max_tiles * (((d + 127) / 128 + 7) / 8));
 #define UP(T, PACKED, MODE) moe_gemm_many_kernel<T, MODE, PACKED><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \

@@ -1517,7 +1517,7 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
         _contig(shared_up.data, "shared up"); _contig(shared_down.data, "shared down")
     lib = build.load("moe")
     total = n * top
-    tile = lib.lcu_moe_tile_rows(total, experts)
+    tile = lib.lcu_moe_tile_rows(_type(h, "moe input"), total, experts)
     max_tiles = min(total, total // tile + experts) if tile else 0
     ints = torch.empty(total + 3 * max_tiles + 1, dtype=torch.int32, device=h.device) if tile else None
     act = torch.empty(total * ff + n * sff, dtype=h.dtype, device=h.device)
@@ -1536,7 +1536,7 @@ MOE_SHARED_ROWS = 32        # tokens up to which a shared expert is computed bes
 def moe_shared_beside(n: int, top: int, experts: int, w_up, w_down) -> bool:
     """Whether ``moe_experts`` computes a shared expert beside the others for ``n`` tokens."""
     return n <= MOE_SHARED_ROWS and isinstance(w_up, PackedExperts) and isinstance(w_down, PackedExperts) \
-        and build.load("moe").lcu_moe_tile_rows(n * top, experts) == 0
+        and n * top <= 16 * experts
 
 
 @dataclass(frozen=True)

@@ -93,3 +93,58 @@ def test_a_shared_expert_beside_the_others(dtype, n, ff, sff, gate):
             a, b = torch.clamp(f(gates[e]) @ x[t], max=2.0), torch.clamp(f(ups[e]) @ x[t], -2.0, 2.0)
             want[t] += w * (f(down[e]) @ (a * torch.sigmoid(1.702 * a) * (b + 1.0)))
     assert_close(out, want, 1e-4 if dtype == "float32" else 3e-2, "output")
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("experts,top,n,all_of", [(16, 1, 64, 49), (16, 1, 65, 65), (16, 1, 128, 97), (17, 1, 129, 129), (70, 4, 200, 33), (1024, 3, 100, 100)])
+def test_an_expert_that_many_tokens_name(dtype, experts, top, n, all_of):
+    """Experts of few rows on average, one of which ``all_of`` of the tokens name: on both sides of the number of pairs from which on they come
+    sorted, in tiles; every row has the bits that it has alone."""
+    from llama_cu_amd.kernels import ops
+    d, ff, tdt = 72, 32, TYPES[dtype]
+    h = rnd(n, d, seed=1).to(tdt).cuda()
+    up, down = rnd(experts, 2 * ff, d, seed=2, std=d ** -0.5).to(tdt).cuda(), rnd(experts, d, ff, seed=3, std=ff ** -0.5).to(tdt).cuda()
+    g = torch.Generator().manual_seed(4)
+    ids = torch.stack([torch.randperm(experts, generator=g)[:top] for _ in range(n)])
+    for t in range(all_of):
+        if not (ids[t] == experts - 1).any():
+            ids[t, t % top] = experts - 1
+    ids, wts = ids.to(torch.int32).cuda(), torch.rand(n, top, generator=g).cuda()
+    packed = ops.pack_experts(up), ops.pack_experts(down)
+    outs = []
+    for u, w in ((up, down), packed):
+        out = torch.empty(n, d, device="cuda")
+        ops.moe_experts(h, ids, wts, u, w, out, gated=True, fresh=True)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    for t in range(0, n, 7):
+        one = torch.empty(1, d, device="cuda")
+        ops.moe_experts(h[t:t + 1], ids[t:t + 1].contiguous(), wts[t:t + 1].contiguous(), *packed, one, gated=True, fresh=True)
+        assert torch.equal(one[0], outs[1][t]), f"token {t}"
+    x, want = h.cpu().to(F64), torch.zeros(n, d, dtype=F64)
+    u, w = up.cpu().to(F64).view(experts, ff // 16, 2, 16, d), down.cpu().to(F64)
+    for t in range(n):
+        for e, weight in zip(ids[t].tolist(), wts[t].cpu().to(F64)):
+            a, b = (u[e, :, k].reshape(ff, d) @ x[t] for k in (0, 1))
+            want[t] += weight * (w[e] @ (a * torch.sigmoid(a) * b))
+    assert_close(outs[0], want, 1e-5 if dtype == "float32" else 2.0 ** -8, "output")      # (one rounding to bfloat16, of the activations, under sums over ff)
+
+
+def test_a_shared_expert_beside_sorted_pairs():
+    """32 tokens of nine experts each: the pairs come in tiles, the shared expert rides along all the same."""
+    from llama_cu_amd.kernels import ops
+    experts, top, n, d, ff, sff = 40, 9, 32, 64, 16, 48
+    h = rnd(n, d, seed=1).cuda()
+    up, down = rnd(experts, 2 * ff, d, seed=2, std=d ** -0.5).cuda(), rnd(experts, d, ff, seed=3, std=ff ** -0.5).cuda()
+    sg, su, sd = rnd(1, sff, d, seed=4, std=d ** -0.5).cuda(), rnd(1, sff, d, seed=5, std=d ** -0.5).cuda(), rnd(1, d, sff, seed=6, std=sff ** -0.5).cuda()
+    g = torch.Generator().manual_seed(7)
+    ids = torch.stack([torch.randperm(experts, generator=g)[:top] for _ in range(n)]).to(torch.int32).cuda()
+    wts = torch.rand(n, top, generator=g).cuda()
+    packed = ops.pack_experts(up), ops.pack_experts(down)
+    assert ops.moe_shared_beside(n, top, experts, *packed)
+    both, alone = torch.empty(n, d, device="cuda"), torch.empty(n, d, device="cuda")
+    ops.moe_experts(h, ids, wts, *packed, both, gated=True, fresh=True, shared_expert=(ops.pack_gated_experts(sg, su), ops.pack_experts(sd)))
+    ops.moe_experts(h, ids, wts, *packed, alone, gated=True, fresh=True)
+    z = h.cpu().to(F64) @ sg[0].cpu().to(F64).T
+    want = alone.cpu().to(F64) + (z * torch.sigmoid(z) * (h.cpu().to(F64) @ su[0].cpu().to(F64).T)) @ sd[0].cpu().to(F64).T
+    assert_close(both, want, 1e-5, "output")
