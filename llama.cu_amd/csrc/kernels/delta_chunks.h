@@ -1,4 +1,4 @@
-// The delta rules over portions of many tokens: chunks of 64 tokens side by side on the 32-bit matrix instruction.
+// The delta rules over portions of many tokens: chunks of 64 tokens side by side on the 64-bit matrix instruction.
 //
 // A token maps a head's state by S <- diag(w) S - al (u^T S) + k v^T, o = S^T r (gated: w one number, al = beta g u, k = u).  Within
 // a chunk, with G_t the product of the decays up to t (per key channel), c_t = u_t^T S_(t-1) and the rows
@@ -10,33 +10,67 @@
 //   Q = tril(r~ k~^T) v - tril(r~ al~^T) N.
 // Two kernels: `maps` makes F, H, P and Q of every chunk and head at once; `chain` walks a request's chunks, 16 value columns a
 // workgroup, and applies them.  A token alone (delta_scan_kernel) is a chain of 0.55 us a token, 0.9 us and more where the decay is per
-// channel; a chunk is one of 2.3 us.  2,048 tokens of one request, 16 heads of 128: gated 1,100 us scanned, maps 68 and chain 79 us in
-// chunks; with decays per channel 1,800 to 2,400 us scanned, 106 and 79 us in chunks.  64 tokens (the fewest that come here) gated 32
-// us scanned, 35 in chunks, with decays per channel 58 and more against 54.
+// channel; a chunk is one of 3.6 us.  2,048 tokens of one request, 16 heads of 128, the whole rule with its preparation and output kernels:
+// gated 1,170 us scanned, 254 in chunks; with decays per channel 2,420 scanned, 350 in chunks (with 32-bit products 175 and 225, and a larger error,
+// below).
 //
-// What bounds them: `maps` runs 4,300 (channel-wise 6,300) matrix instructions of 32 cycles a chunk and head, 14 (21) us on a compute
-// unit's four SIMDs, of which it takes 30 (48): one workgroup of 8 waves fits a compute unit beside its LDS.  `chain` is its 96 matrix
-// instructions a SIMD and chunk (1.3 us) and the round through LDS; the affine form costs `maps` a third more products than c, o and S
+// What bounds them: `maps` runs 4,300 (channel-wise 6,300) matrix instructions of 64 cycles a chunk and head, 28 (42) us on a compute
+// unit's four SIMDs; one workgroup of 8 waves fits a compute unit beside its LDS.  `chain` is its 96 matrix
+// instructions a SIMD and chunk (2.6 us) and the round through LDS; the affine form costs `maps` a third more products than c, o and S
 // in turn would, but leaves one product instead of two, one after the other, on the chain.
 //
 // The decays per channel are at least exp(-exp(-1/2)) = 0.545 a token, so G over a chunk stays above 1e-17 and 1 / G below 1e17: the
 // products u~_t k~_s are of the size of u_t k_s again and lose nothing (a quotient of two rounded numbers).  The gated rule's one decay
 // may be as small as it likes: there the products u k^T and r k^T are weighted by exp(L_t - L_s) <= 1, L the sums of log g in 64-bit.
 //
-// All products are 32-bit with 32-bit sums (v_mfma_f32_16x16x4_f32).  In its operands lane (l, g) of 16 x 4 holds row (or column) l and
-// index g of the summed four, in its results column l and rows 4 g .. 4 g + 3: with the summed index permuted alike on both sides
-// (step e of a tile of 16 takes the indexes 4 g + e) results are the next product's operand as they are.
+// Products and sums are 64-bit (v_mfma_f64_16x16x4_f64, half the rate of the 32-bit instruction), what is held between them is 32-bit, but for
+// the state on its way along the chain: one rounding each of u~, r~, k~, al~, the masked matrices and the maps.  Sums of 64 and 128 terms in
+// 32 bits, one after the other, would be 2 to 3e-7 off where decays are fast and the scan, whose lanes add in a tree, is only 1e-7 off.
+// Measured over 640 tokens of 2 heads of 128 (relative, 2-norm, against 64 bits, scan / chunks), per channel,
+// from decays of 0.98 to 0.55 a token: outputs 6.7e-7 / 6.2e-7 to 1.4e-7 / 1.0e-7, states 1.5e-6 / 1.5e-6 to 4.4e-8 / 4.6e-8; gated, decays of
+// 0.9999 to 0.05: outputs 6.6e-7 / 1.2e-7 to 1.5e-7 / 1.0e-7, states 1.4e-6 / 1.0e-7 to 7.7e-8 / 6.8e-8.
+// In the instruction's operands lane (l, g) of 16 x 4 holds row (or column) l and index g of the summed four, in its results column l and
+// rows g, g + 4, g + 8, g + 12.  Step e of a tile of 16 therefore takes the indexes 4 e + g, so that results are the next product's operand as
+// they are; in LDS and in the maps the sixteen stand so that a lane's four are neighbours (dc_place).
 #pragma once
+#include <limits.h>
 #include <mutex>
 #include "common.h"
 
 constexpr int DELTA_CHUNK = 64;
-constexpr int DELTA_LONG = 64;                   // a request that feeds fewer tokens in a step walks them one by one
 constexpr int DELTA_CHUNK_THREADS = 512;
 constexpr int DELTA_LDM = DELTA_CHUNK + 4;       // rows of a [64][64] matrix in LDS
 constexpr int DELTA_MAX_DEVICES = 16;
 
 typedef __attribute__((ext_vector_type(4))) float dc_f32x4;
+typedef __attribute__((ext_vector_type(4))) double dc_f64x4;
+
+// Which requests of a step go through chunks: those that feed `line` tokens or more, unless more than `most` of them do.
+// line: one request, us scanned / in chunks: 64 tokens of 16 heads of 128 gated 47 / 63, per channel 83 / 96, of 64 gated 35 / 36; 100 tokens 68 /
+// 69, 124 / 104, 49 / 38; 128 tokens 83 / 70, 156 / 106, 60 / 39.  Head sizes for which the scan keeps the state in memory (10 us a token) go
+// there from 64 tokens on (40: 646 / 36).
+// most: scans of many requests and heads run side by side and chunks of small heads are padded to 64 channels: 16 requests of 128 tokens,
+// 16 / 32 heads of 16: gated 69 / 100 and 93 / 175, per channel 97 / 124 and 136 / 224; of 64, gated 103 / 112 and 173 / 206, per channel 231 / 143 and
+// 452 / 271; 8 requests of 256, 16 heads of 16: gated 103 / 97; of 128, 32 heads, 16 requests of 128: gated 502 / 512.
+struct DeltaLine {
+    int line, most;
+    // what holds for a step: the least tokens that a request must feed (called by whole waves)
+    __device__ __forceinline__ int of_step(const int *__restrict__ q_start, int n_req) const {
+        if (most == INT_MAX) return line;
+        const int lane = threadIdx.x % WAVE;
+        int longs = 0;
+        for (int r = 0; r < n_req; r += WAVE) {
+            const int at = min(r + lane, n_req - 1);
+            longs += __popcll(__ballot(r + lane < n_req && q_start[at + 1] - q_start[at] >= line));
+        }
+        return longs > most ? INT_MAX : line;
+    }
+};
+inline DeltaLine delta_line(int heads, int dk, bool gated) {
+    const bool scanned = dk % 16 == 0;                                        // the scan has the state in registers
+    const int crowd = scanned && dk <= (gated ? 64 : 32) ? 128 / heads : INT_MAX;
+    return DeltaLine{scanned ? 128 : 64, crowd > 1 ? crowd : 1};              // (one long request always goes there)
+}
 
 struct DeltaChunkArgs {
     const float *prep;                           // [n, heads, 5 dk] (w | al | u | k | r) or, gated, [n, heads, 2 dk + 4] (u | r | g, beta g, log g, 0)
@@ -50,35 +84,41 @@ struct DeltaChunkArgs {
     float *o;                                    // [n, heads * dv]
     const int *q_start, *ctx_len, *state_slot;
     int n_req, heads, dk, dv, tiles;             // tiles: of 16 value columns
+    DeltaLine line;
 };
 
 // The chunks that a step of n tokens in n_req requests can have: every long request's last one may be cut short.
-__host__ __device__ inline int delta_chunk_slots(int n, int n_req) {
-    const int most = n / DELTA_LONG;
+__host__ __device__ inline int delta_chunk_slots(int n, int n_req, int line) {
+    const int most = n / line;
     return n / DELTA_CHUNK + (most < n_req ? most : n_req);
 }
 // Whether a step may hold a long request (every request feeds a token at least).
-inline bool delta_chunks_possible(int n, int n_req, int dk) { return dk <= 128 && n - n_req + 1 >= DELTA_LONG; }
+inline bool delta_chunks_possible(int n, int n_req, int dk, int line) { return dk <= 128 && n - n_req + 1 >= line; }
 inline int delta_padded(int dk) { return dk <= 64 ? 64 : 128; }
-inline size_t delta_chunk_floats(int n, int n_req, int heads, int dk, int dv) {
-    if (!delta_chunks_possible(n, n_req, dk)) return 0;
+inline size_t delta_chunk_floats(int n, int n_req, int heads, int dk, int dv, bool gated) {
+    const int line = delta_line(heads, dk, gated).line;
+    if (!delta_chunks_possible(n, n_req, dk, line)) return 0;
     const size_t D = delta_padded(dk), V = (size_t)(dv + 15) / 16 * 16;
-    return (size_t)delta_chunk_slots(n, n_req) * heads * (D * D + D * V + DELTA_CHUNK * (D + V));
+    return (size_t)delta_chunk_slots(n, n_req, line) * heads * (D * D + D * V + DELTA_CHUNK * (D + V));
 }
 
-__device__ __forceinline__ dc_f32x4 dc_mma(float4 a, dc_f32x4 b, dc_f32x4 c) {
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[0], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[1], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[2], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[3], c, 0, 0, 0);
+__device__ __forceinline__ dc_f64x4 dc_mma(float4 a, dc_f64x4 b, dc_f64x4 c) {
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.x, b[0], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.y, b[1], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.z, b[2], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.w, b[3], c, 0, 0, 0);
     return c;
 }
+// The place of index k of a tile of sixteen among them: a lane's 4 e + g are neighbours.  (The places' indexes are found the same way.)
+__device__ __forceinline__ int dc_place(int k) { return (k & ~15) + k % 4 * 4 + k % 16 / 4; }
 // Where element (row m, index k) of a tile of 16 x 16 stands in memory: in the order in which a wave's lanes take the tile as the left
 // operand, so that the wave reads whole lines.
-__device__ __forceinline__ int dc_operand(int tile, int m, int k) { return (tile * WAVE + k / 4 * 16 + m) * 4 + k % 4; }
+__device__ __forceinline__ int dc_operand(int tile, int m, int k) { return (tile * WAVE + k % 4 * 16 + m) * 4 + k / 4; }
 // Keeps the compiler from holding what it reads from LDS here in registers until it is read again later: that would spill.
 __device__ __forceinline__ void dc_forget() { asm volatile("" ::: "memory"); }
-__device__ __forceinline__ dc_f32x4 dc_vec(float4 v) { return dc_f32x4{v.x, v.y, v.z, v.w}; }
+__device__ __forceinline__ dc_f64x4 dc_vec(float4 v) { return dc_f64x4{v.x, v.y, v.z, v.w}; }
+__device__ __forceinline__ dc_f32x4 dc_round(dc_f64x4 v) { return dc_f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]}; }
+__device__ __forceinline__ dc_f64x4 dc_zero() { return dc_f64x4{0.0, 0.0, 0.0, 0.0}; }
 
 // LDS of `maps`, in floats: the channel-wise rule holds four [64][DK + 4] arrays, of which the first two make room for the four
 // [64][68] matrices; the gated rule two of each.
@@ -87,7 +127,7 @@ template <bool GATED, int DK> struct DeltaMapsLds {
     static constexpr int FRONT = GATED ? ROWS : (2 * ROWS > 4 * MAT ? 2 * ROWS : 4 * MAT);      // (gated: u stays)
     static constexpr int REST = GATED ? ROWS + 2 * MAT : 2 * ROWS;
     static constexpr int DINV = 4 * 16 * 20;
-    static constexpr int SMALL = 512 + DK;        // gated: the sums of log g in two parts, beta g, weights; G_C
+    static constexpr int SMALL = 448 + 2 * DK;    // gated: the sums of log g in two parts, beta g, weights in 64 bits; G_C in 64 bits
     static constexpr int FLOATS = FRONT + REST + DINV + SMALL;
 };
 
@@ -100,16 +140,19 @@ delta_maps_kernel(DeltaChunkArgs p) {
     float *us = dc_lds, *rs = us + L::ROWS;                                   // u~ and r~ (gated: u and r)
     float *ks = dc_lds + L::FRONT, *as = ks + L::ROWS;                        // k~ and al~ (channel-wise)
     float *m_uk = GATED ? rs + L::ROWS : dc_lds, *m_rk = m_uk + L::MAT, *m_ua = m_rk + L::MAT, *m_ra = m_ua + L::MAT;
-    float *dinv = dc_lds + L::FRONT + L::REST, *small = dinv + L::DINV, *g_all = small + 512;
-    float *l_hi = small, *l_lo = l_hi + C, *bg = l_lo + C, *w_end = bg + C, *w_start = w_end + C;        // gated, by token
+    float *dinv = dc_lds + L::FRONT + L::REST, *small = dinv + L::DINV;
+    double *g_all = (double *)small, *w_end = g_all + DK, *w_start = w_end + C;       // by key and by token; g_all and w_end by place
+    float *l_hi = (float *)(w_start + C), *l_lo = l_hi + C, *bg = l_lo + C;           // gated, by token, bg by place
+    static_assert((L::FRONT + L::REST + L::DINV) % 2 == 0, "64-bit numbers stand at even places");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, l16 = lane & 15, head = blockIdx.y;
     // ---- which request's chunk this is
     int t0 = 0, nt = 0;
     {
+        const int line = p.line.of_step(p.q_start, p.n_req);
         int left = blockIdx.x;
         for (int r = 0; r < p.n_req; ++r) {
             const int a = p.q_start[r], b = p.q_start[r + 1], len = b - a;
-            if (len < DELTA_LONG) continue;
+            if (len < line) continue;
             const int chunks = (len + C - 1) / C;
             if (left < chunks) {
                 t0 = a + left * C;
@@ -135,12 +178,11 @@ delta_maps_kernel(DeltaChunkArgs p) {
                 if (lane >= off) l += before;
             }
             const float hi = (float)l, lo = (float)(l - (double)hi);
-            const float end_hi = __shfl(hi, C - 1, WAVE), end_lo = __shfl(lo, C - 1, WAVE);
             l_hi[lane] = hi;
             l_lo[lane] = lo;
-            bg[lane] = b;
-            w_end[lane] = expf((end_hi - hi) + (end_lo - lo));
-            w_start[lane] = expf(hi + lo);
+            bg[dc_place(lane)] = b;
+            w_end[dc_place(lane)] = exp(__shfl(l, C - 1, WAVE) - l);
+            w_start[lane] = exp(l);
         }
 #pragma unroll
         for (int x = tid; x < C * (DK / 4); x += THREADS) {
@@ -186,14 +228,14 @@ delta_maps_kernel(DeltaChunkArgs p) {
             const float *x = s + (size_t)min(t, nt - 1) * heads * row;
             const bool in = t < nt && c < dk;
             const float al = in ? x[dk] : 0.f, u = in ? x[2 * dk] : 0.f, k = in ? x[3 * dk] : 0.f, r = in ? x[4 * dk] : 0.f;
-            us[t * LD + c] = u * (float)before;
+            us[t * LD + c] = (float)(u * before);
             before *= (double)w[e];
-            const float inv = (float)(1.0 / before);
-            rs[t * LD + c] = r * (float)before;
-            ks[t * LD + c] = k * inv;
-            as[t * LD + c] = al * inv;
+            const double inv = 1.0 / before;
+            rs[t * LD + c] = (float)(r * before);
+            ks[t * LD + c] = (float)(k * inv);
+            as[t * LD + c] = (float)(al * inv);
         }
-        if (grp == GROUPS - 1) g_all[c] = (float)before;
+        if (grp == GROUPS - 1) g_all[dc_place(c)] = before;
     }
     __syncthreads();
     // ---- the matrices: waves 0 to 3 a tile of 16 rows of u's, waves 4 to 7 of r's (the longest strips beside the shortest on a SIMD)
@@ -201,11 +243,11 @@ delta_maps_kernel(DeltaChunkArgs p) {
         const bool of_r = wave >= 4;
         const int a = of_r ? 3 - (wave & 3) : wave & 3;
         const float *left = of_r ? rs : us;
-        dc_f32x4 k4[4], a4[4];
+        dc_f64x4 k4[4], a4[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) k4[c] = a4[c] = dc_f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int c = 0; c < 4; ++c) k4[c] = a4[c] = dc_zero();
         for (int x = 0; x < KT; ++x) {
-            const dc_f32x4 b = dc_vec(*(const float4 *)(left + (16 * a + l16) * LD + 16 * x + 4 * g));
+            const dc_f64x4 b = dc_vec(*(const float4 *)(left + (16 * a + l16) * LD + 16 * x + 4 * g));
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 if (c > a) continue;
@@ -214,34 +256,34 @@ delta_maps_kernel(DeltaChunkArgs p) {
                 if constexpr (!GATED) a4[c] = dc_mma(*(const float4 *)(as + at), b, a4[c]);
             }
         }
-        // this lane's results: token t (of the strip), tokens 16 c + 4 g + i
+        // this lane's results: token t (of the strip), tokens 16 c + 4 i + g
         const int t = 16 * a + l16;
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int s = 16 * c + 4 * g + i;
+                const int s = 16 * c + 4 * i + g;
                 const bool in = of_r ? s <= t : s < t;
                 if constexpr (GATED) {
                     const int from = of_r ? t : max(t - 1, 0);
-                    k4[c][i] = in ? k4[c][i] * expf((l_hi[from] - l_hi[s]) + (l_lo[from] - l_lo[s])) : 0.f;
+                    k4[c][i] = in ? k4[c][i] * (double)expf((l_hi[from] - l_hi[s]) + (l_lo[from] - l_lo[s])) : 0.0;
                 } else {
-                    k4[c][i] = in ? k4[c][i] : 0.f;
-                    a4[c][i] = in ? a4[c][i] : 0.f;
+                    k4[c][i] = in ? k4[c][i] : 0.0;
+                    a4[c][i] = in ? a4[c][i] : 0.0;
                 }
             }
         // (channel-wise) u~ and r~ make room: what the column tiles still need of them goes to registers, below
-        dc_f32x4 um[4], rm[4];
+        dc_f64x4 um[4], rm[4];
         if (wave < KT) {
 #pragma unroll
             for (int b = 0; b < 4; ++b)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int s = 16 * b + 4 * g + i;
+                    const int s = 16 * b + 4 * i + g;
                     um[b][i] = us[s * LD + 16 * wave + l16];
                     rm[b][i] = rs[s * LD + 16 * wave + l16];
                     if constexpr (GATED) {
-                        um[b][i] *= s > 0 ? w_start[s - 1] : 1.f;
+                        um[b][i] *= s > 0 ? w_start[s - 1] : 1.0;
                         rm[b][i] *= w_start[s];
                     }
                 }
@@ -250,8 +292,8 @@ delta_maps_kernel(DeltaChunkArgs p) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             if (c > a) continue;
-            *(dc_f32x4 *)((of_r ? m_rk : m_uk) + t * LDM + 16 * c + 4 * g) = k4[c];
-            if constexpr (!GATED) *(dc_f32x4 *)((of_r ? m_ra : m_ua) + t * LDM + 16 * c + 4 * g) = a4[c];
+            *(dc_f32x4 *)((of_r ? m_rk : m_uk) + t * LDM + 16 * c + 4 * g) = dc_round(k4[c]);
+            if constexpr (!GATED) *(dc_f32x4 *)((of_r ? m_ra : m_ua) + t * LDM + 16 * c + 4 * g) = dc_round(a4[c]);
         }
         __syncthreads();
         // ---- the inverses of the four diagonal blocks I + tril(., -1), a column a lane; a row is on its way while the one before is used
@@ -263,37 +305,37 @@ delta_maps_kernel(DeltaChunkArgs p) {
                 next[j] = *(const float4 *)(m + LDM + 4 * j);
                 if constexpr (GATED) bgs[j] = *(const float4 *)(bg + 16 * wave + 4 * j);
             }
-            float col[16];
-            col[0] = lane == 0 ? 1.f : 0.f;
-            dinv[16 * wave * 20 + lane] = col[0];
+            double col[16];
+            col[0] = lane == 0 ? 1.0 : 0.0;
+            dinv[16 * wave * 20 + dc_place(lane)] = (float)col[0];
 #pragma unroll
             for (int i = 1; i < 16; ++i) {
-                float row[16];
+                double row[16];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    row[4 * j] = next[j].x; row[4 * j + 1] = next[j].y; row[4 * j + 2] = next[j].z; row[4 * j + 3] = next[j].w;
-                    if constexpr (GATED) { row[4 * j] *= bgs[j].x; row[4 * j + 1] *= bgs[j].y; row[4 * j + 2] *= bgs[j].z; row[4 * j + 3] *= bgs[j].w; }
+                    row[j] = next[j].x; row[4 + j] = next[j].y; row[8 + j] = next[j].z; row[12 + j] = next[j].w;
+                    if constexpr (GATED) { row[j] *= bgs[j].x; row[4 + j] *= bgs[j].y; row[8 + j] *= bgs[j].z; row[12 + j] *= bgs[j].w; }
                     if (i < 15) next[j] = *(const float4 *)(m + (i + 1) * LDM + 4 * j);
                 }
-                float v = i == lane ? 1.f : 0.f;
+                double v = i == lane ? 1.0 : 0.0;
 #pragma unroll
                 for (int j = 0; j < i; ++j) v -= row[j] * col[j];
                 col[i] = v;
-                dinv[(16 * wave + i) * 20 + lane] = v;
+                dinv[(16 * wave + i) * 20 + dc_place(lane)] = (float)v;
             }
         }
         __syncthreads();
-        // X = T B for 16 columns: lane (l, g) holds rows 16 a + 4 g + i of column l
-        auto solve = [&](dc_f32x4 *x) {
-            dc_f32x4 bx[4];
+        // X = T B for 16 columns: lane (l, g) holds rows 16 a + 4 i + g of column l
+        auto solve = [&](dc_f64x4 *x) {
+            dc_f64x4 bx[4];
             dc_forget();
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-                dc_f32x4 sum = dc_f32x4{0.f, 0.f, 0.f, 0.f};
+                dc_f64x4 sum = dc_zero();
 #pragma unroll
                 for (int c = 0; c < b; ++c) sum = dc_mma(*(const float4 *)((GATED ? m_uk : m_ua) + (16 * b + l16) * LDM + 16 * c + 4 * g), bx[c], sum);
                 x[b] -= sum;
-                x[b] = dc_mma(*(const float4 *)(dinv + (16 * b + l16) * 20 + 4 * g), x[b], dc_f32x4{0.f, 0.f, 0.f, 0.f});
+                x[b] = dc_mma(*(const float4 *)(dinv + (16 * b + l16) * 20 + 4 * g), x[b], dc_zero());
                 bx[b] = x[b];
                 if constexpr (GATED) bx[b] *= dc_vec(*(const float4 *)(bg + 16 * b + 4 * g));
             }
@@ -309,30 +351,29 @@ delta_maps_kernel(DeltaChunkArgs p) {
             }
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-                dc_f32x4 sum = dc_f32x4{0.f, 0.f, 0.f, 0.f};
+                dc_f64x4 sum = dc_zero();
 #pragma unroll
                 for (int c = 0; c <= b; ++c) sum = dc_mma(*(const float4 *)((GATED ? m_rk : m_ra) + (16 * b + l16) * LDM + 16 * c + 4 * g), um[c], sum);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) pp[dc_operand(b * KT + wave, 4 * g + i, l16)] = rm[b][i] - sum[i];
+                for (int i = 0; i < 4; ++i) pp[dc_operand(b * KT + wave, 4 * i + g, l16)] = (float)(rm[b][i] - sum[i]);
             }
             if constexpr (GATED) {
 #pragma unroll
-                for (int b = 0; b < 4; ++b) um[b] *= dc_vec(*(const float4 *)(w_end + 16 * b + 4 * g));
+                for (int b = 0; b < 4; ++b) um[b] *= *(const dc_f64x4 *)(w_end + 16 * b + 4 * g);
             }
 #pragma unroll 4
             for (int y = 0; y < KT; ++y) {
-                if (y % 2 == 0) dc_forget();
-                dc_f32x4 sum = dc_f32x4{0.f, 0.f, 0.f, 0.f};
+                dc_forget();
+                dc_f64x4 sum = dc_zero();
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
-                    const float *at = (GATED ? us : as) + (16 * b + 4 * g) * LD + 16 * y + l16;
-                    sum = dc_mma(make_float4(at[0], at[LD], at[2 * LD], at[3 * LD]), um[b], sum);
+                    const float *at = (GATED ? us : as) + (16 * b + g) * LD + 16 * y + l16;
+                    sum = dc_mma(make_float4(at[0], at[4 * LD], at[8 * LD], at[12 * LD]), um[b], sum);
                 }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int key = 16 * y + 4 * g + i;
-                    const float one = key == 16 * wave + l16 ? 1.f : 0.f;
-                    ff[dc_operand(y * KT + wave, 4 * g + i, l16)] = GATED ? one * w_start[C - 1] - sum[i] : g_all[key] * (one - sum[i]);
+                    const double one = 16 * y + 4 * i + g == 16 * wave + l16 ? 1.0 : 0.0;
+                    ff[dc_operand(y * KT + wave, 4 * i + g, l16)] = (float)(GATED ? one * w_start[C - 1] - sum[i] : g_all[16 * y + 4 * g + i] * (one - sum[i]));
                 }
             }
         }
@@ -341,21 +382,21 @@ delta_maps_kernel(DeltaChunkArgs p) {
         for (int tile = wave; tile < p.tiles; tile += WAVES) {
             float *qq = p.q + no * C * width, *hh = p.h + no * DK * width;
             const int col = tile * 16 + l16;
-            dc_f32x4 v[4], x[4];
+            dc_f64x4 v[4], x[4];
             dc_forget();
 #pragma unroll
             for (int b = 0; b < 4; ++b)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int s = 16 * b + 4 * g + i;
+                    const int s = 16 * b + 4 * i + g;
                     const size_t tok = t0 + min(s, nt - 1);
                     const int cc = head * dv + min(col, dv - 1);
                     const float e = p.vf ? p.vf[tok * heads * dv + cc] : to_f32(((const T *)p.proj)[tok * p.row_stride + p.off_v + cc]);
-                    v[b][i] = s < nt && col < dv ? e : 0.f;
+                    v[b][i] = s < nt && col < dv ? (double)e : 0.0;
                 }
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-                x[b] = dc_f32x4{0.f, 0.f, 0.f, 0.f};
+                x[b] = dc_zero();
 #pragma unroll
                 for (int c = 0; c <= b; ++c) x[b] = dc_mma(*(const float4 *)(m_uk + (16 * b + l16) * LDM + 16 * c + 4 * g), v[c], x[b]);
             }
@@ -368,32 +409,32 @@ delta_maps_kernel(DeltaChunkArgs p) {
             }
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-                dc_f32x4 sum = dc_f32x4{0.f, 0.f, 0.f, 0.f};
+                dc_f64x4 sum = dc_zero();
 #pragma unroll
                 for (int c = 0; c <= b; ++c) {
                     const int at = (16 * b + l16) * LDM + 16 * c + 4 * g;
                     sum = dc_mma(*(const float4 *)(m_rk + at), v[c], sum);
                     if constexpr (!GATED) sum = dc_mma(*(const float4 *)(m_ra + at), x[c], sum);
                 }
-                *(dc_f32x4 *)(qq + ((size_t)(tile * (C / 16) + b) * WAVE + lane) * 4) = sum;
+                *(dc_f32x4 *)(qq + ((size_t)(tile * (C / 16) + b) * WAVE + lane) * 4) = dc_round(sum);
             }
             if constexpr (GATED) {
 #pragma unroll
-                for (int b = 0; b < 4; ++b) v[b] *= dc_vec(*(const float4 *)(w_end + 16 * b + 4 * g));
+                for (int b = 0; b < 4; ++b) v[b] *= *(const dc_f64x4 *)(w_end + 16 * b + 4 * g);
             }
 #pragma unroll 4
             for (int y = 0; y < KT; ++y) {
-                if (y % 2 == 0) dc_forget();
-                dc_f32x4 sum = dc_f32x4{0.f, 0.f, 0.f, 0.f};
+                dc_forget();
+                dc_f64x4 sum = dc_zero();
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
-                    const int at = (16 * b + 4 * g) * LD + 16 * y + l16;
+                    const int at = (16 * b + g) * LD + 16 * y + l16;
                     const float *kp = (GATED ? us : ks) + at;
-                    sum = dc_mma(make_float4(kp[0], kp[LD], kp[2 * LD], kp[3 * LD]), v[b], sum);
-                    if constexpr (!GATED) sum = dc_mma(make_float4(as[at], as[at + LD], as[at + 2 * LD], as[at + 3 * LD]), x[b], sum);
+                    sum = dc_mma(make_float4(kp[0], kp[4 * LD], kp[8 * LD], kp[12 * LD]), v[b], sum);
+                    if constexpr (!GATED) sum = dc_mma(make_float4(as[at], as[at + 4 * LD], as[at + 8 * LD], as[at + 12 * LD]), x[b], sum);
                 }
-                if constexpr (!GATED) sum *= dc_vec(*(const float4 *)(g_all + 16 * y + 4 * g));
-                *(dc_f32x4 *)(hh + ((size_t)(tile * KT + y) * WAVE + lane) * 4) = sum;
+                if constexpr (!GATED) sum *= *(const dc_f64x4 *)(g_all + 16 * y + 4 * g);
+                *(dc_f32x4 *)(hh + ((size_t)(tile * KT + y) * WAVE + lane) * 4) = dc_round(sum);
             }
         }
     }
@@ -408,20 +449,21 @@ template <int DK>
 __global__ void __launch_bounds__((DK / 16 + DELTA_CHUNK / 16) * WAVE)
 delta_chain_kernel(DeltaChunkArgs p) {
     constexpr int C = DELTA_CHUNK, KT = DK / 16, LD = DK + 4, AHEAD = 3;
-    __shared__ __attribute__((aligned(16))) float st[2][16 * LD];             // S of these columns, a column a row
+    __shared__ __attribute__((aligned(16))) double st[2][16 * LD];            // S of these columns, a column a row, by place
     const int r = blockIdx.x, head = blockIdx.y, tile = blockIdx.z;
     const int t_first = p.q_start[r], t_end = p.q_start[r + 1], q_len = t_end - t_first;
-    if (q_len < DELTA_LONG) return;
+    const int line = p.line.of_step(p.q_start, p.n_req);
+    if (q_len < line) return;
     int slot = 0;
     for (int x = 0; x < r; ++x) {
         const int len = p.q_start[x + 1] - p.q_start[x];
-        if (len >= DELTA_LONG) slot += (len + C - 1) / C;
+        if (len >= line) slot += (len + C - 1) / C;
     }
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, l16 = lane & 15;
     const int dk = p.dk, dv = p.dv, heads = p.heads, width = p.tiles * 16, col = tile * 16 + l16;
     float *mat = p.state + (size_t)p.state_slot[r] * p.slot_stride + (size_t)head * dk * dv;
     const bool of_state = wave < KT;
-    const int y = of_state ? wave : wave - KT, row0 = 16 * y + 4 * g;         // this wave's rows: key channels, or the chunk's tokens
+    const int y = of_state ? wave : wave - KT, row0 = 16 * y + g;             // this wave's rows row0 + 4 i: key channels, or the chunk's tokens
     // the wave's rows of the maps of chunk number `slot + c`
     const float *left = of_state ? p.f + (size_t)y * KT * 256 : p.p + (size_t)y * KT * 256;
     const float *right = of_state ? p.h + (size_t)(tile * KT + y) * 256 : p.q + (size_t)(tile * (C / 16) + y) * 256;
@@ -435,13 +477,13 @@ delta_chain_kernel(DeltaChunkArgs p) {
         for (int x = 0; x < KT; ++x) av[x] = *(const dc_f32x4 *)(lp + 256 * x);
         bv = *(const dc_f32x4 *)(right + no * right_step + 4 * lane);
     };
-    dc_f32x4 s = dc_f32x4{0.f, 0.f, 0.f, 0.f};
+    dc_f64x4 s = dc_zero();
     if (of_state) {
         const bool fresh = p.ctx_len[r] - q_len == 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (!fresh && row0 + i < dk && col < dv) s[i] = mat[(size_t)(row0 + i) * dv + col];
-        *(dc_f32x4 *)(st[0] + l16 * LD + row0) = s;
+            if (!fresh && row0 + 4 * i < dk && col < dv) s[i] = mat[(size_t)(row0 + 4 * i) * dv + col];
+        *(dc_f64x4 *)(st[0] + l16 * LD + 16 * y + 4 * g) = s;
     }
 #pragma unroll
     for (int k = 0; k < AHEAD; ++k)
@@ -453,17 +495,18 @@ delta_chain_kernel(DeltaChunkArgs p) {
         for (int k = 0; k < AHEAD; ++k) {
             const int c = c0 + k;
             if (c >= chunks) break;
-            dc_f32x4 old[KT], s2 = dc_f32x4{0.f, 0.f, 0.f, 0.f};
-            s = b[k];
+            dc_f64x4 s2 = dc_zero();
+            s = dc_f64x4{b[k][0], b[k][1], b[k][2], b[k][3]};
 #pragma unroll
-            for (int x = 0; x < KT; ++x) old[x] = *(const dc_f32x4 *)(st[turn] + l16 * LD + 16 * x + 4 * g);
-#pragma unroll
-            for (int x = 0; x < KT; x += 2)
+            for (int x = 0; x < KT; x += 2) {
+                const dc_f64x4 old = *(const dc_f64x4 *)(st[turn] + l16 * LD + 16 * x + 4 * g);
+                const dc_f64x4 old2 = *(const dc_f64x4 *)(st[turn] + l16 * LD + 16 * x + 16 + 4 * g);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k][x][e], old[x][e], s, 0, 0, 0);
-                    s2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k][x + 1][e], old[x + 1][e], s2, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[k][x][e], old[e], s, 0, 0, 0);
+                    s2 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[k][x + 1][e], old2[e], s2, 0, 0, 0);
                 }
+            }
             s += s2;
             // the sums stand before any branch: behind one that is taken the compiler (ROCm 7.2) counts too few wait states between a
             // matrix instruction and the first use of its result, and the use reads the value of before
@@ -471,12 +514,12 @@ delta_chain_kernel(DeltaChunkArgs p) {
             if (c + AHEAD < chunks) fetch(c + AHEAD, a[k], b[k]);
             turn ^= 1;
             if (of_state) {
-                *(dc_f32x4 *)(st[turn] + l16 * LD + row0) = s;
+                *(dc_f64x4 *)(st[turn] + l16 * LD + 16 * y + 4 * g) = s;
             } else if (col < dv) {
                 const int t0 = t_first + c * C + row0;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (t0 + i < t_end) p.o[((size_t)(t0 + i) * heads + head) * dv + col] = s[i];
+                    if (t0 + 4 * i < t_end) p.o[((size_t)(t0 + 4 * i) * heads + head) * dv + col] = (float)s[i];
             }
             lds_barrier();
         }
@@ -484,7 +527,7 @@ delta_chain_kernel(DeltaChunkArgs p) {
     if (of_state) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (row0 + i < dk && col < dv) mat[(size_t)(row0 + i) * dv + col] = s[i];
+            if (row0 + 4 * i < dk && col < dv) mat[(size_t)(row0 + 4 * i) * dv + col] = (float)s[i];
     }
 }
 
@@ -514,7 +557,7 @@ static int delta_chunks_dk(const DeltaChunkArgs &p, int slots, hipStream_t strea
 // The long requests of a step; `work` holds delta_chunk_floats floats.
 template <class T, bool GATED>
 static int delta_chunks_launch(DeltaChunkArgs p, float *work, int n, hipStream_t stream) {
-    const int slots = delta_chunk_slots(n, p.n_req);
+    const int slots = delta_chunk_slots(n, p.n_req, p.line.line);
     const size_t D = delta_padded(p.dk), all = (size_t)slots * p.heads;
     p.tiles = (p.dv + 15) / 16;
     const size_t V = (size_t)p.tiles * 16;

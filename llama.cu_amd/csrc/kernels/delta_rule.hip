@@ -13,11 +13,10 @@
 //           of its lanes from the request's first token of the step to its last);
 //   out   (parallel): o of each head divided by its root mean square, times a weight, times
 //           sigmoid(gate).
-// A request that feeds DELTA_LONG tokens or more in a step goes through chunks on the matrix cores instead of the scan
-// (delta_chunks.h, heads of up to 128 key channels) if its outputs are rounded to bfloat16: the chunks' 32-bit results are 4e-7 of
-// their size off the recurrence in 64 bits, the scan's 1e-7 to 8e-7 (the smaller the faster a state decays; over 640 to 1,000 tokens).
-// A token's result depends on the tokens before it in its request only; portions below DELTA_LONG tokens are folded in in an
-// order of operations that does not depend on how the request was cut into them, longer ones change roundings.
+// A request that feeds many tokens in a step goes through chunks on the matrix cores instead of the scan (delta_chunks.h, which says from how many on:
+// 128 for most head sizes) if its outputs are rounded to bfloat16; 32-bit models keep the scan, whose bits do not depend on the cut of a prompt.
+// A token's result depends on the tokens before it in its request only; portions that are scanned are folded in in an
+// order of operations that does not depend on how the request was cut into them, chunks change roundings.
 #include <limits.h>
 #include "common.h"
 #include "lane_moves.h"
@@ -119,10 +118,10 @@ template <class T, int DK, bool GATED>
 __global__ void __launch_bounds__(64)
 delta_scan_kernel(const T *__restrict__ proj, int row_stride, int off_v, const float *__restrict__ vf, const float *__restrict__ prep,
                   float *__restrict__ state, size_t slot_stride, float *__restrict__ o, const int *__restrict__ q_start,
-                  const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int heads, int dk_rt, int dv, int below) {
+                  const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int heads, int dk_rt, int dv, int n_req, DeltaLine line) {
     const int r = blockIdx.x, h = blockIdx.y;
     const int t0 = q_start[r], t1 = q_start[r + 1];
-    if (t1 - t0 >= below) return;                             // a request for the chunks
+    if (line.line != INT_MAX && t1 - t0 >= line.of_step(q_start, n_req)) return;      // a request for the chunks
     const bool fresh = ctx_len[r] - (t1 - t0) == 0;          // the request's first token: the state starts at zero
     if constexpr (DK > 0) {
         constexpr int SCAN_GROUPS = scan_groups<T, DK>(), SCAN_COLS = WAVE / SCAN_GROUPS;
@@ -266,19 +265,20 @@ template <class T, bool GATED = false>
 static int delta_scan_launch(const T *proj, int row_stride, int off_v, const float *vf, const float *prep, float *work, float *state,
                              size_t slot_stride, float *o, const int *q_start, const int *ctx_len, const int *state_slot,
                              int n, int n_req, int heads, int dk, int dv, hipStream_t stream) {
-    int below = INT_MAX;
-    if (work && delta_chunks_possible(n, n_req, dk)) {
+    DeltaLine line = {INT_MAX, 0};
+    const DeltaLine chunks = delta_line(heads, dk, GATED);
+    if (work && delta_chunks_possible(n, n_req, dk, chunks.line)) {
         DeltaChunkArgs c = {};
         c.prep = prep; c.proj = proj; c.row_stride = row_stride; c.off_v = off_v; c.vf = vf;
         c.state = state; c.slot_stride = slot_stride; c.o = o;
         c.q_start = q_start; c.ctx_len = ctx_len; c.state_slot = state_slot;
-        c.n_req = n_req; c.heads = heads; c.dk = dk; c.dv = dv;
+        c.n_req = n_req; c.heads = heads; c.dk = dk; c.dv = dv; c.line = chunks;
         const int rc = delta_chunks_launch<T, GATED>(c, work, n, stream);
         if (rc != LCU_OK) return rc;
-        if (n_req == 1) return LCU_OK;                        // (its one request is long: n >= DELTA_LONG)
-        below = DELTA_LONG;
+        if (n_req == 1) return LCU_OK;                        // (its one request is long)
+        line = chunks;
     }
-#define SCAN(DK) delta_scan_kernel<T, DK, GATED><<<dim3(n_req, heads, (dv + (DK ? 64 / scan_groups<T, DK>() : 64) - 1) / (DK ? 64 / scan_groups<T, DK>() : 64)), dim3(64), 0, stream>>>(proj, row_stride, off_v, vf, prep, state, slot_stride, o, q_start, ctx_len, state_slot, heads, dk, dv, below)
+#define SCAN(DK) delta_scan_kernel<T, DK, GATED><<<dim3(n_req, heads, (dv + (DK ? 64 / scan_groups<T, DK>() : 64) - 1) / (DK ? 64 / scan_groups<T, DK>() : 64)), dim3(64), 0, stream>>>(proj, row_stride, off_v, vf, prep, state, slot_stride, o, q_start, ctx_len, state_slot, heads, dk, dv, n_req, line)
     switch (dk) {
     case 16: SCAN(16); break;
     case 32: SCAN(32); break;
@@ -320,8 +320,15 @@ static int delta_rule_t(const T *proj, int row_stride, int off_r, int off_k, int
 // weight: [heads * dv], all 32-bit.  prep: scratch [n, heads, 5, dk], o: scratch [n, heads * dv], work: scratch of
 // lcu_delta_work_floats floats (null: every request is scanned token by token), all 32-bit.
 // state: [slots, heads, dk, dv] 32-bit.  out: [n, heads * dv] of `type`.
-LCU_API long long lcu_delta_work_floats(int n, int n_req, int heads, int dk, int dv) {
-    return n > 0 && n_req > 0 && heads > 0 && dk > 0 && dv > 0 ? (long long)delta_chunk_floats(n, n_req, heads, dk, dv) : 0;
+// The tokens that a request must feed for chunks, and in *most the requests that may.
+LCU_API int lcu_delta_line(int heads, int dk, int gated, int *most) {
+    const DeltaLine line = heads > 0 && dk > 0 && dk <= 128 ? delta_line(heads, dk, gated) : DeltaLine{INT_MAX, 0};
+    *most = line.most;
+    return line.line;
+}
+
+LCU_API long long lcu_delta_work_floats(int n, int n_req, int heads, int dk, int dv, int gated) {
+    return n > 0 && n_req > 0 && heads > 0 && dk > 0 && dv > 0 ? (long long)delta_chunk_floats(n, n_req, heads, dk, dv, gated) : 0;
 }
 
 LCU_API int lcu_delta_rule(const void *proj, int type, int row_stride, int off_r, int off_k, int off_v, int off_g,
@@ -366,6 +373,7 @@ gated_delta_prep_kernel(const float *__restrict__ qkv, const float *__restrict__
     const float beta = sigmoidf_(row[off_b + h]);
     const float lg = -expf(a_log[h]) * softplus_(row[off_a + h] + dt_bias[h]), g = expf(lg);
     float sq = 0.f, sk = 0.f;
+#pragma unroll 4
     for (int i = lane; i < dk; i += 64) {
         sq += q[i] * q[i];
         sk += k[i] * k[i];
@@ -374,11 +382,13 @@ gated_delta_prep_kernel(const float *__restrict__ qkv, const float *__restrict__
     sk = wave_sum_in_place(sk);
     const float qf = 1.0f / sqrtf(sq + 1e-6f) / sqrtf((float)dk), kf = 1.0f / sqrtf(sk + 1e-6f);
     float *out = prep + (size_t)item * (2 * dk + 4);
+#pragma unroll 4
     for (int i = lane; i < dk; i += 64) {
         out[i] = k[i] * kf;
         out[dk + i] = q[i] * qf;
     }
     if (lane < 4) out[2 * dk + lane] = lane == 0 ? g : lane == 1 ? beta * g : lane == 2 ? lg : 0.f;
+#pragma unroll 4
     for (int j = lane; j < dv; j += 64) vb[(size_t)item * dv + j] = beta * v[j];
 }
 

@@ -1366,14 +1366,20 @@ def qk_norm_store(qkv: torch.Tensor, positions: torch.Tensor, n_heads: int, n_kv
 # ------------------------------------------------------------------ the generalised delta rule
 
 
-def _delta_work(lib, n: int, n_req: int, heads: int, key_dim: int, value_dim: int, out: torch.Tensor) -> Optional[torch.Tensor]:
+def _delta_work(lib, step, heads: int, key_dim: int, value_dim: int, gated: bool, out: torch.Tensor) -> Optional[torch.Tensor]:
     """Scratch memory for the delta rules' chunks.  None: everything is scanned token by token, because the step holds no
-    request that feeds enough tokens for chunks, or because the outputs are 32-bit (a chunk's are 4e-7 of their size off the
-    exact ones, where the scan's may be only 1e-7 off; rounded to bfloat16 both are the same)."""
+    request that feeds enough tokens for chunks, or because the outputs are 32-bit: a 32-bit model computes the same bits
+    for a token however its prompt is cut.  (A captured step is replayed for other requests of the same total: there the
+    kernels themselves look who feeds how many, as they always do, and only the total decides whether they are launched.)"""
     if out.dtype == torch.float32:
         return None
+    if not torch.cuda.is_current_stream_capturing():
+        most = ctypes.c_int()
+        line = lib.lcu_delta_line(heads, key_dim, int(gated), ctypes.byref(most))
+        if not 0 < sum(q >= line for q in step.q_lens) <= most.value:
+            return None
     lib.lcu_delta_work_floats.restype = ctypes.c_longlong
-    floats = lib.lcu_delta_work_floats(n, n_req, heads, key_dim, value_dim)
+    floats = lib.lcu_delta_work_floats(step.n, step.n_req, heads, key_dim, value_dim, int(gated))
     return torch.empty(floats, dtype=torch.float32, device=out.device) if floats else None
 
 
@@ -1412,7 +1418,7 @@ def delta_rule(proj: torch.Tensor, offsets: Dict[str, int], w2_t: torch.Tensor, 
     prep = torch.empty((n, heads, 5, key_dim), dtype=torch.float32, device=proj.device)
     o = torch.empty((n, hv), dtype=torch.float32, device=proj.device)
     lib = build.load("delta_rule")
-    work = _delta_work(lib, n, step.n_req, heads, key_dim, value_dim, out)
+    work = _delta_work(lib, step, heads, key_dim, value_dim, False, out)
     _check(lib.lcu_delta_rule(_ptr(proj), _type(proj, "delta projections"), proj.stride(0), offsets["r"], offsets["k"], offsets["v"],
                               offsets["g"], offsets["a"], offsets["l"], _ptr(w2_t), _ptr(w0), _ptr(a_bias), _ptr(weight), _ptr(prep),
                               _ptr(work), _ptr(o), _ptr(state), _ptr(out), _ptr(step.q_start), _ptr(step.ctx_len), _ptr(step.state_slot), n,
@@ -2178,7 +2184,7 @@ def gated_delta_rule(qkv: torch.Tensor, rows: torch.Tensor, off_a: int, off_b: i
     o = torch.empty((n, hv), dtype=torch.float32, device=qkv.device)
     out = torch.empty((n, hv), dtype=out_dtype, device=qkv.device)
     lib = build.load("delta_rule")
-    work = _delta_work(lib, n, step.n_req, heads, key_dim, value_dim, out)
+    work = _delta_work(lib, step, heads, key_dim, value_dim, True, out)
     _check(lib.lcu_gated_delta_rule(_ptr(qkv), _ptr(rows), rows.stride(0), int(off_a), int(off_b), int(off_g), _ptr(a_log), _ptr(dt_bias),
                                     _ptr(weight), _ptr(prep), _ptr(vb), _ptr(work), _ptr(o), _ptr(state), ctypes.c_longlong(slot_stride), _ptr(out),
                                     _type(out, "gated delta out"), _ptr(step.q_start), _ptr(step.ctx_len), _ptr(step.state_slot), n,

@@ -60,7 +60,8 @@ def run_general(args, proj, heads, dim, portions):
 
 @pytest.mark.parametrize("heads,dim,portions,decay", [
     (2, 128, [64], 0.0), (1, 128, [65, 63, 64], 0.0), (2, 128, [129], 9.0), (2, 64, [127, 1, 66], -3.0),
-    (3, 20, [200, 129], 0.0), (1, 72, [128, 128], 9.0), (2, 16, [191], -9.0), (1, 112, [100, 70], 0.0)])
+    (3, 20, [200, 129], 0.0), (1, 72, [128, 128], 9.0), (2, 16, [191], -9.0), (1, 112, [100, 70], 0.0),
+    (2, 128, [128, 127, 130], 0.0), (1, 64, [192, 1, 193], 3.0), (1, 48, [255], 0.0)])
 def test_the_generalised_rule_in_chunks(heads, dim, portions, decay):
     """``decay`` 9: every decay is as small as the rule allows (0.545 a token); -9: close to 1."""
     args, proj, want, S = general(sum(portions), heads, dim, 3, decay, seed=11)
@@ -92,7 +93,8 @@ def gated(T, heads, qk_heads, dk, dv, gate, seed):
 
 @pytest.mark.parametrize("heads,qk_heads,dk,dv,portions,gate", [
     (2, 1, 128, 128, [64], 0.0), (2, 2, 128, 128, [65, 63, 130], -4.0), (4, 2, 64, 20, [127, 1, 66], 0.0), (1, 1, 24, 40, [200], 80.0),
-    (3, 1, 72, 136, [128, 65], 3.0), (2, 2, 16, 16, [191], -9.0), (1, 1, 128, 272, [100], 0.0)])
+    (3, 1, 72, 136, [128, 65], 3.0), (2, 2, 16, 16, [191], -9.0), (1, 1, 128, 272, [100], 0.0),
+    (2, 1, 128, 128, [128, 127, 191], -4.0), (1, 1, 64, 20, [192, 1, 193], 0.0), (1, 1, 128, 272, [255], 0.0)])
 def test_the_gated_rule_in_chunks(heads, qk_heads, dk, dv, portions, gate):
     """``gate`` 80: a token's decay is 0 in 32 bits; -9: it is 1 but for the fourth digit."""
     from llama_cu_amd.kernels import ops
@@ -108,3 +110,65 @@ def test_the_gated_rule_in_chunks(heads, qk_heads, dk, dv, portions, gate):
     assert (state[0] == 7.0).all()
     assert_close(state[1], S, 5e-6, "state")
     assert_close(torch.cat(outs), want, 2.0 ** -8 + 1e-5, "outputs")
+
+
+def rms_off(got, want):
+    return float((got.cpu().to(F64) - want).norm() / want.norm())
+
+
+def raw(kind, dim, decay, T, chunks, seed):
+    """How far the last state and the outputs, both in 32 bits, are off the recurrence in 64 bits (2-norm): scanned, or in chunks."""
+    import ctypes
+    from llama_cu_amd.kernels import build, ops
+    lib, p, heads, step = build.load("delta_rule"), ops._ptr, 2, hand_step([T], [T], [0])
+    hv = heads * dim
+    state, o, out = torch.zeros(1, heads, dim, dim, device="cuda"), torch.empty(T, hv, device="cuda"), torch.empty(T, hv, device="cuda")
+    lib.lcu_delta_work_floats.restype = ctypes.c_longlong
+    floats = lib.lcu_delta_work_floats(T, 1, heads, dim, dim, int(kind == "gated"))
+    assert floats > 0
+    work = torch.empty(floats, device="cuda") if chunks else None
+    steps = (p(step.q_start), p(step.ctx_len), p(step.state_slot), T, 1, heads)
+    if kind == "gated":
+        args, qkv, rows, want, S = gated(T, heads, heads, dim, dim, decay, seed)
+        q, r = qkv.cuda(), rows.cuda()
+        prep, vb = torch.empty(T, heads, 2 * dim + 4, device="cuda"), torch.empty(T, hv, device="cuda")
+        rc = lib.lcu_gated_delta_rule(p(q), p(r), r.stride(0), 0, heads, 2 * heads, *(p(a) for a in args), p(prep), p(vb), p(work), p(o), p(state),
+                                      ctypes.c_longlong(hv * dim), p(out), ops._type(out, "out"), *steps, heads, dim, dim, ctypes.c_float(EPS), ops._stream())
+    else:
+        (off, *args), proj, want, S = general(T, heads, dim, 8, decay, seed)
+        rows = proj.float().cuda()
+        prep = torch.empty(T, heads, 5, dim, device="cuda")
+        rc = lib.lcu_delta_rule(p(rows), ops._type(rows, "rows"), rows.stride(0), *(off[c] for c in "rkvgal"), *(p(a) for a in args), p(prep), p(work),
+                                p(o), p(state), p(out), *steps, dim, dim, 8, ctypes.c_float(EPS), ops._stream())
+    assert rc == 0
+    return rms_off(out, want), rms_off(state[0], S)
+
+
+@pytest.mark.parametrize("kind,decay", [("general", 9.0), ("general", 0.0), ("general", -3.0), ("general", -9.0), ("gated", 3.0), ("gated", 0.0),
+                                        ("gated", -4.0), ("gated", -9.0)])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_chunks_are_no_further_off_than_the_scan(kind, decay, dim):
+    """Decays from the smallest to almost 1: what chunks make, before anything is rounded to bfloat16, beside what the scan makes (mean of three
+    seeds; a tenth and 1e-8 for what seeds differ by)."""
+    scan, chunk = ([raw(kind, dim, decay, 320, c, s) for s in (1, 2, 3)] for c in (False, True))
+    for what, a, b in zip(("outputs", "state"), zip(*scan), zip(*chunk)):
+        assert sum(b) <= 1.1 * sum(a) + 3e-8, f"{what}: scanned {sum(a) / 3:.2e}, in chunks {sum(b) / 3:.2e}"
+
+
+@pytest.mark.parametrize("dim,heads,requests", [(16, 40, 4), (64, 8, 17)])
+def test_many_long_requests_of_small_heads_are_scanned(dim, heads, requests):
+    """More long requests than chunks are good for: the bits that every request has scanned alone in portions too short for chunks."""
+    from llama_cu_amd.kernels import ops
+    T = 130
+    args, qkv, rows, want, S = gated(T, heads, heads, dim, dim, -4.0, seed=3)
+    q, r = qkv.cuda(), rows.cuda()
+    state = torch.full((requests, heads, dim, dim), 7.0, device="cuda")
+    all_of = ops.gated_delta_rule(q.repeat(requests, 1), r.repeat(requests, 1), 0, heads, 2 * heads, *args, state,
+                                  hand_step([T] * requests, [T] * requests, list(range(requests))), heads, heads, dim, dim, EPS, torch.bfloat16)
+    alone, one = torch.full((1, heads, dim, dim), 7.0, device="cuda"), []
+    for a, b in ((0, 60), (60, T)):
+        one.append(ops.gated_delta_rule(q[a:b].contiguous(), r[a:b].contiguous(), 0, heads, 2 * heads, *args, alone, hand_step([b - a], [b], [0]),
+                                        heads, heads, dim, dim, EPS, torch.bfloat16))
+    one = torch.cat(one)
+    for k in range(requests):
+        assert torch.equal(all_of[k * T:(k + 1) * T], one) and torch.equal(state[k], alone[0])
