@@ -11,7 +11,7 @@
 // Two kernels: `maps` makes F, H, P and Q of every chunk and head at once; `chain` walks a request's chunks, 16 value columns a
 // workgroup, and applies them.  A token alone (delta_scan_kernel) is a chain of 0.55 us a token, 0.9 us and more where the decay is per
 // channel; a chunk is one of 3.6 us.  2,048 tokens of one request, 16 heads of 128, the whole rule with its preparation and output kernels:
-// gated 1,170 us scanned, 254 in chunks; with decays per channel 2,420 scanned, 350 in chunks (with 32-bit products 175 and 225, and a larger error,
+// gated 1,170 us scanned, 255 in chunks; with decays per channel 2,420 scanned, 320 in chunks (with 32-bit products 175 and 225, and a larger error,
 // below).
 //
 // What bounds them: `maps` runs 4,300 (channel-wise 6,300) matrix instructions of 64 cycles a chunk and head, 28 (42) us on a compute
@@ -22,6 +22,10 @@
 // The decays per channel are at least exp(-exp(-1/2)) = 0.545 a token, so G over a chunk stays above 1e-17 and 1 / G below 1e17: the
 // products u~_t k~_s are of the size of u_t k_s again and lose nothing (a quotient of two rounded numbers).  The gated rule's one decay
 // may be as small as it likes: there the products u k^T and r k^T are weighted by exp(L_t - L_s) <= 1, L the sums of log g in 64-bit.
+//
+// A chunk multiplies what is not yet there by zeros (the triangles' other halves, tokens beyond the end), which an infinity or NaN does not
+// forgive: it would reach the tokens before it.  So a chunk in which something is not finite, or so large (DELTA_TAME) that a product might not be, is
+// marked by `maps`, and `chain` walks the tokens of that head and request one by one.
 //
 // Products and sums are 64-bit (v_mfma_f64_16x16x4_f64, half the rate of the 32-bit instruction), what is held between them is 32-bit, but for
 // the state on its way along the chain: one rounding each of u~, r~, k~, al~, the masked matrices and the maps.  Sums of 64 and 128 terms in
@@ -36,11 +40,15 @@
 #include <limits.h>
 #include <mutex>
 #include "common.h"
+#include "lane_moves.h"
 
 constexpr int DELTA_CHUNK = 64;
 constexpr int DELTA_CHUNK_THREADS = 512;
 constexpr int DELTA_LDM = DELTA_CHUNK + 4;       // rows of a [64][64] matrix in LDS
 constexpr int DELTA_MAX_DEVICES = 16;
+constexpr float DELTA_TAME = 1e12f;              // vectors up to here: products of two, times 1 / G, stay below 1e42 in 64 bits, F and H below 1e28
+__device__ __forceinline__ bool dc_wild(float x) { return !(fabsf(x) <= DELTA_TAME); }
+__device__ __forceinline__ bool dc_wild(float4 v) { return dc_wild(v.x) || dc_wild(v.y) || dc_wild(v.z) || dc_wild(v.w); }
 
 typedef __attribute__((ext_vector_type(4))) float dc_f32x4;
 typedef __attribute__((ext_vector_type(4))) double dc_f64x4;
@@ -79,6 +87,8 @@ struct DeltaChunkArgs {
     const float *vf;
     float *f, *h, *p, *q;                        // [slot][head] of [DK][DK], [DK][16 tiles], [64][DK], [64][16 tiles], in tiles of 16 x 16: F
                                                  // and P as left operands [row tile][index tile], H and Q as results [column tile][row tile]
+    int *wild;                                   // [slot][head]: whether the chunk must be walked token by token
+    int gated, bf16;                             // the form of prep; the type of proj
     float *state;
     size_t slot_stride;
     float *o;                                    // [n, heads * dv]
@@ -99,7 +109,7 @@ inline size_t delta_chunk_floats(int n, int n_req, int heads, int dk, int dv, bo
     const int line = delta_line(heads, dk, gated).line;
     if (!delta_chunks_possible(n, n_req, dk, line)) return 0;
     const size_t D = delta_padded(dk), V = (size_t)(dv + 15) / 16 * 16;
-    return (size_t)delta_chunk_slots(n, n_req, line) * heads * (D * D + D * V + DELTA_CHUNK * (D + V));
+    return (size_t)delta_chunk_slots(n, n_req, line) * heads * (D * D + D * V + DELTA_CHUNK * (D + V) + 1);
 }
 
 __device__ __forceinline__ dc_f64x4 dc_mma(float4 a, dc_f64x4 b, dc_f64x4 c) {
@@ -165,6 +175,7 @@ delta_maps_kernel(DeltaChunkArgs p) {
     }
     const int dk = p.dk, dv = p.dv, heads = p.heads;
     const size_t no = (size_t)blockIdx.x * heads + head;
+    bool wild = false;
     // ---- the tokens' vectors
     if constexpr (GATED) {
         const int row = 2 * dk + 4;
@@ -172,6 +183,7 @@ delta_maps_kernel(DeltaChunkArgs p) {
             const float *s = p.prep + ((size_t)(t0 + min(lane, nt - 1)) * heads + head) * row + 2 * dk;
             double l = lane < nt ? (double)fmaxf(s[2], -1e4f) : 0.0;          // (a decay of exp(-1e4) is 0 like any smaller one)
             const float b = lane < nt ? s[1] : 0.f;
+            wild |= !(s[2] <= 0.f) || dc_wild(s[1]);
 #pragma unroll
             for (int off = 1; off < C; off <<= 1) {
                 const double before = __shfl_up(l, off, WAVE);
@@ -199,6 +211,7 @@ delta_maps_kernel(DeltaChunkArgs p) {
                 auto rt = [&](int e) { return t < nt && c + e < dk ? s[dk + c + e] : 0.f; };
                 r = make_float4(rt(0), rt(1), rt(2), rt(3));
             }
+            wild |= dc_wild(u) || dc_wild(r);
             *(float4 *)(us + t * LD + c) = u;
             *(float4 *)(rs + t * LD + c) = r;
         }
@@ -216,6 +229,7 @@ delta_maps_kernel(DeltaChunkArgs p) {
             const int t = grp * PER + e;
             w[e] = s[(size_t)min(t, nt - 1) * heads * row];
             if (t >= nt || c >= dk) w[e] = 1.f;
+            wild |= !(w[e] >= 0.5f && w[e] <= 1.f);
             own *= (double)w[e];
         }
         part[grp * DK + c] = own;
@@ -228,6 +242,7 @@ delta_maps_kernel(DeltaChunkArgs p) {
             const float *x = s + (size_t)min(t, nt - 1) * heads * row;
             const bool in = t < nt && c < dk;
             const float al = in ? x[dk] : 0.f, u = in ? x[2 * dk] : 0.f, k = in ? x[3 * dk] : 0.f, r = in ? x[4 * dk] : 0.f;
+            wild |= dc_wild(make_float4(al, u, k, r));
             us[t * LD + c] = (float)(u * before);
             before *= (double)w[e];
             const double inv = 1.0 / before;
@@ -393,6 +408,7 @@ delta_maps_kernel(DeltaChunkArgs p) {
                     const int cc = head * dv + min(col, dv - 1);
                     const float e = p.vf ? p.vf[tok * heads * dv + cc] : to_f32(((const T *)p.proj)[tok * p.row_stride + p.off_v + cc]);
                     v[b][i] = s < nt && col < dv ? (double)e : 0.0;
+                    wild |= s < nt && col < dv && dc_wild(e);
                 }
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
@@ -438,6 +454,43 @@ delta_maps_kernel(DeltaChunkArgs p) {
             }
         }
     }
+    wild = __syncthreads_or(wild);
+    if (tid == 0) p.wild[no] = wild;
+}
+
+// The tokens t0 .. t1 - 1 of a request one by one (delta_rule.hip's recurrence), for 16 value columns: 256 threads, 16 a column with KT key
+// channels each.
+template <int KT>
+__device__ __forceinline__ void delta_walk(const DeltaChunkArgs &p, float *mat, bool fresh, int t0, int t1, int head, int col, int part) {
+    const int dk = p.dk, dv = p.dv, i0 = part * KT, cc = head * dv + min(col, dv - 1);
+    float s[KT];
+#pragma unroll
+    for (int i = 0; i < KT; ++i) s[i] = !fresh && i0 + i < dk && col < dv ? mat[(size_t)(i0 + i) * dv + col] : 0.f;
+    for (int t = t0; t < t1; ++t) {
+        const float *row = p.prep + ((size_t)t * p.heads + head) * (p.gated ? 2 * dk + 4 : 5 * dk);
+        const float v = p.vf ? p.vf[(size_t)t * p.heads * dv + cc] : p.bf16 ? to_f32(((const bf16_t *)p.proj)[(size_t)t * p.row_stride + p.off_v + cc])
+                                                                            : ((const float *)p.proj)[(size_t)t * p.row_stride + p.off_v + cc];
+        const float g = p.gated ? row[2 * dk] : 1.f, bg = p.gated ? row[2 * dk + 1] : 1.f;
+        float u[KT], c = 0.f, o = 0.f;
+#pragma unroll
+        for (int i = 0; i < KT; ++i) {
+            u[i] = i0 + i < dk ? row[(p.gated ? 0 : 2 * dk) + i0 + i] : 0.f;
+            c += u[i] * s[i];
+        }
+        c = sum_over_16(c);
+#pragma unroll
+        for (int i = 0; i < KT; ++i) {
+            if (i0 + i >= dk) continue;
+            if (p.gated) s[i] = g * s[i] + u[i] * (v - bg * c);
+            else s[i] = row[i0 + i] * s[i] - row[dk + i0 + i] * c + row[3 * dk + i0 + i] * v;
+            o += row[(p.gated ? dk : 4 * dk) + i0 + i] * s[i];
+        }
+        o = sum_over_16(o);
+        if (part == 0 && col < dv) p.o[((size_t)t * p.heads + head) * dv + col] = o;
+    }
+#pragma unroll
+    for (int i = 0; i < KT; ++i)
+        if (i0 + i < dk && col < dv) mat[(size_t)(i0 + i) * dv + col] = s[i];
 }
 
 // One workgroup per (request, head, 16 value columns): a wave per 16 key channels, whose part of S stays in registers as the results of
@@ -469,6 +522,13 @@ delta_chain_kernel(DeltaChunkArgs p) {
     const float *right = of_state ? p.h + (size_t)(tile * KT + y) * 256 : p.q + (size_t)(tile * (C / 16) + y) * 256;
     const size_t left_step = of_state ? DK * DK : C * DK, right_step = (size_t)(of_state ? DK : C) * width;
     const int chunks = (q_len + C - 1) / C;
+    const bool fresh = p.ctx_len[r] - q_len == 0;
+    bool wild = false;
+    for (int c = tid; c < chunks; c += blockDim.x) wild |= p.wild[(size_t)(slot + c) * heads + head] != 0;
+    if (__syncthreads_or(wild)) {
+        if (tid < 256) delta_walk<KT>(p, mat, fresh, t_first, t_end, head, tile * 16 + tid / 16, tid % 16);
+        return;
+    }
     dc_f32x4 a[AHEAD][KT], b[AHEAD];
     auto fetch = [&](int c, dc_f32x4 *av, dc_f32x4 &bv) {
         const size_t no = (size_t)(slot + c) * heads + head;
@@ -479,7 +539,6 @@ delta_chain_kernel(DeltaChunkArgs p) {
     };
     dc_f64x4 s = dc_zero();
     if (of_state) {
-        const bool fresh = p.ctx_len[r] - q_len == 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             if (!fresh && row0 + 4 * i < dk && col < dv) s[i] = mat[(size_t)(row0 + 4 * i) * dv + col];
@@ -565,5 +624,8 @@ static int delta_chunks_launch(DeltaChunkArgs p, float *work, int n, hipStream_t
     p.p = p.f + all * D * D;
     p.h = p.p + all * DELTA_CHUNK * D;
     p.q = p.h + all * D * V;
+    p.wild = (int *)(p.q + all * DELTA_CHUNK * V);
+    p.gated = GATED;
+    p.bf16 = sizeof(T) == 2;
     return D == 64 ? delta_chunks_dk<T, GATED, 64>(p, slots, stream) : delta_chunks_dk<T, GATED, 128>(p, slots, stream);
 }

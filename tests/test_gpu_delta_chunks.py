@@ -172,3 +172,52 @@ def test_many_long_requests_of_small_heads_are_scanned(dim, heads, requests):
     one = torch.cat(one)
     for k in range(requests):
         assert torch.equal(all_of[k * T:(k + 1) * T], one) and torch.equal(state[k], alone[0])
+
+
+@pytest.mark.parametrize("what,value", [("r", math.inf), ("k", math.nan), ("v", math.inf), ("v", math.nan), ("a", math.nan), ("l", math.nan),
+                                        ("k", 1e30), ("v", -1e35)])
+@pytest.mark.parametrize("dim", [40, 128])
+def test_the_generalised_rule_passes_nothing_back_in_time(what, value, dim):
+    """An infinity, a NaN or a number whose products overflow in one token of 200: in chunks the tokens before it, the other heads and the other
+    request are what they are without it, and the token and those behind it what the scan makes of them."""
+    heads, T, at = 2, 200, 100
+    args, proj, want, S = general(T, heads, dim, 3, 0.0, seed=11)
+    proj[at, args[0][what] + (0 if what == "l" else dim + 3)] = value                   # (a channel of the second head; l reaches both)
+    whole, state = run_general(args, proj, heads, dim, [T])
+    cut, state2 = run_general(args, proj, heads, dim, [60, 60, 60, 20])
+    assert_close(whole[:at], want[:at], 2.0 ** -8 + 1e-5, "before")
+    if what != "l":
+        assert_close(whole[:, :dim], want[:, :dim], 2.0 ** -8 + 1e-5, "the other head")
+    same_but_for_rounding(whole, cut, 2.0 ** -8)
+    same_but_for_rounding(state, state2, 1e-5)
+
+
+def same_but_for_rounding(a, b, rel):
+    a, b = a.cpu().to(F64), b.cpu().to(F64)
+    assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf())
+    fine = a.isfinite()
+    if fine.any():
+        assert float((a[fine] - b[fine]).abs().max()) <= rel * max(float(b[fine].abs().max()), 1e-30)
+
+
+@pytest.mark.parametrize("what,value", [("q", math.nan), ("k", math.inf), ("v", math.inf), ("a", math.nan), ("a", math.inf), ("b", math.nan), ("v", 1e30)])
+def test_the_gated_rule_passes_nothing_back_in_time(what, value):
+    from llama_cu_amd.kernels import ops
+    heads, dk, dv, T, at = 2, 64, 24, 200, 100
+    args, qkv, rows, want, S = gated(T, heads, heads, dk, dv, -2.0, seed=21)
+    if what in "qkv":
+        qkv[at, {"q": 0, "k": heads * dk, "v": 2 * heads * dk}[what] + (dv if what == "v" else dk) + 3] = value
+    else:
+        rows[at, {"a": 0, "b": heads}[what] + 1] = value
+    outs = []
+    for portions in ([T], [60, 60, 60, 20]):
+        state, got, n0 = torch.full((2, heads, dk, dv), 7.0, device="cuda"), [], 0
+        for n in portions:
+            got.append(ops.gated_delta_rule(qkv[n0:n0 + n].cuda(), rows[n0:n0 + n].cuda(), 0, heads, 2 * heads, *args, state,
+                                            hand_step([n], [n0 + n], [1]), heads, heads, dk, dv, EPS, torch.bfloat16))
+            n0 += n
+        outs.append((torch.cat(got), state[1]))
+    assert_close(outs[0][0][:at], want[:at], 2.0 ** -8 + 1e-5, "before")
+    assert_close(outs[0][0][:, :dv], want[:, :dv], 2.0 ** -8 + 1e-5, "the other head")
+    for a, b, rel in zip(*outs, (2.0 ** -8, 1e-5)):
+        same_but_for_rounding(a, b, rel)
