@@ -567,8 +567,9 @@ delta_chain_kernel(DeltaChunkArgs p) {
                 }
             }
             s += s2;
-            // the sums stand before any branch: behind one that is taken the compiler (ROCm 7.2) counts too few wait states between a
-            // matrix instruction and the first use of its result, and the use reads the value of before
+            // the sums stand before any branch: behind the one over the next loads the compiler (ROCm 7.2) has left too few wait states where it is
+            // taken (3 of 10, with sums in 32 bits; it counted the instructions that the branch passes by), and the use read the value
+            // of before.  What holds for every kernel, that no use comes too early on any way, a test reads from the built instructions
             asm volatile("" : "+v"(s));
             if (c + AHEAD < chunks) fetch(c + AHEAD, a[k], b[k]);
             turn ^= 1;
