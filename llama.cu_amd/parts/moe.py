@@ -200,8 +200,10 @@ class GatedMoE(Part):
         if self.shared is not None:
             self.shared.load(tensors, build)
             sg, su, sd = (tensors[nm[k]] for k in ("shared_gate", "shared_up", "shared_down"))
-            if build.pack_weights and sg.shape[0] % 16 == 0 and sg.dtype == su.dtype == sd.dtype == self.w_down.dtype:
-                # steps of few tokens compute it beside the experts, from a copy in their order
+            if build.pack_weights and sg.shape[0] % 16 == 0 and sg.dtype == su.dtype == sd.dtype == self.w_down.dtype == torch.bfloat16:
+                # steps of few tokens compute it beside the experts, from a copy in their order.  Its sums run in another order than the dense
+                # products', which the other steps take, and its rows are not rounded before the gate: not in 32 bits, where a token's bits do
+                # not depend on how many are with it
                 self.shared_expert = (ops.pack_gated_experts(sg[None], su[None]), ops.pack_experts(sd[None]))
         self.dtype = build.dtype
 

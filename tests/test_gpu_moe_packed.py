@@ -148,3 +148,29 @@ def test_a_shared_expert_beside_sorted_pairs():
     z = h.cpu().to(F64) @ sg[0].cpu().to(F64).T
     want = alone.cpu().to(F64) + (z * torch.sigmoid(z) * (h.cpu().to(F64) @ su[0].cpu().to(F64).T)) @ sd[0].cpu().to(F64).T
     assert_close(both, want, 1e-5, "output")
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_token_with_few_and_with_more_others(dtype, gated):
+    """A mixture with a shared expert whose matrices are packed, on both sides of the number of tokens up to which the shared expert is computed
+    beside the others: in 32 bits a token has the same bits, in bfloat16 the two are one rounding of the shared row and one of its
+    activations apart."""
+    from llama_cu_amd.kernels import ops
+    from llama_cu_amd.parts.base import BuildContext
+    from llama_cu_amd.parts.moe import GatedMoE
+    d, ff, sff, experts, top, tdt = 520, 48, 528, 12, 2, TYPES[dtype]      # (K beyond 256: the two paths cut their sums at other places)
+    part = GatedMoE(d, ff, experts, top, shared_size=sff, shared_gated=gated)
+    tensors = {n: rnd(*t.shape, seed=k, std=t.shape[-1] ** -0.5).to(tdt).cuda() for k, (n, t) in enumerate(part.tensors().items())}
+    part.load(tensors, BuildContext(tdt, torch.device("cuda"), 64, 16, pack_weights=True))
+    h, few = rnd(3 * ops.MOE_SHARED_ROWS, d, seed=99).to(tdt).cuda(), ops.MOE_SHARED_ROWS
+    whole = part.forward(h)
+    for n in (1, few - 1, few, few + 1):
+        for first in (0, h.shape[0] - n):
+            got = part.forward(h[first:first + n].contiguous())
+            if dtype == "float32":
+                assert torch.equal(got, whole[first:first + n]), n
+            else:
+                # a rounding is at most 2^-9 of a value: one of sff activations under weights of sff ** -0.5 each (2^-9 of the largest together, and
+                # the other path's as much), one of the shared row
+                assert_close(got, whole[first:first + n].cpu().to(F64), 3 * 2.0 ** -9, f"{n}")
