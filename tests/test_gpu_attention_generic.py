@@ -67,3 +67,34 @@ def test_edges(kind, dh, dv, page, window, chunk, extras):
             want[t, h] = attend(q[t, h * dh:(h + 1) * dh].to(F64), ks[r][:p + 1, g].to(F64), vs[r][:p + 1, g].to(F64), scale, lo,
                                 float(slopes[h]) if extras else 0.0, sinks[h].to(F64) if extras else None, cap)
     assert_close(out, want.view(n, -1), 2e-6 if kind == "float32" else 2.0 ** -8, f"{dh} {dv}")     # 32-bit sums of up to 640 terms; one rounding
+
+
+@pytest.mark.parametrize("kind,dh,dv", [("float32", 64, 64), ("float32", 128, 96), ("float32", 96, 40), ("bfloat16", 128, 128), ("float32", 256, 200), ("bfloat16", 576, 512)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_a_token_among_few_and_among_many(kind, dh, dv, window):
+    """Single tokens of 1 to 300 keys, so many (token, head) pairs that workgroups have eight, four or two waves: the same bits."""
+    from llama_cu_amd.kernels import ops
+    tdt, nh, nkv, page, n = TYPES[kind], 8, 2, 16, 280
+    ctx = [1 + (37 * r) % 300 for r in range(n)]
+    ctx[:8] = [1, 16, 17, 112, 113, 128, 129, 300]
+    most = -(-max(ctx) // page)
+    table = torch.stack([torch.randperm(64, generator=torch.Generator().manual_seed(r))[:most] for r in range(n)]).to(torch.int32).cuda()
+    cache = torch.randn(64, 1, nkv * (dh + dv) * page, generator=torch.Generator().manual_seed(1)).to(tdt).cuda()
+    q = rnd(n, nh * dh, seed=2).to(tdt).cuda()
+    lengths = torch.tensor(ctx, dtype=torch.int32).cuda()
+
+    def run(first, count):
+        out = torch.empty(count, nh * dv, dtype=tdt, device="cuda")
+        each = torch.arange(count + 1, dtype=torch.int32, device="cuda")
+        return ops.paged_attention_generic(q[first:first + count], out, cache, table[first:first + count].contiguous(), each, lengths[first:first + count].contiguous(),
+                                           each[:count].contiguous(), nh, nkv, dh, page, dh ** -0.5, window, None, dv)
+    whole = run(0, n)                                        # 2,240 pairs
+    for first, count in ((0, 255), (0, 256), (150, 128), (8, 127), (0, 8), (77, 1)):
+        assert torch.equal(run(first, count), whole[first:first + count]), (first, count)
+    for r in range(8):                                       # ... and the right ones
+        pages = table[r].long().cpu()
+        keys = cache[pages, 0, :nkv * dh * page].cpu().view(most, nkv, dh // 8, page, 8).permute(1, 0, 3, 2, 4).reshape(nkv, most * page, dh)[:, :ctx[r]].to(F64)
+        values = cache[pages, 0, nkv * dh * page:].cpu().view(most, nkv, dv, page).permute(1, 0, 3, 2).reshape(nkv, most * page, dv)[:, :ctx[r]].to(F64)
+        want = torch.cat([attend(q[r, h * dh:(h + 1) * dh].cpu().to(F64), keys[h // 4], values[h // 4], dh ** -0.5, max(0, ctx[r] - window) if window else 0, 0.0, None, 0.0)
+                          for h in range(nh)])
+        assert_close(whole[r], want, 2e-6 if kind == "float32" else 2.0 ** -8, f"{r}")
