@@ -13,7 +13,8 @@
 // 8192 x 2048: 7.4 / 7.8 / - / 12.9 at 8, 9.4 / 11.0 / 9.4 / 13.0 at 32; SwiGLU of 5632 x 2048: 6.8 / 9.9 / - / 14 at 8, 7.4 / 10.7 / - / 14 at
 // 16, 9.2 / 14.5 / 8.5 / 14 at 32, 15.1 / - / 16.1 / 15 at 64; 4096 x 4096: 9.9 / 8.0 at 8 (a wave's share of K and X grow: the
 // weight-streaming kernel).  What bounds it is latency up to 16 rows, beyond it the rows' way from the L2 caches: 1.6 us for every 16 of
-// them at K = 2048.
+// them at K = 2048.  Groups with a gate (a latent's heads): 16 of 128 x 512 3.5 / 4.1 / - / 12.3 at 8 rows, 4.2 / 5.9 / - / 10.9 at 32, 5.4 / - / - / 11.3 at
+// 64; 64 of 128 x 512 4.5 / 6.1, 5.3 / 9.1 and 8.1 / 11.6 (library) there.
 //
 // Groups: X is [groups][M, K], group g's rows x_group elements further, and multiplies the rows g * N / groups .. of W.
 #include "common.h"

@@ -54,6 +54,25 @@ def test_swiglu(m, n, k, limit):
     assert_close(got, want, BF16_REL, f"{m} x {n} x {k}")
 
 
+@pytest.mark.parametrize("m", [8, 64])
+def test_stores_round_to_the_nearest(m):
+    """What is stored in 16 bits is off by half a unit of the last place at most, evenly on both sides: a root mean square of 1 / sqrt(12) of a unit
+    (cut off it would be 1 / sqrt(3)) and a mean of nothing.  The bounds above, of the largest value, would let a cut pass."""
+    from llama_cu_amd.kernels import ops
+    n, k = 4096, 512
+    x, w = operands(m, n, k, seed=51)
+    packed, product, gate = ops.pack_weight(w), f64(x) @ f64(w).t(), rnd(m, n, seed=53).bfloat16().cuda()
+    g, u = product.split(n // 2, dim=1)
+    for what, got, want in (("plain", ops.gemm_wavek(x, packed), product), ("gated", ops.gemm_wavek(x, packed, gate=gate), product * torch.sigmoid(f64(gate))),
+                            ("swiglu", ops.gemm_wavek(x, packed, swiglu=True), g * torch.sigmoid(g) * u)):
+        # (values of which a 32-bit sum's error, some 1e-7 of the largest, is no part of a unit)
+        big = want.abs() > 0.01 * want.abs().mean()
+        want, got = want[big], f64(got)[big]
+        off = (got - want) * torch.sign(want) / torch.exp2(torch.floor(torch.log2(want.abs())) - 7)
+        assert off.square().mean().sqrt() < 1.02 * 12 ** -0.5, what
+        assert off.mean().abs() < 6 * (12 * off.numel()) ** -0.5 + 1e-3, what      # six deviations of the mean
+
+
 @pytest.mark.parametrize("m,n,k,groups", [(2, 16, 128, 3), (33, 2048, 256, 4), (64, 112, 384, 2)])
 def test_groups(m, n, k, groups):
     from llama_cu_amd.kernels import ops
