@@ -48,9 +48,6 @@ __device__ __forceinline__ void load8(const bf16_t *p, float (&v)[8]) {
     }
 }
 
-// true or false as a type
-template <bool B> struct Flag { static constexpr bool value = B; };
-
 // NV: values of a lane, NV * 64 >= dv.  KP > 0: dh is at most 32 * KP, a lane keeps its KP pieces of the query in registers.
 // WAVES: waves of the workgroup, each of which does the work of AG_WAVES / WAVES, one after the other (the same bits).
 template <class T, int NV, int KP, int WAVES>
@@ -186,32 +183,32 @@ paged_attention_generic_kernel(const T *__restrict__ q, int q_stride, T *__restr
     }
     __syncthreads();
     if ((int)threadIdx.x >= dv) return;
-    auto merge = [&](auto whole) {
-        constexpr bool ALL = decltype(whole)::value;             // every wave has keys
-        float top = -INFINITY;
+    // (what a wave without keys would have left is read with the others, all at once, and not used)
+    float top = -INFINITY, keep[AG_WAVES], total = 0.f;
 #pragma unroll
-        for (int w = 0; w < AG_WAVES; ++w)
-            if (ALL || has_keys(w)) top = fmaxf(top, tops[w]);
-        if (sinks) top = fmaxf(top, sinks[h]);                  // the sink's term stands in the denominator beside the keys'
-        float keep[AG_WAVES], total = 0.f;
+    for (int w = 0; w < AG_WAVES; ++w) {
+        const float x = tops[w];
+        keep[w] = has_keys(w) ? x : -INFINITY;
+        top = fmaxf(top, keep[w]);
+    }
+    if (sinks) top = fmaxf(top, sinks[h]);                      // the sink's term stands in the denominator beside the keys'
+#pragma unroll
+    for (int w = 0; w < AG_WAVES; ++w) {
+        const float x = sums[w];
+        keep[w] = keep[w] == -INFINITY ? 0.f : expf(keep[w] - top);
+        total = has_keys(w) ? fmaf(x, keep[w], total) : total;
+    }
+    if (sinks) total += expf(sinks[h] - top);
+    const float inv = 1.f / total;
+    for (int d = threadIdx.x; d < dv; d += WAVES * WAVE) {
+        float x = 0.f;
 #pragma unroll
         for (int w = 0; w < AG_WAVES; ++w) {
-            if (!ALL && !has_keys(w)) continue;
-            keep[w] = tops[w] == -INFINITY ? 0.f : expf(tops[w] - top);
-            total += sums[w] * keep[w];
+            const float y = outs[w][d];
+            x = has_keys(w) ? fmaf(y, keep[w], x) : x;
         }
-        if (sinks) total += expf(sinks[h] - top);
-        const float inv = 1.f / total;
-        for (int d = threadIdx.x; d < dv; d += WAVES * WAVE) {
-            float x = 0.f;
-#pragma unroll
-            for (int w = 0; w < AG_WAVES; ++w)
-                if (ALL || has_keys(w)) x += outs[w][d] * keep[w];
-            out[(size_t)t * out_stride + (size_t)h * dv + d] = from_f32<T>(x * inv);
-        }
-    };
-    if (blocks >= AG_WAVES - 1) merge(Flag<true>());
-    else merge(Flag<false>());
+        out[(size_t)t * out_stride + (size_t)h * dv + d] = from_f32<T>(x * inv);
+    }
 }
 
 // q: [n, q_stride] (head h of token t at t*q_stride + h*dh), out: [n, out_stride].
