@@ -663,7 +663,8 @@ __device__ __forceinline__ void mul_frag_f32(const FragF32<MT> &f, f32x4 (&acc)[
             for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[j][e], f.x[m][j][e], acc[m], 0, 0, 0);
 }
 
-template <int MT, bool PAIR>
+// PAIR: SwiGLU; SCALED: with sumsq_in; ADDS: accumulate or norm_w
+template <int MT, bool PAIR, bool SCALED, bool ADDS>
 __global__ void __launch_bounds__(F32_WAVES *WAVE)
 gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W, int ldw, float *__restrict__ Y,
                        int ldy, int M, int N, int K, F32Extra ex) {
@@ -685,15 +686,10 @@ gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__rest
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int nsteps = (K + 63) / 64;
-    FragF32<MT> fa, fb;
-    int s = wave;
-    if (s < nsteps) load_frag_f32<MT>(fa, wrow, xrow, xvalid, s, grp, K);
-    if (s + F32_WAVES < nsteps) load_frag_f32<MT>(fb, wrow, xrow, xvalid, s + F32_WAVES, grp, K);
     // a wave stores sixteen tokens in the end; what it adds to, and the norm's weights, are on their way meanwhile
     const int tok = m0 + 16 * wave + l16;
-    const bool adds = !PAIR && (ex.accumulate || ex.norm_w) && wave < MT;
     float old[4] = {}, nw[4] = {};
-    if (adds) {
+    if (ADDS && wave < MT) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int n = n0 + 4 * grp + r;
@@ -703,7 +699,11 @@ gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__rest
             }
         }
     }
-    if (ex.sumsq_in) {
+    FragF32<MT> fa, fb;
+    int s = wave;
+    if (s < nsteps) load_frag_f32<MT>(fa, wrow, xrow, xvalid, s, grp, K);
+    if (s + F32_WAVES < nsteps) load_frag_f32<MT>(fb, wrow, xrow, xvalid, s + F32_WAVES, grp, K);
+    if constexpr (SCALED) {
         for (int r = wave; r < 16 * MT && m0 + r < M; r += F32_WAVES) {
             float t = 0.f;
             for (int i = lane; i < ex.n_in; i += WAVE) t += ex.sumsq_in[(size_t)(m0 + r) * ex.n_in + i];
@@ -724,7 +724,7 @@ gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__rest
     f32x4 sum = red[0][wave][lane];
 #pragma unroll
     for (int w = 1; w < F32_WAVES; ++w) sum += red[w][wave][lane];
-    if (ex.sumsq_in) sum *= factor[16 * wave + l16];
+    if constexpr (SCALED) sum *= factor[16 * wave + l16];
     if constexpr (PAIR) {                                    // the up rows' sums are 32 lanes further
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -740,14 +740,14 @@ gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__rest
     for (int r = 0; r < 4; ++r) {
         const int n = n0 + 4 * grp + r;
         if (tok >= M || n >= N) continue;
-        const float v = adds ? old[r] + ex.scale * sum[r] : sum[r];
+        const float v = ADDS ? old[r] + ex.scale * sum[r] : sum[r];
         Y[(size_t)tok * ldy + n] = v;
-        if (ex.norm_w) {
+        if (ADDS && ex.norm_w) {
             ex.h_out[(size_t)tok * ex.ldh + n] = v * nw[r];
             ss += v * v;
         }
     }
-    if (ex.norm_w) {                                         // every lane takes part: the others bring zero
+    if (ADDS && ex.norm_w) {                                 // every lane takes part: the others bring zero
         ss += __shfl_xor(ss, 16, WAVE);
         ss += __shfl_xor(ss, 32, WAVE);
         if (grp == 0 && tok < M) ex.sumsq_out[(size_t)tok * gridDim.x + blockIdx.x] = ss;
@@ -775,10 +775,15 @@ LCU_API int lcu_gemm_skinny_f32(const float *X, int ldx, const float *W, int ldw
     const int tiles = (M + rows - 1) / rows;
     if (tiles > 65535) return LCU_BAD_ARGUMENT;
     const dim3 grid(swiglu ? (N + 7) / 8 : (N + 15) / 16, tiles), block(F32_WAVES * WAVE);
-#define GO(MT, PAIR) gemm_skinny_f32_kernel<MT, PAIR><<<grid, block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, ex)
-    if (rows == 16) { if (swiglu) GO(1, true); else GO(1, false); }
-    else if (swiglu) GO(4, true);
-    else GO(4, false);
+    // What a product does besides is known when it is compiled: a form that looks at F32Extra for it, behind the loads that are on their way, took
+    // 5.0 us for two rows of 1024 x 1024 with the matrix in the caches and 2.5 for 64 x 64, now 4.7 and 2.3.
+#define GO(MT, PAIR, SCALED, ADDS) gemm_skinny_f32_kernel<MT, PAIR, SCALED, ADDS><<<grid, block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, ex)
+#define ROWS(MT, PAIR, ADDS) do { if (sumsq_in) GO(MT, PAIR, true, ADDS); else GO(MT, PAIR, false, ADDS); } while (0)
+#define FORMS(MT) do { if (swiglu) ROWS(MT, true, false); else if (accumulate || norm_w) ROWS(MT, false, true); else ROWS(MT, false, false); } while (0)
+    if (rows == 16) FORMS(1);
+    else FORMS(4);
+#undef FORMS
+#undef ROWS
 #undef GO
     LCU_LAUNCH_CHECK();
     return LCU_OK;
