@@ -776,7 +776,7 @@ LCU_API int lcu_gemm_skinny_f32(const float *X, int ldx, const float *W, int ldw
     if (tiles > 65535) return LCU_BAD_ARGUMENT;
     const dim3 grid(swiglu ? (N + 7) / 8 : (N + 15) / 16, tiles), block(F32_WAVES * WAVE);
     // What a product does besides is known when it is compiled: a form that looks at F32Extra for it, behind the loads that are on their way, took
-    // 5.0 us for two rows of 1024 x 1024 with the matrix in the caches and 2.5 for 64 x 64, now 4.7 and 2.3.
+    // 4.9 us for two rows of 1024 x 1024 with the matrix in the caches and 2.5 for 64 x 64, now 4.6 and 2.3.
 #define GO(MT, PAIR, SCALED, ADDS) gemm_skinny_f32_kernel<MT, PAIR, SCALED, ADDS><<<grid, block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, ex)
 #define ROWS(MT, PAIR, ADDS) do { if (sumsq_in) GO(MT, PAIR, true, ADDS); else GO(MT, PAIR, false, ADDS); } while (0)
 #define FORMS(MT) do { if (swiglu) ROWS(MT, true, false); else if (accumulate || norm_w) ROWS(MT, false, true); else ROWS(MT, false, false); } while (0)

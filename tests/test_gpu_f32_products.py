@@ -54,3 +54,20 @@ def test_residual_and_the_next_norm(m, n, k):
         ops.gemm_skinny_f32_add_norm(xg, wg, whole[:, 2:2 + n], ng.bfloat16())
     with pytest.raises(ops.KernelError):
         ops.gemm_skinny_f32_add_norm(xg, wg, whole[:, :n - 1], ng)
+
+
+@pytest.mark.parametrize("scaled", [False, True])
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("m", [3, 70])
+def test_every_form_of_a_plain_product(m, accumulate, scaled):
+    from llama_cu_amd.kernels import ops
+    n, k = 1028, 136                                          # (70 rows: 16 a workgroup; 1,000: 64)
+    for rows in (m, 1000) if m == 70 else (m,):
+        x, w, base, shares = rnd(rows, k, seed=1), rnd(n, k, seed=2, std=k ** -0.5), rnd(rows, n, seed=3), rnd(rows, 5, seed=4).abs()
+        out = base.cuda()
+        kw = dict(row_sumsq=shares.cuda(), norm_width=k, eps=1e-5) if scaled else {}
+        ops.gemm_skinny_f32(x.cuda(), w.cuda(), out=out, accumulate=accumulate, **kw)
+        want = x.to(F64) @ w.to(F64).t()
+        if scaled:
+            want = want * torch.rsqrt(shares.to(F64).sum(1, keepdim=True) / k + 1e-5)
+        assert_close(out, want + base.to(F64) if accumulate else want, REL, f"{rows}")
