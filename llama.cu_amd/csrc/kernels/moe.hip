@@ -66,9 +66,12 @@ moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, cons
                 for (int e = 0; e < 8; ++e) x[k][e] = to_f32(in.v[e]);
             }
         }
-        // two rows of the router at a time, so that 17 rows on 16 waves (16 experts and a gate) are not two trips to memory
-        for (int e = wave; e < experts; e += 2 * (THREADS / WAVE)) {
-            const int e2 = e + THREADS / WAVE;
+        // two rows of the router at a time, so that 17 rows on 16 waves (16 experts and a gate) are not two trips to memory; but one where a wave has
+        // many long rows, which are trips enough and twice of which leave no room for the next ones' loads (1,024 rows of 4,096, one token: 183 us, two at a
+        // time 222)
+        const bool two = experts <= 64 + MOE_MAX_EXTRA || d <= ROUTE_CHUNKS * 256;
+        for (int e = wave; e < experts; e += (two ? 2 : 1) * (THREADS / WAVE)) {
+            const int e2 = two ? e + THREADS / WAVE : experts;
             const float *w = router + (size_t)e * d, *v = router + (size_t)(e2 < experts ? e2 : e) * d;
             float acc = 0.f, acc2 = 0.f;
             if (e2 < experts) {
