@@ -38,6 +38,7 @@
 // they are; in LDS and in the maps the sixteen stand so that a lane's four are neighbours (dc_place).
 #pragma once
 #include <limits.h>
+#include <math.h>
 #include <mutex>
 #include "common.h"
 #include "lane_moves.h"
@@ -53,31 +54,49 @@ __device__ __forceinline__ bool dc_wild(float4 v) { return dc_wild(v.x) || dc_wi
 typedef __attribute__((ext_vector_type(4))) float dc_f32x4;
 typedef __attribute__((ext_vector_type(4))) double dc_f64x4;
 
-// Which requests of a step go through chunks: those that feed `line` tokens or more, unless more than `most` of them do.
-// line: one request, us scanned / in chunks: 64 tokens of 16 heads of 128 gated 47 / 63, per channel 83 / 96, of 64 gated 35 / 36; 100 tokens 68 /
-// 69, 124 / 104, 49 / 38; 128 tokens 83 / 70, 156 / 106, 60 / 39.  Head sizes for which the scan keeps the state in memory (10 us a token) go
-// there from 64 tokens on (40: 646 / 36).
-// most: scans of many requests and heads run side by side and chunks of small heads are padded to 64 channels: 16 requests of 128 tokens,
-// 16 / 32 heads of 16: gated 69 / 100 and 93 / 175, per channel 97 / 124 and 136 / 224; of 64, gated 103 / 112 and 173 / 206, per channel 231 / 143 and
-// 452 / 271; 8 requests of 256, 16 heads of 16: gated 103 / 97; of 128, 32 heads, 16 requests of 128: gated 502 / 512.
+// Which requests of a step go through chunks: those that feed `line` tokens or more, if all of those take less time so.  The times, in ns, of
+// what is measured: a scan is the longest request's chain, and the work of all tokens and heads where they fill the card; chunks are two launches,
+// the longest request's chain, and the work of all chunks and heads (a chunk that is cut short counts whole).  Chunks must be faster by a fifth.
+// One MI355X, the whole rule, gated heads of 128 / 64 / 16 and per-channel ones, us scanned / in chunks: 16 heads, one request of 130 tokens 82 / 77, 71 / 45 (of 64), 100 /
+// 77 (160 tokens); 16 requests of 130 tokens 269 / 371, 8 of 256 340 / 238.  Over 2,130 steps of 1 to 32 requests of 64 to 2,000 tokens, 4 to 64 heads of 16 to 128, this rule
+// takes 0.69 of the scan's time (the better one of the two 0.67) and 1.05 at the worst; by the number of tokens alone, 128, and of requests it took 0.70 and 2.2.
+// Head sizes for which the scan keeps the state in memory (10 us a token; 40: 646 / 36) go there from 64 tokens on.
 struct DeltaLine {
-    int line, most;
-    // what holds for a step: the least tokens that a request must feed (called by whole waves)
+    int line;                                    // INT_MAX: everything is scanned
+    int scan, scan_longest, scan_token;          // ns: a step, a token of the longest request, a token
+    int chunked, chunked_longest, chunk;
+    __host__ __device__ bool chunks_pay(int longest, int tokens, int chunks) const {
+        const long long a = scan + (long long)scan_longest * longest + (long long)scan_token * tokens;
+        const long long b = chunked + (long long)chunked_longest * ((longest + 63) / 64) + (long long)chunk * chunks;
+        return longest >= line && 6 * b < 5 * a;
+    }
+    // what holds for a step: the least tokens that a request must feed (called by whole waves; sums of less than 2^24, exact in 32-bit)
     __device__ __forceinline__ int of_step(const int *__restrict__ q_start, int n_req) const {
-        if (most == INT_MAX) return line;
         const int lane = threadIdx.x % WAVE;
-        int longs = 0;
-        for (int r = 0; r < n_req; r += WAVE) {
-            const int at = min(r + lane, n_req - 1);
-            longs += __popcll(__ballot(r + lane < n_req && q_start[at + 1] - q_start[at] >= line));
+        float longest = 0.f, tokens = 0.f, chunks = 0.f;
+        for (int r = lane; r < n_req; r += WAVE) {
+            const int len = q_start[r + 1] - q_start[r];
+            if (len < line) continue;
+            longest = fmaxf(longest, (float)len);
+            tokens += (float)len;
+            chunks += (float)((len + 63) / 64);
         }
-        return longs > most ? INT_MAX : line;
+        return chunks_pay((int)wave_max_in_place(longest), (int)wave_sum_in_place(tokens), (int)wave_sum_in_place(chunks)) ? line : INT_MAX;
     }
 };
-inline DeltaLine delta_line(int heads, int dk, bool gated) {
-    const bool scanned = dk % 16 == 0;                                        // the scan has the state in registers
-    const int crowd = scanned && dk <= (gated ? 64 : 32) ? 128 / heads : INT_MAX;
-    return DeltaLine{scanned ? 128 : 64, crowd > 1 ? crowd : 1};              // (one long request always goes there)
+inline DeltaLine delta_line(int heads, int dk, int dv, bool gated) {
+    const double wide = (double)dv / dk, sq = (double)dk * dk;               // (the work of a token grows with both sizes)
+    auto times = [&](double x) { return (int)fmin(x, 1e9); };
+    DeltaLine l = {};
+    l.line = 64;
+    l.scan = 9000;
+    l.scan_longest = dk % 16 ? 10000 : times(gated ? 290 + 1.2 * dk : 470 + 2.1 * dk);         // (else the scan has the state in registers)
+    l.scan_token = times(heads * wide * (gated ? 0.7 + 2.6e-4 * sq : 0.6 + 9e-4 * sq));
+    const bool half = dk <= 64;
+    l.chunked = gated ? (half ? 34000 : 54000) : (half ? 38000 : 72000);
+    l.chunked_longest = gated ? (half ? 800 : 900) : (half ? 700 : 800);
+    l.chunk = times(heads * (0.5 + 0.5 * wide) * (gated ? (half ? 165 : 350) : (half ? 190 : 460)));
+    return l;
 }
 
 struct DeltaChunkArgs {
@@ -88,6 +107,7 @@ struct DeltaChunkArgs {
     float *f, *h, *p, *q;                        // [slot][head] of [DK][DK], [DK][16 tiles], [64][DK], [64][16 tiles], in tiles of 16 x 16: F
                                                  // and P as left operands [row tile][index tile], H and Q as results [column tile][row tile]
     int *wild;                                   // [slot][head]: whether the chunk must be walked token by token
+    int *done;                                   // [request]: whether it went through chunks
     int gated, bf16;                             // the form of prep; the type of proj
     float *state;
     size_t slot_stride;
@@ -106,10 +126,15 @@ __host__ __device__ inline int delta_chunk_slots(int n, int n_req, int line) {
 inline bool delta_chunks_possible(int n, int n_req, int dk, int line) { return dk <= 128 && n - n_req + 1 >= line; }
 inline int delta_padded(int dk) { return dk <= 64 ? 64 : 128; }
 inline size_t delta_chunk_floats(int n, int n_req, int heads, int dk, int dv, bool gated) {
-    const int line = delta_line(heads, dk, gated).line;
+    const int line = delta_line(heads, dk, dv, gated).line;
     if (!delta_chunks_possible(n, n_req, dk, line)) return 0;
     const size_t D = delta_padded(dk), V = (size_t)(dv + 15) / 16 * 16;
-    return (size_t)delta_chunk_slots(n, n_req, line) * heads * (D * D + D * V + DELTA_CHUNK * (D + V) + 1);
+    return (size_t)delta_chunk_slots(n, n_req, line) * heads * (D * D + D * V + DELTA_CHUNK * (D + V) + 1) + n_req;
+}
+
+// Where in `work` the kernels leave which requests went through chunks.
+inline const int *delta_done(const float *work, int n, int n_req, int heads, int dk, int dv, bool gated) {
+    return (const int *)work + delta_chunk_floats(n, n_req, heads, dk, dv, gated) - n_req;
 }
 
 __device__ __forceinline__ dc_f64x4 dc_mma(float4 a, dc_f64x4 b, dc_f64x4 c) {
@@ -506,6 +531,7 @@ delta_chain_kernel(DeltaChunkArgs p) {
     const int r = blockIdx.x, head = blockIdx.y, tile = blockIdx.z;
     const int t_first = p.q_start[r], t_end = p.q_start[r + 1], q_len = t_end - t_first;
     const int line = p.line.of_step(p.q_start, p.n_req);
+    if (head == 0 && tile == 0 && threadIdx.x == 0) p.done[r] = q_len >= line;
     if (q_len < line) return;
     int slot = 0;
     for (int x = 0; x < r; ++x) {
@@ -626,6 +652,7 @@ static int delta_chunks_launch(DeltaChunkArgs p, float *work, int n, hipStream_t
     p.h = p.p + all * DELTA_CHUNK * D;
     p.q = p.h + all * D * V;
     p.wild = (int *)(p.q + all * DELTA_CHUNK * V);
+    p.done = p.wild + all;
     p.gated = GATED;
     p.bf16 = sizeof(T) == 2;
     return D == 64 ? delta_chunks_dk<T, GATED, 64>(p, slots, stream) : delta_chunks_dk<T, GATED, 128>(p, slots, stream);

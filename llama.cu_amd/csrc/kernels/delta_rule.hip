@@ -13,8 +13,8 @@
 //           of its lanes from the request's first token of the step to its last);
 //   out   (parallel): o of each head divided by its root mean square, times a weight, times
 //           sigmoid(gate).
-// A request that feeds many tokens in a step goes through chunks on the matrix cores instead of the scan (delta_chunks.h, which says from how many on:
-// 128 for most head sizes) if its outputs are rounded to bfloat16; 32-bit models keep the scan, whose bits do not depend on the cut of a prompt.
+// A request that feeds many tokens in a step goes through chunks on the matrix cores instead of the scan (delta_chunks.h, which says when: from some
+// 64 to 200 tokens on) if its outputs are rounded to bfloat16; 32-bit models keep the scan, whose bits do not depend on the cut of a prompt.
 // A token's result depends on the tokens before it in its request only; portions that are scanned are folded in in an
 // order of operations that does not depend on how the request was cut into them, chunks change roundings.
 #include <limits.h>
@@ -118,10 +118,10 @@ template <class T, int DK, bool GATED>
 __global__ void __launch_bounds__(64)
 delta_scan_kernel(const T *__restrict__ proj, int row_stride, int off_v, const float *__restrict__ vf, const float *__restrict__ prep,
                   float *__restrict__ state, size_t slot_stride, float *__restrict__ o, const int *__restrict__ q_start,
-                  const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int heads, int dk_rt, int dv, int n_req, DeltaLine line) {
+                  const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int heads, int dk_rt, int dv, const int *__restrict__ done) {
     const int r = blockIdx.x, h = blockIdx.y;
     const int t0 = q_start[r], t1 = q_start[r + 1];
-    if (line.line != INT_MAX && t1 - t0 >= line.of_step(q_start, n_req)) return;      // a request for the chunks
+    if (done && done[r]) return;                             // it went through chunks
     const bool fresh = ctx_len[r] - (t1 - t0) == 0;          // the request's first token: the state starts at zero
     if constexpr (DK > 0) {
         constexpr int SCAN_GROUPS = scan_groups<T, DK>(), SCAN_COLS = WAVE / SCAN_GROUPS;
@@ -265,8 +265,8 @@ template <class T, bool GATED = false>
 static int delta_scan_launch(const T *proj, int row_stride, int off_v, const float *vf, const float *prep, float *work, float *state,
                              size_t slot_stride, float *o, const int *q_start, const int *ctx_len, const int *state_slot,
                              int n, int n_req, int heads, int dk, int dv, hipStream_t stream) {
-    DeltaLine line = {INT_MAX, 0};
-    const DeltaLine chunks = delta_line(heads, dk, GATED);
+    const int *done = nullptr;
+    const DeltaLine chunks = delta_line(heads, dk, dv, GATED);
     if (work && delta_chunks_possible(n, n_req, dk, chunks.line)) {
         DeltaChunkArgs c = {};
         c.prep = prep; c.proj = proj; c.row_stride = row_stride; c.off_v = off_v; c.vf = vf;
@@ -275,10 +275,10 @@ static int delta_scan_launch(const T *proj, int row_stride, int off_v, const flo
         c.n_req = n_req; c.heads = heads; c.dk = dk; c.dv = dv; c.line = chunks;
         const int rc = delta_chunks_launch<T, GATED>(c, work, n, stream);
         if (rc != LCU_OK) return rc;
-        if (n_req == 1) return LCU_OK;                        // (its one request is long)
-        line = chunks;
+        if (n_req == 1 && chunks.chunks_pay(n, n, (n + DELTA_CHUNK - 1) / DELTA_CHUNK)) return LCU_OK;
+        done = delta_done(work, n, n_req, heads, dk, dv, GATED);
     }
-#define SCAN(DK) delta_scan_kernel<T, DK, GATED><<<dim3(n_req, heads, (dv + (DK ? 64 / scan_groups<T, DK>() : 64) - 1) / (DK ? 64 / scan_groups<T, DK>() : 64)), dim3(64), 0, stream>>>(proj, row_stride, off_v, vf, prep, state, slot_stride, o, q_start, ctx_len, state_slot, heads, dk, dv, n_req, line)
+#define SCAN(DK) delta_scan_kernel<T, DK, GATED><<<dim3(n_req, heads, (dv + (DK ? 64 / scan_groups<T, DK>() : 64) - 1) / (DK ? 64 / scan_groups<T, DK>() : 64)), dim3(64), 0, stream>>>(proj, row_stride, off_v, vf, prep, state, slot_stride, o, q_start, ctx_len, state_slot, heads, dk, dv, done)
     switch (dk) {
     case 16: SCAN(16); break;
     case 32: SCAN(32); break;
@@ -320,11 +320,18 @@ static int delta_rule_t(const T *proj, int row_stride, int off_r, int off_k, int
 // weight: [heads * dv], all 32-bit.  prep: scratch [n, heads, 5, dk], o: scratch [n, heads * dv], work: scratch of
 // lcu_delta_work_floats floats (null: every request is scanned token by token), all 32-bit.
 // state: [slots, heads, dk, dv] 32-bit.  out: [n, heads * dv] of `type`.
-// The tokens that a request must feed for chunks, and in *most the requests that may.
-LCU_API int lcu_delta_line(int heads, int dk, int gated, int *most) {
-    const DeltaLine line = heads > 0 && dk > 0 && dk <= 128 ? delta_line(heads, dk, gated) : DeltaLine{INT_MAX, 0};
-    *most = line.most;
-    return line.line;
+// Whether requests of a step that feeds q_lens (host memory) tokens go through chunks, if it has the memory for them.
+LCU_API int lcu_delta_chunked(const int *q_lens, int n_req, int heads, int dk, int dv, int gated) {
+    if (heads <= 0 || dk <= 0 || dk > 128 || dv <= 0) return 0;
+    const DeltaLine line = delta_line(heads, dk, dv, gated);
+    int longest = 0, tokens = 0, chunks = 0;
+    for (int r = 0; r < n_req; ++r) {
+        if (q_lens[r] < line.line) continue;
+        longest = longest > q_lens[r] ? longest : q_lens[r];
+        tokens += q_lens[r];
+        chunks += (q_lens[r] + DELTA_CHUNK - 1) / DELTA_CHUNK;
+    }
+    return line.chunks_pay(longest, tokens, chunks);
 }
 
 LCU_API long long lcu_delta_work_floats(int n, int n_req, int heads, int dk, int dv, int gated) {

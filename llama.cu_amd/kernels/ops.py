@@ -1366,18 +1366,33 @@ def qk_norm_store(qkv: torch.Tensor, positions: torch.Tensor, n_heads: int, n_kv
 # ------------------------------------------------------------------ the generalised delta rule
 
 
+@dataclass(frozen=True)
+class DeltaPlan:
+    """Whether a step's delta rule goes through chunks: what its launches follow from, beside the step's sizes."""
+    chunked: bool
+
+    @property
+    def signature(self):
+        return self.chunked
+
+
+def plan_delta(step, heads: int, key_dim: int, value_dim: int, gated: bool) -> DeltaPlan:
+    """The DeltaPlan of ``step`` for layers with these heads (one per step and kind of layer, kept in ``step.scratch``)."""
+    key = ("delta", heads, key_dim, value_dim, gated)
+    plan = step.scratch.get(key)
+    if plan is None:
+        lens = (ctypes.c_int * step.n_req)(*step.q_lens)
+        plan = step.scratch[key] = DeltaPlan(bool(build.load("delta_rule").lcu_delta_chunked(lens, step.n_req, heads, key_dim, value_dim, int(gated))))
+    return plan
+
+
 def _delta_work(lib, step, heads: int, key_dim: int, value_dim: int, gated: bool, out: torch.Tensor) -> Optional[torch.Tensor]:
     """Scratch memory for the delta rules' chunks.  None: everything is scanned token by token, because the step holds no
-    request that feeds enough tokens for chunks, or because the outputs are 32-bit: a 32-bit model computes the same bits
-    for a token however its prompt is cut.  (A captured step is replayed for other requests of the same total: there the
-    kernels themselves look who feeds how many, as they always do, and only the total decides whether they are launched.)"""
-    if out.dtype == torch.float32:
+    requests for which chunks pay, or because the outputs are 32-bit: a 32-bit model computes the same bits
+    for a token however its prompt is cut.  (A captured step is replayed for other requests of the same total, of which the same holds:
+    there the kernels themselves look who feeds how many, as they always do.)"""
+    if out.dtype == torch.float32 or step.decode_only or not plan_delta(step, heads, key_dim, value_dim, gated).chunked:
         return None
-    if not torch.cuda.is_current_stream_capturing():
-        most = ctypes.c_int()
-        line = lib.lcu_delta_line(heads, key_dim, int(gated), ctypes.byref(most))
-        if not 0 < sum(q >= line for q in step.q_lens) <= most.value:
-            return None
     lib.lcu_delta_work_floats.restype = ctypes.c_longlong
     floats = lib.lcu_delta_work_floats(step.n, step.n_req, heads, key_dim, value_dim, int(gated))
     return torch.empty(floats, dtype=torch.float32, device=out.device) if floats else None

@@ -206,7 +206,8 @@ class BuildContext:
     device: torch.device
     max_positions: int
     page_size: int
-    pack_weights: bool = True        # keep a second copy of bfloat16 matrices in the order the decode kernel streams them
+    pack_weights: bool = True        # keep a second copy of bfloat16 matrices in the order the decode kernel streams them (of experts, of both types,
+                                     # in the experts' kernels' order; of a bfloat16 shared expert a third, in theirs)
 
 
 @dataclass

@@ -75,6 +75,10 @@ class GeneralDelta(Part):
         self.norm = tensors[nm["norm"]].float().contiguous()
         self.dtype = build.dtype
 
+    def prepare(self, step) -> None:
+        if self.dtype != torch.float32 and not step.decode_only:
+            ops.plan_delta(step, self.heads, self.head_dim, self.head_dim, gated=False)
+
     def forward(self, h, step, cache, out_dtype=None):
         if cache.state is None:
             raise ops.KernelError("general_delta: the layer was given no state slots")
@@ -149,6 +153,10 @@ class GatedDelta(Part):
         self.conv_w = torch.cat([f32("q_conv"), f32("k_conv"), f32("v_conv")]).contiguous()
         self.a_log, self.dt_bias, self.norm = f32("a_log"), f32("dt_bias"), f32("norm")
         self.dtype = build.dtype
+
+    def prepare(self, step) -> None:
+        if self.dtype != torch.float32 and not step.decode_only:
+            ops.plan_delta(step, self.heads, self.head_dim, self.value_dim, gated=True)
 
     def forward(self, h, step, cache, out_dtype=None, state: Optional[torch.Tensor] = None):
         state = state if state is not None else cache.state

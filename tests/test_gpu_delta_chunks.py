@@ -221,3 +221,28 @@ def test_the_gated_rule_passes_nothing_back_in_time(what, value):
     assert_close(outs[0][0][:, :dv], want[:, :dv], 2.0 ** -8 + 1e-5, "the other head")
     for a, b, rel in zip(*outs, (2.0 ** -8, 1e-5)):
         same_but_for_rounding(a, b, rel)
+
+
+@pytest.mark.parametrize("heads,dk,dv,lens,chunked", [
+    (2, 128, 128, [256, 257, 255, 193], True), (1, 128, 272, [400, 64, 63, 1], True), (3, 64, 20, [1, 320, 129, 7], True), (2, 40, 40, [64, 63, 65], True),
+    (4, 16, 48, [500, 100], True), (2, 128, 128, [100, 64], False), (2, 64, 64, [63, 1], False), (32, 16, 16, [65] * 5, False)])
+def test_long_and_short_requests_in_a_step(heads, dk, dv, lens, chunked):
+    """Requests of chunks and of the scan side by side, where chunks pay and where they do not (then each has the bits that it has alone)."""
+    from llama_cu_amd.kernels import ops
+    n = len(lens)
+    each = [gated(T, heads, heads, dk, dv, -2.0, seed=31 + 2 * r) for r, T in enumerate(lens)]
+    args, step = each[0][0], hand_step(lens, lens, list(range(n)))
+    assert ops.plan_delta(step, heads, dk, dv, True).chunked == chunked
+    state = torch.full((n, heads, dk, dv), 7.0, device="cuda")
+    out = ops.gated_delta_rule(torch.cat([e[1] for e in each]).cuda(), torch.cat([e[2] for e in each]).cuda(), 0, heads, 2 * heads, *args, state, step,
+                               heads, heads, dk, dv, EPS, torch.bfloat16).split(lens)
+    for r, (_, qkv, rows, want, S) in enumerate(each):
+        assert_close(state[r], S, 5e-6, f"state {r}")
+        assert_close(out[r], want, 2.0 ** -8 + 1e-5, f"outputs {r}")
+        if not chunked:
+            alone, got = torch.full((1, heads, dk, dv), 7.0, device="cuda"), []
+            for at in range(0, lens[r], 50):
+                to = min(lens[r], at + 50)
+                got.append(ops.gated_delta_rule(qkv[at:to].cuda(), rows[at:to].cuda(), 0, heads, 2 * heads, *args, alone, hand_step([to - at], [to], [0]),
+                                                heads, heads, dk, dv, EPS, torch.bfloat16))
+            assert torch.equal(torch.cat(got), out[r]) and torch.equal(alone[0], state[r])
