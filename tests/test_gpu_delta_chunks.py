@@ -246,3 +246,27 @@ def test_long_and_short_requests_in_a_step(heads, dk, dv, lens, chunked):
                 got.append(ops.gated_delta_rule(qkv[at:to].cuda(), rows[at:to].cuda(), 0, heads, 2 * heads, *args, alone, hand_step([to - at], [to], [0]),
                                                 heads, heads, dk, dv, EPS, torch.bfloat16))
             assert torch.equal(torch.cat(got), out[r]) and torch.equal(alone[0], state[r])
+
+
+@pytest.mark.parametrize("name", ["B", "D"])
+def test_steps_of_equal_sizes_with_and_without_chunks(name):
+    """Captured steps of 126 tokens and two requests, some of which go through chunks: each kind replays its own launches."""
+    from divasun_common import tokens_of
+    from test_gpu_divasun import model, runner_for
+    cfg, _, folder = model(name)
+    kinds = [[63, 63], [125, 1], [1, 125], [63, 63], [124, 2]] * 3
+
+    def run(use_graphs):
+        r, outs = runner_for(folder, "bfloat16", use_graphs=use_graphs), []
+        for i, lens in enumerate(kinds):
+            toks = [tokens_of(cfg["vocab"], n, 100 * i + n + k) for k, n in enumerate(lens)]
+            outs.append(r.step([2 * i, 2 * i + 1], toks).float().cpu())
+            torch.cuda.synchronize()
+            for rid in (2 * i, 2 * i + 1):                   # and a step of single tokens on the states
+                outs.append(r.step([rid], [[5]]).float().cpu())
+                r.end(rid)
+        return outs, r
+    (eager, _), (graphed, r) = run(False), run(True)
+    assert sum(r.step_graph_replays.values()) >= (len(kinds) - 4 if name == "D" else 1) and len(r._step_graphs) >= 2
+    for i, (a, b) in enumerate(zip(eager, graphed)):
+        assert torch.isfinite(a).all() and torch.equal(a, b), f"step {i}"
