@@ -9,7 +9,7 @@
 // rows and features end where they do.
 //
 // One MI355X, weights out of memory, beside the weight-streaming kernel, the row-sharing one and the library's, us a product (graph of
-// products one after the other): 2048 x 2048: 4.6 / 5.0 / - / 8.1 at 8 rows, 7.1 / 8.2 / 7.8 / 8.3 at 32, 10.9 / - / 12.1 / 8.7 at 64;
+// products one after the other): 2048 x 2048: 5.0 / 4.8 / - / 8.1 at 8 rows, 7.1 / 8.2 / 7.8 / 8.3 at 32, 10.9 / - / 12.1 / 8.7 at 64;
 // 8192 x 2048: 7.4 / 7.8 / - / 12.9 at 8, 9.4 / 11.0 / 9.4 / 13.0 at 32; SwiGLU of 5632 x 2048: 6.8 / 9.9 / - / 14 at 8, 7.4 / 10.7 / - / 14 at
 // 16, 9.2 / 14.5 / 8.5 / 14 at 32, 15.1 / - / 16.1 / 15 at 64; 4096 x 4096: 9.9 / 8.0 at 8 (a wave's share of K and X grow: the
 // weight-streaming kernel).  What bounds it is latency up to 16 rows, beyond it the rows' way from the L2 caches: 1.6 us for every 16 of

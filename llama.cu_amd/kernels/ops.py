@@ -875,15 +875,28 @@ def wavek_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.stride(-2) % 8 == 0 and (x.dim() == 2 or x.stride(0) % 8 == 0) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def wavek_preferred(m: int, n: int, k: int, swiglu: bool = False) -> bool:
+def wavek_wide(n: int) -> bool:
+    """Whether a workgroup of ``gemm_wavek`` takes 32 features instead of 16: where those of 16 would be more than compute units."""
+    return n > TUNING.wavek_wide_per_cu * TUNING.compute_units
+
+
+def wavek_preferred(m: int, n: int, k: int, swiglu: bool = False, grouped: bool = False) -> bool:
     """Whether ``gemm_wavek`` is the fastest choice for ``m`` rows and a packed ``[n, k]`` weight (``TUNING``'s numbers)."""
     t = TUNING
     if min(n, k) < t.wavek_least or k > t.wavek_max_k or n > 32 * t.compute_units:                    # (more workgroups of 32 features than compute units: a second round)
         return False
     if swiglu:
-        return m <= WAVEK_MAX_ROWS
-    if m <= t.wavek_few_rows:
-        return n >= t.wavek_wide_features
+        if m <= t.wavek_middle_rows or k <= t.wavek_short_k:
+            return m <= WAVEK_MAX_ROWS
+        if m <= t.wavek_rows:
+            return k <= t.wavek_middle_k or n > t.wavek_swiglu_features
+        return m <= WAVEK_MAX_ROWS and (n >= t.wavek_swiglu_features or (m <= t.wavek_more_rows and k <= t.wavek_middle_k and 2 * n >= t.wavek_swiglu_features))
+    if m <= (t.wavek_few_group_rows if grouped else t.wavek_few_rows):
+        return wavek_wide(n)
+    if k > t.wavek_middle_k and m > t.wavek_middle_rows and not grouped:
+        if m > t.wavek_rows:
+            return m <= t.wavek_more_rows and wavek_wide(n)
+        return 4 * t.compute_units < n <= t.wavek_wide_per_cu * t.compute_units or n > 24 * t.compute_units
     return m <= t.wavek_rows or (m <= WAVEK_MAX_ROWS and k <= t.wavek_short_k) or (m <= t.wavek_more_rows and n >= t.wavek_more_features)
 
 
@@ -919,7 +932,7 @@ def gemm_wavek(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = N
     epi = 2 if swiglu else 3 if gate is not None else 1 if dtype == torch.float32 else 0
     lib = build.load("gemm_wavek")
     _check(lib.lcu_gemm_wavek(_ptr(x), x.stride(-2), ctypes.c_longlong(x.stride(0) if x.dim() == 3 else 0), groups, _ptr(w), _ptr(out), out.stride(0),
-                              _ptr(gate), gate.stride(0) if gate is not None else 0, m, n, k, epi, int(n >= TUNING.wavek_wide_features),
+                              _ptr(gate), gate.stride(0) if gate is not None else 0, m, n, k, epi, int(wavek_wide(n)),
                               _ptr(row_sumsq), row_sumsq.shape[1] if row_sumsq is not None else 0, int(norm_width), ctypes.c_float(eps),
                               ctypes.c_float(act_alpha), ctypes.c_float(act_limit), _stream()), "gemm_wavek")
     return out

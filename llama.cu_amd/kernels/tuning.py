@@ -61,15 +61,24 @@ class Tuning:
     mid_max_slices: int = 8
     # ---- the product whose waves share out K (gemm_wavek.hip, up to 64 rows)
     # (its numbers stand in gemm_wavek.hip; measured with widths of 1024 and 2048)
-    wavek_wide_features: int = 4096     # 32 features a workgroup instead of 16 from this many on
+    wavek_wide_per_cu: int = 16         # 32 features a workgroup instead of 16 beyond so many features a compute unit (4096 x 2048 at 4 / 33 rows: 6.2 / 9.8 us
+                                        # with 32, 5.4 / 8.4 with 16; 5120 x 2048 6.4 / 9.9 and 7.0 / 14.8)
     wavek_max_k: int = 3072             # with a longer K the weight-streaming kernel is faster (K = 4096: 8.0 us against 9.9 at 8 rows)
     wavek_least: int = 512              # features and K from which on it was measured: below either, the general path
-    wavek_few_rows: int = 4             # up to here a plain product goes to it from wavek_wide_features features on only (below the
-                                        # two are equal)
-    wavek_rows: int = 32                # up to here every plain product does,
+    wavek_few_rows: int = 11            # up to here a plain product goes to it beyond wavek_wide_per_cu only (up to there the weight-streaming
+                                        # kernel takes 0.95 of its time at 4, 5 and 8 rows, 1.06 at 16)
+    wavek_few_group_rows: int = 4       # ... and one in groups (16 groups of 128 x 512 at 5 rows: 3.4 us against 4.0)
+    wavek_rows: int = 32                # up to here every plain product does, but for those of more than wavek_middle_rows with a K beyond
+    wavek_middle_rows: int = 24         # wavek_middle_k where its workgroups are few or just too many for one a compute unit (32 rows, 3072 columns, 512 / 5120
+    wavek_middle_k: int = 2048          # features: 9.3 / 12.4 us against 7.5 / 12.1; 2048 features 9.7 against 10.2)
     wavek_short_k: int = 1024           # ... up to 64 rows with a K up to this (2048 x 768: 5.7 us against the library's 7.2 at 64 rows),
     wavek_more_rows: int = 48           # ... and up to here from so many features on (3072 x 2048: 9.2 us against 10.2 to 10.6; at 64 rows
-    wavek_more_features: int = 3072     # 11.1 against 10.9, with 2048 features 9.0 against 8.3 at 48)
+    wavek_more_features: int = 3072     # 11.1 against 10.9, with 2048 features 9.0 against 8.3 at 48), with a K beyond wavek_middle_k beyond wavek_wide_per_cu
+                                        # only (48 rows, 3072 x 2816 12.2 against 9.9, 5120 x 2816 14.3 against 14.9)
+    wavek_swiglu_features: int = 5632   # gate and up rows from which on SwiGLU goes to it with more than wavek_rows rows and a K beyond wavek_short_k, from half of
+                                        # them on with up to wavek_more_rows and a K up to wavek_middle_k; beyond them with more than
+                                        # wavek_middle_rows and a K beyond wavek_middle_k (whole feed-forwards at 64 rows, K of 2048 / 3072: 1024 features 20.2 / 24.8 us
+                                        # against 15.5 / 17.3, 5632 27.7 / 32.2 against 29.7 / 33.2)
     # ---- the library's product of many rows (parts/linear.library_friendly_rows)
     library_rows: int = -1              # rows of zeros behind each half of a plain gate/up matrix: -1 times the library once per
                                         # shape at load and fills up where that is 15 % faster (the outcome can differ from box

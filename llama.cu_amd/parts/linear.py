@@ -59,7 +59,7 @@ def _split(weight):
 
 def wavek_takes(x: torch.Tensor, packed: Optional[torch.Tensor], swiglu: bool = False) -> bool:
     """Whether the product whose waves share out K is the choice for these rows and this packed matrix."""
-    return packed is not None and ops.wavek_preferred(x.shape[-2], packed.shape[0], packed.shape[1], swiglu) and ops.wavek_supported(x, packed)
+    return packed is not None and ops.wavek_preferred(x.shape[-2], packed.shape[0], packed.shape[1], swiglu, x.dim() == 3) and ops.wavek_supported(x, packed)
 
 
 def _plain_rows(out: torch.Tensor) -> bool:

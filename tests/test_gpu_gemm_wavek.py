@@ -110,3 +110,18 @@ def test_what_it_refuses():
                 lambda: ops.gemm_wavek(x, packed, row_sumsq=torch.ones(3, 1, device="cuda"), norm_width=256)):
         with pytest.raises(ops.KernelError):
             bad()
+
+
+@pytest.mark.parametrize("m", [24, 25, 32, 33, 48, 49, 64, 65])
+@pytest.mark.parametrize("ff,k", [(512, 1024), (512, 2048), (1408, 2048), (2816, 2048), (512, 3072), (2816, 3072), (2832, 3072)])
+def test_the_rule_of_swiglu_against_the_general_path(m, ff, k):
+    """A feed-forward on both sides of the rule's lines, against 64 bits."""
+    from llama_cu_amd.parts.base import BuildContext, PartSpec, make_part
+    part = make_part("ffn", PartSpec("swiglu", {"hidden_size": k, "intermediate_size": ff}))
+    w = {n: rnd(*s.shape, seed=60 + i, std=s.shape[-1] ** -0.5).bfloat16() for i, (n, s) in enumerate(sorted(part.tensors().items()))}
+    part.load({n: t.cuda() for n, t in w.items()}, BuildContext(torch.bfloat16, torch.device("cuda"), 64, 16, pack_weights=True))
+    x = rnd(m, k, seed=70).bfloat16().cuda()
+    gate, up, down = (next(f64(t) for n, t in w.items() if what in n) for what in ("gate", "up", "down"))
+    g, u = f64(x) @ gate.t(), f64(x) @ up.t()
+    # up to four roundings, of gate, up, activation and output, each 2^-9 of a value at most; an activation's slope is below 1.1
+    assert_close(part.forward(x), (g * torch.sigmoid(g) * u) @ down.t(), 2.0 ** -6, f"{m} x {ff} x {k}")
