@@ -1,0 +1,64 @@
+// A step's arrays (tokens, positions, block tables, task lists) from pinned host memory to their places on the device.
+//
+// What a decode step brings is a few hundred bytes to some tens of kilobytes, spread over arrays of fixed capacity.  One copy of the whole
+// capacity is a job of the copy engine with a signal on either side of it, between two steps of the queue: 26 us stood between one captured step and the
+// next with it, 10 with this kernel (40 launches replayed; 40,000 entries of capacity, 4,000 in use).  The kernel is bound by one trip over the host's bus, so every
+// piece is on its way at once: 16 bytes a thread, the pieces behind one another over the grid.
+#include "common.h"
+
+constexpr int ARRAY_PIECES = 24;                 // pieces a launch takes (the arguments of a launch are a few hundred bytes)
+
+// `rows` rows that begin at `at` and then every `stride` entries, in both arrays: the first `cols` of a row's `width` entries come over, zeros stand
+// behind them; all in units of 16 bytes
+struct ArrayPiece { int at, cols, rows, stride, width; };
+struct ArrayPieces { ArrayPiece p[ARRAY_PIECES]; };
+
+// Loads that see what the host wrote last, whatever the device's caches hold of the same addresses.
+__device__ __forceinline__ uint64_t host_load(const uint64_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+
+__global__ void __launch_bounds__(256)
+step_arrays_kernel(const uint64_t *__restrict__ host, uint64_t *__restrict__ dev, ArrayPieces pieces, int n_pieces, int total) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+        int left = i, k = 0;
+        while (k + 1 < n_pieces && left >= pieces.p[k].width * pieces.p[k].rows) { left -= pieces.p[k].width * pieces.p[k].rows; ++k; }
+        const ArrayPiece q = pieces.p[k];
+        const int col = left % q.width;
+        const size_t at = 2 * ((size_t)q.at + (size_t)(left / q.width) * q.stride + col);
+        const uint64_t lo = col < q.cols ? host_load(host + at) : 0, hi = col < q.cols ? host_load(host + at + 1) : 0;
+        dev[at] = lo;
+        dev[at + 1] = hi;
+    }
+}
+
+// The address under which the device reads pinned host memory.
+LCU_API int lcu_host_on_device(void *host, void **on_device) {
+    if (!host || !on_device) return LCU_BAD_ARGUMENT;
+    const hipError_t e = hipHostGetDevicePointer(on_device, host, 0);
+    if (e != hipSuccess) { (void)hipGetLastError(); return LCU_UNSUPPORTED; }
+    return LCU_OK;
+}
+
+// host, dev: arrays of `size` 32-bit entries, 16-byte aligned (host: as lcu_host_on_device names it).  pieces: n_pieces times (at, cols, rows, stride, width)
+// in entries, rows as they are and the others multiples of 4, cols <= width <= stride (of a single row: any stride): see ArrayPiece.
+LCU_API int lcu_step_arrays(const void *host, void *dev, long long size, const int *pieces, int n_pieces, hipStream_t stream) {
+    if (n_pieces < 0 || size < 0 || (n_pieces && (!host || !dev || !pieces)) || ((uintptr_t)host | (uintptr_t)dev) % 16) return LCU_BAD_ARGUMENT;
+    for (int done = 0; done < n_pieces;) {
+        ArrayPieces a{};
+        int n = 0;
+        long long total = 0;
+        for (; n < ARRAY_PIECES && done < n_pieces; ++done) {
+            const int at = pieces[5 * done], cols = pieces[5 * done + 1], rows = pieces[5 * done + 2], stride = pieces[5 * done + 3], width = pieces[5 * done + 4];
+            if (at < 0 || cols < 0 || rows < 0 || stride < 0 || width < cols || (at | cols | stride | width) % 4) return LCU_BAD_ARGUMENT;
+            if (width == 0 || rows == 0) continue;
+            if ((long long)at + (long long)(rows - 1) * stride + width > size || (rows > 1 && stride < width)) return LCU_BAD_ARGUMENT;
+            a.p[n++] = ArrayPiece{at / 4, cols / 4, rows, stride / 4, width / 4};
+            total += (long long)(width / 4) * rows;
+        }
+        if (!n) continue;
+        if (total > 0x7fffffffLL - 256 * 256) return LCU_BAD_ARGUMENT;
+        const long long blocks = (total + 255) / 256;
+        step_arrays_kernel<<<(unsigned)(blocks < 256 ? blocks : 256), 256, 0, stream>>>((const uint64_t *)host, (uint64_t *)dev, a, n, (int)total);
+        LCU_LAUNCH_CHECK();
+    }
+    return LCU_OK;
+}

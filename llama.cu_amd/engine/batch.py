@@ -16,6 +16,7 @@ from typing import List, Optional, Sequence
 import torch
 
 from ..cache import CacheManager
+from ..kernels import ops
 
 
 @dataclass
@@ -84,9 +85,12 @@ class StepContext:
 
 
 class BatchBuilder:
-    """Lays the arrays of a step out in one pinned host buffer and one device buffer of
-    fixed capacity, so a step costs one host-to-device copy and the device addresses
-    never change (a captured graph can read them)."""
+    """Lays the arrays of a step out in a pinned host buffer and one device buffer of
+    fixed capacity, so a step costs one launch that brings over what it uses of them, and the device addresses
+    never change (a captured graph can read them).  The steps take turns over ``RING`` host buffers, and an event is recorded once
+    in half a ring: recording one costs the queue 4 us, as much as a small kernel, and with several buffers the host need not wait for the
+    step before last to begin."""
+    RING = 8
 
     def __init__(self, cache: CacheManager, max_tokens: int, max_reqs: int, max_pages: Sequence[int],
                  device: torch.device, extra_ints: Optional[int] = None):
@@ -111,13 +115,34 @@ class BatchBuilder:
             self.offsets[name] = (total, size)
             total += (size + 3) // 4 * 4
         pin = device.type == "cuda"
-        self.host = torch.zeros(total, dtype=torch.int32, pin_memory=pin)
         self.dev = torch.zeros(total, dtype=torch.int32, device=device)
-        self._copied: Optional[torch.cuda.Event] = None
+        self._ring = torch.zeros((self.RING if pin else 1, total), dtype=torch.int32, pin_memory=pin)     # (one piece: pinning is slow)
+        self._seen_as = [ops.host_on_device(self._ring) + 4 * total * i for i in range(self.RING)] if pin else []
+        self._turn = 0                          # whose turn it is
+        self._begun = False                     # whether the buffer whose turn it is may be written
+        self._read: List[List[torch.cuda.Event]] = [[], []]   # per half of the ring: behind the last reads of its buffers
+        self._stream: Optional[torch.cuda.Stream] = None      # where the half's buffers were read last, if no event stands behind that yet
+        self._extras_now = set()                # the names that this step has asked for
+
+    @property
+    def host(self) -> torch.Tensor:
+        """The buffer of the step that is being built."""
+        return self._ring[self._turn]
 
     def _h(self, name: str) -> torch.Tensor:
         o, s = self.offsets[name]
         return self.host[o:o + s]
+
+    def _begin(self) -> None:
+        """Wait until what the buffer whose turn it is held before has been read."""
+        if self._begun:
+            return
+        half = len(self._ring) // 2
+        if half and self._turn % half == 0:
+            for event in self._read[self._turn // half]:
+                event.synchronize()
+            self._read[self._turn // half] = []
+        self._begun = True
 
     def _d(self, name: str, count: int) -> torch.Tensor:
         o, s = self.offsets[name]
@@ -126,6 +151,8 @@ class BatchBuilder:
     def extra(self, name: str, size: int):
         """``(host, device)`` views of ``size`` entries that ``name`` owns from its first call on (the same
         addresses in every step)."""
+        self._begin()
+        self._extras_now.add(name)
         at = self._extras.get(name)
         if at is None:
             if self._extra_used + size > self.extra_ints:
@@ -138,12 +165,41 @@ class BatchBuilder:
         o = self.offsets["extra"][0] + at[0]
         return self.host[o:o + size], self.dev[o:o + size]
 
+    def _pieces(self):
+        """What the step uses of the arrays, as ``ops.step_arrays`` takes it."""
+        def whole(at, count):
+            count = (count + 3) // 4 * 4
+            return (at, count, 1, 0, count)
+        out = [whole(self.offsets[name][0], count) for name, count in self._used if count]
+        for g, (rows, cols) in enumerate(self._used_tables):
+            at, mp = self.offsets[f"block_table{g}"][0], self.max_pages[g]
+            # of every request's row the pages that the longest context reaches (rows that do not begin on 16 bytes: everything)
+            out.append((at, min((cols + 3) // 4 * 4, mp), rows, mp, mp) if mp % 4 == 0 else whole(at, rows * mp))
+        base = self.offsets["extra"][0]
+        return out + [whole(base + self._extras[name][0], self._extras[name][1]) for name in sorted(self._extras_now)]
+
     def upload(self) -> None:
-        """The step's arrays go to the device (one copy on the current stream)."""
-        self.dev.copy_(self.host, non_blocking=True)
-        if self.device.type == "cuda":
-            self._copied = torch.cuda.Event()
-            self._copied.record()
+        """What the step uses of the arrays goes to the device (on the current stream)."""
+        self._begin()
+        if not self._seen_as:
+            self.dev.copy_(self.host)
+        else:
+            stream = torch.cuda.current_stream(self.device)
+            half, turn = len(self._ring) // 2, self._turn
+            if self._stream is not None and self._stream != stream:        # (steps on several streams in turn)
+                self._read[turn // half].append(self._stream.record_event())
+            if torch.cuda.current_device() == self.device.index:
+                ops.step_arrays(self._seen_as[turn], self.dev, self._pieces())
+            else:
+                with torch.cuda.device(self.device):
+                    ops.step_arrays(self._seen_as[turn], self.dev, self._pieces())
+            self._stream = stream
+            if turn % half == half - 1:
+                self._read[turn // half].append(stream.record_event())
+                self._stream = None
+            self._turn = (turn + 1) % len(self._ring)
+        self._begun = False
+        self._extras_now = set()
 
     def build(self, req_ids: Sequence[int], tokens: Sequence[Sequence[int]], want: Sequence[Sequence[int]],
               vocab_size: int, feed: Sequence[tuple] = (), upload: bool = True) -> StepContext:
@@ -160,8 +216,8 @@ class BatchBuilder:
         if n > self.max_tokens or n_req > self.max_reqs:
             raise ValueError(f"step of {n} tokens / {n_req} requests exceeds the builder's capacity "
                              f"({self.max_tokens} / {self.max_reqs})")
-        if self._copied is not None:
-            self._copied.synchronize()          # the last copy out of the host buffer has ended
+        self._begin()
+        self._extras_now = set()
         flat = [t for ts in tokens for t in ts]
         lo, hi = min(flat), max(flat)
         if lo < 0 or hi >= vocab_size:
@@ -192,6 +248,12 @@ class BatchBuilder:
                               self.max_pages, [ptr(f"slots{g}") for g in range(len(self.max_pages))])
         ctx_lens = self._h("ctx_len")[:n_req].tolist()
         self._h("decode_order")[:n_req] = torch.tensor(sorted(range(n_req), key=lambda i: -ctx_lens[i]), dtype=torch.int32)
+        state_slots = self._h("state_slot")[:n_req].tolist()
+        longest = max(ctx_lens)
+        self._used = [("tokens", n), ("positions", n), ("req_of_token", n), ("logit_rows", len(rows)), ("q_start", n_req + 1), ("ctx_len", n_req),
+                      ("state_slot", n_req), ("decode_order", n_req), ("feed_src", len(feed)), ("feed_dst", len(feed))]
+        self._used += [(f"slots{g}", n) for g in range(len(self.max_pages))]
+        self._used_tables = [(n_req, -(-longest // group.page_size)) for group in self.cache.groups]
         if upload:
             self.upload()
         return StepContext(
@@ -202,7 +264,7 @@ class BatchBuilder:
             block_tables=[self._d(f"block_table{g}", n_req * mp).view(n_req, mp) for g, mp in enumerate(self.max_pages)],
             slot_maps=[self._d(f"slots{g}", n) for g in range(len(self.max_pages))],
             q_lens=n_new, ctx_lens=ctx_lens, req_ids=list(req_ids),
-            state_slots=self._h("state_slot")[:n_req].tolist(),
+            state_slots=state_slots,
             feed_src=self._d("feed_src", len(feed)) if feed else None,
             feed_dst=self._d("feed_dst", len(feed)) if feed else None,
             decode_order=self._d("decode_order", n_req), builder=self)

@@ -130,6 +130,29 @@ def _check(rc: int, name: str) -> None:
     raise KernelError(f"{name}: launch failed with HIP error {rc}")
 
 
+# ------------------------------------------------------------------ a step's arrays
+
+
+def host_on_device(host: torch.Tensor) -> int:
+    """The address under which kernels read the pinned host tensor ``host``."""
+    if not host.is_pinned():
+        raise KernelError("host_on_device: the tensor must lie in pinned host memory")
+    at = ctypes.c_void_p()
+    _check(build.load("step_arrays").lcu_host_on_device(_ptr(host), ctypes.byref(at)), "host_on_device")
+    return at.value
+
+
+def step_arrays(host: int, dev: torch.Tensor, pieces) -> None:
+    """Pieces of an int32 array in pinned host memory (``host``: its address as ``host_on_device`` gives it) to the same places of ``dev``, on
+    the current stream: ``pieces`` holds ``(at, cols, rows, stride, width)`` in entries (multiples of 4, but for ``rows``): ``rows`` rows
+    that begin at entry ``at`` and then every ``stride``, of whose ``width`` entries the first ``cols`` come over and the others become zero."""
+    _gpu(dev)
+    _i32(dev, "step_arrays dev")
+    flat = [v for piece in pieces for v in piece]
+    _check(build.load("step_arrays").lcu_step_arrays(ctypes.c_void_p(host), _ptr(dev), ctypes.c_longlong(dev.numel()), (ctypes.c_int * len(flat))(*flat), len(pieces),
+                                                     _stream()), "step_arrays")
+
+
 # ------------------------------------------------------------------ elementwise
 
 
