@@ -6,7 +6,7 @@
 //            over all experts, the choice by s + a correction per expert, and the chosen scores divided by their sum (or as
 //            they are) times a factor as weights; the choice may be limited to the experts of the best groups; rows of the router's matrix behind the experts' are gates: sigmoid of their logit goes out per
 //            token; the last experts may be identity experts, which have no matrices and return their input;
-//   group:   the (token, choice) pairs sorted by expert and cut into tiles of up to 64 rows of one expert, on the
+//   group:   the (token, choice) pairs sorted by expert and cut into tiles of up to 128 rows of one expert, on the
 //            device (nothing comes back to the host); where experts have few pairs a product's workgroups look for theirs
 //            themselves instead;
 //   up:      act = gelu(W_up[e] (weight * h))    the weight scales what goes INTO the expert; or, gated:
@@ -22,7 +22,7 @@
 #include "lane_moves.h"
 
 constexpr int MOE_MAX_EXPERTS = 1024;
-constexpr int MOE_TILE_ROWS = 64;        // rows of a tile of the kernel for many rows
+constexpr int MOE_TILE_ROWS = 128;       // rows of a tile of the kernel for many rows at most
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
@@ -206,7 +206,8 @@ moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, cons
 // One block.  ids: [total] experts of the (token, choice) pairs in flat order.  Writes
 // sorted_to_flat [total] (the pairs sorted by expert), and the tiles of up to rows_per_tile rows:
 // tile_expert, tile_begin (first sorted row), tile_rows, each [max_tiles], and n_tiles [1].  Only the first `tiled`
-// experts get tiles: the ones behind them have no matrices (identity experts), and their pairs are only sorted.
+// experts get tiles: the ones behind them have no matrices (identity experts), and their pairs are only sorted.  An expert's tiles are as few as
+// can be and of nearly the same size, a multiple of 16 rows but for the last.
 // A thread an expert: the pairs and tiles before its own by a sum over the threads (one thread that walked 1,024 experts took 40 us).
 static_assert(MOE_MAX_EXPERTS <= 1024, "a thread an expert");
 __global__ void __launch_bounds__(1024)
@@ -235,10 +236,11 @@ moe_group_kernel(const int *__restrict__ ids, int total, int experts, int *__res
     at -= pairs;
     tile -= tiles;
     if (e < experts) cursor[e] = at;
+    const int even = tiles ? ((pairs + tiles - 1) / tiles + 15) / 16 * 16 : 0;
     for (int k = 0; k < tiles && tile + k < max_tiles; ++k) {
         tile_expert[tile + k] = e;
-        tile_begin[tile + k] = at + k * rows_per_tile;
-        tile_rows[tile + k] = min(pairs - k * rows_per_tile, rows_per_tile);
+        tile_begin[tile + k] = at + k * even;
+        tile_rows[tile + k] = min(pairs - k * even, even);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < total; i += blockDim.x) sorted_to_flat[atomicAdd(&cursor[ids[i]], 1)] = i;
@@ -334,6 +336,10 @@ template <class T, bool PACKED> struct Unit {
     __device__ __forceinline__ typename M::frag load(int step) const {
         if (PACKED) return __builtin_nontemporal_load((const typename M::frag *)(p + (size_t)step * WAVE * M::PER_LANE));
         return step * M::KSTEP < k_left ? M::load(p + step * M::KSTEP) : M::zero();
+    }
+    // the same for a piece that several workgroups read; not PACKED and beyond K: a piece of the row that exists
+    __device__ __forceinline__ typename M::frag cached(int step) const {
+        return M::load(PACKED ? p + (size_t)step * WAVE * M::PER_LANE : p + min(step * M::KSTEP, k_left - M::PER_LANE));
     }
 };
 
@@ -489,129 +495,138 @@ moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__
     }
 }
 
-// Many rows an expert (prompts): tiles of up to 64 rows; a block of four waves takes a tile and 128
-// features.  Rows and weights go through LDS in steps of 128 bytes of k, the next step's loads on their
-// way while one is multiplied; a wave multiplies 32 features with all 64 rows (eight sums).
-template <class T, int MODE, bool PACKED>
-__global__ void __launch_bounds__(256)
-moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__ w, size_t w_expert_stride, int N, int K,
-                     const int *__restrict__ sorted_to_flat, const float *__restrict__ wts,
-                     const int *__restrict__ tile_expert, const int *__restrict__ tile_begin,
-                     const int *__restrict__ tile_rows, const int *__restrict__ n_tiles, int max_tiles, T *__restrict__ out_t,
-                     float *__restrict__ out_f, int out_stride, int top, int add, float alpha, float limit) {
+// Many rows an expert (prompts): tiles of up to 96 or 128 rows; a block of four waves takes a tile and 128 features, a wave 32 of them with all
+// rows.  The rows go through LDS in steps of 128 bytes of k, in two buffers in turn with one barrier a step; no two waves want the same piece of the
+// matrix, so each loads its own straight into registers.  Both are two steps ahead.  MT: tiles of 16 rows that are multiplied.
+// What bounds it are the turns of loads, LDS and barrier of the two blocks that a compute unit holds (half the matrix instructions take as long) and, up
+// to 50 rows an expert, the matrices out of memory.  Tiles of 64 rows whose matrices went through LDS too took, per pass of both products, 16 experts
+// of 2048 x 2048 with 2,014 tokens of two each 241 us, now 176; gated, 2 x 1024: 180 and 139; 200 tokens of two 77 and 51.  (Rows copied into LDS by the
+// loads themselves, four buffers, the barrier in the middle of the instructions: the same times; 64 rows and three blocks: 5 to 30 % longer.)
+template <class T, int MODE, bool PACKED, int MT>
+__device__ __forceinline__ void moe_many_tile(T *__restrict__ xs, const T *__restrict__ x, int x_stride, const T *__restrict__ we, int N, int K,
+                                              const int *__restrict__ sorted_to_flat, const float *__restrict__ wts, int n0, int row0, int rows,
+                                              T *__restrict__ out_t, float *__restrict__ out_f, int out_stride, int top, int add, float alpha, float limit) {
     typedef Mma<T> M;
     typedef typename M::frag frag;
     constexpr int PL = M::PER_LANE;                 // elements in 16 bytes
     constexpr int KS = 128 / sizeof(T);             // elements of k a step
     constexpr int CH = KS / PL;                     // 16-byte pieces of a row a step: 8
-    constexpr int LD = KS + PL;                     // a row in LDS, with a piece of padding against bank conflicts
-    __shared__ __attribute__((aligned(16))) T xs[64 * LD];
-    __shared__ __attribute__((aligned(16))) T ws[128 * LD];
-    // Workgroups go to the chip's eight dies in turn (workgroup i to die i % 8), and each die has an L2 of its own.  The
-    // tiles of one expert want the same block of its matrix: a die takes the feature blocks die, die + 8, ... and walks
-    // the tiles of each in turn, so that a block of a matrix comes from memory to one die only.
-    const int n_fb = (N + 127) / 128, die = blockIdx.x % 8, at = blockIdx.x / 8;
-    const int fb = die + 8 * (at / max_tiles), tile = at % max_tiles;
-    if (fb >= n_fb || tile >= n_tiles[0]) return;
-    const int n0 = fb * 128;
-    const int e = tile_expert[tile], row0 = tile_begin[tile], rows = tile_rows[tile];
+    constexpr int SS = KS / M::KSTEP;               // units of k a step: 2
+    constexpr int XP = MT / 2;                      // rows that a thread copies
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, g = lane / 16, l16 = lane % 16;
     const int ch = tid % CH;                        // this thread's piece of k in every row it copies
-    const T *xptr[2];
-    float xsc[2];
+    unsigned xrow[XP];                              // (a row's number, not its address: registers are short)
+    float xsc[XP];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < XP; ++i) {
         const int r = tid / CH + 32 * i;
-        const int srow = row0 + (r < rows ? r : 0);
-        if (MODE != MOE_DOWN) {
-            const int flat = sorted_to_flat[srow];
-            xptr[i] = x + (size_t)(flat / top) * x_stride + ch * PL;
-            xsc[i] = MODE == MOE_UP ? wts[flat] : 1.f;
-        } else {
-            xptr[i] = x + (size_t)srow * x_stride + ch * PL;
-            xsc[i] = 1.f;
-        }
+        const int srow = row0 + (r < rows ? r : 0), flat = MODE != MOE_DOWN ? sorted_to_flat[srow] : srow;
+        xrow[i] = MODE != MOE_DOWN ? flat / top : flat;
+        xsc[i] = MODE == MOE_UP ? wts[flat] : 1.f;
     }
-    // the weight's piece i of this thread: row wr[i] of the tile, 16 bytes of k from element wk on
-    constexpr int SS = KS / M::KSTEP;               // units of k a step
-    const int steps = (K + M::KSTEP - 1) / M::KSTEP;
-    const T *wptr[4];
-    int wr[4], wk;
+    const int units = (K + M::KSTEP - 1) / M::KSTEP, steps = (units + SS - 1) / SS, tile0 = n0 / 16 + 2 * wave;
+    const Unit<T, PACKED> w0(we, tile0, N, K, units, lane), w1(we, tile0 + 1, N, K, units, lane);
+    frag xreg[2][XP], a[2][SS][2];
+    const int full = K / KS;                        // steps that are all within K
+    // every load is issued, with a place that exists: beyond the last step it is the last step's, beyond K the last piece of the row
+    auto rows_of = [&](auto buf, int step) {
+        const unsigned k = min(min(step, steps - 1) * KS + ch * PL, K - PL);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if (PACKED) {                               // a wave takes whole units: pieces tid + 256 i of [8 tiles of rows][SS][64 lanes]
-            const int unit = wave + 4 * i, rt = unit / SS, tiles = (N + 15) / 16, t = n0 / 16 + rt;
-            wr[i] = 16 * rt + l16;
-            wk = unit % SS * M::KSTEP + g * PL;     // (4 units are whole rows of units: the same for every i)
-            wptr[i] = w + (size_t)e * w_expert_stride + (((size_t)(t < tiles ? t : tiles - 1) * steps + unit % SS) * WAVE + lane) * PL;
-        } else {
-            const int fr = n0 + tid / CH + 32 * i;
-            wr[i] = tid / CH + 32 * i;
-            wk = ch * PL;
-            wptr[i] = w + (size_t)e * w_expert_stride + (size_t)(fr < N ? fr : N - 1) * K + ch * PL;
-        }
-    }
-    frag xreg[2], wreg[4];
-    auto from_memory = [&](int k0) {
-        const bool in = k0 + ch * PL < K, w_in = PACKED ? k0 + wk / M::KSTEP * M::KSTEP < K : in;
+        for (int i = 0; i < XP; ++i) xreg[decltype(buf)::value][i] = M::load(x + ((size_t)xrow[i] * (unsigned)x_stride + k));
+    };
+    auto weights_of = [&](auto buf, int step) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) wreg[i] = w_in ? M::load(wptr[i] + (PACKED ? (size_t)(k0 / M::KSTEP) * WAVE * PL : k0)) : M::zero();
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            xreg[i] = in ? M::load(xptr[i] + k0) : M::zero();
-            if (MODE == MOE_UP) xreg[i] = M::scaled(xreg[i], xsc[i]);
+        for (int u = 0; u < SS; ++u) {
+            const int s = min(min(step, steps - 1) * SS + u, units - 1);
+            a[decltype(buf)::value][u][0] = w0.cached(s);
+            a[decltype(buf)::value][u][1] = w1.cached(s);
         }
     };
-    f32x4 acc[2][4], sum[2][4];
+    auto rows_to_lds = [&](auto buf, int step) {
+        constexpr int B = decltype(buf)::value;
+        if (step >= full) {                         // the last step, partly beyond K (a branch, no select in every step)
+            asm volatile("");
+            if (step * KS + ch * PL >= K)
+#pragma unroll
+                for (int i = 0; i < XP; ++i) xreg[B][i] = M::zero();
+        }
+#pragma unroll
+        for (int i = 0; i < XP; ++i) {
+            frag v = xreg[B][i];
+            if (MODE == MOE_UP) v = M::scaled(v, xsc[i]);
+            *(frag *)(xs + (B * 16 * MT + tid / CH + 32 * i) * KS + (ch ^ (tid / CH % 8)) * PL) = v;
+        }
+    };
+    f32x4 acc[2][MT], sum[2][MT];
 #pragma unroll
     for (int ft = 0; ft < 2; ++ft)
 #pragma unroll
-        for (int m = 0; m < 4; ++m) acc[ft][m] = sum[ft][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    from_memory(0);
-    int left = quarter_steps(steps) / SS;           // steps of this part that are left
-    // (one buffer and two barriers a step: with two buffers in turn and one barrier the kernel was a quarter slower, its
-    // workgroups being fewer on a compute unit)
-    for (int k0 = 0; k0 < K; k0 += KS) {
-        __syncthreads();                            // the step before has been read
-#pragma unroll
-        for (int i = 0; i < 2; ++i) *(frag *)(xs + (tid / CH + 32 * i) * LD + ch * PL) = xreg[i];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) *(frag *)(ws + wr[i] * LD + wk) = wreg[i];
-        __syncthreads();
+        for (int m = 0; m < MT; ++m) acc[ft][m] = sum[ft][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int part = quarter_steps(units) / SS;     // steps of a part of K
+    int left = part;                                // of this part that are left
+    auto one = [&](auto buf, int step) {
+        constexpr int B = decltype(buf)::value;
+        lds_barrier();                              // this step's rows are there, the step before has been read
+        rows_of(buf, step + 2);
         if (left == 0) {
-            left = quarter_steps(steps) / SS;
+            left = part;
 #pragma unroll
             for (int ft = 0; ft < 2; ++ft)
 #pragma unroll
-                for (int m = 0; m < 4; ++m) {
+                for (int m = 0; m < MT; ++m) {
                     sum[ft][m] += acc[ft][m];
                     acc[ft][m] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
         }
         --left;
-        if (k0 + KS < K) from_memory(k0 + KS);
+        if (step >= full) {
+            asm volatile("");
 #pragma unroll
-        for (int ks = 0; ks < KS / M::KSTEP; ++ks) {
-            frag a[2], b[4];
-#pragma unroll
-            for (int ft = 0; ft < 2; ++ft) a[ft] = *(const frag *)(ws + (32 * wave + 16 * ft + l16) * LD + ks * M::KSTEP + g * PL);
-#pragma unroll
-            for (int m = 0; m < 4; ++m) b[m] = *(const frag *)(xs + (16 * m + l16) * LD + ks * M::KSTEP + g * PL);
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                if (16 * m < rows) {
-#pragma unroll
-                    for (int ft = 0; ft < 2; ++ft) acc[ft][m] = M::mma(a[ft], b[m], acc[ft][m]);
-                }
-            }
+            for (int u = 0; u < SS; ++u)
+                if (step * SS + u >= units || (!PACKED && (step * SS + u) * M::KSTEP + g * PL >= K)) a[B][u][0] = a[B][u][1] = M::zero();
         }
+        __builtin_amdgcn_sched_barrier(0);
+        // piece p of row r lies at p ^ (r % 8) of the row: whichever lanes the LDS serves together, they are in different banks
+        frag b[SS * MT];
+#pragma unroll
+        for (int i = 0; i < SS * MT; ++i)
+            b[i] = *(const frag *)(xs + (B * 16 * MT + 16 * (i % MT) + l16) * KS + ((i / MT * 4 + g) ^ (l16 % 8)) * PL);
+#pragma unroll
+        for (int i = 0; i < SS * MT; ++i) {
+            const int u = i / MT, m = i % MT;
+            acc[0][m] = M::mma(a[B][u][0], b[i], acc[0][m]);
+            acc[1][m] = M::mma(a[B][u][1], b[i], acc[1][m]);
+        }
+        // RA reads of rows are always on their way ahead of the products
+        constexpr int RA = 4, PER = 2 * (sizeof(T) == 4 ? 4 : 1);
+        __builtin_amdgcn_sched_group_barrier(0x100, RA, 0);
+#pragma unroll
+        for (int i = RA; i < SS * MT; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, PER * RA, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        weights_of(buf, step + 2);
+        rows_to_lds(Int<1 - B>(), step + 1);
+    };
+    rows_of(Int<0>(), 0);
+    weights_of(Int<0>(), 0);
+    rows_of(Int<1>(), 1);
+    weights_of(Int<1>(), 1);
+    rows_to_lds(Int<0>(), 0);
+    int step = 0;
+    for (; step + 1 < steps; step += 2) {
+        one(Int<0>(), step);
+        one(Int<1>(), step + 1);
     }
+    if (step < steps) one(Int<0>(), step);
 #pragma unroll
     for (int ft = 0; ft < 2; ++ft)
 #pragma unroll
-        for (int m = 0; m < 4; ++m) acc[ft][m] = sum[ft][m] + acc[ft][m];
+        for (int m = 0; m < MT; ++m) acc[ft][m] = sum[ft][m] + acc[ft][m];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < MT; ++m) {
         const int r = 16 * m + l16;
         if (r >= rows) continue;
         const int srow = row0 + r;
@@ -620,18 +635,42 @@ moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict_
             const int flat = sorted_to_flat[srow];
             dst = add ? flat / top : flat;
         }
-        if (MODE == MOE_UP_GATED) {                 // the wave's first 16 rows are a gate block, its second the up block that meets it
+        if constexpr (MODE == MOE_UP_GATED) {       // the wave's first 16 rows are a gate block, its second the up block that meets it
+            const int col = (n0 + 32 * wave) / 2 + 4 * g;
+            Quad<T> q;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int col = (n0 + 32 * wave) / 2 + 4 * g + i;
-                if (col < N / 2) out_t[(size_t)dst * out_stride + col] = from_f32<T>(gate_up_of(acc[0][m][i], acc[1][m][i], alpha, limit));
-            }
-            continue;
+            for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gate_up_of(acc[0][m][i], acc[1][m][i], alpha, limit));
+            if (col < N / 2) *(Quad<T> *)(out_t + (size_t)dst * out_stride + col) = q;
+        } else {
+#pragma unroll
+            for (int ft = 0; ft < 2; ++ft) moe_store<T, MODE>(acc[ft][m], dst, n0 + 32 * wave + 16 * ft + 4 * g, N, out_t, out_f, out_stride, add);
         }
-#pragma unroll
-        for (int ft = 0; ft < 2; ++ft)
-            moe_store<T, MODE == MOE_UP_GATED ? MOE_UP : MODE>(acc[ft][m], dst, n0 + 32 * wave + 16 * ft + 4 * g, N, out_t, out_f, out_stride, add);
     }
+}
+
+template <class T, int MODE, bool PACKED>
+__global__ void __launch_bounds__(256, 2)
+moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__ w, size_t w_expert_stride, int N, int K,
+                     const int *__restrict__ sorted_to_flat, const float *__restrict__ wts,
+                     const int *__restrict__ tile_expert, const int *__restrict__ tile_begin,
+                     const int *__restrict__ tile_rows, const int *__restrict__ n_tiles, int max_tiles, T *__restrict__ out_t,
+                     float *__restrict__ out_f, int out_stride, int top, int add, float alpha, float limit) {
+    __shared__ __attribute__((aligned(16))) T xs[2 * MOE_TILE_ROWS * 128 / sizeof(T)];
+    // Workgroups go to the chip's eight dies in turn (workgroup i to die i % 8), and each die has an L2 of its own.  The work, in the order
+    // four tiles after four tiles, their feature blocks, the tiles, is cut into eight pieces: what a die has at hand at a time are a few
+    // tiles' rows and a few experts' matrices, and each comes to one die (at the pieces' borders two).
+    // (By feature blocks, every die read every row: 16 experts, 200 tokens of two 65 us, 51 so; 2,040 tokens 157 and 142.)
+    const int n_fb = (N + 127) / 128, tiles = n_tiles[0], each = (tiles * n_fb + 7) / 8, at = blockIdx.x / 8, item = blockIdx.x % 8 * each + at;
+    if (at >= each || item >= tiles * n_fb) return;
+    const int first = item / (4 * n_fb) * 4, rest = item - first * n_fb, side = min(4, tiles - first), fb = rest / side, tile = first + rest % side;
+    const T *we = w + (size_t)tile_expert[tile] * w_expert_stride;
+    const int row0 = tile_begin[tile], rows = tile_rows[tile];
+#define TILE(MT) moe_many_tile<T, MODE, PACKED, MT>(xs, x, x_stride, we, N, K, sorted_to_flat, wts, fb * 128, row0, rows, out_t, out_f, out_stride, top, add, alpha, limit)
+    if (rows > 96) TILE(8);
+    else if (rows > 64) TILE(6);
+    else if (rows > 32) TILE(4);
+    else TILE(2);
+#undef TILE
 }
 
 // out[t, c] (+)= sum_k wts[t, k] * y[t * top + k, c]  (in the order of k; wts null: ones)  + gate[t] * shared[t, c]  (shared null: nothing;
@@ -664,10 +703,12 @@ moe_combine_kernel(float *__restrict__ out, const float *__restrict__ y, const f
 }
 
 // Rows of a tile for n * top pairs over so many experts: while an expert has 16 rows or fewer on average the kernel for few rows, with no
-// tiles up to MOE_LIST pairs (0; MOE_LIST_F32 in 32 bits) and tiles of 16 beyond; else 64.  The caller sizes its scratch with it: max_tiles = min(total,
-// total / rows + experts), or 0.
+// tiles up to MOE_LIST pairs (0; MOE_LIST_F32 in 32 bits) and tiles of 16 beyond.  Else 96 (128 rows: 2,014 tokens of two on 16 experts 176 -> 195 us, 512 on 8 experts of 4096 x 4096 241 -> 257; more work in a block leaves more
+// compute units without any at the end), but 128 where an expert's rows on average are just more than a tile of 96 and would make two (100 rows: 84 -> 66 us).  The caller sizes its
+// scratch with it: max_tiles = min(total, total / rows + experts), or 0.
 LCU_API int lcu_moe_tile_rows(int type, int total, int experts) {
-    return (long long)total > 16ll * experts ? MOE_TILE_ROWS : total > (type == LCU_F32 ? MOE_LIST_F32 : MOE_LIST) ? 16 : 0;
+    if ((long long)total > 16ll * experts) return (long long)total > 80ll * experts && (long long)total <= 120ll * experts ? MOE_TILE_ROWS : 96;
+    return total > (type == LCU_F32 ? MOE_LIST_F32 : MOE_LIST) ? 16 : 0;
 }
 
 // h: [n, d] of `type`; router: [experts, d] 32-bit; ids, wts: [n * top].
@@ -701,7 +742,7 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
 // token's input.  shared (null or
 // [n, d] of `type`) with shared_gate (null or [n] 32-bit): rows that are added beside the experts', times the gate.  shared_up,
 // shared_down (null, or the matrices [2 * shared_ff, d] and [d, shared_ff] of a shared expert that is computed here, with silu, in the order of Unit
-// like w_up and w_down; only where lcu_moe_tile_rows does not say 64): act then holds n * shared_ff elements more and y n rows more.
+// like w_up and w_down; only where lcu_moe_tile_rows says 16 or 0): act then holds n * shared_ff elements more and y n rows more.
 LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float *wts, int *ints, int max_tiles,
                             const void *w_up, int packed_up, const void *w_down, int packed_down, void *act, float *y, float *out, int n, int d, int ff,
                             int experts, int top, int gated, const void *shared, const float *shared_gate, const void *shared_up,
@@ -714,7 +755,7 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
         return LCU_BAD_ARGUMENT;
     const int total = n * top;
     const int tile_rows = lcu_moe_tile_rows(type, total, experts);
-    const bool few = tile_rows < MOE_TILE_ROWS;
+    const bool few = tile_rows <= 16;
     if (shared_up && (!shared_down || shared || !gated || !few || !packed_up || !packed_down || shared_ff <= 0 || shared_ff % 16)) return LCU_BAD_ARGUMENT;
     const int add = top == 1 && !gated;
     float *down_to = add ? out : y;
@@ -758,7 +799,7 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
 #undef DOWN
     } else {
         // flat grids: the kernel shares them out over the dies itself
-        const dim3 block(256), gu(8 * max_tiles * (((up_rows + 127) / 128 + 7) / 8)), gd(8 * max_tiles * (((d + 127) / 128 + 7) / 8));
+        const dim3 block(256), gu((max_tiles * ((up_rows + 127) / 128) + 7) / 8 * 8), gd((max_tiles * ((d + 127) / 128) + 7) / 8 * 8);
 #define UP(T, PACKED, MODE) moe_gemm_many_kernel<T, MODE, PACKED><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \
                                                 sorted, wts, t_exp, t_beg, t_rows, n_tiles, max_tiles, (T *)act, nullptr, ff, top, 0, alpha, limit)
 #define DOWN(T, PACKED, MODE) moe_gemm_many_kernel<T, MODE, PACKED><<<gd, block, 0, stream>>>((const T *)act, ff, (const T *)w_down, down_stride, d, ff, \

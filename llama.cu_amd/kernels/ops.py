@@ -1578,7 +1578,7 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
     max_tiles = min(total, total // tile + experts) if tile else 0
     ints = torch.empty(total + 3 * max_tiles + 1, dtype=torch.int32, device=h.device) if tile else None
     act = torch.empty(total * ff + n * sff, dtype=h.dtype, device=h.device)
-    y = torch.empty((total + (n if sff else 0), d), dtype=torch.float32, device=h.device) if (top > 1 or gated) else None
+    y = torch.empty((total + (n if sff else 0), d), dtype=torch.float32, device=h.device) if (top > 1 or gated or tile > 16) else None
     _check(lib.lcu_moe_experts(_ptr(h), _type(h, "moe input"), _ptr(ids), _ptr(wts), _ptr(ints), max_tiles, _ptr(up),
                                int(up is not w_up), _ptr(down), int(down is not w_down), _ptr(act), _ptr(y), _ptr(out), n, d, ff, experts, top, int(bool(gated)),
                                _ptr(shared), _ptr(shared_gate if shared is not None or sff else None), _ptr(shared_up.data if sff else None),

@@ -174,3 +174,37 @@ def test_a_token_with_few_and_with_more_others(dtype, gated):
                 # a rounding is at most 2^-9 of a value: one of sff activations under weights of sff ** -0.5 each (2^-9 of the largest together, and
                 # the other path's as much), one of the shared row
                 assert_close(got, whole[first:first + n].cpu().to(F64), 3 * 2.0 ** -9, f"{n}")
+
+
+# an expert's tiles at their edges (of 96 rows, and of 128 where there are 80 to 120 an expert on average), beside experts with few rows and with none;
+# K of less than a step, of whole steps, and one that ends within a unit of the last; features that end within a block, fewer blocks than dies
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("counts,d,ff", [((17, 96, 97, 0, 33, 193), 264, 48), ((128, 129, 81, 95, 0, 100), 1096, 272), ((1, 600, 31, 65), 40, 1040),
+                                         ((32, 64, 127, 96, 1, 288), 64, 16)])
+@pytest.mark.parametrize("gated,pack", [(True, True), (True, False), (False, True), (False, False)])
+def test_tiles_of_many_rows(dtype, counts, d, ff, gated, pack):
+    from llama_cu_amd.kernels import ops
+    experts, n, tdt = len(counts), sum(counts), TYPES[dtype]
+    order = torch.randperm(n, generator=torch.Generator().manual_seed(0))
+    ids = torch.repeat_interleave(torch.arange(experts, dtype=torch.int32), torch.tensor(counts))[order].view(n, 1).cuda()
+    h, wts = rnd(n, d, seed=1).to(tdt).cuda(), torch.rand(n, 1, generator=torch.Generator().manual_seed(2)).cuda()
+    gate, up = (rnd(experts, ff, d, seed=k, std=d ** -0.5).to(tdt).cuda() for k in (3, 4))
+    down = rnd(experts, d, ff, seed=5, std=ff ** -0.5).to(tdt).cuda()
+    u, w = ops.gated_rows(gate, up) if gated else up, down
+    if pack:
+        u, w = ops.pack_experts(u), ops.pack_experts(w)
+
+    def run(part):
+        out = torch.zeros(part.stop - part.start, d, device="cuda")
+        return ops.moe_experts(h[part].contiguous(), ids[part].contiguous(), wts[part].contiguous(), u, w, out, **({"gated": True, "fresh": True} if gated else {}))
+    got = run(slice(0, n))
+    few = 16 * experts                     # steps of so few take the kernel for few rows: a token has the same bits
+    assert torch.equal(got, torch.cat([run(slice(a, min(n, a + few))) for a in range(0, n, few)]))
+    e, x, s = ids[:, 0].long().cpu(), h.cpu().to(F64), wts.cpu().to(F64)
+    g, v, y = gate.cpu().to(F64)[e], up.cpu().to(F64)[e], down.cpu().to(F64)[e]
+    if gated:
+        a = torch.einsum("nfd,nd->nf", g, x)
+        want = s * torch.einsum("ndf,nf->nd", y, a * torch.sigmoid(a) * torch.einsum("nfd,nd->nf", v, x))
+    else:
+        want = torch.einsum("ndf,nf->nd", y, torch.nn.functional.gelu(torch.einsum("nfd,nd->nf", v, x * s)))
+    assert_close(got, want, 1e-4 if dtype == "float32" else 3e-2, "output")
