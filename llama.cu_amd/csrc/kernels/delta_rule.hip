@@ -16,13 +16,15 @@
 // A request that feeds many tokens in a step goes through chunks on the matrix cores instead of the scan (delta_chunks.h, which says when: from some
 // 64 to 200 tokens on) if its outputs are rounded to bfloat16; 32-bit models keep the scan, whose bits do not depend on the cut of a prompt.
 // A token's result depends on the tokens before it in its request only; portions that are scanned are folded in in an
-// order of operations that does not depend on how the request was cut into them, chunks change roundings.
+// order of operations that does not depend on how the request was cut into them, chunks change roundings.  Where every request feeds one token
+// the three are one kernel (the gated rule, with its convolution: two), with the same bits.
 #include <limits.h>
 #include "common.h"
 #include "lane_moves.h"
 #include "delta_chunks.h"
 
 constexpr int MAX_RANK = 512;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 constexpr float DECAY_SCALE = 0.6065306597126334f;      // exp(-1/2)
 
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + expf(-z)); }
@@ -192,7 +194,7 @@ delta_scan_kernel(const T *__restrict__ proj, int row_stride, int off_v, const f
                     const float gd = vec[turn][b][NV * VEC], c = v[b] - vec[turn][b][NV * VEC + 1] * us;
 #pragma unroll
                     for (int i = 0; i < SL; ++i) {
-                        S[i] = gd * S[i] + U[i] * c;
+                        S[i] = __builtin_fmaf(gd, S[i], U[i] * c);       // (written out: the kernel for one token rounds alike)
                         acc4[i & 3] += S[i] * R[i];
                     }
                 } else {
@@ -352,6 +354,177 @@ LCU_API int lcu_delta_rule(const void *proj, int type, int row_stride, int off_r
     return LCU_BAD_ARGUMENT;
 }
 
+// ---------------------------------------------------------------- one token a request
+// A step in which every request feeds one token (decoding).  What the kernels above take a launch each for, 2 to 5 us of which most is the way of their
+// inputs from another kernel's stores, is one workgroup's work here: a workgroup per (request, head), whose four waves take 32 columns of S at
+// a time.  A lane holds four neighbouring columns (16-byte loads) of SL = DK / 8 key channels, the groups of lanes as in the scan; every sum is made in
+// the scan's order, so a token has the same bits either way.  The matrices are on their way while the token's vectors are made.
+// Few requests wait for memory's latency, many for the matrices, read and written once.  16 heads of 128 x 128, rank 64, a chain of such steps: 1 request 9.1 ->
+// 6.3 us, 16 requests 23.9 -> 9.0, 200 requests 246 -> 68; the gated rule with its convolution and products 18.7 -> 15.5, 27.4 -> 19.9, 224 -> 91.  (Heads of 32
+// with a rank of 512, 200 requests: 59 and 61, each request reads the decay's second matrix.)
+template <int DK> struct SingleColumns {
+    static constexpr int SL = DK / 8, SLP = SL + 4, VEC = 8 * SLP;      // a vector in LDS: the groups' shares, four floats of padding behind each
+    f32x4_t S[SL];
+    __device__ __forceinline__ void load(const float *m, int g, int col, int dv, bool fresh) {
+#pragma unroll
+        for (int i = 0; i < SL; ++i) S[i] = fresh ? f32x4_t{0.f, 0.f, 0.f, 0.f} : *(const f32x4_t *)(m + (size_t)(g * SL + i) * dv + col);
+    }
+    __device__ __forceinline__ void store(float *m, int g, int col, int dv) const {
+#pragma unroll
+        for (int i = 0; i < SL; ++i) *(f32x4_t *)(m + (size_t)(g * SL + i) * dv + col) = S[i];
+    }
+    // u^T S of the four columns: U, the unit key's share of the lane's group
+    __device__ __forceinline__ f32x4_t times(const float *U) const {
+        f32x4_t p[4] = {};
+#pragma unroll
+        for (int i = 0; i < SL; ++i) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) p[i & 3][e] += U[i] * S[i][e];
+        }
+        f32x4_t out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = sum_over_groups<8>((p[0][e] + p[1][e]) + (p[2][e] + p[3][e]));
+        return out;
+    }
+};
+// where element i of a vector stands in LDS
+template <int DK> __device__ __forceinline__ int single_at(int i) { return i / SingleColumns<DK>::SL * SingleColumns<DK>::SLP + i % SingleColumns<DK>::SL; }
+
+constexpr int SINGLE_MAX_DV = 512;
+
+// The general rule from its projections to what the output matrix reads.  The arithmetic is that of delta_prep_kernel, delta_scan_kernel and delta_out_kernel.
+template <class T, int DK>
+__global__ void __launch_bounds__(256)
+delta_single_kernel(const T *__restrict__ proj, int row_stride, int off_r, int off_k, int off_v, int off_g, int off_a, int off_l,
+                    const float *__restrict__ w2t, const float *__restrict__ w0, const float *__restrict__ a_bias, const float *__restrict__ weight,
+                    float *__restrict__ state, T *__restrict__ out, const int *__restrict__ ctx_len, const int *__restrict__ state_slot,
+                    int heads, int dv, int rank, float eps) {
+    typedef SingleColumns<DK> C;
+    constexpr int SL = C::SL, HALVES = (DK + WAVE - 1) / WAVE, AHEAD = 16;
+    __shared__ __attribute__((aligned(16))) float th[MAX_RANK], vec[5][C::VEC], part[4][HALVES][WAVE], os[SINGLE_MAX_DV];
+    const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane / 8;
+    const bool fresh = ctx_len[r] == 1;
+    const T *row = proj + (size_t)r * row_stride;
+    float *m = state + ((size_t)state_slot[r] * heads + h) * DK * dv;
+    C c;
+    int col = 32 * wave + lane % 8 * 4;
+    // every load whose place is known goes out first: with each where it is used six trips to memory stood behind one another (14.8 us, the three
+    // kernels 16.2)
+    const int quarter = (rank + 3) / 4, j0 = wave * quarter, j1 = min(rank, j0 + quarter);
+    auto second = [&](int j, int b) { return w2t[(size_t)min(j, rank - 1) * heads * DK + h * DK + min(b * WAVE + lane, DK - 1)]; };
+    float lo = 0.f, k2[HALVES], w2[AHEAD][HALVES], v[4], mine[5], out_w = 0.f, out_g = 0.f;
+    if ((int)threadIdx.x < rank) lo = to_f32(row[off_l + threadIdx.x]);
+#pragma unroll
+    for (int b = 0; b < HALVES; ++b) k2[b] = b * WAVE + lane < DK ? to_f32(row[off_k + h * DK + b * WAVE + lane]) : 0.f;
+    {
+        const int ch = h * DK + min((int)threadIdx.x, DK - 1);
+        mine[0] = w0[ch];
+        mine[1] = to_f32(row[off_a + ch]);
+        mine[2] = a_bias[ch];
+        mine[3] = to_f32(row[off_k + ch]);
+        mine[4] = to_f32(row[off_r + ch]);
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+#pragma unroll
+        for (int b = 0; b < HALVES; ++b) w2[j][b] = second(j0 + j, b);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = to_f32(row[off_v + h * dv + min(col, dv - 4) + e]);
+    if ((int)threadIdx.x < dv) {
+        out_w = weight[h * dv + threadIdx.x];
+        out_g = to_f32(row[off_g + h * dv + threadIdx.x]);
+    }
+    c.load(m, g, min(col, dv - 4), dv, fresh);
+    __builtin_amdgcn_sched_barrier(0);
+    // the token's vectors
+    if ((int)threadIdx.x < rank) th[threadIdx.x] = tanhf(lo);
+    for (int x = threadIdx.x + 256; x < rank; x += 256) th[x] = tanhf(to_f32(row[off_l + x]));
+    float ss = 0.f;
+#pragma unroll
+    for (int b = 0; b < HALVES; ++b) ss = __builtin_fmaf(k2[b], k2[b], ss);      // (as the other kernel's loop does it; of two products the compiler may round either)
+    const float inv = 1.0f / sqrtf(wave_sum_in_place(ss) + 1e-6f);
+    lds_barrier();
+    float z[HALVES] = {};
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+        if (j0 + j >= j1) break;
+#pragma unroll
+        for (int b = 0; b < HALVES; ++b) z[b] = __builtin_fmaf(w2[j][b], th[j0 + j], z[b]);
+    }
+#pragma unroll 8
+    for (int j = j0 + AHEAD; j < j1; ++j) {
+#pragma unroll
+        for (int b = 0; b < HALVES; ++b) z[b] = __builtin_fmaf(second(j, b), th[j], z[b]);
+    }
+#pragma unroll
+    for (int b = 0; b < HALVES; ++b) part[wave][b][lane] = z[b];
+    lds_barrier();
+    if (threadIdx.x < DK) {
+        const int i = threadIdx.x, b = i / WAVE, l = i % WAVE, at = single_at<DK>(i);
+        const float sum = (part[0][b][l] + part[1][b][l]) + (part[2][b][l] + part[3][b][l]);
+        const float u = mine[3] * inv;
+        vec[0][at] = expf(-DECAY_SCALE * sigmoidf_(mine[0] + sum));
+        vec[1][at] = sigmoidf_(mine[1] + mine[2]) * u;
+        vec[2][at] = u;
+        vec[3][at] = mine[3];
+        vec[4][at] = mine[4];
+    }
+    lds_barrier();
+    const float *W = vec[0] + g * C::SLP, *AU = W + C::VEC, *U = W + 2 * C::VEC, *K = W + 3 * C::VEC, *R = W + 4 * C::VEC;
+    for (;;) {
+        const bool live = col < dv;
+        const f32x4_t us = c.times(U);
+#pragma unroll
+        for (int i = 0; i < SL; ++i) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c.S[i][e] = W[i] * c.S[i][e] - AU[i] * us[e] + K[i] * v[e];
+        }
+        const f32x4_t o = c.times(R);
+        if (live) {
+            c.store(m, g, col, dv);
+            if (g == 0) *(f32x4_t *)(os + col) = o;
+        }
+        col += 128;
+        if (col - lane % 8 * 4 >= dv) break;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = to_f32(row[off_v + h * dv + min(col, dv - 4) + e]);
+        c.load(m, g, min(col, dv - 4), dv, fresh);
+    }
+    lds_barrier();
+    ss = 0.f;
+    for (int j = lane; j < dv; j += 64) ss += os[j] * os[j];
+    const float f = rsqrtf(wave_sum(ss) / (float)dv + eps);
+    for (int j = threadIdx.x; j < dv; j += 256) {
+        const int ch = h * dv + j;
+        const bool first = j == (int)threadIdx.x;
+        const float gate = sigmoidf_(first ? out_g : to_f32(row[off_g + ch]));
+        out[(size_t)r * heads * dv + ch] = from_f32<T>(os[j] * f * (first ? out_w : weight[ch]) * gate);
+    }
+}
+
+// Sizes for which the kernels for one token a request are there: whole groups of key channels, four columns an access.
+static bool single_sizes(int heads, int dk, int dv) {
+    return heads > 0 && heads <= 65535 && (dk == 32 || dk == 64 || dk == 96 || dk == 128) && dv > 0 && dv % 4 == 0 && dv <= SINGLE_MAX_DV;
+}
+LCU_API int lcu_delta_single_takes(int heads, int dk, int dv) { return single_sizes(heads, dk, dv); }
+
+// lcu_delta_rule for a step in which every request feeds one token (row r is request r's), where lcu_delta_single_takes says so; state 16-byte aligned.
+LCU_API int lcu_delta_single(const void *proj, int type, int row_stride, int off_r, int off_k, int off_v, int off_g, int off_a, int off_l,
+                             const float *w2, const float *w0, const float *a_bias, const float *weight, float *state, void *out, const int *ctx_len,
+                             const int *state_slot, int n_req, int heads, int dk, int dv, int rank, float eps, hipStream_t stream) {
+    if (n_req <= 0) return LCU_OK;
+    if (rank <= 0 || rank > MAX_RANK || (type != LCU_F32 && type != LCU_BF16) || (uintptr_t)state % 16) return LCU_BAD_ARGUMENT;
+    if (!single_sizes(heads, dk, dv)) return LCU_UNSUPPORTED;
+#define GO(T, DK) delta_single_kernel<T, DK><<<dim3(n_req, heads), dim3(256), 0, stream>>>((const T *)proj, row_stride, off_r, off_k, off_v, off_g, off_a, off_l, w2, w0, a_bias, weight, state, (T *)out, ctx_len, state_slot, heads, dv, rank, eps)
+#define SIZES(T) do { if (dk == 32) GO(T, 32); else if (dk == 64) GO(T, 64); else if (dk == 96) GO(T, 96); else GO(T, 128); } while (0)
+    if (type == LCU_F32) SIZES(float);
+    else SIZES(bf16_t);
+#undef SIZES
+#undef GO
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
+}
+
 // ---------------------------------------------------------------- the gated delta rule
 // One decay and one rate per head and token:  S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q,  with q and k
 // unit vectors per head (q also times dk^-1/2).  Written out, S <- g S - (beta g k)(k^T S) + k (beta v)^T with S as the
@@ -437,6 +610,171 @@ LCU_API int lcu_gated_delta_rule(const float *qkv, const float *rows, int row_st
         gated_delta_out_kernel<float><<<dim3(n, heads), dim3(64), 0, stream>>>(o, rows, row_stride, off_g, weight, (float *)out, heads, dv, eps);
     else
         gated_delta_out_kernel<bf16_t><<<dim3(n, heads), dim3(64), 0, stream>>>(o, rows, row_stride, off_g, weight, (bf16_t *)out, heads, dv, eps);
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
+}
+
+// One token a request, in two kernels: the convolution and the vectors, then the recurrence and the output.  (One kernel for both would have a workgroup
+// per query/key head, whose channels several value heads read and one must move on: four of them for a request with four such heads.)
+// The convolution of causal_conv.hip (taps oldest first, silu behind it) and gated_delta_prep_kernel: a workgroup per (request, query/key head).
+constexpr int SINGLE_MAX_TAPS = 8, SINGLE_MAX_GROUP = 64;
+__global__ void __launch_bounds__(1024)
+gated_delta_single_prep_kernel(const float *__restrict__ rows, int row_stride, int off_a, int off_b, const float *__restrict__ conv_w, int taps,
+                               float *__restrict__ inputs, size_t slot_stride, const float *__restrict__ a_log, const float *__restrict__ dt_bias,
+                               float *__restrict__ prep, float *__restrict__ vb, const int *__restrict__ ctx_len, const int *__restrict__ state_slot,
+                               int heads, int qk_heads, int dk, int dv) {
+    __shared__ float q[128], k[128], numbers[SINGLE_MAX_GROUP][4];
+    const int r = blockIdx.x, qh = blockIdx.y, threads = blockDim.x, lane = threadIdx.x & 63, group = heads / qk_heads;
+    const int channels = 2 * qk_heads * dk + heads * dv;
+    const bool fresh = ctx_len[r] == 1;
+    const float *row = rows + (size_t)r * row_stride;
+    float *st = inputs + (size_t)state_slot[r] * slot_stride;
+    float beta = 0.f, a = 0.f, al = 0.f, db = 0.f;
+    if ((int)threadIdx.x < group) {
+        const int h = qh * group + threadIdx.x;
+        beta = row[off_b + h];
+        a = row[off_a + h];
+        al = a_log[h];
+        db = dt_bias[h];
+    }
+    for (int x = threadIdx.x; x < 2 * dk + group * dv; x += threads) {
+        const int c = x < dk ? qh * dk + x : x < 2 * dk ? (qk_heads + qh) * dk + x - dk : 2 * qk_heads * dk + qh * group * dv + x - 2 * dk;
+        const float cur = row[c], last = conv_w[(size_t)c * taps + taps - 1], rate = x < 2 * dk ? 0.f : row[off_b + qh * group + (x - 2 * dk) / dv];
+        float v[SINGLE_MAX_TAPS - 1], w[SINGLE_MAX_TAPS - 1];
+#pragma unroll
+        for (int i = 0; i < SINGLE_MAX_TAPS - 1; ++i) {      // (all loads before the first store)
+            const bool in = i < taps - 1;
+            v[i] = in && !fresh ? st[(size_t)i * channels + c] : 0.f;
+            w[i] = in ? conv_w[(size_t)c * taps + i] : 0.f;
+        }
+        float acc = 0.f;
+#pragma unroll
+        for (int i = 0; i < SINGLE_MAX_TAPS - 1; ++i)
+            if (i < taps - 1) acc = __builtin_fmaf(w[i], v[i], acc);
+        acc = __builtin_fmaf(last, cur, acc);
+#pragma unroll
+        for (int i = 0; i < SINGLE_MAX_TAPS - 1; ++i)
+            if (i > 0 && i < taps - 1) st[(size_t)(i - 1) * channels + c] = v[i];
+        if (taps > 1) st[(size_t)(taps - 2) * channels + c] = cur;
+        const float y = acc / (1.0f + expf(-acc));
+        if (x < dk) q[x] = y;
+        else if (x < 2 * dk) k[x - dk] = y;
+        else {
+            const int h = qh * group + (x - 2 * dk) / dv, j = (x - 2 * dk) % dv;
+            vb[((size_t)r * heads + h) * dv + j] = sigmoidf_(rate) * y;
+        }
+    }
+    if ((int)threadIdx.x < group) {
+        const float lg = -expf(al) * softplus_(a + db), gd = expf(lg);
+        float *to = numbers[threadIdx.x];
+        to[0] = gd;
+        to[1] = sigmoidf_(beta) * gd;
+        to[2] = lg;
+        to[3] = 0.f;
+    }
+    lds_barrier();
+    float sq = 0.f, sk = 0.f;
+    for (int i = lane; i < dk; i += 64) {
+        sq = __builtin_fmaf(q[i], q[i], sq);
+        sk = __builtin_fmaf(k[i], k[i], sk);
+    }
+    sq = wave_sum_in_place(sq);
+    sk = wave_sum_in_place(sk);
+    const float qf = 1.0f / sqrtf(sq + 1e-6f) / sqrtf((float)dk), kf = 1.0f / sqrtf(sk + 1e-6f);
+    const int per = 2 * dk + 4;
+    for (int x = threadIdx.x; x < group * per; x += threads) {
+        const int i = x % per;
+        prep[((size_t)r * heads + qh * group) * per + x] = i < dk ? k[i] * kf : i < 2 * dk ? q[i - dk] * qf : numbers[x / per][i - 2 * dk];
+    }
+}
+
+// The recurrence and gated_delta_out_kernel: a workgroup per (request, value head).
+template <class T, int DK>
+__global__ void __launch_bounds__(256)
+gated_delta_single_kernel(const float *__restrict__ prep, const float *__restrict__ vb, const float *__restrict__ rows, int row_stride, int off_g,
+                          const float *__restrict__ weight, float *__restrict__ state, size_t slot_stride, T *__restrict__ out,
+                          const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int heads, int dv, float eps) {
+    typedef SingleColumns<DK> C;
+    constexpr int SL = C::SL;
+    __shared__ __attribute__((aligned(16))) float os[SINGLE_MAX_DV];
+    const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane / 8;
+    const bool fresh = ctx_len[r] == 1;
+    const size_t item = (size_t)r * heads + h;
+    float *m = state + (size_t)state_slot[r] * slot_stride + (size_t)h * DK * dv;
+    const float *p = prep + item * (2 * DK + 4);
+    C c;
+    int col = 32 * wave + lane % 8 * 4;
+    c.load(m, g, min(col, dv - 4), dv, fresh);
+    float U[SL], R[SL];
+#pragma unroll
+    for (int i = 0; i < SL; i += 4) {
+        *(f32x4_t *)(U + i) = *(const f32x4_t *)(p + g * SL + i);
+        *(f32x4_t *)(R + i) = *(const f32x4_t *)(p + DK + g * SL + i);
+    }
+    const float gd = p[2 * DK], bg = p[2 * DK + 1];
+    f32x4_t v = *(const f32x4_t *)(vb + item * dv + min(col, dv - 4));
+    float out_w = 0.f, out_g = 0.f;
+    if ((int)threadIdx.x < dv) {
+        out_w = weight[threadIdx.x];
+        out_g = rows[(size_t)r * row_stride + off_g + h * dv + threadIdx.x];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    for (;;) {
+        const bool live = col < dv;
+        const f32x4_t us = c.times(U);
+        f32x4_t e4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) e4[e] = v[e] - bg * us[e];
+#pragma unroll
+        for (int i = 0; i < SL; ++i) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c.S[i][e] = __builtin_fmaf(gd, c.S[i][e], U[i] * e4[e]);
+        }
+        const f32x4_t o = c.times(R);
+        if (live) {
+            c.store(m, g, col, dv);
+            if (g == 0) *(f32x4_t *)(os + col) = o;
+        }
+        col += 128;
+        if (col - lane % 8 * 4 >= dv) break;
+        v = *(const f32x4_t *)(vb + item * dv + min(col, dv - 4));
+        c.load(m, g, min(col, dv - 4), dv, fresh);
+    }
+    lds_barrier();
+    float ss = 0.f;
+    for (int j = lane; j < dv; j += 64) ss += os[j] * os[j];
+    const float f = 1.0f / sqrtf(wave_sum(ss) / (float)dv + eps);
+    for (int j = threadIdx.x; j < dv; j += 256) {
+        const bool first = j == (int)threadIdx.x;
+        const float z = first ? out_g : rows[(size_t)r * row_stride + off_g + h * dv + j];
+        out[item * dv + j] = from_f32<T>(os[j] * f * (first ? out_w : weight[j]) * (z / (1.0f + expf(-z))));
+    }
+}
+
+LCU_API int lcu_gated_delta_single_takes(int heads, int qk_heads, int dk, int dv, int taps, long long slot_stride) {
+    return single_sizes(heads, dk, dv) && qk_heads > 0 && heads % qk_heads == 0 && heads / qk_heads <= SINGLE_MAX_GROUP && taps >= 1 && taps <= SINGLE_MAX_TAPS && slot_stride % 4 == 0;
+}
+
+// lcu_causal_conv (silu, no bias, over the rows' first 2 * qk_heads * dk + heads * dv columns) and lcu_gated_delta_rule for a step in which every request
+// feeds one token, where lcu_gated_delta_single_takes says so.  inputs: the convolution's [taps - 1, channels] of slot 0; both states' slots lie
+// slot_stride apart, the matrices 16-byte aligned.  prep, vb: as above.
+LCU_API int lcu_gated_delta_single(const float *rows, int row_stride, int off_a, int off_b, int off_g, const float *conv_w, int taps, float *inputs,
+                                   const float *a_log, const float *dt_bias, const float *weight, float *prep, float *vb, float *state,
+                                   long long slot_stride, void *out, int out_type, const int *ctx_len, const int *state_slot, int n_req, int heads,
+                                   int qk_heads, int dk, int dv, float eps, hipStream_t stream) {
+    if (n_req <= 0) return LCU_OK;
+    if ((out_type != LCU_F32 && out_type != LCU_BF16) || ((uintptr_t)state | (uintptr_t)prep | (uintptr_t)vb) % 16 || (taps > 1 && !inputs)) return LCU_BAD_ARGUMENT;
+    if (!lcu_gated_delta_single_takes(heads, qk_heads, dk, dv, taps, slot_stride)) return LCU_UNSUPPORTED;
+    const int wide = 2 * dk + heads / qk_heads * dv;          // a thread a channel, if there are so many
+    gated_delta_single_prep_kernel<<<dim3(n_req, qk_heads), dim3(wide >= 1024 ? 1024 : (wide + 63) / 64 * 64), 0, stream>>>(rows, row_stride, off_a, off_b, conv_w, taps, inputs, (size_t)slot_stride, a_log,
+                                                                                   dt_bias, prep, vb, ctx_len, state_slot, heads, qk_heads, dk, dv);
+    LCU_LAUNCH_CHECK();
+#define GO(T, DK) gated_delta_single_kernel<T, DK><<<dim3(n_req, heads), dim3(256), 0, stream>>>(prep, vb, rows, row_stride, off_g, weight, state, (size_t)slot_stride, (T *)out, ctx_len, state_slot, heads, dv, eps)
+#define SIZES(T) do { if (dk == 32) GO(T, 32); else if (dk == 64) GO(T, 64); else if (dk == 96) GO(T, 96); else GO(T, 128); } while (0)
+    if (out_type == LCU_F32) SIZES(float);
+    else SIZES(bf16_t);
+#undef SIZES
+#undef GO
     LCU_LAUNCH_CHECK();
     return LCU_OK;
 }

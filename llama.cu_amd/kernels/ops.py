@@ -1466,9 +1466,14 @@ def delta_rule(proj: torch.Tensor, offsets: Dict[str, int], w2_t: torch.Tensor, 
         out = torch.empty((n, hv), dtype=proj.dtype, device=proj.device)
     if out.shape != (n, hv) or out.dtype != proj.dtype or not out.is_contiguous():
         raise KernelError("delta_rule out: wrong shape, type or layout")
+    lib = build.load("delta_rule")
+    if step.decode_only and n == step.n_req and state.data_ptr() % 16 == 0 and lib.lcu_delta_single_takes(heads, key_dim, value_dim):
+        _check(lib.lcu_delta_single(_ptr(proj), _type(proj, "delta projections"), proj.stride(0), offsets["r"], offsets["k"], offsets["v"],
+                                    offsets["g"], offsets["a"], offsets["l"], _ptr(w2_t), _ptr(w0), _ptr(a_bias), _ptr(weight), _ptr(state), _ptr(out),
+                                    _ptr(step.ctx_len), _ptr(step.state_slot), n, heads, key_dim, value_dim, rank, ctypes.c_float(eps), _stream()), "delta_single")
+        return out
     prep = torch.empty((n, heads, 5, key_dim), dtype=torch.float32, device=proj.device)
     o = torch.empty((n, hv), dtype=torch.float32, device=proj.device)
-    lib = build.load("delta_rule")
     work = _delta_work(lib, step, heads, key_dim, value_dim, False, out)
     _check(lib.lcu_delta_rule(_ptr(proj), _type(proj, "delta projections"), proj.stride(0), offsets["r"], offsets["k"], offsets["v"],
                               offsets["g"], offsets["a"], offsets["l"], _ptr(w2_t), _ptr(w0), _ptr(a_bias), _ptr(weight), _ptr(prep),
@@ -2240,6 +2245,43 @@ def gated_delta_rule(qkv: torch.Tensor, rows: torch.Tensor, off_a: int, off_b: i
                                     _ptr(weight), _ptr(prep), _ptr(vb), _ptr(work), _ptr(o), _ptr(state), ctypes.c_longlong(slot_stride), _ptr(out),
                                     _type(out, "gated delta out"), _ptr(step.q_start), _ptr(step.ctx_len), _ptr(step.state_slot), n,
                                     step.n_req, heads, qk_heads, key_dim, value_dim, ctypes.c_float(eps), _stream()), "gated_delta_rule")
+    return out
+
+
+def gated_delta_single_takes(step, state: torch.Tensor, heads: int, qk_heads: int, key_dim: int, value_dim: int, taps: int) -> bool:
+    """Whether ``gated_delta_single`` runs this step: every request feeds one token, and the sizes are its kernels'."""
+    return bool(step.decode_only and step.n == step.n_req and state.data_ptr() % 16 == 0 and build.load("delta_rule").lcu_gated_delta_single_takes(
+        heads, qk_heads, key_dim, value_dim, taps, ctypes.c_longlong(state.stride(0))))
+
+
+def gated_delta_single(rows: torch.Tensor, off_a: int, off_b: int, off_g: int, conv_w: torch.Tensor, inputs: Optional[torch.Tensor], a_log: torch.Tensor,
+                       dt_bias: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, step, heads: int, qk_heads: int, key_dim: int, value_dim: int,
+                       eps: float, out_dtype: torch.dtype) -> torch.Tensor:
+    """``causal_conv`` (silu, over the rows' first columns: q, k, v; its state ``inputs``) and ``gated_delta_rule`` behind it, for a step in which every
+    request feeds one token (``gated_delta_single_takes``)."""
+    _gpu(rows, conv_w, inputs, a_log, dt_bias, weight, state)
+    _rows(rows, "gated delta rows")
+    n, hv = rows.shape[0], heads * value_dim
+    channels, taps = 2 * qk_heads * key_dim + hv, conv_w.shape[1]
+    if rows.dtype != torch.float32 or rows.stride(1) != 1 or n != step.n:
+        raise KernelError("gated_delta_single: the rows must be the step's, float32 [n, *] with contiguous columns")
+    if conv_w.shape[0] != channels or conv_w.dtype != torch.float32 or not conv_w.is_contiguous():
+        raise KernelError(f"gated_delta_single: the convolution's weight must be contiguous float32 [{channels}, taps]")
+    for name, off, width in (("q, k, v", 0, channels), ("a", off_a, heads), ("b", off_b, heads), ("g", off_g, hv)):
+        if off < 0 or off + width > rows.shape[1]:
+            raise KernelError(f"gated_delta_single: the columns of {name!r} lie outside the rows' {rows.shape[1]} columns")
+    _f32_vec(a_log, "gated delta A_log", heads); _f32_vec(dt_bias, "gated delta dt_bias", heads)
+    _f32_vec(weight, "gated delta norm weight", value_dim)
+    slot_stride = _slot_state(state, (heads, key_dim, value_dim), "gated_delta_single", step)
+    if taps > 1 and (inputs is None or _slot_state(inputs, (taps - 1, channels), "gated_delta_single", step) != slot_stride and state.shape[0] > 1):
+        raise KernelError("gated_delta_single: the convolution's inputs must lie in the matrices' slots")
+    prep = torch.empty((n, heads, 2 * key_dim + 4), dtype=torch.float32, device=rows.device)
+    vb = torch.empty((n, hv), dtype=torch.float32, device=rows.device)
+    out = torch.empty((n, hv), dtype=out_dtype, device=rows.device)
+    _check(build.load("delta_rule").lcu_gated_delta_single(
+        _ptr(rows), rows.stride(0), int(off_a), int(off_b), int(off_g), _ptr(conv_w), taps, _ptr(inputs if taps > 1 else None), _ptr(a_log), _ptr(dt_bias), _ptr(weight),
+        _ptr(prep), _ptr(vb), _ptr(state), ctypes.c_longlong(slot_stride), _ptr(out), _type(out, "gated delta out"), _ptr(step.ctx_len), _ptr(step.state_slot), n,
+        heads, qk_heads, key_dim, value_dim, ctypes.c_float(eps), _stream()), "gated_delta_single")
     return out
 
 

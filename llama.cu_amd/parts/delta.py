@@ -166,6 +166,10 @@ class GatedDelta(Part):
         matrices = state[:, :self.state_size].view(slots, self.heads, self.head_dim, self.value_dim)
         inputs = state[:, self.state_size:].view(slots, self.taps - 1, self.channels) if self.taps > 1 else None
         rows = linear(h, self.w_in, out_dtype=torch.float32)
+        if ops.gated_delta_single_takes(step, matrices, self.heads, self.qk_heads, self.head_dim, self.value_dim, self.taps):
+            y = ops.gated_delta_single(rows, self.off_a, self.off_b, self.off_g, self.conv_w, inputs, self.a_log, self.dt_bias, self.norm, matrices, step,
+                                       self.heads, self.qk_heads, self.head_dim, self.value_dim, self.norm_eps, self.dtype)
+            return linear(y, self.w_o, out_dtype=out_dtype or self.dtype)
         qkv = ops.causal_conv(rows, 0, self.conv_w, None, inputs, step, torch.float32, activation="silu")
         y = ops.gated_delta_rule(qkv, rows, self.off_a, self.off_b, self.off_g, self.a_log, self.dt_bias, self.norm, matrices,
                                  step, self.heads, self.qk_heads, self.head_dim, self.value_dim, self.norm_eps, self.dtype)

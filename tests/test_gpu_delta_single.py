@@ -1,0 +1,69 @@
+"""Delta rules in steps in which every request feeds one token (kernels of their own) against the same tokens beside a request that feeds two, which go
+through the scan: the same bits, outputs and states."""
+import pytest
+import torch
+
+from test_gpu_divasun import TYPES, hand_step, rnd
+from test_gpu_mufotar import built
+
+pytestmark = pytest.mark.gpu
+
+REQUESTS = 5
+
+
+def steps(slots_of):
+    """Three tokens of every request in steps of single tokens, then the same with a last request that feeds two a step: ``(q_lens, ctx, slots)``."""
+    for k in range(3):
+        ctx = [1 + k + 3 * (r % 2) for r in range(REQUESTS)]            # (some requests' first token, some with tokens before it)
+        yield ([1] * REQUESTS, ctx, slots_of[:REQUESTS]), ([1] * REQUESTS + [2], ctx + [2 * k + 2], slots_of)
+
+
+# every size of key channels; columns in whole sets of 128, with a rest of less than a wave's 32, fewer than a wave's, the most there are
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,dk,dv,rank", [(2, 128, 128, 64), (3, 32, 132, 3), (1, 64, 4, 1), (2, 96, 300, 9), (1, 128, 512, 33)])
+def test_the_generalised_rule(dtype, heads, dk, dv, rank):
+    from llama_cu_amd.kernels import build, ops
+    assert build.load("delta_rule").lcu_delta_single_takes(heads, dk, dv) and not build.load("delta_rule").lcu_delta_single_takes(heads, dk + 16, dv)
+    hk, hv, tdt = heads * dk, heads * dv, TYPES[dtype]
+    off = {"r": 0, "k": hk, "v": 2 * hk, "g": 2 * hk + hv, "a": 2 * hk + 2 * hv, "l": 3 * hk + 2 * hv}
+    args = (rnd(rank, hk, seed=3).cuda(), rnd(hk, seed=4).cuda(), rnd(hk, seed=5).cuda(), (rnd(hv, seed=6) + 1).cuda())
+    a = rnd(REQUESTS + 1, heads, dk, dv, seed=7).cuda()
+    b = a.clone()
+    for k, (one, two) in enumerate(steps([3, 0, 5, 1, 4, 2])):
+        rows = rnd(REQUESTS + 2, 3 * hk + 2 * hv + rank, seed=10 + k).to(tdt).cuda()
+        got = ops.delta_rule(rows[:REQUESTS].contiguous(), off, *args, a, hand_step(*one), heads, dk, dv, 1e-4)
+        want = ops.delta_rule(rows, off, *args, b, hand_step(*two), heads, dk, dv, 1e-4)
+        assert torch.equal(got, want[:REQUESTS]) and torch.equal(a[[3, 0, 5, 1, 4]], b[[3, 0, 5, 1, 4]]), k
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,qk_heads,dk,dv,taps", [(4, 2, 128, 128, 4), (3, 3, 32, 132, 1), (2, 1, 64, 4, 2), (4, 1, 96, 300, 8), (1, 1, 128, 512, 3)])
+def test_the_gated_rule(dtype, heads, qk_heads, dk, dv, taps):
+    from llama_cu_amd.kernels import ops
+    d, tdt = 56, TYPES[dtype]
+    shape = {"hidden_size": d, "heads": heads, "qk_heads": qk_heads, "head_dim": dk, "value_dim": dv, "taps": taps, "norm_eps": 1e-5}
+    from llama_cu_amd.parts import PartSpec, make_part
+    names = make_part("mixer", PartSpec("gated_delta", shape)).tensors()
+    part = built("mixer", "gated_delta", shape, {n: rnd(*t.shape, seed=k, std=t.shape[-1] ** -0.5 if len(t.shape) > 1 else 1.0) for k, (n, t) in enumerate(names.items())}, tdt)
+    a, b = (part.cache_need().allocate(-1, 0, 0, REQUESTS + 1, tdt, torch.device("cuda")) for _ in range(2))
+    a.state.copy_(rnd(*a.state.shape, seed=99))
+    b.state.copy_(a.state)
+    matrices = a.state[:, :part.state_size].view(-1, heads, dk, dv)
+    for k, (one, two) in enumerate(steps([3, 0, 5, 1, 4, 2])):
+        rows = rnd(REQUESTS + 2, d, seed=10 + k).to(tdt).cuda()
+        assert ops.gated_delta_single_takes(hand_step(*one), matrices, heads, qk_heads, dk, dv, taps) == (a.state.stride(0) % 4 == 0)
+        got = part.forward(rows[:REQUESTS].contiguous(), hand_step(*one), a)
+        want = part.forward(rows, hand_step(*two), b)
+        assert torch.equal(got, want[:REQUESTS]) and torch.equal(a.state[[3, 0, 5, 1, 4]], b.state[[3, 0, 5, 1, 4]]), k
+
+
+def test_a_state_of_one_slot():
+    shape = {"hidden_size": 24, "heads": 2, "qk_heads": 1, "head_dim": 32, "value_dim": 8, "taps": 3, "norm_eps": 1e-5}
+    from llama_cu_amd.parts import PartSpec, make_part
+    names = make_part("mixer", PartSpec("gated_delta", shape)).tensors()
+    part = built("mixer", "gated_delta", shape, {n: rnd(*t.shape, seed=k) for k, (n, t) in enumerate(names.items())}, torch.float32)
+    a, b = (part.cache_need().allocate(-1, 0, 0, n, torch.float32, torch.device("cuda")) for n in (1, 2))
+    rows = rnd(4, 24, seed=9).cuda()
+    want = part.forward(rows, hand_step([4], [4], [1]), b)
+    got = torch.cat([part.forward(rows[k:k + 1].contiguous(), hand_step([1], [k + 1], [0]), a) for k in range(4)])
+    assert torch.equal(got, want) and torch.equal(a.state[0], b.state[1])
