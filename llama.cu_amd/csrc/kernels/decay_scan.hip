@@ -545,8 +545,23 @@ struct DsSingle {
     int silu;
 };
 
-template <class TI, class T, int V>
-__global__ void __launch_bounds__(256)
+// The sum over the block with barriers that leave loads on their way (block_sum's order).
+__device__ __forceinline__ float block_sum_lds(float v, float *scratch) {
+    v = wave_sum(v);
+    lds_barrier();
+    if ((threadIdx.x & (WAVE - 1)) == 0) scratch[threadIdx.x / WAVE] = v;
+    lds_barrier();
+    float t = 0.f;
+    for (int i = 0; i < (int)blockDim.x / WAVE; ++i) t += scratch[i];
+    return t;
+}
+
+// What bounds it is the state, read and written once; all that a workgroup needs beside it is asked for first and the state's first pieces behind that, so that
+// nothing waits for memory twice (the state after the rows, the gate and the weight where they are used: 64 requests, 16 heads of 128 x 128 36.3 us, 8 heads
+// gated 23.0; now 34.2 and 19.4 inside a step, and 29 where the state is streamed, 4.6 TB/s).
+// STREAM: the state's loads and stores are non-temporal.
+template <class TI, class T, int V, bool STREAM>
+__global__ void __launch_bounds__(256, 4)
 ds_single_kernel(DsSingle p) {
     constexpr int KEEP = 16;                      // pieces of the state a thread loads at a time
     __shared__ float qk[2][256];
@@ -560,41 +575,68 @@ ds_single_kernel(DsSingle p) {
     const int groups = (dv + V - 1) / V;          // of V columns
     const int cols = min(groups, 256), nrows = 256 / cols, my_row = tid / cols, my_col = tid % cols;
     const bool works = my_row < nrows;
-    float a, b, m_now = 0.f;
+    const int qc = min(tid, d - 1), vc = min(tid, dv - 1);
+    float *N = slot + p.n_off + (size_t)h * d + qc;
+    const TI q_in = row[p.q_off + h * d + qc], k_in = row[p.k_off + h * d + qc], v_in = row[p.v_off + h * dv + vc], g_in = row[p.g_off + h * dv + vc];
+    const float w_in = p.weight[h * dv + vc];
+    float a, b = 1.f, m = 0.f, n_in = 0.f, zi = 0.f, zf = 0.f, bi = 0.f, bf = 0.f;
     if (p.decay) {
         a = p.decay[h];
-        b = 1.f;
     } else {
-        const float m = fresh ? 0.f : slot[p.m_off + h];
-        const float gi = p.cap * tanhf((p.z[(size_t)t * p.ldz + h] + p.bias_i[h]) / p.cap);
-        const float f = log_sigmoid_f(p.cap * tanhf((p.z[(size_t)t * p.ldz + p.heads + h] + p.bias_f[h]) / p.cap));
+        if (!fresh) { m = slot[p.m_off + h]; n_in = *N; }
+        zi = p.z[(size_t)t * p.ldz + h];
+        zf = p.z[(size_t)t * p.ldz + p.heads + h];
+        bi = p.bias_i[h];
+        bf = p.bias_f[h];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    DsVec<float, V> s[KEEP];
+    auto load_state = [&](int i0, int c) {
+#pragma unroll
+        for (int x = 0; x < KEEP; ++x) {
+            if (fresh) {
+#pragma unroll
+                for (int e = 0; e < V; ++e) s[x].v[e] = 0.f;
+            } else {
+                const float *from = S + (size_t)min(i0 + x * nrows, d - 1) * dv + c;
+                if constexpr (STREAM) s[x] = __builtin_bit_cast(DsVec<float, V>, __builtin_nontemporal_load((const f32x4 *)from));
+                else s[x] = *(const DsVec<float, V> *)from;
+            }
+        }
+    };
+    load_state(min(my_row, d - 1), min(my_col, groups - 1) * V);
+    __builtin_amdgcn_sched_barrier(0);
+    float m_now = 0.f;
+    if (!p.decay) {
+        const float gi = p.cap * tanhf((zi + bi) / p.cap);
+        const float f = log_sigmoid_f(p.cap * tanhf((zf + bf) / p.cap));
         m_now = fmaxf(f + m, gi);
         a = expf(f + m - m_now);
         b = expf(gi - m_now);
     }
     if (fresh) a = 0.f;                           // the state is zero: what the slot held is not used (it is not read either)
+    asm volatile("" ::"v"(a), "v"(b));            // (every thread has read m before the barrier)
     for (int c = tid; c < d; c += 256) {
-        float q = to_f32(row[p.q_off + h * d + c]), k = to_f32(row[p.k_off + h * d + c]);
+        float q = to_f32(c == tid ? q_in : row[p.q_off + h * d + c]), k = to_f32(c == tid ? k_in : row[p.k_off + h * d + c]);
         if (p.silu) { q = silu_for<T>(q); k = silu_for<T>(k); }
         qk[0][c] = to_f32(from_f32<T>(q));
         qk[1][c] = to_f32(from_f32<T>(k));
     }
     for (int c = tid; c < dv; c += 256) {
-        float v = to_f32(row[p.v_off + h * dv + c]);
+        float v = to_f32(c == tid ? v_in : row[p.v_off + h * dv + c]);
         if (p.silu) v = silu_for<T>(v);
         vs[c] = to_f32(from_f32<T>(v));
     }
-    __syncthreads();                              // (every thread has read m)
+    lds_barrier();
     float inv = 1.f;
     if (!p.decay) {
         float den = 0.f;
         if (tid < d) {
-            float *N = slot + p.n_off + (size_t)h * d + tid;
-            const float n_new = fmaf(b, qk[1][tid], fresh ? 0.f : a * *N);
+            const float n_new = fmaf(b, qk[1][tid], fresh ? 0.f : a * n_in);
             *N = n_new;
             den = n_new * qk[0][tid];
         }
-        den = p.scale * block_sum(den, scratch);
+        den = p.scale * block_sum_lds(den, scratch);
         inv = 1.0f / (fmaxf(fabsf(den), expf(-m_now)) + 1e-6f);
         if (tid == 0) slot[p.m_off + h] = m_now;
     }
@@ -606,17 +648,7 @@ ds_single_kernel(DsSingle p) {
 #pragma unroll
         for (int e = 0; e < V; ++e) { acc[e] = 0.f; v[e] = on && c + e < dv ? b * vs[c + e] : 0.f; }
         for (int i0 = my_row; on && i0 < d; i0 += KEEP * nrows) {
-            DsVec<float, V> s[KEEP];
-#pragma unroll
-            for (int x = 0; x < KEEP; ++x) {
-                const int i = i0 + x * nrows;
-                if (fresh) {
-#pragma unroll
-                    for (int e = 0; e < V; ++e) s[x].v[e] = 0.f;
-                } else {
-                    s[x] = *(const DsVec<float, V> *)(S + (size_t)min(i, d - 1) * dv + c);
-                }
-            }
+            if (c0 || i0 != my_row) load_state(i0, c);
 #pragma unroll
             for (int x = 0; x < KEEP; ++x) {
                 const int i = i0 + x * nrows;
@@ -627,13 +659,14 @@ ds_single_kernel(DsSingle p) {
                     s[x].v[e] = fmaf(a, s[x].v[e], k * v[e]);
                     acc[e] = fmaf(q, s[x].v[e], acc[e]);
                 }
-                *(DsVec<float, V> *)(S + (size_t)i * dv + c) = s[x];
+                if constexpr (STREAM) __builtin_nontemporal_store(__builtin_bit_cast(f32x4, s[x]), (f32x4 *)(S + (size_t)i * dv + c));
+                else *(DsVec<float, V> *)(S + (size_t)i * dv + c) = s[x];
             }
         }
-        __syncthreads();                          // (red is free again)
+        lds_barrier();                            // (red is free again)
 #pragma unroll
         for (int e = 0; e < V; ++e) red[tid * V + e] = acc[e];
-        __syncthreads();
+        lds_barrier();
         for (int x = tid; x < cols * V; x += 256) {
             const int cc = c0 * V + x;
             if (cc >= dv) continue;
@@ -644,13 +677,13 @@ ds_single_kernel(DsSingle p) {
             sq += o * o;
         }
     }
-    const float total = block_sum(sq, scratch);   // (its barriers make vs visible)
+    const float total = block_sum_lds(sq, scratch);   // (its barriers make vs visible)
     const float f = p.factor * (p.decay ? 1.f : rsqrtf(total / (float)dv + p.eps));
     if (p.decay && tid == 0) p.sumsq[(size_t)t * p.heads + h] = total;
     T *out = (T *)p.out + (size_t)t * p.out_stride + h * dv;
     for (int c = tid; c < dv; c += 256) {
-        const float z = to_f32(row[p.g_off + h * dv + c]);
-        out[c] = from_f32<T>(vs[c] * f * p.weight[h * dv + c] * sigmoid_f(z));
+        const float z = to_f32(c == tid ? g_in : row[p.g_off + h * dv + c]);
+        out[c] = from_f32<T>(vs[c] * f * (c == tid ? w_in : p.weight[h * dv + c]) * sigmoid_f(z));
     }
 }
 
@@ -776,11 +809,15 @@ LCU_API int lcu_decay_scan_single(const void *rows, int type, int row_stride, in
     p.q_start = q_start; p.ctx_len = ctx_len; p.state_slot = state_slot;
     p.heads = heads; p.d = d; p.dv = dv; p.scale = scale; p.eps = eps; p.factor = factor; p.silu = silu;
     const bool wide = dv % 4 == 0 && slot_stride % 4 == 0 && (uintptr_t)state % 16 == 0;
+    // A state of this size is in no cache when its layer's turn comes again: past the caches it is a fifth faster (64 requests of 16 heads of 128 x 128,
+    // 67 MB: 34.9 us, 29.0 so; 128 of 8, gated: 38.3 and 30.9; but half of that, which a few layers leave in the last-level cache, 15.8 and 18.2)
+    const bool stream_past = wide && (long long)n_req * heads * d * dv * 4 >= (48ll << 20);
     const dim3 grid(n_req, heads), block(256);
-#define GO(TI, T)                                                                 \
-    do {                                                                          \
-        if (wide) ds_single_kernel<TI, T, 4><<<grid, block, 0, stream>>>(p);      \
-        else ds_single_kernel<TI, T, 1><<<grid, block, 0, stream>>>(p);           \
+#define GO(TI, T)                                                                       \
+    do {                                                                                \
+        if (stream_past) ds_single_kernel<TI, T, 4, true><<<grid, block, 0, stream>>>(p);  \
+        else if (wide) ds_single_kernel<TI, T, 4, false><<<grid, block, 0, stream>>>(p);   \
+        else ds_single_kernel<TI, T, 1, false><<<grid, block, 0, stream>>>(p);             \
     } while (0)
     if (type == LCU_F32 && out_type == LCU_F32) GO(float, float);
     else if (type == LCU_F32 && out_type == LCU_BF16) GO(float, bf16_t);

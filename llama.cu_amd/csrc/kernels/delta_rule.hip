@@ -362,16 +362,24 @@ LCU_API int lcu_delta_rule(const void *proj, int type, int row_stride, int off_r
 // Few requests wait for memory's latency, many for the matrices, read and written once.  16 heads of 128 x 128, rank 64, a chain of such steps: 1 request 9.1 ->
 // 6.3 us, 16 requests 23.9 -> 9.0, 200 requests 246 -> 68; the gated rule with its convolution and products 18.7 -> 15.5, 27.4 -> 19.9, 224 -> 91.  (Heads of 32
 // with a rank of 512, 200 requests: 59 and 61, each request reads the decay's second matrix.)
-template <int DK> struct SingleColumns {
+// STREAM: the state's loads and stores are non-temporal.
+template <int DK, bool STREAM = false> struct SingleColumns {
     static constexpr int SL = DK / 8, SLP = SL + 4, VEC = 8 * SLP;      // a vector in LDS: the groups' shares, four floats of padding behind each
     f32x4_t S[SL];
     __device__ __forceinline__ void load(const float *m, int g, int col, int dv, bool fresh) {
 #pragma unroll
-        for (int i = 0; i < SL; ++i) S[i] = fresh ? f32x4_t{0.f, 0.f, 0.f, 0.f} : *(const f32x4_t *)(m + (size_t)(g * SL + i) * dv + col);
+        for (int i = 0; i < SL; ++i) {
+            const f32x4_t *from = (const f32x4_t *)(m + (size_t)(g * SL + i) * dv + col);
+            S[i] = fresh ? f32x4_t{0.f, 0.f, 0.f, 0.f} : STREAM ? __builtin_nontemporal_load(from) : *from;
+        }
     }
     __device__ __forceinline__ void store(float *m, int g, int col, int dv) const {
 #pragma unroll
-        for (int i = 0; i < SL; ++i) *(f32x4_t *)(m + (size_t)(g * SL + i) * dv + col) = S[i];
+        for (int i = 0; i < SL; ++i) {
+            f32x4_t *to = (f32x4_t *)(m + (size_t)(g * SL + i) * dv + col);
+            if (STREAM) __builtin_nontemporal_store(S[i], to);
+            else *to = S[i];
+        }
     }
     // u^T S of the four columns: U, the unit key's share of the lane's group
     __device__ __forceinline__ f32x4_t times(const float *U) const {
@@ -393,13 +401,13 @@ template <int DK> __device__ __forceinline__ int single_at(int i) { return i / S
 constexpr int SINGLE_MAX_DV = 512;
 
 // The general rule from its projections to what the output matrix reads.  The arithmetic is that of delta_prep_kernel, delta_scan_kernel and delta_out_kernel.
-template <class T, int DK>
+template <class T, int DK, bool STREAM>
 __global__ void __launch_bounds__(256)
 delta_single_kernel(const T *__restrict__ proj, int row_stride, int off_r, int off_k, int off_v, int off_g, int off_a, int off_l,
                     const float *__restrict__ w2t, const float *__restrict__ w0, const float *__restrict__ a_bias, const float *__restrict__ weight,
                     float *__restrict__ state, T *__restrict__ out, const int *__restrict__ ctx_len, const int *__restrict__ state_slot,
                     int heads, int dv, int rank, float eps) {
-    typedef SingleColumns<DK> C;
+    typedef SingleColumns<DK, STREAM> C;
     constexpr int SL = C::SL, HALVES = (DK + WAVE - 1) / WAVE, AHEAD = 16;
     __shared__ __attribute__((aligned(16))) float th[MAX_RANK], vec[5][C::VEC], part[4][HALVES][WAVE], os[SINGLE_MAX_DV];
     const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane / 8;
@@ -506,6 +514,9 @@ delta_single_kernel(const T *__restrict__ proj, int row_stride, int off_r, int o
 static bool single_sizes(int heads, int dk, int dv) {
     return heads > 0 && heads <= 65535 && (dk == 32 || dk == 64 || dk == 96 || dk == 128) && dv > 0 && dv % 4 == 0 && dv <= SINGLE_MAX_DV;
 }
+// A step's states of this size are in no cache when their layer's turn comes again, and what they leave there would push out what is (64 requests of 16 heads of
+// 128 x 128 over eight layers, the decay scans' kernel: 34.9 us a layer, 29.0 past the caches; below, the last-level cache holds a few layers')
+static bool past_caches(int n_req, int heads, int dk, int dv) { return (long long)n_req * heads * dk * dv * 4 >= (48ll << 20); }
 LCU_API int lcu_delta_single_takes(int heads, int dk, int dv) { return single_sizes(heads, dk, dv); }
 
 // lcu_delta_rule for a step in which every request feeds one token (row r is request r's), where lcu_delta_single_takes says so; state 16-byte aligned.
@@ -515,7 +526,8 @@ LCU_API int lcu_delta_single(const void *proj, int type, int row_stride, int off
     if (n_req <= 0) return LCU_OK;
     if (rank <= 0 || rank > MAX_RANK || (type != LCU_F32 && type != LCU_BF16) || (uintptr_t)state % 16) return LCU_BAD_ARGUMENT;
     if (!single_sizes(heads, dk, dv)) return LCU_UNSUPPORTED;
-#define GO(T, DK) delta_single_kernel<T, DK><<<dim3(n_req, heads), dim3(256), 0, stream>>>((const T *)proj, row_stride, off_r, off_k, off_v, off_g, off_a, off_l, w2, w0, a_bias, weight, state, (T *)out, ctx_len, state_slot, heads, dv, rank, eps)
+    const bool past = past_caches(n_req, heads, dk, dv);
+#define GO(T, DK) (past ? delta_single_kernel<T, DK, true> : delta_single_kernel<T, DK, false>)<<<dim3(n_req, heads), dim3(256), 0, stream>>>((const T *)proj, row_stride, off_r, off_k, off_v, off_g, off_a, off_l, w2, w0, a_bias, weight, state, (T *)out, ctx_len, state_slot, heads, dv, rank, eps)
 #define SIZES(T) do { if (dk == 32) GO(T, 32); else if (dk == 64) GO(T, 64); else if (dk == 96) GO(T, 96); else GO(T, 128); } while (0)
     if (type == LCU_F32) SIZES(float);
     else SIZES(bf16_t);
@@ -689,12 +701,12 @@ gated_delta_single_prep_kernel(const float *__restrict__ rows, int row_stride, i
 }
 
 // The recurrence and gated_delta_out_kernel: a workgroup per (request, value head).
-template <class T, int DK>
+template <class T, int DK, bool STREAM>
 __global__ void __launch_bounds__(256)
 gated_delta_single_kernel(const float *__restrict__ prep, const float *__restrict__ vb, const float *__restrict__ rows, int row_stride, int off_g,
                           const float *__restrict__ weight, float *__restrict__ state, size_t slot_stride, T *__restrict__ out,
                           const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int heads, int dv, float eps) {
-    typedef SingleColumns<DK> C;
+    typedef SingleColumns<DK, STREAM> C;
     constexpr int SL = C::SL;
     __shared__ __attribute__((aligned(16))) float os[SINGLE_MAX_DV];
     const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane / 8;
@@ -769,7 +781,8 @@ LCU_API int lcu_gated_delta_single(const float *rows, int row_stride, int off_a,
     gated_delta_single_prep_kernel<<<dim3(n_req, qk_heads), dim3(wide >= 1024 ? 1024 : (wide + 63) / 64 * 64), 0, stream>>>(rows, row_stride, off_a, off_b, conv_w, taps, inputs, (size_t)slot_stride, a_log,
                                                                                    dt_bias, prep, vb, ctx_len, state_slot, heads, qk_heads, dk, dv);
     LCU_LAUNCH_CHECK();
-#define GO(T, DK) gated_delta_single_kernel<T, DK><<<dim3(n_req, heads), dim3(256), 0, stream>>>(prep, vb, rows, row_stride, off_g, weight, state, (size_t)slot_stride, (T *)out, ctx_len, state_slot, heads, dv, eps)
+    const bool past = past_caches(n_req, heads, dk, dv);
+#define GO(T, DK) (past ? gated_delta_single_kernel<T, DK, true> : gated_delta_single_kernel<T, DK, false>)<<<dim3(n_req, heads), dim3(256), 0, stream>>>(prep, vb, rows, row_stride, off_g, weight, state, (size_t)slot_stride, (T *)out, ctx_len, state_slot, heads, dv, eps)
 #define SIZES(T) do { if (dk == 32) GO(T, 32); else if (dk == 64) GO(T, 64); else if (dk == 96) GO(T, 96); else GO(T, 128); } while (0)
     if (out_type == LCU_F32) SIZES(float);
     else SIZES(bf16_t);

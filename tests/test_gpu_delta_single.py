@@ -67,3 +67,32 @@ def test_a_state_of_one_slot():
     want = part.forward(rows, hand_step([4], [4], [1]), b)
     got = torch.cat([part.forward(rows[k:k + 1].contiguous(), hand_step([1], [k + 1], [0]), a) for k in range(4)])
     assert torch.equal(got, want) and torch.equal(a.state[0], b.state[1])
+
+
+def test_states_that_no_cache_holds():
+    """A step whose states are streamed past the caches (48 MB and more) against its halves, whose are not: the same bits."""
+    from llama_cu_amd.kernels import ops
+    n, heads, dk, dv, rank = 25, 8, 128, 512, 5
+    hk, hv = heads * dk, heads * dv
+    off = {"r": 0, "k": hk, "v": 2 * hk, "g": 2 * hk + hv, "a": 2 * hk + 2 * hv, "l": 3 * hk + 2 * hv}
+    args = (rnd(rank, hk, seed=3).cuda(), rnd(hk, seed=4).cuda(), rnd(hk, seed=5).cuda(), (rnd(hv, seed=6) + 1).cuda())
+    gated = (rnd(heads, seed=13).cuda(), rnd(heads, seed=14).cuda(), rnd(dv, seed=15).cuda())
+    channels = 2 * hk + hv
+    conv_w = rnd(channels, 3, seed=16).cuda()
+    rows, wide = rnd(n, 3 * hk + 2 * hv + rank, seed=7).cuda(), rnd(n, channels + 2 * heads + hv, seed=8).cuda()
+    a = torch.randn(n, heads, dk, dv, generator=torch.Generator("cuda").manual_seed(9), device="cuda")
+    slots = torch.randn(n, heads * dk * dv + 2 * channels, generator=torch.Generator("cuda").manual_seed(10), device="cuda")
+
+    def run(first, last, state, both):
+        step = hand_step([1] * (last - first), [1 + r % 3 for r in range(first, last)], list(range(first, last)))
+        y = ops.delta_rule(rows[first:last].contiguous(), off, *args, state, step, heads, dk, dv, 1e-4)
+        m = heads * dk * dv
+        z = ops.gated_delta_single(wide[first:last].contiguous(), channels, channels + heads, channels + 2 * heads, conv_w, both[:, m:].view(n, 2, channels), *gated,
+                                   both[:, :m].view(n, heads, dk, dv), step, heads, heads, dk, dv, 1e-4, torch.bfloat16)
+        return y, z
+    b, both = a.clone(), slots.clone()
+    got = run(0, n, a, slots)
+    halves = [run(0, 12, b, both), run(12, n, b, both)]
+    for k in range(2):
+        assert torch.equal(got[k], torch.cat([h[k] for h in halves]))
+    assert torch.equal(a, b) and torch.equal(slots, both)

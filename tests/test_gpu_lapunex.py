@@ -290,6 +290,20 @@ def test_single_tokens_of_many_requests_and_rows_that_wait_for_their_norm():
                 assert_close(got[r], reference(f64(rows[r].float()))[-1], 3e-2, f"{count} requests, {r}")
 
 
+@pytest.mark.parametrize("kind", ["lightning", "memory"])
+def test_single_tokens_whose_states_no_cache_holds(kind):
+    """A step of single tokens whose states are streamed past the caches (48 MB and more) against its halves, whose are not: the same bits."""
+    d, heads, count = 64, 12, 17
+    part, _, _ = lightning_part([1.0 - 0.1 / (k + 1) for k in range(heads)], 256, 256, d, "float32") if kind == "lightning" else memory_part(heads, 256, 256, 9.0, d, "float32")
+    a, b = state_of(part, count), state_of(part, count)
+    a.state.copy_(torch.randn(a.state.shape, generator=torch.Generator("cuda").manual_seed(1), device="cuda"))
+    b.state.copy_(a.state)
+    rows, ctx = rnd(count, d, seed=2).cuda(), [1 + r % 3 for r in range(count)]
+    got = part.forward(rows, hand_step([1] * count, ctx, list(range(count))), a)
+    halves = [part.forward(rows[x:y].contiguous(), hand_step([1] * (y - x), ctx[x:y], list(range(x, y))), b).clone() for x, y in ((0, 9), (9, count))]
+    assert torch.equal(got, torch.cat(halves)) and torch.equal(a.state, b.state)
+
+
 @pytest.mark.parametrize("dtype,n,d,ff,experts,top,groups", [
     ("float32", 70, 64, 32, 12, 3, (3, 2)), ("float32", 9, 72, 24, 6, 6, (2, 2)), ("float32", 200, 40, 16, 4, 1, (4, 1)), ("bfloat16", 33, 64, 48, 12, 3, (4, 2)),
     ("bfloat16", 300, 76, 20, 9, 2, (3, 1)), ("float32", 5, 38, 8, 1, 1, None), ("bfloat16", 600, 128, 64, 8, 2, (4, 1)), ("float32", 40, 64, 16, 160, 5, (8, 3))])
