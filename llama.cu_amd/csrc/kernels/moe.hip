@@ -20,6 +20,7 @@
 #include "common.h"
 #include "gate_act.h"
 #include "lane_moves.h"
+#include "pair_sum.h"
 
 constexpr int MOE_MAX_EXPERTS = 1024;
 constexpr int MOE_TILE_ROWS = 128;       // rows of a tile of the kernel for many rows at most
@@ -673,33 +674,24 @@ moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict_
 #undef TILE
 }
 
-// out[t, c] (+)= sum_k wts[t, k] * y[t * top + k, c]  (in the order of k; wts null: ones)  + gate[t] * shared[t, c]  (shared null: nothing;
-// shared32: the same rows in 32 bits)
-// fresh: out is written, not added to (what it held is not read).  ids (null: none), real, h: a pair whose expert is
-// `real` or beyond is an identity expert, whose output is the token's input row h[t] itself.  Four columns a thread; d is a multiple of 4.
+// out[t] = the token's sum (pair_sum.h).  Four columns a thread; d is a multiple of 4.
 template <class T>
 __global__ void __launch_bounds__(256)
-moe_combine_kernel(float *__restrict__ out, const float *__restrict__ y, const float *__restrict__ wts,
-                   const T *__restrict__ shared, const float *__restrict__ shared32, const float *__restrict__ gate, int n, int d, int top,
-                   int fresh, const int *__restrict__ ids, int real, const T *__restrict__ h) {
+moe_combine_kernel(float *out, PairSum p, int n, int d) {
     const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (c >= d) return;
-    auto four = [](const T *p) {
-        const Quad<T> q = *(const Quad<T> *)p;
-        return f32x4{to_f32(q.v[0]), to_f32(q.v[1]), to_f32(q.v[2]), to_f32(q.v[3])};
-    };
-    for (size_t t = blockIdx.y; t < (size_t)n; t += gridDim.y) {
-        f32x4 acc = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *(const f32x4 *)(out + t * d + c);
-        for (int k = 0; k < top; ++k) {
-            const float w = wts ? wts[t * top + k] : 1.f;
-            if (ids && ids[t * top + k] >= real) acc += w * four(h + t * d + c);
-            else acc += w * *(const f32x4 *)(y + (t * top + k) * d + c);
-        }
-        const float g = gate ? gate[t] : 1.f;
-        if (shared) acc += g * four(shared + t * d + c);
-        if (shared32) acc += g * *(const f32x4 *)(shared32 + t * d + c);
-        *(f32x4 *)(out + t * d + c) = acc;
-    }
+    for (size_t t = blockIdx.y; t < (size_t)n; t += gridDim.y) *(pair_f32x4 *)(out + t * d + c) = pair_sum4<T>(p, t, c, d);
+}
+
+// out: [n, d] 32-bit (p->base may be the same memory); p: in host memory.
+LCU_API int lcu_moe_combine(float *out, const PairSum *p, int type, int n, int d, hipStream_t stream) {
+    if (n <= 0) return LCU_OK;
+    if (!out || !p || !pair_sum_ok(*p, type, d) || (uintptr_t)out % 16 || (type != LCU_F32 && type != LCU_BF16)) return LCU_BAD_ARGUMENT;
+    const dim3 gc((d + 1023) / 1024, n < 65535 ? n : 65535), block(256);
+    if (type == LCU_BF16) moe_combine_kernel<bf16_t><<<gc, block, 0, stream>>>(out, *p, n, d);
+    else moe_combine_kernel<float><<<gc, block, 0, stream>>>(out, *p, n, d);
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
 }
 
 // Rows of a tile for n * top pairs over so many experts: while an expert has 16 rows or fewer on average the kernel for few rows, with no
@@ -742,11 +734,11 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
 // token's input.  shared (null or
 // [n, d] of `type`) with shared_gate (null or [n] 32-bit): rows that are added beside the experts', times the gate.  shared_up,
 // shared_down (null, or the matrices [2 * shared_ff, d] and [d, shared_ff] of a shared expert that is computed here, with silu, in the order of Unit
-// like w_up and w_down; only where lcu_moe_tile_rows says 16 or 0): act then holds n * shared_ff elements more and y n rows more.
+// like w_up and w_down; defer: with top > 1 or gated the sum is left to whoever reads y; only where lcu_moe_tile_rows says 16 or 0): act then holds n * shared_ff elements more and y n rows more.
 LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float *wts, int *ints, int max_tiles,
                             const void *w_up, int packed_up, const void *w_down, int packed_down, void *act, float *y, float *out, int n, int d, int ff,
                             int experts, int top, int gated, const void *shared, const float *shared_gate, const void *shared_up,
-                            const void *shared_down, int shared_ff, int fresh, int identity, float alpha, float limit, hipStream_t stream) {
+                            const void *shared_down, int shared_ff, int fresh, int identity, float alpha, float limit, int defer, hipStream_t stream) {
     if (n <= 0) return LCU_OK;
     const int per = type == LCU_BF16 ? 8 : 4;
     if (d <= 0 || ff <= 0 || d % per || ff % per || experts <= 0 || experts > MOE_MAX_EXPERTS || top <= 0 ||
@@ -812,15 +804,9 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
 #undef DOWN
     }
 #undef TYPED
-    if (!add) {
-        const dim3 gc((d + 1023) / 1024, n < 65535 ? n : 65535);
-        const int *idp = identity ? ids : nullptr;
-        const float *shared32 = shared_up ? y + (size_t)total * d : nullptr;
-#define COMBINE(T) moe_combine_kernel<T><<<gc, dim3(256), 0, stream>>>(out, y, gated ? wts : nullptr, (const T *)shared, shared32, shared_gate, n, d, top, fresh, idp, experts, (const T *)h)
-        if (type == LCU_BF16) COMBINE(bf16_t);
-        else COMBINE(float);
-#undef COMBINE
-        LCU_LAUNCH_CHECK();
+    if (!add && !defer) {
+        const PairSum p = {fresh ? nullptr : out, y, gated ? wts : nullptr, shared, shared_up ? y + (size_t)total * d : nullptr, shared_gate, identity ? ids : nullptr, h, top, experts};
+        return lcu_moe_combine(out, &p, type, n, d, stream);
     }
     return LCU_OK;
 }

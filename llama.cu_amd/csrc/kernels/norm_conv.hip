@@ -11,6 +11,7 @@
 // last T - 1 rows of earlier steps) and rows before position 0 are zeros.
 #include "common.h"
 #include "rows.h"
+#include "pair_sum.h"
 
 constexpr int NC_THREADS = 256;
 constexpr int MAX_TAPS = 16;
@@ -55,8 +56,35 @@ layernorm_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes
 // thread adds, and so a row's bits, depend on d alone.  (A 32-bit model gives a token the same bits in a portion, whose norm and
 // convolution are kernels of their own, and alone.)  2,048 rows of 64 or 100: 4.9 and 5.6 us with 512 threads, 3.6 and 4.0 with 256; one odd row of
 // 513: 2.7 us with 512, 3.4 with 256 (2,048 of them 7.5 and 6.3).  WIDE: every address lets four elements be read at once.
-template <class TD, int T, int V, int PT, bool WIDE>
-__device__ __forceinline__ void take_row(float *xr, const TD *delta, int planes, size_t plane_stride, size_t row_at, int d, float eps,
+// D: where delta comes from: planes of rows, or a token's experts (beside another branch's rows).
+template <class T> struct PlanesOf {
+    const T *p;
+    int planes;
+    size_t stride;
+    __device__ __forceinline__ bool any() const { return p != nullptr; }
+    template <int V, bool WIDE> __device__ __forceinline__ void first(size_t row, int c, int d, float *out) const { load_some<T, V, WIDE>(p + row * d + c, out); }
+    template <int V, bool WIDE> __device__ __forceinline__ void add_rest(size_t row, int c, int d, float *out) const {
+        for (int k = 1; k < planes; ++k) {
+            float more[V];
+            load_some<T, V, WIDE>(p + k * stride + row * d + c, more);
+#pragma unroll
+            for (int e = 0; e < V; ++e) out[e] += more[e];
+        }
+    }
+};
+template <class T> struct PairsOf {
+    PairSum p;
+    __device__ __forceinline__ bool any() const { return true; }
+    template <int V, bool WIDE> __device__ __forceinline__ void first(size_t row, int c, int d, float *out) const {
+        static_assert(V == 4 && WIDE, "");
+        const pair_f32x4 v = pair_sum4<T>(p, row, c, d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = v[e];
+    }
+    template <int V, bool WIDE> __device__ __forceinline__ void add_rest(size_t, int, int, float *) const {}
+};
+template <class D, int T, int V, int PT, bool WIDE>
+__device__ __forceinline__ void take_row(float *xr, const D &delta, size_t row, int d, float eps,
                                          float (&v)[PT][V], float &mean, float &rstd, float (*scratch)[16]) {
     float sum = 0.f, first[PT][V];                   // (the row and the first plane are on their way before anything is added or written)
 #pragma unroll
@@ -66,21 +94,16 @@ __device__ __forceinline__ void take_row(float *xr, const TD *delta, int planes,
         for (int e = 0; e < V; ++e) v[i][e] = first[i][e] = 0.f;
         if (c < d) {
             load_some<float, V, WIDE>(xr + c, v[i]);
-            if (delta) load_some<TD, V, WIDE>(delta + row_at + c, first[i]);
+            if (delta.any()) delta.template first<V, WIDE>(row, c, d, first[i]);
         }
     }
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
         const int c = (threadIdx.x + T * i) * V;
-        if (delta && c < d) {
+        if (delta.any() && c < d) {
 #pragma unroll
             for (int e = 0; e < V; ++e) v[i][e] += first[i][e];
-            for (int p = 1; p < planes; ++p) {
-                float more[V];
-                load_some<TD, V, WIDE>(delta + p * plane_stride + row_at + c, more);
-#pragma unroll
-                for (int e = 0; e < V; ++e) v[i][e] += more[e];
-            }
+            delta.template add_rest<V, WIDE>(row, c, d, v[i]);
             store_some<float, V, WIDE>(xr + c, v[i]);
         }
 #pragma unroll
@@ -100,9 +123,9 @@ __device__ __forceinline__ void take_row(float *xr, const TD *delta, int planes,
 
 // The same for rows of up to T * V * PT elements: the row stays in registers between its one read and its writes.  With 256
 // threads and single elements 2,048 rows of 2,048 with two 32-bit outputs took 21.8 us, now 14.2, one row 5.5, now 2.3.
-template <class TD, class TO, int T, int V, int PT, bool WIDE>
+template <class D, class TO, int T, int V, int PT, bool WIDE>
 __global__ void __launch_bounds__(T)
-layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes, size_t plane_stride,
+layernorm_row_kernel(float *__restrict__ x, const D delta,
                      const float *__restrict__ w1, const float *__restrict__ b1, TO *__restrict__ out1,
                      const float *__restrict__ w2, const float *__restrict__ b2, TO *__restrict__ out2, int d, float eps) {
     __shared__ float scratch[2][16];
@@ -121,7 +144,7 @@ layernorm_row_kernel(float *__restrict__ x, const TD *__restrict__ delta, int pl
             }
         }
     }
-    take_row<TD, T, V, PT, WIDE>(x + row_at, delta, planes, plane_stride, row_at, d, eps, v, mean, rstd, scratch);
+    take_row<D, T, V, PT, WIDE>(x + row_at, delta, blockIdx.x, d, eps, v, mean, rstd, scratch);
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
         const int c = (threadIdx.x + T * i) * V;
@@ -150,7 +173,7 @@ LCU_API int lcu_layernorm(float *x, const void *delta, int delta_type, int plane
     const bool four = d % 4 == 0;
     const bool wide = four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) && four_ok(out1, out_type) &&
                       four_ok(w2, LCU_F32) && four_ok(b2, LCU_F32) && four_ok(out2, out_type);
-#define ROW(TD, TO, T, V, PT, WIDE) layernorm_row_kernel<TD, TO, T, V, PT, WIDE><<<grid, dim3(T), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
+#define ROW(TD, TO, T, V, PT, WIDE) layernorm_row_kernel<PlanesOf<TD>, TO, T, V, PT, WIDE><<<grid, dim3(T), 0, stream>>>(x, PlanesOf<TD>{(const TD *)delta, planes, stride}, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
 #define GO(TD, TO)                                                                                                           \
     do {                                                                                                                     \
         if (four && d <= 1024) { if (wide) ROW(TD, TO, 256, 4, 1, true); else ROW(TD, TO, 256, 4, 1, false); }               \
@@ -169,6 +192,25 @@ LCU_API int lcu_layernorm(float *x, const void *delta, int delta_type, int plane
     else return LCU_BAD_ARGUMENT;
 #undef ROW
 #undef GO
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
+}
+
+// The same with a token's experts' sum (in host memory; type: of the model) as delta.  d a multiple of 4, at most 4096, everything aligned for four.
+LCU_API int lcu_layernorm_pairs(float *x, const PairSum *pairs, int type, const float *w1, const float *b1, void *out1, const float *w2, const float *b2,
+                                void *out2, int out_type, int n, int d, float eps, hipStream_t stream) {
+    if (n <= 0) return LCU_OK;
+    if (!x || !pairs || !w1 || !b1 || !out1 || (w2 && (!b2 || !out2)) || !pair_sum_ok(*pairs, type, d) || d > 4096 || !four_ok(x, LCU_F32) ||
+        !four_ok(w1, LCU_F32) || !four_ok(b1, LCU_F32) || !four_ok(out1, out_type) || !four_ok(w2, LCU_F32) || !four_ok(b2, LCU_F32) || !four_ok(out2, out_type))
+        return LCU_BAD_ARGUMENT;
+#define ROW(T_, TO, T, PT) layernorm_row_kernel<PairsOf<T_>, TO, T, 4, PT, true><<<dim3(n), dim3(T), 0, stream>>>(x, PairsOf<T_>{*pairs}, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
+#define GO(T_, TO) do { if (d <= 1024) ROW(T_, TO, 256, 1); else if (d <= 2048) ROW(T_, TO, 512, 1); else ROW(T_, TO, 512, 2); } while (0)
+    if (type == LCU_F32 && out_type == LCU_F32) GO(float, float);
+    else if (type == LCU_BF16 && out_type == LCU_F32) GO(bf16_t, float);
+    else if (type == LCU_BF16 && out_type == LCU_BF16) GO(bf16_t, bf16_t);
+    else return LCU_BAD_ARGUMENT;
+#undef GO
+#undef ROW
     LCU_LAUNCH_CHECK();
     return LCU_OK;
 }
@@ -278,9 +320,9 @@ LCU_API int lcu_short_conv(const void *h, int h_type, long long set_stride_h, co
 // of taps where a thread reads its 4 TAPS weights in pieces of four, or 0 (one by one, up to FUSED_TAPS).  With 256 threads,
 // single numbers and the two sets one after the other four rows of 2,048 with four taps took 13.8 us, now 5.0.
 constexpr int FUSED_TAPS = 8;
-template <class TD, class TO, int T, int V, int PT, bool WIDE, int TAPS>
+template <class D, class TO, int T, int V, int PT, bool WIDE, int TAPS>
 __global__ void __launch_bounds__(T)
-norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int planes, size_t plane_stride,
+norm_conv_single_kernel(float *__restrict__ x, const D delta,
                         const float *__restrict__ w1, const float *__restrict__ b1, const float *__restrict__ w2,
                         const float *__restrict__ b2, const float *__restrict__ cw, float *__restrict__ st,
                         TO *__restrict__ out, size_t set_stride_out, const int *__restrict__ ctx_len,
@@ -327,7 +369,7 @@ norm_conv_single_kernel(float *__restrict__ x, const TD *__restrict__ delta, int
             }
         }
     }
-    take_row<TD, T, V, PT, WIDE>(x + (size_t)r * d, delta, planes, plane_stride, (size_t)r * d, d, eps, v, mean, rstd, scratch);
+    take_row<D, T, V, PT, WIDE>(x + (size_t)r * d, delta, r, d, eps, v, mean, rstd, scratch);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         if (s >= sets) break;
@@ -366,7 +408,7 @@ LCU_API int lcu_norm_conv_single(float *x, const void *delta, int delta_type, in
     const int dt = delta ? delta_type : LCU_F32;
     const bool wide = four_ok(x, LCU_F32) && four_ok(delta, dt) && four_ok(w1, LCU_F32) && four_ok(b1, LCU_F32) &&
                       four_ok(w2, LCU_F32) && four_ok(b2, LCU_F32) && four_ok(cw, LCU_F32) && four_ok(state, LCU_F32) && four_ok(out, out_type);
-#define ROW(TD, TO, T, V, PT, WIDE, TAPS) norm_conv_single_kernel<TD, TO, T, V, PT, WIDE, TAPS><<<grid, dim3(T), 0, stream>>>(x, (const TD *)delta, planes, stride, w1, b1, w2, b2, cw, state, (TO *)out, stride, ctx_len, state_slot, d, taps, sets, eps)
+#define ROW(TD, TO, T, V, PT, WIDE, TAPS) norm_conv_single_kernel<PlanesOf<TD>, TO, T, V, PT, WIDE, TAPS><<<grid, dim3(T), 0, stream>>>(x, PlanesOf<TD>{(const TD *)delta, planes, stride}, w1, b1, w2, b2, cw, state, (TO *)out, stride, ctx_len, state_slot, d, taps, sets, eps)
 #define SIZED(TD, TO, V, PT, WIDE, TAPS) do { if (d <= 1024) ROW(TD, TO, 256, V, PT, WIDE, TAPS); else ROW(TD, TO, 512, V, PT, WIDE, TAPS); } while (0)
 #define GO(TD, TO)                                                      \
     do {                                                                \
@@ -395,3 +437,31 @@ LCU_API int lcu_norm_conv_single(float *x, const void *delta, int delta_type, in
     return LCU_OK;
 }
 
+// The same with a token's experts' sum (in host memory; type: of the model, and of out) as delta.  d a multiple of 4, everything aligned for four.
+LCU_API int lcu_norm_conv_single_pairs(float *x, const PairSum *pairs, int type, const float *w1, const float *b1, const float *w2, const float *b2,
+                                       const float *cw, float *state, void *out, const int *ctx_len, const int *state_slot, int n, int d, int taps, int sets,
+                                       float eps, hipStream_t stream) {
+    if (n <= 0) return LCU_OK;
+    if (!x || !pairs || d > 2048 || taps < 1 || taps > 8 || sets < 1 || sets > 2 || !w1 || !b1 || (sets == 2 && (!w2 || !b2)) || !cw || (taps > 1 && !state) ||
+        !pair_sum_ok(*pairs, type, d) || !four_ok(x, LCU_F32) || !four_ok(w1, LCU_F32) || !four_ok(b1, LCU_F32) || !four_ok(w2, LCU_F32) || !four_ok(b2, LCU_F32) ||
+        !four_ok(cw, LCU_F32) || !four_ok(state, LCU_F32) || !four_ok(out, type))
+        return LCU_BAD_ARGUMENT;
+    const size_t stride = (size_t)n * d;
+#define ROW(T_, T, TAPS) norm_conv_single_kernel<PairsOf<T_>, T_, T, 4, 1, true, TAPS><<<dim3(n), dim3(T), 0, stream>>>(x, PairsOf<T_>{*pairs}, w1, b1, w2, b2, cw, state, (T_ *)out, stride, ctx_len, state_slot, d, taps, sets, eps)
+#define SIZED(T_, TAPS) do { if (d <= 1024) ROW(T_, 256, TAPS); else ROW(T_, 512, TAPS); } while (0)
+#define GO(T_)                              \
+    do {                                    \
+        if (taps == 2) SIZED(T_, 2);        \
+        else if (taps == 3) SIZED(T_, 3);   \
+        else if (taps == 4) SIZED(T_, 4);   \
+        else SIZED(T_, 0);                  \
+    } while (0)
+    if (type == LCU_BF16) GO(bf16_t);
+    else if (type == LCU_F32) GO(float);
+    else return LCU_BAD_ARGUMENT;
+#undef GO
+#undef SIZED
+#undef ROW
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
+}

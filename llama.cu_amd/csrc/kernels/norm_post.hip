@@ -8,6 +8,7 @@
 // factors themselves (a model that stores them around zero adds the one when it loads them).  The order of the sums
 // depends on the width and the block size only.
 #include "rows.h"
+#include "pair_sum.h"
 
 constexpr int NP_KEEP = 8;          // elements of a row that a thread keeps in registers: rows up to 8 x the block's threads are read once
 
@@ -78,13 +79,26 @@ norm_post_kernel(float *__restrict__ x, const TA *__restrict__ a, const float *_
 // rows, all loads first, two barriers.  (With 1,024 threads and single elements one row of 2,048 took 3.7 us, now 2.2, 16 rows 4.7, now 3.1; 2,048 rows
 // 10.8, now 9.2.)
 constexpr int NP_ROW_THREADS = 512;
-template <class TA, class TO, int PT>
+// A: where the sublayer's output comes from: rows, or a token's experts.  (Their sum in a kernel in front was 4.7 us a layer in a step of 16 tokens and 11.7 in one of
+// 2,040, most of it the way through memory: ralepel 12.54 -> 12.12 ms a pass without it.)
+template <class T> struct RowsOf {
+    const T *p;
+    __device__ __forceinline__ void four(size_t row, int c, int d, float *out) const { load_as_f32<T, 4>(p + row * d + c, out); }
+};
+template <class T> struct PairsOf {
+    PairSum p;
+    __device__ __forceinline__ void four(size_t row, int c, int d, float *out) const {
+        const pair_f32x4 v = pair_sum4<T>(p, row, c, d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = v[e];
+    }
+};
+template <class A, class TO, int PT>
 __global__ void __launch_bounds__(NP_ROW_THREADS)
-norm_post_row_kernel(float *__restrict__ x, const TA *__restrict__ a, const float *__restrict__ a_bias, const float *__restrict__ w_post, float eps_post,
+norm_post_row_kernel(float *__restrict__ x, const A a, const float *__restrict__ a_bias, const float *__restrict__ w_post, float eps_post,
                      const float *__restrict__ w_pre, float eps_pre, TO *__restrict__ out, int d) {
     __shared__ float scratch[2][16];
     float *xr = x + (size_t)blockIdx.x * d;
-    const TA *ar = a + (size_t)blockIdx.x * d;
     float v[PT][4], xs[PT][4], wp[PT][4], wq[PT][4], acc = 0.f;
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
@@ -92,10 +106,10 @@ norm_post_row_kernel(float *__restrict__ x, const TA *__restrict__ a, const floa
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[i][e] = 0.f;
         if (c >= d) continue;
-        load_as_f32<TA, 4>(ar + c, v[i]);
         load_as_f32<float, 4>(xr + c, xs[i]);
         load_as_f32<float, 4>(w_post + c, wp[i]);
         if (w_pre) load_as_f32<float, 4>(w_pre + c, wq[i]);
+        a.four(blockIdx.x, c, d, v[i]);
         if (a_bias) {
             float b[4];
             load_as_f32<float, 4>(a_bias + c, b);
@@ -145,7 +159,7 @@ LCU_API int lcu_norm_post(float *x, const void *a, int a_type, const float *a_bi
     dim3 grid(n);
     const bool four = d % 4 == 0 && d <= 8 * NP_ROW_THREADS && four_ok(x, LCU_F32) && four_ok(a, a_type) && four_ok(a_bias, LCU_F32) &&
                       four_ok(w_post, LCU_F32) && four_ok(w_pre, LCU_F32) && four_ok(out, out_type);
-#define FOUR(TA, TO, PT) norm_post_row_kernel<TA, TO, PT><<<grid, dim3(NP_ROW_THREADS), 0, stream>>>(x, (const TA *)a, a_bias, w_post, eps_post, w_pre, eps_pre, (TO *)out, d)
+#define FOUR(TA, TO, PT) norm_post_row_kernel<RowsOf<TA>, TO, PT><<<grid, dim3(NP_ROW_THREADS), 0, stream>>>(x, RowsOf<TA>{(const TA *)a}, a_bias, w_post, eps_post, w_pre, eps_pre, (TO *)out, d)
 #define GO(TA, TO) do { if (four && d <= 4 * NP_ROW_THREADS) FOUR(TA, TO, 1); else if (four) FOUR(TA, TO, 2); \
                         else if (wide) norm_post_kernel<TA, TO, 1024><<<grid, dim3(1024), 0, stream>>>(x, (const TA *)a, a_bias, w_post, eps_post, w_pre, eps_pre, (TO *)out, d); \
                         else norm_post_kernel<TA, TO, 256><<<grid, dim3(256), 0, stream>>>(x, (const TA *)a, a_bias, w_post, eps_post, w_pre, eps_pre, (TO *)out, d); } while (0)
@@ -156,6 +170,21 @@ LCU_API int lcu_norm_post(float *x, const void *a, int a_type, const float *a_bi
     else return LCU_BAD_ARGUMENT;
 #undef GO
 #undef FOUR
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
+}
+
+// The same with a token's experts' sum (in host memory; type: of the model, and of out) in the place of a.  d a multiple of 4, at most 8 * NP_ROW_THREADS.
+LCU_API int lcu_norm_post_pairs(float *x, const PairSum *pairs, int type, const float *w_post, float eps_post, const float *w_pre, float eps_pre, void *out, int n,
+                                int d, hipStream_t stream) {
+    if (n <= 0) return LCU_OK;
+    if (!x || !pairs || !w_post || (w_pre && !out) || !pair_sum_ok(*pairs, type, d) || d > 8 * NP_ROW_THREADS || !four_ok(x, LCU_F32) || !four_ok(w_post, LCU_F32) ||
+        !four_ok(w_pre, LCU_F32) || !four_ok(out, type) || (type != LCU_F32 && type != LCU_BF16))
+        return LCU_BAD_ARGUMENT;
+#define GO(T, PT) norm_post_row_kernel<PairsOf<T>, T, PT><<<dim3(n), dim3(NP_ROW_THREADS), 0, stream>>>(x, PairsOf<T>{*pairs}, nullptr, w_post, eps_post, w_pre, eps_pre, (T *)out, d)
+    if (type == LCU_BF16) { if (d <= 4 * NP_ROW_THREADS) GO(bf16_t, 1); else GO(bf16_t, 2); }
+    else { if (d <= 4 * NP_ROW_THREADS) GO(float, 1); else GO(float, 2); }
+#undef GO
     LCU_LAUNCH_CHECK();
     return LCU_OK;
 }

@@ -1278,7 +1278,14 @@ def layernorm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: fl
               bias2: Optional[torch.Tensor] = None, out2: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``y = (x' - mean) * rsqrt(var + eps) * weight + bias`` with ``x' = x + delta`` (rows, or planes
     ``[planes, n, d]`` that are added one after the other), in 32-bit; ``x`` (float32, the residual stream) takes
-    the sum in.  With ``weight2``, ``bias2``, ``out2`` a second norm of the same rows is written in the same pass."""
+    the sum in.  With ``weight2``, ``bias2``, ``out2`` a second norm of the same rows is written in the same pass.  ``delta`` may be a ``PairSum``."""
+    pairs = None
+    if isinstance(delta, PairSum):
+        if (delta.n, delta.d) == tuple(x.shape) and pair_sum_takes(delta.d, x, weight, bias, out, weight2, bias2, out2) \
+                and (out.dtype == torch.float32 or out.dtype == delta.dtype):
+            pairs, delta = delta, None
+        else:
+            delta = delta.rows()
     _gpu(x, weight, bias, out, delta, weight2, bias2, out2)
     _rows(x, "norm input"); _contig(x, "norm input"); _contig(out, "norm out")
     n, d = x.shape
@@ -1290,6 +1297,10 @@ def layernorm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: fl
         raise KernelError("layernorm out: wrong shape, type or layout")
     if (weight2 is None) != (out2 is None) or (weight2 is None) != (bias2 is None):
         raise KernelError("layernorm: a second norm needs its weight, its bias and its output")
+    if pairs is not None:
+        _check(build.load("norm_conv").lcu_layernorm_pairs(_ptr(x), ctypes.byref(pairs.args()), pairs.type(), _ptr(weight), _ptr(bias), _ptr(out), _ptr(weight2),
+                                                           _ptr(bias2), _ptr(out2), _type(out, "norm out"), n, d, ctypes.c_float(eps), _stream()), "layernorm_pairs")
+        return out
     planes = 0
     if delta is not None:
         _contig(delta, "norm delta")
@@ -1332,6 +1343,12 @@ def norm_conv_single(x: torch.Tensor, delta: Optional[torch.Tensor], weights, bi
     """For a step in which every request feeds one token: ``layernorm`` (with the residual sum), ``short_conv`` and the
     states' update in one kernel.  ``weights``, ``biases``: one or two float32 vectors each (the norms of the one or two
     sets); the rest as in ``short_conv``; ``out [sets, n, d]``."""
+    pairs = None
+    if isinstance(delta, PairSum):
+        if (delta.n, delta.d) == tuple(x.shape) and pair_sum_takes(delta.d, x, conv_weight, state, out, *weights, *biases) and out.dtype == delta.dtype:
+            pairs, delta = delta, None
+        else:
+            delta = delta.rows()
     _gpu(x, delta, conv_weight, state, out, *weights, *biases)
     _rows(x, "norm input"); _contig(x, "norm input"); _contig(out, "conv out"); _contig(conv_weight, "conv weight"); _contig(state, "conv state")
     n, d = x.shape
@@ -1346,6 +1363,12 @@ def norm_conv_single(x: torch.Tensor, delta: Optional[torch.Tensor], weights, bi
     if taps > 1 and (state.dtype != torch.float32 or state.dim() != 4 or state.shape[1:] != (sets, taps - 1, d)
                      or max(step.state_slots, default=0) >= state.shape[0]):
         raise KernelError(f"norm_conv_single: state must be float32 [slots, {sets}, {taps - 1}, {d}] and hold every request's slot")
+    if pairs is not None:
+        _check(build.load("norm_conv").lcu_norm_conv_single_pairs(
+            _ptr(x), ctypes.byref(pairs.args()), pairs.type(), _ptr(weights[0]), _ptr(biases[0]), _ptr(weights[1] if sets == 2 else None),
+            _ptr(biases[1] if sets == 2 else None), _ptr(conv_weight), _ptr(state if taps > 1 else None), _ptr(out), _ptr(step.ctx_len), _ptr(step.state_slot),
+            n, d, taps, sets, ctypes.c_float(eps), _stream()), "norm_conv_single_pairs")
+        return out
     planes = 0
     if delta is not None:
         _contig(delta, "norm delta")
@@ -1522,7 +1545,7 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, top: int, bias: Optional[to
 def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
                 out: torch.Tensor, gated: bool = False, shared: Optional[torch.Tensor] = None,
                 shared_gate: Optional[torch.Tensor] = None, fresh: bool = False, identity: int = 0,
-                act_alpha: float = 1.0, act_limit: float = 0.0, shared_expert: Optional[tuple] = None) -> torch.Tensor:
+                act_alpha: float = 1.0, act_limit: float = 0.0, shared_expert: Optional[tuple] = None, defer: bool = False):
     """``out[t] += sum over t's experts e of  w_down[e] @ gelu(w_up[e] @ (weight * h[t]))`` (the exact gelu; the
     weight scales what goes INTO the expert, not what comes out).  ``w_up [experts, ff, d]``, ``w_down [experts, d, ff]`` in ``h``'s type,
     ``out`` float32 ``[n, d]``.  ``gated``: ``out[t] += sum_e weight * w_down[e] @ (silu(gate[e] @ h[t]) * (up[e] @ h[t]))``
@@ -1532,7 +1555,8 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
     identity`` experts, of which the last ``identity`` have no matrices: their output is ``weight * h[t]`` (gated form only).
     ``act_limit`` > 0: the limited activation (``swiglu``) with ``act_alpha`` instead of silu.  ``shared_expert``: in the place of
     ``shared`` the matrices (``[1, 2 * sff, d]`` as ``gated_rows`` lays them out and ``[1, d, sff]``, both packed) of an expert with
-    silu that every token uses, computed beside the others; where ``moe_shared_beside`` says so."""
+    silu that every token uses, computed beside the others; where ``moe_shared_beside`` says so.  ``defer``: the experts' outputs may come back as a
+    ``PairSum`` that whoever uses the sum adds up (``out``, unless ``fresh``, is then one of its terms and not written)."""
     up, down = (w.data if isinstance(w, PackedExperts) else w for w in (w_up, w_down))
     _gpu(h, ids, wts, up, down, out, shared, shared_gate)
     _rows(h, "moe input")
@@ -1588,8 +1612,51 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
                                int(up is not w_up), _ptr(down), int(down is not w_down), _ptr(act), _ptr(y), _ptr(out), n, d, ff, experts, top, int(bool(gated)),
                                _ptr(shared), _ptr(shared_gate if shared is not None or sff else None), _ptr(shared_up.data if sff else None),
                                _ptr(shared_down.data if sff else None), sff, int(bool(fresh)), identity, ctypes.c_float(act_alpha),
-                               ctypes.c_float(act_limit), _stream()), "moe_experts")
+                               ctypes.c_float(act_limit), int(bool(defer)), _stream()), "moe_experts")
+    if defer and (gated or top > 1):
+        return PairSum(n, d, h.dtype, top, y, wts if gated else None, None if fresh else out, shared, y[total:] if sff else None,
+                       shared_gate if shared is not None or sff else None, ids if identity else None, h if identity else None, experts)
     return out
+
+
+class _PairSumArgs(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in ("base", "y", "wts", "shared", "shared32", "gate", "ids", "h")] + [("top", ctypes.c_int), ("real", ctypes.c_int)]
+
+
+@dataclass
+class PairSum:
+    """Float32 rows ``[n, d]`` that stand in memory as the terms of their sum: what a token's experts gave (``y [n * top, d]``, times ``wts``), beside ``base``
+    and a shared expert's rows.  The norms that add a branch to the residual stream take them where ``pair_sum_takes`` says so; ``rows()`` adds them up."""
+    n: int
+    d: int
+    dtype: torch.dtype
+    top: int
+    y: torch.Tensor
+    wts: Optional[torch.Tensor]
+    base: Optional[torch.Tensor]
+    shared: Optional[torch.Tensor]
+    shared32: Optional[torch.Tensor]
+    gate: Optional[torch.Tensor]
+    ids: Optional[torch.Tensor]
+    h: Optional[torch.Tensor]
+    real: int
+
+    def args(self) -> _PairSumArgs:
+        at = lambda t: t.data_ptr() if t is not None else None
+        return _PairSumArgs(at(self.base), at(self.y), at(self.wts), at(self.shared), at(self.shared32), at(self.gate), at(self.ids), at(self.h), self.top, self.real)
+
+    def type(self) -> int:
+        return BF16 if self.dtype == torch.bfloat16 else F32
+
+    def rows(self) -> torch.Tensor:
+        out = self.base if self.base is not None else torch.empty((self.n, self.d), dtype=torch.float32, device=self.y.device)
+        _check(build.load("moe").lcu_moe_combine(_ptr(out), ctypes.byref(self.args()), self.type(), self.n, self.d, _stream()), "moe_combine")
+        return out
+
+
+def pair_sum_takes(d: int, *operands) -> bool:
+    """Whether the norms' kernels add up a ``PairSum`` of width ``d`` beside these operands (rows in registers, four elements an access)."""
+    return d % 4 == 0 and d <= 4096 and all(t is None or t.data_ptr() % 16 == 0 for t in operands)
 
 
 MOE_SHARED_ROWS = 32        # tokens up to which a shared expert is computed beside the others (each 16 read its matrices once)
@@ -1661,7 +1728,19 @@ def norm_post(x: torch.Tensor, a: torch.Tensor, w_post: torch.Tensor, eps_post: 
     follows, in ``out_dtype``; one kernel.  The weights are float32 factors.  ``copy`` (without ``w_pre``; taken as
     asked for where ``out_dtype`` is given without ``w_pre``): the new stream itself comes back, rounded to
     ``out_dtype``, for a sublayer that reads the stream without a norm.
-    ``a_bias`` (float32 ``[d]``): a bias that ``a`` still lacks; ``a + a_bias`` is what is normed."""
+    ``a_bias`` (float32 ``[d]``): a bias that ``a`` still lacks; ``a + a_bias`` is what is normed.  ``a`` may be a ``PairSum``."""
+    if isinstance(a, PairSum):
+        n, d = x.shape
+        want = out_dtype if out_dtype is not None else torch.float32          # (the type that rows() would hand on)
+        if x.shape != (a.n, a.d) or a_bias is not None or not pair_sum_takes(d, x, w_post, w_pre) or x.dtype != torch.float32 or not x.is_contiguous() \
+                or ((w_pre is not None or copy or out_dtype is not None) and want != a.dtype):
+            return norm_post(x, a.rows(), w_post, eps_post, w_pre, eps_pre, out_dtype, a_bias, copy)
+        _gpu(x, w_post, w_pre)
+        _f32_vec(w_post, "norm weight", d); _f32_vec(w_pre, "norm weight", d)
+        out = torch.empty((n, d), dtype=a.dtype, device=x.device) if w_pre is not None or copy or (copy is None and out_dtype is not None) else None
+        _check(build.load("norm_post").lcu_norm_post_pairs(_ptr(x), ctypes.byref(a.args()), a.type(), _ptr(w_post), ctypes.c_float(eps_post), _ptr(w_pre),
+                                                           ctypes.c_float(eps_pre), _ptr(out), n, d, _stream()), "norm_post_pairs")
+        return out
     _gpu(x, a, w_post, w_pre, a_bias)
     _rows(x, "residual stream"); _contig(x, "residual stream"); _contig(a, "sublayer output")
     n, d = x.shape

@@ -269,6 +269,8 @@ class Part:
     #
     # norm:  ``deferrable``: the norm is a factor per row times a weight per column (``weight``, ``size``,
     #        ``eps``), so the factor may be applied after the next matrix product (ScaledRows);
+    #        ``ends_in_pairs`` (feed-forwards and blocks): ``forward(..., pairs_ok=True)`` may return an ops.PairSum in the place of float32 rows;
+    #        ``takes_pairs``: a block's ``pending`` may be one
     #        ``takes_planes``: ``forward(x, delta)`` also takes float32 planes ``[planes, rows, width]``
     #        of partial sums as ``delta``;
     #        ``delta_scale``: what ``delta`` is multiplied by before it is added to the stream, also by a
@@ -296,6 +298,8 @@ class Part:
     splits_output = False
     own_output = True
     takes_planes = False
+    takes_pairs = False
+    ends_in_pairs = False
     ends_in_norm = False
     ends_in_planes = False
     ends_in_next_norm = False

@@ -201,7 +201,21 @@ class ParallelBlock(Part):
     def takes_planes(self) -> bool:
         return bool(self.norm1.takes_planes)
 
-    def forward(self, x: torch.Tensor, pending, step, cache, next_norm=None, planes_ok=False):
+    @property
+    def takes_pairs(self) -> bool:
+        return self._pair            # (sums of other sizes than the norms' kernels add up are added up in front of them)
+
+    @property
+    def ends_in_pairs(self) -> bool:
+        return self.ffn is not None and self.ffn.ends_in_pairs
+
+    def _end(self, h, out, pairs_ok):
+        """``out`` and the feed-forward of ``h``."""
+        if self.ffn is None:
+            return out
+        return self.ffn.forward(h, add_to=out, pairs_ok=True) if pairs_ok and self.ffn.ends_in_pairs else self.ffn.forward(h, add_to=out)
+
+    def forward(self, x: torch.Tensor, pending, step, cache, next_norm=None, planes_ok=False, pairs_ok=False):
         n, d = x.shape
         conv = self.taps > 0
         # with a convolution behind them the norms write 32-bit rows, which are rounded once, after the convolution
@@ -213,7 +227,7 @@ class ParallelBlock(Part):
             h = ops.norm_conv_single(x, pending, [p.weight for p in norms], [p.bias for p in norms], self.norm1.eps,
                                      self.conv_weight, state, torch.empty((self.sets, n, d), dtype=self.dtype, device=x.device), step)
             out = self.mixer.forward(h[0], step, cache, out_dtype=torch.float32)
-            return self.ffn.forward(h[self.sets - 1], add_to=out) if self.ffn is not None else out
+            return self._end(h[self.sets - 1], out, pairs_ok)
         h = torch.empty((self.sets, n, d), dtype=mid, device=x.device)
         if self._pair:
             two = self.norm2 is not None
@@ -229,9 +243,7 @@ class ParallelBlock(Part):
             state = cache.more["conv"] if self.taps > 1 else torch.empty((1, self.sets, 0, d), dtype=torch.float32, device=x.device)
             h = ops.short_conv(h, self.conv_weight, state, torch.empty((self.sets, n, d), dtype=self.dtype, device=x.device), step)
         out = self.mixer.forward(h[0], step, cache, out_dtype=torch.float32)
-        if self.ffn is not None:
-            out = self.ffn.forward(h[self.sets - 1], add_to=out)
-        return out
+        return self._end(h[self.sets - 1], out, pairs_ok)
 
 
 register_part("block", "parallel", ParallelBlock)
@@ -267,6 +279,10 @@ class _SublayersInTurn(Part):
 
     def cache_need(self):
         return self.mixer.cache_need()
+
+    def _feed(self, h):
+        """The feed-forward's output for the norm behind it (``ops.norm_post``, which adds up a token's experts itself)."""
+        return self.ffn.forward(h, pairs_ok=True) if self.ffn.ends_in_pairs else self.ffn.forward(h)
 
     def prepare(self, step) -> None:
         for _, part in self._children():
@@ -322,7 +338,7 @@ class SandwichBlock(_SublayersInTurn):
         last, post = a, self.post1
         if self.ffn is not None:
             h2 = ops.norm_post(x, a, self.post1.weight32, self.post1.eps, self.norm2.weight32, self.norm2.eps, out_dtype=self.dtype)
-            last, post = self.ffn.forward(h2), self.post2
+            last, post = self._feed(h2), self.post2
         if next_norm is not None:
             return NormedRows(ops.norm_post(x, last, post.weight32, post.eps, next_norm.weight32, next_norm.eps, out_dtype=self.dtype))
         ops.norm_post(x, last, post.weight32, post.eps)
@@ -387,7 +403,7 @@ class PostNormBlock(_SublayersInTurn):
         last, post, bias = a, self.post1, (self.mixer.output_bias if later else None)
         if self.ffn is not None:
             h2 = self._sum_and_read(x, a, self.post1, bias, self._reads)
-            last, post, bias = self.ffn.forward(h2), self.post2, None
+            last, post, bias = self._feed(h2), self.post2, None
         if next_norm is not None:
             return NormedRows(self._sum_and_read(x, last, post, bias, next_norm))
         self._sum_and_read(x, last, post, bias, None)

@@ -198,6 +198,9 @@ class DecoderModel:
                         takes = step.logits_all and self.final_norm.takes_planes
                     if takes:
                         kw["planes_ok"] = True
+                # the same for the sum of a token's experts
+                if layer.ends_in_pairs and nothing_between and follower.takes_pairs:
+                    kw["pairs_ok"] = True
                 pending = layer.forward(x, pending, step, caches[i], **kw)
             if step.n_logits == 0:
                 return torch.empty((0, self.spec.vocab_size), dtype=torch.float32, device=x.device)

@@ -66,13 +66,15 @@ class SigmoidMoE(Part):
             self.w_up, self.w_down = ops.pack_experts(self.w_up), ops.pack_experts(self.w_down)
         self.dtype = build.dtype
 
-    def forward(self, h, add_to: Optional[torch.Tensor] = None):
+    ends_in_pairs = True         # beside another branch's rows (add_to)
+
+    def forward(self, h, add_to: Optional[torch.Tensor] = None, pairs_ok: bool = False):
         """``add_to``: float32 ``[n, d]`` that takes the output in (and is returned); without it the output comes
-        back in the compute type."""
+        back in the compute type.  ``pairs_ok``: with ``add_to`` the sum may come back as an ops.PairSum."""
         ids, wts = ops.moe_route(h, self.router, self.top)
         out = add_to if add_to is not None else torch.zeros((h.shape[0], self.hidden_size), dtype=torch.float32, device=h.device)
-        ops.moe_experts(h, ids, wts, self.w_up, self.w_down, out)
-        return out if add_to is not None else out.to(self.dtype)
+        summed = ops.moe_experts(h, ids, wts, self.w_up, self.w_down, out, defer=pairs_ok and add_to is not None)
+        return summed if add_to is not None else out.to(self.dtype)
 
 
 register_part("ffn", "sigmoid_moe", SigmoidMoE)
@@ -207,14 +209,17 @@ class GatedMoE(Part):
                 self.shared_expert = (ops.pack_gated_experts(sg[None], su[None]), ops.pack_experts(sd[None]))
         self.dtype = build.dtype
 
-    def forward(self, h, add_to: Optional[torch.Tensor] = None):
-        """``add_to``: float32 ``[n, d]`` that takes the output in (and is returned); without it the output is new rows."""
+    ends_in_pairs = True
+
+    def forward(self, h, add_to: Optional[torch.Tensor] = None, pairs_ok: bool = False):
+        """``add_to``: float32 ``[n, d]`` that takes the output in (and is returned); without it the output is new rows.  ``pairs_ok``: either may come back as an
+        ops.PairSum."""
         if self.pad_width:
             out = self._experts(torch.nn.functional.pad(h, (0, self.pad_width)), None)[:, :self.hidden_size].contiguous()
             return out if add_to is None else ops.scaled_sum(add_to, out, 1.0)
-        return self._experts(h, add_to)
+        return self._experts(h, add_to, pairs_ok)
 
-    def _experts(self, h, add_to):
+    def _experts(self, h, add_to, pairs_ok=False):
         over_all = self.scoring == "softmax_all"
         routed = ops.moe_route(h, self.router, self.top, bias=self.bias, softmax_chosen=not over_all, softmax_all=over_all,
                                extra=self.gates, **self.choice)
@@ -223,11 +228,9 @@ class GatedMoE(Part):
         out = add_to if not fresh else torch.empty((h.shape[0], h.shape[1]), dtype=torch.float32, device=h.device)
         if self.shared is not None:
             beside = self.shared_expert is not None and ops.moe_shared_beside(h.shape[0], ids.shape[1], self.experts, self.w_gate_up, self.w_down)
-            ops.moe_experts(h, ids, wts, self.w_gate_up, self.w_down, out, gated=True, shared=None if beside else self.shared.forward(h),
+            return ops.moe_experts(h, ids, wts, self.w_gate_up, self.w_down, out, gated=True, defer=pairs_ok, shared=None if beside else self.shared.forward(h),
                             shared_expert=self.shared_expert if beside else None, shared_gate=routed[2] if self.gates else None, fresh=fresh, identity=self.identity, **self.act)
-        else:
-            ops.moe_experts(h, ids, wts, self.w_gate_up, self.w_down, out, gated=True, fresh=fresh, identity=self.identity, **self.act)
-        return out
+        return ops.moe_experts(h, ids, wts, self.w_gate_up, self.w_down, out, gated=True, defer=pairs_ok, fresh=fresh, identity=self.identity, **self.act)
 
 
 register_part("ffn", "gated_moe", GatedMoE)
