@@ -23,7 +23,7 @@ import torch
 from ..kernels import ops
 from ..weights.loader import fused_rows
 from .base import BuildContext, Part, ScaledRows, SlotState, StreamsEnd, TensorSpec, register_part
-from .linear import Weight, end_in_norm, finish, linear_scaled, project, skinny_takes
+from .linear import Weight, end_in_norm, finish, linear_planes, linear_scaled, mid_takes, project, skinny_takes
 
 
 class _DecayScan(Part):
@@ -123,6 +123,12 @@ class Lightning(_DecayScan):
             scaled = ScaledRows(out, sumsq, self.output_width, self.norm_eps)
             fused = end_in_norm(scaled, self.w_o, into) if isinstance(into, StreamsEnd) else None
             return fused if fused is not None else linear_scaled(scaled, self.w_o, out_dtype=self.dtype)
+        if step.decode_only and planes_ok and self.dtype == torch.bfloat16 and out_dtype in (None, self.dtype) \
+                and ops.ADD_NORM_MAX_ROWS < n <= ops.MID_MAX_SCALED_ROWS and mid_takes(n, self.w_o):
+            # more of them: the same factor in the product that shares the rows through LDS (applied by a kernel in front it was 4.6 us a layer)
+            out = self._operand(h)
+            sumsq = self._scan(h, step, cache, out, 1.0, state, scaled_rows=True)
+            return linear_planes(ScaledRows(out, sumsq, self.output_width, self.norm_eps), self.w_o)
         return super().forward(h, step, cache, out_dtype=out_dtype, planes_ok=planes_ok, into=into, state=state)
 
 

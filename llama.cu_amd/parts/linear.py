@@ -221,9 +221,12 @@ def mid_takes(n_rows: int, weight: Union[torch.Tensor, Weight]) -> bool:
 
 def linear_planes(a: torch.Tensor, weight: Union[torch.Tensor, Weight]) -> torch.Tensor:
     """``a @ weight.T`` as float32 planes ``[planes, rows, out]`` of partial sums over slices of K
-    (``mid_takes`` says when); the norm that follows adds them to the residual stream."""
+    (``mid_takes`` says when); the norm that follows adds them to the residual stream.  ``a``: bfloat16 rows, or up to ``ops.MID_MAX_SCALED_ROWS``
+    ScaledRows (every slice's sums take the factor)."""
     w, packed = _split(weight)
     slices = _mid_slices(w.shape[0], w.shape[1])
+    if isinstance(a, ScaledRows):
+        return ops.gemm_mid(a.rows, w if packed is None else packed, slices=slices, packed=packed is not None, row_sumsq=a.sumsq, norm_width=a.width, eps=a.eps)
     if packed is not None:
         return ops.gemm_mid(a, packed, slices=slices, packed=True)
     return ops.gemm_mid(a, w, slices=slices)

@@ -290,6 +290,26 @@ def test_single_tokens_of_many_requests_and_rows_that_wait_for_their_norm():
                 assert_close(got[r], reference(f64(rows[r].float()))[-1], 3e-2, f"{count} requests, {r}")
 
 
+@pytest.mark.parametrize("count,planes", [(33, True), (50, True), (64, True), (65, False)])
+def test_single_tokens_whose_norm_the_product_with_shared_rows_applies(count, planes):
+    """From 33 to 64 requests the norm over the heads is a factor in the output product's partial sums; beyond, a kernel applies it."""
+    d = 128
+    part, plain, _ = lightning_part([0.9, 0.99, 0.5, 0.7, 0.95, 0.8, 0.999, 0.6], 128, 128, d, "bfloat16", pack=True)
+    lens = [1 + r % 4 for r in range(count)]
+    rows = [rnd(n + 1, d, seed=100 + r).bfloat16() for r, n in enumerate(lens)]
+    results = []
+    for ok in (True, False):
+        cache = state_of(part, count)
+        part.forward(torch.cat([x[:-1] for x in rows]).cuda(), hand_step(lens, lens, list(range(count))), cache)
+        results.append(part.forward(torch.stack([x[-1] for x in rows]).cuda(), hand_step([1] * count, [n + 1 for n in lens], list(range(count))), cache, planes_ok=ok))
+    got, other = results
+    assert (got.dtype == torch.float32 and got.dim() == 3) or not planes
+    got = got.float().sum(0) if got.dim() == 3 else got
+    for r in range(0, count, 4):
+        assert_close(got[r], plain(f64(rows[r].float()))[-1], 3e-2, f"{r}")
+    assert_close(got, f64(other.float().cpu()), 3e-2)
+
+
 @pytest.mark.parametrize("kind", ["lightning", "memory"])
 def test_single_tokens_whose_states_no_cache_holds(kind):
     """A step of single tokens whose states are streamed past the caches (48 MB and more) against its halves, whose are not: the same bits."""
