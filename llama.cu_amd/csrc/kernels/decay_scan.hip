@@ -558,7 +558,7 @@ __device__ __forceinline__ float block_sum_lds(float v, float *scratch) {
 
 // What bounds it is the state, read and written once; all that a workgroup needs beside it is asked for first and the state's first pieces behind that, so that
 // nothing waits for memory twice (the state after the rows, the gate and the weight where they are used: 64 requests, 16 heads of 128 x 128 36.3 us, 8 heads
-// gated 23.0; now 34.2 and 19.4 inside a step, and 29 where the state is streamed, 4.6 TB/s).
+// gated 23.0; with that and the streamed states below, which leave the others in the cache, 27.3 and 14.8 inside a step, 4.9 TB/s).
 // STREAM: the state's loads and stores are non-temporal.
 template <class TI, class T, int V, bool STREAM>
 __global__ void __launch_bounds__(256, 4)
