@@ -7,6 +7,7 @@ typedef __attribute__((ext_vector_type(4))) float pair_f32x4;
 template <class T> struct alignas(4 * sizeof(T)) PairQuad { T v[4]; };
 
 // row t: base[t] (null: 0) + sum_k wts[t, k] * y[t * top + k]  (in the order of k; wts null: ones)  + gate[t] * (shared[t] or shared32[t])  (gate null: 1).
+// A pair's product is rounded before it is added, the shared row's is not.
 // ids (null: none), real, h: a pair whose expert is `real` or beyond is an identity expert, whose output is the token's input row h[t] itself.
 // shared and h are of the model's type, all else 32-bit; all rows are contiguous and aligned for four of their elements.
 struct PairSum {
@@ -21,6 +22,7 @@ struct PairSum {
 // Columns c .. c + 3 of row t of width d.
 template <class T>
 __device__ __forceinline__ pair_f32x4 pair_sum4(const PairSum &p, size_t t, int c, int d) {
+#pragma clang fp contract(off)
     auto four = [](const void *base, size_t at) {
         const PairQuad<T> q = *(const PairQuad<T> *)((const T *)base + at);
         return pair_f32x4{to_f32(q.v[0]), to_f32(q.v[1]), to_f32(q.v[2]), to_f32(q.v[3])};
@@ -47,7 +49,7 @@ __device__ __forceinline__ pair_f32x4 pair_sum4(const PairSum &p, size_t t, int 
         for (int u = 0; u < 2; ++u) {
             if (k0 + u >= p.top) break;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(w[u], mine[u] ? own[e] : row[u][e], acc[e]);
+            for (int e = 0; e < 4; ++e) acc[e] += w[u] * (mine[u] ? own[e] : row[u][e]);
         }
     }
     if (p.shared || p.shared32) {

@@ -31,6 +31,24 @@ def pair_sum(n, d, dtype, top, base, wts, shared, identity, seed=0):
     return ops.PairSum(n, d, tdt, top, c(y), c(w), c(b), c(s), c(s32), c(gate), c(ids), c(h), real), want
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("base", [True, False])
+@pytest.mark.parametrize("shared", [None, "rows", "32"])
+@pytest.mark.parametrize("top", [1, 2, 3])
+def test_roundings_of_its_terms(dtype, base, shared, top):
+    """Bit for bit: an expert's product is rounded, then added; the shared expert's is added in one rounding."""
+    n, d = 7, 1028
+    p, _ = pair_sum(n, d, dtype, top, base, True, shared, True, seed=3)
+    c = lambda t: t.cpu() if t is not None else None
+    y, w, ids, h, own, gate = c(p.y).view(n, top, d), c(p.wts), c(p.ids), c(p.h).float(), c(p.shared if p.shared is not None else p.shared32), c(p.gate)
+    want = c(p.base).clone() if base else torch.zeros(n, d)
+    for k in range(top):
+        want = want + w[:, k:k + 1] * torch.where((ids[:, k] >= p.real)[:, None], h, y[:, k])
+    if shared:
+        want = (want.to(F64) + gate[:, None].to(F64) * own.to(F64)).float()          # (the product of two 32-bit numbers is exact in 64 bits)
+    assert torch.equal(p.rows().cpu(), want)
+
+
 # widths of one and of two pieces a thread at both numbers of threads, with rests; beyond and beside what the norms' kernels add up
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("n,d,top,base,wts,shared,identity", [
