@@ -7,6 +7,7 @@
 #include "common.h"
 
 constexpr int ARRAY_PIECES = 24;                 // pieces a launch takes (the arguments of a launch are a few hundred bytes)
+constexpr int ARRAY_BLOCKS = 64;                 // workgroups a launch has at most (each marks that it has read its part; 64 bring 256 KB over in one trip)
 
 // `rows` rows that begin at `at` and then every `stride` entries, in both arrays: the first `cols` of a row's `width` entries come over, zeros stand
 // behind them; all in units of 16 bytes
@@ -17,7 +18,7 @@ struct ArrayPieces { ArrayPiece p[ARRAY_PIECES]; };
 __device__ __forceinline__ uint64_t host_load(const uint64_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 
 __global__ void __launch_bounds__(256)
-step_arrays_kernel(const uint64_t *__restrict__ host, uint64_t *__restrict__ dev, ArrayPieces pieces, int n_pieces, int total) {
+step_arrays_kernel(const uint64_t *__restrict__ host, uint64_t *__restrict__ dev, ArrayPieces pieces, int n_pieces, int total, int *marks, int ticket) {
     for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
         int left = i, k = 0;
         while (k + 1 < n_pieces && left >= pieces.p[k].width * pieces.p[k].rows) { left -= pieces.p[k].width * pieces.p[k].rows; ++k; }
@@ -28,6 +29,10 @@ step_arrays_kernel(const uint64_t *__restrict__ host, uint64_t *__restrict__ dev
         dev[at] = lo;
         dev[at + 1] = hi;
     }
+    // The host's memory has been read (what was loaded is behind the barrier, as every wave has it in registers to store it): the host may write there again.  A mark
+    // costs the queue nothing, where an event behind every launch took 4 us.
+    __syncthreads();
+    if (marks && threadIdx.x == 0) __hip_atomic_store(marks + blockIdx.x, ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The address under which the device reads pinned host memory.
@@ -40,25 +45,35 @@ LCU_API int lcu_host_on_device(void *host, void **on_device) {
 
 // host, dev: arrays of `size` 32-bit entries, 16-byte aligned (host: as lcu_host_on_device names it).  pieces: n_pieces times (at, cols, rows, stride, width)
 // in entries, rows as they are and the others multiples of 4, cols <= width <= stride (of a single row: any stride): see ArrayPiece.
-LCU_API int lcu_step_arrays(const void *host, void *dev, long long size, const int *pieces, int n_pieces, hipStream_t stream) {
-    if (n_pieces < 0 || size < 0 || (n_pieces && (!host || !dev || !pieces)) || ((uintptr_t)host | (uintptr_t)dev) % 16) return LCU_BAD_ARGUMENT;
-    for (int done = 0; done < n_pieces;) {
+// marks (null: none): ARRAY_BLOCKS ints in pinned host memory, under their address on the device; *n_marks of them, as many as come back, hold `ticket` once all of `host`
+// that is wanted has been read.
+LCU_API int lcu_step_arrays(const void *host, void *dev, long long size, const int *pieces, int n_pieces, int *marks, int ticket, int *n_marks, hipStream_t stream) {
+    if (n_marks) *n_marks = 0;
+    if ((marks && !n_marks) || n_pieces < 0 || size < 0 || (n_pieces && (!host || !dev || !pieces)) || ((uintptr_t)host | (uintptr_t)dev) % 16) return LCU_BAD_ARGUMENT;
+    int end = 0;                                 // behind the last piece with anything in it: its launch, the last one, leaves the marks
+    for (int i = 0; i < n_pieces; ++i) {
+        const int *p = pieces + 5 * i, at = p[0], cols = p[1], rows = p[2], stride = p[3], width = p[4];
+        if (at < 0 || cols < 0 || rows < 0 || stride < 0 || width < cols || (at | cols | stride | width) % 4) return LCU_BAD_ARGUMENT;
+        if (width == 0 || rows == 0) continue;
+        if ((long long)at + (long long)(rows - 1) * stride + width > size || (rows > 1 && stride < width)) return LCU_BAD_ARGUMENT;
+        end = i + 1;
+    }
+    for (int done = 0; done < end;) {
         ArrayPieces a{};
         int n = 0;
         long long total = 0;
-        for (; n < ARRAY_PIECES && done < n_pieces; ++done) {
-            const int at = pieces[5 * done], cols = pieces[5 * done + 1], rows = pieces[5 * done + 2], stride = pieces[5 * done + 3], width = pieces[5 * done + 4];
-            if (at < 0 || cols < 0 || rows < 0 || stride < 0 || width < cols || (at | cols | stride | width) % 4) return LCU_BAD_ARGUMENT;
+        for (; n < ARRAY_PIECES && done < end; ++done) {
+            const int *p = pieces + 5 * done, rows = p[2], width = p[4];
             if (width == 0 || rows == 0) continue;
-            if ((long long)at + (long long)(rows - 1) * stride + width > size || (rows > 1 && stride < width)) return LCU_BAD_ARGUMENT;
-            a.p[n++] = ArrayPiece{at / 4, cols / 4, rows, stride / 4, width / 4};
+            a.p[n++] = ArrayPiece{p[0] / 4, p[1] / 4, rows, p[3] / 4, width / 4};
             total += (long long)(width / 4) * rows;
         }
-        if (!n) continue;
-        if (total > 0x7fffffffLL - 256 * 256) return LCU_BAD_ARGUMENT;
-        const long long blocks = (total + 255) / 256;
-        step_arrays_kernel<<<(unsigned)(blocks < 256 ? blocks : 256), 256, 0, stream>>>((const uint64_t *)host, (uint64_t *)dev, a, n, (int)total);
+        if (total > 0x7fffffffLL - ARRAY_BLOCKS * 256) return LCU_BAD_ARGUMENT;
+        const int blocks = total > ARRAY_BLOCKS * 256 ? ARRAY_BLOCKS : (int)((total + 255) / 256);
+        const bool last = done == end;
+        step_arrays_kernel<<<blocks, 256, 0, stream>>>((const uint64_t *)host, (uint64_t *)dev, a, n, (int)total, last ? marks : nullptr, ticket);
         LCU_LAUNCH_CHECK();
+        if (last && marks) *n_marks = blocks;
     }
     return LCU_OK;
 }

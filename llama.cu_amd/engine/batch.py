@@ -17,6 +17,7 @@ import torch
 
 from ..cache import CacheManager
 from ..kernels import ops
+from .host_reads import MARKS, HostReads
 
 
 @dataclass
@@ -87,9 +88,8 @@ class StepContext:
 class BatchBuilder:
     """Lays the arrays of a step out in a pinned host buffer and one device buffer of
     fixed capacity, so a step costs one launch that brings over what it uses of them, and the device addresses
-    never change (a captured graph can read them).  The steps take turns over ``RING`` host buffers, and an event is recorded once
-    in half a ring: recording one costs the queue 4 us, as much as a small kernel, and with several buffers the host need not wait for the
-    step before last to begin."""
+    never change (a captured graph can read them).  The steps take turns over ``RING`` host buffers, so that the host need not wait for the
+    step before last to begin; each says itself when it has been read (``HostReads``)."""
     RING = 8
 
     def __init__(self, cache: CacheManager, max_tokens: int, max_reqs: int, max_pages: Sequence[int],
@@ -116,12 +116,15 @@ class BatchBuilder:
             total += (size + 3) // 4 * 4
         pin = device.type == "cuda"
         self.dev = torch.zeros(total, dtype=torch.int32, device=device)
-        self._ring = torch.zeros((self.RING if pin else 1, total), dtype=torch.int32, pin_memory=pin)     # (one piece: pinning is slow)
-        self._seen_as = [ops.host_on_device(self._ring) + 4 * total * i for i in range(self.RING)] if pin else []
+        places = self.RING if pin else 1
+        self._reads = HostReads(torch.zeros(HostReads.entries(places, places * total), dtype=torch.int32, pin_memory=pin), places)     # (one piece: pinning is slow)
+        self._reads.belongs_to(self)
+        self._ring = self._reads.data.view(places, total)
+        base = ops.host_on_device(self._reads.memory) if pin else 0
+        self._marks_at = [base + 4 * MARKS * i for i in range(places)] if pin else []
+        self._seen_as = [base + 4 * (MARKS * places + total * i) for i in range(places)] if pin else []
         self._turn = 0                          # whose turn it is
         self._begun = False                     # whether the buffer whose turn it is may be written
-        self._read: List[List[torch.cuda.Event]] = [[], []]   # per half of the ring: behind the last reads of its buffers
-        self._stream: Optional[torch.cuda.Stream] = None      # where the half's buffers were read last, if no event stands behind that yet
         self._extras_now = set()                # the names that this step has asked for
 
     @property
@@ -135,13 +138,8 @@ class BatchBuilder:
 
     def _begin(self) -> None:
         """Wait until what the buffer whose turn it is held before has been read."""
-        if self._begun:
-            return
-        half = len(self._ring) // 2
-        if half and self._turn % half == 0:
-            for event in self._read[self._turn // half]:
-                event.synchronize()
-            self._read[self._turn // half] = []
+        if not self._begun:
+            self._reads.wait(self._turn)
         self._begun = True
 
     def _d(self, name: str, count: int) -> torch.Tensor:
@@ -185,18 +183,10 @@ class BatchBuilder:
             self.dev.copy_(self.host)
         else:
             stream = torch.cuda.current_stream(self.device)
-            half, turn = len(self._ring) // 2, self._turn
-            if self._stream is not None and self._stream != stream:        # (steps on several streams in turn)
-                self._read[turn // half].append(self._stream.record_event())
-            if torch.cuda.current_device() == self.device.index:
-                ops.step_arrays(self._seen_as[turn], self.dev, self._pieces())
-            else:
-                with torch.cuda.device(self.device):
-                    ops.step_arrays(self._seen_as[turn], self.dev, self._pieces())
-            self._stream = stream
-            if turn % half == half - 1:
-                self._read[turn // half].append(stream.record_event())
-                self._stream = None
+            turn, ticket = self._turn, self._reads.next_ticket()
+            with torch.cuda.device(self.device):
+                left = ops.step_arrays(self._seen_as[turn], self.dev, self._pieces(), self._marks_at[turn], ticket)
+            self._reads.launched(turn, left, ticket, stream)
             self._turn = (turn + 1) % len(self._ring)
         self._begun = False
         self._extras_now = set()
