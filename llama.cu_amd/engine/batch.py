@@ -125,6 +125,7 @@ class BatchBuilder:
         self._seen_as = [base + 4 * (MARKS * places + total * i) for i in range(places)] if pin else []
         self._turn = 0                          # whose turn it is
         self._begun = False                     # whether the buffer whose turn it is may be written
+        self._brought = False                   # whether its arrays have gone to the device
         self._extras_now = set()                # the names that this step has asked for
 
     @property
@@ -177,19 +178,19 @@ class BatchBuilder:
         return out + [whole(base + self._extras[name][0], self._extras[name][1]) for name in sorted(self._extras_now)]
 
     def upload(self) -> None:
-        """What the step uses of the arrays goes to the device (on the current stream)."""
+        """What the step uses of the arrays goes to the device (on the current stream); again, with what ``extra`` has added, if it has gone before."""
         self._begin()
         if not self._seen_as:
             self.dev.copy_(self.host)
         else:
             stream = torch.cuda.current_stream(self.device)
             turn, ticket = self._turn, self._reads.next_ticket()
+            if self._brought:
+                self._reads.wait(turn)
             with torch.cuda.device(self.device):
                 left = ops.step_arrays(self._seen_as[turn], self.dev, self._pieces(), self._marks_at[turn], ticket)
             self._reads.launched(turn, left, ticket, stream)
-            self._turn = (turn + 1) % len(self._ring)
-        self._begun = False
-        self._extras_now = set()
+        self._brought = True
 
     def build(self, req_ids: Sequence[int], tokens: Sequence[Sequence[int]], want: Sequence[Sequence[int]],
               vocab_size: int, feed: Sequence[tuple] = (), upload: bool = True) -> StepContext:
@@ -206,6 +207,9 @@ class BatchBuilder:
         if n > self.max_tokens or n_req > self.max_reqs:
             raise ValueError(f"step of {n} tokens / {n_req} requests exceeds the builder's capacity "
                              f"({self.max_tokens} / {self.max_reqs})")
+        if self._brought:                       # (the buffer stays the last step's until another step is built)
+            self._turn = (self._turn + 1) % len(self._ring)
+            self._begun = self._brought = False
         self._begin()
         self._extras_now = set()
         flat = [t for ts in tokens for t in ts]

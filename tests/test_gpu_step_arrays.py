@@ -132,6 +132,25 @@ def test_steps_that_queue_up_bring_their_own_arrays(ordered):
         assert tokens.tolist() == [(5 * k + j) % 50 for j in range(1 + k % 3)] and ctx.tolist() == [length], k
 
 
+def test_a_step_may_go_to_the_device_again():
+    """With what was added to its arrays after the first time, and with its other arrays as they were; the next step's come behind it."""
+    cache, builder = builder_of(96)
+    cache.add(0)
+    length = 0
+    for k in range(2 * builder.RING + 1):
+        tokens = [(11 * k + j) % 50 for j in range(1 + k % 2)]
+        length += len(tokens)
+        assert cache.reserve(0, length)
+        step = builder.build([0], [tokens], [[0]], 50)
+        cache.commit(0)
+        host, dev = step.extra("late", 8)
+        host[:8] = torch.arange(8, dtype=torch.int32) + 100 * k
+        step.tokens.zero_()                          # (what the second launch brings is not what the first one left)
+        builder.upload()
+        assert step.tokens.tolist() == tokens and step.ctx_len.tolist() == [length] and step.q_start.tolist() == [0, len(tokens)]
+        assert dev.tolist() == [100 * k + j for j in range(8)]
+
+
 @pytest.mark.parametrize("positions", [96, 90])
 def test_steps_in_turn_bring_their_own_arrays(positions):
     """More steps than the builder has room for, on two streams in turn, the host waiting for one when it goes on with the other: all arrays of each step are its own."""
