@@ -86,10 +86,11 @@ class StepContext:
 
 
 class BatchBuilder:
-    """Lays the arrays of a step out in a pinned host buffer and one device buffer of
-    fixed capacity, so a step costs one launch that brings over what it uses of them, and the device addresses
-    never change (a captured graph can read them).  The steps take turns over ``RING`` host buffers, so that the host need not wait for the
-    step before last to begin; each says itself when it has been read (``HostReads``)."""
+    """Lays the arrays of a step out in host memory and one device buffer of
+    fixed capacity, so a step costs one launch that brings over what it uses of them, and the addresses
+    never change (a captured graph can read the device's).  What a step uses is packed into pinned memory (``HostReads``) of the size of the arrays, where
+    ``RING`` steps find room one behind the other if they are small, so that the host need not wait for the step before last to begin.  (Whole arrays for each
+    of eight steps were eight times as much to pin, and the memory of small models came back from a graph's capture 2.5 ms later.)"""
     RING = 8
 
     def __init__(self, cache: CacheManager, max_tokens: int, max_reqs: int, max_pages: Sequence[int],
@@ -116,32 +117,17 @@ class BatchBuilder:
             total += (size + 3) // 4 * 4
         pin = device.type == "cuda"
         self.dev = torch.zeros(total, dtype=torch.int32, device=device)
-        places = self.RING if pin else 1
-        self._reads = HostReads(torch.zeros(HostReads.entries(places, places * total), dtype=torch.int32, pin_memory=pin), places)     # (one piece: pinning is slow)
-        self._reads.belongs_to(self)
-        self._ring = self._reads.data.view(places, total)
-        base = ops.host_on_device(self._reads.memory) if pin else 0
-        self._marks_at = [base + 4 * MARKS * i for i in range(places)] if pin else []
-        self._seen_as = [base + 4 * (MARKS * places + total * i) for i in range(places)] if pin else []
-        self._turn = 0                          # whose turn it is
-        self._begun = False                     # whether the buffer whose turn it is may be written
-        self._brought = False                   # whether its arrays have gone to the device
-        self._extras_now = set()                # the names that this step has asked for
-
-    @property
-    def host(self) -> torch.Tensor:
-        """The buffer of the step that is being built."""
-        return self._ring[self._turn]
+        self.host = torch.zeros(total, dtype=torch.int32)
+        self._reads: Optional[HostReads] = None
+        if pin:
+            self._reads = HostReads(torch.zeros(HostReads.entries(self.RING, total), dtype=torch.int32, pin_memory=True), self.RING)
+            self._reads.belongs_to(self)
+            self._pinned_at = ops.host_on_device(self._reads.memory)
+        self._used, self._used_tables = [], []  # what the step that was built last uses of the arrays
 
     def _h(self, name: str) -> torch.Tensor:
         o, s = self.offsets[name]
         return self.host[o:o + s]
-
-    def _begin(self) -> None:
-        """Wait until what the buffer whose turn it is held before has been read."""
-        if not self._begun:
-            self._reads.wait(self._turn)
-        self._begun = True
 
     def _d(self, name: str, count: int) -> torch.Tensor:
         o, s = self.offsets[name]
@@ -150,8 +136,6 @@ class BatchBuilder:
     def extra(self, name: str, size: int):
         """``(host, device)`` views of ``size`` entries that ``name`` owns from its first call on (the same
         addresses in every step)."""
-        self._begin()
-        self._extras_now.add(name)
         at = self._extras.get(name)
         if at is None:
             if self._extra_used + size > self.extra_ints:
@@ -174,23 +158,22 @@ class BatchBuilder:
             at, mp = self.offsets[f"block_table{g}"][0], self.max_pages[g]
             # of every request's row the pages that the longest context reaches (rows that do not begin on 16 bytes: everything)
             out.append((at, min((cols + 3) // 4 * 4, mp), rows, mp, mp) if mp % 4 == 0 else whole(at, rows * mp))
-        base = self.offsets["extra"][0]
-        return out + [whole(base + self._extras[name][0], self._extras[name][1]) for name in sorted(self._extras_now)]
+        # what the parts have asked for so far, whether they ask again for this step or write where they wrote before
+        return out + ([whole(self.offsets["extra"][0], self._extra_used)] if self._extra_used else [])
 
     def upload(self) -> None:
         """What the step uses of the arrays goes to the device (on the current stream); again, with what ``extra`` has added, if it has gone before."""
-        self._begin()
-        if not self._seen_as:
+        if self._reads is None:
             self.dev.copy_(self.host)
-        else:
-            stream = torch.cuda.current_stream(self.device)
-            turn, ticket = self._turn, self._reads.next_ticket()
-            if self._brought:
-                self._reads.wait(turn)
-            with torch.cuda.device(self.device):
-                left = ops.step_arrays(self._seen_as[turn], self.dev, self._pieces(), self._marks_at[turn], ticket)
-            self._reads.launched(turn, left, ticket, stream)
-        self._brought = True
+            return
+        reads, pieces = self._reads, self._pieces()
+        size = sum(cols * rows for _, cols, rows, _, _ in pieces)
+        place, start = reads.room(size)
+        ticket, stream = reads.next_ticket(), torch.cuda.current_stream(self.device)
+        with torch.cuda.device(self.device):
+            marks = ops.step_arrays(self._pinned_at + 4 * (reads.memory.numel() - reads.data.numel() + start), self.dev, pieces, self._pinned_at + 4 * MARKS * place, ticket,
+                                    self.host, reads.data[start:start + size])
+        reads.launched(place, marks, ticket, stream)
 
     def build(self, req_ids: Sequence[int], tokens: Sequence[Sequence[int]], want: Sequence[Sequence[int]],
               vocab_size: int, feed: Sequence[tuple] = (), upload: bool = True) -> StepContext:
@@ -207,11 +190,6 @@ class BatchBuilder:
         if n > self.max_tokens or n_req > self.max_reqs:
             raise ValueError(f"step of {n} tokens / {n_req} requests exceeds the builder's capacity "
                              f"({self.max_tokens} / {self.max_reqs})")
-        if self._brought:                       # (the buffer stays the last step's until another step is built)
-            self._turn = (self._turn + 1) % len(self._ring)
-            self._begun = self._brought = False
-        self._begin()
-        self._extras_now = set()
         flat = [t for ts in tokens for t in ts]
         lo, hi = min(flat), max(flat)
         if lo < 0 or hi >= vocab_size:

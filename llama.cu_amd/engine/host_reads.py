@@ -42,8 +42,7 @@ def _leave(reads: "HostReads") -> None:
 
 
 class HostReads:
-    """``places`` parts of the int32 tensor ``memory`` (pinned), each of which one launch reads at a time.  ``data``: the tensor behind the
-    marks; who shares it out among the places is the owner's business."""
+    """The int32 tensor ``memory`` (pinned): marks for ``places`` launches, and ``data`` behind them, of which each launch reads a part (``room``)."""
 
     def __init__(self, memory: torch.Tensor, places: int):
         _sweep()
@@ -51,6 +50,8 @@ class HostReads:
         self.data = memory[self.places * MARKS:]
         self._marks = (ctypes.c_int * (self.places * MARKS)).from_address(memory.data_ptr())
         self._ticket = 0
+        self._rooms: collections.deque = collections.deque()      # (place, start, end) of the parts that were given out last, the oldest first
+        self._next = self._head = 0
         self._awaited: List[Optional[Tuple[int, int, object]]] = [None] * self.places     # (marks, ticket, stream) of the launch that reads the place
 
     @staticmethod
@@ -62,6 +63,20 @@ class HostReads:
         """The memory stays until the launches that are queued when ``owner`` goes have read it.  (Nothing is asked of the GPU then: an owner may go while
         a graph is captured, and nobody waits for it.)"""
         weakref.finalize(owner, _leave, self).atexit = False
+
+    def room(self, size: int) -> Tuple[int, int]:
+        """``(place, start)``: so many entries of ``data`` (16-byte pieces) for the next launch, behind the last ones or at the beginning again.  Waits for the launches that read there
+        before, oldest first, and for the oldest of all if as many as there are places are still to read."""
+        size = (size + 3) // 4 * 4
+        if size > self.data.numel():
+            raise ValueError(f"{size} entries do not fit in the {self.data.numel()} that there are")
+        start = self._head if self._head + size <= self.data.numel() else 0
+        while len(self._rooms) == self.places or any(a < start + size and start < b for _, a, b in self._rooms):
+            self.wait(self._rooms.popleft()[0])
+        place = self._next
+        self._rooms.append((place, start, start + size))
+        self._next, self._head = (place + 1) % self.places, start + size
+        return place, start
 
     def next_ticket(self) -> int:
         self._ticket = self._ticket % 0x7fffffff + 1
@@ -94,4 +109,5 @@ class HostReads:
                 continue
             self._awaited[place][2].synchronize()        # a step of more than a second, or one that failed
             if not self.done(place):
+                self._awaited[place] = None
                 raise RuntimeError("a step's arrays were never read: its launch was recorded and not run, or failed")

@@ -142,17 +142,24 @@ def host_on_device(host: torch.Tensor) -> int:
     return at.value
 
 
-def step_arrays(host: int, dev: torch.Tensor, pieces, marks: int = 0, ticket: int = 0) -> int:
+def step_arrays(host: int, dev: torch.Tensor, pieces, marks: int = 0, ticket: int = 0, arrays: Optional[torch.Tensor] = None, packed: Optional[torch.Tensor] = None) -> int:
     """Pieces of an int32 array in pinned host memory (``host``: its address as ``host_on_device`` gives it) to the same places of ``dev``, on
     the current stream: ``pieces`` holds ``(at, cols, rows, stride, width)`` in entries (multiples of 4, but for ``rows``): ``rows`` rows
     that begin at entry ``at`` and then every ``stride``, of whose ``width`` entries the first ``cols`` come over and the others become zero.
+    ``arrays`` (int32, in ordinary host memory, as large as ``dev``): the pieces are its own; what comes over is copied first, one piece behind the
+    other, to ``packed``, the pinned memory that is at ``host``.
     The allocator of pinned memory knows nothing of this read.  ``marks``: where ``HostReads`` keeps the 64 marks of the memory (an address as
     ``host_on_device`` gives it); as many of them as are returned hold ``ticket`` once the memory has been read."""
     _gpu(dev)
     _i32(dev, "step_arrays dev")
+    if arrays is not None:
+        _i32(arrays, "step_arrays arrays", dev.numel()); _i32(packed, "step_arrays packed")
+        if arrays.is_cuda or packed.is_cuda:
+            raise KernelError("step_arrays: the arrays and the memory they are packed into lie on the host")
     flat = [v for piece in pieces for v in piece]
     left = ctypes.c_int(0)
-    _check(build.load("step_arrays").lcu_step_arrays(ctypes.c_void_p(host), _ptr(dev), ctypes.c_longlong(dev.numel()), (ctypes.c_int * len(flat))(*flat), len(pieces),
+    _check(build.load("step_arrays").lcu_step_arrays(_ptr(arrays), _ptr(packed), ctypes.c_longlong(packed.numel() if arrays is not None else 0), ctypes.c_void_p(host), _ptr(dev),
+                                                     ctypes.c_longlong(dev.numel()), (ctypes.c_int * len(flat))(*flat), len(pieces),
                                                      ctypes.c_void_p(marks), int(ticket), ctypes.byref(left), _stream()), "step_arrays")
     return left.value
 

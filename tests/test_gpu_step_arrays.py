@@ -25,6 +25,33 @@ def test_pieces_come_over_and_nothing_else_changes(pieces):
         assert torch.equal(dev.cpu(), want)
 
 
+@pytest.mark.parametrize("pieces", [[(0, 4, 1, 0, 4)], [(0, 1020, 1, 0, 1024), (1024, 4, 7, 12, 8), (1200, 0, 2, 8, 8), (2000, 2096, 1, 0, 2096)],
+                                    [(8 * i, 4, 1, 0, 4 + 4 * (i % 2)) for i in range(61)], [(0, 262140, 1, 0, 262140)], []])
+def test_pieces_of_ordinary_memory_come_over_packed(pieces):
+    """What stands in pinned memory is the pieces, one behind the other, and no more."""
+    from llama_cu_amd.kernels import ops
+    n = 262144
+    size = sum(cols * rows for _, cols, rows, _, _ in pieces)
+    host = torch.arange(1, n + 1, dtype=torch.int32)
+    pinned = torch.zeros(n + 8, dtype=torch.int32).pin_memory()
+    dev = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+    at = ops.host_on_device(pinned)
+    for turn in range(3):
+        host += turn
+        want = dev.cpu()
+        for a, cols, rows, stride, width in pieces:
+            for r in range(rows):
+                want[a + r * stride:a + r * stride + cols] = host[a + r * stride:a + r * stride + cols]
+                want[a + r * stride + cols:a + r * stride + width] = 0
+        ops.step_arrays(at + 16, dev, pieces, arrays=host, packed=pinned[4:4 + size])
+        torch.cuda.synchronize()
+        assert torch.equal(dev.cpu(), want)
+        assert not pinned[:4].any() and not pinned[4 + size:].any()
+    if size:
+        with pytest.raises(ops.KernelError):
+            ops.step_arrays(at + 16, dev, pieces, arrays=host, packed=pinned[4:size])
+
+
 def test_pieces_outside_the_array_are_refused():
     from llama_cu_amd.kernels import ops
     host = torch.zeros(64, dtype=torch.int32).pin_memory()

@@ -76,6 +76,38 @@ def test_waiting(monkeypatch):
         r.wait(1)
 
 
+def test_room_is_given_again_when_it_has_been_read():
+    """Parts of all sizes in turn: none overlaps one that is still to be read, and nobody waits who need not."""
+    gen = torch.Generator().manual_seed(5)
+    r = reads_of(4, 64)
+    waited, queued = [], []                           # queued: (place, start, end, ticket), read from the front on
+
+    def wait(place):
+        if not r.done(place):
+            waited.append(place)
+            while not r.done(place):
+                p, _, _, t = queued.pop(0)
+                mark(r, p, 1, t)
+    r.wait = wait
+    for turn in range(400):
+        size = int(torch.randint(1, 65 if turn % 7 == 0 else 20, (1,), generator=gen))
+        before = list(queued)
+        del waited[:]
+        place, start = r.room(size)
+        assert start % 4 == 0 and start + size <= 64
+        assert all(place != p and (end <= start or start + size <= a) for p, a, end, _ in queued)
+        assert not waited or len(before) == 4 or any(a < start + size and start < end for _, a, end, _ in before)
+        t = r.next_ticket()
+        r.launched(place, 1, t, None)
+        queued.append((place, start, start + size, t))
+        if turn % 3 == 0:                             # the oldest is read
+            p, _, _, t = queued.pop(0)
+            mark(r, p, 1, t)
+    with pytest.raises(ValueError):
+        r.room(65)
+    assert reads_of(2, 64).room(64) == (0, 0)
+
+
 def test_memory_stays_until_it_has_been_read():
     host_reads._sweep()
     before = len(host_reads._left)
