@@ -123,11 +123,13 @@ class BatchBuilder:
             self._reads = HostReads(torch.zeros(HostReads.entries(self.RING, total), dtype=torch.int32, pin_memory=True), self.RING)
             self._reads.belongs_to(self)
             self._pinned_at = ops.host_on_device(self._reads.memory)
+        self._views = {name: self.host[o:o + s] for name, (o, s) in self.offsets.items()}
+        self._tables = [f"block_table{g}" for g in range(len(self.max_pages))]
+        self._slots = [f"slots{g}" for g in range(len(self.max_pages))]
         self._used, self._used_tables = [], []  # what the step that was built last uses of the arrays
 
     def _h(self, name: str) -> torch.Tensor:
-        o, s = self.offsets[name]
-        return self.host[o:o + s]
+        return self._views[name]
 
     def _d(self, name: str, count: int) -> torch.Tensor:
         o, s = self.offsets[name]
@@ -149,30 +151,47 @@ class BatchBuilder:
         return self.host[o:o + size], self.dev[o:o + size]
 
     def _pieces(self):
-        """What the step uses of the arrays, as ``ops.step_arrays`` takes it."""
-        def whole(at, count):
-            count = (count + 3) // 4 * 4
-            return (at, count, 1, 0, count)
-        out = [whole(self.offsets[name][0], count) for name, count in self._used if count]
-        for g, (rows, cols) in enumerate(self._used_tables):
-            at, mp = self.offsets[f"block_table{g}"][0], self.max_pages[g]
-            # of every request's row the pages that the longest context reaches (rows that do not begin on 16 bytes: everything)
-            out.append((at, min((cols + 3) // 4 * 4, mp), rows, mp, mp) if mp % 4 == 0 else whole(at, rows * mp))
-        # what the parts have asked for so far, whether they ask again for this step or write where they wrote before
-        return out + ([whole(self.offsets["extra"][0], self._extra_used)] if self._extra_used else [])
+        """What the step uses of the arrays, as ``ops.step_arrays`` takes it, and how many entries these are."""
+        out, size = [], 0
+        for name, count in self._used:
+            if count:
+                count = (count + 3) & -4
+                out += (self.offsets[name][0], count, 1, 0, count)
+                size += count
+        for name, mp, (rows, cols) in zip(self._tables, self.max_pages, self._used_tables):
+            at = self.offsets[name][0]
+            if mp % 4 == 0:
+                # of every request's row the pages that the longest context reaches
+                cols = min((cols + 3) & -4, mp)
+                out += (at, cols, rows, mp, mp)
+                size += cols * rows
+            else:
+                # (rows that do not begin on 16 bytes: everything)
+                count = (rows * mp + 3) & -4
+                out += (at, count, 1, 0, count)
+                size += count
+        if self._extra_used:
+            # what the parts have asked for so far, whether they ask again for this step or write where they wrote before
+            out += (self.offsets["extra"][0], self._extra_used, 1, 0, self._extra_used)
+            size += self._extra_used
+        return out, size
 
     def upload(self) -> None:
         """What the step uses of the arrays goes to the device (on the current stream); again, with what ``extra`` has added, if it has gone before."""
         if self._reads is None:
             self.dev.copy_(self.host)
             return
-        reads, pieces = self._reads, self._pieces()
-        size = sum(cols * rows for _, cols, rows, _, _ in pieces)
+        reads = self._reads
+        pieces, size = self._pieces()
         place, start = reads.room(size)
         ticket, stream = reads.next_ticket(), torch.cuda.current_stream(self.device)
-        with torch.cuda.device(self.device):
-            marks = ops.step_arrays(self._pinned_at + 4 * (reads.memory.numel() - reads.data.numel() + start), self.dev, pieces, self._pinned_at + 4 * MARKS * place, ticket,
-                                    self.host, reads.data[start:start + size])
+        args = (self._pinned_at + 4 * (reads.memory.numel() - reads.data.numel() + start), self.dev, pieces, self._pinned_at + 4 * MARKS * place, ticket, self.host,
+                reads.data[start:start + size])
+        if torch.cuda.current_device() == self.device.index:
+            marks = ops.step_arrays(*args)
+        else:
+            with torch.cuda.device(self.device):
+                marks = ops.step_arrays(*args)
         reads.launched(place, marks, ticket, stream)
 
     def build(self, req_ids: Sequence[int], tokens: Sequence[Sequence[int]], want: Sequence[Sequence[int]],
@@ -214,17 +233,17 @@ class BatchBuilder:
                 ends.append(at - 1)
             self._h("feed_src")[:len(feed)] = torch.tensor([f[0] for f in feed], dtype=torch.int32)
             self._h("feed_dst")[:len(feed)] = torch.tensor([ends[f[1]] for f in feed], dtype=torch.int32)
-        ptr = lambda name: self._h(name).data_ptr()
+        base = self.host.data_ptr()
+        ptr = lambda name: base + 4 * self.offsets[name][0]
         self.cache.fill_batch(req_ids, n_new, ptr("positions"), ptr("req_of_token"), ptr("q_start"), ptr("ctx_len"),
-                              ptr("state_slot"), [ptr(f"block_table{g}") for g in range(len(self.max_pages))],
-                              self.max_pages, [ptr(f"slots{g}") for g in range(len(self.max_pages))])
+                              ptr("state_slot"), [ptr(name) for name in self._tables], self.max_pages, [ptr(name) for name in self._slots])
         ctx_lens = self._h("ctx_len")[:n_req].tolist()
         self._h("decode_order")[:n_req] = torch.tensor(sorted(range(n_req), key=lambda i: -ctx_lens[i]), dtype=torch.int32)
         state_slots = self._h("state_slot")[:n_req].tolist()
         longest = max(ctx_lens)
         self._used = [("tokens", n), ("positions", n), ("req_of_token", n), ("logit_rows", len(rows)), ("q_start", n_req + 1), ("ctx_len", n_req),
                       ("state_slot", n_req), ("decode_order", n_req), ("feed_src", len(feed)), ("feed_dst", len(feed))]
-        self._used += [(f"slots{g}", n) for g in range(len(self.max_pages))]
+        self._used += [(name, n) for name in self._slots]
         self._used_tables = [(n_req, -(-longest // group.page_size)) for group in self.cache.groups]
         if upload:
             self.upload()

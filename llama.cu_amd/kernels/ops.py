@@ -144,7 +144,7 @@ def host_on_device(host: torch.Tensor) -> int:
 
 def step_arrays(host: int, dev: torch.Tensor, pieces, marks: int = 0, ticket: int = 0, arrays: Optional[torch.Tensor] = None, packed: Optional[torch.Tensor] = None) -> int:
     """Pieces of an int32 array in pinned host memory (``host``: its address as ``host_on_device`` gives it) to the same places of ``dev``, on
-    the current stream: ``pieces`` holds ``(at, cols, rows, stride, width)`` in entries (multiples of 4, but for ``rows``): ``rows`` rows
+    the current stream: ``pieces`` holds ``(at, cols, rows, stride, width)``, as tuples or one behind the other, in entries (multiples of 4, but for ``rows``): ``rows`` rows
     that begin at entry ``at`` and then every ``stride``, of whose ``width`` entries the first ``cols`` come over and the others become zero.
     ``arrays`` (int32, in ordinary host memory, as large as ``dev``): the pieces are its own; what comes over is copied first, one piece behind the
     other, to ``packed``, the pinned memory that is at ``host``.
@@ -156,10 +156,10 @@ def step_arrays(host: int, dev: torch.Tensor, pieces, marks: int = 0, ticket: in
         _i32(arrays, "step_arrays arrays", dev.numel()); _i32(packed, "step_arrays packed")
         if arrays.is_cuda or packed.is_cuda:
             raise KernelError("step_arrays: the arrays and the memory they are packed into lie on the host")
-    flat = [v for piece in pieces for v in piece]
+    flat = pieces if pieces and isinstance(pieces[0], int) else [v for piece in pieces for v in piece]
     left = ctypes.c_int(0)
     _check(build.load("step_arrays").lcu_step_arrays(_ptr(arrays), _ptr(packed), ctypes.c_longlong(packed.numel() if arrays is not None else 0), ctypes.c_void_p(host), _ptr(dev),
-                                                     ctypes.c_longlong(dev.numel()), (ctypes.c_int * len(flat))(*flat), len(pieces),
+                                                     ctypes.c_longlong(dev.numel()), (ctypes.c_int * len(flat))(*flat), len(flat) // 5,
                                                      ctypes.c_void_p(marks), int(ticket), ctypes.byref(left), _stream()), "step_arrays")
     return left.value
 
