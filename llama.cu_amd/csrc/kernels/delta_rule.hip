@@ -519,6 +519,19 @@ static bool single_sizes(int heads, int dk, int dv) {
 static bool past_caches(int n_req, int heads, int dk, int dv) { return (long long)n_req * heads * dk * dv * 4 >= (48ll << 20); }
 LCU_API int lcu_delta_single_takes(int heads, int dk, int dv) { return single_sizes(heads, dk, dv); }
 
+// Whether the one kernel takes less time than the three.  Where heads have few columns its workgroups, eight on a compute unit at a time, have little to do behind what each makes
+// anew, the decay's product over the rank above all, and from some thousands of them on the kernels that share that win.  64 heads of 64 x 4, rank 8: 256 requests
+// 78 us, with three kernels 46, 64 requests 23 and 19, 16 requests 8.3 and 9.5; 32 heads of 32 x 16, rank 64: 96 requests 16 and 18, 256 requests 35 and 33; 32 of 32 x 32,
+// rank 512, 256 requests: 79 and 70, rank 64 36 and 54.  And where a few workgroups walk the most columns behind the longest ranks: 4 heads of
+// 128 x 512, rank 512, one request 19.7 and 16.2, rank 64 12.0 and 13.3, 32 workgroups 21.3 and 26.6.
+LCU_API int lcu_delta_single_pays(int n_req, int heads, int dk, int dv, int rank) {
+    const long long items = (long long)n_req * heads;
+    const bool long_rank = rank > 256;
+    if (dv <= 16) return long_rank ? items * dk < 65536 : dv >= 12 ? items <= 4096 : items * dk <= 65536;
+    if (dv < 32 || (dv == 32 && dk < 64)) return !long_rank || items <= 3072;
+    return !(long_rank && dk * dv > 128 * 384 && items <= 8);
+}
+
 // lcu_delta_rule for a step in which every request feeds one token (row r is request r's), where lcu_delta_single_takes says so; state 16-byte aligned.
 LCU_API int lcu_delta_single(const void *proj, int type, int row_stride, int off_r, int off_k, int off_v, int off_g, int off_a, int off_l,
                              const float *w2, const float *w0, const float *a_bias, const float *weight, float *state, void *out, const int *ctx_len,
@@ -765,6 +778,15 @@ gated_delta_single_kernel(const float *__restrict__ prep, const float *__restric
 
 LCU_API int lcu_gated_delta_single_takes(int heads, int qk_heads, int dk, int dv, int taps, long long slot_stride) {
     return single_sizes(heads, dk, dv) && qk_heads > 0 && heads % qk_heads == 0 && heads / qk_heads <= SINGLE_MAX_GROUP && taps >= 1 && taps <= SINGLE_MAX_TAPS && slot_stride % 4 == 0;
+}
+
+// Whether they take less time than the convolution's two kernels and the rule's three.  Not, as above, with few columns and many workgroups (16 heads of 128 x 4 with 4 for
+// queries and keys, with the products: 128 requests 28 us and 26, 32 of 128 x 16, 96 requests 41 and 41, 16 of 64 x 12, 128 requests 23 and 26), nor where a few workgroups have
+// the convolution of many channels each (8 heads of 128 x 512 with one for queries and keys: one request 30 and 24, 8 requests 35 and 34; with two 27 and 24, four requests 29 and 30).
+LCU_API int lcu_gated_delta_single_pays(int n_req, int heads, int qk_heads, int dk, int dv) {
+    const long long items = (long long)n_req * heads, channels = (long long)(heads / qk_heads) * dv + 2 * dk;
+    if (dv <= 16 && !(dv >= 12 ? dk <= 64 || items <= 2048 : items * dk <= 131072)) return 0;
+    return channels < 2304 || items * 64 >= channels;
 }
 
 // lcu_causal_conv (silu, no bias, over the rows' first 2 * qk_heads * dk + heads * dv columns) and lcu_gated_delta_rule for a step in which every request

@@ -1501,7 +1501,8 @@ def delta_rule(proj: torch.Tensor, offsets: Dict[str, int], w2_t: torch.Tensor, 
     if out.shape != (n, hv) or out.dtype != proj.dtype or not out.is_contiguous():
         raise KernelError("delta_rule out: wrong shape, type or layout")
     lib = build.load("delta_rule")
-    if step.decode_only and n == step.n_req and state.data_ptr() % 16 == 0 and lib.lcu_delta_single_takes(heads, key_dim, value_dim):
+    if step.decode_only and n == step.n_req and state.data_ptr() % 16 == 0 and lib.lcu_delta_single_takes(heads, key_dim, value_dim) \
+            and lib.lcu_delta_single_pays(n, heads, key_dim, value_dim, rank):
         _check(lib.lcu_delta_single(_ptr(proj), _type(proj, "delta projections"), proj.stride(0), offsets["r"], offsets["k"], offsets["v"],
                                     offsets["g"], offsets["a"], offsets["l"], _ptr(w2_t), _ptr(w0), _ptr(a_bias), _ptr(weight), _ptr(state), _ptr(out),
                                     _ptr(step.ctx_len), _ptr(step.state_slot), n, heads, key_dim, value_dim, rank, ctypes.c_float(eps), _stream()), "delta_single")
@@ -2339,9 +2340,11 @@ def gated_delta_rule(qkv: torch.Tensor, rows: torch.Tensor, off_a: int, off_b: i
 
 
 def gated_delta_single_takes(step, state: torch.Tensor, heads: int, qk_heads: int, key_dim: int, value_dim: int, taps: int) -> bool:
-    """Whether ``gated_delta_single`` runs this step: every request feeds one token, and the sizes are its kernels'."""
-    return bool(step.decode_only and step.n == step.n_req and state.data_ptr() % 16 == 0 and build.load("delta_rule").lcu_gated_delta_single_takes(
-        heads, qk_heads, key_dim, value_dim, taps, ctypes.c_longlong(state.stride(0))))
+    """Whether ``gated_delta_single`` runs this step: every request feeds one token, the sizes are its kernels', and they take less time than the others."""
+    lib = build.load("delta_rule")
+    return bool(step.decode_only and step.n == step.n_req and state.data_ptr() % 16 == 0
+                and lib.lcu_gated_delta_single_takes(heads, qk_heads, key_dim, value_dim, taps, ctypes.c_longlong(state.stride(0)))
+                and lib.lcu_gated_delta_single_pays(step.n, heads, qk_heads, key_dim, value_dim))
 
 
 def gated_delta_single(rows: torch.Tensor, off_a: int, off_b: int, off_g: int, conv_w: torch.Tensor, inputs: Optional[torch.Tensor], a_log: torch.Tensor,

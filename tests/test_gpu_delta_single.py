@@ -96,3 +96,38 @@ def test_states_that_no_cache_holds():
     for k in range(2):
         assert torch.equal(got[k], torch.cat([h[k] for h in halves]))
     assert torch.equal(a, b) and torch.equal(slots, both)
+
+
+def test_steps_that_the_other_kernels_take_in_less_time():
+    """Many heads of few columns, and few workgroups with the longest columns behind long ranks or the convolution of many channels: both sides of the lines."""
+    from llama_cu_amd.kernels import build, ops
+    lib = build.load("delta_rule")
+    for (n, heads, dk, dv, rank), pays in [((200, 16, 128, 128, 64), 1), ((256, 64, 64, 4, 8), 0), ((16, 64, 64, 4, 8), 1), ((64, 64, 32, 16, 64), 1), ((65, 64, 32, 16, 64), 0),
+                                           ((64, 16, 64, 16, 512), 0), ((63, 16, 64, 16, 512), 1), ((256, 32, 32, 32, 512), 0), ((256, 32, 32, 32, 256), 1), ((96, 32, 32, 32, 512), 1),
+                                           ((256, 32, 128, 32, 512), 1), ((1, 8, 128, 512, 512), 0), ((1, 9, 128, 512, 512), 1), ((1, 8, 128, 512, 256), 1), ((1, 1, 128, 384, 512), 1)]:
+        assert lib.lcu_delta_single_pays(n, heads, dk, dv, rank) == pays, (n, heads, dk, dv, rank)
+    for (n, heads, qk_heads, dk, dv), pays in [((1, 32, 16, 128, 128), 1), ((200, 8, 2, 128, 128), 1), ((256, 64, 16, 64, 4), 0), ((32, 64, 16, 64, 4), 1), ((128, 16, 4, 128, 16), 1),
+                                               ((129, 16, 4, 128, 16), 0), ((256, 64, 64, 64, 16), 1), ((1, 8, 1, 128, 512), 0), ((8, 8, 1, 128, 512), 0), ((9, 8, 1, 128, 512), 1),
+                                               ((1, 8, 2, 128, 512), 0), ((5, 8, 2, 128, 512), 1), ((1, 8, 8, 128, 512), 1)]:
+        assert lib.lcu_gated_delta_single_pays(n, heads, qk_heads, dk, dv) == pays, (n, heads, qk_heads, dk, dv)
+    state = torch.zeros(64, 64, 64, 4, device="cuda")
+    assert ops.gated_delta_single_takes(hand_step([1] * 32, [2] * 32, list(range(32))), state, 64, 16, 64, 4, 4)
+    assert not ops.gated_delta_single_takes(hand_step([1] * 64, [2] * 64, list(range(64))), state, 64, 16, 64, 4, 4)
+
+
+@pytest.mark.parametrize("n,part,heads,dk,dv,rank", [(65, 13, 64, 32, 4, 5), (9, 3, 2, 128, 512, 300)])
+def test_single_tokens_that_go_the_other_way(n, part, heads, dk, dv, rank):
+    """Of a step and its parts one side goes through the one kernel, the other through the three: the same bits."""
+    from llama_cu_amd.kernels import build, ops
+    lib = build.load("delta_rule")
+    assert lib.lcu_delta_single_pays(n, heads, dk, dv, rank) != lib.lcu_delta_single_pays(part, heads, dk, dv, rank)
+    hk, hv = heads * dk, heads * dv
+    off = {"r": 0, "k": hk, "v": 2 * hk, "g": 2 * hk + hv, "a": 2 * hk + 2 * hv, "l": 3 * hk + 2 * hv}
+    args = (rnd(rank, hk, seed=3).cuda(), rnd(hk, seed=4).cuda(), rnd(hk, seed=5).cuda(), (rnd(hv, seed=6) + 1).cuda())
+    rows = rnd(n, 3 * hk + 2 * hv + rank, seed=7).cuda()
+    a = rnd(n, heads, dk, dv, seed=8).cuda()
+    b, ctx = a.clone(), [1 + r % 3 for r in range(n)]
+    got = ops.delta_rule(rows, off, *args, a, hand_step([1] * n, ctx, list(range(n))), heads, dk, dv, 1e-4)
+    want = torch.cat([ops.delta_rule(rows[f:f + part].contiguous(), off, *args, b, hand_step([1] * part, ctx[f:f + part], list(range(f, f + part))), heads, dk, dv, 1e-4)
+                      for f in range(0, n, part)])
+    assert torch.equal(got, want) and torch.equal(a, b)
