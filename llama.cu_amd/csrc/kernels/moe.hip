@@ -496,7 +496,7 @@ moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__
     }
 }
 
-// Many rows an expert (prompts): tiles of up to 96 or 128 rows; a block of four waves takes a tile and 128 features, a wave 32 of them with all
+// Many rows an expert (prompts): tiles of up to 32, 64, 96 or 128 rows; a block of four waves takes a tile and 128 features, a wave 32 of them with all
 // rows.  The rows go through LDS in steps of 128 bytes of k, in two buffers in turn with one barrier a step; no two waves want the same piece of the
 // matrix, so each loads its own straight into registers.  Both are two steps ahead.  MT: tiles of 16 rows that are multiplied.
 // What bounds it are the turns of loads, LDS and barrier of the two blocks that a compute unit holds (half the matrix instructions take as long) and, up
@@ -695,12 +695,35 @@ LCU_API int lcu_moe_combine(float *out, const PairSum *p, int type, int n, int d
 }
 
 // Rows of a tile for n * top pairs over so many experts: while an expert has 16 rows or fewer on average the kernel for few rows, with no
-// tiles up to MOE_LIST pairs (0; MOE_LIST_F32 in 32 bits) and tiles of 16 beyond.  Else 96 (128 rows: 2,014 tokens of two on 16 experts 176 -> 195 us, 512 on 8 experts of 4096 x 4096 241 -> 257; more work in a block leaves more
-// compute units without any at the end), but 128 where an expert's rows on average are just more than a tile of 96 and would make two (100 rows: 84 -> 66 us).  The caller sizes its
-// scratch with it: max_tiles = min(total, total / rows + experts), or 0.
-LCU_API int lcu_moe_tile_rows(int type, int total, int experts) {
-    if ((long long)total > 16ll * experts) return (long long)total > 80ll * experts && (long long)total <= 120ll * experts ? MOE_TILE_ROWS : 96;
-    return total > (type == LCU_F32 ? MOE_LIST_F32 : MOE_LIST) ? 16 : 0;
+// tiles up to MOE_LIST pairs (0; MOE_LIST_F32 in 32 bits) and tiles of 16 beyond.  In 32 bits 32 then: the products are bound by their matrix instructions, and small tiles
+// are shared out evenly over the compute units.  In bfloat16 what should take least: the two products' workgroups (a tile and 128 features each) in turns of as many as there are compute
+// units, a turn as long as the K of its product times the rows that a workgroup multiplies and what it spends besides, 60 rows' time; as many tiles as there are where every
+// token chooses evenly, with one and a half times their deviation, and workgroups of the rows of the largest expert of so many.
+// Measured with 2 to 64 experts of 520 x 272 to 4096 x 4096 and 17 to 1,024 rows each on average, evenly and with a few experts taking most, 288 shapes: bfloat16 0.9 % (3.9 % unevenly)
+// more than the best of the four sizes, 17 % at most, 32 bits 2.8 % and 0.2 %, 16 % at most.  Always 96, but 128 for 80 to 120 rows, was 11 % and 10 % more, 32 bits 31 % and 51 %; tiles of
+// 64 10 % and 9 %, 32 bits 15 % and 24 %.  (us a pass of both products, with 32, 64, 96 and 128 rows: 16 experts, gated, of 1024 x 512, 88 rows 34, 31, 37, 41, 212 rows 52, 45, 51, 47; of 2048 x
+// 1024, 88 rows 90, 75, 86, 64, 256 rows 168, 139, 119, 132; 32 bits, 8 of 1024 x 1024, 88 rows: 59, 94, 131, 165.)
+// The caller sizes its scratch with it: max_tiles = min(total, total / rows + experts), or 0.
+LCU_API int lcu_moe_tile_rows(int type, int total, int experts, int up_rows, int d, int ff) {
+    if ((long long)total <= 16ll * experts) return total > (type == LCU_F32 ? MOE_LIST_F32 : MOE_LIST) ? 16 : 0;
+    if (type == LCU_F32) return 32;
+    const double mean = (double)total / experts, deviation = sqrt(mean), most = mean + (1 + log2((double)experts) / 6) * deviation;
+    int best = 0;
+    double least = 0;
+    for (int tile = most <= 32 ? 64 : 32; tile <= MOE_TILE_ROWS; tile += 32) {      // (half empty tiles take no longer than full ones of half the rows, and hold an expert that has a few rows more)
+        const int all = (int)fmax((mean - 6 * deviation) / tile, 1);      // tiles that every expert has
+        double per = all, spread = 0;                // tiles of an expert and their variance
+        for (int j = all; j <= (int)(most / tile) + 2; ++j) {
+            const double beyond = 0.5 * erfc((j * tile + 0.5 - mean) / deviation * 0.70710678118654752);   // the share of the experts with more than j tiles' rows
+            per += beyond;
+            spread += beyond * (1 - beyond);
+        }
+        const double tiles = fmin(experts * ceil(most / tile), experts * per + 1.5 * sqrt(experts * spread)), rows = fmin(tile, ceil(most / ceil(mean / tile) / 32) * 32);
+        auto turns = [&](int features) { return ceil(tiles * ((features + 127) / 128) / 256); };
+        const double time = (turns(up_rows) * d + turns(d) * ff) * (60 + rows);
+        if (!best || time < least) { best = tile; least = time; }
+    }
+    return best;
 }
 
 // h: [n, d] of `type`; router: [experts, d] 32-bit; ids, wts: [n * top].
@@ -724,8 +747,9 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
     return LCU_OK;
 }
 
+// tile_rows: what lcu_moe_tile_rows says, or beyond 16 another multiple of 16 up to MOE_TILE_ROWS (the results are the same).
 // ints: scratch of total + 3 * max_tiles + 1 entries, laid out as sorted_to_flat, tile_expert, tile_begin,
-// tile_rows, n_tiles (null where lcu_moe_tile_rows says 0).
+// tile_rows, n_tiles (null with tile_rows 0).
 // w_up: [experts, ff, d], w_down: [experts, d, ff] of `type`; packed_up, packed_down: in the order of Unit.  act: scratch [total, ff] of `type`; y: scratch
 // [total, d] 32-bit (only read and written when top > 1 or gated).  out: [n, d] 32-bit, added to.
 // gated: w_up is [experts, 2 * ff, d], in turns 16 rows of the gate matrix and the 16 rows of the up matrix that meet
@@ -735,7 +759,7 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
 // [n, d] of `type`) with shared_gate (null or [n] 32-bit): rows that are added beside the experts', times the gate.  shared_up,
 // shared_down (null, or the matrices [2 * shared_ff, d] and [d, shared_ff] of a shared expert that is computed here, with silu, in the order of Unit
 // like w_up and w_down; defer: with top > 1 or gated the sum is left to whoever reads y; only where lcu_moe_tile_rows says 16 or 0): act then holds n * shared_ff elements more and y n rows more.
-LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float *wts, int *ints, int max_tiles,
+LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float *wts, int tile_rows, int *ints, int max_tiles,
                             const void *w_up, int packed_up, const void *w_down, int packed_down, void *act, float *y, float *out, int n, int d, int ff,
                             int experts, int top, int gated, const void *shared, const float *shared_gate, const void *shared_up,
                             const void *shared_down, int shared_ff, int fresh, int identity, float alpha, float limit, int defer, hipStream_t stream) {
@@ -746,8 +770,8 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
         (identity && !gated) || experts + identity > MOE_MAX_EXPERTS)
         return LCU_BAD_ARGUMENT;
     const int total = n * top;
-    const int tile_rows = lcu_moe_tile_rows(type, total, experts);
     const bool few = tile_rows <= 16;
+    if (tile_rows < 0 || tile_rows > MOE_TILE_ROWS || tile_rows % 16) return LCU_BAD_ARGUMENT;
     if (shared_up && (!shared_down || shared || !gated || !few || !packed_up || !packed_down || shared_ff <= 0 || shared_ff % 16)) return LCU_BAD_ARGUMENT;
     const int add = top == 1 && !gated;
     float *down_to = add ? out : y;

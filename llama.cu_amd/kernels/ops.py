@@ -1554,6 +1554,11 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, top: int, bias: Optional[to
     return (ids, wts, gates) if extra else (ids, wts)
 
 
+def moe_tile_rows(type_code: int, total: int, experts: int, up_rows: int, d: int, ff: int) -> int:
+    """Rows of the tiles into which an expert's pairs are cut (0: none are)."""
+    return build.load("moe").lcu_moe_tile_rows(type_code, total, experts, up_rows, d, ff)
+
+
 def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
                 out: torch.Tensor, gated: bool = False, shared: Optional[torch.Tensor] = None,
                 shared_gate: Optional[torch.Tensor] = None, fresh: bool = False, identity: int = 0,
@@ -1615,12 +1620,12 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
         _contig(shared_up.data, "shared up"); _contig(shared_down.data, "shared down")
     lib = build.load("moe")
     total = n * top
-    tile = lib.lcu_moe_tile_rows(_type(h, "moe input"), total, experts)
+    tile = moe_tile_rows(_type(h, "moe input"), total, experts, w_up.shape[1], d, ff)
     max_tiles = min(total, total // tile + experts) if tile else 0
     ints = torch.empty(total + 3 * max_tiles + 1, dtype=torch.int32, device=h.device) if tile else None
     act = torch.empty(total * ff + n * sff, dtype=h.dtype, device=h.device)
     y = torch.empty((total + (n if sff else 0), d), dtype=torch.float32, device=h.device) if (top > 1 or gated or tile > 16) else None
-    _check(lib.lcu_moe_experts(_ptr(h), _type(h, "moe input"), _ptr(ids), _ptr(wts), _ptr(ints), max_tiles, _ptr(up),
+    _check(lib.lcu_moe_experts(_ptr(h), _type(h, "moe input"), _ptr(ids), _ptr(wts), tile, _ptr(ints), max_tiles, _ptr(up),
                                int(up is not w_up), _ptr(down), int(down is not w_down), _ptr(act), _ptr(y), _ptr(out), n, d, ff, experts, top, int(bool(gated)),
                                _ptr(shared), _ptr(shared_gate if shared is not None or sff else None), _ptr(shared_up.data if sff else None),
                                _ptr(shared_down.data if sff else None), sff, int(bool(fresh)), identity, ctypes.c_float(act_alpha),

@@ -208,3 +208,34 @@ def test_tiles_of_many_rows(dtype, counts, d, ff, gated, pack):
     else:
         want = torch.einsum("ndf,nf->nd", y, torch.nn.functional.gelu(torch.einsum("nfd,nd->nf", v, x * s)))
     assert_close(got, want, 1e-4 if dtype == "float32" else 3e-2, "output")
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("counts,d,ff", [((17, 96, 97, 0, 33, 193), 264, 48), ((128, 129, 81, 95, 0, 100), 1096, 272), ((1, 600, 31, 65), 40, 1040)])
+@pytest.mark.parametrize("gated,pack", [(True, True), (False, False)])
+def test_tiles_of_every_size(dtype, counts, d, ff, gated, pack, monkeypatch):
+    """Which rows share a tile changes no bit."""
+    from llama_cu_amd.kernels import ops
+    experts, n, tdt = len(counts), sum(counts), TYPES[dtype]
+    order = torch.randperm(n, generator=torch.Generator().manual_seed(0))
+    ids = torch.repeat_interleave(torch.arange(experts, dtype=torch.int32), torch.tensor(counts))[order].view(n, 1).cuda()
+    h, wts = rnd(n, d, seed=1).to(tdt).cuda(), torch.rand(n, 1, generator=torch.Generator().manual_seed(2)).cuda()
+    gate, up = (rnd(experts, ff, d, seed=k, std=d ** -0.5).to(tdt).cuda() for k in (3, 4))
+    u, w = ops.gated_rows(gate, up) if gated else up, rnd(experts, d, ff, seed=5, std=ff ** -0.5).to(tdt).cuda()
+    if pack:
+        u, w = ops.pack_experts(u), ops.pack_experts(w)
+    got = []
+    for tile in (16, 32, 48, 64, 96, 112, 128):
+        monkeypatch.setattr(ops, "moe_tile_rows", lambda *sizes: tile)
+        got.append(ops.moe_experts(h, ids, wts, u, w, torch.zeros(n, d, device="cuda"), **({"gated": True, "fresh": True} if gated else {})))
+    for g in got[1:]:
+        assert torch.equal(g, got[0])
+
+
+def test_tiles_that_leave_no_compute_unit_idle():
+    """Small products in small tiles, large ones in tiles that fill the compute units in whole turns; (type: 1 bfloat16, 0 32 bits)."""
+    from llama_cu_amd.kernels import ops
+    for sizes, rows in [((1, 400, 16, 1024, 1024, 512), 32), ((1, 1400, 16, 1024, 1024, 512), 64), ((1, 2200, 16, 1024, 1024, 512), 96), ((1, 3400, 16, 1024, 1024, 512), 128),
+                        ((0, 700, 8, 1024, 1024, 1024), 32), ((0, 280, 4, 544, 520, 272), 32), ((1, 4028, 16, 2048, 2048, 2048), 96), ((1, 1400, 16, 2048, 2048, 1024), 128),
+                        ((1, 256, 16, 2048, 2048, 1024), 16), ((1, 16, 16, 2048, 2048, 1024), 0)]:
+        assert ops.moe_tile_rows(*sizes) == rows, sizes
