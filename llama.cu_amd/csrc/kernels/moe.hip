@@ -680,13 +680,13 @@ __global__ void __launch_bounds__(256)
 moe_combine_kernel(float *out, PairSum p, int n, int d) {
     const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (c >= d) return;
-    for (size_t t = blockIdx.y; t < (size_t)n; t += gridDim.y) *(pair_f32x4 *)(out + t * d + c) = pair_sum4<T>(p, t, c, d);
+    for (size_t t = blockIdx.y; t < (size_t)n; t += gridDim.y) *(pair_f32x4_at *)(out + t * d + c) = pair_sum4<T>(p, t, c, d);
 }
 
 // out: [n, d] 32-bit (p->base may be the same memory); p: in host memory.
 LCU_API int lcu_moe_combine(float *out, const PairSum *p, int type, int n, int d, hipStream_t stream) {
     if (n <= 0) return LCU_OK;
-    if (!out || !p || !pair_sum_ok(*p, type, d) || (uintptr_t)out % 16 || (type != LCU_F32 && type != LCU_BF16)) return LCU_BAD_ARGUMENT;
+    if (!out || !p || !pair_sum_ok(*p, d) || (type != LCU_F32 && type != LCU_BF16)) return LCU_BAD_ARGUMENT;
     const dim3 gc((d + 1023) / 1024, n < 65535 ? n : 65535), block(256);
     if (type == LCU_BF16) moe_combine_kernel<bf16_t><<<gc, block, 0, stream>>>(out, *p, n, d);
     else moe_combine_kernel<float><<<gc, block, 0, stream>>>(out, *p, n, d);

@@ -200,7 +200,7 @@ LCU_API int lcu_layernorm(float *x, const void *delta, int delta_type, int plane
 LCU_API int lcu_layernorm_pairs(float *x, const PairSum *pairs, int type, const float *w1, const float *b1, void *out1, const float *w2, const float *b2,
                                 void *out2, int out_type, int n, int d, float eps, hipStream_t stream) {
     if (n <= 0) return LCU_OK;
-    if (!x || !pairs || !w1 || !b1 || !out1 || (w2 && (!b2 || !out2)) || !pair_sum_ok(*pairs, type, d) || d > 4096 || !four_ok(x, LCU_F32) ||
+    if (!x || !pairs || !w1 || !b1 || !out1 || (w2 && (!b2 || !out2)) || !pair_sum_ok(*pairs, d) || d > 4096 || !four_ok(x, LCU_F32) ||
         !four_ok(w1, LCU_F32) || !four_ok(b1, LCU_F32) || !four_ok(out1, out_type) || !four_ok(w2, LCU_F32) || !four_ok(b2, LCU_F32) || !four_ok(out2, out_type))
         return LCU_BAD_ARGUMENT;
 #define ROW(T_, TO, T, PT) layernorm_row_kernel<PairsOf<T_>, TO, T, 4, PT, true><<<dim3(n), dim3(T), 0, stream>>>(x, PairsOf<T_>{*pairs}, w1, b1, (TO *)out1, w2, b2, (TO *)out2, d, eps)
@@ -443,7 +443,7 @@ LCU_API int lcu_norm_conv_single_pairs(float *x, const PairSum *pairs, int type,
                                        float eps, hipStream_t stream) {
     if (n <= 0) return LCU_OK;
     if (!x || !pairs || d > 2048 || taps < 1 || taps > 8 || sets < 1 || sets > 2 || !w1 || !b1 || (sets == 2 && (!w2 || !b2)) || !cw || (taps > 1 && !state) ||
-        !pair_sum_ok(*pairs, type, d) || !four_ok(x, LCU_F32) || !four_ok(w1, LCU_F32) || !four_ok(b1, LCU_F32) || !four_ok(w2, LCU_F32) || !four_ok(b2, LCU_F32) ||
+        !pair_sum_ok(*pairs, d) || !four_ok(x, LCU_F32) || !four_ok(w1, LCU_F32) || !four_ok(b1, LCU_F32) || !four_ok(w2, LCU_F32) || !four_ok(b2, LCU_F32) ||
         !four_ok(cw, LCU_F32) || !four_ok(state, LCU_F32) || !four_ok(out, type))
         return LCU_BAD_ARGUMENT;
     const size_t stride = (size_t)n * d;

@@ -178,7 +178,7 @@ LCU_API int lcu_norm_post(float *x, const void *a, int a_type, const float *a_bi
 LCU_API int lcu_norm_post_pairs(float *x, const PairSum *pairs, int type, const float *w_post, float eps_post, const float *w_pre, float eps_pre, void *out, int n,
                                 int d, hipStream_t stream) {
     if (n <= 0) return LCU_OK;
-    if (!x || !pairs || !w_post || (w_pre && !out) || !pair_sum_ok(*pairs, type, d) || d > 8 * NP_ROW_THREADS || !four_ok(x, LCU_F32) || !four_ok(w_post, LCU_F32) ||
+    if (!x || !pairs || !w_post || (w_pre && !out) || !pair_sum_ok(*pairs, d) || d > 8 * NP_ROW_THREADS || !four_ok(x, LCU_F32) || !four_ok(w_post, LCU_F32) ||
         !four_ok(w_pre, LCU_F32) || !four_ok(out, type) || (type != LCU_F32 && type != LCU_BF16))
         return LCU_BAD_ARGUMENT;
 #define GO(T, PT) norm_post_row_kernel<PairsOf<T>, T, PT><<<dim3(n), dim3(NP_ROW_THREADS), 0, stream>>>(x, PairsOf<T>{*pairs}, nullptr, w_post, eps_post, w_pre, eps_pre, (T *)out, d)

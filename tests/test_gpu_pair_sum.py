@@ -94,3 +94,29 @@ def test_the_norms_with_their_convolutions_add_it_up(dtype, d, taps, sets):
         to += [a, state, out]
     for k, (g, r) in enumerate(zip(got, ref)):
         assert torch.equal(g, r), k
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_rows_that_begin_at_any_element(dtype):
+    """Contiguous rows within a larger tensor, one element past its start: taken by the experts as they are, and by the norms."""
+    from llama_cu_amd.kernels import ops
+    n, d, ff, experts, tdt = 5, 64, 32, 4, TYPES[dtype]
+
+    def past(t):
+        whole = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        part = whole[1:].view(t.shape)
+        part.copy_(t)
+        return part
+    gate, up, down = (rnd(experts, *s, seed=k, std=0.1).to(tdt).cuda() for k, s in enumerate(((ff, d), (ff, d), (d, ff))))
+    w = ops.gated_rows(gate, up)
+    ids = torch.randint(0, experts + 2, (n, 2), generator=torch.Generator().manual_seed(1), dtype=torch.int32).cuda()
+    h, shared, out, wts = rnd(n, d, seed=5).to(tdt).cuda(), rnd(n, d, seed=6).to(tdt).cuda(), rnd(n, d, seed=7).cuda(), rnd(n, 2, seed=8).cuda()
+    run = lambda h, shared, out, **kw: ops.moe_experts(h, ids, wts, w, down, out, gated=True, shared=shared, identity=2, **kw)
+    want = run(h, shared, out.clone())
+    assert torch.equal(run(past(h), past(shared), past(out)), want)
+    vec = lambda k: (rnd(d, seed=k) + 1).cuda()
+    x, a, b = rnd(n, d, seed=9).cuda(), torch.empty(n, d, dtype=tdt, device="cuda"), torch.empty(n, d, dtype=tdt, device="cuda")
+    x2 = x.clone()
+    ops.layernorm(x, vec(1), vec(2), 1e-5, a, delta=want)
+    ops.layernorm(x2, vec(1), vec(2), 1e-5, b, delta=run(past(h), past(shared), past(out), defer=True))
+    assert torch.equal(x, x2) and torch.equal(a, b)
