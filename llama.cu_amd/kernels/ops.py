@@ -1311,6 +1311,7 @@ def layernorm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: fl
     if pairs is not None:
         _check(build.load("norm_conv").lcu_layernorm_pairs(_ptr(x), ctypes.byref(pairs.args()), pairs.type(), _ptr(weight), _ptr(bias), _ptr(out), _ptr(weight2),
                                                            _ptr(bias2), _ptr(out2), _type(out, "norm out"), n, d, ctypes.c_float(eps), _stream()), "layernorm_pairs")
+        pairs.added()
         return out
     planes = 0
     if delta is not None:
@@ -1379,6 +1380,7 @@ def norm_conv_single(x: torch.Tensor, delta: Optional[torch.Tensor], weights, bi
             _ptr(x), ctypes.byref(pairs.args()), pairs.type(), _ptr(weights[0]), _ptr(biases[0]), _ptr(weights[1] if sets == 2 else None),
             _ptr(biases[1] if sets == 2 else None), _ptr(conv_weight), _ptr(state if taps > 1 else None), _ptr(out), _ptr(step.ctx_len), _ptr(step.state_slot),
             n, d, taps, sets, ctypes.c_float(eps), _stream()), "norm_conv_single_pairs")
+        pairs.added()
         return out
     planes = 0
     if delta is not None:
@@ -1643,7 +1645,8 @@ class _PairSumArgs(ctypes.Structure):
 @dataclass
 class PairSum:
     """Float32 rows ``[n, d]`` that stand in memory as the terms of their sum: what a token's experts gave (``y [n * top, d]``, times ``wts``), beside ``base``
-    and a shared expert's rows.  The norms that add a branch to the residual stream take them where ``pair_sum_takes`` says so; ``rows()`` adds them up."""
+    and a shared expert's rows.  The norms that add a branch to the residual stream take them where ``pair_sum_takes`` says so; ``rows()`` adds them up.  Either happens
+    once: ``rows()`` may write where ``base`` is, and the terms, ``top`` times as large as the sum, are let go of then."""
     n: int
     d: int
     dtype: torch.dtype
@@ -1659,15 +1662,23 @@ class PairSum:
     real: int
 
     def args(self) -> _PairSumArgs:
+        if self.y is None:
+            raise KernelError("a sum of experts' rows is added up once")
         at = lambda t: t.data_ptr() if t is not None else None
         return _PairSumArgs(at(self.base), at(self.y), at(self.wts), at(self.shared), at(self.shared32), at(self.gate), at(self.ids), at(self.h), self.top, self.real)
+
+    def added(self) -> None:
+        """What adds it up has been launched (the allocator gives memory out again in the order of the stream)."""
+        self.base = self.y = self.wts = self.shared = self.shared32 = self.gate = self.ids = self.h = None
 
     def type(self) -> int:
         return BF16 if self.dtype == torch.bfloat16 else F32
 
     def rows(self) -> torch.Tensor:
+        args = self.args()
         out = self.base if self.base is not None else torch.empty((self.n, self.d), dtype=torch.float32, device=self.y.device)
-        _check(build.load("moe").lcu_moe_combine(_ptr(out), ctypes.byref(self.args()), self.type(), self.n, self.d, _stream()), "moe_combine")
+        _check(build.load("moe").lcu_moe_combine(_ptr(out), ctypes.byref(args), self.type(), self.n, self.d, _stream()), "moe_combine")
+        self.added()
         return out
 
 
@@ -1757,6 +1768,7 @@ def norm_post(x: torch.Tensor, a: torch.Tensor, w_post: torch.Tensor, eps_post: 
         out = torch.empty((n, d), dtype=a.dtype, device=x.device) if w_pre is not None or copy or (copy is None and out_dtype is not None) else None
         _check(build.load("norm_post").lcu_norm_post_pairs(_ptr(x), ctypes.byref(a.args()), a.type(), _ptr(w_post), ctypes.c_float(eps_post), _ptr(w_pre),
                                                            ctypes.c_float(eps_pre), _ptr(out), n, d, _stream()), "norm_post_pairs")
+        a.added()
         return out
     _gpu(x, a, w_post, w_pre, a_bias)
     _rows(x, "residual stream"); _contig(x, "residual stream"); _contig(a, "sublayer output")

@@ -120,3 +120,20 @@ def test_rows_that_begin_at_any_element(dtype):
     ops.layernorm(x, vec(1), vec(2), 1e-5, a, delta=want)
     ops.layernorm(x2, vec(1), vec(2), 1e-5, b, delta=run(past(h), past(shared), past(out), defer=True))
     assert torch.equal(x, x2) and torch.equal(a, b)
+
+
+def test_a_sum_is_added_up_once():
+    """A second time would add the terms twice where the sum lies in one of them; and they are let go of."""
+    from llama_cu_amd.kernels import ops
+    vec = (rnd(64, seed=1) + 1).cuda()
+    uses = [lambda p: p.rows(), lambda p: ops.norm_post(rnd(3, 64).cuda(), p, vec, 1e-5),
+            lambda p: ops.layernorm(rnd(3, 64).cuda(), vec, vec, 1e-5, torch.empty(3, 64, device="cuda"), delta=p),
+            lambda p: ops.norm_conv_single(rnd(3, 64).cuda(), p, [vec], [vec], 1e-5, torch.ones(1, 64, 1, device="cuda"), torch.empty(3, 1, 0, 64, device="cuda"),
+                                           torch.empty(1, 3, 64, device="cuda"), hand_step([1] * 3, [1, 2, 3], [0, 1, 2]))]
+    for use in uses:
+        p, _ = pair_sum(3, 64, "float32", 2, True, True, None, False)
+        use(p)
+        assert p.y is None and p.base is None
+        for again in uses:
+            with pytest.raises(ops.KernelError):
+                again(p)
