@@ -654,7 +654,7 @@ __global__ void __launch_bounds__(256, 2)
 moe_gemm_many_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__ w, size_t w_expert_stride, int N, int K,
                      const int *__restrict__ sorted_to_flat, const float *__restrict__ wts,
                      const int *__restrict__ tile_expert, const int *__restrict__ tile_begin,
-                     const int *__restrict__ tile_rows, const int *__restrict__ n_tiles, int max_tiles, T *__restrict__ out_t,
+                     const int *__restrict__ tile_rows, const int *__restrict__ n_tiles, T *__restrict__ out_t,
                      float *__restrict__ out_f, int out_stride, int top, int add, float alpha, float limit) {
     __shared__ __attribute__((aligned(16))) T xs[2 * MOE_TILE_ROWS * 128 / sizeof(T)];
     // Workgroups go to the chip's eight dies in turn (workgroup i to die i % 8), and each die has an L2 of its own.  The work, in the order
@@ -758,7 +758,8 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
 // token's input.  shared (null or
 // [n, d] of `type`) with shared_gate (null or [n] 32-bit): rows that are added beside the experts', times the gate.  shared_up,
 // shared_down (null, or the matrices [2 * shared_ff, d] and [d, shared_ff] of a shared expert that is computed here, with silu, in the order of Unit
-// like w_up and w_down; defer: with top > 1 or gated the sum is left to whoever reads y; only where lcu_moe_tile_rows says 16 or 0): act then holds n * shared_ff elements more and y n rows more.
+// like w_up and w_down; only with tile_rows 16 or 0): act then holds n * shared_ff elements more and y n rows more.
+// defer: with top > 1 or gated, and any tile_rows, the sum is left to whoever reads y, and out is not used.
 LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float *wts, int tile_rows, int *ints, int max_tiles,
                             const void *w_up, int packed_up, const void *w_down, int packed_down, void *act, float *y, float *out, int n, int d, int ff,
                             int experts, int top, int gated, const void *shared, const float *shared_gate, const void *shared_up,
@@ -771,7 +772,7 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
         return LCU_BAD_ARGUMENT;
     const int total = n * top;
     const bool few = tile_rows <= 16;
-    if (tile_rows < 0 || tile_rows > MOE_TILE_ROWS || tile_rows % 16) return LCU_BAD_ARGUMENT;
+    if (tile_rows < 0 || tile_rows > MOE_TILE_ROWS || tile_rows % 16 || (!tile_rows && total > (type == LCU_F32 ? MOE_LIST_F32 : MOE_LIST))) return LCU_BAD_ARGUMENT;
     if (shared_up && (!shared_down || shared || !gated || !few || !packed_up || !packed_down || shared_ff <= 0 || shared_ff % 16)) return LCU_BAD_ARGUMENT;
     const int add = top == 1 && !gated;
     float *down_to = add ? out : y;
@@ -817,9 +818,9 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
         // flat grids: the kernel shares them out over the dies itself
         const dim3 block(256), gu((max_tiles * ((up_rows + 127) / 128) + 7) / 8 * 8), gd((max_tiles * ((d + 127) / 128) + 7) / 8 * 8);
 #define UP(T, PACKED, MODE) moe_gemm_many_kernel<T, MODE, PACKED><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \
-                                                sorted, wts, t_exp, t_beg, t_rows, n_tiles, max_tiles, (T *)act, nullptr, ff, top, 0, alpha, limit)
+                                                sorted, wts, t_exp, t_beg, t_rows, n_tiles, (T *)act, nullptr, ff, top, 0, alpha, limit)
 #define DOWN(T, PACKED, MODE) moe_gemm_many_kernel<T, MODE, PACKED><<<gd, block, 0, stream>>>((const T *)act, ff, (const T *)w_down, down_stride, d, ff, \
-                                                sorted, wts, t_exp, t_beg, t_rows, n_tiles, max_tiles, nullptr, down_to, d, top, add, 0.f, 0.f)
+                                                sorted, wts, t_exp, t_beg, t_rows, n_tiles, nullptr, down_to, d, top, add, 0.f, 0.f)
         int packed = packed_up;
         if (gated) { TYPED(UP, MOE_UP_GATED); } else { TYPED(UP, MOE_UP); }
         packed = packed_down;

@@ -1562,7 +1562,7 @@ def moe_tile_rows(type_code: int, total: int, experts: int, up_rows: int, d: int
 
 
 def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
-                out: torch.Tensor, gated: bool = False, shared: Optional[torch.Tensor] = None,
+                out: Optional[torch.Tensor], gated: bool = False, shared: Optional[torch.Tensor] = None,
                 shared_gate: Optional[torch.Tensor] = None, fresh: bool = False, identity: int = 0,
                 act_alpha: float = 1.0, act_limit: float = 0.0, shared_expert: Optional[tuple] = None, defer: bool = False):
     """``out[t] += sum over t's experts e of  w_down[e] @ gelu(w_up[e] @ (weight * h[t]))`` (the exact gelu; the
@@ -1575,12 +1575,15 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
     ``act_limit`` > 0: the limited activation (``swiglu``) with ``act_alpha`` instead of silu.  ``shared_expert``: in the place of
     ``shared`` the matrices (``[1, 2 * sff, d]`` as ``gated_rows`` lays them out and ``[1, d, sff]``, both packed) of an expert with
     silu that every token uses, computed beside the others; where ``moe_shared_beside`` says so.  ``defer``: the experts' outputs may come back as a
-    ``PairSum`` that whoever uses the sum adds up (``out``, unless ``fresh``, is then one of its terms and not written)."""
+    ``PairSum`` that whoever uses the sum adds up (``out``, unless ``fresh``, is then one of its terms and not written; with ``fresh`` it may be None)."""
     up, down = (w.data if isinstance(w, PackedExperts) else w for w in (w_up, w_down))
     _gpu(h, ids, wts, up, down, out, shared, shared_gate)
     _rows(h, "moe input")
+    if out is None and not (fresh and gated and defer):
+        raise KernelError("moe_experts: only a sum that is left to others and begins afresh needs no out")
     for t, what in ((h, "moe input"), (ids, "moe ids"), (wts, "moe weights"), (up, "moe up"), (down, "moe down"), (out, "moe out")):
-        _contig(t, what)
+        if t is not None:
+            _contig(t, what)
     n, d = h.shape
     experts, ff = w_down.shape[0], w_down.shape[2] if len(w_down.shape) == 3 else 0
     if len(w_up.shape) != 3 or len(w_down.shape) != 3 or w_up.shape != (experts, (2 if gated else 1) * ff, d) or w_down.shape[1] != d \
@@ -1589,7 +1592,7 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
     top = ids.shape[1] if ids.dim() == 2 else 0
     if ids.shape != (n, top) or ids.dtype != torch.int32 or wts.shape != (n, top) or wts.dtype != torch.float32 or top < 1:
         raise KernelError("moe_experts: ids (int32) and weights (float32) must be [n, top]")
-    if out.shape != (n, d) or out.dtype != torch.float32:
+    if out is not None and (out.shape != (n, d) or out.dtype != torch.float32):
         raise KernelError("moe_experts: out must be float32 [n, d]")
     per = 8 if h.dtype == torch.bfloat16 else 4
     if d % per or ff % (16 if gated else per):
@@ -1626,7 +1629,7 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w_up: tor
     max_tiles = min(total, total // tile + experts) if tile else 0
     ints = torch.empty(total + 3 * max_tiles + 1, dtype=torch.int32, device=h.device) if tile else None
     act = torch.empty(total * ff + n * sff, dtype=h.dtype, device=h.device)
-    y = torch.empty((total + (n if sff else 0), d), dtype=torch.float32, device=h.device) if (top > 1 or gated or tile > 16) else None
+    y = torch.empty((total + (n if sff else 0), d), dtype=torch.float32, device=h.device) if (top > 1 or gated) else None
     _check(lib.lcu_moe_experts(_ptr(h), _type(h, "moe input"), _ptr(ids), _ptr(wts), tile, _ptr(ints), max_tiles, _ptr(up),
                                int(up is not w_up), _ptr(down), int(down is not w_down), _ptr(act), _ptr(y), _ptr(out), n, d, ff, experts, top, int(bool(gated)),
                                _ptr(shared), _ptr(shared_gate if shared is not None or sff else None), _ptr(shared_up.data if sff else None),

@@ -225,7 +225,7 @@ class GatedMoE(Part):
                                extra=self.gates, **self.choice)
         ids, wts = routed[0], routed[1]
         fresh = add_to is None
-        out = add_to if not fresh else torch.empty((h.shape[0], h.shape[1]), dtype=torch.float32, device=h.device)
+        out = add_to if not fresh else None if pairs_ok else torch.empty((h.shape[0], h.shape[1]), dtype=torch.float32, device=h.device)
         if self.shared is not None:
             beside = self.shared_expert is not None and ops.moe_shared_beside(h.shape[0], ids.shape[1], self.experts, self.w_gate_up, self.w_down)
             return ops.moe_experts(h, ids, wts, self.w_gate_up, self.w_down, out, gated=True, defer=pairs_ok, shared=None if beside else self.shared.forward(h),

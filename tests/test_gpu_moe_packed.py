@@ -239,3 +239,24 @@ def test_tiles_that_leave_no_compute_unit_idle():
                         ((0, 700, 8, 1024, 1024, 1024), 32), ((0, 280, 4, 544, 520, 272), 32), ((1, 4028, 16, 2048, 2048, 2048), 96), ((1, 1400, 16, 2048, 2048, 1024), 128),
                         ((1, 256, 16, 2048, 2048, 1024), 16), ((1, 16, 16, 2048, 2048, 1024), 0)]:
         assert ops.moe_tile_rows(*sizes) == rows, sizes
+
+
+@pytest.mark.parametrize("gated", [True, False])
+def test_memory_that_nobody_reads_is_not_asked_for(gated):
+    """One expert a token that is not gated adds its rows where they belong; a sum that begins afresh and is left to others has no rows of its own."""
+    from llama_cu_amd.kernels import ops
+    n, d, ff, experts = 512, 2048, 64, 4
+    h = rnd(n, d, seed=1).to(torch.bfloat16).cuda()
+    ids, wts = (torch.arange(n, dtype=torch.int32)[:, None] % experts).cuda(), torch.ones(n, 1, device="cuda")
+    up, down = (torch.zeros(experts, r, k, dtype=torch.bfloat16, device="cuda") for r, k in (((2 if gated else 1) * ff, d), (d, ff)))
+    out = torch.zeros(n, d, device="cuda") if not gated else None
+    with pytest.raises(ops.KernelError):
+        ops.moe_experts(h, ids, wts, up, down, None, gated=gated)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    kept = ops.moe_experts(h, ids, wts, up, down, out, gated=gated, fresh=gated, defer=gated)
+    more = torch.cuda.max_memory_allocated() - before
+    assert more <= 4 * n * d * gated + 2 * n * ff + (1 << 16), more            # (the pairs' rows, the activations, the lists)
+    if gated:
+        assert torch.equal(kept.rows(), torch.zeros(n, d, device="cuda"))
