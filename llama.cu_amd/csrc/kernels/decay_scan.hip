@@ -604,7 +604,7 @@ ds_single_kernel(DsSingle p) {
             }
         }
     };
-    load_state(min(my_row, d - 1), min(my_col, groups - 1) * V);
+    if (my_row < d) load_state(my_row, min(my_col, groups - 1) * V);
     __builtin_amdgcn_sched_barrier(0);
     float m_now = 0.f;
     if (!p.decay) {
@@ -671,7 +671,7 @@ ds_single_kernel(DsSingle p) {
             const int cc = c0 * V + x;
             if (cc >= dv) continue;
             float o = 0.f;
-            for (int w = 0; w < nrows; ++w) o += red[w * cols * V + x];
+            for (int w = 0; w < min(nrows, d); ++w) o += red[w * cols * V + x];       // (rows of threads beyond the state's are zeros)
             o *= p.scale * inv;
             vs[cc] = o;                           // (v of these columns has been used)
             sq += o * o;

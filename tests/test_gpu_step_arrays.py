@@ -87,7 +87,9 @@ def builder_of(positions, max_tokens=32):
     from llama_cu_amd.engine.batch import BatchBuilder
     groups = [CacheGroup(40, 8, 0), CacheGroup(20, 16, 0)]
     cache = CacheManager(groups, 4)
-    return cache, BatchBuilder(cache, max_tokens, 4, [-(-positions // g.page_size) for g in groups], torch.device("cuda:0"))
+    builder = BatchBuilder(cache, max_tokens, 4, [-(-positions // g.page_size) for g in groups], torch.device("cuda:0"))
+    torch.cuda.synchronize()                # (its device buffer is cleared on this stream; the steps may come on others)
+    return cache, builder
 
 
 def busy(a, times=200):
