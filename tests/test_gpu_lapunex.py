@@ -291,9 +291,14 @@ def test_single_tokens_of_many_requests_and_rows_that_wait_for_their_norm():
 
 
 @pytest.mark.parametrize("count,planes", [(33, True), (50, True), (64, True), (65, False)])
-def test_single_tokens_whose_norm_the_product_with_shared_rows_applies(count, planes):
-    """From 33 to 64 requests the norm over the heads is a factor in the output product's partial sums; beyond, a kernel applies it."""
+def test_single_tokens_whose_norm_the_product_with_shared_rows_applies(count, planes, monkeypatch):
+    """From 33 to 64 requests the norm over the heads is a factor in the output product's partial sums; beyond, and where nobody takes partial sums, a kernel applies it."""
+    from llama_cu_amd.parts import decay_scan as module
+    from llama_cu_amd.parts.base import ScaledRows
     d = 128
+    products, scans = [], []
+    monkeypatch.setattr(module, "linear_planes", lambda a, w, f=module.linear_planes: (products.append(isinstance(a, ScaledRows)), f(a, w))[1])
+    monkeypatch.setattr(module.ops, "decay_scan", lambda *a, f=module.ops.decay_scan, **kw: (scans.append(bool(kw.get("scaled_rows"))), f(*a, **kw))[1])
     part, plain, _ = lightning_part([0.9, 0.99, 0.5, 0.7, 0.95, 0.8, 0.999, 0.6], 128, 128, d, "bfloat16", pack=True)
     lens = [1 + r % 4 for r in range(count)]
     rows = [rnd(n + 1, d, seed=100 + r).bfloat16() for r, n in enumerate(lens)]
@@ -301,9 +306,11 @@ def test_single_tokens_whose_norm_the_product_with_shared_rows_applies(count, pl
     for ok in (True, False):
         cache = state_of(part, count)
         part.forward(torch.cat([x[:-1] for x in rows]).cuda(), hand_step(lens, lens, list(range(count))), cache)
+        del products[:], scans[:]
         results.append(part.forward(torch.stack([x[-1] for x in rows]).cuda(), hand_step([1] * count, [n + 1 for n in lens], list(range(count))), cache, planes_ok=ok))
+        assert scans == [planes and ok] and products == [True] * (planes and ok)      # (the ordinary product with partial sums has finished rows)
     got, other = results
-    assert (got.dtype == torch.float32 and got.dim() == 3) or not planes
+    assert got.dtype == torch.float32 and got.dim() == 3 if planes else got.dtype == torch.bfloat16 or got.dim() == 3
     got = got.float().sum(0) if got.dim() == 3 else got
     for r in range(0, count, 4):
         assert_close(got[r], plain(f64(rows[r].float()))[-1], 3e-2, f"{r}")
