@@ -360,8 +360,8 @@ LCU_API int lcu_delta_rule(const void *proj, int type, int row_stride, int off_r
 // a time.  A lane holds four neighbouring columns (16-byte loads) of SL = DK / 8 key channels, the groups of lanes as in the scan; every sum is made in
 // the scan's order, so a token has the same bits either way.  The matrices are on their way while the token's vectors are made.
 // Few requests wait for memory's latency, many for the matrices, read and written once.  16 heads of 128 x 128, rank 64, a chain of such steps: 1 request 9.1 ->
-// 6.3 us, 16 requests 23.9 -> 9.0, 200 requests 246 -> 68; the gated rule with its convolution and products 18.7 -> 15.5, 27.4 -> 19.9, 224 -> 91.  (Heads of 32
-// with a rank of 512, 200 requests: 59 and 61, each request reads the decay's second matrix.)
+// 6.3 us, 16 requests 23.9 -> 9.0, 200 requests 246 -> 68; the gated rule with its convolution and products 18.7 -> 15.5, 27.4 -> 19.9, 224 -> 91.  (Where it is
+// longer: lcu_delta_single_pays.)
 // STREAM: the state's loads and stores are non-temporal.
 template <int DK, bool STREAM = false> struct SingleColumns {
     static constexpr int SL = DK / 8, SLP = SL + 4, VEC = 8 * SLP;      // a vector in LDS: the groups' shares, four floats of padding behind each
@@ -514,8 +514,10 @@ delta_single_kernel(const T *__restrict__ proj, int row_stride, int off_r, int o
 static bool single_sizes(int heads, int dk, int dv) {
     return heads > 0 && heads <= 65535 && (dk == 32 || dk == 64 || dk == 96 || dk == 128) && dv > 0 && dv % 4 == 0 && dv <= SINGLE_MAX_DV;
 }
-// A step's states of this size are in no cache when their layer's turn comes again, and what they leave there would push out what is (64 requests of 16 heads of
-// 128 x 128 over eight layers, the decay scans' kernel: 34.9 us a layer, 29.0 past the caches; below, the last-level cache holds a few layers')
+// A step's states of this size are in no cache when their layer's turn comes again, and what they leave there would push out what is.  16 heads of 128 x 128 over eight
+// layers, us a layer: 48 MB 26.8, past the caches 21.8, 64 MB 34.4 and 26.9 (the gated rule with its convolution 41.4 and 35.1; with 40 MB of something else read between the layers 55.9
+// and 49.0); 8 heads of 64 x 256, 48 MB 24.6 and 23.0.  Below it goes either way: 32 MB 15.1 and 12.8, but 15.6 and 17.2; four layers alone, all of whose states the
+// last-level cache holds, lose at 48 MB too (18.7 and 23.6).
 static bool past_caches(int n_req, int heads, int dk, int dv) { return (long long)n_req * heads * dk * dv * 4 >= (48ll << 20); }
 LCU_API int lcu_delta_single_takes(int heads, int dk, int dv) { return single_sizes(heads, dk, dv); }
 

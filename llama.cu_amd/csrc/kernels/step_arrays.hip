@@ -1,9 +1,9 @@
-// A step's arrays (tokens, positions, block tables, task lists) from pinned host memory to their places on the device.
+// A step's arrays (tokens, positions, block tables, task lists) from host memory, packed into pinned memory, to their places on the device.
 //
 // What a decode step brings is a few hundred bytes to some tens of kilobytes, spread over arrays of fixed capacity.  One copy of the whole
 // capacity is a job of the copy engine with a signal on either side of it, between two steps of the queue: 26 us stood between one captured step and the
 // next with it, 10 with this kernel (40 launches replayed; 40,000 entries of capacity, 4,000 in use).  The kernel is bound by one trip over the host's bus, so every
-// piece is on its way at once: 16 bytes a thread, the pieces behind one another over the grid.
+// piece is on its way at once: 16 bytes a thread, the pieces behind one another over the grid.  (5.3 to 7.8 us a launch in steps of 1 to 64 requests.)
 #include <string.h>
 #include "common.h"
 

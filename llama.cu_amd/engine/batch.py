@@ -1,5 +1,5 @@
 """The batch of one step, as the model's parts see it, and the builder that lays it
-out in pinned host memory and brings it to the device in one copy.
+out in host memory and brings what the step uses of it to the device in one launch.
 
 The reference builds the same facts per round: the tokens, their positions
 (``pos()``), the rows whose output is wanted (``out_idx()``) and one ``Req{cache, pos,
@@ -62,7 +62,7 @@ class StepContext:
     def extra(self, name: str, size: int):
         """``(host, device)``: two int32 arrays of ``size`` entries under ``name`` in the step's own memory, for what
         a part derives from the batch on the host before the step runs (``Part.prepare``): the host array goes to
-        the device with the batch's one copy, and the device array's address is the same in every step, so a
+        the device with the batch's own arrays; both arrays' addresses are the same in every step, so a
         captured graph reads the new step's values.  None if the step was not made by a builder."""
         return self.builder.extra(name, size) if self.builder is not None else None
 
