@@ -176,7 +176,7 @@ def test_a_token_with_few_and_with_more_others(dtype, gated):
                 assert_close(got, whole[first:first + n].cpu().to(F64), 3 * 2.0 ** -9, f"{n}")
 
 
-# an expert's tiles at their edges (of 96 rows, and of 128 where there are 80 to 120 an expert on average), beside experts with few rows and with none;
+# an expert's tiles at their edges (of 32 to 128 rows, by the sizes), beside experts with few rows and with none;
 # K of less than a step, of whole steps, and one that ends within a unit of the last; features that end within a block, fewer blocks than dies
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("counts,d,ff", [((17, 96, 97, 0, 33, 193), 264, 48), ((128, 129, 81, 95, 0, 100), 1096, 272), ((1, 600, 31, 65), 40, 1040),
