@@ -34,7 +34,7 @@
 // first, adds them in a fixed order and leaves the factors in LDS for the epilogue.
 #include "common.h"
 #include "gate_act.h"
-#include "kv_layout.h"
+#include "qkv_store.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -463,9 +463,7 @@ LCU_API int lcu_gemm_mid_bf16_scaled(const void *X, int ldx, const void *W, int 
 template <int MT, bool PACKED>
 __global__ void __launch_bounds__((MID_CONSUMERS + mid_producers(MT)) * WAVE)
 gemm_mid_qkv_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict__ W, int ldw, int M, int K,
-                    bf16_t *__restrict__ q_out, int ldq, const int *__restrict__ positions, const int *__restrict__ slots,
-                    const float *__restrict__ cos_t, const float *__restrict__ sin_t, int max_pos, bf16_t *__restrict__ cache,
-                    int heads, int kv_heads, int head_dim, int page) {
+                    QkvStore store) {
     static_assert(MID_CONSUMERS == 4, "the four matrix instructions of a macro-step go to four waves");
     extern __shared__ __attribute__((aligned(16))) char xs[];      // the ring of X; at the end the waves' sums
     constexpr int BUF = 16 * MT * MID_XROW;
@@ -496,7 +494,7 @@ gemm_mid_qkv_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restr
             return;
         }
     }
-    const int per_head = head_dim / 32;
+    const int head_dim = store.head_dim, per_head = head_dim / 32;
     const int head = blockIdx.x / per_head, c = blockIdx.x % per_head;
     __amdgpu_buffer_rsrc_t wb[2];
 #pragma unroll
@@ -563,8 +561,6 @@ gemm_mid_qkv_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restr
 #pragma unroll
         for (int m = 0; m < MT; ++m) sums[((wave * 2 + t) * MT + m) * WAVE + lane] = acc[t][m];
     lds_barrier();
-    const int half_dim = head_dim / 2;
-    const bool is_q = head < heads, is_k = !is_q && head < heads + kv_heads;
 #pragma unroll
     for (int mi = 0; mi < (MT + MID_CONSUMERS - 1) / MID_CONSUMERS; ++mi) {
         const int m = wave + MID_CONSUMERS * mi;
@@ -582,53 +578,8 @@ gemm_mid_qkv_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restr
         // the lane holds dims i0 .. i0 + 3 (tile 0) and head_dim/2 + i0 .. (tile 1) of token 16 m + l16
         const int tok = 16 * m + l16;
         if (tok >= M) continue;
-        const int i0 = 16 * c + 4 * grp;
-        const int pos = positions[tok];
-        const bool in_table = pos >= 0 && pos < max_pos;
-        const int slot = slots ? slots[tok] : -1;
-        bf16_t *pg = nullptr;
-        int place = 0;
-        if (!is_q && slot >= 0) {
-            pg = cache + (size_t)(slot / page) * kv_page_elems(kv_heads, head_dim, page);
-            place = slot % page;
-        }
-        bf16_t va[4], vb[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            // rounded to bfloat16 before the rotation, as the plain product stores them for the rotation
-            // kernel: a token's query and key are made the same way whichever kernel makes them
-            float a = to_f32(from_f32<bf16_t>(sum[0][r])), b = to_f32(from_f32<bf16_t>(sum[1][r]));
-            if (is_q || is_k) {
-                float cs = __uint_as_float(0x7fc00000u), sn = cs;         // a position outside the table gives NaN
-                if (in_table) { cs = cos_t[(size_t)pos * half_dim + i0 + r]; sn = sin_t[(size_t)pos * half_dim + i0 + r]; }
-                float ra, rb;
-                rotate_pair(a, b, cs, sn, ra, rb);
-                a = ra; b = rb;
-            }
-            va[r] = from_f32<bf16_t>(a);
-            vb[r] = from_f32<bf16_t>(b);
-        }
-        if (is_q) {
-            bf16_t *qo = q_out + (size_t)tok * ldq + (size_t)head * head_dim;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) { qo[i0 + r] = va[r]; qo[i0 + half_dim + r] = vb[r]; }
-        } else if (pg) {
-            if (is_k) {
-                const int kvh = head - heads;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    pg[kv_key_offset(kvh, place, i0 + r, head_dim, page)] = va[r];
-                    pg[kv_key_offset(kvh, place, i0 + half_dim + r, head_dim, page)] = vb[r];
-                }
-            } else {
-                const int kvh = head - heads - kv_heads;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    pg[kv_value_offset(kv_heads, kvh, place, i0 + r, head_dim, page)] = va[r];
-                    pg[kv_value_offset(kv_heads, kvh, place, i0 + half_dim + r, head_dim, page)] = vb[r];
-                }
-            }
-        }
+        const float lo[4] = {sum[0][0], sum[0][1], sum[0][2], sum[0][3]}, hi[4] = {sum[1][0], sum[1][1], sum[1][2], sum[1][3]};
+        qkv_store(store, head, tok, 16 * c + 4 * grp, lo, hi);
     }
 }
 
@@ -651,6 +602,7 @@ LCU_API int lcu_gemm_mid_bf16_qkv_rope(const void *X, int ldx, const void *W, in
     if ((uintptr_t)X % 16 || (uintptr_t)W % 16) return LCU_BAD_ARGUMENT;
 #if LCU_MID_CONSUMERS == 4
     const dim3 grid((heads + 2 * kv_heads) * (head_dim / 32));
+    const QkvStore store = {positions, slots, cos_t, sin_t, max_pos, (bf16_t *)cache, (bf16_t *)q_out, ldq, heads, kv_heads, head_dim, page};
 #define GO(MT_, P_)                                                                                                         \
     do {                                                                                                                    \
         auto kernel = gemm_mid_qkv_kernel<MT_, P_>;                                                                         \
@@ -665,8 +617,7 @@ LCU_API int lcu_gemm_mid_bf16_qkv_rope(const void *X, int ldx, const void *W, in
             }                                                                                                               \
         }                                                                                                                   \
         kernel<<<grid, dim3((MID_CONSUMERS + mid_producers(MT_)) * WAVE), lds, stream>>>(                                   \
-            (const bf16_t *)X, ldx, (const bf16_t *)W, ldw, M, K, (bf16_t *)q_out, ldq, positions, slots, cos_t, sin_t,    \
-            max_pos, (bf16_t *)cache, heads, kv_heads, head_dim, page);                                                     \
+            (const bf16_t *)X, ldx, (const bf16_t *)W, ldw, M, K, store);                                                   \
     } while (0)
 #define GO_MT(MT_)                   \
     do {                             \

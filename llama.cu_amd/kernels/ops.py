@@ -67,6 +67,11 @@ def _rows(t: torch.Tensor, what: str) -> None:
                           f"strides {tuple(t.stride())}")
 
 
+def _near(x: torch.Tensor) -> torch.Tensor:
+    """Rows whose places fit the 32 bits in which the products of few rows keep them (rows 2^24 elements apart are copied together)."""
+    return x if x.stride(-2) < 1 << 24 else x.contiguous()
+
+
 def _contig(t: torch.Tensor, what: str) -> None:
     if not t.is_contiguous():
         raise KernelError(f"{what}: must be contiguous")
@@ -830,6 +835,7 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
         raise KernelError(f"gemm_skinny out: shape {tuple(out.shape)}, expected {(m, width)}")
     tiles = tiles or ((4 if (m > 8 or packed) else 2) if swiglu else _skinny_tiles(width, m, packed))
     waves = waves or (8 if width <= TUNING.skinny_eight_waves_to else 4)
+    x = _near(x)
     lib = build.load("gemm_skinny")
     if row_sumsq is not None:
         if row_sumsq.dtype != torch.float32 or row_sumsq.dim() != 2 or row_sumsq.shape[0] != m or not row_sumsq.is_contiguous() \
@@ -878,6 +884,7 @@ def gemm_skinny_grouped(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, pac
     while rows % (16 * tiles):
         tiles //= 2
     waves = waves or (8 if n <= TUNING.skinny_eight_waves_to and k > 512 else 4)      # (a wave needs a macro-step of 128 to work on)
+    x = _near(x)
     lib = build.load("gemm_skinny")
     _check(lib.lcu_gemm_skinny_bf16_grouped(_ptr(x), x.stride(1), ctypes.c_longlong(x.stride(0)), _ptr(w), w.stride(0), rows, _ptr(out),
                                             out.stride(0), m, n, k, _EPILOGUES["f32" if out.dtype == torch.float32 else "bf16"], tiles,
@@ -915,23 +922,21 @@ def wavek_wide(n: int) -> bool:
 
 
 def wavek_preferred(m: int, n: int, k: int, swiglu: bool = False, grouped: bool = False) -> bool:
-    """Whether ``gemm_wavek`` is the fastest choice for ``m`` rows and a packed ``[n, k]`` weight (``TUNING``'s numbers)."""
+    """Whether ``gemm_wavek`` is the fastest choice for ``m`` rows and a packed ``[n, k]`` weight (``TUNING``'s numbers; ``n`` counts all groups)."""
     t = TUNING
-    if min(n, k) < t.wavek_least or k > t.wavek_max_k or n > 32 * t.compute_units:                    # (more workgroups of 32 features than compute units: a second round)
+    if m > WAVEK_MAX_ROWS or k > t.wavek_max_k or n > 32 * t.compute_units:                    # (more workgroups of 32 features than compute units: a second round)
         return False
     if swiglu:
-        if m <= t.wavek_middle_rows or k <= t.wavek_short_k:
-            return m <= WAVEK_MAX_ROWS
-        if m <= t.wavek_rows:
-            return k <= t.wavek_middle_k or n > t.wavek_swiglu_features
-        return m <= WAVEK_MAX_ROWS and (n >= t.wavek_swiglu_features or (m <= t.wavek_more_rows and k <= t.wavek_middle_k and 2 * n >= t.wavek_swiglu_features))
-    if m <= (t.wavek_few_group_rows if grouped else t.wavek_few_rows):
+        return min(n, k) >= t.wavek_swiglu_least
+    if k < t.wavek_short_k:
+        return True
+    if m <= t.wavek_few_rows:
         return wavek_wide(n)
-    if k > t.wavek_middle_k and m > t.wavek_middle_rows and not grouped:
-        if m > t.wavek_rows:
-            return m <= t.wavek_more_rows and wavek_wide(n)
-        return 4 * t.compute_units < n <= t.wavek_wide_per_cu * t.compute_units or n > 24 * t.compute_units
-    return m <= t.wavek_rows or (m <= WAVEK_MAX_ROWS and k <= t.wavek_short_k) or (m <= t.wavek_more_rows and n >= t.wavek_more_features)
+    if n < t.wavek_few_features and k * m > t.wavek_few_features_work:
+        return False
+    if n > t.wavek_many_features and m > t.wavek_many_rows and k > t.wavek_short_k:
+        return False
+    return n >= t.wavek_least_features or m <= t.wavek_least_rows
 
 
 def gemm_wavek(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None,
@@ -964,6 +969,7 @@ def gemm_wavek(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = N
         if row_sumsq.dtype != torch.float32 or row_sumsq.dim() != 2 or row_sumsq.shape[0] != m or norm_width <= 0 or groups != 1:
             raise KernelError(f"gemm_wavek: row sums {row_sumsq.dtype} {tuple(row_sumsq.shape)} do not go with {m} rows")
     epi = 2 if swiglu else 3 if gate is not None else 1 if dtype == torch.float32 else 0
+    x = _near(x)
     lib = build.load("gemm_wavek")
     _check(lib.lcu_gemm_wavek(_ptr(x), x.stride(-2), ctypes.c_longlong(x.stride(0) if x.dim() == 3 else 0), groups, _ptr(w), _ptr(out), out.stride(0),
                               _ptr(gate), gate.stride(0) if gate is not None else 0, m, n, k, epi, int(wavek_wide(n)),
@@ -1056,6 +1062,7 @@ def gemm_skinny_add_norm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tenso
     parts = (n + 16 * tiles - 1) // (16 * tiles)
     h = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
     sumsq = torch.empty((m, parts), dtype=torch.float32, device=x.device)
+    x = _near(x)
     lib = build.load("gemm_skinny")
     _check(lib.lcu_gemm_skinny_bf16_add_norm(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(residual), residual.stride(0),
                                              m, n, k, _ptr(norm_weight), _type(norm_weight, "norm weight"), _ptr(h),
@@ -1092,6 +1099,7 @@ def gemm_skinny_streams(x: torch.Tensor, w: torch.Tensor, streams: torch.Tensor,
     parts = (n + 16 * tiles - 1) // (16 * tiles)
     h = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
     sumsq = torch.empty((m, parts), dtype=torch.float32, device=x.device)
+    x = _near(x)
     lib = build.load("gemm_skinny")
     _check(lib.lcu_gemm_skinny_bf16_streams(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(streams), streams.stride(0), int(count), m, n, k,
                                             _ptr(mix), _ptr(out_weights), _ptr(read), _ptr(norm_weight), _ptr(h), h.stride(0), _ptr(sumsq), parts,
@@ -1174,6 +1182,7 @@ def gemm_skinny_qkv_rope(x: torch.Tensor, w: torch.Tensor, positions: torch.Tens
         n_in = row_sumsq.shape[1]
     q = torch.empty((m, heads * head_dim), dtype=torch.bfloat16, device=x.device)
     waves = waves or 8
+    x = _near(x)
     lib = build.load("gemm_skinny")
     _check(lib.lcu_gemm_skinny_bf16_qkv_rope(_ptr(x), x.stride(0), _ptr(w), w.stride(0), m, k, _ptr(q), q.stride(0),
                                              _ptr(positions), _ptr(slots), _ptr(cos), _ptr(sin), cos.shape[0], _ptr(cache),
@@ -1186,6 +1195,17 @@ def mid_qkv_rope_supported(x: torch.Tensor, w: torch.Tensor, heads: int, kv_head
     """Whether ``gemm_mid_qkv_rope`` takes these operands: what ``gemm_mid`` takes, and whole heads whose halves
     are multiples of 16."""
     return (head_dim % 32 == 0 and w.dim() == 2 and w.shape[0] == (heads + 2 * kv_heads) * head_dim and mid_supported(x, w))
+
+
+def _check_qkv(what: str, positions, slots, cos, sin, cache, m: int, kv_heads: int, head_dim: int, page_size: int) -> None:
+    _i32(positions, "positions", m); _i32(slots, "cache slots", m)
+    if cos.shape != sin.shape or cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.dim() != 2 \
+            or cos.shape[1] * 2 != head_dim or not cos.is_contiguous() or not sin.is_contiguous():
+        raise KernelError(f"{what}: rotation tables must be two contiguous float32 tensors [max_pos, head_dim/2]")
+    _contig(cache, "cache")
+    if cache.dtype != torch.bfloat16 or cache.dim() != 3 or cache.shape[1] != 2 \
+            or cache.shape[2] != kv_heads * head_dim * page_size or page_size % 8:
+        raise KernelError(f"{what}: cache {cache.dtype} {tuple(cache.shape)}, expected bfloat16 [pages, 2, {kv_heads * head_dim * page_size}]")
 
 
 def gemm_mid_qkv_rope(x: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor,
@@ -1202,19 +1222,34 @@ def gemm_mid_qkv_rope(x: torch.Tensor, w: torch.Tensor, positions: torch.Tensor,
     if w.shape[1] != k or not mid_qkv_rope_supported(x, w, heads, kv_heads, head_dim):
         raise KernelError(f"gemm_mid_qkv_rope: x {tuple(x.shape)} {x.dtype} with w {tuple(w.shape)} {w.dtype}, {heads} + 2 * "
                           f"{kv_heads} heads of {head_dim} is not supported")
-    _i32(positions, "positions", m); _i32(slots, "cache slots", m)
-    if cos.shape != sin.shape or cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.dim() != 2 \
-            or cos.shape[1] * 2 != head_dim or not cos.is_contiguous() or not sin.is_contiguous():
-        raise KernelError("rotation tables must be two contiguous float32 tensors [max_pos, head_dim/2]")
-    _contig(cache, "cache")
-    if cache.dtype != torch.bfloat16 or cache.dim() != 3 or cache.shape[1] != 2 \
-            or cache.shape[2] != kv_heads * head_dim * page_size or page_size % 8:
-        raise KernelError(f"cache: {cache.dtype} {tuple(cache.shape)}, expected bfloat16 [pages, 2, {kv_heads * head_dim * page_size}]")
+    _check_qkv("gemm_mid_qkv_rope", positions, slots, cos, sin, cache, m, kv_heads, head_dim, page_size)
     q = torch.empty((m, heads * head_dim), dtype=torch.bfloat16, device=x.device)
     lib = build.load("gemm_mid")
     _check(lib.lcu_gemm_mid_bf16_qkv_rope(_ptr(x), x.stride(0), _ptr(w), w.stride(0), m, k, _ptr(q), q.stride(0),
                                           _ptr(positions), _ptr(slots), _ptr(cos), _ptr(sin), cos.shape[0], _ptr(cache),
                                           heads, kv_heads, head_dim, page_size, int(packed), _stream()), "gemm_mid_qkv_rope")
+    return q
+
+
+def wavek_qkv_rope_supported(x: torch.Tensor, w: torch.Tensor, heads: int, kv_heads: int, head_dim: int) -> bool:
+    """Whether ``gemm_wavek_qkv_rope`` takes these operands: what ``gemm_wavek`` takes, and whole heads whose halves are multiples of 16."""
+    return head_dim % 32 == 0 and w.dim() == 2 and w.shape[0] == (heads + 2 * kv_heads) * head_dim and x.dim() == 2 and wavek_supported(x, w)
+
+
+def gemm_wavek_qkv_rope(x: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                        cache: torch.Tensor, heads: int, kv_heads: int, head_dim: int, page_size: int) -> torch.Tensor:
+    """``gemm_mid_qkv_rope`` by the kernel whose waves share out K: up to 64 rows, ``w`` the result of ``pack_weight``."""
+    _gpu(x, w, positions, slots, cos, sin, cache)
+    if not wavek_qkv_rope_supported(x, w, heads, kv_heads, head_dim) or not w.is_contiguous() or x.stride(0) < x.shape[1]:
+        raise KernelError(f"gemm_wavek_qkv_rope: x {tuple(x.shape)} {x.dtype} with w {tuple(w.shape)} {w.dtype}, {heads} + 2 * "
+                          f"{kv_heads} heads of {head_dim} is not supported")
+    m, k = x.shape
+    _check_qkv("gemm_wavek_qkv_rope", positions, slots, cos, sin, cache, m, kv_heads, head_dim, page_size)
+    q = torch.empty((m, heads * head_dim), dtype=torch.bfloat16, device=x.device)
+    x = _near(x)
+    lib = build.load("gemm_wavek")
+    _check(lib.lcu_gemm_wavek_qkv_rope(_ptr(x), x.stride(0), _ptr(w), m, k, _ptr(q), q.stride(0), _ptr(positions), _ptr(slots), _ptr(cos), _ptr(sin),
+                                       cos.shape[0], _ptr(cache), heads, kv_heads, head_dim, page_size, _stream()), "gemm_wavek_qkv_rope")
     return q
 
 
@@ -1267,6 +1302,7 @@ def _skinny_f32(x, w, out, accumulate=False, scale=1.0, swiglu=False, row_sumsq=
     if row_sumsq is not None and (row_sumsq.dtype != torch.float32 or row_sumsq.dim() != 2 or row_sumsq.shape[0] != m
                                   or not row_sumsq.is_contiguous() or norm_width <= 0):
         raise KernelError("gemm_skinny_f32: row_sumsq must be a contiguous float32 [rows, parts] tensor, with the norm's width")
+    x = _near(x)
     lib = build.load("gemm_skinny")
     _check(lib.lcu_gemm_skinny_f32(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), m, n, k,
                                    int(bool(accumulate)), ctypes.c_float(scale), int(bool(swiglu)),

@@ -63,22 +63,25 @@ class Tuning:
     # (its numbers stand in gemm_wavek.hip; measured with widths of 1024 and 2048)
     wavek_wide_per_cu: int = 16         # 32 features a workgroup instead of 16 beyond so many features a compute unit (4096 x 2048 at 4 / 33 rows: 6.2 / 9.8 us
                                         # with 32, 5.4 / 8.4 with 16; 5120 x 2048 6.4 / 9.9 and 7.0 / 14.8)
-    wavek_max_k: int = 3072             # with a longer K the weight-streaming kernel is faster (K = 4096: 8.0 us against 9.9 at 8 rows)
-    wavek_least: int = 512              # features and K from which on it was measured: below either, the general path
-    wavek_few_rows: int = 11            # up to here a plain product goes to it beyond wavek_wide_per_cu only (up to there the weight-streaming
-                                        # kernel takes 0.95 of its time at 4, 5 and 8 rows, 1.06 at 16)
-    wavek_few_group_rows: int = 4       # ... and one in groups (16 groups of 128 x 512 at 5 rows: 3.4 us against 4.0)
-    wavek_rows: int = 32                # up to here every plain product does, but for those of more than wavek_middle_rows with a K beyond
-    wavek_middle_rows: int = 24         # wavek_middle_k where its workgroups are few or just too many for one a compute unit (32 rows, 3072 columns, 512 / 5120
-    wavek_middle_k: int = 2048          # features: 9.3 / 12.4 us against 7.5 / 12.1; 2048 features 9.7 against 10.2)
-    wavek_short_k: int = 1024           # ... up to 64 rows with a K up to this (2048 x 768: 5.7 us against the library's 7.2 at 64 rows),
-    wavek_more_rows: int = 48           # ... and up to here from so many features on (3072 x 2048: 9.2 us against 10.2 to 10.6; at 64 rows
-    wavek_more_features: int = 3072     # 11.1 against 10.9, with 2048 features 9.0 against 8.3 at 48), with a K beyond wavek_middle_k beyond wavek_wide_per_cu
-                                        # only (48 rows, 3072 x 2816 12.2 against 9.9, 5120 x 2816 14.3 against 14.9)
-    wavek_swiglu_features: int = 5632   # gate and up rows from which on SwiGLU goes to it with more than wavek_rows rows and a K beyond wavek_short_k, from half of
-                                        # them on with up to wavek_more_rows and a K up to wavek_middle_k; beyond them with more than
-                                        # wavek_middle_rows and a K beyond wavek_middle_k (whole feed-forwards at 64 rows, K of 2048 / 3072: 1024 features 20.2 / 24.8 us
-                                        # against 15.5 / 17.3, 5632 27.7 / 32.2 against 29.7 / 33.2)
+    wavek_max_k: int = 4096             # the longest K measured (4096 features, K = 4096: 8.6 us against the weight-streaming kernel's 9.1 at 16 rows, 10.7
+                                        # against 14.4 and the library's 13.2 at 32, 14.7 against 15.3 at 64)
+    wavek_short_k: int = 1024           # with a K below it is the fastest at any number of rows (2048 x 512: 2.7 us against 2.8 at 1 row, 3.4 against 3.8 at 24, 4.2
+                                        # against the library's 7.0 at 64; 16 groups of 128 x 128 2.5 against 2.8 at 8 rows, 2.8 against 4.6 at 32, 3.2 against 4.9 at 64)
+    wavek_few_rows: int = 8             # up to here a plain product goes to it beyond wavek_wide_per_cu only (5120 x 2048: 6.4 us against 6.8 at 8 rows; with 2048
+                                        # features 4.4 and 4.4, with 6144 x 4096 11.7 and 11.0); from 9 rows on 0.97 of the weight-streaming kernel's time, at 24 0.92
+    wavek_few_features: int = 1024      # few workgroups, each with much to do: below so many features not where K times the rows is beyond
+    wavek_few_features_work: int = 98304    # this (512 x 4096 at 64 rows 12.6 us against the library's 11.3, 64 x 2048 7.5 against 5.2; at 48 6.4 against 7.7)
+    wavek_least_features: int = 64      # below so many, and a K that is not short, only up to
+    wavek_least_rows: int = 24          # so many rows (16 x 1024: 3.6 us against 3.9 at 24, 4.2 against 3.9 at 48)
+    wavek_many_features: int = 6144     # beyond so many features, with a K beyond wavek_short_k, up to
+    wavek_many_rows: int = 48           # so many rows (8192 x 2048 at 64 rows 12.4 us against the library's 13.7 with the matrix out of memory, 11.8 against 11.0 in a
+                                        # model that runs its layers in a loop and finds it in the last-level cache; 10.7 against 13.9 at 48)
+    wavek_swiglu_least: int = 512       # gate and up rows and K from which on SwiGLU was measured (1024 x 512 to 8192 x 4096: the library's product alone, without
+                                        # the activation kernel's 2 us, is 1 us faster at most, at 48 rows of 2816 x 3072; the row-sharing kernel 1.5 us slower at 64 rows and 0.9
+                                        # faster at 24 to 32 rows of 8192, which go to it: mid_swiglu_features)
+    wavek_qkv_rows: int = 32            # q/k/v with the rotation and the cache write in its epilogue goes to it above so many rows and up to 64, where the row-sharing
+                                        # kernel would be taken (48 heads of 128, K = 4096: 20.0 us against 21.9 at 64 rows, 18.0 against 18.8 at 48; 15.5 against 14.8 at
+                                        # 24; 24 heads, K = 2048: 12.1 against 12.9 at 64, 10.8 against 10.7 at 48)
     # ---- the library's product of many rows (parts/linear.library_friendly_rows)
     library_rows: int = -1              # rows of zeros behind each half of a plain gate/up matrix: -1 times the library once per
                                         # shape at load and fills up where that is 15 % faster (the outcome can differ from box

@@ -325,6 +325,9 @@ def linear_qkv_rope(h, weight: Union[torch.Tensor, Weight], positions, slots, co
     rows = h.rows if isinstance(h, ScaledRows) else h
     if not (rows.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and cache_pages.dtype == torch.bfloat16):
         return None
+    if not isinstance(h, ScaledRows) and mid_qkv_takes(rows.shape[0], whole) and rows.shape[0] > ops.TUNING.wavek_qkv_rows \
+            and ops.wavek_qkv_rope_supported(rows, packed, heads, kv_heads, head_dim):
+        return ops.gemm_wavek_qkv_rope(rows, packed, positions, slots, cos, sin, cache_pages, heads, kv_heads, head_dim, page_size)
     if not isinstance(h, ScaledRows) and mid_qkv_takes(rows.shape[0], whole) \
             and ops.mid_qkv_rope_supported(rows, weight, heads, kv_heads, head_dim):
         return ops.gemm_mid_qkv_rope(rows, packed, positions, slots, cos, sin, cache_pages, heads, kv_heads, head_dim,
