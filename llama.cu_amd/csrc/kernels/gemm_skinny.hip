@@ -13,7 +13,12 @@
 //   * a wave keeps the loads of several macro-steps in flight while it multiplies one;
 //   * v_mfma_f32_16x16x32_bf16 with A = W tile, B = X^T: the 16 columns are 16 tokens,
 //     MT such tiles for up to 32 tokens (more rows go to gemm_mid.hip, which shares them through LDS).
+//     X comes in by quads of lanes and is turned into the operands' order in registers (quad_rows.h).
 // The waves' partial sums are added in LDS in a fixed order.
+//
+// One MI355X, packed weights out of memory, us a product (in brackets with X loaded in the operands' order, a cycle of a compute unit for every
+// lane): 2048 x 2048 4.0 (4.2) at 1 row, 4.4 (4.8) at 8, 5.2 (6.2) at 16; 4096 x 4096 7.8 (8.3) at 8, 9.1 (10.7) at 16; 4096 x 14336 22.0 (22.6) at
+// 1, 22.7 (25.3) at 8, 25.0 (32.9) at 16; SwiGLU of 28672 x 4096 41.1 (41.8) at 8, 42.0 (43.8) at 16.
 //
 // W may also be given packed (lcu_pack_weight / the wrapper's pack_weight): the 16 x 128 block
 // of a tile and a macro-step lies in 4 KB of its own, ordered [j][lane][8] as the lanes load it,
@@ -32,11 +37,13 @@
 #include "lane_moves.h"
 #include "gate_act.h"
 #include "kv_layout.h"
+#include "quad_rows.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
+constexpr int SK_MAX_LDX = 1 << 24;
 enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_ADD_F32 = 2, EPI_SWIGLU = 3, EPI_ADD_NORM = 4, EPI_QKV_ROPE = 5, EPI_STREAMS = 6 };
 
 // What two epilogues need beside Y, so that no kernel stands between a projection that ends
@@ -93,10 +100,11 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-template <int NT, int MT>
+// LOADS: loads of 128 k of sixteen rows of X (quad_rows.h): fewer than four for up to eight rows.
+template <int NT, int MT, int LOADS>
 struct Frag {
     u32x4 w[NT][4];
-    u32x4 x[MT][4];
+    u32x4 x[MT][LOADS];
 };
 
 // A weight is read once per product and never again before the caches have turned over: the loads of a packed
@@ -107,11 +115,12 @@ struct Frag {
 // decode step of 8 requests took 5.5 ms with them and plain rows).
 __device__ __forceinline__ u32x4 stream_load(const u32x4 *p) { return __builtin_nontemporal_load(p); }
 
-// The lane's loads of macro-step s: k = 128 s + 32 grp + 8 j .. + 7 for j = 0..3.
-template <int NT, int MT, bool PACKED>
-__device__ __forceinline__ void load_frag(Frag<NT, MT> &f, const bf16_t *const (&wrow)[NT], const bf16_t *const (&xrow)[MT],
-                                          const bool (&xvalid)[MT], int s, int grp, int K) {
-    const int kb = 128 * s + 32 * grp;
+// The lane's loads of macro-step s: W's k = 128 s + 32 grp + 8 j .. + 7 for j = 0..3; X as quad_rows.h says, through a buffer that ends with the
+// last row's k (rows beyond it read zeros), x_place the lane's place in its first four rows and x_four the bytes of four rows.
+template <int NT, int MT, bool PACKED, int LOADS>
+__device__ __forceinline__ void load_frag(Frag<NT, MT, LOADS> &f, const bf16_t *const (&wrow)[NT], __amdgpu_buffer_rsrc_t xb, uint32_t x_place,
+                                          uint32_t x_four, int s, int lane, int K) {
+    const int grp = lane >> 4, kb = 128 * s + 32 * grp;
     const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
     if (128 * (s + 1) <= K) {
         // packed: wrow is the lane's place in the tile's first block; blocks are 2048 elements,
@@ -125,37 +134,42 @@ __device__ __forceinline__ void load_frag(Frag<NT, MT> &f, const bf16_t *const (
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) f.x[m][j] = xvalid[m] ? *(const u32x4 *)(xrow[m] + kb + 8 * j) : zero;
+            for (int i = 0; i < LOADS; ++i)
+                f.x[m][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, x_place + (4 * m + i) * x_four + 256u * s, 0, 0));
     } else {                                   // the last, partial macro-step (K is a multiple of 8)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int j = 0; j < 4; ++j) f.w[t][j] = (kb + 8 * j + 8 <= K) ? *(const u32x4 *)(wrow[t] + kb + 8 * j) : zero;
+        const bool in = 128 * s + quad_k(lane) + 8 <= K;         // (what lies behind a row's k may be NaN)
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                f.x[m][j] = (xvalid[m] && kb + 8 * j + 8 <= K) ? *(const u32x4 *)(xrow[m] + kb + 8 * j) : zero;
+            for (int i = 0; i < LOADS; ++i)
+                f.x[m][i] = in ? __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, x_place + (4 * m + i) * x_four + 256u * s, 0, 0)) : zero;
     }
 }
 
-template <int NT, int MT>
-__device__ __forceinline__ void mul_frag(const Frag<NT, MT> &f, f32x4 (&acc)[NT][MT]) {
+template <int NT, int MT, int LOADS>
+__device__ __forceinline__ void mul_frag(const Frag<NT, MT, LOADS> &f, f32x4 (&acc)[NT][MT]) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int m = 0; m < MT; ++m) {
+        u32x4 x[4];
+        quad_operands<LOADS>(f.x[m], x);
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int m = 0; m < MT; ++m) acc[t][m] = mfma16(f.w[t][j], f.x[m][j], acc[t][m]);
+            for (int t = 0; t < NT; ++t) acc[t][m] = mfma16(f.w[t][j], x[j], acc[t][m]);
+    }
 }
 
-template <int NT, int MT, int EPI, int SK_WAVES, bool PACKED>
+template <int NT, int MT, int EPI, int SK_WAVES, bool PACKED, int LOADS>
 __global__ void __launch_bounds__(SK_WAVES *WAVE)
 gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict__ W, int ldw, void *__restrict__ Y,
                    int ldy, int M, int N, int K, SkinnyExtra ex) {
     __shared__ float red[SK_WAVES][NT * MT * 4][WAVE];
     __shared__ float row_scale[16 * MT];
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int l16 = lane & 15, grp = lane >> 4;
     // the rows of W of tile t: for SwiGLU tile 0 are gate rows, tile 1 the up rows N/2 further
     const int n_out = EPI == EPI_SWIGLU ? N / 2 : N;                 // width of Y
@@ -176,13 +190,11 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
                            : W + (size_t)row * ldw;
     }
     if (ex.group_rows > 0) X += (size_t)(n0 / ex.group_rows) * ex.x_group_stride;      // (a workgroup's rows lie in one group)
-    const bf16_t *xrow[MT];
-    bool xvalid[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        xvalid[m] = 16 * m + l16 < M;
-        xrow[m] = X + (size_t)(xvalid[m] ? 16 * m + l16 : 0) * ldx;
-    }
+    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(X), 0, (uint32_t)((M - 1) * ldx + K) * 2u, 0x00020000);
+    uint32_t x_place = (uint32_t)(quad_load_row(0, lane) * ldx + quad_k(lane)) * 2u;
+    asm("" : "+v"(x_place));                    // (else every tile's place is multiplied out in front of the loop, a register each)
+    const uint32_t x_four = 8u * ldx;
+    const int col = quad_row(l16);              // the token of the tile that the lane's column of the products is
     f32x4 acc[NT][MT];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -221,21 +233,21 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
 
     // A ring of STAGES macro-steps in flight per wave: with few workgroups per compute unit
     // (small N) this is what keeps enough bytes on their way from HBM.
-    constexpr int STAGES = NT * MT == 1 ? 4 : (NT * MT == 2 ? 3 : 2);
+    constexpr int STAGES = NT * MT == 1 ? 4 : NT * MT == 2 ? 3 : NT * MT == 8 && SK_WAVES == 8 ? 1 : 2;      // (the last for want of registers)
     const int nsteps = (K + 127) / 128;
-    Frag<NT, MT> f[STAGES];
+    Frag<NT, MT, LOADS> f[STAGES];
     int s = wave;
 #pragma unroll
     for (int i = 0; i < STAGES; ++i)
-        if (s + i * SK_WAVES < nsteps) load_frag<NT, MT, PACKED>(f[i], wrow, xrow, xvalid, s + i * SK_WAVES, grp, K);
+        if (s + i * SK_WAVES < nsteps) load_frag<NT, MT, PACKED, LOADS>(f[i], wrow, xb, x_place, x_four, s + i * SK_WAVES, lane, K);
     for (; s < nsteps; s += STAGES * SK_WAVES) {
 #pragma unroll
         for (int i = 0; i < STAGES; ++i) {
             const int cur = s + i * SK_WAVES;
             if (cur < nsteps) {
-                mul_frag<NT, MT>(f[i], acc);
+                mul_frag<NT, MT, LOADS>(f[i], acc);
                 if (cur + STAGES * SK_WAVES < nsteps)
-                    load_frag<NT, MT, PACKED>(f[i], wrow, xrow, xvalid, cur + STAGES * SK_WAVES, grp, K);
+                    load_frag<NT, MT, PACKED, LOADS>(f[i], wrow, xb, x_place, x_four, cur + STAGES * SK_WAVES, lane, K);
             }
         }
     }
@@ -260,11 +272,11 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
                 for (int w = 1; w < SK_WAVES; ++w) sum += red[w][i][lane];
                 acc[t][m][r] = sum;
             }
-    // ---- epilogue: the lane holds, per tile, features 4 grp + r of token 16 m + l16
+    // ---- epilogue: the lane holds, per tile, features 4 grp + r of token 16 m + col
     if (EPI != EPI_ADD_NORM && ex.sumsq_in != nullptr) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            const float rs = row_scale[16 * m + l16];
+            const float rs = row_scale[16 * m + col];
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -272,12 +284,12 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
         }
     }
     if (EPI == EPI_QKV_ROPE) {
-        // the lane holds dims i = 16 c + 4 grp + r (tile 0) and i + head_dim/2 (tile 1) of token 16 m + l16
+        // the lane holds dims i = 16 c + 4 grp + r (tile 0) and i + head_dim/2 (tile 1) of token 16 m + col
         const int dh = ex.head_dim, half_dim = dh / 2;
         const bool is_q = rope_head < ex.heads, is_k = !is_q && rope_head < ex.heads + ex.kv_heads;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            const int tok = 16 * m + l16;
+            const int tok = 16 * m + col;
             if (tok >= M) continue;
             const int pos = ex.positions[tok];
             const bool in_table = pos >= 0 && pos < ex.max_pos;
@@ -326,7 +338,7 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
         const int S = ex.streams;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            const int tok = 16 * m + l16;
+            const int tok = 16 * m + col;
             float ss = 0.f;
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
@@ -364,7 +376,7 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
     if (EPI == EPI_ADD_NORM) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            const int tok = 16 * m + l16;
+            const int tok = 16 * m + col;
             float ss = 0.f;
 #pragma unroll
             for (int t = 0; t < NT; ++t)
@@ -387,7 +399,7 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        const int tok = 16 * m + l16;
+        const int tok = 16 * m + col;
         if (tok >= M) continue;
         if (EPI == EPI_SWIGLU) {
 #pragma unroll
@@ -420,6 +432,18 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
     }
 }
 
+// (plain rows of W take their time whatever the rows of X do)
+#define RUN(E, GRID, BLOCK)                                                            \
+    do {                                                                               \
+        if (!packed) RUN_AS(E, GRID, BLOCK, false, 4);                                 \
+        else if constexpr (MT > 1) RUN_AS(E, GRID, BLOCK, true, 4);                    \
+        else if (M <= 4) RUN_AS(E, GRID, BLOCK, true, 1);                              \
+        else if (M <= 8) RUN_AS(E, GRID, BLOCK, true, 2);                              \
+        else RUN_AS(E, GRID, BLOCK, true, 4);                                          \
+    } while (0)
+#define RUN_AS(E, GRID, BLOCK, PACKED, LOADS)                                                                                \
+    gemm_skinny_kernel<NT, MT, E, WAVES, PACKED, LOADS><<<GRID, BLOCK, 0, stream>>>((const bf16_t *)X, ldx, (const bf16_t *)W, ldw, Y, ldy, M, N, K, ex)
+
 template <int NT, int MT, int WAVES>
 static int launch_epi(const void *X, int ldx, const void *W, int ldw, void *Y, int ldy, int M, int N, int K, int epi,
                       int packed, const SkinnyExtra &ex, hipStream_t stream) {
@@ -427,8 +451,7 @@ static int launch_epi(const void *X, int ldx, const void *W, int ldw, void *Y, i
     const dim3 grid((N + 16 * NT - 1) / (16 * NT));
 #define GO(E)                                                                                                                      \
     do {                                                                                                                           \
-        if (packed) gemm_skinny_kernel<NT, MT, E, WAVES, true><<<grid, block, 0, stream>>>((const bf16_t *)X, ldx, (const bf16_t *)W, ldw, Y, ldy, M, N, K, ex); \
-        else gemm_skinny_kernel<NT, MT, E, WAVES, false><<<grid, block, 0, stream>>>((const bf16_t *)X, ldx, (const bf16_t *)W, ldw, Y, ldy, M, N, K, ex);       \
+        RUN(E, grid, block);                                                                                                       \
     } while (0)
     switch (epi) {
     case EPI_BF16: GO(EPI_BF16); break;
@@ -443,10 +466,7 @@ static int launch_epi(const void *X, int ldx, const void *W, int ldw, void *Y, i
     case EPI_QKV_ROPE:
         if constexpr (MT <= 2 && NT == 2) {
             const dim3 rgrid((ex.heads + 2 * ex.kv_heads) * (ex.head_dim / 32));
-            if (packed) gemm_skinny_kernel<NT, MT, EPI_QKV_ROPE, WAVES, true><<<rgrid, block, 0, stream>>>(
-                (const bf16_t *)X, ldx, (const bf16_t *)W, ldw, Y, ldy, M, N, K, ex);
-            else gemm_skinny_kernel<NT, MT, EPI_QKV_ROPE, WAVES, false><<<rgrid, block, 0, stream>>>(
-                (const bf16_t *)X, ldx, (const bf16_t *)W, ldw, Y, ldy, M, N, K, ex);
+            RUN(EPI_QKV_ROPE, rgrid, block);
             break;
         }
         return LCU_UNSUPPORTED;
@@ -461,13 +481,11 @@ template <int NT, int MT, int WAVES>
 static int launch_swiglu(const void *X, int ldx, const void *W, int ldw, void *Y, int ldy, int M, int N, int K,
                          int packed, const SkinnyExtra &ex, hipStream_t stream) {
     const int groups = (N / 2 + 8 * NT - 1) / (8 * NT);
-    if (packed) gemm_skinny_kernel<NT, MT, EPI_SWIGLU, WAVES, true><<<dim3(groups), dim3(WAVES * WAVE), 0, stream>>>(
-        (const bf16_t *)X, ldx, (const bf16_t *)W, ldw, Y, ldy, M, N, K, ex);
-    else gemm_skinny_kernel<NT, MT, EPI_SWIGLU, WAVES, false><<<dim3(groups), dim3(WAVES * WAVE), 0, stream>>>(
-        (const bf16_t *)X, ldx, (const bf16_t *)W, ldw, Y, ldy, M, N, K, ex);
+    RUN(EPI_SWIGLU, dim3(groups), dim3(WAVES * WAVE));
     LCU_LAUNCH_CHECK();
     return LCU_OK;
 }
+#undef RUN
 
 // X: [M, K] bfloat16 rows ldx apart; W: [N, K] bfloat16 rows ldw apart; Y: [M, N] rows ldy
 // apart (for the SwiGLU epilogue [M, N/2]: W holds N/2 gate rows, then N/2 up rows).
@@ -479,7 +497,7 @@ static int skinny_bf16(const void *X, int ldx, const void *W, int ldw, void *Y, 
     if (M <= 0 || N <= 0) return LCU_OK;
     // a packed weight is whole blocks of 16 rows x 128 k (and for SwiGLU each half is)
     if (packed && (K % 128 || N % 16 || (epilogue == EPI_SWIGLU && N % 32))) return LCU_BAD_ARGUMENT;
-    if (M > 32 || K <= 0 || K % 8 || ldx % 8 || ldw % 8 || ldx < K || ldw < K) return LCU_BAD_ARGUMENT;
+    if (M > 32 || K <= 0 || K % 8 || ldx % 8 || ldw % 8 || ldx < K || ldw < K || ldx >= SK_MAX_LDX) return LCU_BAD_ARGUMENT;      // (a load's place in the rows is 32 bits)
     if (waves != 4 && waves != 8) return LCU_BAD_ARGUMENT;
     const int mt = (M + 15) / 16;
     if (epilogue == EPI_SWIGLU) {
@@ -620,9 +638,9 @@ LCU_API int lcu_gemm_skinny_bf16_qkv_rope(const void *X, int ldx, const void *W,
 // rows may wait for their normalisation (sumsq_in), the result may go into the residual stream, with the next norm's weight on its
 // way out (norm_w), and gate and up rows may meet in SwiGLU (PAIR: the matrix tile's sixteen rows are eight gate rows and the eight up rows
 // that meet them, so that there are as many workgroups as without).  What
-// bounds it at few tokens is latency (a launch, one round of loads, 0.9 us of matrix instructions), not the matrix: us at 2 tokens, 1024 x 1024
-// 5.5, with the rows' factor 5.9, with residual and norm weight 6.2, SwiGLU of 2816 x 1024 6.5 (and 3.3 and 3.5 for the kernels that ran
-// between); 32000 x 1024 32.5 (4.0 TB/s).
+// bounds it at few tokens is latency (a launch, one round of loads, 0.9 us of matrix instructions), not the matrix: us at 2 tokens, matrices out of
+// memory, 1024 x 1024 4.8, SwiGLU of 2816 x 1024 6.4; 32000 x 1024 29 (4.5 TB/s).  At 250 tokens 1024 x 1024 10.8, 2048 x 2048 34.2.  With both operands loaded
+// in the operands' order (a cycle a lane, quad_rows.h) they were 5.0, 6.7, 33.6, 14.5 and 50.5.
 constexpr int F32_WAVES = 8;
 
 struct F32Extra {
@@ -633,61 +651,37 @@ struct F32Extra {
     float act_alpha, act_limit;
 };
 
-template <int MT>
-struct FragF32 {
-    f32x4 w[4];
-    f32x4 x[MT][4];
-};
-
-template <int MT>
-__device__ __forceinline__ void load_frag_f32(FragF32<MT> &f, const float *wrow, const float *const (&xrow)[MT],
-                                              const bool (&xvalid)[MT], int s, int grp, int K) {
-    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int kb = 64 * s + 16 * j + 4 * grp;
-        const bool in = kb + 4 <= K;                        // K is a multiple of 4
-        f.w[j] = in ? *(const f32x4 *)(wrow + kb) : zero;
-#pragma unroll
-        for (int m = 0; m < MT; ++m) f.x[m][j] = (in && xvalid[m]) ? *(const f32x4 *)(xrow[m] + kb) : zero;
-    }
-}
-
-template <int MT>
-__device__ __forceinline__ void mul_frag_f32(const FragF32<MT> &f, f32x4 (&acc)[MT]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[j][e], f.x[m][j][e], acc[m], 0, 0, 0);
-}
-
+// Both operands come in by quads of lanes (quad_rows.h, four k where bfloat16 has eight): W's load i brings lane (g, a, b) row 4 a + i, so that
+// the operands' rows are in order, X's row 4 i + a, so that few rows take fewer loads; operand j then holds k = 64 s + 16 g + 4 j .. of its row.
 // PAIR: SwiGLU; SCALED: with sumsq_in; ADDS: accumulate or norm_w
-template <int MT, bool PAIR, bool SCALED, bool ADDS>
-__global__ void __launch_bounds__(F32_WAVES *WAVE)
+template <int MT, bool PAIR, bool SCALED, bool ADDS, int LOADS>
+__global__ void __launch_bounds__(F32_WAVES *WAVE, MT == 1 && !(ADDS && LOADS == 4) ? 4 : 2)      // (two workgroups of sixteen rows a compute unit: 32000 x 1024 at 16 rows 41 us, with one 46)
 gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W, int ldw, float *__restrict__ Y,
                        int ldy, int M, int N, int K, F32Extra ex) {
     __shared__ f32x4 red[F32_WAVES][MT][WAVE];
     __shared__ float factor[16 * MT];
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-    const int l16 = lane & 15, grp = lane >> 4;
+    const int l16 = lane & 15, grp = lane >> 4, col = quad_row(l16);      // (the token of the tile that the lane's column is)
     const int n0 = blockIdx.x * (PAIR ? 8 : 16), m0 = blockIdx.y * 16 * MT;
     // (a row beyond the end is read, not stored)
-    const float *wrow = W + (size_t)(PAIR ? min(n0 + (l16 & 7), N - 1) + (l16 < 8 ? 0 : N) : min(n0 + l16, N - 1)) * ldw;
-    const float *xrow[MT];
-    bool xvalid[MT];
+    const float *wrow[4];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        xvalid[m] = m0 + 16 * m + l16 < M;
-        xrow[m] = X + (size_t)(xvalid[m] ? m0 + 16 * m + l16 : 0) * ldx;
+    for (int i = 0; i < 4; ++i) {
+        const int r = 4 * ((lane >> 2) & 3) + i;
+        wrow[i] = W + (size_t)(PAIR ? min(n0 + (r & 7), N - 1) + (r < 8 ? 0 : N) : min(n0 + r, N - 1)) * ldw;
     }
+    // X's rows from the workgroup's first on, up to the last one's k: rows beyond it read zeros
+    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(X + (size_t)m0 * ldx), 0,
+                                                                       (uint32_t)(min(M - 1 - m0, 16 * MT - 1) * ldx + K) * 4u, 0x00020000);
+    uint32_t x_place = (uint32_t)(quad_load_row(0, lane) * ldx + 16 * (lane >> 4) + 4 * (lane & 3)) * 4u;
+    asm("" : "+v"(x_place));                                 // (else every tile's place is multiplied out in front of the loop, a register each)
+    const uint32_t x_four = 16u * ldx;
     f32x4 acc[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int nsteps = (K + 63) / 64;
     // a wave stores sixteen tokens in the end; what it adds to, and the norm's weights, are on their way meanwhile
-    const int tok = m0 + 16 * wave + l16;
+    const int tok = m0 + 16 * wave + col;
     float old[4] = {}, nw[4] = {};
     if (ADDS && wave < MT) {
 #pragma unroll
@@ -699,10 +693,32 @@ gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__rest
             }
         }
     }
-    FragF32<MT> fa, fb;
+    // macro-steps whose loads are on their way: of the matrix two, of up to eight rows two, of more rows a tile's next when it is used
+    constexpr int ROWS_AHEAD = LOADS < 4 ? 2 : 1, AHEAD = 2;
+    quad_u32x4 w[AHEAD][4], x[ROWS_AHEAD][MT][LOADS];
+    const quad_u32x4 zero = quad_u32x4{0u, 0u, 0u, 0u};
+    const int k_lane = 16 * grp + 4 * (lane & 3);            // (K is a multiple of 4)
+    auto load_w = [&](int u, int s) {
+        const bool in = 64 * s + k_lane + 4 <= K;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[u][i] = in ? *(const quad_u32x4 *)(wrow[i] + 64 * s + k_lane) : zero;
+    };
+    auto load_x = [&](int u, int m, int s) {
+        const bool in = 64 * s + k_lane + 4 <= K;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            x[u][m][i] = in ? __builtin_bit_cast(quad_u32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, x_place + (4 * m + i) * x_four + 256u * s, 0, 0)) : zero;
+    };
     int s = wave;
-    if (s < nsteps) load_frag_f32<MT>(fa, wrow, xrow, xvalid, s, grp, K);
-    if (s + F32_WAVES < nsteps) load_frag_f32<MT>(fb, wrow, xrow, xvalid, s + F32_WAVES, grp, K);
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+        if (s + u * F32_WAVES < nsteps) load_w(u, s + u * F32_WAVES);
+#pragma unroll
+    for (int u = 0; u < ROWS_AHEAD; ++u)
+        if (s + u * F32_WAVES < nsteps) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) load_x(u, m, s + u * F32_WAVES);
+        }
     if constexpr (SCALED) {
         for (int r = wave; r < 16 * MT && m0 + r < M; r += F32_WAVES) {
             float t = 0.f;
@@ -711,11 +727,26 @@ gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__rest
             if (lane == 0) factor[r] = rsqrtf(t / (float)ex.norm_width + ex.eps);
         }
     }
-    for (; s < nsteps; s += 2 * F32_WAVES) {
-        mul_frag_f32<MT>(fa, acc);
-        if (s + 2 * F32_WAVES < nsteps) load_frag_f32<MT>(fa, wrow, xrow, xvalid, s + 2 * F32_WAVES, grp, K);
-        if (s + F32_WAVES < nsteps) mul_frag_f32<MT>(fb, acc);
-        if (s + 3 * F32_WAVES < nsteps) load_frag_f32<MT>(fb, wrow, xrow, xvalid, s + 3 * F32_WAVES, grp, K);
+    for (; s < nsteps; s += AHEAD * F32_WAVES) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int cur = s + u * F32_WAVES;
+            if (cur >= nsteps) break;
+            quad_u32x4 wt[4];
+            quad_operands<4>(w[u], wt);
+            if (cur + AHEAD * F32_WAVES < nsteps) load_w(u, cur + AHEAD * F32_WAVES);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                quad_u32x4 xt[4];
+                quad_operands<LOADS>(x[u % ROWS_AHEAD][m], xt);
+                if (cur + ROWS_AHEAD * F32_WAVES < nsteps) load_x(u % ROWS_AHEAD, m, cur + ROWS_AHEAD * F32_WAVES);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(wt[j][e]), __uint_as_float(xt[j][e]), acc[m], 0, 0, 0);
+            }
+        }
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m) red[wave][m][lane] = acc[m];
@@ -724,7 +755,7 @@ gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__rest
     f32x4 sum = red[0][wave][lane];
 #pragma unroll
     for (int w = 1; w < F32_WAVES; ++w) sum += red[w][wave][lane];
-    if constexpr (SCALED) sum *= factor[16 * wave + l16];
+    if constexpr (SCALED) sum *= factor[16 * wave + col];
     if constexpr (PAIR) {                                    // the up rows' sums are 32 lanes further
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -763,25 +794,27 @@ LCU_API int lcu_gemm_skinny_f32(const float *X, int ldx, const float *W, int ldw
                                 int K, int accumulate, float scale, int swiglu, const float *sumsq_in, int n_in, int norm_width, float eps,
                                 const float *norm_w, float *h_out, int ldh, float *sumsq_out, float act_alpha, float act_limit, hipStream_t stream) {
     if (M <= 0 || N <= 0) return LCU_OK;
-    if (K <= 0 || K % 4 || ldx % 4 || ldw % 4 || ldx < K || ldw < K || ldy < N) return LCU_BAD_ARGUMENT;
+    if (K <= 0 || K % 4 || ldx % 4 || ldw % 4 || ldx < K || ldw < K || ldy < N || ldx >= SK_MAX_LDX) return LCU_BAD_ARGUMENT;
     if ((sumsq_in && (n_in <= 0 || norm_width <= 0)) || (norm_w && (!h_out || !sumsq_out || ldh < N || swiglu)) || (swiglu && accumulate))
         return LCU_BAD_ARGUMENT;
     F32Extra ex = {accumulate, scale, sumsq_in, n_in, norm_width, eps, norm_w, h_out, ldh, sumsq_out, act_alpha, act_limit};
     // 16 tokens a workgroup, each of which reads its rows of W (from the L2 caches, but for the first), while the matrix instructions are
     // what takes the time: up to 32 tokens, and up to three workgroups a compute unit.  One MI355X, us with 16 / 64 tokens a
-    // workgroup: 1024 x 1024 at 62 tokens 6.8 / 14.6, at 128 10.5 / 15.0, at 250 (1,024 workgroups) 18.2 / 15.0; 2816 x 1024 at 62 (704) 15.0 / 16.1;
-    // 32000 x 1024 at 62 127 / 117, at 32 70 (77 with 32 tokens a workgroup).
+    // workgroup: 1024 x 1024 at 62 tokens 6.1 / 10.4, at 128 8.1 / 10.5, at 250 (1,024 workgroups) 13.8 / 10.8; 1536 x 1024 at 128 (768) 11.4 / 11.4; SwiGLU of
+    // 2816 x 1024 at 62 (704) 12.1 / 11.8; 32000 x 1024 at 62 96 / 83, at 32 58 / 81; 2048 x 2048 at 62 (512) 14.5 / 18.3, at 128 (1,024) 22.8 / 18.8.
     const int rows = M <= 32 || ((N + 15) / 16) * ((M + 15) / 16) <= 768 ? 16 : 64;
     const int tiles = (M + rows - 1) / rows;
     if (tiles > 65535) return LCU_BAD_ARGUMENT;
     const dim3 grid(swiglu ? (N + 7) / 8 : (N + 15) / 16, tiles), block(F32_WAVES * WAVE);
     // What a product does besides is known when it is compiled: a form that looks at F32Extra for it, behind the loads that are on their way, took
     // 4.9 us for two rows of 1024 x 1024 with the matrix in the caches and 2.5 for 64 x 64, now 4.6 and 2.3.
-#define GO(MT, PAIR, SCALED, ADDS) gemm_skinny_f32_kernel<MT, PAIR, SCALED, ADDS><<<grid, block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, ex)
-#define ROWS(MT, PAIR, ADDS) do { if (sumsq_in) GO(MT, PAIR, true, ADDS); else GO(MT, PAIR, false, ADDS); } while (0)
-#define FORMS(MT) do { if (swiglu) ROWS(MT, true, false); else if (accumulate || norm_w) ROWS(MT, false, true); else ROWS(MT, false, false); } while (0)
-    if (rows == 16) FORMS(1);
-    else FORMS(4);
+#define GO(MT, PAIR, SCALED, ADDS, LOADS) gemm_skinny_f32_kernel<MT, PAIR, SCALED, ADDS, LOADS><<<grid, block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, ex)
+#define ROWS(MT, PAIR, ADDS, LOADS) do { if (sumsq_in) GO(MT, PAIR, true, ADDS, LOADS); else GO(MT, PAIR, false, ADDS, LOADS); } while (0)
+#define FORMS(MT, LOADS) do { if (swiglu) ROWS(MT, true, false, LOADS); else if (accumulate || norm_w) ROWS(MT, false, true, LOADS); else ROWS(MT, false, false, LOADS); } while (0)
+    if (rows > 16) FORMS(4, 4);
+    else if (M <= 4) FORMS(1, 1);
+    else if (M <= 8) FORMS(1, 2);
+    else FORMS(1, 4);
 #undef FORMS
 #undef ROWS
 #undef GO

@@ -1,0 +1,98 @@
+"""Products whose rows come in by quads of lanes (``quad_rows.h``), at the edges of the loads' and the tiles' row counts.  Operands are small whole numbers,
+whose products and sums are whole numbers below 2^24: every result is the exact one or a row or a k is in the wrong place."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def whole(shape, seed, lo=-3, hi=4):
+    return torch.randint(lo, hi, shape, generator=torch.Generator().manual_seed(seed)).double()
+
+
+def rows_of(x, rows_behind=0):
+    """``x`` on the GPU as rows of a wider array whose other elements are NaN."""
+    wide = torch.full((x.shape[0] + rows_behind, x.shape[1] + 16), float("nan"), dtype=BF16, device="cuda")
+    wide[:x.shape[0], 8:8 + x.shape[1]] = x.to(BF16).cuda()
+    return wide[:x.shape[0], 8:8 + x.shape[1]]
+
+
+@pytest.mark.parametrize("m", [1, 3, 4, 5, 7, 8, 9, 15, 16, 17, 24, 31, 32])
+def test_few_rows(m):
+    from llama_cu_amd.kernels import ops
+    for n, k, tiles in ((48, 256, 1), (80, 1408, 2), (64, 640, 4), (16, 6400, 1)):
+        x, w = whole((m, k), 1), whole((n, k), 2)
+        want, rows, wg = x @ w.t(), rows_of(x, m % 2), w.to(BF16).cuda()
+        for waves in (4, 8):
+            for weight, packed in ((wg, False), (ops.pack_weight(wg), True)):
+                got = ops.gemm_skinny(rows, weight, out_dtype=torch.float32, tiles=tiles, waves=waves, packed=packed)
+                assert torch.equal(got.cpu().double(), want), (n, k, tiles, waves, packed)
+    x, w = whole((m, 200), 3), whole((40, 200), 4)           # a last macro-step that is not whole, NaN behind it
+    assert torch.equal(ops.gemm_skinny(rows_of(x), w.to(BF16).cuda(), out_dtype=torch.float32).cpu().double(), x @ w.t())
+
+
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16, 17, 32, 33, 48, 49, 63, 64])
+def test_waves_that_share_out_k(m):
+    from llama_cu_amd.kernels import ops
+    for n, k in ((48, 128), (4112, 256), (80, 1152), (32, 2176), (16, 6400)):
+        x, w = whole((m, k), 5), whole((n, k), 6)
+        got = ops.gemm_wavek(rows_of(x, m % 2), ops.pack_weight(w.to(BF16).cuda()), out_dtype=torch.float32)
+        assert torch.equal(got.cpu().double(), x @ w.t()), (n, k)
+    x, w = whole((m, 3 * 128), 7), whole((3 * 16, 128), 8)
+    got = ops.gemm_wavek(rows_of(x).unflatten(1, (3, 128)).transpose(0, 1), ops.pack_weight(w.to(BF16).cuda()), out_dtype=torch.float32)
+    assert torch.equal(got.cpu().double(), torch.cat([x[:, 128 * g:128 * g + 128] @ w[16 * g:16 * g + 16].t() for g in range(3)], 1))
+
+
+@pytest.mark.parametrize("m", [2, 5, 16, 33, 48, 49, 64])
+@pytest.mark.parametrize("heads,kv_heads,dim,k", [(4, 1, 64, 256), (3, 2, 128, 1152), (2, 2, 32, 128)])
+def test_q_k_v_as_the_row_sharing_kernel_makes_them(m, heads, kv_heads, dim, k):
+    """Exact sums, so both kernels round, rotate and store the same numbers; positions beyond the table and tokens without a place among them."""
+    from llama_cu_amd.kernels import ops
+    x = rows_of(whole((m, k), 9))
+    w = ops.pack_weight(whole(((heads + 2 * kv_heads) * dim, k), 10).to(BF16).cuda())
+    pos = torch.arange(m, dtype=torch.int32) * 3 % 50
+    slots = torch.randperm(80, generator=torch.Generator().manual_seed(11))[:m].to(torch.int32)
+    pos[m // 2], slots[m - 1] = 70, -1
+    ang = torch.arange(64)[:, None] * torch.linspace(0.1, 1.0, dim // 2)[None]
+    tables = torch.cos(ang).cuda().contiguous(), torch.sin(ang).cuda().contiguous()
+    caches = [torch.zeros(5, 2, kv_heads * dim * 16, dtype=BF16, device="cuda") for _ in range(2)]
+    a = ops.gemm_wavek_qkv_rope(x, w, pos.cuda(), slots.cuda(), *tables, caches[0], heads, kv_heads, dim, 16)
+    b = ops.gemm_mid_qkv_rope(x, w, pos.cuda(), slots.cuda(), *tables, caches[1], heads, kv_heads, dim, 16, packed=True)
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16)) and torch.equal(caches[0].view(torch.int16), caches[1].view(torch.int16))
+
+
+def test_rows_far_apart():
+    from llama_cu_amd.kernels import ops
+    x, w = whole((2, 128), 12), whole((32, 128), 13)
+    far = torch.empty(2, 1 << 24, dtype=BF16, device="cuda")[:, :128]
+    far.copy_(x.to(BF16))
+    packed = ops.pack_weight(w.to(BF16).cuda())
+    for got in (ops.gemm_skinny(far, packed, out_dtype=torch.float32, packed=True), ops.gemm_wavek(far, packed, out_dtype=torch.float32)):
+        assert torch.equal(got.cpu().double(), x @ w.t())
+
+
+@pytest.mark.parametrize("m", [33, 64])
+def test_which_kernel_makes_q_k_v(m, monkeypatch):
+    from llama_cu_amd.kernels import ops
+    from llama_cu_amd.parts.linear import Weight, linear_qkv_rope
+    calls = []
+    real = ops.gemm_wavek_qkv_rope
+    monkeypatch.setattr(ops, "gemm_wavek_qkv_rope", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    x, z = rows_of(whole((m, 256), 14)), torch.zeros(m, dtype=torch.int32, device="cuda")
+    weight = Weight(whole((6 * 64, 256), 15).to(BF16).cuda())
+    table, cache = torch.ones(8, 32, device="cuda"), torch.zeros(1, 2, 64 * 16, dtype=BF16, device="cuda")
+    got = linear_qkv_rope(x, weight, z, z - 1, table, torch.zeros_like(table), cache, 4, 1, 64, 16)
+    assert calls and torch.equal(got.double().cpu(), (x.double().cpu() @ weight.plain[:256].double().cpu().t()).to(BF16).double())
+
+
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16, 17, 63, 64, 65, 900])
+def test_32_bit_rows(m):
+    from llama_cu_amd.kernels import ops
+    for n, k in ((16, 64), (72, 1088), (40, 68), (1024, 132), (32, 4160)):
+        x, w = whole((m, k), 16), whole((n, k), 17)
+        wide = torch.full((m, k + 8), float("nan"), device="cuda")
+        wide[:, 4:4 + k] = x.cuda()
+        assert torch.equal(ops.gemm_skinny_f32(wide[:, 4:4 + k], w.float().cuda()).cpu().double(), x @ w.t()), (n, k)
