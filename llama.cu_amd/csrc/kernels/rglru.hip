@@ -8,7 +8,7 @@
 //
 // Per request the state is [taps, width] floats: rows 0 .. taps-2 the last taps-1 rows of xin (oldest first), row
 // taps-1 the recurrence's S.  It is taken as zero where the request's first token of the step stands at position 0.
-// Two kernels: the convolution with the gates (a workgroup per tile of tokens, block of channels and tile of outputs; the
+// In general two kernels: the convolution with the gates (a workgroup per tile of tokens, block of channels and tile of outputs; the
 // block's two matrices are given transposed, [block][in][out], so that the lanes read neighbours), and the scan (a
 // thread per request and channel walks the request's tokens in their order, then leaves the state; the state is read by
 // the first kernel and written by the second alone).  Everything that does not depend on the token before (the gelu of
@@ -277,6 +277,285 @@ rglru_gates_rows_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
     }
 }
 
+// Blocks of a multiple of sixteen channels, up to RG_MFMA_BS: the gates' products on the 32-bit matrix instruction (true 32-bit products and
+// sums).  Lane (l, g) of 16 x 4 brings, of the sixteen k that four instructions take, those from 4 g on; the matrices stand in that order
+// (lcu_rglru), so that a wave's load is 1 KB in one piece.
+//
+// Many tokens: a workgroup takes 16 TT tokens and a block of channels, makes u for them (in LDS), and each of its waves takes 16 output
+// channels of both gates at a time.  One MI355X, width 2048 in 16 blocks, 4 taps, with the scan behind it: 8 requests of 235 tokens 68 us (a thread
+// an output channel and the sums on the vector unit: 105), 65 tokens 18 (47).  The matrix instructions are 14 us of the first, the functions (exp, expm1,
+// tanh) 15, the scan 30.
+constexpr int RG_MFMA_BS = 192, RG_MFMA_TAPS = 4, RG_MFMA_WIDE = 256, RG_MFMA_THREADS = 256;
+typedef __attribute__((ext_vector_type(4))) float rg_f32x4;
+
+// the matrices' four pieces from input channel k0 on for 16 output channels (beyond the end: times zeros of u)
+__device__ __forceinline__ void rg_fetch(rg_f32x4 (&w)[2][4], const float *__restrict__ gates, int block, int tile, int tiles, int lane, int k0) {
+    const float *at = gates + (size_t)(block * tiles + tile) * tiles * 512 + 4 * lane;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) w[q][j] = *(const rg_f32x4 *)(at + 512 * (k0 / 16 + j < tiles ? k0 / 16 + j : 0) + 256 * q);
+}
+
+template <class TI, int TT>
+__global__ void __launch_bounds__(RG_MFMA_THREADS, 3)
+rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, const float *__restrict__ bias,
+                        const float *__restrict__ conv_w, const float *__restrict__ conv_b, const float *__restrict__ state,
+                        const float *__restrict__ gates,
+                        const float *__restrict__ ba, const float *__restrict__ bi, const float *__restrict__ lam, float c_exp,
+                        float *__restrict__ a_out, float *__restrict__ gx_out, float *__restrict__ y_out, int y_off,
+                        const int *__restrict__ q_start, const int *__restrict__ ctx_len, const int *__restrict__ req_of_token,
+                        const int *__restrict__ state_slot, int n, int width, int bs, int taps) {
+    constexpr int TOK = 16 * TT, STEP = 64;                               // tokens; input channels whose columns are asked for together
+    extern __shared__ __attribute__((aligned(16))) float us_tile[];       // [TOK][ld], zeros from bs on
+    const int ld = (bs + STEP - 1) / STEP * STEP + 4;
+    const int b = blockIdx.y, tok0 = blockIdx.x * TOK, nt = min(TOK, n - tok0);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
+    const int tiles = bs / 16, waves = RG_MFMA_THREADS / WAVE;
+    rg_f32x4 w[2][4];
+    rg_fetch(w, gates, b, min(wave, tiles - 1), tiles, lane, 0);
+    // ---- u
+    if (taps <= RG_MFMA_TAPS) {
+        // a thread walks a run of the tokens for one channel, with the tokens before it at hand, sixteen at a time
+        __shared__ int first_row[TOK], ahead[TOK], slot_of[TOK];          // of a token's request: its first row, the tokens before that, its slot
+        if (threadIdx.x < TOK) {
+            const int r = req_of_token[tok0 + min((int)threadIdx.x, nt - 1)], t0 = q_start[r];
+            first_row[threadIdx.x] = t0;
+            ahead[threadIdx.x] = ctx_len[r] - (q_start[r + 1] - t0);
+            slot_of[threadIdx.x] = state_slot[r];
+        }
+        __syncthreads();
+        constexpr int BATCH = 16;
+        const int runs = max(1, min(TOK / BATCH, RG_MFMA_THREADS / bs)), per = (TOK + runs - 1) / runs;
+        for (int x = threadIdx.x; x < runs * bs; x += RG_MFMA_THREADS) {
+            const int i = x % bs, c = b * bs + i, s0 = x / bs * per, s1 = min(TOK, s0 + per);
+            const float bx = bias ? bias[x_off + c] : 0.f, cb = conv_b ? conv_b[c] : 0.f;
+            float cw[RG_MFMA_TAPS], v[RG_MFMA_TAPS];                      // v[j]: the token taps - 1 - j before the next one
+#pragma unroll
+            for (int j = 0; j < RG_MFMA_TAPS; ++j) cw[j] = conv_w[(size_t)c * taps + min(j, taps - 1)];
+            const TI *col = rows + x_off + c;
+            v[0] = 0.f;
+#pragma unroll
+            for (int j = 0; j < RG_MFMA_TAPS - 1; ++j)
+                v[j + 1] = to_f32(col[(size_t)max(0, min(n - 1, tok0 + s0 - (taps - 1 - j))) * row_stride]) + bx;
+            for (int tb = s0; tb < s1; tb += BATCH) {
+                float xs[BATCH];
+#pragma unroll
+                for (int e = 0; e < BATCH; ++e) xs[e] = to_f32(col[(size_t)min(n - 1, tok0 + tb + e) * row_stride]) + bx;
+#pragma unroll
+                for (int e = 0; e < BATCH; ++e) {
+                    const int tt = tb + e, t = tok0 + tt;
+                    if (tt >= s1) break;
+#pragma unroll
+                    for (int j = 0; j < RG_MFMA_TAPS - 1; ++j) v[j] = v[j + 1];
+#pragma unroll
+                    for (int j = 0; j < RG_MFMA_TAPS; ++j)
+                        if (j == taps - 1) v[j] = xs[e];
+                    float use[RG_MFMA_TAPS];
+#pragma unroll
+                    for (int j = 0; j < RG_MFMA_TAPS; ++j) use[j] = v[j];
+                    const int t0 = first_row[tt];
+                    if (t - t0 < taps - 1) {                              // (the tokens before it are not all in the step)
+                        const float *st = state + (size_t)slot_of[tt] * taps * width + c;
+#pragma unroll
+                        for (int j = 0; j < RG_MFMA_TAPS - 1; ++j) {
+                            const int m = t0 - (t - (taps - 1 - j));      // so many tokens before the step's first
+                            if (j < taps - 1 && m > 0) use[j] = ahead[tt] - m >= 0 ? st[(size_t)(taps - 1 - m) * width] : 0.f;
+                        }
+                    }
+                    float acc = cb;
+#pragma unroll
+                    for (int j = 0; j < RG_MFMA_TAPS; ++j)
+                        if (j < taps) acc = fmaf(cw[j], use[j], acc);
+                    us_tile[tt * ld + i] = tt < nt ? acc : 0.f;
+                }
+            }
+        }
+    } else {
+        for (int x = threadIdx.x; x < TOK * bs; x += RG_MFMA_THREADS) {
+            const int tt = x / bs, i = x % bs;
+            float acc = 0.f;
+            if (tt < nt) {
+                const int t = tok0 + tt, r = req_of_token[t], t0 = q_start[r];
+                const int first_pos = ctx_len[r] - (q_start[r + 1] - t0);
+                acc = conv_at(rows, row_stride, x_off, bias, conv_w, conv_b, state + (size_t)state_slot[r] * taps * width, t, t0, first_pos, b * bs + i, width, taps);
+            }
+            us_tile[tt * ld + i] = acc;
+        }
+    }
+    for (int x = threadIdx.x; x < TOK * (ld - 4 - bs); x += RG_MFMA_THREADS) us_tile[x / (ld - 4 - bs) * ld + bs + x % (ld - 4 - bs)] = 0.f;
+    __syncthreads();
+    // ---- the gates, 16 output channels at a time
+    for (int tile = wave; tile < tiles; tile += waves) {
+        const int o = 16 * tile + l16, c = b * bs + o;
+        int lane_tok = 4 * g;                                             // (opaque: else sixteen tokens' addresses are made in front of the loop)
+        asm volatile("" : "+v"(lane_tok));
+        const float l = lam[c], ba_c = ba[c], bi_c = bi[c], by = bias ? bias[y_off + c] : 0.f;
+        rg_f32x4 acc[2][TT];
+#pragma unroll
+        for (int m = 0; m < TT; ++m) acc[0][m] = acc[1][m] = rg_f32x4{0.f, 0.f, 0.f, 0.f};
+        if (tile != wave) rg_fetch(w, gates, b, tile, tiles, lane, 0);
+        for (int k = 0; k < bs; k += STEP) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int m = 0; m < TT; ++m) {
+                    const rg_f32x4 x = *(const rg_f32x4 *)(us_tile + (16 * m + l16) * ld + k + 16 * j + 4 * g);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) acc[q][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[q][j][e], acc[q][m], 0, 0, 0);
+                }
+            if (k + STEP < bs) rg_fetch(w, gates, b, tile, tiles, lane, k + STEP);
+        }
+        asm volatile("" : "+v"(lane_tok));
+        float y_in[TT][4];
+#pragma unroll
+        for (int m = 0; m < TT; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y_in[m][r] = to_f32(rows[(size_t)min(n - 1, tok0 + 16 * m + lane_tok + r) * row_stride + y_off + c]);
+        const float sp = l > 20.f ? l : log1pf(expf(l));                  // softplus
+#pragma unroll
+        for (int m = 0; m < TT; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int tt = 16 * m + lane_tok + r, t = tok0 + tt;
+                if (tt >= nt) continue;
+                const float gr = 1.0f / (1.0f + expf(-(acc[0][m][r] + ba_c)));
+                const float gate = 1.0f / (1.0f + expf(-(acc[1][m][r] + bi_c)));
+                const float log_a = -c_exp * gr * sp;
+                const float mult = sqrtf(-expm1f(2.0f * log_a));
+                a_out[tile_index(t, c, n)] = expf(log_a);
+                gx_out[tile_index(t, c, n)] = mult * gate * us_tile[tt * ld + o];
+                y_out[tile_index(t, c, n)] = gelu_tanh(y_in[m][r] + by);
+            }
+    }
+}
+
+// A step in which every request feeds one token (token i is request i's): the gates as above, the recurrence's step and the state's update in one
+// kernel.  A workgroup takes four tokens and a block of channels; whatever of a slot's state belongs to a channel is read and written by
+// its threads alone.  Eight waves share out the output channels and, where there are waves enough, the input channels (their sums are
+// added through LDS in a fixed order); then a thread an element for the functions, which with the lanes that hold the sums were four one after
+// the other, most of them of tokens that are not there.  Latency bounds it: four trips to memory, 1.7 us of matrix instructions.  One MI355X, 4 taps, us
+// beside the sliced kernel and the scan: width 2048 in 16 blocks 7.6 / 10.4 with 8 requests, 8.1 / 13.5 with 64; width 1024 in 16 blocks 5.6 / 7.9 with 8.
+constexpr int RG_ONE_TOK = 4, RG_ONE_THREADS = 512;
+__host__ __device__ inline int rg_one_parts(int tiles) { return max(1, min(RG_ONE_THREADS / WAVE / tiles, tiles)); }
+
+template <class TI, class T, int V>
+__global__ void __launch_bounds__(RG_ONE_THREADS)
+rglru_single_kernel(const TI *__restrict__ rows, int row_stride, int y_off, int x_off, const float *__restrict__ bias,
+                    const float *__restrict__ conv_w, const float *__restrict__ conv_b, float *__restrict__ state,
+                    const float *__restrict__ gates, const float *__restrict__ ba, const float *__restrict__ bi, const float *__restrict__ lam, float c_exp,
+                    T *__restrict__ out, const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int n, int width, int bs, int taps) {
+    extern __shared__ __attribute__((aligned(16))) float us_tile[];       // [4][ld], then the sums [parts][2][4][ld]
+    const int ld = bs + 4, b = blockIdx.y, tok0 = blockIdx.x * RG_ONE_TOK, nt = min(RG_ONE_TOK, n - tok0);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
+    const int tiles = bs / 16, parts = rg_one_parts(tiles), items = tiles * parts;      // 16 output channels and a part of the input channels
+    float *sums = us_tile + RG_ONE_TOK * ld;
+    rg_f32x4 w[2][4];
+    if (wave < items) rg_fetch(w, gates, b, wave % tiles, tiles, lane, wave / tiles * tiles / parts * 16);
+    // ---- u, V neighbouring channels of a token a thread
+    typedef float fv __attribute__((ext_vector_type(V)));
+    auto load = [](const float *q) { return *(const fv *)q; };
+    for (int x = threadIdx.x; x < nt * (bs / V); x += RG_ONE_THREADS) {
+        const int tt = x / (bs / V), i = x % (bs / V) * V, c = b * bs + i, t = tok0 + tt;
+        const int before = ctx_len[t] - 1;                                // how many tokens the request has behind it
+        float *st = state + (size_t)state_slot[t] * taps * width + c;
+        const TI *xp = rows + (size_t)t * row_stride + x_off + c;
+        fv here, old[RG_MFMA_TAPS - 1], acc = {}, zero = {};
+        if constexpr (V == 1) here[0] = to_f32(xp[0]);
+        else if constexpr (sizeof(TI) == 4) here = load((const float *)xp);
+        else {
+            const uint2 two = *(const uint2 *)xp;
+            here = fv{__uint_as_float(two.x << 16), __uint_as_float(two.x & 0xffff0000u), __uint_as_float(two.y << 16), __uint_as_float(two.y & 0xffff0000u)};
+        }
+        float cw[V * RG_MFMA_TAPS];
+        if (V == 4 && taps == 4) {
+#pragma unroll
+            for (int k = 0; k < V; ++k) {
+                const float4 four = *(const float4 *)(conv_w + (size_t)c * 4 + 4 * k);
+                cw[4 * k] = four.x; cw[4 * k + 1] = four.y; cw[4 * k + 2] = four.z; cw[4 * k + 3] = four.w;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < V; ++k)
+#pragma unroll
+                for (int j = 0; j < RG_MFMA_TAPS; ++j) cw[4 * k + j] = conv_w[(size_t)(c + k) * taps + min(j, taps - 1)];
+        }
+#pragma unroll
+        for (int j = 0; j < RG_MFMA_TAPS - 1; ++j) old[j] = load(st + (size_t)min(j, taps - 1) * width);
+        if (bias) {
+#pragma unroll
+            for (int k = 0; k < V; ++k) here[k] += bias[x_off + c + k];
+        }
+        if (conv_b) acc = load(conv_b + c);
+#pragma unroll
+        for (int j = 0; j < RG_MFMA_TAPS; ++j) {
+            const int back = taps - 1 - j;
+            if (j < taps) {
+                const fv v = back == 0 ? here : before >= back ? old[j < RG_MFMA_TAPS - 1 ? j : 0] : zero;
+#pragma unroll
+                for (int k = 0; k < V; ++k) acc[k] = fmaf(cw[4 * k + j], v[k], acc[k]);
+                if (j > 0) *(fv *)(st + (size_t)(j - 1) * width) = v;     // a row up; the oldest goes
+            }
+        }
+        *(fv *)(us_tile + tt * ld + i) = acc;
+    }
+    // what a thread needs in the end for its first element
+    float e_lam = 0.f, e_ba = 0.f, e_bi = 0.f, e_y = 0.f, e_s = 0.f;
+    auto fetch_end = [&](int x) {
+        const int t = tok0 + x / bs, c = b * bs + x % bs;
+        e_lam = lam[c];
+        e_ba = ba[c];
+        e_bi = bi[c];
+        e_y = to_f32(rows[(size_t)t * row_stride + y_off + c]) + (bias ? bias[y_off + c] : 0.f);
+        e_s = ctx_len[t] > 1 ? state[((size_t)state_slot[t] * taps + taps - 1) * width + c] : 0.f;
+    };
+    if ((int)threadIdx.x < nt * bs) fetch_end(threadIdx.x);
+    __syncthreads();
+    // ---- the gates (the instruction's other rows are the last token's again)
+    for (int item = wave; item < items; item += RG_ONE_THREADS / WAVE) {
+        const int tile = item % tiles, part = item / tiles, j0 = part * tiles / parts, j1 = (part + 1) * tiles / parts;      // (in sixteens)
+        rg_f32x4 acc[2] = {rg_f32x4{0.f, 0.f, 0.f, 0.f}, rg_f32x4{0.f, 0.f, 0.f, 0.f}};
+        const float *up = us_tile + min(l16, nt - 1) * ld + 4 * g;
+        for (int jb = j0; jb < j1; jb += 4) {
+            if (jb > j0 || item != wave) rg_fetch(w, gates, b, tile, tiles, lane, 16 * jb);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (jb + j >= j1) break;
+                const rg_f32x4 x = *(const rg_f32x4 *)(up + 16 * (jb + j));
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[q][j][e], acc[q], 0, 0, 0);
+            }
+        }
+        if (g < RG_ONE_TOK / 4) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sums[((part * 2 + q) * RG_ONE_TOK + 4 * g + r) * ld + 16 * tile + l16] = acc[q][r];
+        }
+    }
+    __syncthreads();
+    for (int x = threadIdx.x; x < nt * bs; x += RG_ONE_THREADS) {
+        const int tt = x / bs, o = x % bs, t = tok0 + tt, c = b * bs + o;
+        if (x != (int)threadIdx.x) fetch_end(x);                          // (blocks of more than 128 channels)
+        float sa = 0.f, si = 0.f;
+        for (int k = 0; k < parts; ++k) {
+            sa += sums[(2 * k * RG_ONE_TOK + tt) * ld + o];
+            si += sums[((2 * k + 1) * RG_ONE_TOK + tt) * ld + o];
+        }
+        const float gr = 1.0f / (1.0f + expf(-(sa + e_ba)));
+        const float gate = 1.0f / (1.0f + expf(-(si + e_bi)));
+        const float log_a = -c_exp * gr * (e_lam > 20.f ? e_lam : log1pf(expf(e_lam)));
+        const float mult = sqrtf(-expm1f(2.0f * log_a));
+        const float S = fmaf(expf(log_a), e_s, mult * gate * us_tile[tt * ld + o]);
+        state[((size_t)state_slot[t] * taps + taps - 1) * width + c] = S;
+        out[(size_t)t * width + c] = from_f32<T>(S * gelu_tanh(e_y));
+    }
+}
+
 // The recurrence over [s0, s1) from S, in the tokens' order; with WRITE the outputs too.  RG_BATCH tokens at a time: their
 // loads go out together.  prod (if not null) receives the product of the decays.
 template <class T, bool WRITE>
@@ -366,19 +645,53 @@ rglru_scan_kernel(const TI *__restrict__ rows, int row_stride, int y_off, int x_
 
 // rows: [n, row_stride] of in_type, yin at y_off and xin at x_off (width each); bias: null or float32 over the row's
 // columns.  conv_w [width, taps], conv_b [width] (may be null), wa_t / wi_t [blocks, bs, bs] transposed ([in][out]),
-// ba / bi / lam [width], all float32.  state: float32 [slots, taps, width].  a, gx, y: float32 scratch of n * (width rounded up to 64) floats each.
+// ba / bi / lam [width], all float32; gates (may be null): both matrices in the order in which the matrix instruction takes them, [blocks][bs / 16 output
+// tiles][bs / 16 input tiles][2][64 lanes (l, g)][4]: output 16 tile + l, input 16 tile + 4 g + e, for bs a multiple of 16 up to 192 (then wa_t and wi_t are
+// not read).  single: every request feeds one token.  state: float32 [slots, taps, width].  a, gx, y: float32 scratch of n * (width rounded up to 64) floats each.
 // out: [n, width] of out_type.
 LCU_API int lcu_rglru(const void *rows, int in_type, int row_stride, int y_off, int x_off, const float *bias,
-                      const float *conv_w, const float *conv_b, const float *wa_t, const float *wi_t, const float *ba,
+                      const float *conv_w, const float *conv_b, const float *wa_t, const float *wi_t, const float *gates, const float *ba,
                       const float *bi, const float *lam, float c_exp, float *state, float *a, float *gx, float *y, void *out,
                       int out_type, const int *q_start, const int *ctx_len, const int *req_of_token, const int *state_slot,
-                      int n, int n_req, int width, int blocks, int taps, hipStream_t stream) {
+                      int n, int n_req, int width, int blocks, int taps, int single, hipStream_t stream) {
     if (n <= 0 || n_req <= 0) return LCU_OK;
     if (width <= 0 || blocks <= 0 || width % blocks || width / blocks > RG_MAX_BS || taps < 1 || taps > 16 || n_req > 65535 ||
         !rows || !conv_w || !wa_t || !wi_t || !ba || !bi || !lam || !state || !a || !gx || !y || !out)
         return LCU_BAD_ARGUMENT;
     const int bs = width / blocks;
-    if (n > RG_FEW_ROWS) {
+    if ((in_type != LCU_F32 && in_type != LCU_BF16) || (out_type != LCU_F32 && out_type != LCU_BF16) || (in_type == LCU_BF16 && out_type == LCU_F32))
+        return LCU_BAD_ARGUMENT;
+    const bool matrix = gates != nullptr;
+    if (matrix && (bs % 16 || bs > RG_MFMA_BS || (uintptr_t)gates % 16)) return LCU_BAD_ARGUMENT;
+    if (matrix && single && n == n_req && taps <= RG_MFMA_TAPS) {
+        const bool fours = x_off % 4 == 0 && row_stride % 4 == 0 && ((uintptr_t)rows | (uintptr_t)conv_w | (uintptr_t)conv_b | (uintptr_t)state) % 16 == 0;
+        const int parts = rg_one_parts(bs / 16);
+        const dim3 grid((n + RG_ONE_TOK - 1) / RG_ONE_TOK, blocks);
+        const size_t lds = (size_t)(2 * parts + 1) * RG_ONE_TOK * (bs + 4) * sizeof(float);
+#define ONE(TI, T, V)                                                                                                                      \
+    rglru_single_kernel<TI, T, V><<<grid, dim3(RG_ONE_THREADS), lds, stream>>>((const TI *)rows, row_stride, y_off, x_off, bias, conv_w, conv_b, state, gates, ba, \
+                                                                              bi, lam, c_exp, (T *)out, ctx_len, state_slot, n, width, bs, taps)
+#define STEP(TI, T) do { if (fours) ONE(TI, T, 4); else ONE(TI, T, 1); } while (0)
+        if (in_type == LCU_BF16) STEP(bf16_t, bf16_t);
+        else if (out_type == LCU_BF16) STEP(float, bf16_t);
+        else STEP(float, float);
+#undef STEP
+#undef ONE
+        LCU_LAUNCH_CHECK();
+        return LCU_OK;
+    }
+    if (matrix && n > RG_FEW_ROWS) {
+        // 64 tokens a workgroup where those are RG_MFMA_WIDE at least (the matrices are read for each), else 16
+        const bool wide = (long long)((n + 63) / 64) * blocks >= RG_MFMA_WIDE;
+#define GATES(TI, TT)                                                                                                                          \
+    rglru_gates_mfma_kernel<TI, TT><<<dim3((n + 16 * TT - 1) / (16 * TT), blocks), dim3(RG_MFMA_THREADS), 16 * TT * ((bs + 63) / 64 * 64 + 4) * sizeof(float), stream>>>( \
+        (const TI *)rows, row_stride, x_off, bias, conv_w, conv_b, state, gates, ba, bi, lam, c_exp, a, gx, y, y_off, q_start, ctx_len, req_of_token,      \
+        state_slot, n, width, bs, taps)
+        if (in_type == LCU_F32) { if (wide) GATES(float, 4); else GATES(float, 1); }
+        else { if (wide) GATES(bf16_t, 4); else GATES(bf16_t, 1); }
+#undef GATES
+        LCU_LAUNCH_CHECK();
+    } else if (n > RG_FEW_ROWS) {
         const int bs4 = (bs + 3) / 4 * 4;
         dim3 grid((n + RG_ROWS - 1) / RG_ROWS, blocks), block(bs >= 256 ? 256 : (bs + 63) / 64 * 64);
         const size_t lds = (size_t)RG_ROWS * bs4 * sizeof(float);

@@ -2209,17 +2209,33 @@ def retention(rows: torch.Tensor, offsets: Dict[str, int], decay: torch.Tensor, 
 # ------------------------------------------------------------------ the gated linear recurrent unit
 
 
+RGLRU_GATES_MAX = 192
+
+
+def pack_rglru_gates(wa_t: torch.Tensor, wi_t: torch.Tensor) -> Optional[torch.Tensor]:
+    """The two gates' matrices ``[blocks, in, out]`` float32 in the order in which the matrix instruction takes them, ``[blocks, out / 16, in / 16, 2,
+    64, 4]``; None where ``rglru`` has no such kernel (blocks that are no multiple of 16, or of more than 192 channels)."""
+    blocks, bs, _ = wa_t.shape
+    if bs % 16 or bs > RGLRU_GATES_MAX:
+        return None
+    t = bs // 16
+    # input 16 i + 4 g + e, output 16 o + l: [blocks, i, g, e, o, l] -> [blocks, o, i, g, l, e]
+    both = [m.reshape(blocks, t, 4, 4, t, 16).permute(0, 4, 1, 2, 5, 3) for m in (wa_t, wi_t)]
+    return torch.stack(both, dim=3).reshape(blocks, t, t, 2, 64, 4).contiguous()
+
+
 def rglru(rows: torch.Tensor, y_off: int, x_off: int, bias: Optional[torch.Tensor], conv_w: torch.Tensor,
           conv_b: Optional[torch.Tensor], wa_t: torch.Tensor, wi_t: torch.Tensor, ba: torch.Tensor, bi: torch.Tensor,
-          lam: torch.Tensor, c_exp: float, state: torch.Tensor, step, out_dtype: torch.dtype) -> torch.Tensor:
+          lam: torch.Tensor, c_exp: float, state: torch.Tensor, step, out_dtype: torch.dtype, gates: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The recurrent block between its input product and its output product.  ``rows [n, *]`` holds the two branches
     (``width`` columns each at ``y_off`` and ``x_off``; ``bias`` float32 over the rows' columns is added).  ``u`` = causal
     convolution of the x branch (``conv_w [width, taps]``, the last column the current token's; ``conv_b``); gates ``r =
     sigmoid(Wa u + ba)``, ``i = sigmoid(Wi u + bi)`` with block-diagonal matrices given transposed (``wa_t``, ``wi_t``
     ``[blocks, in, out]``); ``a = exp(-c_exp r softplus(lam))``; ``S <- a S + sqrt(1 - a^2) i u``; returns ``S *
     gelu_tanh(y branch)`` as ``[n, width]`` in ``out_dtype``.  ``state [slots, taps, width]`` float32: the last ``taps -
-    1`` rows of the x branch, then ``S``; taken as zero at a request's position 0."""
-    _gpu(rows, bias, conv_w, conv_b, wa_t, wi_t, ba, bi, lam, state)
+    1`` rows of the x branch, then ``S``; taken as zero at a request's position 0.  ``gates``: the result of ``pack_rglru_gates`` for the
+    two matrices: their products are then made on the matrix instruction."""
+    _gpu(rows, bias, conv_w, conv_b, wa_t, wi_t, ba, bi, lam, state, gates)
     _rows(rows, "rglru rows")
     n, cols = rows.shape
     if conv_w.dim() != 2 or conv_w.dtype != torch.float32 or not conv_w.is_contiguous():
@@ -2240,14 +2256,18 @@ def rglru(rows: torch.Tensor, y_off: int, x_off: int, bias: Optional[torch.Tenso
         raise KernelError(f"rglru: state must be contiguous float32 [slots, {taps}, {width}]")
     if n != step.n or max(step.state_slots, default=0) >= state.shape[0]:
         raise KernelError("rglru: the rows are not the step's, or a request's slot lies outside the state")
+    if gates is not None:
+        t = wa_t.shape[1] // 16
+        if gates.dtype != torch.float32 or gates.shape != (blocks, t, t, 2, 64, 4) or wa_t.shape[1] % 16 or not gates.is_contiguous():
+            raise KernelError(f"rglru: gates {gates.dtype} {tuple(gates.shape)} are not what pack_rglru_gates makes of {tuple(wa_t.shape)}")
     scratch = torch.empty((3, n, (width + 63) // 64 * 64), dtype=torch.float32, device=rows.device)
     out = torch.empty((n, width), dtype=out_dtype, device=rows.device)
     lib = build.load("rglru")
     _check(lib.lcu_rglru(_ptr(rows), _type(rows, "rglru rows"), rows.stride(0), int(y_off), int(x_off), _ptr(bias), _ptr(conv_w),
-                         _ptr(conv_b), _ptr(wa_t), _ptr(wi_t), _ptr(ba), _ptr(bi), _ptr(lam), ctypes.c_float(c_exp), _ptr(state),
+                         _ptr(conv_b), _ptr(wa_t), _ptr(wi_t), _ptr(gates), _ptr(ba), _ptr(bi), _ptr(lam), ctypes.c_float(c_exp), _ptr(state),
                          _ptr(scratch[0]), _ptr(scratch[1]), _ptr(scratch[2]), _ptr(out), _type(out, "rglru out"), _ptr(step.q_start),
                          _ptr(step.ctx_len), _ptr(step.req_of_token), _ptr(step.state_slot), n, step.n_req, width, blocks, taps,
-                         _stream()), "rglru")
+                         int(step.decode_only and n == step.n_req), _stream()), "rglru")
     return out
 
 

@@ -66,6 +66,7 @@ class RGLRU(Part):
         self.conv_w, self.conv_b = f32("conv"), f32("conv_bias")
         self.wa_t = f32("a_gate").transpose(1, 2).contiguous()
         self.wi_t = f32("i_gate").transpose(1, 2).contiguous()
+        self.gates = ops.pack_rglru_gates(self.wa_t, self.wi_t)
         self.ba, self.bi = f32("a_gate_bias").reshape(w).contiguous(), f32("i_gate_bias").reshape(w).contiguous()
         self.lam = f32("lam")
         self.dtype = build.dtype
@@ -76,7 +77,7 @@ class RGLRU(Part):
             raise ops.KernelError("rglru: the layer was given no state slots")
         rows = linear(h, self.w_in, out_dtype=torch.float32)
         y = ops.rglru(rows, 0, self.width, self.bias, self.conv_w, self.conv_b, self.wa_t, self.wi_t, self.ba, self.bi,
-                      self.lam, self.c, state, step, self.dtype)
+                      self.lam, self.c, state, step, self.dtype, gates=self.gates)
         return linear(y, self.w_o, out_dtype=out_dtype or self.dtype)
 
 
