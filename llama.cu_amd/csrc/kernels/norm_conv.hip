@@ -11,6 +11,7 @@
 // last T - 1 rows of earlier steps) and rows before position 0 are zeros.
 #include "common.h"
 #include "rows.h"
+#include "conv_rows.h"
 #include "pair_sum.h"
 
 constexpr int NC_THREADS = 256;
@@ -241,10 +242,39 @@ short_conv_kernel(const TI *__restrict__ h, size_t set_stride_h, const TW *__res
             float v;
             if (t - back >= first) v = to_f32(hs[(size_t)(t - back) * d + c]);
             else v = state[(size_t)(taps - 1 - (first - (t - back))) * d + c];
-            acc += to_f32(w[(size_t)c * taps + j]) * v;
+            acc = fmaf(to_f32(w[(size_t)c * taps + j]), v, acc);
         }
         out[s * set_stride_out + (size_t)t * d + c] = from_f32<TO>(acc);
     }
+}
+
+// Many tokens (conv_rows.h): the same sums in the same order.
+template <class TI, class TW, class TO, int TAPS>
+__global__ void __launch_bounds__(CONV_RUN_THREADS)
+short_conv_rows_kernel(const TI *__restrict__ h, size_t set_stride_h, const TW *__restrict__ cw, const float *__restrict__ st, TO *__restrict__ out, size_t set_stride_out, const int *__restrict__ q_start,
+                       const int *__restrict__ ctx_len, const int *__restrict__ req_of_token,
+                       const int *__restrict__ state_slot, int n, int d) {
+    const int t0 = blockIdx.x * CONV_RUN, count = min(CONV_RUN, n - t0), s = blockIdx.y, c = (blockIdx.z * CONV_RUN_THREADS + threadIdx.x) * 4;
+    if (c >= d) return;
+    const TI *hs = h + s * set_stride_h;
+    const TW *w = cw + (size_t)s * d * TAPS;
+    TO *o = out + s * set_stride_out + (size_t)t0 * d + c;
+    float k[4 * TAPS];
+#pragma unroll
+    for (int q = 0; q < TAPS; ++q) load_as_f32<TW, 4>(w + (size_t)c * TAPS + 4 * q, k + 4 * q);
+    conv_run<TAPS>(hs + c, d, t0, count, req_of_token, q_start, ctx_len, state_slot, d,
+                   [&](int slot) { return st + ((size_t)slot * gridDim.y + s) * (TAPS - 1) * d + c; },
+                   [&](int i, float (*row)[4], int pos, bool) {
+        float acc[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = row[TAPS - 1][e];
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j)
+            if (pos >= TAPS - 1 - j)                             // (else there is no such row)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = fmaf(k[e * TAPS + j], row[j][e], acc[e]);
+        store_f32<TO, 4>(o + (size_t)i * d, acc);
+    });
 }
 
 // After the convolution has run: every request's state becomes the last taps - 1 rows up to
@@ -290,7 +320,17 @@ LCU_API int lcu_short_conv(const void *h, int h_type, long long set_stride_h, co
     if (d <= 0 || taps < 1 || taps > MAX_TAPS || sets < 1 || sets > 8 || h_type != LCU_F32 && h_type != LCU_BF16) return LCU_BAD_ARGUMENT;
     if (w_type != h_type && !(w_type == LCU_F32) && !(h_type == LCU_F32 && w_type == LCU_BF16)) return LCU_BAD_ARGUMENT;
     dim3 grid(n, sets), block(NC_THREADS);
-#define GO(TI, TW, TO) short_conv_kernel<TI, TW, TO><<<grid, block, 0, stream>>>((const TI *)h, (size_t)set_stride_h, (const TW *)cw, state, (TO *)out, (size_t)set_stride_out, q_start, ctx_len, req_of_token, state_slot, d, taps)
+    const bool rows = n >= CONV_RUN_TOKENS && n / CONV_RUN_A_REQUEST >= n_req && d % 4 == 0 && taps > 1 && taps <= CONV_RUN_TAPS && set_stride_h % 4 == 0 && set_stride_out % 4 == 0 && four_ok(h, h_type) &&
+                      four_ok(cw, w_type) && four_ok(state, LCU_F32) && four_ok(out, out_type);
+    const dim3 rgrid((n + CONV_RUN - 1) / CONV_RUN, sets, (d / 4 + CONV_RUN_THREADS - 1) / CONV_RUN_THREADS);
+#define ROWS(TI, TW, TO, TAPS) short_conv_rows_kernel<TI, TW, TO, TAPS><<<rgrid, dim3(CONV_RUN_THREADS), 0, stream>>>((const TI *)h, (size_t)set_stride_h, (const TW *)cw, state, (TO *)out, (size_t)set_stride_out, q_start, ctx_len, req_of_token, state_slot, n, d)
+#define GO(TI, TW, TO)                                                                                                                                          \
+    do {                                                                                                                                                        \
+        if (rows && taps == 4) ROWS(TI, TW, TO, 4);                                                                                                             \
+        else if (rows && taps == 3) ROWS(TI, TW, TO, 3);                                                                                                        \
+        else if (rows) ROWS(TI, TW, TO, 2);                                                                                                                     \
+        else short_conv_kernel<TI, TW, TO><<<grid, block, 0, stream>>>((const TI *)h, (size_t)set_stride_h, (const TW *)cw, state, (TO *)out, (size_t)set_stride_out, q_start, ctx_len, req_of_token, state_slot, d, taps); \
+    } while (0)
     if (h_type == LCU_F32 && w_type == LCU_F32 && out_type == LCU_F32) GO(float, float, float);
     else if (h_type == LCU_F32 && w_type == LCU_F32 && out_type == LCU_BF16) GO(float, float, bf16_t);
     else if (h_type == LCU_F32 && w_type == LCU_BF16 && out_type == LCU_BF16) GO(float, bf16_t, bf16_t);
@@ -299,6 +339,7 @@ LCU_API int lcu_short_conv(const void *h, int h_type, long long set_stride_h, co
     else if (h_type == LCU_BF16 && w_type == LCU_F32 && out_type == LCU_BF16) GO(bf16_t, float, bf16_t);
     else return LCU_BAD_ARGUMENT;
 #undef GO
+#undef ROWS
     LCU_LAUNCH_CHECK();
     if (update && taps > 1) {
         dim3 ugrid(n_req, sets, (d + NC_THREADS - 1) / NC_THREADS);
