@@ -44,79 +44,13 @@ constexpr int ROUTE_CHUNKS = 8;                  // rows of up to 8 * 512 elemen
 // groups (ties: the lower index) can be chosen.  extra: rows of `router` behind the experts' (at most MOE_MAX_EXTRA); gates [n, extra] takes sigmoid
 // of their logits (they are no experts and are never chosen).
 constexpr int MOE_MAX_EXTRA = 8;
-template <class T, int THREADS>
-__global__ void __launch_bounds__(THREADS)
-moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, const float *__restrict__ bias, int *__restrict__ ids,
-                 float *__restrict__ wts, float *__restrict__ gates, int d, int n_experts, int top, int mode, int extra, int groups, int keep,
-                 int renorm, float scale) {
-    __shared__ float z[MOE_MAX_EXPERTS + MOE_MAX_EXTRA];
-    __shared__ float zc[MOE_MAX_EXPERTS];
-    __shared__ float sc[MOE_MAX_EXPERTS];
-    const float *logit_bias = mode == 2 ? nullptr : bias;
-    const int experts = n_experts + extra;          // rows of the router's matrix
-    const int t = blockIdx.x, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    const T *row = h + (size_t)t * d;
-    if (d % 8 == 0 && d <= ROUTE_CHUNKS * 512) {
-        float x[ROUTE_CHUNKS][8];
-#pragma unroll
-        for (int k = 0; k < ROUTE_CHUNKS; ++k) {
-            const int c = k * 512 + lane * 8;
-            if (c < d) {
-                const Row8<T> in = *(const Row8<T> *)(row + c);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[k][e] = to_f32(in.v[e]);
-            }
-        }
-        // two rows of the router at a time, so that 17 rows on 16 waves (16 experts and a gate) are not two trips to memory; but one where a wave has
-        // many long rows, which are trips enough and twice of which leave no room for the next ones' loads (1,024 rows of 4,096, one token: 183 us, two at a
-        // time 222)
-        const bool two = experts <= 64 + MOE_MAX_EXTRA || d <= ROUTE_CHUNKS * 256;
-        for (int e = wave; e < experts; e += (two ? 2 : 1) * (THREADS / WAVE)) {
-            const int e2 = two ? e + THREADS / WAVE : experts;
-            const float *w = router + (size_t)e * d, *v = router + (size_t)(e2 < experts ? e2 : e) * d;
-            float acc = 0.f, acc2 = 0.f;
-            if (e2 < experts) {
-#pragma unroll
-                for (int k = 0; k < ROUTE_CHUNKS; ++k) {
-                    const int c = k * 512 + lane * 8;
-                    if (c < d) {
-                        const f32x4 w0 = *(const f32x4 *)(w + c), w1 = *(const f32x4 *)(w + c + 4), v0 = *(const f32x4 *)(v + c), v1 = *(const f32x4 *)(v + c + 4);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) { acc += x[k][i] * w0[i]; acc2 += x[k][i] * v0[i]; }
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) { acc += x[k][4 + i] * w1[i]; acc2 += x[k][4 + i] * v1[i]; }
-                    }
-                }
-                acc2 = wave_sum_in_place(acc2);
-                if (lane == 0) z[e2] = acc2 + (logit_bias && e2 < n_experts ? logit_bias[e2] : 0.f);
-            } else {
-#pragma unroll
-                for (int k = 0; k < ROUTE_CHUNKS; ++k) {
-                    const int c = k * 512 + lane * 8;
-                    if (c < d) {
-                        const f32x4 w0 = *(const f32x4 *)(w + c), w1 = *(const f32x4 *)(w + c + 4);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) acc += x[k][i] * w0[i];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) acc += x[k][4 + i] * w1[i];
-                    }
-                }
-            }
-            acc = wave_sum_in_place(acc);
-            if (lane == 0) z[e] = acc + (logit_bias && e < n_experts ? logit_bias[e] : 0.f);
-        }
-    } else {
-        for (int e = wave; e < experts; e += THREADS / WAVE) {
-            const float *w = router + (size_t)e * d;
-            float acc = 0.f;
-            for (int c = lane; c < d; c += WAVE) acc += to_f32(row[c]) * w[c];
-            acc = wave_sum_in_place(acc);
-            if (lane == 0) z[e] = acc + (logit_bias && e < n_experts ? logit_bias[e] : 0.f);
-        }
-    }
-    __syncthreads();
-    // the first wave does the rest alone
-    if (wave != 0) return;
+// From so many values on four tokens a workgroup.  One MI355X, us, one and four, 64 experts: 1,000 tokens of 2048 22.2, 18.2 and of 1024 12.9, 12.3, of 512 8.0, 10.9;
+// 512 of 2048 13.6, 17.9
+constexpr int MOE_ROUTE_VALUES = 2000000;
+// The choice and its weights from a token's logits z, by one wave.  zc, sc: LDS, a number an expert each.
+__device__ __forceinline__ void route_choose(float *z, float *zc, float *sc, int t, int lane, const float *__restrict__ bias, int *__restrict__ ids,
+                                             float *__restrict__ wts, float *__restrict__ gates, int n_experts, int top, int mode, int extra, int groups,
+                                             int keep, int renorm, float scale) {
     for (int e = lane; e < extra; e += WAVE) gates[(size_t)t * extra + e] = 1.0f / (1.0f + expf(-z[n_experts + e]));
     const bool one_each = n_experts <= WAVE;         // an expert a lane: the choice stays in registers
     if (mode == 2) {                                 // scores over all experts; z becomes what the choice goes by
@@ -201,6 +135,134 @@ moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, cons
         const float sum = wave_sum_in_place(part);
         for (int k = lane; k < top; k += WAVE) wts[(size_t)t * top + k] = expf(zc[k] - z0) / sum;
     }
+}
+
+template <class T, int THREADS>
+__global__ void __launch_bounds__(THREADS)
+moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, const float *__restrict__ bias, int *__restrict__ ids,
+                 float *__restrict__ wts, float *__restrict__ gates, int d, int n_experts, int top, int mode, int extra, int groups, int keep,
+                 int renorm, float scale) {
+    __shared__ float z[MOE_MAX_EXPERTS + MOE_MAX_EXTRA];
+    __shared__ float zc[MOE_MAX_EXPERTS];
+    __shared__ float sc[MOE_MAX_EXPERTS];
+    const float *logit_bias = mode == 2 ? nullptr : bias;
+    const int experts = n_experts + extra;          // rows of the router's matrix
+    const int t = blockIdx.x, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    const T *row = h + (size_t)t * d;
+    if (d % 8 == 0 && d <= ROUTE_CHUNKS * 512) {
+        float x[ROUTE_CHUNKS][8];
+#pragma unroll
+        for (int k = 0; k < ROUTE_CHUNKS; ++k) {
+            const int c = k * 512 + lane * 8;
+            if (c < d) {
+                const Row8<T> in = *(const Row8<T> *)(row + c);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[k][e] = to_f32(in.v[e]);
+            }
+        }
+        // two rows of the router at a time, so that 17 rows on 16 waves (16 experts and a gate) are not two trips to memory; but one where a wave has
+        // many long rows, which are trips enough and twice of which leave no room for the next ones' loads (1,024 rows of 4,096, one token: 183 us, two at a
+        // time 222)
+        const bool two = experts <= 64 + MOE_MAX_EXTRA || d <= ROUTE_CHUNKS * 256;
+        for (int e = wave; e < experts; e += (two ? 2 : 1) * (THREADS / WAVE)) {
+            const int e2 = two ? e + THREADS / WAVE : experts;
+            const float *w = router + (size_t)e * d, *v = router + (size_t)(e2 < experts ? e2 : e) * d;
+            float acc = 0.f, acc2 = 0.f;
+            if (e2 < experts) {
+#pragma unroll
+                for (int k = 0; k < ROUTE_CHUNKS; ++k) {
+                    const int c = k * 512 + lane * 8;
+                    if (c < d) {
+                        const f32x4 w0 = *(const f32x4 *)(w + c), w1 = *(const f32x4 *)(w + c + 4), v0 = *(const f32x4 *)(v + c), v1 = *(const f32x4 *)(v + c + 4);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) { acc += x[k][i] * w0[i]; acc2 += x[k][i] * v0[i]; }
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) { acc += x[k][4 + i] * w1[i]; acc2 += x[k][4 + i] * v1[i]; }
+                    }
+                }
+                acc2 = wave_sum_in_place(acc2);
+                if (lane == 0) z[e2] = acc2 + (logit_bias && e2 < n_experts ? logit_bias[e2] : 0.f);
+            } else {
+#pragma unroll
+                for (int k = 0; k < ROUTE_CHUNKS; ++k) {
+                    const int c = k * 512 + lane * 8;
+                    if (c < d) {
+                        const f32x4 w0 = *(const f32x4 *)(w + c), w1 = *(const f32x4 *)(w + c + 4);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc += x[k][i] * w0[i];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc += x[k][4 + i] * w1[i];
+                    }
+                }
+            }
+            acc = wave_sum_in_place(acc);
+            if (lane == 0) z[e] = acc + (logit_bias && e < n_experts ? logit_bias[e] : 0.f);
+        }
+    } else {
+        for (int e = wave; e < experts; e += THREADS / WAVE) {
+            const float *w = router + (size_t)e * d;
+            float acc = 0.f;
+            for (int c = lane; c < d; c += WAVE) acc += to_f32(row[c]) * w[c];
+            acc = wave_sum_in_place(acc);
+            if (lane == 0) z[e] = acc + (logit_bias && e < n_experts ? logit_bias[e] : 0.f);
+        }
+    }
+    __syncthreads();
+    // the first wave does the rest alone
+    if (wave != 0) return;
+    route_choose(z, zc, sc, t, lane, bias, ids, wts, gates, n_experts, top, mode, extra, groups, keep, renorm, scale);
+}
+
+// Rows of CHUNKS * 512 elements: no load hangs on a comparison, so a wave asks for its tokens' rows and its first two rows of the router at once, and
+// from then on for the next row while it works on one (the loop above waits for every 512 elements in turn).  TOKENS tokens a workgroup: the router's
+// matrix comes out of the second-level cache once for all of them, which bounds long steps, and a wave each makes their choices.  The same sums in the
+// same order.  One MI355X, d = 2048, 2,000 tokens: 16 experts and a gate 8.9 us (15.5), 256 experts 69 (156); 300 tokens 5.8 (6.7), 41 (69).  Small steps, which
+// share the rows out over the waves of 1,024 threads, gain nothing: 16 tokens and experts 5.1 (4.8).
+template <class T, int THREADS, int CHUNKS, int TOKENS>
+__global__ void __launch_bounds__(THREADS)
+moe_route_rows_kernel(const T *__restrict__ h, const float *__restrict__ router, const float *__restrict__ bias, int *__restrict__ ids,
+                      float *__restrict__ wts, float *__restrict__ gates, int n, int n_experts, int top, int mode, int extra, int groups, int keep,
+                      int renorm, float scale) {
+    extern __shared__ float lds[];
+    constexpr int WAVES = THREADS / WAVE, D = CHUNKS * 512;
+    static_assert(TOKENS <= WAVES, "a wave a token");
+    const float *logit_bias = mode == 2 ? nullptr : bias;
+    const int experts = n_experts + extra, t0 = blockIdx.x * TOKENS, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    float x[TOKENS][CHUNKS][8];
+    f32x4 w[2 * CHUNKS], next[2 * CHUNKS];
+    auto fetch = [&](int e, f32x4 *to) {
+        const float *from = router + (size_t)min(e, experts - 1) * D + lane * 8;
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k) { to[2 * k] = *(const f32x4 *)(from + k * 512); to[2 * k + 1] = *(const f32x4 *)(from + k * 512 + 4); }
+    };
+    fetch(wave, w);
+#pragma unroll
+    for (int b = 0; b < TOKENS; ++b)
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k) {
+            const Row8<T> in = *(const Row8<T> *)(h + (size_t)min(t0 + b, n - 1) * D + k * 512 + lane * 8);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[b][k][i] = to_f32(in.v[i]);
+        }
+    for (int e = wave; e < experts; e += WAVES) {
+        fetch(e + WAVES, next);
+#pragma unroll
+        for (int b = 0; b < TOKENS; ++b) {
+            float acc = 0.f;
+#pragma unroll
+            for (int k = 0; k < CHUNKS; ++k)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc = fmaf(x[b][k][i], w[2 * k + i / 4][i % 4], acc);
+            acc = wave_sum_in_place(acc);
+            if (lane == 0) lds[b * 3 * experts + e] = acc + (logit_bias && e < n_experts ? logit_bias[e] : 0.f);
+        }
+#pragma unroll
+        for (int k = 0; k < 2 * CHUNKS; ++k) w[k] = next[k];
+    }
+    __syncthreads();
+    if (wave >= TOKENS || t0 + wave >= n) return;
+    float *z = lds + wave * 3 * experts;
+    route_choose(z, z + experts, z + 2 * experts, t0 + wave, lane, bias, ids, wts, gates, n_experts, top, mode, extra, groups, keep, renorm, scale);
 }
 
 // ---------------------------------------------------------------- group
@@ -738,11 +800,30 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
         (groups > 1 && (mode != 2 || experts % groups || keep < 1 || keep > groups || top > keep * (experts / groups))))
         return LCU_BAD_ARGUMENT;
     const bool few = n <= 256 && experts > 4;
-#define GO(T, TH) moe_route_kernel<T, TH><<<dim3(n), dim3(TH), 0, stream>>>((const T *)h, router, bias, ids, wts, gates, d, experts, top, mode, extra, groups, keep, renorm, scale)
-    if (type == LCU_F32) { if (few) GO(float, 1024); else GO(float, 256); }
-    else if (type == LCU_BF16) { if (few) GO(bf16_t, 1024); else GO(bf16_t, 256); }
-    else return LCU_BAD_ARGUMENT;
+    if (type != LCU_F32 && type != LCU_BF16) return LCU_BAD_ARGUMENT;
+#define ARGS experts, top, mode, extra, groups, keep, renorm, scale
+#define ROWS(T, TH, CHUNKS, TOKENS)                                                                                                                 \
+    moe_route_rows_kernel<T, TH, CHUNKS, TOKENS><<<dim3((n + TOKENS - 1) / TOKENS), dim3(TH), TOKENS * 3 * (experts + extra) * sizeof(float), stream>>>( \
+        (const T *)h, router, bias, ids, wts, gates, n, ARGS)
+#define CHUNKED(T, CHUNKS)                                  \
+    do {                                                    \
+        if ((long long)n * d < MOE_ROUTE_VALUES) ROWS(T, 256, CHUNKS, 1);  \
+        else ROWS(T, 256, CHUNKS, 4);                       \
+    } while (0)
+#define GO(T)                                                                                                                       \
+    do {                                                                                                                            \
+        if (few) moe_route_kernel<T, 1024><<<dim3(n), dim3(1024), 0, stream>>>((const T *)h, router, bias, ids, wts, gates, d, ARGS); \
+        else if (d == 512) CHUNKED(T, 1);                                                                                           \
+        else if (d == 1024) CHUNKED(T, 2);                                                                                          \
+        else if (d == 2048) CHUNKED(T, 4);                                                                                          \
+        else moe_route_kernel<T, 256><<<dim3(n), dim3(256), 0, stream>>>((const T *)h, router, bias, ids, wts, gates, d, ARGS);      \
+    } while (0)
+    if (type == LCU_F32) GO(float);
+    else GO(bf16_t);
 #undef GO
+#undef CHUNKED
+#undef ROWS
+#undef ARGS
     LCU_LAUNCH_CHECK();
     return LCU_OK;
 }
