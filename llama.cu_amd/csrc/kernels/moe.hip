@@ -362,21 +362,6 @@ enum { MOE_UP = 0, MOE_DOWN = 1, MOE_UP_GATED = 2 };
 //   MOE_UP_GATED: x = h [n, K], not scaled; w[e] holds N = 2 * features rows, in turns 16 rows of the gate matrix and the
 //             16 rows of the up matrix that meet them; out_t = act [total, N / 2] at the pair's row,
 //             silu(gate) * up, or with limit > 0 the limited form with alpha and limit.
-template <class T, int MODE>
-__device__ __forceinline__ void moe_store(const f32x4 &acc, int dst, int col0, int N, T *__restrict__ out_t,
-                                          float *__restrict__ out_f, int out_stride, int add) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int col = col0 + i;
-        if (col >= N) continue;
-        if (MODE == MOE_UP) {
-            out_t[(size_t)dst * out_stride + col] = from_f32<T>(gelu_erf(acc[i]));
-        } else {
-            float *o = out_f + (size_t)dst * out_stride + col;
-            *o = add ? *o + acc[i] : acc[i];
-        }
-    }
-}
 
 // Where a lane's part of the matrix lies: lane (g, l16) of unit (16 rows, KSTEP of k) takes row l16, PER_LANE elements from k = g *
 // PER_LANE on.  PACKED: w[e] is [ceil(N / 16)][ceil(K / KSTEP)][64 lanes][PER_LANE], zeros beyond N and K: a wave's load is one piece
@@ -563,7 +548,7 @@ moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__
 // matrix, so each loads its own straight into registers.  Both are two steps ahead.  MT: tiles of 16 rows that are multiplied.
 // What bounds it are the turns of loads, LDS and barrier of the two blocks that a compute unit holds (half the matrix instructions take as long) and, up
 // to 50 rows an expert, the matrices out of memory.  Tiles of 64 rows whose matrices went through LDS too took, per pass of both products, 16 experts
-// of 2048 x 2048 with 2,014 tokens of two each 241 us, now 176; gated, 2 x 1024: 180 and 139; 200 tokens of two 77 and 51.  (Rows copied into LDS by the
+// of 2048 x 2048 with 2,014 tokens of two each 241 us, now 155; gated, 2 x 1024: 180 and 132; 200 tokens of two 77 and 51.  (Rows copied into LDS by the
 // loads themselves, four buffers, the barrier in the middle of the instructions: the same times; 64 rows and three blocks: 5 to 30 % longer.)
 template <class T, int MODE, bool PACKED, int MT>
 __device__ __forceinline__ void moe_many_tile(T *__restrict__ xs, const T *__restrict__ x, int x_stride, const T *__restrict__ we, int N, int K,
@@ -688,25 +673,54 @@ __device__ __forceinline__ void moe_many_tile(T *__restrict__ xs, const T *__res
     for (int ft = 0; ft < 2; ++ft)
 #pragma unroll
         for (int m = 0; m < MT; ++m) acc[ft][m] = sum[ft][m] + acc[ft][m];
+    // The results go out through LDS, 64 rows at a time: a wave then stores whole lines (from where the products leave them a store was 64 separate words, and the
+    // activation's code stood here 64 times).  Four neighbouring features q of row r lie at q ^ (r % 8).  One MI355X, 4,096 pairs, us: K of 64, all but the loop, up with gelu to
+    // 2,048 features 24.5, now 19.1, down 26.9 and 14.5; both products of 2048 x 2048 185 and 155.
+    constexpr int EP = MT < 4 ? MT : 4, QUADS = MODE == MOE_UP_GATED ? 16 : 32, ROWS = 256 / QUADS;      // quads of features of a row, rows stored at a time
+    float *out_rows = (float *)xs;
+    const int q = tid % QUADS, r_in = tid / QUADS, col = n0 / (32 / QUADS) + 4 * q;
+    int dst[16 * MT / ROWS];
+    if (MODE == MOE_DOWN) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int r = 16 * m + l16;
-        if (r >= rows) continue;
-        const int srow = row0 + r;
-        int dst = srow;
-        if (MODE == MOE_DOWN) {
-            const int flat = sorted_to_flat[srow];
-            dst = add ? flat / top : flat;
+        for (int i = 0; i < 16 * MT / ROWS; ++i) {
+            dst[i] = sorted_to_flat[row0 + min(r_in + ROWS * i, rows - 1)];
+            if (add) dst[i] /= top;
         }
-        if constexpr (MODE == MOE_UP_GATED) {       // the wave's first 16 rows are a gate block, its second the up block that meets it
-            const int col = (n0 + 32 * wave) / 2 + 4 * g;
-            Quad<T> q;
+    }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gate_up_of(acc[0][m][i], acc[1][m][i], alpha, limit));
-            if (col < N / 2) *(Quad<T> *)(out_t + (size_t)dst * out_stride + col) = q;
+    for (int m0 = 0; m0 < MT; m0 += EP) {
+        lds_barrier();                              // what lay there has been read
+#pragma unroll
+        for (int m = m0; m < m0 + EP && m < MT; ++m)
+#pragma unroll
+            for (int ft = 0; ft < 2; ++ft) *(f32x4 *)(out_rows + (16 * (m - m0) + l16) * 128 + 4 * ((8 * wave + 4 * ft + g) ^ (l16 % 8))) = acc[ft][m];
+        lds_barrier();
+        auto at = [&](int r, int quad) { return *(const f32x4 *)(out_rows + r * 128 + 4 * (quad ^ (r % 8))); };
+        const int here = min(rows - 16 * m0, 16 * EP);
+        if constexpr (MODE == MOE_DOWN) {
+#pragma unroll
+            for (int i = 0; i < 16 * (MT - m0 < EP ? MT - m0 : EP) / ROWS; ++i) {
+                const int r = r_in + ROWS * i;
+                if (r >= here || col >= N) continue;
+                pair_f32x4_at *o = (pair_f32x4_at *)(out_f + (size_t)dst[16 * m0 / ROWS + i] * out_stride + col);
+                const f32x4 v = at(r, q);
+                *o = add ? *o + v : v;
+            }
         } else {
+#pragma unroll 1
+            for (int r = r_in; r < here; r += ROWS) {
+                Quad<T> to;
+                if constexpr (MODE == MOE_UP_GATED) {       // a wave's first 16 features are a gate block, its second the up block that meets it
+                    const f32x4 gate = at(r, 8 * (q / 4) + q % 4), up = at(r, 8 * (q / 4) + 4 + q % 4);
 #pragma unroll
-            for (int ft = 0; ft < 2; ++ft) moe_store<T, MODE>(acc[ft][m], dst, n0 + 32 * wave + 16 * ft + 4 * g, N, out_t, out_f, out_stride, add);
+                    for (int i = 0; i < 4; ++i) to.v[i] = from_f32<T>(gate_up_of(gate[i], up[i], alpha, limit));
+                } else {
+                    const f32x4 v = at(r, q);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) to.v[i] = from_f32<T>(gelu_erf(v[i]));
+                }
+                if (col < (MODE == MOE_UP_GATED ? N / 2 : N)) *(Quad<T> *)(out_t + (size_t)(row0 + 16 * m0 + r) * out_stride + col) = to;
+            }
         }
     }
 }
@@ -763,8 +777,8 @@ LCU_API int lcu_moe_combine(float *out, const PairSum *p, int type, int n, int d
 // token chooses evenly, with one and a half times their deviation, and workgroups of the rows of the largest expert of so many.
 // Measured with 2 to 64 experts of 520 x 272 to 4096 x 4096 and 17 to 1,024 rows each on average, evenly and with a few experts taking most, 288 shapes: bfloat16 0.9 % (3.9 % unevenly)
 // more than the best of the four sizes, 17 % at most, 32 bits 2.8 % and 0.2 %, 16 % at most.  Always 96, but 128 for 80 to 120 rows, was 11 % and 10 % more, 32 bits 31 % and 51 %; tiles of
-// 64 10 % and 9 %, 32 bits 15 % and 24 %.  (us a pass of both products, with 32, 64, 96 and 128 rows: 16 experts, gated, of 1024 x 512, 88 rows 34, 31, 37, 41, 212 rows 52, 45, 51, 47; of 2048 x
-// 1024, 88 rows 90, 75, 86, 64, 256 rows 168, 139, 119, 132; 32 bits, 8 of 1024 x 1024, 88 rows: 59, 94, 131, 165.)
+// 64 10 % and 9 %, 32 bits 15 % and 24 %.  (us a pass of both products, with 32, 64, 96 and 128 rows: 16 experts, gated, of 1024 x 512, 88 rows 30, 27, 32, 34, 252 rows 53, 50, 45, 50; of 2048 x
+// 1024, 88 rows 71, 55, 65, 55, 252 rows 135, 111, 100, 109; 32 bits, 8 of 1024 x 1024, 88 rows: 59, 94, 131, 165.  The 60 rows' time: over 40 shapes 20 to 70 were tried, 50 and 60 are best.)
 // The caller sizes its scratch with it: max_tiles = min(total, total / rows + experts), or 0.
 LCU_API int lcu_moe_tile_rows(int type, int total, int experts, int up_rows, int d, int ff) {
     if ((long long)total <= 16ll * experts) return total > (type == LCU_F32 ? MOE_LIST_F32 : MOE_LIST) ? 16 : 0;
