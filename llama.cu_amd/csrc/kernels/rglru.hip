@@ -646,8 +646,8 @@ rglru_scan_kernel(const TI *__restrict__ rows, int row_stride, int y_off, int x_
 // rows: [n, row_stride] of in_type, yin at y_off and xin at x_off (width each); bias: null or float32 over the row's
 // columns.  conv_w [width, taps], conv_b [width] (may be null), wa_t / wi_t [blocks, bs, bs] transposed ([in][out]),
 // ba / bi / lam [width], all float32; gates (may be null): both matrices in the order in which the matrix instruction takes them, [blocks][bs / 16 output
-// tiles][bs / 16 input tiles][2][64 lanes (l, g)][4]: output 16 tile + l, input 16 tile + 4 g + e, for bs a multiple of 16 up to 192 (then wa_t and wi_t are
-// not read).  single: every request feeds one token.  state: float32 [slots, taps, width].  a, gx, y: float32 scratch of n * (width rounded up to 64) floats each.
+// tiles][bs / 16 input tiles][2][64 lanes (l, g)][4]: output 16 tile + l, input 16 tile + 4 g + e, for bs a multiple of 16 up to 192 (read in steps of
+// more than 64 tokens, and of single tokens with bfloat16 outputs).  single: every request feeds one token.  state: float32 [slots, taps, width].  a, gx, y: float32 scratch of n * (width rounded up to 64) floats each.
 // out: [n, width] of out_type.
 LCU_API int lcu_rglru(const void *rows, int in_type, int row_stride, int y_off, int x_off, const float *bias,
                       const float *conv_w, const float *conv_b, const float *wa_t, const float *wi_t, const float *gates, const float *ba,
@@ -663,18 +663,18 @@ LCU_API int lcu_rglru(const void *rows, int in_type, int row_stride, int y_off, 
         return LCU_BAD_ARGUMENT;
     const bool matrix = gates != nullptr;
     if (matrix && (bs % 16 || bs > RG_MFMA_BS || (uintptr_t)gates % 16)) return LCU_BAD_ARGUMENT;
-    if (matrix && single && n == n_req && taps <= RG_MFMA_TAPS) {
+    // (with 32-bit outputs the sliced kernel: there a token's bits do not depend on whether it comes alone or in a portion of up to 64)
+    if (matrix && single && n == n_req && taps <= RG_MFMA_TAPS && out_type == LCU_BF16) {
         const bool fours = x_off % 4 == 0 && row_stride % 4 == 0 && ((uintptr_t)rows | (uintptr_t)conv_w | (uintptr_t)conv_b | (uintptr_t)state) % 16 == 0;
         const int parts = rg_one_parts(bs / 16);
         const dim3 grid((n + RG_ONE_TOK - 1) / RG_ONE_TOK, blocks);
         const size_t lds = (size_t)(2 * parts + 1) * RG_ONE_TOK * (bs + 4) * sizeof(float);
-#define ONE(TI, T, V)                                                                                                                      \
-    rglru_single_kernel<TI, T, V><<<grid, dim3(RG_ONE_THREADS), lds, stream>>>((const TI *)rows, row_stride, y_off, x_off, bias, conv_w, conv_b, state, gates, ba, \
-                                                                              bi, lam, c_exp, (T *)out, ctx_len, state_slot, n, width, bs, taps)
-#define STEP(TI, T) do { if (fours) ONE(TI, T, 4); else ONE(TI, T, 1); } while (0)
-        if (in_type == LCU_BF16) STEP(bf16_t, bf16_t);
-        else if (out_type == LCU_BF16) STEP(float, bf16_t);
-        else STEP(float, float);
+#define ONE(TI, V)                                                                                                                         \
+    rglru_single_kernel<TI, bf16_t, V><<<grid, dim3(RG_ONE_THREADS), lds, stream>>>((const TI *)rows, row_stride, y_off, x_off, bias, conv_w, conv_b, state, gates, ba, \
+                                                                              bi, lam, c_exp, (bf16_t *)out, ctx_len, state_slot, n, width, bs, taps)
+#define STEP(TI) do { if (fours) ONE(TI, 4); else ONE(TI, 1); } while (0)
+        if (in_type == LCU_BF16) STEP(bf16_t);
+        else STEP(float);
 #undef STEP
 #undef ONE
         LCU_LAUNCH_CHECK();

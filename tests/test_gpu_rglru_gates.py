@@ -51,8 +51,10 @@ class Unit:
 @pytest.mark.parametrize("width,blocks,taps", [(64, 4, 4), (96, 2, 1), (256, 2, 3), (384, 2, 4), (128, 1, 2), (2048, 16, 4), (40, 2, 4), (64, 1, 5)])
 @pytest.mark.parametrize("n", [1, 7, 16, 17, 64])
 @pytest.mark.parametrize("offsets", [(3, 5), (0, 8)])
-def test_steps_of_single_tokens(width, blocks, taps, n, offsets):
-    """Requests at their first token, within the convolution's reach of it and far behind it, from slots in no order; the other slots stay."""
+@pytest.mark.parametrize("out_type", [torch.bfloat16, torch.float32])
+def test_steps_of_single_tokens(width, blocks, taps, n, offsets, out_type):
+    """Requests at their first token, within the convolution's reach of it and far behind it, from slots in no order; the other slots stay.  With
+    32-bit outputs the bits are those of the same tokens without the packed gates, alone or in portions."""
     from llama_cu_amd.kernels import ops
     unit = Unit(width, blocks, taps, offsets=offsets)
     args = unit.args()
@@ -61,14 +63,17 @@ def test_steps_of_single_tokens(width, blocks, taps, n, offsets):
     slots = torch.randperm(n + 2, generator=torch.Generator().manual_seed(21))[:n].tolist()
     old = rnd(n + 2, taps, width, seed=22)
     state = old.clone().cuda()
-    got = ops.rglru(rows.cuda(), *args, state, hand_step([1] * n, ctx, slots), torch.float32, gates=unit.gates)
+    got = ops.rglru(rows.cuda(), *args, state, hand_step([1] * n, ctx, slots), out_type, gates=unit.gates)
+    if out_type == torch.float32:
+        plain = old.clone().cuda()
+        assert torch.equal(got, ops.rglru(rows.cuda(), *args, plain, hand_step([1] * n, ctx, slots), out_type)) and torch.equal(state, plain)
     for i in range(n):
         have = old[slots[i]].clone()
         for k in range(taps - 1):                       # rows of tokens before the request's first are zeros, whatever the slot holds
             if taps - 1 - k > ctx[i] - 1:
                 have[k] = 0.0
         want, after = unit.want(rows[i:i + 1], have if ctx[i] > 1 else None)
-        assert_close(got[i:i + 1], want, 2e-5, f"request {i}")
+        assert_close(got[i:i + 1], want, 2e-5 if out_type == torch.float32 else 2.0 ** -8, f"request {i}")
         assert_close(state[slots[i]], after, 2e-5, f"state {i}")
     others = [s for s in range(n + 2) if s not in slots]
     assert torch.equal(state[others].cpu(), old[others])
