@@ -68,8 +68,11 @@ def _rows(t: torch.Tensor, what: str) -> None:
 
 
 def _near(x: torch.Tensor) -> torch.Tensor:
-    """Rows whose places fit the 32 bits in which the products of few rows keep them (rows 2^24 elements apart are copied together)."""
-    return x if x.stride(-2) < 1 << 24 else x.contiguous()
+    """Rows whose places fit the 32 bits in which the products of few rows keep them: rows 2^24 elements apart are copied together, and one row, whose
+    stride says nothing (``contiguous`` leaves it as it is), is seen with its own length."""
+    if x.stride(-2) < 1 << 24:
+        return x
+    return x[..., 0, :].unsqueeze(-2) if x.shape[-2] == 1 else x.contiguous()
 
 
 def _contig(t: torch.Tensor, what: str) -> None:

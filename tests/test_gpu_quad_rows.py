@@ -74,6 +74,40 @@ def test_rows_far_apart():
         assert torch.equal(got.cpu().double(), x @ w.t())
 
 
+@pytest.mark.parametrize("m", [1, 2, 3])
+def test_rows_far_apart_in_every_form(m):
+    """One row among them, whose stride says nothing: 2^24 elements and more are no reason to refuse it."""
+    from llama_cu_amd.kernels import ops
+    x, w = whole((m, 128), 18), whole((192, 128), 19)
+    want = x @ w.t()
+
+    def far(dtype):
+        rows = torch.empty(m, (1 << 24) + 8, dtype=dtype, device="cuda")[:, :128]
+        rows.copy_(x.to(dtype))
+        return rows
+
+    xb, xf, wb, wf = far(BF16), far(torch.float32), w.to(BF16).cuda(), w.float().cuda()
+    packed = ops.pack_weight(wb)
+    same = lambda got: torch.equal(got.double().cpu(), want)
+    assert same(ops.gemm_skinny(xb, wb, out_dtype=torch.float32)) and same(ops.gemm_skinny(xb, packed, out_dtype=torch.float32, packed=True))
+    assert same(ops.gemm_wavek(xb, packed, out_dtype=torch.float32)) and same(ops.gemm_skinny_f32(xf, wf))
+    one = x[:1] @ w[:192].t()                           # two groups of the same row, a view whose groups and rows are all far apart
+    pair = xb[:1].unsqueeze(0).expand(2, 1, 128)
+    for got in (ops.gemm_wavek(pair, packed, out_dtype=torch.float32),
+                ops.gemm_skinny_grouped(pair, packed, torch.empty(1, 192, dtype=torch.float32, device="cuda"), packed=True)):
+        assert torch.equal(got.double().cpu(), one)
+    for add_norm, rows, weight in ((ops.gemm_skinny_add_norm, xb, wb), (ops.gemm_skinny_f32_add_norm, xf, wf)):
+        residual = torch.zeros(m, 192, device="cuda")
+        add_norm(rows, weight, residual, torch.ones(192, device="cuda"))
+        assert same(residual)
+    pos = torch.zeros(m, dtype=torch.int32, device="cuda")
+    tables = torch.ones(8, 16, device="cuda"), torch.zeros(8, 16, device="cuda")
+    cache = torch.zeros(1, 2, 32 * 16, dtype=BF16, device="cuda")
+    for got in (ops.gemm_wavek_qkv_rope(xb, packed, pos, pos - 1, *tables, cache, 4, 1, 32, 16),
+                ops.gemm_skinny_qkv_rope(xb, packed, pos, pos - 1, *tables, cache, 4, 1, 32, 16, packed=True)):
+        assert torch.equal(got.double().cpu(), want[:, :128].to(BF16).double())
+
+
 @pytest.mark.parametrize("m", [33, 64])
 def test_which_kernel_makes_q_k_v(m, monkeypatch):
     from llama_cu_amd.kernels import ops
