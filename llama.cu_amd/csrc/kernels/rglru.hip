@@ -277,18 +277,23 @@ rglru_gates_rows_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
     }
 }
 
-// Blocks of a multiple of sixteen channels, up to RG_MFMA_BS: the gates' products on the 32-bit matrix instruction (true 32-bit products and
-// sums).  Lane (l, g) of 16 x 4 brings, of the sixteen k that four instructions take, those from 4 g on; the matrices stand in that order
-// (lcu_rglru), so that a wave's load is 1 KB in one piece.
+// Blocks of a multiple of sixteen channels, up to RG_MFMA_BS: the gates' products on the 32-bit matrix instruction.  It adds its four products one
+// after the other, each multiplication and addition rounded once, as a chain of fmaf does (131,072 sums of each of several ranges compared, bit for
+// bit); so its instructions take the input channels in their order, and the sums have the bits of the kernels above.  Lane (l, g) of 16 x 4 brings,
+// of the sixteen k that four instructions take, those with k % 4 = g: the matrices stand in that order (lcu_rglru), so that a wave's load is 1 KB in
+// one piece, and u lies in LDS so that a lane's four are side by side (rg_place).
 //
 // Many tokens: a workgroup takes 16 TT tokens and a block of channels, makes u for them (in LDS), and each of its waves takes 16 output
-// channels of both gates at a time.  One MI355X, width 2048 in 16 blocks, 4 taps, with the scan behind it: 8 requests of 235 tokens 68 us (a thread
-// an output channel and the sums on the vector unit: 105), 65 tokens 18 (47).  The matrix instructions are 14 us of the first, the functions (exp, expm1,
+// channels of both gates at a time.  One MI355X, width 2048 in 16 blocks, 4 taps, with the scan behind it: 8 requests of 235 tokens 71 us (a thread
+// an output channel and the sums on the vector unit: 108), 65 tokens 19 (47).  The matrix instructions are 14 us of the first, the functions (exp, expm1,
 // tanh) 15, the scan 30.
 constexpr int RG_MFMA_BS = 192, RG_MFMA_TAPS = 4, RG_MFMA_WIDE = 256, RG_MFMA_THREADS = 256;
 typedef __attribute__((ext_vector_type(4))) float rg_f32x4;
 
-// the matrices' four pieces from input channel k0 on for 16 output channels (beyond the end: times zeros of u)
+// where input channel i of a block stands in LDS
+__device__ __forceinline__ int rg_place(int i) { return (i & ~15) + 4 * (i & 3) + ((i >> 2) & 3); }
+
+// the matrices' four pieces from input channel k0 on for 16 output channels (beyond the end: pieces that are not used)
 __device__ __forceinline__ void rg_fetch(rg_f32x4 (&w)[2][4], const float *__restrict__ gates, int block, int tile, int tiles, int lane, int k0) {
     const float *at = gates + (size_t)(block * tiles + tile) * tiles * 512 + 4 * lane;
 #pragma unroll
@@ -307,15 +312,15 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
                         const int *__restrict__ q_start, const int *__restrict__ ctx_len, const int *__restrict__ req_of_token,
                         const int *__restrict__ state_slot, int n, int width, int bs, int taps) {
     constexpr int TOK = 16 * TT, STEP = 64;                               // tokens; input channels whose columns are asked for together
-    extern __shared__ __attribute__((aligned(16))) float us_tile[];       // [TOK][ld], zeros from bs on
-    const int ld = (bs + STEP - 1) / STEP * STEP + 4;
+    extern __shared__ __attribute__((aligned(16))) float us_tile[];       // [TOK][ld]
+    const int ld = bs + 4;
     const int b = blockIdx.y, tok0 = blockIdx.x * TOK, nt = min(TOK, n - tok0);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
     const int tiles = bs / 16, waves = RG_MFMA_THREADS / WAVE;
     rg_f32x4 w[2][4];
     rg_fetch(w, gates, b, min(wave, tiles - 1), tiles, lane, 0);
     // ---- u
-    if (taps <= RG_MFMA_TAPS) {
+    if (TT > 1 || taps <= RG_MFMA_TAPS) {
         // a thread walks a run of the tokens for one channel, with the tokens before it at hand, sixteen at a time
         __shared__ int first_row[TOK], ahead[TOK], slot_of[TOK];          // of a token's request: its first row, the tokens before that, its slot
         if (threadIdx.x < TOK) {
@@ -367,7 +372,7 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
 #pragma unroll
                     for (int j = 0; j < RG_MFMA_TAPS; ++j)
                         if (j < taps) acc = fmaf(cw[j], use[j], acc);
-                    us_tile[tt * ld + i] = tt < nt ? acc : 0.f;
+                    us_tile[tt * ld + rg_place(i)] = tt < nt ? acc : 0.f;
                 }
             }
         }
@@ -380,10 +385,9 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
                 const int first_pos = ctx_len[r] - (q_start[r + 1] - t0);
                 acc = conv_at(rows, row_stride, x_off, bias, conv_w, conv_b, state + (size_t)state_slot[r] * taps * width, t, t0, first_pos, b * bs + i, width, taps);
             }
-            us_tile[tt * ld + i] = acc;
+            us_tile[tt * ld + rg_place(i)] = acc;
         }
     }
-    for (int x = threadIdx.x; x < TOK * (ld - 4 - bs); x += RG_MFMA_THREADS) us_tile[x / (ld - 4 - bs) * ld + bs + x % (ld - 4 - bs)] = 0.f;
     __syncthreads();
     // ---- the gates, 16 output channels at a time
     for (int tile = wave; tile < tiles; tile += waves) {
@@ -397,7 +401,8 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
         if (tile != wave) rg_fetch(w, gates, b, tile, tiles, lane, 0);
         for (int k = 0; k < bs; k += STEP) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < 4; ++j) {
+                if (k + 16 * j >= bs) break;
 #pragma unroll
                 for (int m = 0; m < TT; ++m) {
                     const rg_f32x4 x = *(const rg_f32x4 *)(us_tile + (16 * m + l16) * ld + k + 16 * j + 4 * g);
@@ -406,6 +411,7 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
 #pragma unroll
                         for (int q = 0; q < 2; ++q) acc[q][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[q][j][e], acc[q][m], 0, 0, 0);
                 }
+            }
             if (k + STEP < bs) rg_fetch(w, gates, b, tile, tiles, lane, k + STEP);
         }
         asm volatile("" : "+v"(lane_tok));
@@ -426,7 +432,7 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
                 const float log_a = -c_exp * gr * sp;
                 const float mult = sqrtf(-expm1f(2.0f * log_a));
                 a_out[tile_index(t, c, n)] = expf(log_a);
-                gx_out[tile_index(t, c, n)] = mult * gate * us_tile[tt * ld + o];
+                gx_out[tile_index(t, c, n)] = mult * gate * us_tile[tt * ld + rg_place(o)];
                 y_out[tile_index(t, c, n)] = gelu_tanh(y_in[m][r] + by);
             }
     }
@@ -434,51 +440,55 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
 
 // A step in which every request feeds one token (token i is request i's): the gates as above, the recurrence's step and the state's update in one
 // kernel.  A workgroup takes four tokens and a block of channels; whatever of a slot's state belongs to a channel is read and written by
-// its threads alone.  Eight waves share out the output channels and, where there are waves enough, the input channels (their sums are
-// added through LDS in a fixed order); then a thread an element for the functions, which with the lanes that hold the sums were four one after
-// the other, most of them of tokens that are not there.  Latency bounds it: four trips to memory, 1.7 us of matrix instructions.  One MI355X, 4 taps, us
-// beside the sliced kernel and the scan: width 2048 in 16 blocks 7.6 / 10.4 with 8 requests, 8.1 / 13.5 with 64; width 1024 in 16 blocks 5.6 / 7.9 with 8.
-constexpr int RG_ONE_TOK = 4, RG_ONE_THREADS = 512;
-__host__ __device__ inline int rg_one_parts(int tiles) { return max(1, min(RG_ONE_THREADS / WAVE / tiles, tiles)); }
+// its threads alone.  Eight waves share out the output channels, 16 at a time, the first of which a wave asks for in front of everything; then a thread an
+// element for the functions, which with the lanes that hold the sums were four one after the other, most of them of tokens that are not there.  The sums are
+// those of `slices` equal parts of the input channels, added in their order: RG_SLICES up to RG_FEW_ROWS tokens, one beyond, as the kernels above have them, so
+// that a token's bits do not depend on what else a step of so many tokens holds.  32-bit rows whose fours are aligned (the layer's), up to four taps, slices of whole matrix
+// instructions.  Latency bounds it: four trips to memory, 1.7 us of matrix instructions.  One MI355X, 4 taps, us beside the sliced kernel and the scan: width 2048
+// in 16 blocks 8.0 / 10.9 with 8 requests, 8.8 / 14.0 with 64; width 1024 in 16 blocks 5.8 / 8.5 with 8.  (Blocks of 192 channels, whose twelve sixteens do not fit the
+// registers: 24 / 10.4.)
+constexpr int RG_ONE_TOK = 4, RG_ONE_THREADS = 512, RG_ONE_BS = 128;
 
-template <class TI, class T, int V>
+// MOST: sixteens of input channels at most
+template <class T, int MOST>
 __global__ void __launch_bounds__(RG_ONE_THREADS)
-rglru_single_kernel(const TI *__restrict__ rows, int row_stride, int y_off, int x_off, const float *__restrict__ bias,
+rglru_single_kernel(const float *__restrict__ rows, int row_stride, int y_off, int x_off, const float *__restrict__ bias,
                     const float *__restrict__ conv_w, const float *__restrict__ conv_b, float *__restrict__ state,
                     const float *__restrict__ gates, const float *__restrict__ ba, const float *__restrict__ bi, const float *__restrict__ lam, float c_exp,
-                    T *__restrict__ out, const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int n, int width, int bs, int taps) {
-    extern __shared__ __attribute__((aligned(16))) float us_tile[];       // [4][ld], then the sums [parts][2][4][ld]
+                    T *__restrict__ out, const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int n, int width, int bs, int taps, int slices) {
+    __shared__ __attribute__((aligned(16))) float us_tile[RG_ONE_TOK * (16 * MOST + 4)], sums[2][RG_ONE_TOK][16 * MOST];
     const int ld = bs + 4, b = blockIdx.y, tok0 = blockIdx.x * RG_ONE_TOK, nt = min(RG_ONE_TOK, n - tok0);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
-    const int tiles = bs / 16, parts = rg_one_parts(tiles), items = tiles * parts;      // 16 output channels and a part of the input channels
-    float *sums = us_tile + RG_ONE_TOK * ld;
-    rg_f32x4 w[2][4];
-    if (wave < items) rg_fetch(w, gates, b, wave % tiles, tiles, lane, wave / tiles * tiles / parts * 16);
-    // ---- u, V neighbouring channels of a token a thread
-    typedef float fv __attribute__((ext_vector_type(V)));
-    auto load = [](const float *q) { return *(const fv *)q; };
-    for (int x = threadIdx.x; x < nt * (bs / V); x += RG_ONE_THREADS) {
-        const int tt = x / (bs / V), i = x % (bs / V) * V, c = b * bs + i, t = tok0 + tt;
+    const int tiles = bs / 16, each = bs / 4 / slices;                    // matrix instructions a slice
+    rg_f32x4 w[2][MOST];
+    auto fetch = [&](int tile) {
+        const float *at = gates + (size_t)(b * tiles + tile) * tiles * 512 + 4 * lane;
+#pragma unroll
+        for (int j = 0; j < MOST; ++j) {
+            if (j >= tiles) break;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) w[q][j] = *(const rg_f32x4 *)(at + 512 * j + 256 * q);
+        }
+    };
+    if (wave < tiles) fetch(wave);
+    // ---- u, four neighbouring channels of a token a thread
+    auto load = [](const float *q) { return *(const rg_f32x4 *)q; };
+    for (int x = threadIdx.x; x < nt * (bs / 4); x += RG_ONE_THREADS) {
+        const int tt = x / (bs / 4), i = x % (bs / 4) * 4, c = b * bs + i, t = tok0 + tt;
         const int before = ctx_len[t] - 1;                                // how many tokens the request has behind it
         float *st = state + (size_t)state_slot[t] * taps * width + c;
-        const TI *xp = rows + (size_t)t * row_stride + x_off + c;
-        fv here, old[RG_MFMA_TAPS - 1], acc = {}, zero = {};
-        if constexpr (V == 1) here[0] = to_f32(xp[0]);
-        else if constexpr (sizeof(TI) == 4) here = load((const float *)xp);
-        else {
-            const uint2 two = *(const uint2 *)xp;
-            here = fv{__uint_as_float(two.x << 16), __uint_as_float(two.x & 0xffff0000u), __uint_as_float(two.y << 16), __uint_as_float(two.y & 0xffff0000u)};
-        }
-        float cw[V * RG_MFMA_TAPS];
-        if (V == 4 && taps == 4) {
+        rg_f32x4 here = load(rows + (size_t)t * row_stride + x_off + c), old[RG_MFMA_TAPS - 1], acc = {}, zero = {};
+        float cw[4 * RG_MFMA_TAPS];
+        if (taps == 4) {
 #pragma unroll
-            for (int k = 0; k < V; ++k) {
-                const float4 four = *(const float4 *)(conv_w + (size_t)c * 4 + 4 * k);
-                cw[4 * k] = four.x; cw[4 * k + 1] = four.y; cw[4 * k + 2] = four.z; cw[4 * k + 3] = four.w;
+            for (int k = 0; k < 4; ++k) {
+                const rg_f32x4 four = load(conv_w + (size_t)c * 4 + 4 * k);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) cw[4 * k + j] = four[j];
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < V; ++k)
+            for (int k = 0; k < 4; ++k)
 #pragma unroll
                 for (int j = 0; j < RG_MFMA_TAPS; ++j) cw[4 * k + j] = conv_w[(size_t)(c + k) * taps + min(j, taps - 1)];
         }
@@ -486,20 +496,21 @@ rglru_single_kernel(const TI *__restrict__ rows, int row_stride, int y_off, int 
         for (int j = 0; j < RG_MFMA_TAPS - 1; ++j) old[j] = load(st + (size_t)min(j, taps - 1) * width);
         if (bias) {
 #pragma unroll
-            for (int k = 0; k < V; ++k) here[k] += bias[x_off + c + k];
+            for (int k = 0; k < 4; ++k) here[k] += bias[x_off + c + k];
         }
         if (conv_b) acc = load(conv_b + c);
 #pragma unroll
         for (int j = 0; j < RG_MFMA_TAPS; ++j) {
             const int back = taps - 1 - j;
             if (j < taps) {
-                const fv v = back == 0 ? here : before >= back ? old[j < RG_MFMA_TAPS - 1 ? j : 0] : zero;
+                const rg_f32x4 v = back == 0 ? here : before >= back ? old[j < RG_MFMA_TAPS - 1 ? j : 0] : zero;
 #pragma unroll
-                for (int k = 0; k < V; ++k) acc[k] = fmaf(cw[4 * k + j], v[k], acc[k]);
-                if (j > 0) *(fv *)(st + (size_t)(j - 1) * width) = v;     // a row up; the oldest goes
+                for (int k = 0; k < 4; ++k) acc[k] = fmaf(cw[4 * k + j], v[k], acc[k]);
+                if (j > 0) *(rg_f32x4 *)(st + (size_t)(j - 1) * width) = v;      // a row up; the oldest goes
             }
         }
-        *(fv *)(us_tile + tt * ld + i) = acc;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) us_tile[tt * ld + rg_place(i + k)] = acc[k];
     }
     // what a thread needs in the end for its first element
     float e_lam = 0.f, e_ba = 0.f, e_bi = 0.f, e_y = 0.f, e_s = 0.f;
@@ -514,43 +525,46 @@ rglru_single_kernel(const TI *__restrict__ rows, int row_stride, int y_off, int 
     if ((int)threadIdx.x < nt * bs) fetch_end(threadIdx.x);
     __syncthreads();
     // ---- the gates (the instruction's other rows are the last token's again)
-    for (int item = wave; item < items; item += RG_ONE_THREADS / WAVE) {
-        const int tile = item % tiles, part = item / tiles, j0 = part * tiles / parts, j1 = (part + 1) * tiles / parts;      // (in sixteens)
-        rg_f32x4 acc[2] = {rg_f32x4{0.f, 0.f, 0.f, 0.f}, rg_f32x4{0.f, 0.f, 0.f, 0.f}};
+    for (int tile = wave; tile < tiles; tile += RG_ONE_THREADS / WAVE) {
+        if (tile != wave) fetch(tile);
         const float *up = us_tile + min(l16, nt - 1) * ld + 4 * g;
-        for (int jb = j0; jb < j1; jb += 4) {
-            if (jb > j0 || item != wave) rg_fetch(w, gates, b, tile, tiles, lane, 16 * jb);
+        const rg_f32x4 none = {0.f, 0.f, 0.f, 0.f};
+        rg_f32x4 acc[2] = {none, none}, sum[2] = {none, none};
+        int left = each;                                                  // instructions until the slice's sums are whole
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (jb + j >= j1) break;
-                const rg_f32x4 x = *(const rg_f32x4 *)(up + 16 * (jb + j));
+        for (int j = 0; j < MOST; ++j) {
+            if (j >= tiles) break;
+            const rg_f32x4 x = *(const rg_f32x4 *)(up + 16 * j);
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
+            for (int e = 0; e < 4; ++e) {
 #pragma unroll
-                    for (int q = 0; q < 2; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[q][j][e], acc[q], 0, 0, 0);
+                for (int q = 0; q < 2; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[q][j][e], acc[q], 0, 0, 0);
+                if (--left == 0) {
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        sum[q] += acc[q];
+                        acc[q] = none;
+                    }
+                    left = each;
+                }
             }
         }
         if (g < RG_ONE_TOK / 4) {
 #pragma unroll
             for (int q = 0; q < 2; ++q)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) sums[((part * 2 + q) * RG_ONE_TOK + 4 * g + r) * ld + 16 * tile + l16] = acc[q][r];
+                for (int r = 0; r < 4; ++r) sums[q][4 * g + r][16 * tile + l16] = sum[q][r];
         }
     }
     __syncthreads();
     for (int x = threadIdx.x; x < nt * bs; x += RG_ONE_THREADS) {
         const int tt = x / bs, o = x % bs, t = tok0 + tt, c = b * bs + o;
         if (x != (int)threadIdx.x) fetch_end(x);                          // (blocks of more than 128 channels)
-        float sa = 0.f, si = 0.f;
-        for (int k = 0; k < parts; ++k) {
-            sa += sums[(2 * k * RG_ONE_TOK + tt) * ld + o];
-            si += sums[((2 * k + 1) * RG_ONE_TOK + tt) * ld + o];
-        }
-        const float gr = 1.0f / (1.0f + expf(-(sa + e_ba)));
-        const float gate = 1.0f / (1.0f + expf(-(si + e_bi)));
+        const float gr = 1.0f / (1.0f + expf(-(sums[0][tt][o] + e_ba)));
+        const float gate = 1.0f / (1.0f + expf(-(sums[1][tt][o] + e_bi)));
         const float log_a = -c_exp * gr * (e_lam > 20.f ? e_lam : log1pf(expf(e_lam)));
         const float mult = sqrtf(-expm1f(2.0f * log_a));
-        const float S = fmaf(expf(log_a), e_s, mult * gate * us_tile[tt * ld + o]);
+        const float S = fmaf(expf(log_a), e_s, mult * gate * us_tile[tt * ld + rg_place(o)]);
         state[((size_t)state_slot[t] * taps + taps - 1) * width + c] = S;
         out[(size_t)t * width + c] = from_f32<T>(S * gelu_tanh(e_y));
     }
@@ -646,8 +660,8 @@ rglru_scan_kernel(const TI *__restrict__ rows, int row_stride, int y_off, int x_
 // rows: [n, row_stride] of in_type, yin at y_off and xin at x_off (width each); bias: null or float32 over the row's
 // columns.  conv_w [width, taps], conv_b [width] (may be null), wa_t / wi_t [blocks, bs, bs] transposed ([in][out]),
 // ba / bi / lam [width], all float32; gates (may be null): both matrices in the order in which the matrix instruction takes them, [blocks][bs / 16 output
-// tiles][bs / 16 input tiles][2][64 lanes (l, g)][4]: output 16 tile + l, input 16 tile + 4 g + e, for bs a multiple of 16 up to 192 (read in steps of
-// more than 64 tokens, and of single tokens with bfloat16 outputs).  single: every request feeds one token.  state: float32 [slots, taps, width].  a, gx, y: float32 scratch of n * (width rounded up to 64) floats each.
+// tiles][bs / 16 input tiles][2][64 lanes (l, g)][4]: output 16 tile + l, input 16 tile + 4 e + g, for bs a multiple of 16 up to 192 (read in steps of
+// more than 64 tokens and of single tokens).  single: every request feeds one token.  state: float32 [slots, taps, width].  a, gx, y: float32 scratch of n * (width rounded up to 64) floats each.
 // out: [n, width] of out_type.
 LCU_API int lcu_rglru(const void *rows, int in_type, int row_stride, int y_off, int x_off, const float *bias,
                       const float *conv_w, const float *conv_b, const float *wa_t, const float *wi_t, const float *gates, const float *ba,
@@ -663,17 +677,15 @@ LCU_API int lcu_rglru(const void *rows, int in_type, int row_stride, int y_off, 
         return LCU_BAD_ARGUMENT;
     const bool matrix = gates != nullptr;
     if (matrix && (bs % 16 || bs > RG_MFMA_BS || (uintptr_t)gates % 16)) return LCU_BAD_ARGUMENT;
-    // (with 32-bit outputs the sliced kernel: there a token's bits do not depend on whether it comes alone or in a portion of up to 64)
-    if (matrix && single && n == n_req && taps <= RG_MFMA_TAPS && out_type == LCU_BF16) {
-        const bool fours = x_off % 4 == 0 && row_stride % 4 == 0 && ((uintptr_t)rows | (uintptr_t)conv_w | (uintptr_t)conv_b | (uintptr_t)state) % 16 == 0;
-        const int parts = rg_one_parts(bs / 16);
-        const dim3 grid((n + RG_ONE_TOK - 1) / RG_ONE_TOK, blocks);
-        const size_t lds = (size_t)(2 * parts + 1) * RG_ONE_TOK * (bs + 4) * sizeof(float);
-#define ONE(TI, V)                                                                                                                         \
-    rglru_single_kernel<TI, bf16_t, V><<<grid, dim3(RG_ONE_THREADS), lds, stream>>>((const TI *)rows, row_stride, y_off, x_off, bias, conv_w, conv_b, state, gates, ba, \
-                                                                              bi, lam, c_exp, (bf16_t *)out, ctx_len, state_slot, n, width, bs, taps)
-#define STEP(TI) do { if (fours) ONE(TI, 4); else ONE(TI, 1); } while (0)
-        if (in_type == LCU_BF16) STEP(bf16_t);
+    const int slices = n > RG_FEW_ROWS ? 1 : RG_SLICES;
+    // (a matrix instruction's four input channels lie in one slice)
+    if (matrix && single && n == n_req && taps <= RG_MFMA_TAPS && bs <= RG_ONE_BS && in_type == LCU_F32 && bs % (4 * slices) == 0 && x_off % 4 == 0 && row_stride % 4 == 0 &&
+        ((uintptr_t)rows | (uintptr_t)conv_w | (uintptr_t)conv_b | (uintptr_t)state) % 16 == 0) {
+#define ONE(T, MOST)                                                                                                                                                      \
+    rglru_single_kernel<T, MOST><<<dim3((n + RG_ONE_TOK - 1) / RG_ONE_TOK, blocks), dim3(RG_ONE_THREADS), 0, stream>>>((const float *)rows, row_stride, y_off, x_off, bias, conv_w, \
+                                                                              conv_b, state, gates, ba, bi, lam, c_exp, (T *)out, ctx_len, state_slot, n, width, bs, taps, slices)
+#define STEP(T) do { if (bs <= 64) ONE(T, 4); else ONE(T, RG_ONE_BS / 16); } while (0)
+        if (out_type == LCU_BF16) STEP(bf16_t);
         else STEP(float);
 #undef STEP
 #undef ONE
@@ -681,10 +693,11 @@ LCU_API int lcu_rglru(const void *rows, int in_type, int row_stride, int y_off, 
         return LCU_OK;
     }
     if (matrix && n > RG_FEW_ROWS) {
-        // 64 tokens a workgroup where those are RG_MFMA_WIDE at least (the matrices are read for each), else 16
-        const bool wide = (long long)((n + 63) / 64) * blocks >= RG_MFMA_WIDE;
+        // 64 tokens a workgroup where those are RG_MFMA_WIDE at least (the matrices are read for each), else 16; 16 with more taps, whose convolution is a chain of loads a
+        // tap (8 requests of 235 tokens, width 2048 in 16 blocks, 5 taps: 95 us, with 64 tokens a workgroup 122, on the vector unit 113)
+        const bool wide = taps <= RG_MFMA_TAPS && (long long)((n + 63) / 64) * blocks >= RG_MFMA_WIDE;
 #define GATES(TI, TT)                                                                                                                          \
-    rglru_gates_mfma_kernel<TI, TT><<<dim3((n + 16 * TT - 1) / (16 * TT), blocks), dim3(RG_MFMA_THREADS), 16 * TT * ((bs + 63) / 64 * 64 + 4) * sizeof(float), stream>>>( \
+    rglru_gates_mfma_kernel<TI, TT><<<dim3((n + 16 * TT - 1) / (16 * TT), blocks), dim3(RG_MFMA_THREADS), 16 * TT * (bs + 4) * sizeof(float), stream>>>( \
         (const TI *)rows, row_stride, x_off, bias, conv_w, conv_b, state, gates, ba, bi, lam, c_exp, a, gx, y, y_off, q_start, ctx_len, req_of_token,      \
         state_slot, n, width, bs, taps)
         if (in_type == LCU_F32) { if (wide) GATES(float, 4); else GATES(float, 1); }

@@ -2222,8 +2222,8 @@ def pack_rglru_gates(wa_t: torch.Tensor, wi_t: torch.Tensor) -> Optional[torch.T
     if bs % 16 or bs > RGLRU_GATES_MAX:
         return None
     t = bs // 16
-    # input 16 i + 4 g + e, output 16 o + l: [blocks, i, g, e, o, l] -> [blocks, o, i, g, l, e]
-    both = [m.reshape(blocks, t, 4, 4, t, 16).permute(0, 4, 1, 2, 5, 3) for m in (wa_t, wi_t)]
+    # input 16 i + 4 e + g, output 16 o + l: [blocks, i, e, g, o, l] -> [blocks, o, i, g, l, e]
+    both = [m.reshape(blocks, t, 4, 4, t, 16).permute(0, 4, 1, 3, 5, 2) for m in (wa_t, wi_t)]
     return torch.stack(both, dim=3).reshape(blocks, t, t, 2, 64, 4).contiguous()
 
 
@@ -2237,7 +2237,7 @@ def rglru(rows: torch.Tensor, y_off: int, x_off: int, bias: Optional[torch.Tenso
     ``[blocks, in, out]``); ``a = exp(-c_exp r softplus(lam))``; ``S <- a S + sqrt(1 - a^2) i u``; returns ``S *
     gelu_tanh(y branch)`` as ``[n, width]`` in ``out_dtype``.  ``state [slots, taps, width]`` float32: the last ``taps -
     1`` rows of the x branch, then ``S``; taken as zero at a request's position 0.  ``gates``: the result of ``pack_rglru_gates`` for the
-    two matrices: their products are then made on the matrix instruction."""
+    two matrices: their products are then made on the matrix instruction (the bits are the same)."""
     _gpu(rows, bias, conv_w, conv_b, wa_t, wi_t, ba, bi, lam, state, gates)
     _rows(rows, "rglru rows")
     n, cols = rows.shape

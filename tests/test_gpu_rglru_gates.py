@@ -100,3 +100,44 @@ def test_many_tokens_and_then_one(width, blocks, taps, lens, dtype):
         assert_close(part, want[:k], rel, f"request {i}")
         assert_close(then[i:i + 1], want[k:], rel, f"request {i}, the token behind")
         assert_close(state[slots[i]], after, 1e-4, f"state {i}")
+
+
+def both_ways(unit, args, rows, state, lens, ctx, slots, out_type):
+    """The same step with the packed gates and without them: outputs and the states behind it."""
+    from llama_cu_amd.kernels import ops
+    got = []
+    for gates in (unit.gates, None):
+        after = state.clone()
+        got.append((ops.rglru(rows, *args, after, hand_step(lens, ctx, slots), out_type, gates=gates), after))
+    return got
+
+
+@pytest.mark.parametrize("types", [(torch.float32, torch.bfloat16), (torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("width,blocks,taps", [(64, 2, 4), (16, 1, 4), (128, 2, 3), (96, 2, 2), (96, 1, 4), (2048, 16, 4), (192, 1, 1), (320, 2, 4), (128, 2, 5)])
+def test_bits_do_not_depend_on_the_kernel(width, blocks, taps, types):
+    """The kernels that take the packed gates add a token's products in the order of those without: single tokens up to 64 (eight parts of the input channels) and
+    beyond (one), four channels a thread and one, blocks whose parts are no whole matrix instruction; portions whose tokens come in tiles of 16."""
+    ti, to = types
+    for offsets in ((0, 8), (3, 5)):
+        unit = Unit(width, blocks, taps, offsets=offsets)
+        args = unit.args()
+        for n in (1, 5, 64, 65, 130):
+            rows, old = rnd(n, 2 * width + 8, seed=60).to(ti).cuda(), rnd(n, taps, width, seed=61).cuda()
+            (a, sa), (b, sb) = both_ways(unit, args, rows, old, [1] * n, [1 + (3 * i) % 7 for i in range(n)], list(range(n))[::-1], to)
+            assert torch.equal(a, b) and torch.equal(sa, sb), (offsets, n)
+        lens = [41, 1, 2, 30, 1]
+        rows, old = rnd(sum(lens), 2 * width + 8, seed=62).to(ti).cuda(), rnd(5, taps, width, seed=63).cuda()
+        (a, sa), (b, sb) = both_ways(unit, args, rows, old, lens, [41, 4, 2, 90, 2], [4, 2, 0, 1, 3], to)
+        assert torch.equal(a, b) and torch.equal(sa, sb), offsets
+
+
+@pytest.mark.parametrize("types", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("width,blocks,taps", [(2048, 16, 4), (1280, 16, 4), (3072, 16, 3), (1024, 64, 4), (768, 16, 2), (1024, 16, 6)])
+def test_bits_of_many_tokens(width, blocks, taps, types):
+    """64 tokens a workgroup, whose convolution a thread walks in one run, in two and in pieces that are no whole batch of sixteen."""
+    ti, to = types
+    unit = Unit(width, blocks, taps, offsets=(0, 8))
+    lens = [700, 1, 3, 64, 560]
+    rows, old = rnd(sum(lens), 2 * width + 8, seed=64).to(ti).cuda(), rnd(5, taps, width, seed=65).cuda()
+    (a, sa), (b, sb) = both_ways(unit, unit.args(), rows, old, lens, [700, 2, 40, 66, 560], [0, 3, 1, 4, 2], to)
+    assert torch.equal(a, b) and torch.equal(sa, sb)
