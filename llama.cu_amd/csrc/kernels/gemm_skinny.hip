@@ -100,11 +100,11 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// LOADS: loads of 128 k of sixteen rows of X (quad_rows.h): fewer than four for up to eight rows.
+// LOADS: loads of 128 k of the last tile's rows of X (quad_rows.h), fewer than four for up to eight of them; the tiles before take four.
 template <int NT, int MT, int LOADS>
 struct Frag {
     u32x4 w[NT][4];
-    u32x4 x[MT][LOADS];
+    u32x4 x[MT][4];
 };
 
 // A weight is read once per product and never again before the caches have turned over: the loads of a packed
@@ -134,7 +134,7 @@ __device__ __forceinline__ void load_frag(Frag<NT, MT, LOADS> &f, const bf16_t *
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int i = 0; i < LOADS; ++i)
+            for (int i = 0; i < (m < MT - 1 ? 4 : LOADS); ++i)
                 f.x[m][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, x_place + (4 * m + i) * x_four + 256u * s, 0, 0));
     } else {                                   // the last, partial macro-step (K is a multiple of 8)
 #pragma unroll
@@ -145,7 +145,7 @@ __device__ __forceinline__ void load_frag(Frag<NT, MT, LOADS> &f, const bf16_t *
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int i = 0; i < LOADS; ++i)
+            for (int i = 0; i < (m < MT - 1 ? 4 : LOADS); ++i)
                 f.x[m][i] = in ? __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, x_place + (4 * m + i) * x_four + 256u * s, 0, 0)) : zero;
     }
 }
@@ -155,7 +155,13 @@ __device__ __forceinline__ void mul_frag(const Frag<NT, MT, LOADS> &f, f32x4 (&a
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
         u32x4 x[4];
-        quad_operands<LOADS>(f.x[m], x);
+        if (m < MT - 1) quad_operands<4>(f.x[m], x);
+        else {
+            u32x4 few[LOADS];
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) few[i] = f.x[m][i];
+            quad_operands<LOADS>(few, x);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -233,7 +239,9 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
 
     // A ring of STAGES macro-steps in flight per wave: with few workgroups per compute unit
     // (small N) this is what keeps enough bytes on their way from HBM.
-    constexpr int STAGES = NT * MT == 1 ? 4 : NT * MT == 2 ? 3 : NT * MT == 8 && SK_WAVES == 8 ? 1 : 2;      // (the last for want of registers)
+    // Two tiles of rows with four of features: two as well while the second tile has up to eight rows (25 to 32 rows want the registers).  SwiGLU, us, 17 to 24 rows with two stages (with
+    // one, and all eight loads of rows): 7168 x 8192 33.0 to 34.1 (37.2 to 38.1), 2048 x 6144 23.3 to 24.3 (27.0 to 27.4), 7680 x 16384 65.8 to 67.9 (74.8 to 75.2).
+    constexpr int STAGES = NT * MT == 1 ? 4 : NT * MT == 2 ? 3 : NT * MT == 8 && SK_WAVES == 8 && LOADS == 4 ? 1 : 2;
     const int nsteps = (K + 127) / 128;
     Frag<NT, MT, LOADS> f[STAGES];
     int s = wave;
@@ -432,13 +440,13 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
     }
 }
 
-// (plain rows of W take their time whatever the rows of X do)
+// (plain rows of W take their time whatever the rows of X do; a last tile of few rows takes fewer loads where it is the only tile or where that leaves registers for a second stage)
 #define RUN(E, GRID, BLOCK)                                                            \
     do {                                                                               \
         if (!packed) RUN_AS(E, GRID, BLOCK, false, 4);                                 \
-        else if constexpr (MT > 1) RUN_AS(E, GRID, BLOCK, true, 4);                    \
-        else if (M <= 4) RUN_AS(E, GRID, BLOCK, true, 1);                              \
-        else if (M <= 8) RUN_AS(E, GRID, BLOCK, true, 2);                              \
+        else if constexpr (MT > 1 && !(NT * MT == 8 && WAVES == 8)) RUN_AS(E, GRID, BLOCK, true, 4); \
+        else if (M - 16 * (MT - 1) <= 4) RUN_AS(E, GRID, BLOCK, true, 1);              \
+        else if (M - 16 * (MT - 1) <= 8) RUN_AS(E, GRID, BLOCK, true, 2);              \
         else RUN_AS(E, GRID, BLOCK, true, 4);                                          \
     } while (0)
 #define RUN_AS(E, GRID, BLOCK, PACKED, LOADS)                                                                                \

@@ -130,3 +130,17 @@ def test_32_bit_rows(m):
         wide = torch.full((m, k + 8), float("nan"), device="cuda")
         wide[:, 4:4 + k] = x.cuda()
         assert torch.equal(ops.gemm_skinny_f32(wide[:, 4:4 + k], w.float().cuda()).cpu().double(), x @ w.t()), (n, k)
+
+
+@pytest.mark.parametrize("m", [17, 20, 21, 24, 25, 32])
+def test_four_tiles_and_a_last_one_of_few_rows(m):
+    """The loads of the second sixteen rows: one, two and four, several macro-steps a wave; sums below 2^24, and SwiGLU's bfloat16 rounding of its 32-bit functions."""
+    from llama_cu_amd.kernels import ops
+    for n, k in ((64, 3200), (128, 5120)):
+        x, w = whole((m, k), 20), whole((n, k), 21)
+        packed, rows = ops.pack_weight(w.to(BF16).cuda()), rows_of(x, m % 2)
+        assert torch.equal(ops.gemm_skinny(rows, packed, out_dtype=torch.float32, tiles=4, waves=8, packed=True).cpu().double(), x @ w.t())
+        sums = (x @ w.t()) / 64                              # (a gate that does not saturate: the rows in 64ths)
+        want = torch.nn.functional.silu(sums[:, :n // 2]) * sums[:, n // 2:]
+        got = ops.gemm_skinny(rows_of(x / 64, m % 2), packed, swiglu=True, tiles=4, waves=8, packed=True).cpu().double()
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-30).all()
