@@ -21,6 +21,7 @@
 #include "gate_act.h"
 #include "lane_moves.h"
 #include "pair_sum.h"
+#include "rows.h"
 
 constexpr int MOE_MAX_EXPERTS = 1024;
 constexpr int MOE_TILE_ROWS = 128;       // rows of a tile of the kernel for many rows at most
@@ -44,9 +45,6 @@ constexpr int ROUTE_CHUNKS = 8;                  // rows of up to 8 * 512 elemen
 // groups (ties: the lower index) can be chosen.  extra: rows of `router` behind the experts' (at most MOE_MAX_EXTRA); gates [n, extra] takes sigmoid
 // of their logits (they are no experts and are never chosen).
 constexpr int MOE_MAX_EXTRA = 8;
-// From so many values on four tokens a workgroup.  One MI355X, us, one and four, 64 experts: 1,000 tokens of 2048 22.2, 18.2 and of 1024 12.9, 12.3, of 512 8.0, 10.9;
-// 512 of 2048 13.6, 17.9
-constexpr int MOE_ROUTE_VALUES = 2000000;
 // The choice and its weights from a token's logits z, by one wave.  zc, sc: LDS, a number an expert each.
 __device__ __forceinline__ void route_choose(float *z, float *zc, float *sc, int t, int lane, const float *__restrict__ bias, int *__restrict__ ids,
                                              float *__restrict__ wts, float *__restrict__ gates, int n_experts, int top, int mode, int extra, int groups,
@@ -216,17 +214,17 @@ moe_route_kernel(const T *__restrict__ h, const float *__restrict__ router, cons
 // Rows of CHUNKS * 512 elements: no load hangs on a comparison, so a wave asks for its tokens' rows and its first two rows of the router at once, and
 // from then on for the next row while it works on one (the loop above waits for every 512 elements in turn).  TOKENS tokens a workgroup: the router's
 // matrix comes out of the second-level cache once for all of them, which bounds long steps, and a wave each makes their choices.  The same sums in the
-// same order.  One MI355X, d = 2048, 2,000 tokens: 16 experts and a gate 8.9 us (15.5), 256 experts 69 (156); 300 tokens 5.8 (6.7), 41 (69).  Small steps, which
+// same order.  One MI355X, 2,000 tokens, us: 16 experts and a gate, rows of 1024 6.5 (9.9), 2048 8.5 (16.3), 4096 20.4 (29.2); 256 experts 42 (72), 54 (142), 151 (309).  Small steps, which
 // share the rows out over the waves of 1,024 threads, gain nothing: 16 tokens and experts 5.1 (4.8).
-template <class T, int THREADS, int CHUNKS, int TOKENS>
-__global__ void __launch_bounds__(THREADS)
+constexpr int ROUTE_THREADS = 256;
+template <class T, int CHUNKS, int TOKENS>
+__global__ void __launch_bounds__(ROUTE_THREADS)
 moe_route_rows_kernel(const T *__restrict__ h, const float *__restrict__ router, const float *__restrict__ bias, int *__restrict__ ids,
                       float *__restrict__ wts, float *__restrict__ gates, int n, int n_experts, int top, int mode, int extra, int groups, int keep,
                       int renorm, float scale) {
     extern __shared__ float lds[];
-    constexpr int WAVES = THREADS / WAVE, D = CHUNKS * 512;
+    constexpr int WAVES = ROUTE_THREADS / WAVE, D = CHUNKS * 512;
     static_assert(TOKENS <= WAVES, "a wave a token");
-    const float *logit_bias = mode == 2 ? nullptr : bias;
     const int experts = n_experts + extra, t0 = blockIdx.x * TOKENS, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     float x[TOKENS][CHUNKS][8];
     f32x4 w[2 * CHUNKS], next[2 * CHUNKS];
@@ -239,11 +237,7 @@ moe_route_rows_kernel(const T *__restrict__ h, const float *__restrict__ router,
 #pragma unroll
     for (int b = 0; b < TOKENS; ++b)
 #pragma unroll
-        for (int k = 0; k < CHUNKS; ++k) {
-            const Row8<T> in = *(const Row8<T> *)(h + (size_t)min(t0 + b, n - 1) * D + k * 512 + lane * 8);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) x[b][k][i] = to_f32(in.v[i]);
-        }
+        for (int k = 0; k < CHUNKS; ++k) load_as_f32<T, 8>(h + (size_t)min(t0 + b, n - 1) * D + k * 512 + lane * 8, x[b][k]);
     for (int e = wave; e < experts; e += WAVES) {
         fetch(e + WAVES, next);
 #pragma unroll
@@ -254,7 +248,7 @@ moe_route_rows_kernel(const T *__restrict__ h, const float *__restrict__ router,
 #pragma unroll
                 for (int i = 0; i < 8; ++i) acc = fmaf(x[b][k][i], w[2 * k + i / 4][i % 4], acc);
             acc = wave_sum_in_place(acc);
-            if (lane == 0) lds[b * 3 * experts + e] = acc + (logit_bias && e < n_experts ? logit_bias[e] : 0.f);
+            if (lane == 0) lds[b * 3 * experts + e] = acc;
         }
 #pragma unroll
         for (int k = 0; k < 2 * CHUNKS; ++k) w[k] = next[k];
@@ -262,7 +256,24 @@ moe_route_rows_kernel(const T *__restrict__ h, const float *__restrict__ router,
     __syncthreads();
     if (wave >= TOKENS || t0 + wave >= n) return;
     float *z = lds + wave * 3 * experts;
+    if (mode != 2 && bias) {                                     // (here, all at once: in the loop every row would wait for its number)
+        for (int e = lane; e < n_experts; e += WAVE) z[e] += bias[e];
+        __threadfence_block();
+    }
     route_choose(z, z + experts, z + 2 * experts, t0 + wave, lane, bias, ids, wts, gates, n_experts, top, mode, extra, groups, keep, renorm, scale);
+}
+
+// Tokens a workgroup of it for `chunks` * 512 elements and so many rows of the router, 0: the general kernel.  The line lies where a workgroup more on every compute unit costs as
+// much as its tokens share.  Measured from 512 to 4,096 elements, 4 to 256 rows and 64 to 2,000 tokens, bfloat16, 64 rows, us with the general kernel, 1, 2 and 4 tokens: 400 tokens
+// of 1024 9.2, 6.8, 7.6, 10.6, of 3072 17.0, 16.7, 11.7, 17.0; 520 of 2048 15.5, 16.3, 11.5, 13.8, of 4096 26.8, 30.5, 24.6, 21.8; 1,000 of 1024 11.6, 11.9, 8.6, 10.8; 2,000 of 2048 41.2, 36.8, 23.8,
+// 17.6, of 3072 60.9, 57.4, 31.8, 33.7 (four tokens of more than 2048 and two of 4096 leave a compute unit one workgroup).  Four rows, one a wave, leave nothing to
+// ask for early, and in 32 bits the tokens' rows are most of what is read: 520 tokens of 2048 4.1, 4.7, 4.5, 4.5, 2,000 8.1, 8.9, 7.3, 6.8, of 3072 9.6, 12.2, 10.0, 11.2.  A form that masks the last
+// 512, for the widths between, took up to a quarter longer: with 16 rows and 1,000 tokens of 1000 elements as long as the general kernel (6.8 us), of 1528 too (7.8).
+static int route_tokens(int n, int chunks, int rows, int type) {
+    const long long values = (long long)n * chunks * 512;
+    if (type == LCU_F32 && rows <= ROUTE_THREADS / WAVE && chunks >= 4 && (chunks > 4 || values < 2000000)) return 0;
+    if (chunks <= 4) return values < 750000 ? 1 : values < 3000000 ? 2 : 4;
+    return chunks < 8 || n <= 512 ? 2 : 4;
 }
 
 // ---------------------------------------------------------------- group
@@ -816,27 +827,27 @@ LCU_API int lcu_moe_route(const void *h, int type, const float *router, const fl
     const bool few = n <= 256 && experts > 4;
     if (type != LCU_F32 && type != LCU_BF16) return LCU_BAD_ARGUMENT;
 #define ARGS experts, top, mode, extra, groups, keep, renorm, scale
-#define ROWS(T, TH, CHUNKS, TOKENS)                                                                                                                 \
-    moe_route_rows_kernel<T, TH, CHUNKS, TOKENS><<<dim3((n + TOKENS - 1) / TOKENS), dim3(TH), TOKENS * 3 * (experts + extra) * sizeof(float), stream>>>( \
-        (const T *)h, router, bias, ids, wts, gates, n, ARGS)
-#define CHUNKED(T, CHUNKS)                                  \
-    do {                                                    \
-        if ((long long)n * d < MOE_ROUTE_VALUES) ROWS(T, 256, CHUNKS, 1);  \
-        else ROWS(T, 256, CHUNKS, 4);                       \
+#define GENERAL(T, TH) moe_route_kernel<T, TH><<<dim3(n), dim3(TH), 0, stream>>>((const T *)h, router, bias, ids, wts, gates, d, ARGS)
+#define ROWS(T, CHUNKS, TOKENS)                                                                                                                          \
+    case 8 * CHUNKS + TOKENS:                                                                                                                             \
+        moe_route_rows_kernel<T, CHUNKS, TOKENS><<<dim3((n + TOKENS - 1) / TOKENS), dim3(ROUTE_THREADS), TOKENS * 3 * (experts + extra) * sizeof(float), stream>>>( \
+            (const T *)h, router, bias, ids, wts, gates, n, ARGS);                                                                                        \
+        break;
+#define GO(T)                                                                                                                                            \
+    do {                                                                                                                                                  \
+        if (few) GENERAL(T, 1024);                                                                                                                        \
+        else switch (8 * chunks + tokens) {                                                                                                               \
+            ROWS(T, 1, 1) ROWS(T, 1, 2) ROWS(T, 1, 4) ROWS(T, 2, 1) ROWS(T, 2, 2) ROWS(T, 2, 4) ROWS(T, 3, 1) ROWS(T, 3, 2) ROWS(T, 3, 4)                   \
+            ROWS(T, 4, 1) ROWS(T, 4, 2) ROWS(T, 4, 4) ROWS(T, 5, 2) ROWS(T, 6, 2) ROWS(T, 7, 2) ROWS(T, 8, 2) ROWS(T, 8, 4)                                 \
+            default: GENERAL(T, 256);                                                                                                                     \
+        }                                                                                                                                                 \
     } while (0)
-#define GO(T)                                                                                                                       \
-    do {                                                                                                                            \
-        if (few) moe_route_kernel<T, 1024><<<dim3(n), dim3(1024), 0, stream>>>((const T *)h, router, bias, ids, wts, gates, d, ARGS); \
-        else if (d == 512) CHUNKED(T, 1);                                                                                           \
-        else if (d == 1024) CHUNKED(T, 2);                                                                                          \
-        else if (d == 2048) CHUNKED(T, 4);                                                                                          \
-        else moe_route_kernel<T, 256><<<dim3(n), dim3(256), 0, stream>>>((const T *)h, router, bias, ids, wts, gates, d, ARGS);      \
-    } while (0)
+    const int chunks = d / 512, tokens = d % 512 || chunks > ROUTE_CHUNKS ? 0 : route_tokens(n, chunks, experts + extra, type);
     if (type == LCU_F32) GO(float);
     else GO(bf16_t);
 #undef GO
-#undef CHUNKED
 #undef ROWS
+#undef GENERAL
 #undef ARGS
     LCU_LAUNCH_CHECK();
     return LCU_OK;
