@@ -136,8 +136,9 @@ static int causal_conv_t(const TI *x, int x_stride, int x_off, const float *w, c
     }
     const int in = sizeof(TI) == 2 ? LCU_BF16 : LCU_F32, to = sizeof(TO) == 2 ? LCU_BF16 : LCU_F32;
     // In runs from a million values on: the activation of eight tokens in a row is a long chain.  One MI355X, us: 64 tokens of 3072 channels 8.5 (5.5 so), 250 of
-    // 3072 8.8 (8.0), 1,944 of 1536 11.9 (21.9)
-    const bool rows = (long long)n * channels >= CONV_RUN_VALUES && n / CONV_RUN_A_REQUEST >= n_req && taps > 1 && taps <= CONV_RUN_TAPS && channels % 4 == 0 && x_stride % 4 == 0 && out_stride % 4 == 0 &&
+    // 3072 8.8 (8.0), 1,944 of 1536 11.9 (21.9).  And from eight tokens a request on: single tokens' windows are made of the states, so 60 of them and a prompt of 300,
+    // 3072 channels, took 11.4 (9.9 so), 64 and a prompt of 1,500 15.3 (31.4)
+    const bool rows = (long long)n * channels >= CONV_RUN_VALUES && n / (2 * CONV_RUN_A_REQUEST) >= n_req && taps > 1 && taps <= CONV_RUN_TAPS && channels % 4 == 0 && x_stride % 4 == 0 && out_stride % 4 == 0 &&
                       four_ok(x + x_off, in) && four_ok(out, to) && four_ok(w, LCU_F32) && four_ok(bias, LCU_F32) && slot_stride % 4 == 0 && four_ok(state, LCU_F32);
 #define ROWS(TAPS)                                                                                                                                      \
     causal_conv_rows_kernel<TI, TO, TAPS><<<dim3((channels / 4 + CONV_RUN_THREADS - 1) / CONV_RUN_THREADS, (n + CONV_RUN - 1) / CONV_RUN), dim3(CONV_RUN_THREADS), 0, stream>>>( \

@@ -8,8 +8,10 @@
 // 12 (37); 2,000 rows of 3072 channels, 32-bit out, with silu 17 (37).
 constexpr int CONV_RUN = 8, CONV_RUN_THREADS = 256, CONV_RUN_TAPS = 4;
 // Steps of four tokens a request and more, and so many tokens in all.  Against a thread a token and channel, us: 100 requests of one token, 2 x 1024
-// channels 6.3 (4.7), 64 tokens of one 4.7 (4.7), at 2048 channels 4.8 (7.2).
-constexpr int CONV_RUN_TOKENS = 64, CONV_RUN_A_REQUEST = 4;
+// channels 6.3 (4.7), 64 tokens of one 4.7 (4.7), at 2048 channels 4.8 (7.2).  Up to 512 channels, where a workgroup walks a row in two steps at most, only
+// with CONV_RUN_NARROW values or more: 250 tokens of one, 2 x 64 channels, with the state behind it 6.9 (6.0), 2 x 512 7.1 (7.0); 60 single tokens and a prompt
+// of 300 9.3 (8.3), 2 x 1024 10.9 (11.4); 2,000 of one, 2 x 512 8.0 (16.1).
+constexpr int CONV_RUN_TOKENS = 64, CONV_RUN_A_REQUEST = 4, CONV_RUN_NARROW = 1 << 19;
 
 // h: the step's first row at the thread's first channel.  emit(k, window, pos, fresh): token k of the run, at position pos of its request, whose
 // first row of the step is its first at all if fresh;
@@ -30,21 +32,34 @@ __device__ __forceinline__ void conv_run(const TI *__restrict__ h, size_t stride
         pos[k] = ctx_len[r[k]] - (q_start[r[k] + 1] - (t0 + k));
         slot[k] = state_slot[r[k]];
     }
+    // four tokens at a time: what their windows want of requests' states is asked for before the first of them is made, so single tokens side by side are
+    // two trips to memory and not eight (60 of them and a prompt of 300, 2 x 1024 channels, with the states behind it: 10.9 us, one by one 12.0)
+    constexpr int SIDE = 4;
 #pragma unroll
-    for (int k = 0; k < CONV_RUN; ++k) {
-        if (k >= count) break;
-        const int into = t0 + k - first[k];                      // rows of the request before this one
-        if (into >= TAPS - 1) emit(k, &row[k], pos[k], pos[k] == into);
-        else {
+    for (int k0 = 0; k0 < CONV_RUN; k0 += SIDE) {
+        if (k0 >= count) break;
+        float old[SIDE][TAPS - 1][4];
+#pragma unroll
+        for (int b = 0; b < SIDE; ++b) {
+            const int k = k0 + b, into = t0 + k - first[k];      // rows of the request before this one (looked up for the run's last token where there are fewer)
+            if (into >= TAPS - 1) continue;
             const float *st = state_rows(slot[k]);
-            float old[TAPS - 1][4], window[TAPS][4];
 #pragma unroll
-            for (int j = 0; j < TAPS - 1; ++j) load_as_f32<float, 4>(st + min(j + into, TAPS - 2) * d, old[j]);
+            for (int j = 0; j < TAPS - 1; ++j) load_as_f32<float, 4>(st + min(j + into, TAPS - 2) * d, old[b][j]);
+        }
 #pragma unroll
-            for (int j = 0; j < TAPS; ++j)
+        for (int b = 0; b < SIDE; ++b) {
+            const int k = k0 + b, into = t0 + k - first[k];
+            if (k >= count) break;
+            if (into >= TAPS - 1) emit(k, &row[k], pos[k], pos[k] == into);
+            else {
+                float window[TAPS][4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) window[j][e] = j + into >= TAPS - 1 || j == TAPS - 1 ? row[k + j][e] : old[min(j, TAPS - 2)][e];
-            emit(k, window, pos[k], pos[k] == into);
+                for (int j = 0; j < TAPS; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) window[j][e] = j + into >= TAPS - 1 || j == TAPS - 1 ? row[k + j][e] : old[b][min(j, TAPS - 2)][e];
+                emit(k, window, pos[k], pos[k] == into);
+            }
         }
     }
 }

@@ -320,7 +320,7 @@ LCU_API int lcu_short_conv(const void *h, int h_type, long long set_stride_h, co
     if (d <= 0 || taps < 1 || taps > MAX_TAPS || sets < 1 || sets > 8 || h_type != LCU_F32 && h_type != LCU_BF16) return LCU_BAD_ARGUMENT;
     if (w_type != h_type && !(w_type == LCU_F32) && !(h_type == LCU_F32 && w_type == LCU_BF16)) return LCU_BAD_ARGUMENT;
     dim3 grid(n, sets), block(NC_THREADS);
-    const bool rows = n >= CONV_RUN_TOKENS && n / CONV_RUN_A_REQUEST >= n_req && d % 4 == 0 && taps > 1 && taps <= CONV_RUN_TAPS && set_stride_h % 4 == 0 && set_stride_out % 4 == 0 && four_ok(h, h_type) &&
+    const bool rows = n >= CONV_RUN_TOKENS && n / CONV_RUN_A_REQUEST >= n_req && (d > 2 * NC_THREADS || (long long)n * sets * d >= CONV_RUN_NARROW) && d % 4 == 0 && taps > 1 && taps <= CONV_RUN_TAPS && set_stride_h % 4 == 0 && set_stride_out % 4 == 0 && four_ok(h, h_type) &&
                       four_ok(cw, w_type) && four_ok(state, LCU_F32) && four_ok(out, out_type);
     const dim3 rgrid((n + CONV_RUN - 1) / CONV_RUN, sets, (d / 4 + CONV_RUN_THREADS - 1) / CONV_RUN_THREADS);
 #define ROWS(TI, TW, TO, TAPS) short_conv_rows_kernel<TI, TW, TO, TAPS><<<rgrid, dim3(CONV_RUN_THREADS), 0, stream>>>((const TI *)h, (size_t)set_stride_h, (const TW *)cw, state, (TO *)out, (size_t)set_stride_out, q_start, ctx_len, req_of_token, state_slot, n, d)

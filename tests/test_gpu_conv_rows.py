@@ -50,6 +50,27 @@ def test_short_convolution(types, d, taps):
         assert_close(part, want, 1e-6 if to == torch.float32 else 2.0 ** -8, f"request {r}")
 
 
+@pytest.mark.parametrize("ti,to", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("d,taps,long", [(516, 2, 90), (520, 3, 300), (1024, 4, 300), (512, 4, 497), (512, 4, 498), (40, 2, 6600)])
+def test_short_convolution_of_single_tokens_beside_a_prompt(ti, to, d, taps, long):
+    """Eight tokens a thread, each its request's only one, at their first position, within the convolution's reach of it and behind it, then a prompt that
+    begins inside a run: the bits and the states of the same requests in steps of fewer than 64 tokens, on both sides of the line for few channels."""
+    from llama_cu_amd.kernels import ops
+    sets, lens = 2, [1] * 13 + [long, 1]
+    ctx = [k + (i % 4 if k == 1 else 0) for i, k in enumerate(lens)]
+    h, w = rnd(sets, sum(lens), d, seed=11).to(ti).cuda(), rnd(sets, d, taps, seed=12, std=0.5).cuda().to(ti)
+    before = rnd(len(lens), sets, taps - 1, d, seed=13).cuda()
+    states = [before.clone() for _ in range(2)]
+    run = lambda rows, state, step: ops.short_conv(rows.contiguous(), w, state, torch.empty(rows.shape, dtype=to, device="cuda"), step)
+    whole = run(h, states[0], hand_step(lens, ctx, list(range(len(lens)))))
+    parts = [run(h[:, :13], states[1], hand_step(lens[:13], ctx[:13], list(range(13))))]
+    for a in range(0, long, 50):
+        k = min(50, long - a)
+        parts.append(run(h[:, 13 + a:13 + a + k], states[1], hand_step([k], [a + k], [13])))
+    parts.append(run(h[:, -1:], states[1], hand_step([1], ctx[-1:], [14])))
+    assert torch.equal(whole, torch.cat(parts, dim=1)) and torch.equal(*states)
+
+
 @pytest.mark.parametrize("types", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16)])
 @pytest.mark.parametrize("channels,taps,offset,bias,act", [(40, 2, 8, True, "silu"), (3072, 4, 0, False, "silu"), (1100, 3, 4, True, None), (40, 4, 3, True, None),
                                                            (38, 4, 0, False, None), (64, 6, 0, True, "silu")])
