@@ -925,7 +925,8 @@ def wavek_wide(n: int) -> bool:
 
 
 def wavek_preferred(m: int, n: int, k: int, swiglu: bool = False, grouped: bool = False) -> bool:
-    """Whether ``gemm_wavek`` is the fastest choice for ``m`` rows and a packed ``[n, k]`` weight (``TUNING``'s numbers; ``n`` counts all groups)."""
+    """Whether ``gemm_wavek`` is the fastest choice for ``m`` rows and a packed ``[n, k]`` weight (``TUNING``'s numbers; ``n`` counts all groups,
+    which share no row: ``grouped``)."""
     t = TUNING
     if m > WAVEK_MAX_ROWS or k > t.wavek_max_k or n > 32 * t.compute_units:                    # (more workgroups of 32 features than compute units: a second round)
         return False
@@ -933,13 +934,22 @@ def wavek_preferred(m: int, n: int, k: int, swiglu: bool = False, grouped: bool 
         return min(n, k) >= t.wavek_swiglu_least
     if k < t.wavek_short_k:
         return True
-    if m <= t.wavek_few_rows:
+    if not grouped and n >= t.skinny_two_tiles_from and k > t.wavek_two_tiles_k and m <= t.wavek_two_tiles_rows:
+        return False
+    few = t.wavek_few_group_rows if grouped else t.wavek_wide_few_rows if n > t.wavek_wide_few_features and k <= t.wavek_wide_few_k else t.wavek_few_rows
+    if m <= few:
         return wavek_wide(n)
     if n < t.wavek_few_features and k * m > t.wavek_few_features_work:
         return False
     if n > t.wavek_many_features and m > t.wavek_many_rows and k > t.wavek_short_k:
         return False
     return n >= t.wavek_least_features or m <= t.wavek_least_rows
+
+
+def library_before_wavek(m: int, n: int, k: int) -> bool:
+    """Whether the library's plain bfloat16 product is the faster one of this size, where ``gemm_wavek`` is taken by the rest of its range."""
+    t = TUNING
+    return t.wavek_library_rows < m < WAVEK_MAX_ROWS and t.wavek_few_features < n <= t.wavek_library_features and k > t.wavek_library_k
 
 
 def gemm_wavek(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None,

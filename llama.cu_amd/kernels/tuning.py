@@ -60,7 +60,7 @@ class Tuning:
     mid_min_slice_steps: int = 4        # a slice of K keeps at least this many macro-steps of 128
     mid_max_slices: int = 8
     # ---- the product whose waves share out K (gemm_wavek.hip, up to 64 rows)
-    # (its numbers stand in gemm_wavek.hip; measured with widths of 1024 and 2048)
+    # (its numbers stand in gemm_wavek.hip; measured with 64 to 8192 features, K of 128 to 4096 and the matrix out of memory)
     wavek_wide_per_cu: int = 16         # 32 features a workgroup instead of 16 beyond so many features a compute unit (4096 x 2048 at 4 / 33 rows: 6.2 / 9.8 us
                                         # with 32, 5.4 / 8.4 with 16; 5120 x 2048 6.4 / 9.9 and 7.0 / 14.8)
     wavek_max_k: int = 4096             # the longest K measured (4096 features, K = 4096: 8.6 us against the weight-streaming kernel's 9.1 at 16 rows, 10.7
@@ -68,7 +68,14 @@ class Tuning:
     wavek_short_k: int = 1024           # with a K below it is the fastest at any number of rows (2048 x 512: 2.7 us against 2.8 at 1 row, 3.4 against 3.8 at 24, 4.2
                                         # against the library's 7.0 at 64; 16 groups of 128 x 128 2.5 against 2.8 at 8 rows, 2.8 against 4.6 at 32, 3.2 against 4.9 at 64)
     wavek_few_rows: int = 8             # up to here a plain product goes to it beyond wavek_wide_per_cu only (5120 x 2048: 6.4 us against 6.8 at 8 rows; with 2048
-                                        # features 4.4 and 4.4, with 6144 x 4096 11.7 and 11.0); from 9 rows on 0.97 of the weight-streaming kernel's time, at 24 0.92
+                                        # features 4.4 and 4.4); from 9 rows on 0.97 of the weight-streaming kernel's time, at 24 0.92
+    wavek_wide_few_rows: int = 12       # ... up to here beyond wavek_wide_few_features with a K up to wavek_wide_few_k (4096 x 1408 at 9 and 12 rows 5.0 and 5.0 us
+    wavek_wide_few_features: int = 3072  # against the weight-streaming kernel's 4.7 and 4.7, 4096 x 2816 7.1 and 6.9 against 6.9 and 6.7; 3072 x 2048 5.3 and 5.3, 4096 x 4096
+    wavek_wide_few_k: int = 2816        # 9.0 against 9.1)
+    wavek_few_group_rows: int = 4       # ... up to here a product in groups (2 of 1024 x 1024 with a gate at 8 rows: 4.0 us against 4.4; without one 3.4 to 3.5 either way)
+    wavek_two_tiles_k: int = 3840       # with a longer K, and features from skinny_two_tiles_from on, the weight-streaming kernel is faster up to
+    wavek_two_tiles_rows: int = 16      # so many rows (8192 x 4096: 15.0 us against 13.5 at 1 to 16 rows, 16.8 against 16.7 at 17; 6144 x 4096 11.8 to 12.5 against 11.3 to 12.0;
+                                        # 8192 x 3840 12.4 to 13.3 against 12.8 to 13.5)
     wavek_few_features: int = 1024      # few workgroups, each with much to do: below so many features not where K times the rows is beyond
     wavek_few_features_work: int = 98304    # this (512 x 4096 at 64 rows 12.6 us against the library's 11.3, 64 x 2048 7.5 against 5.2; at 48 6.4 against 7.7)
     wavek_least_features: int = 64      # below so many, and a K that is not short, only up to
@@ -76,6 +83,9 @@ class Tuning:
     wavek_many_features: int = 6144     # beyond so many features, with a K beyond wavek_short_k, up to
     wavek_many_rows: int = 48           # so many rows (8192 x 2048 at 64 rows 12.4 us against the library's 13.7 with the matrix out of memory, 11.8 against 11.0 in a
                                         # model that runs its layers in a loop and finds it in the last-level cache; 10.7 against 13.9 at 48)
+    wavek_library_rows: int = 48        # above so many rows and below 64, up to wavek_library_features and with a K beyond wavek_library_k, the library's plain product is
+    wavek_library_features: int = 4096  # faster (2048 x 3072: 11.1 us against 10.3 at 49 to 63 rows, 11.1 against 15.6 at 64, 10.0 against 10.3 at 48; 4096 x 4096 15.0 against
+    wavek_library_k: int = 2688         # 14.0; 1280 x 2816 9.9 against 9.6; 1024 x 2816 9.7 against 11.2, 2048 x 2688 9.7 against 13.6, 4352 x 4096 15.9 against 16.9)
     wavek_swiglu_least: int = 512       # gate and up rows and K from which on SwiGLU was measured (1024 x 512 to 8192 x 4096: the library's product alone, without
                                         # the activation kernel's 2 us, is 1 us faster at most, at 48 rows of 2816 x 3072; the row-sharing kernel 1.5 us slower at 64 rows and 0.9
                                         # faster at 24 to 32 rows of 8192, which go to it: mid_swiglu_features)

@@ -75,7 +75,8 @@ def linear(x: torch.Tensor, weight: Union[torch.Tensor, Weight], out_dtype: Opti
     out_dtype = out.dtype if out is not None else (out_dtype or x.dtype)
     all_bf16 = x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
     if (all_bf16 and packed is not None and packed.shape == weight.shape and not accumulate and x.dim() == 2 and wavek_takes(x, packed)
-            and out_dtype in (torch.bfloat16, torch.float32) and (out is None or _plain_rows(out))):
+            and out_dtype in (torch.bfloat16, torch.float32) and (out is None or _plain_rows(out))
+            and not (out_dtype == torch.bfloat16 and ops.library_before_wavek(x.shape[0], *weight.shape))):
         return ops.gemm_wavek(x, packed, out=out, out_dtype=out_dtype)
     if all_bf16 and ops.skinny_supported(x, weight, out_dtype) and (
             accumulate or ops.skinny_preferred(x.shape[0], weight.shape[0], weight.shape[1], out_dtype, packed is not None)):

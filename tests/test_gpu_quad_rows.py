@@ -144,3 +144,12 @@ def test_four_tiles_and_a_last_one_of_few_rows(m):
         want = torch.nn.functional.silu(sums[:, :n // 2]) * sums[:, n // 2:]
         got = ops.gemm_skinny(rows_of(x / 64, m % 2), packed, swiglu=True, tiles=4, waves=8, packed=True).cpu().double()
         assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 6144, 4096), (17, 6144, 4096), (9, 4096, 1408), (48, 1152, 2816), (49, 1152, 2816), (63, 1152, 2816), (64, 1152, 2816)])
+def test_products_on_both_sides_of_a_line(m, n, k):
+    """The kernels and the library's product between which ``linear`` chooses: exact sums, rounded once."""
+    from llama_cu_amd.parts.linear import Weight, linear
+    x, w = whole((m, k), 22), whole((n, k), 23)
+    got = linear(rows_of(x, m % 2), Weight(w.to(BF16).cuda()))
+    assert torch.equal(got.double().cpu(), (x @ w.t()).to(BF16).double())

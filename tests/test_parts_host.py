@@ -44,3 +44,16 @@ def test_the_rows_of_zeros_for_the_library_can_be_fixed_instead_of_timed(monkeyp
     assert linear.library_friendly_rows(11008, 4096, "cpu") == 12288
     assert linear.library_friendly_rows(14336, 4096, "cpu") == 14336
     assert linear.library_friendly_rows(176, 64, "cpu") == 176            # small matrices stay as they are
+
+
+def test_which_products_the_waves_that_share_out_k_take():
+    """The rule's lines, both sides of each (``TUNING`` says what was measured there)."""
+    from llama_cu_amd.kernels import ops
+    takes = ops.wavek_preferred
+    assert not takes(12, 4096, 2048) and takes(13, 4096, 2048) and takes(9, 3072, 2048) and takes(9, 4096, 2944) and not takes(8, 4096, 2944)
+    assert not takes(16, 6144, 4096) and takes(17, 6144, 4096) and takes(16, 6144, 3840) and takes(16, 6128, 4096)
+    assert not takes(4, 2048, 1024, grouped=True) and takes(5, 2048, 1024, grouped=True) and not takes(5, 2048, 1024)
+    assert takes(64, 64, 896) and not takes(64, 8192, 2048) and not takes(65, 2048, 512) and not takes(20, 2048, 4224)
+    library = ops.library_before_wavek
+    assert library(49, 2048, 2816) and library(63, 4096, 4096)
+    assert not any(library(*s) for s in ((48, 2048, 2816), (64, 2048, 2816), (49, 1024, 2816), (49, 4112, 2816), (49, 2048, 2688)))
