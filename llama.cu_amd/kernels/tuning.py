@@ -90,8 +90,10 @@ class Tuning:
                                         # the activation kernel's 2 us, is 1 us faster at most, at 48 rows of 2816 x 3072; the row-sharing kernel 1.5 us slower at 64 rows and 0.9
                                         # faster at 24 to 32 rows of 8192, which go to it: mid_swiglu_features)
     wavek_qkv_rows: int = 32            # q/k/v with the rotation and the cache write in its epilogue goes to it above so many rows and up to 64, where the row-sharing
-                                        # kernel would be taken (48 heads of 128, K = 4096: 20.0 us against 21.9 at 64 rows, 18.0 against 18.8 at 48; 15.5 against 14.8 at
-                                        # 24; 24 heads, K = 2048: 12.1 against 12.9 at 64, 10.8 against 10.7 at 48)
+                                        # kernel would be taken, whatever K (us at 33, 48 and 64 rows, 48 heads of 128, K = 4096: 17.8, 18.3, 19.5 against 19.0, 19.2, 21.2, K = 8192:
+                                        # 28.2, 30.2, 32.0 against 32.6, 31.0, 35.1; 24 heads, K = 512: 6.1, 6.4, 7.2 against 6.2, 6.3, 7.5, K = 2048: 10.5, 10.9, 12.3
+                                        # against 10.7, 10.5, 12.6; 8 heads of 64, K = 8192: 21.8, 23.4, 26.6 against 27.8, 27.8, 31.2; measured for 8 to 64 heads); 15.5
+                                        # against 14.8 at 24 rows, 48 heads, K = 4096
     # ---- the library's product of many rows (parts/linear.library_friendly_rows)
     library_rows: int = -1              # rows of zeros behind each half of a plain gate/up matrix: -1 times the library once per
                                         # shape at load and fills up where that is 15 % faster (the outcome can differ from box
