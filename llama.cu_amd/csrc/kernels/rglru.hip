@@ -440,8 +440,8 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
 
 // A step in which every request feeds one token (token i is request i's): the gates as above, the recurrence's step and the state's update in one
 // kernel.  A workgroup takes four tokens and a block of channels; whatever of a slot's state belongs to a channel is read and written by
-// its threads alone.  Eight waves share out the output channels, 16 at a time, the first of which a wave asks for in front of everything; then a thread an
-// element for the functions, which with the lanes that hold the sums were four one after the other, most of them of tokens that are not there.  The sums are
+// its threads alone.  A wave takes 16 output channels, whose matrices it asks for in front of everything; then a thread an element for the functions,
+// which with the lanes that hold the sums were four one after the other, most of them of tokens that are not there.  The sums are
 // those of `slices` equal parts of the input channels, added in their order: RG_SLICES up to RG_FEW_ROWS tokens, one beyond, as the kernels above have them, so
 // that a token's bits do not depend on what else a step of so many tokens holds.  32-bit rows whose fours are aligned (the layer's), up to four taps, slices of whole matrix
 // instructions.  Latency bounds it: four trips to memory, 1.7 us of matrix instructions.  One MI355X, 4 taps, us beside the sliced kernel and the scan: width 2048
@@ -461,16 +461,15 @@ rglru_single_kernel(const float *__restrict__ rows, int row_stride, int y_off, i
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
     const int tiles = bs / 16, each = bs / 4 / slices;                    // matrix instructions a slice
     rg_f32x4 w[2][MOST];
-    auto fetch = [&](int tile) {
-        const float *at = gates + (size_t)(b * tiles + tile) * tiles * 512 + 4 * lane;
+    if (wave < tiles) {
+        const float *at = gates + (size_t)(b * tiles + wave) * tiles * 512 + 4 * lane;
 #pragma unroll
         for (int j = 0; j < MOST; ++j) {
             if (j >= tiles) break;
 #pragma unroll
             for (int q = 0; q < 2; ++q) w[q][j] = *(const rg_f32x4 *)(at + 512 * j + 256 * q);
         }
-    };
-    if (wave < tiles) fetch(wave);
+    }
     // ---- u, four neighbouring channels of a token a thread
     auto load = [](const float *q) { return *(const rg_f32x4 *)q; };
     for (int x = threadIdx.x; x < nt * (bs / 4); x += RG_ONE_THREADS) {
@@ -512,21 +511,21 @@ rglru_single_kernel(const float *__restrict__ rows, int row_stride, int y_off, i
 #pragma unroll
         for (int k = 0; k < 4; ++k) us_tile[tt * ld + rg_place(i + k)] = acc[k];
     }
-    // what a thread needs in the end for its first element
+    // what a thread needs in the end for its element
+    static_assert(RG_ONE_TOK * RG_ONE_BS <= RG_ONE_THREADS && RG_ONE_BS / 16 <= RG_ONE_THREADS / WAVE, "an element a thread, sixteen output channels a wave");
+    const int e_tt = threadIdx.x / bs, e_o = threadIdx.x % bs, e_t = tok0 + e_tt, e_c = b * bs + e_o;
+    const bool e_in = e_tt < nt;
     float e_lam = 0.f, e_ba = 0.f, e_bi = 0.f, e_y = 0.f, e_s = 0.f;
-    auto fetch_end = [&](int x) {
-        const int t = tok0 + x / bs, c = b * bs + x % bs;
-        e_lam = lam[c];
-        e_ba = ba[c];
-        e_bi = bi[c];
-        e_y = to_f32(rows[(size_t)t * row_stride + y_off + c]) + (bias ? bias[y_off + c] : 0.f);
-        e_s = ctx_len[t] > 1 ? state[((size_t)state_slot[t] * taps + taps - 1) * width + c] : 0.f;
-    };
-    if ((int)threadIdx.x < nt * bs) fetch_end(threadIdx.x);
+    if (e_in) {
+        e_lam = lam[e_c];
+        e_ba = ba[e_c];
+        e_bi = bi[e_c];
+        e_y = to_f32(rows[(size_t)e_t * row_stride + y_off + e_c]) + (bias ? bias[y_off + e_c] : 0.f);
+        e_s = ctx_len[e_t] > 1 ? state[((size_t)state_slot[e_t] * taps + taps - 1) * width + e_c] : 0.f;
+    }
     __syncthreads();
     // ---- the gates (the instruction's other rows are the last token's again)
-    for (int tile = wave; tile < tiles; tile += RG_ONE_THREADS / WAVE) {
-        if (tile != wave) fetch(tile);
+    if (wave < tiles) {
         const float *up = us_tile + min(l16, nt - 1) * ld + 4 * g;
         const rg_f32x4 none = {0.f, 0.f, 0.f, 0.f};
         rg_f32x4 acc[2] = {none, none}, sum[2] = {none, none};
@@ -553,20 +552,18 @@ rglru_single_kernel(const float *__restrict__ rows, int row_stride, int y_off, i
 #pragma unroll
             for (int q = 0; q < 2; ++q)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) sums[q][4 * g + r][16 * tile + l16] = sum[q][r];
+                for (int r = 0; r < 4; ++r) sums[q][4 * g + r][16 * wave + l16] = sum[q][r];
         }
     }
     __syncthreads();
-    for (int x = threadIdx.x; x < nt * bs; x += RG_ONE_THREADS) {
-        const int tt = x / bs, o = x % bs, t = tok0 + tt, c = b * bs + o;
-        if (x != (int)threadIdx.x) fetch_end(x);                          // (blocks of more than 128 channels)
-        const float gr = 1.0f / (1.0f + expf(-(sums[0][tt][o] + e_ba)));
-        const float gate = 1.0f / (1.0f + expf(-(sums[1][tt][o] + e_bi)));
+    if (e_in) {
+        const float gr = 1.0f / (1.0f + expf(-(sums[0][e_tt][e_o] + e_ba)));
+        const float gate = 1.0f / (1.0f + expf(-(sums[1][e_tt][e_o] + e_bi)));
         const float log_a = -c_exp * gr * (e_lam > 20.f ? e_lam : log1pf(expf(e_lam)));
         const float mult = sqrtf(-expm1f(2.0f * log_a));
-        const float S = fmaf(expf(log_a), e_s, mult * gate * us_tile[tt * ld + rg_place(o)]);
-        state[((size_t)state_slot[t] * taps + taps - 1) * width + c] = S;
-        out[(size_t)t * width + c] = from_f32<T>(S * gelu_tanh(e_y));
+        const float S = fmaf(expf(log_a), e_s, mult * gate * us_tile[e_tt * ld + rg_place(e_o)]);
+        state[((size_t)state_slot[e_t] * taps + taps - 1) * width + e_c] = S;
+        out[(size_t)e_t * width + e_c] = from_f32<T>(S * gelu_tanh(e_y));
     }
 }
 
