@@ -37,6 +37,7 @@
 #include "lane_moves.h"
 #include "gate_act.h"
 #include "kv_layout.h"
+#include "qkv_store.h"
 #include "quad_rows.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -73,15 +74,7 @@ struct SkinnyExtra {
     int n_in;
     int norm_width;
     float eps;
-    // EPI_QKV_ROPE
-    const int *positions;      // [M]
-    const int *slots;          // [M] page * page_size + place, or -1: store nothing
-    const float *cos_t, *sin_t;  // [max_pos, head_dim / 2]
-    int max_pos;
-    bf16_t *cache;             // this layer's pages
-    bf16_t *q_out;             // [M, heads * head_dim] rows ldq apart
-    int ldq;
-    int heads, kv_heads, head_dim, page;
+    QkvStore qkv;              // EPI_QKV_ROPE
     // EPI_ADD_NORM: what the product is multiplied by before it is added to the residual stream
     float res_scale;
     // EPI_SWIGLU: limit > 0 asks for the limited activation (gate_act.h)
@@ -182,14 +175,14 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
     // SwiGLU: the first NT/2 tiles are gate rows, the other NT/2 the up rows N/2 further
     const int n0 = blockIdx.x * 16 * (EPI == EPI_SWIGLU ? NT / 2 : NT);
     // q/k/v with rotation: workgroup b has, of head b / (head_dim/32), the dims 16 c .. and head_dim/2 + 16 c ..
-    const int rope_head = EPI == EPI_QKV_ROPE ? blockIdx.x / (ex.head_dim / 32) : 0;
-    const int rope_c = EPI == EPI_QKV_ROPE ? blockIdx.x % (ex.head_dim / 32) : 0;
+    const int rope_head = EPI == EPI_QKV_ROPE ? blockIdx.x / (ex.qkv.head_dim / 32) : 0;
+    const int rope_c = EPI == EPI_QKV_ROPE ? blockIdx.x % (ex.qkv.head_dim / 32) : 0;
     const bf16_t *wrow[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         const int half = t / (NT / 2 > 0 ? NT / 2 : 1);              // 0: gate tiles, 1: up tiles (SwiGLU)
         int row = EPI == EPI_SWIGLU ? n0 + 16 * (t % (NT / 2 > 0 ? NT / 2 : 1)) + l16 + half * n_out : n0 + 16 * t + l16;
-        if (EPI == EPI_QKV_ROPE) row = rope_head * ex.head_dim + t * (ex.head_dim / 2) + 16 * rope_c + l16;
+        if (EPI == EPI_QKV_ROPE) row = rope_head * ex.qkv.head_dim + t * (ex.qkv.head_dim / 2) + 16 * rope_c + l16;
         const int limit = EPI == EPI_SWIGLU ? (half + 1) * n_out : N;
         row = row < limit ? row : limit - 1;                          // a row beyond the end is read, not stored
         wrow[t] = PACKED ? W + ((size_t)(row / 16) * (K / 128)) * 2048 + (size_t)lane * 8   // (the tile of the row)
@@ -293,51 +286,12 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
     }
     if (EPI == EPI_QKV_ROPE) {
         // the lane holds dims i = 16 c + 4 grp + r (tile 0) and i + head_dim/2 (tile 1) of token 16 m + col
-        const int dh = ex.head_dim, half_dim = dh / 2;
-        const bool is_q = rope_head < ex.heads, is_k = !is_q && rope_head < ex.heads + ex.kv_heads;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const int tok = 16 * m + col;
             if (tok >= M) continue;
-            const int pos = ex.positions[tok];
-            const bool in_table = pos >= 0 && pos < ex.max_pos;
-            const int slot = ex.slots ? ex.slots[tok] : -1;
-            bf16_t *pg = nullptr;
-            int place = 0;
-            if (!is_q && slot >= 0) {
-                pg = ex.cache + (size_t)(slot / ex.page) * kv_page_elems(ex.kv_heads, dh, ex.page);
-                place = slot % ex.page;
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = 16 * rope_c + 4 * grp + r;
-                // rounded to bfloat16 before the rotation, as the product's plain epilogue stores them for
-                // the rotation kernel: a token's query and key are the same bits whichever way they are made
-                float a = to_f32(from_f32<bf16_t>(acc[0][m][r])), b = to_f32(from_f32<bf16_t>(acc[NT - 1][m][r]));
-                if (is_q || is_k) {
-                    float c = __uint_as_float(0x7fc00000u), sn = c;         // a position outside the table gives NaN
-                    if (in_table) { c = ex.cos_t[(size_t)pos * half_dim + i]; sn = ex.sin_t[(size_t)pos * half_dim + i]; }
-                    float ra, rb;
-                    rotate_pair(a, b, c, sn, ra, rb);
-                    a = ra; b = rb;
-                }
-                const bf16_t va = from_f32<bf16_t>(a), vb = from_f32<bf16_t>(b);
-                if (is_q) {
-                    bf16_t *qo = ex.q_out + (size_t)tok * ex.ldq + (size_t)rope_head * dh;
-                    qo[i] = va;
-                    qo[i + half_dim] = vb;
-                } else if (pg) {
-                    if (is_k) {
-                        const int kvh = rope_head - ex.heads;
-                        pg[kv_key_offset(kvh, place, i, dh, ex.page)] = va;
-                        pg[kv_key_offset(kvh, place, i + half_dim, dh, ex.page)] = vb;
-                    } else {
-                        const int kvh = rope_head - ex.heads - ex.kv_heads;
-                        pg[kv_value_offset(ex.kv_heads, kvh, place, i, dh, ex.page)] = va;
-                        pg[kv_value_offset(ex.kv_heads, kvh, place, i + half_dim, dh, ex.page)] = vb;
-                    }
-                }
-            }
+            const float lo[4] = {acc[0][m][0], acc[0][m][1], acc[0][m][2], acc[0][m][3]}, hi[4] = {acc[NT - 1][m][0], acc[NT - 1][m][1], acc[NT - 1][m][2], acc[NT - 1][m][3]};
+            qkv_store(ex.qkv, rope_head, tok, 16 * rope_c + 4 * grp, lo, hi);
         }
         return;
     }
@@ -473,7 +427,7 @@ static int launch_epi(const void *X, int ldx, const void *W, int ldw, void *Y, i
         return LCU_UNSUPPORTED;
     case EPI_QKV_ROPE:
         if constexpr (MT <= 2 && NT == 2) {
-            const dim3 rgrid((ex.heads + 2 * ex.kv_heads) * (ex.head_dim / 32));
+            const dim3 rgrid((ex.qkv.heads + 2 * ex.qkv.kv_heads) * (ex.qkv.head_dim / 32));
             RUN(EPI_QKV_ROPE, rgrid, block);
             break;
         }
@@ -625,9 +579,7 @@ LCU_API int lcu_gemm_skinny_bf16_qkv_rope(const void *X, int ldx, const void *W,
         return LCU_BAD_ARGUMENT;
     SkinnyExtra ex = {};
     ex.sumsq_in = sumsq_in; ex.n_in = n_in; ex.norm_width = norm_width; ex.eps = eps;
-    ex.positions = positions; ex.slots = slots; ex.cos_t = cos_t; ex.sin_t = sin_t; ex.max_pos = max_pos;
-    ex.cache = (bf16_t *)cache; ex.q_out = (bf16_t *)q_out; ex.ldq = ldq;
-    ex.heads = heads; ex.kv_heads = kv_heads; ex.head_dim = head_dim; ex.page = page;
+    ex.qkv = {positions, slots, cos_t, sin_t, max_pos, (bf16_t *)cache, (bf16_t *)q_out, ldq, heads, kv_heads, head_dim, page};
     const int N = (heads + 2 * kv_heads) * head_dim;
     return skinny_bf16(X, ldx, W, ldw, q_out, N, M, N, K, EPI_QKV_ROPE, 2, waves, w_packed, ex, stream);
 }
