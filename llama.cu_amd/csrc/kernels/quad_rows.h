@@ -20,8 +20,6 @@ __device__ __forceinline__ int quad_row(int c) { return 4 * (c & 3) + (c >> 2); 
 __device__ __forceinline__ int quad_k(int lane) { return 32 * (lane >> 4) + 8 * (lane & 3); }
 __device__ __forceinline__ int quad_load_row(int i, int lane) { return 4 * i + ((lane >> 2) & 3); }
 
-constexpr int quad_loads(int rows) { return rows <= 4 ? 1 : rows <= 8 ? 2 : 4; }
-
 // Between registers and lanes the rule is: lo <- where `keep`: lo, else hi of the partner lane; hi <- where `keep`: lo of the partner lane, else
 // hi.  The partner is one or two lanes away; keep is the mask of the lanes without that bit.  32 instructions for sixteen rows of 128 k, whose
 // operand out of another lane makes them twice as slow as others: 2 us of the 8.3 that 64 rows of 2048 x 2048 take.  (Left to the compiler, a
