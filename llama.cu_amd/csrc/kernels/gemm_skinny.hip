@@ -33,6 +33,7 @@
 // Grouped: W is several matrices of group_rows rows one above the other, and each multiplies rows of X of its own
 // (group g reads X + g * x_group_stride): one product per head, or several projections of differently mixed rows, in
 // one launch.  Their outputs may be multiplied by the sigmoid of a gate [M, N] on the way out.
+#include <type_traits>
 #include "common.h"
 #include "lane_moves.h"
 #include "gate_act.h"
@@ -599,9 +600,10 @@ LCU_API int lcu_gemm_skinny_bf16_qkv_rope(const void *X, int ldx, const void *W,
 // way out (norm_w), and gate and up rows may meet in SwiGLU (PAIR: the matrix tile's sixteen rows are eight gate rows and the eight up rows
 // that meet them, so that there are as many workgroups as without).  What
 // bounds it at few tokens is latency (a launch, one round of loads, 0.9 us of matrix instructions), not the matrix: us at 2 tokens, matrices out of
-// memory, 1024 x 1024 4.8, SwiGLU of 2816 x 1024 6.4; 32000 x 1024 29 (4.5 TB/s).  At 250 tokens 1024 x 1024 10.8, 2048 x 2048 34.2.  With both operands loaded
-// in the operands' order (a cycle a lane, quad_rows.h) they were 5.0, 6.7, 33.6, 14.5 and 50.5.
-constexpr int F32_WAVES = 8;
+// memory, 1024 x 1024 4.5, SwiGLU of 2816 x 1024 5.4; 32000 x 1024 25 (5.2 TB/s).  At 250 tokens 1024 x 1024 10.3, 2048 x 2048 31.5.  With both operands loaded
+// in the operands' order (a cycle a lane, quad_rows.h) and a condition of the lanes' at every load they were 5.3, 5.9, 31.5, 14.9 and 49.3; with the first of the two mended 5.1, 6.1, 26.9, 11.4 and
+// 34.1 (and longer than before it where K is no multiple of 64: 4096 x 1000 at 1 row 5.7, 6.4, now 5.7).  Rows that begin between lines and are short remain: 512 x 272 2.9, now 3.1.
+constexpr int F32_WAVES = 8, COMPUTE_UNITS = 256;
 
 struct F32Extra {
     int accumulate;
@@ -613,14 +615,14 @@ struct F32Extra {
 
 // Both operands come in by quads of lanes (quad_rows.h, four k where bfloat16 has eight): W's load i brings lane (g, a, b) row 4 a + i, so that
 // the operands' rows are in order, X's row 4 i + a, so that few rows take fewer loads; operand j then holds k = 64 s + 16 g + 4 j .. of its row.
-// PAIR: SwiGLU; SCALED: with sumsq_in; ADDS: accumulate or norm_w
-template <int MT, bool PAIR, bool SCALED, bool ADDS, int LOADS>
-__global__ void __launch_bounds__(F32_WAVES *WAVE, MT == 1 && !(ADDS && LOADS == 4) ? 4 : 2)      // (two workgroups of sixteen rows a compute unit: 32000 x 1024 at 16 rows 41 us, with one 46)
+// PAIR: SwiGLU; SCALED: with sumsq_in; ADDS: accumulate or norm_w; TWO: sixteen rows in 128 registers, for grids of more workgroups than compute units
+template <int MT, bool PAIR, bool SCALED, bool ADDS, int LOADS, bool TWO = false>
+__global__ void __launch_bounds__(F32_WAVES *WAVE, MT == 1 && (LOADS < 4 || TWO) ? 4 : 2)      // (up to eight rows, or TWO: two workgroups a compute unit)
 gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W, int ldw, float *__restrict__ Y,
                        int ldy, int M, int N, int K, F32Extra ex) {
     __shared__ f32x4 red[F32_WAVES][MT][WAVE];
     __shared__ float factor[16 * MT];
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int l16 = lane & 15, grp = lane >> 4, col = quad_row(l16);      // (the token of the tile that the lane's column is)
     const int n0 = blockIdx.x * (PAIR ? 8 : 16), m0 = blockIdx.y * 16 * MT;
     // (a row beyond the end is read, not stored)
@@ -653,61 +655,95 @@ gemm_skinny_f32_kernel(const float *__restrict__ X, int ldx, const float *__rest
             }
         }
     }
-    // macro-steps whose loads are on their way: of the matrix two, of up to eight rows two, of more rows a tile's next when it is used
+    // macro-steps whose loads are on their way: of the matrix two, of up to eight rows two, of more rows a tile's next when it is used.  Every load is issued under
+    // no condition of a lane's, with a place that exists, and what lies beyond K is taken out when it is used: with the condition at the load the ring's
+    // waits were for everything on its way
     constexpr int ROWS_AHEAD = LOADS < 4 ? 2 : 1, AHEAD = 2;
     quad_u32x4 w[AHEAD][4], x[ROWS_AHEAD][MT][LOADS];
-    const quad_u32x4 zero = quad_u32x4{0u, 0u, 0u, 0u};
     const int k_lane = 16 * grp + 4 * (lane & 3);            // (K is a multiple of 4)
     auto load_w = [&](int u, int s) {
-        const bool in = 64 * s + k_lane + 4 <= K;
+        const int k = min(64 * s + k_lane, K - 4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[u][i] = in ? *(const quad_u32x4 *)(wrow[i] + 64 * s + k_lane) : zero;
+        for (int i = 0; i < 4; ++i) w[u][i] = *(const quad_u32x4 *)(wrow[i] + k);
     };
     auto load_x = [&](int u, int m, int s) {
-        const bool in = 64 * s + k_lane + 4 <= K;
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i)
-            x[u][m][i] = in ? __builtin_bit_cast(quad_u32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, x_place + (4 * m + i) * x_four + 256u * s, 0, 0)) : zero;
+        for (int i = 0; i < LOADS; ++i) x[u][m][i] = __builtin_bit_cast(quad_u32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, x_place + (4 * m + i) * x_four + 256u * s, 0, 0));
     };
-    int s = wave;
+    auto load_rows = [&](int u, int s) {
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u)
-        if (s + u * F32_WAVES < nsteps) load_w(u, s + u * F32_WAVES);
+        for (int m = 0; m < MT; ++m) load_x(u, m, s);
+    };
+    // operand j: k = 64 s + 16 grp + 4 j ..
+    auto within_k = [&](quad_u32x4 (&v)[4], int s) {
+        if (64 * s + 64 <= K) return;
+        asm volatile("");                                    // (a branch, no selection where there is nothing to take out)
 #pragma unroll
-    for (int u = 0; u < ROWS_AHEAD; ++u)
-        if (s + u * F32_WAVES < nsteps) {
+        for (int j = 0; j < 4; ++j) v[j] = 64 * s + 16 * grp + 4 * j + 4 <= K ? v[j] : quad_u32x4{0u, 0u, 0u, 0u};
+    };
+    // macro-step s out of w[U]; MORE_W, MORE_X: the loads that take its registers are asked for
+    auto step = [&](auto U, int s, auto MORE_W, auto MORE_X) {
+        constexpr int u = decltype(U)::value, ux = u % ROWS_AHEAD;
+        quad_u32x4 wt[4];
+        quad_operands<4, TWO>(w[u], wt);
+        within_k(wt, s);
+        if constexpr (decltype(MORE_W)::value) load_w(u, s + AHEAD * F32_WAVES);
 #pragma unroll
-            for (int m = 0; m < MT; ++m) load_x(u, m, s + u * F32_WAVES);
+        for (int m = 0; m < MT; ++m) {
+            quad_u32x4 xt[4];
+            quad_operands<LOADS, TWO>(x[ux][m], xt);
+            within_k(xt, s);
+            if constexpr (decltype(MORE_X)::value) load_x(ux, m, s + ROWS_AHEAD * F32_WAVES);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(wt[j][e]), __uint_as_float(xt[j][e]), acc[m], 0, 0, 0);
         }
-    if constexpr (SCALED) {
-        for (int r = wave; r < 16 * MT && m0 + r < M; r += F32_WAVES) {
-            float t = 0.f;
-            for (int i = lane; i < ex.n_in; i += WAVE) t += ex.sumsq_in[(size_t)(m0 + r) * ex.n_in + i];
-            t = wave_sum_in_place(t);
-            if (lane == 0) factor[r] = rsqrtf(t / (float)ex.norm_width + ex.eps);
-        }
-    }
-    for (; s < nsteps; s += AHEAD * F32_WAVES) {
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-            const int cur = s + u * F32_WAVES;
-            if (cur >= nsteps) break;
-            quad_u32x4 wt[4];
-            quad_operands<4>(w[u], wt);
-            if (cur + AHEAD * F32_WAVES < nsteps) load_w(u, cur + AHEAD * F32_WAVES);
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                quad_u32x4 xt[4];
-                quad_operands<LOADS>(x[u % ROWS_AHEAD][m], xt);
-                if (cur + ROWS_AHEAD * F32_WAVES < nsteps) load_x(u % ROWS_AHEAD, m, cur + ROWS_AHEAD * F32_WAVES);
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(wt[j][e]), __uint_as_float(xt[j][e]), acc[m], 0, 0, 0);
+    };
+    auto factors = [&]() {
+        if constexpr (SCALED) {
+            for (int r = wave; r < 16 * MT && m0 + r < M; r += F32_WAVES) {
+                float t = 0.f;
+                for (int i = lane; i < ex.n_in; i += WAVE) t += ex.sumsq_in[(size_t)(m0 + r) * ex.n_in + i];
+                t = wave_sum_in_place(t);
+                if (lane == 0) factor[r] = rsqrtf(t / (float)ex.norm_width + ex.eps);
             }
         }
+    };
+    constexpr std::integral_constant<int, 0> at0;
+    constexpr std::integral_constant<int, 1> at1;
+    constexpr std::true_type more;
+    constexpr std::false_type last;
+    constexpr std::bool_constant<ROWS_AHEAD == 1> rows_more;
+    int s = wave, left = (nsteps - wave + F32_WAVES - 1) / F32_WAVES;      // the wave's macro-steps
+    if (left >= 2) {
+        load_w(0, s);
+        load_rows(0, s);
+        load_w(1, s + F32_WAVES);
+        if constexpr (ROWS_AHEAD == 2) load_rows(1, s + F32_WAVES);
+        factors();
+        for (; left >= 4; left -= 2, s += 2 * F32_WAVES) {
+            step(at0, s, more, more);
+            step(at1, s + F32_WAVES, more, more);
+        }
+        if (left == 3) {
+            step(at0, s, more, more);
+            step(at1, s + F32_WAVES, last, rows_more);
+            step(at0, s + 2 * F32_WAVES, last, last);
+        } else {
+            step(at0, s, last, rows_more);
+            step(at1, s + F32_WAVES, last, last);
+        }
+    } else {
+        if (left > 0) {
+            load_w(0, s);
+            load_rows(0, s);
+        }
+        factors();
+        if (left > 0) step(at0, s, last, last);
     }
+    asm volatile("s_nop 3" : "+v"(acc[MT - 1]));             // the last matrix instruction's wait, which the compiler leaves a state short behind the branches
 #pragma unroll
     for (int m = 0; m < MT; ++m) red[wave][m][lane] = acc[m];
     __syncthreads();
@@ -768,13 +804,17 @@ LCU_API int lcu_gemm_skinny_f32(const float *X, int ldx, const float *W, int ldw
     const dim3 grid(swiglu ? (N + 7) / 8 : (N + 15) / 16, tiles), block(F32_WAVES * WAVE);
     // What a product does besides is known when it is compiled: a form that looks at F32Extra for it, behind the loads that are on their way, took
     // 4.9 us for two rows of 1024 x 1024 with the matrix in the caches and 2.5 for 64 x 64, now 4.6 and 2.3.
-#define GO(MT, PAIR, SCALED, ADDS, LOADS) gemm_skinny_f32_kernel<MT, PAIR, SCALED, ADDS, LOADS><<<grid, block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, ex)
-#define ROWS(MT, PAIR, ADDS, LOADS) do { if (sumsq_in) GO(MT, PAIR, true, ADDS, LOADS); else GO(MT, PAIR, false, ADDS, LOADS); } while (0)
-#define FORMS(MT, LOADS) do { if (swiglu) ROWS(MT, true, false, LOADS); else if (accumulate || norm_w) ROWS(MT, false, true, LOADS); else ROWS(MT, false, false, LOADS); } while (0)
-    if (rows > 16) FORMS(4, 4);
-    else if (M <= 4) FORMS(1, 1);
-    else if (M <= 8) FORMS(1, 2);
-    else FORMS(1, 4);
+#define GO(MT, PAIR, SCALED, ADDS, LOADS, TWO) gemm_skinny_f32_kernel<MT, PAIR, SCALED, ADDS, LOADS, TWO><<<grid, block, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, ex)
+#define ROWS(MT, PAIR, ADDS, LOADS, TWO) do { if (sumsq_in) GO(MT, PAIR, true, ADDS, LOADS, TWO); else GO(MT, PAIR, false, ADDS, LOADS, TWO); } while (0)
+#define FORMS(MT, LOADS, TWO) do { if (swiglu) ROWS(MT, true, false, LOADS, TWO); else if (accumulate || norm_w) ROWS(MT, false, true, LOADS, false); else ROWS(MT, false, false, LOADS, TWO); } while (0)
+    // Two workgroups a compute unit where there are more than compute units; registers to spare where not.  us, two and one: 32000 x 1024 at 9 / 16 / 32 rows 28.7, 30.5, 51.3 and 34.8, 36.3, 61.4,
+    // 520 x 272 at 128 (264 workgroups) 4.8 and 5.7; 1024 x 1024 at 9 / 16 (64) 5.7, 5.8 and 5.2, 5.2.  (What it adds to leaves no registers for it.)
+    const bool two = (long long)grid.x * grid.y > COMPUTE_UNITS;
+    if (rows > 16) FORMS(4, 4, false);
+    else if (M <= 4) FORMS(1, 1, false);
+    else if (M <= 8) FORMS(1, 2, false);
+    else if (two) FORMS(1, 4, true);
+    else FORMS(1, 4, false);
 #undef FORMS
 #undef ROWS
 #undef GO

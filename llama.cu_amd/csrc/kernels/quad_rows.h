@@ -67,6 +67,27 @@ __device__ __forceinline__ void quad_transpose(const quad_u32x4 (&r)[4], quad_u3
     x[2] = quad_u32x4{o[0], o[1], o[2], o[3]};
     x[3] = quad_u32x4{p[0], p[1], p[2], p[3]};
 }
+// the same in two halves, so that the second one's results may have the first one's operands' registers: 16 fewer, a wait more
+__device__ __forceinline__ void quad_transpose_in_less(const quad_u32x4 (&r)[4], quad_u32x4 (&x)[4]) {
+    uint32_t e[4], f[4], g[4], h[4], m[4], n[4], o[4], p[4];
+    asm("s_nop 1\n\t"
+        "s_mov_b64 vcc, %[k1]\n\t" QUAD_TAKE(e, b, a, QUAD_1) QUAD_TAKE(g, d, c, QUAD_1)
+        "s_not_b64 vcc, vcc\n\t" QUAD_TAKE(f, a, b, QUAD_1) QUAD_TAKE(h, c, d, QUAD_1)
+        : QUAD_REGS("=&v", e, e), QUAD_REGS("=&v", f, f), QUAD_REGS("=&v", g, g), QUAD_REGS("=&v", h, h)
+        : QUAD_REGS("v", a, r[0]), QUAD_REGS("v", b, r[1]), QUAD_REGS("v", c, r[2]), QUAD_REGS("v", d, r[3]), [k1] "s"(QUAD_KEEP_1)
+        : "vcc", "scc");
+    asm("s_nop 1\n\t"
+        "s_mov_b64 vcc, %[k2]\n\t" QUAD_TAKE(m, g, e, QUAD_2) QUAD_TAKE(n, h, f, QUAD_2)
+        "s_not_b64 vcc, vcc\n\t" QUAD_TAKE(o, e, g, QUAD_2) QUAD_TAKE(p, f, h, QUAD_2)
+        "s_nop 1"
+        : QUAD_REGS("=&v", m, m), QUAD_REGS("=&v", n, n), QUAD_REGS("=&v", o, o), QUAD_REGS("=&v", p, p)
+        : QUAD_REGS("v", e, e), QUAD_REGS("v", f, f), QUAD_REGS("v", g, g), QUAD_REGS("v", h, h), [k2] "s"(QUAD_KEEP_2)
+        : "vcc", "scc");
+    x[0] = quad_u32x4{m[0], m[1], m[2], m[3]};
+    x[1] = quad_u32x4{n[0], n[1], n[2], n[3]};
+    x[2] = quad_u32x4{o[0], o[1], o[2], o[3]};
+    x[3] = quad_u32x4{p[0], p[1], p[2], p[3]};
+}
 #undef QUAD_1
 #undef QUAD_2
 #undef QUAD_TAKE
@@ -82,8 +103,8 @@ __device__ __forceinline__ quad_u32x4 quad_perm(const quad_u32x4 &v) {
     return o;
 }
 
-// r: what the loads brought; x: the operands
-template <int LOADS>
+// r: what the loads brought; x: the operands; LESS: in fewer registers
+template <int LOADS, bool LESS = false>
 __device__ __forceinline__ void quad_operands(const quad_u32x4 (&r)[LOADS], quad_u32x4 (&x)[4]) {
     static_assert(LOADS == 1 || LOADS == 2 || LOADS == 4, "rows in fours");
     if constexpr (LOADS == 1) {
@@ -95,6 +116,8 @@ __device__ __forceinline__ void quad_operands(const quad_u32x4 (&r)[LOADS], quad
         quad_swap(r[0], r[1], x[0], x[1]);
         x[2] = quad_perm<0x4E>(x[0]);
         x[3] = quad_perm<0x4E>(x[1]);
+    } else if constexpr (LESS) {
+        quad_transpose_in_less(r, x);
     } else {
         quad_transpose(r, x);
     }

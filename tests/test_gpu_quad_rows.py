@@ -2,6 +2,8 @@
 whose products and sums are whole numbers below 2^24: every result is the exact one or a row or a k is in the wrong place."""
 from __future__ import annotations
 
+import math
+
 import pytest
 import torch
 
@@ -153,3 +155,26 @@ def test_products_on_both_sides_of_a_line(m, n, k):
     x, w = whole((m, k), 22), whole((n, k), 23)
     got = linear(rows_of(x, m % 2), Weight(w.to(BF16).cuda()))
     assert torch.equal(got.double().cpu(), (x @ w.t()).to(BF16).double())
+
+
+@pytest.mark.parametrize("m", [3, 7, 16, 70])
+@pytest.mark.parametrize("k", [4, 272, 512, 1000, 1536, 1796, 2564])
+def test_macro_steps_of_a_wave_in_32_bits(m, k):
+    """None to six macro-steps of 64 a wave, the last one whole and not; a grid of fewer and of more workgroups than compute units; NaN behind the rows' ends, infinity in the
+    matrix' last column.  Whole numbers: the sums are exact."""
+    from llama_cu_amd.kernels import ops
+    for n in (40, 4112):
+        x, w = whole((m, k), 24), whole((n, k), 25)
+        wide = torch.full((m, k + 20), float("nan"), device="cuda")
+        wide[:, 4:4 + k] = x.float().cuda()
+        rows = torch.full((n, k + 20), float("nan"), device="cuda")
+        rows[:, 8:8 + k] = w.float().cuda()
+        want, add = x @ w.t(), whole((m, n), 26).float().cuda()
+        assert torch.equal(ops.gemm_skinny_f32(wide[:, 4:4 + k], rows[:, 8:8 + k]).double().cpu(), want)
+        got = ops.gemm_skinny_f32(wide[:, 4:4 + k], rows[:, 8:8 + k], out=add.clone(), accumulate=True)
+        assert torch.equal(got.double().cpu(), want + add.double().cpu())
+        rows[5, 8 + k - 1] = float("inf")                    # a row of its own: no other feature sees it, and of its sums those whose token is not zero there are infinite
+        got = ops.gemm_skinny_f32(wide[:, 4:4 + k], rows[:, 8:8 + k]).double().cpu()
+        last = x[:, -1]
+        assert torch.equal(got[:, :5], want[:, :5]) and torch.equal(got[:, 6:], want[:, 6:])
+        assert torch.equal(torch.isnan(got[:, 5]), last == 0) and torch.equal(got[last != 0, 5], last[last != 0] * math.inf)
