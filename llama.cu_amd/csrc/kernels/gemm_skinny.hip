@@ -395,14 +395,19 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
     }
 }
 
-// (plain rows of W take their time whatever the rows of X do; a last tile of few rows takes fewer loads where it is the only tile or where that leaves registers for a second stage)
+// (a last tile of few rows takes fewer loads where it is the only tile or where that leaves registers for a second stage.  Plain matrices, us at 1, 4 and 8 rows with that and with
+// four loads: 2048 x 2048 4.7, 4.7, 4.9 and 5.3, 5.3, 5.4, 14336 x 4096 24.4, 24.5, 26.2 and 27.5, 27.7, 28.8)
 #define RUN(E, GRID, BLOCK)                                                            \
     do {                                                                               \
-        if (!packed) RUN_AS(E, GRID, BLOCK, false, 4);                                 \
-        else if constexpr (MT > 1 && !(NT * MT == 8 && WAVES == 8)) RUN_AS(E, GRID, BLOCK, true, 4); \
-        else if (M - 16 * (MT - 1) <= 4) RUN_AS(E, GRID, BLOCK, true, 1);              \
-        else if (M - 16 * (MT - 1) <= 8) RUN_AS(E, GRID, BLOCK, true, 2);              \
-        else RUN_AS(E, GRID, BLOCK, true, 4);                                          \
+        if (packed) RUN_LOADS(E, GRID, BLOCK, true, MT == 1 || (NT * MT == 8 && WAVES == 8)); \
+        else RUN_LOADS(E, GRID, BLOCK, false, MT == 1);                                \
+    } while (0)
+#define RUN_LOADS(E, GRID, BLOCK, PACKED, FEW)                                         \
+    do {                                                                               \
+        if constexpr (!(FEW)) RUN_AS(E, GRID, BLOCK, PACKED, 4);                       \
+        else if (M - 16 * (MT - 1) <= 4) RUN_AS(E, GRID, BLOCK, PACKED, 1);            \
+        else if (M - 16 * (MT - 1) <= 8) RUN_AS(E, GRID, BLOCK, PACKED, 2);            \
+        else RUN_AS(E, GRID, BLOCK, PACKED, 4);                                        \
     } while (0)
 #define RUN_AS(E, GRID, BLOCK, PACKED, LOADS)                                                                                \
     gemm_skinny_kernel<NT, MT, E, WAVES, PACKED, LOADS><<<GRID, BLOCK, 0, stream>>>((const bf16_t *)X, ldx, (const bf16_t *)W, ldw, Y, ldy, M, N, K, ex)
@@ -449,6 +454,7 @@ static int launch_swiglu(const void *X, int ldx, const void *W, int ldw, void *Y
     return LCU_OK;
 }
 #undef RUN
+#undef RUN_LOADS
 
 // X: [M, K] bfloat16 rows ldx apart; W: [N, K] bfloat16 rows ldw apart; Y: [M, N] rows ldy
 // apart (for the SwiGLU epilogue [M, N/2]: W holds N/2 gate rows, then N/2 up rows).
