@@ -42,37 +42,54 @@ delta_prep_kernel(const T *__restrict__ proj, int row_stride, int off_r, int off
                   const float *__restrict__ a_bias, float *__restrict__ prep, int n, int heads, int dk, int rank) {
     extern __shared__ __attribute__((aligned(16))) float th[];         // [rank][TB]
     __shared__ float part[4][TB][WAVE], inv[TB];
-    const int t0 = blockIdx.x * TB, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t0 = blockIdx.x * TB, h = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nt = min(TB, n - t0), i = blockIdx.z * WAVE + lane, c = h * dk + min(i, dk - 1);
-    // What does not wait for the others is asked for first: the wave's own tokens' values and the first of its quarter of w2t (one MI355X, 2,014 tokens of 16
-    // heads of 128, rank 64: 40 us, 48 with every load where its value is used)
-    constexpr int OWN = (TB + 3) / 4, FIRST = 16;
+    // EARLY: what does not wait for the others is asked for first, the wave's own tokens' values and the first of its quarter of w2t (one MI355X, 2,014 tokens of 16
+    // heads of 128, rank 64: 40 us, 48 with every load where its value is used).  One token's four waves would ask for the same rows (16 tokens of 16 heads of 128, the whole rule: 10.9 us, 10.7 so)
+    constexpr bool EARLY = TB > 1;
+    constexpr int OWN = (TB + 3) / 4, FIRST = 16, SIDE = TB > 1 ? 4 : 1;
     const int quarter = (rank + 3) / 4, j0 = wave * quarter, j1 = min(rank, j0 + quarter);
     const float *w = w2t + c;                                 // (neighbouring lanes, neighbouring addresses)
     float kv[OWN], av[OWN], rv[OWN], ka[OWN], kb[OWN], wv[FIRST];
+    if constexpr (EARLY) {
 #pragma unroll
-    for (int o = 0; o < OWN; ++o) {
-        const T *row = proj + (size_t)(t0 + min(wave + 4 * o, nt - 1)) * row_stride, *k = row + off_k + h * dk;
-        ka[o] = to_f32(k[min(lane, dk - 1)]);
-        kb[o] = to_f32(k[min(lane + WAVE, dk - 1)]);
-        kv[o] = to_f32(row[off_k + c]);
-        av[o] = to_f32(row[off_a + c]);
-        rv[o] = to_f32(row[off_r + c]);
+        for (int o = 0; o < OWN; ++o) {
+            const T *row = proj + (size_t)(t0 + min(wave + 4 * o, nt - 1)) * row_stride, *k = row + off_k + h * dk;
+            ka[o] = to_f32(k[min(lane, dk - 1)]);
+            kb[o] = to_f32(k[min(lane + WAVE, dk - 1)]);
+            kv[o] = to_f32(row[off_k + c]);
+            av[o] = to_f32(row[off_a + c]);
+            rv[o] = to_f32(row[off_r + c]);
+        }
+#pragma unroll
+        for (int x = 0; x < FIRST; ++x) wv[x] = w[(size_t)max(min(j0 + x, j1 - 1), 0) * heads * dk];
     }
+    // (the projection's values by fours: one after the other a rank of 256 is eight trips to memory.  With w2t by sixteens, the next behind them, the whole rule of 2,000 tokens and 16 heads
+    // of 64 with 16 value columns, bfloat16, rank 64, 256 and 400: 124, 145 and 166 us; the compiler's eight at a time 124, 166 and 202)
+    for (int x0 = threadIdx.x; x0 < rank * TB; x0 += 256 * SIDE) {
+        float l[SIDE];
 #pragma unroll
-    for (int x = 0; x < FIRST; ++x) wv[x] = w[(size_t)max(min(j0 + x, j1 - 1), 0) * heads * dk];
-    for (int x = threadIdx.x; x < rank * TB; x += 256) {
-        const int t = x / rank, j = x % rank;
-        th[j * TB + t] = t < nt ? tanhf(to_f32(proj[(size_t)(t0 + t) * row_stride + off_l + j])) : 0.f;
+        for (int b = 0; b < SIDE; ++b) {
+            const int x = min(x0 + 256 * b, rank * TB - 1);
+            l[b] = to_f32(proj[(size_t)(t0 + min(x / rank, nt - 1)) * row_stride + off_l + x % rank]);
+        }
+#pragma unroll
+        for (int b = 0; b < SIDE; ++b) {
+            const int x = x0 + 256 * b, t = x / rank;
+            if (x < rank * TB) th[x % rank * TB + t] = t < nt ? tanhf(l[b]) : 0.f;
+        }
     }
 #pragma unroll
     for (int o = 0; o < OWN; ++o) {
         const int t = wave + 4 * o;
         if (t >= nt) break;
         const T *row = proj + (size_t)(t0 + t) * row_stride + off_k + h * dk;
-        float ss = lane < dk ? ka[o] * ka[o] : 0.f;
-        if (lane + WAVE < dk) ss = fmaf(kb[o], kb[o], ss);
-        for (int x = lane + 2 * WAVE; x < dk; x += WAVE) {
+        float ss = 0.f;
+        if constexpr (EARLY) {
+            ss = lane < dk ? ka[o] * ka[o] : 0.f;
+            if (lane + WAVE < dk) ss = fmaf(kb[o], kb[o], ss);
+        }
+        for (int x = lane + (EARLY ? 2 * WAVE : 0); x < dk; x += WAVE) {
             const float kk = to_f32(row[x]);
             ss = fmaf(kk, kk, ss);
         }
@@ -83,17 +100,36 @@ delta_prep_kernel(const T *__restrict__ proj, int row_stride, int off_r, int off
     float z[TB];
 #pragma unroll
     for (int t = 0; t < TB; ++t) z[t] = 0.f;
+    if constexpr (EARLY) {
+        // sixteen at a time, the next on their way meanwhile
+        for (int j = j0; j < j1; j += FIRST) {
+            float next[FIRST];
+            if (j + FIRST < j1) {
 #pragma unroll
-    for (int x = 0; x < FIRST; ++x) {
-        if (j0 + x >= j1) break;
+                for (int x = 0; x < FIRST; ++x) next[x] = w[(size_t)min(j + FIRST + x, j1 - 1) * heads * dk];
+            }
+            auto add = [&](int x) {
 #pragma unroll
-        for (int t = 0; t < TB; ++t) z[t] = fmaf(wv[x], th[(j0 + x) * TB + t], z[t]);
-    }
+                for (int t = 0; t < TB; ++t) z[t] = fmaf(wv[x], th[(j + x) * TB + t], z[t]);
+            };
+            if (j + FIRST <= j1) {
+#pragma unroll
+                for (int x = 0; x < FIRST; ++x) add(x);
+            } else {
+#pragma unroll
+                for (int x = 0; x < FIRST; ++x)
+                    if (j + x < j1) add(x);
+            }
+#pragma unroll
+            for (int x = 0; x < FIRST; ++x) wv[x] = next[x];
+        }
+    } else {
 #pragma unroll 8
-    for (int j = j0 + FIRST; j < j1; ++j) {
-        const float v = w[(size_t)j * heads * dk];
+        for (int j = j0; j < j1; ++j) {
+            const float v = w[(size_t)j * heads * dk];
 #pragma unroll
-        for (int t = 0; t < TB; ++t) z[t] = fmaf(v, th[j * TB + t], z[t]);
+            for (int t = 0; t < TB; ++t) z[t] = fmaf(v, th[j * TB + t], z[t]);
+        }
     }
 #pragma unroll
     for (int t = 0; t < TB; ++t) part[wave][t][lane] = z[t];
@@ -104,6 +140,12 @@ delta_prep_kernel(const T *__restrict__ proj, int row_stride, int off_r, int off
         const int t = wave + 4 * o;
         if (t >= nt) break;
         const float sum = (part[0][t][lane] + part[1][t][lane]) + (part[2][t][lane] + part[3][t][lane]);
+        if constexpr (!EARLY) {
+            const T *row = proj + (size_t)(t0 + t) * row_stride;
+            kv[o] = to_f32(row[off_k + c]);
+            av[o] = to_f32(row[off_a + c]);
+            rv[o] = to_f32(row[off_r + c]);
+        }
         const float u = kv[o] * inv[t];
         float *out = prep + ((size_t)(t0 + t) * heads + h) * 5 * dk;
         out[i] = expf(-DECAY_SCALE * sigmoidf_(w0[c] + sum));
