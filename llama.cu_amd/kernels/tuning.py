@@ -88,7 +88,9 @@ class Tuning:
     wavek_library_k: int = 2688         # 14.0; 1280 x 2816 9.9 against 9.6; 1024 x 2816 9.7 against 11.2, 2048 x 2688 9.7 against 13.6, 4352 x 4096 15.9 against 16.9)
     wavek_swiglu_least: int = 512       # gate and up rows and K from which on SwiGLU was measured (1024 x 512 to 8192 x 4096: the library's product alone, without
                                         # the activation kernel's 2 us, is 1 us faster at most, at 48 rows of 2816 x 3072; the row-sharing kernel 1.5 us slower at 64 rows and 0.9
-                                        # faster at 24 to 32 rows of 8192, which go to it: mid_swiglu_features)
+                                        # faster at 24 to 32 rows of 8192, which go to it: mid_swiglu_features).  With that kernel, matrices out of memory, at 33, 48, 49 and 63 rows: 2048 x 3072 11.3,
+                                        # 11.5, 12.4, 12.5 us against the library's 12.7, 12.6, 12.6, 12.8, 1536 x 4096 13.1, 13.4, 14.6, 15.1 against 14.5 (out of the last-level cache the
+                                        # library's are 10.2 and 11.4)
     wavek_qkv_rows: int = 32            # q/k/v with the rotation and the cache write in its epilogue goes to it above so many rows and up to 64, where the row-sharing
                                         # kernel would be taken, whatever K (us at 33, 48 and 64 rows, 48 heads of 128, K = 4096: 17.8, 18.3, 19.5 against 19.0, 19.2, 21.2, K = 8192:
                                         # 28.2, 30.2, 32.0 against 32.6, 31.0, 35.1; 24 heads, K = 512: 6.1, 6.4, 7.2 against 6.2, 6.3, 7.5, K = 2048: 10.5, 10.9, 12.3
