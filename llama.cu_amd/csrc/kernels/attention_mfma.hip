@@ -16,8 +16,8 @@
 // the heads of a group for one token, for several tokens if the group is small.
 //
 //   decode kernel   one token per request, v_mfma_f32_16x16x32_bf16 (blocks of 16 rows; a lane
-//                   owns row lane % 16 and 8 of each 32 keys, 4 of each tile of 16, which are
-//                   neighbours in memory).  A workgroup of 4 waves takes one request and
+//                   owns row lane % 16 and 8 of each 32 keys, neighbours in memory).  A
+//                   workgroup of 8 waves (4 with sixteen rows) takes one request and
 //                   key/value head and one of `n_splits` equal parts of its keys; the
 //                   waves take 32-key steps in turn and merge through LDS; parts are
 //                   merged by a second kernel.
@@ -130,76 +130,55 @@ __device__ __forceinline__ void attn_init(AttnState<DH, QB> &st) {
     }
 }
 
-// The lane's share of the keys and values of one step: the 32 keys k0 .. k0+31 (k0 a
-// multiple of 32) of key/value head kvh, as two tiles of 16 keys.
+// The lane's share of the keys and values of one step: the 32 keys k0 .. k0+31 (k0 a multiple of 32) of key/value head kvh, as two tiles
+// of 16 keys.  Of the values a lane has eight neighbouring keys of one tile, a load of 16 bytes; the weights come to them between the
+// products (attn_softmax).  (As four neighbours of each tile, where the scores leave the weights, they were loads of 8 bytes, which a compute
+// unit takes a lane at a time.  One MI355X, us, of that and of this: 8 requests of 512 keys, 16 heads of 128 over 4, 8.9 and 8.1, of 1,024 14.9 and 13.3; 1 request of 2,000
+// 24.4 and 21.3; 64 requests of 150 to 1,500, 32 heads over 8, 37.0 and 36.5.  In the first product's order, too, the halves of a line would be two
+// loads, and non-temporal ones fetch the line twice: 9.5 instead of 8.1.)
 template <int DH>
 struct KVFrag {
     u32x4 k[2][DH / 32];    // tile t, dims 32*kb + 8*grp .. + 7 of key 16*t + lane%16
-    u32x2 v[DH / 16][2];    // dim 16*dt + lane%16, keys 16*t + 4*grp .. + 3
+    u32x4 v[DH / 16];       // dim 16*dt + lane%16, keys mix_key(grp) .. + 7
 };
+// the first of the lane's eight keys in the second product
+__device__ __forceinline__ int mix_key(int grp) { return 16 * (grp & 1) + 8 * (grp >> 1); }
+
+// The two pages that hold the keys k0 .. k0+15 and k0+16 .. k0+31 and the places of these in them, asked for a step before the loads that want them.
+// (Pages of 16 tokens need no division, which would stand between a workgroup's start and its first load: 0.4 us.)
+struct KVPages {
+    int page[2], tok[2];
+};
+__device__ __forceinline__ KVPages kv_pages(const int *__restrict__ bt, int max_pages, int page, int k0) {
+    KVPages at;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        int i = (k0 + 16 * t) / 16;
+        at.tok[t] = 0;
+        if (page != 16) {
+            const int tile = i, tiles = page / 16;
+            i = tile / tiles;
+            at.tok[t] = 16 * (tile - i * tiles);
+        }
+        at.page[t] = bt[min(i, max_pages - 1)];       // a tile beyond the context is masked; keep the read in bounds
+    }
+    return at;
+}
 
 // The decode kernel reads a request's keys and values once a step: its loads are non-temporal (see gemm_skinny.hip's
 // stream_load), so that they do not displace the weights' neighbours and the rows in the caches.
-constexpr int DEC_STREAM = 2;
-
-// The numbers of the two pages that hold the keys k0 .. k0+15 and k0+16 .. k0+31 (where k0 is a scalar, the table is read through the
-// scalar unit).
-__device__ __forceinline__ void kv_pages(int (&pid)[2], const int *__restrict__ bt, int max_pages, int page, int k0) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        int pi = (k0 + 16 * t) / page;
-        pi = pi < max_pages ? pi : max_pages - 1;       // a tile beyond the context is masked; keep the read in bounds
-        pid[t] = bt[pi];
-    }
-}
-
-// The loads are buffer loads whose buffer is the page: page, head, token and slice of dims
-// make a scalar offset, and the lane adds one offset for the keys and one for the values that
-// are the same in every step, so no addresses are held in vector registers.  pid: kv_pages of
-// k0, read a step earlier so that no load waits for the table.  A page holds less than 2 GiB
-// (the host checks).
 template <int DH>
-__device__ __forceinline__ void load_kv(KVFrag<DH> &f, const bf16_t *__restrict__ cache, const int (&pid)[2], int page,
-                                        size_t page_elems, int nkvh, int kvh, int k0, int l16, int grp) {
-    constexpr uint32_t E = sizeof(bf16_t);
-    const uint32_t k_lane = ((uint32_t)grp * page + l16) * 8 * E;       // keys: [dim/8][token][8]
-    const uint32_t v_lane = ((uint32_t)l16 * page + 4 * grp) * E;       // values: [dim][token]
-    const uint32_t k_head = (uint32_t)kvh * (DH / 8) * page * 8 * E;
-    const uint32_t v_head = (uint32_t)(nkvh + kvh) * DH * page * E;
+__device__ __forceinline__ void load_kv(KVFrag<DH> &f, const bf16_t *__restrict__ cache, const KVPages &at, int page, size_t page_elems, int nkvh, int kvh, int l16, int grp) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const __amdgpu_buffer_rsrc_t pg = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<bf16_t *>(cache + (size_t)pid[t] * page_elems), 0, (uint32_t)(page_elems * E), 0x00020000);
-        // the token's place in the page goes into the lane's offset (one addition for the keys, one for
-        // the values), so that the scalar offsets are the same in every step
-        const uint32_t tok0 = (k0 + 16 * t) % page;
-        const uint32_t k_off = k_lane + tok0 * 8 * E, v_off = v_lane + tok0 * E;
+        const bf16_t *kp = cache + (size_t)at.page[t] * page_elems + ((size_t)(kvh * (DH / 8) + grp) * page + at.tok[t] + l16) * 8;
 #pragma unroll
-        for (int kb = 0; kb < DH / 32; ++kb)
-            f.k[t][kb] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(pg, k_off, k_head + (uint32_t)(4 * kb) * page * 8 * E, DEC_STREAM));
-#pragma unroll
-        for (int dt = 0; dt < DH / 16; ++dt)
-            f.v[dt][t] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(pg, v_off, v_head + (uint32_t)(16 * dt) * page * E, DEC_STREAM));
+        for (int kb = 0; kb < DH / 32; ++kb) f.k[t][kb] = __builtin_nontemporal_load((const u32x4 *)(kp + (size_t)4 * kb * page * 8));
     }
-}
-
-// The same loads with a full address in every lane (pid: the two pages, read by the lanes too).
-template <int DH>
-__device__ __forceinline__ void load_kv_flat(KVFrag<DH> &f, const bf16_t *__restrict__ cache, const int (&pid)[2], int page, size_t page_elems, int nkvh, int kvh, int k0, int l16,
-                                             int grp) {
-    const size_t v_off = (size_t)nkvh * DH * page + (size_t)kvh * DH * page + 4 * grp;
+    const int key = mix_key(grp);
+    const bf16_t *vp = cache + (size_t)(key & 16 ? at.page[1] : at.page[0]) * page_elems + ((size_t)(nkvh + kvh) * DH + l16) * page + (key & 16 ? at.tok[1] : at.tok[0]) + (key & 15);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int j = k0 + 16 * t;
-        const bf16_t *pg = cache + (size_t)pid[t] * page_elems;
-        const int tok0 = j % page;
-        const bf16_t *kp = pg + ((size_t)kvh * (DH / 8) * page + tok0 + l16) * 8;
-#pragma unroll
-        for (int kb = 0; kb < DH / 32; ++kb) f.k[t][kb] = __builtin_nontemporal_load((const u32x4 *)(kp + (size_t)(4 * kb + grp) * page * 8));
-        const bf16_t *vp = pg + v_off + tok0;
-#pragma unroll
-        for (int dt = 0; dt < DH / 16; ++dt) f.v[dt][t] = __builtin_nontemporal_load((const u32x2 *)(vp + (size_t)(16 * dt + l16) * page));
-    }
+    for (int dt = 0; dt < DH / 16; ++dt) f.v[dt] = __builtin_nontemporal_load((const u32x4 *)(vp + (size_t)16 * dt * page));
 }
 
 // One step of the online softmax on loaded keys and values, in three parts.  p_row / lo_row:
@@ -237,7 +216,8 @@ __device__ __forceinline__ float max_over_groups(float x) {
 
 // The softmax of the step, online: new maxima and sums, the output rescaled, the weights as
 // bfloat16 operands.
-// The lane's eight scores are four keys of each tile, k0 + 16 t + 4 grp .. + 3.
+// The lane's eight scores are four keys of each tile, k0 + 16 t + 4 grp .. + 3; the weights leave as those of eight neighbours of one
+// tile, k0 + mix_key(grp) .. + 7: groups 1 and 3 give their four of the first tile for the four of the second that groups 0 and 2 have.
 template <int DH, int QB, bool MASK>
 __device__ __forceinline__ void attn_softmax(const f32x4 (&s)[QB][2], int k0, AttnState<DH, QB> &st, const int (&p_row)[QB],
                                              const int (&lo_row)[QB], float scale_log2, int grp, u32x4 (&pb)[QB]) {
@@ -285,28 +265,26 @@ __device__ __forceinline__ void attn_softmax(const f32x4 (&s)[QB][2], int k0, At
 #pragma unroll
             for (int dt = 0; dt < DH / 16; ++dt) st.o[b][dt] *= alpha;
         }
-        pb[b] = u32x4{pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7])};
+        const auto lo = __builtin_amdgcn_permlane16_swap(pack_bf16(p[0], p[1]), pack_bf16(p[4], p[5]), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(pack_bf16(p[2], p[3]), pack_bf16(p[6], p[7]), false, false);
+        pb[b] = u32x4{lo[0], hi[0], lo[1], hi[1]};
     }
 }
 
 // O^T += V^T P^T
 template <int DH, int QB, bool MASK>
-__device__ __forceinline__ void attn_mix(const u32x2 (&v)[DH / 16][2], const u32x4 (&pb)[QB], int k0, int p_max, int lo_min,
+__device__ __forceinline__ void attn_mix(const u32x4 (&v)[DH / 16], const u32x4 (&pb)[QB], int k0, int p_max, int lo_min,
                                          int grp, AttnState<DH, QB> &st) {
 #pragma unroll
     for (int dt = 0; dt < DH / 16; ++dt) {
-        u32x2 v0 = v[dt][0], v1 = v[dt][1];
+        u32x4 a = v[dt];
         if (MASK) {
             // values of keys that no row sees are taken as zero: their memory may hold anything
-            const int j0 = k0 + 4 * grp, j1 = k0 + 16 + 4 * grp;
+            const int j0 = k0 + mix_key(grp);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t keep = (r & 1) ? 0x0000ffffu : 0xffff0000u;   // clears element r of its dword
-                if (j0 + r > p_max || j0 + r < lo_min) { if (r < 2) v0.x &= keep; else v0.y &= keep; }
-                if (j1 + r > p_max || j1 + r < lo_min) { if (r < 2) v1.x &= keep; else v1.y &= keep; }
-            }
+            for (int r = 0; r < 8; ++r)
+                if (j0 + r > p_max || j0 + r < lo_min) a[r / 2] &= (r & 1) ? 0x0000ffffu : 0xffff0000u;   // clears element r % 2 of its dword
         }
-        const u32x4 a = u32x4{v0.x, v0.y, v1.x, v1.y};
 #pragma unroll
         for (int b = 0; b < QB; ++b) st.o[b][dt] = mfma16(a, pb[b], st.o[b][dt]);
     }
@@ -342,22 +320,18 @@ __device__ __forceinline__ void load_q(const bf16_t *__restrict__ qrow, bool val
 }
 
 // ============================================================================ decode
-#ifndef LCU_DEC_WAVES
-#define LCU_DEC_WAVES 4
-#endif
-constexpr int DEC_WAVES = LCU_DEC_WAVES;
-#ifndef LCU_DEC_MIN_WAVES
-#define LCU_DEC_MIN_WAVES 2      // two waves per SIMD: measured faster than one with more registers
-#endif
-
-template <int DH, bool FLAT>
-__global__ void __launch_bounds__(DEC_WAVES *WAVE, LCU_DEC_MIN_WAVES)
+// WAVES: 8, or 4 where the rows of a workgroup are sixteen (their sums of eight waves would be more LDS than a launch gets unasked).  What bounds it over few
+// requests is how much one compute unit asks for at a time: with 4 waves everywhere a wave walked twice the steps, 2.5 us each: 8 requests of 1,024
+// keys, 16 heads of 128 over 4, 18.1 us and 14.9 with 8, 64 requests of 150 to 1,500, 32 heads over 8, 40.8 and 37.0; 32 requests of 20 to 100 keys 5.1 and 5.2
+// (16 waves want more than their 128 registers each).
+template <int DH, int WAVES>
+__global__ void __launch_bounds__(WAVES *WAVE, 2)
 attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__restrict__ out, int out_stride,
                         const bf16_t *__restrict__ cache, const int *__restrict__ block_table, int max_pages,
                         const int *__restrict__ q_start, const int *__restrict__ ctx_len,
                         const int *__restrict__ req_list, int nh, int nkvh, int page, float scale_log2, int window,
                         int n_splits, float *__restrict__ part_o, float *__restrict__ part_ml SCORE_KPARAMS) {
-    // [waves][16][DH + 4] outputs, then [waves][16][2] (m, l).  The four words more a row spread the sixteen rows over the banks
+    // [waves][held][DH + 4] outputs, then [waves][held][2] (m, l), held the most rows of a workgroup.  The four words more a row spread the sixteen rows over the banks
     extern __shared__ __attribute__((aligned(16))) float lds[];
     constexpr int PITCH = DH + 4;
     const int g = nh / nkvh;
@@ -367,15 +341,18 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     const int kvh = (blockIdx.x / chunks) % nkvh;
     const int chunk = blockIdx.x % chunks;
     const int split = blockIdx.y;
-    // the wave's number as a scalar: its steps' pages are then read through the scalar unit, and
-    // no wait for a page number stands between the loads of keys and values in flight
-    const int lane = threadIdx.x & (WAVE - 1), wave = FLAT ? threadIdx.x / WAVE : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int l16 = lane & 15, grp = lane >> 4;
+    const int held = g < 16 ? g : 16;
     const int rows = (g - 16 * chunk) < 16 ? (g - 16 * chunk) : 16;
     const int *bt = block_table + (size_t)r * max_pages;
-    int pid[2];
-    // without a window a request's one part begins with its first key: its pages are asked for together with its length
-    if (FLAT && window == 0) kv_pages(pid, bt, max_pages, page, wave * 32);
+    // without a window a request's one part begins with its first key: its first pages are asked for together with its length
+    const bool known = window == 0 && n_splits == 1;
+    KVPages ida, idb;
+    if (known) {
+        ida = kv_pages(bt, max_pages, page, wave * 32);
+        idb = kv_pages(bt, max_pages, page, (wave + WAVES) * 32);
+    }
     const int token = q_start[r];
     const int p = ctx_len[r] - 1;
     const int lo = first_key(p, window);
@@ -399,46 +376,24 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     const int first = lo / 32, last = p / 32, nblk = last - first + 1;
     const int b0 = first + (int)((long long)nblk * split / n_splits);
     const int b1 = first + (int)((long long)nblk * (split + 1) / n_splits);
-    // the wave's steps are blk, blk + 4, ...; the next step's loads are in flight while one is computed
+    // the wave's steps are blk, blk + WAVES, ...; the next step's loads are in flight while one is computed, and the pages of the
+    // step after it are known
     KVFrag<DH> fa, fb;
-    if (FLAT) {
-        int blk = b0 + wave;
-        if (window != 0) kv_pages(pid, bt, max_pages, page, blk * 32);
-        if (blk < b1) load_kv_flat<DH>(fa, cache, pid, page, page_elems, nkvh, kvh, blk * 32, l16, grp);
-        for (; blk < b1; blk += 2 * DEC_WAVES) {
-            const int nb = blk + DEC_WAVES, nb2 = blk + 2 * DEC_WAVES;
-            if (nb < b1) {
-                kv_pages(pid, bt, max_pages, page, nb * 32);
-                load_kv_flat<DH>(fb, cache, pid, page, page_elems, nkvh, kvh, nb * 32, l16, grp);
-            }
-            attn_block<DH, 1>(fa, blk * 32, blk * 32 + 31 > p || blk * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
-            if (nb2 < b1) {
-                kv_pages(pid, bt, max_pages, page, nb2 * 32);
-                load_kv_flat<DH>(fa, cache, pid, page, page_elems, nkvh, kvh, nb2 * 32, l16, grp);
-            }
-            if (nb < b1)
-                attn_block<DH, 1>(fb, nb * 32, nb * 32 + 31 > p || nb * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
-        }
-    } else {
-        // the pages of the step after the next are already known
-        int ida[2], idb[2];
-        int blk = b0 + wave;
-        kv_pages(ida, bt, max_pages, page, blk * 32);
-        kv_pages(idb, bt, max_pages, page, (blk + DEC_WAVES) * 32);
-        if (blk < b1) load_kv<DH>(fa, cache, ida, page, page_elems, nkvh, kvh, blk * 32, l16, grp);
-        kv_pages(ida, bt, max_pages, page, (blk + 2 * DEC_WAVES) * 32);
-        for (; blk < b1; blk += 2 * DEC_WAVES) {
-            const int nb = blk + DEC_WAVES, nb2 = blk + 2 * DEC_WAVES;
-            if (nb < b1) load_kv<DH>(fb, cache, idb, page, page_elems, nkvh, kvh, nb * 32, l16, grp);
-            kv_pages(idb, bt, max_pages, page, (nb + 2 * DEC_WAVES) * 32);
-            __builtin_amdgcn_sched_barrier(0);         // asked for before the arithmetic, there after it
-            attn_block<DH, 1>(fa, blk * 32, blk * 32 + 31 > p || blk * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
-            if (nb2 < b1) load_kv<DH>(fa, cache, ida, page, page_elems, nkvh, kvh, nb2 * 32, l16, grp);
-            kv_pages(ida, bt, max_pages, page, (nb2 + 2 * DEC_WAVES) * 32);
-            __builtin_amdgcn_sched_barrier(0);
-            if (nb < b1)
-                attn_block<DH, 1>(fb, nb * 32, nb * 32 + 31 > p || nb * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
-        }
+    int blk = b0 + wave;
+    if (!known) {
+        ida = kv_pages(bt, max_pages, page, blk * 32);
+        idb = kv_pages(bt, max_pages, page, (blk + WAVES) * 32);
+    }
+    if (blk < b1) load_kv<DH>(fa, cache, ida, page, page_elems, nkvh, kvh, l16, grp);
+    for (; blk < b1; blk += 2 * WAVES) {
+        const int nb = blk + WAVES, nb2 = blk + 2 * WAVES;
+        if (nb < b1) load_kv<DH>(fb, cache, idb, page, page_elems, nkvh, kvh, l16, grp);
+        ida = kv_pages(bt, max_pages, page, nb2 * 32);
+        idb = kv_pages(bt, max_pages, page, (nb2 + WAVES) * 32);
+        attn_block<DH, 1>(fa, blk * 32, blk * 32 + 31 > p || blk * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
+        if (nb2 < b1) load_kv<DH>(fa, cache, ida, page, page_elems, nkvh, kvh, l16, grp);
+        if (nb < b1)
+            attn_block<DH, 1>(fb, nb * 32, nb * 32 + 31 > p || nb * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
     }
     // ---- merge the waves (rows that are no head are not looked at).  What bounds the kernel over few keys is the way from one load to the
     // next and this merge: one MI355X, inside a step, 16 requests of 64 to 206 keys, 16 heads of 128 over 4: 9.6 us with a word a lane and
@@ -447,30 +402,30 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     l_all += __shfl_xor(l_all, 16, WAVE);
     l_all += __shfl_xor(l_all, 32, WAVE);
     float *lds_o = lds;
-    float *lds_ml = lds + DEC_WAVES * 16 * PITCH;
+    float *lds_ml = lds + WAVES * held * PITCH;
     if (l16 < rows) {
 #pragma unroll
-        for (int dt = 0; dt < DH / 16; ++dt) *(f32x4 *)(lds_o + (wave * 16 + l16) * PITCH + 16 * dt + 4 * grp) = st.o[0][dt];
+        for (int dt = 0; dt < DH / 16; ++dt) *(f32x4 *)(lds_o + (wave * held + l16) * PITCH + 16 * dt + 4 * grp) = st.o[0][dt];
         if (grp == 0) {
-            lds_ml[(wave * 16 + l16) * 2 + 0] = st.m[0];
-            lds_ml[(wave * 16 + l16) * 2 + 1] = l_all;
+            lds_ml[(wave * held + l16) * 2 + 0] = st.m[0];
+            lds_ml[(wave * held + l16) * 2 + 1] = l_all;
         }
     }
     __syncthreads();
     const bool four = ((uintptr_t)out & 7) == 0;       // (out_stride is a multiple of four)
-    for (int idx = threadIdx.x; idx < rows * (DH / 4); idx += DEC_WAVES * WAVE) {
+    for (int idx = threadIdx.x; idx < rows * (DH / 4); idx += WAVES * WAVE) {
         const int row = idx / (DH / 4), d = idx % (DH / 4) * 4;
         float M = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < DEC_WAVES; ++w) M = fmaxf(M, lds_ml[(w * 16 + row) * 2]);
+        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, lds_ml[(w * held + row) * 2]);
         const float M_safe = M == -INFINITY ? 0.f : M;
         float L = 0.f;
         f32x4 val = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < DEC_WAVES; ++w) {
-            const float f = exp2f(lds_ml[(w * 16 + row) * 2] - M_safe);
-            L += lds_ml[(w * 16 + row) * 2 + 1] * f;
-            val += *(const f32x4 *)(lds_o + (w * 16 + row) * PITCH + d) * f;
+        for (int w = 0; w < WAVES; ++w) {
+            const float f = exp2f(lds_ml[(w * held + row) * 2] - M_safe);
+            L += lds_ml[(w * held + row) * 2 + 1] * f;
+            val += *(const f32x4 *)(lds_o + (w * held + row) * PITCH + d) * f;
         }
         const int head = head0 + row;
         if (n_splits == 1) {
@@ -557,16 +512,11 @@ static int launch_decode(const void *q, int q_stride, void *out, int out_stride,
                          int n_splits, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
     const int g = nh / nkvh, chunks = (g + 15) / 16;
     const float scale_log2 = SCORE_LOG2(scale);
-    const size_t lds_bytes = (size_t)DEC_WAVES * 16 * (DH + 4 + 2) * sizeof(float);
-    dim3 grid(n_req * nkvh * chunks, n_splits), block(DEC_WAVES * WAVE);
-    // Two ways to address the pages (the same arithmetic, the same results).  FLAT: every lane holds
-    // full addresses and reads the block table itself.  Not FLAT: the wave's number and with it the
-    // pages are scalar, the loads are buffer loads with one lane offset for keys and one for values,
-    // and the table is read a step ahead.  Measured on the Llama-3-8B shape, whole decode step: the
-    // second is 1 % faster where a part is a few steps long (8 requests of 2k keys in 4 parts), the
-    // first 2 % faster where a wave walks many steps (32 or 64 requests, one part each).
-    const bool flat = n_splits == 1;
-    (flat ? attention_decode_kernel<DH, true> : attention_decode_kernel<DH, false>)<<<grid, block, lds_bytes, stream>>>(
+    const int held = g < 16 ? g : 16, waves = held < 16 ? 8 : 4;
+    const size_t lds_bytes = (size_t)waves * held * (DH + 4 + 2) * sizeof(float);
+    static_assert(8 * 15 * (128 + 4 + 2) * sizeof(float) <= 65536, "what a launch gets unasked");
+    dim3 grid(n_req * nkvh * chunks, n_splits), block(waves * WAVE);
+    (waves == 8 ? attention_decode_kernel<DH, 8> : attention_decode_kernel<DH, 4>)<<<grid, block, lds_bytes, stream>>>(
         (const bf16_t *)q, q_stride, (bf16_t *)out, out_stride, (const bf16_t *)cache, block_table, max_pages, q_start,
         ctx_len, req_list, nh, nkvh, page, scale_log2, window, n_splits, part_o, part_ml SCORE_KARGS(scale));
     LCU_LAUNCH_CHECK();

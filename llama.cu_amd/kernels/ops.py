@@ -638,8 +638,8 @@ def plan_attention(step, n_heads: int, n_kv_heads: int, window: int = 0, biased:
 
 def decode_splits(n_req: int, n_heads: int, n_kv_heads: int, max_ctx_len: int) -> int:
     """Into how many parts the decode kernel cuts each request's keys (the numbers are ``TUNING``'s).
-    Few requests: about one workgroup for each compute unit, no part shorter than 512 keys, at most
-    32 parts (measured from 2k to 128k keys: more parts cost more in the merge than they gain; a
+    Few requests: about one workgroup for each compute unit, one part up to 512 keys, beyond them parts of 512 keys but
+    up to 8 shorter ones, at most 32 parts (measured from 2k to 128k keys: more parts cost more in the merge than they gain; a
     single request with 128k keys wants 32).  Between half the chip's worth of workgroups and all of
     it (17 to 31 requests of 8 key/value heads), where one part leaves compute units idle and two
     parts are a wave and a bit: one part up to 1k keys, beyond that up to 4 parts of at least 1024
@@ -655,7 +655,8 @@ def decode_splits(n_req: int, n_heads: int, n_kv_heads: int, max_ctx_len: int) -
     base = max(1, n_req * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16))
     rounded = 1 << max(int(max_ctx_len) - 1, 0).bit_length()     # up to a power of two: the choice changes rarely
     if base <= t.decode_few_workgroups:
-        return max(1, min(t.decode_max_parts, t.compute_units // base, rounded // t.decode_min_part_keys))
+        parts = rounded // t.decode_min_part_keys
+        return max(1, min(t.decode_max_parts, t.compute_units // base, max(parts, t.decode_few_parts) if parts > 1 else parts))
     most = min(t.decode_long_max_parts, rounded // t.decode_long_part_keys) \
         if (rounded >= t.decode_long_context and base < t.compute_units) else 1
     fill = [(base * s / t.compute_units) / -(-base * s // t.compute_units) for s in range(1, most + 1)]

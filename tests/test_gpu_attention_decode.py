@@ -31,3 +31,22 @@ def test_stores(nh, nkv, dh, window, splits):
         ops.attention_decode(q, odd[:, 2:2 + nh * dh], cache, table, starts, lens, n, nh, nkv, dh, page, scale, window, splits)
         assert torch.equal(odd[:, 2:2 + nh * dh], even)
         assert (odd[:, :2] == 0).all() and (odd[:, 2 + nh * dh:] == 0).all()
+
+
+@pytest.mark.parametrize("nh,nkv,dh", [(15, 1, 128), (16, 1, 128), (17, 1, 32)])
+@pytest.mark.parametrize("page", [16, 48, 64])
+@pytest.mark.parametrize("splits", [1, 8])
+def test_rows_waves_and_pages(nh, nkv, dh, page, splits):
+    """Fifteen rows a workgroup are the most that eight waves share, sixteen go to four; pages of 16 tokens and of several times as many; lengths at the
+    edges of a step of 32 keys, of a round of the waves and of the parts."""
+    from llama_cu_amd.kernels import ops
+    ctx = [1, 16, 17, 32, 128, 129, 256, 257, 513]
+    n, most = len(ctx), -(-max(ctx) // page)
+    cache = rnd(n * most + 1, 2, nkv * dh * page, seed=4).bfloat16().cuda()
+    table = (torch.randperm(n * most, generator=torch.Generator().manual_seed(5)) + 1).to(torch.int32).view(n, most).contiguous().cuda()
+    q = rnd(n, nh * dh, seed=6).bfloat16().cuda()
+    starts, of, lens = torch.arange(n + 1, dtype=torch.int32).cuda(), torch.arange(n, dtype=torch.int32).cuda(), torch.tensor(ctx, dtype=torch.int32).cuda()
+    got, wanted = torch.empty(n, nh * dh, dtype=torch.bfloat16, device="cuda"), torch.empty(n, nh * dh, dtype=torch.bfloat16, device="cuda")
+    ops.paged_attention_generic(q, wanted, cache, table, starts, lens, of, nh, nkv, dh, page, dh ** -0.5, 0)
+    ops.attention_decode(q, got, cache, table, starts, lens, n, nh, nkv, dh, page, dh ** -0.5, 0, splits)
+    assert_close(got, wanted, 3 * 2.0 ** -8, "against the generic kernel")        # the weights and both outputs rounded to bfloat16
