@@ -554,6 +554,110 @@ moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__
     }
 }
 
+// The least pairs (one to eight tokens of two, say): a workgroup looks for the blockIdx.y-th expert that any of them names, so the launch holds no
+// workgroups of experts without a pair, and has eight waves, a quarter of K and one of the two tiles each, with eight steps on their way: few workgroups then
+// ask for as much at a time as many would.  The sums are added up as in the kernel for few rows: the same bits.  What bounds it is the way of the numbers of the experts
+// and of their matrices' first lines through memory, one after the other.  One MI355X, both products, us, with the kernel for few rows everywhere and now: a token of two experts of
+// 2 x 1024 x 2048 with a shared one of 704 13.6 and 11.9, two tokens 19.5 and 17.5; a token of two of 2 x 1408 x 2048 14.4 and 11.9, of four of 2 x 512 x 2048 13.1 and 10.9, of one of
+// 2 x 3584 x 1024 16.5 and 13.1.  From some 400 workgroups on four waves with two tiles each read the rows half as often: four tokens of two of 2 x 1408 x 2048 23.7 and 25.4, eight of
+// four of 2 x 512 x 2048 29.3 and 46.6.
+constexpr int MOE_SLOTS = 64, MOE_SLOT_ROWS = 16;      // pairs, a lane each; tokens
+constexpr int MOE_SLOT_WORKGROUPS = 384;               // of the experts that pairs name, at most
+template <class T, int MODE, bool PACKED>
+__global__ void __launch_bounds__(512)
+moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__ w, size_t w_expert_stride, int N, int K,
+                      const int *__restrict__ ids, int total, const float *__restrict__ wts, T *__restrict__ out_t,
+                      float *__restrict__ out_f, int out_stride, int top, int add, float alpha, float limit, int experts, int slots,
+                      const T *__restrict__ sx, const T *__restrict__ sw, int s_n, int s_k, T *__restrict__ s_out_t, float *__restrict__ s_out_f) {
+    typedef Mma<T> M;
+    typedef typename M::frag frag;
+    constexpr bool GATED = MODE == MOE_UP_GATED, UP = MODE != MOE_DOWN;
+    constexpr int AHEAD = 8;
+    __shared__ f32x4 red[4][2][WAVE];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, g = lane / 16, l16 = lane % 16;
+    const int part = wave & 3, side = wave >> 2;
+    const bool shared = (int)blockIdx.y == slots;
+    const T *we = sw;
+    int count = total, flat = l16;                   // of row l16
+    if (shared) {                                    // every token's rows [n, s_k] and a matrix of its own size
+        count /= top;
+        top = 1;
+        x = sx;
+        N = s_n;
+        K = s_k;
+        x_stride = GATED ? x_stride : s_k;
+        out_t = s_out_t;
+        out_f = s_out_f;
+        out_stride = GATED ? s_n / 2 : out_stride;
+        alpha = 1.f;
+        limit = 0.f;
+        flat = min(l16, count - 1);
+    } else {
+        const int mine = lane < total ? ids[lane] : -1;
+        bool first = mine >= 0 && mine < experts;    // (identity experts have no matrices)
+        for (int j = 0; j < total - 1; ++j) first = first && !(j < lane && __builtin_amdgcn_readlane(mine, j) == mine);
+        unsigned long long which = __ballot(first);
+        if ((int)blockIdx.y >= __popcll(which)) return;
+        for (int y = 0; y < (int)blockIdx.y; ++y) which &= which - 1;
+        const int e = __builtin_amdgcn_readlane(mine, __builtin_ctzll(which));
+        unsigned long long pairs = __ballot(mine == e);
+        count = __popcll(pairs);
+        for (int r = 0; r < min(l16, count - 1); ++r) pairs &= pairs - 1;
+        flat = __builtin_ctzll(pairs);
+        we = w + (size_t)e * w_expert_stride;
+    }
+    if ((int)blockIdx.x * 32 >= N) return;
+    const int tile0 = 2 * blockIdx.x, steps = (K + M::KSTEP - 1) / M::KSTEP, per = quarter_steps(steps);
+    const int s0 = min(steps, part * per), s1 = min(steps, s0 + per);
+    const Unit<T, PACKED> wu(we, tile0 + side, N, K, steps, lane);
+    const T *xr = x + (size_t)(UP ? flat / top : flat) * x_stride + g * M::PER_LANE;
+    const float sc = MODE == MOE_UP ? wts[flat] : 1.f;
+    const int x_left = K - g * M::PER_LANE;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    frag a[AHEAD], b[AHEAD];
+    auto fetch = [&](int u, int s) {
+        a[u] = wu.load(s);
+        b[u] = s * M::KSTEP < x_left ? M::load(xr + s * M::KSTEP) : M::zero();
+    };
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+        if (s0 + u < s1) fetch(u, s0 + u);
+    for (int s = s0; s < s1; s += AHEAD) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            if (s + u >= s1) break;
+            acc = M::mma(a[u], MODE == MOE_UP ? M::scaled(b[u], sc) : b[u], acc);
+            if (s + u + AHEAD < s1) fetch(u, s + u + AHEAD);
+        }
+    }
+    red[part][side][lane] = acc;
+    __syncthreads();
+    // the first wave stores (with two products' sums the first two, one each): four neighbouring features of a row a lane
+    if (wave >= (GATED ? 1 : 2)) return;
+    const f32x4 v = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
+    const int dst = !UP && add ? flat / top : flat;
+    if (l16 >= count) return;
+    if constexpr (GATED) {
+        const f32x4 up = ((red[0][1][lane] + red[1][1][lane]) + red[2][1][lane]) + red[3][1][lane];
+        Quad<T> q;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gate_up_of(v[i], up[i], alpha, limit));
+        *(Quad<T> *)(out_t + (size_t)dst * out_stride + tile0 * 8 + 4 * g) = q;
+    } else {
+        const int col = (tile0 + wave) * 16 + 4 * g; // (N is a multiple of 4)
+        if (col >= N) return;
+        if constexpr (MODE == MOE_UP) {
+            Quad<T> q;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gelu_erf(v[i]));
+            *(Quad<T> *)(out_t + (size_t)dst * out_stride + col) = q;
+        } else {
+            f32x4 *o = (f32x4 *)(out_f + (size_t)dst * out_stride + col);
+            *o = add ? *o + v : v;
+        }
+    }
+}
+
 // Many rows an expert (prompts): tiles of up to 32, 64, 96 or 128 rows; a block of four waves takes a tile and 128 features, a wave 32 of them with all
 // rows.  The rows go through LDS in steps of 128 bytes of k, in two buffers in turn with one barrier a step; no two waves want the same piece of the
 // matrix, so each loads its own straight into registers.  Both are two steps ahead.  MT: tiles of 16 rows that are multiplied.
@@ -908,6 +1012,16 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
         const int with = (tile_rows ? max_tiles : experts) + (shared_up ? 1 : 0), s_rows = 2 * shared_ff, wider = shared_up && s_rows > up_rows ? s_rows : up_rows;
         const size_t act_end = (size_t)total * ff;
         const dim3 block(256), gu((wider + 31) / 32, with), gd((d + 31) / 32, with);
+        const int slots = total < experts ? total : experts;
+        const bool least = !tile_rows && total <= MOE_SLOTS && n <= MOE_SLOT_ROWS;
+        const dim3 su(gu.x, slots + (shared_up ? 1 : 0)), sd(gd.x, su.y);
+        const bool up_slots = least && (up_rows + 31) / 32 * slots <= MOE_SLOT_WORKGROUPS, down_slots = least && (d + 31) / 32 * slots <= MOE_SLOT_WORKGROUPS;
+#define UP_SLOTS(T, PACKED, MODE) moe_gemm_slots_kernel<T, MODE, PACKED><<<su, dim3(512), 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \
+                                                ids, total, wts, (T *)act, nullptr, ff, top, 0, alpha, limit, experts, slots, \
+                                                (const T *)h, (const T *)shared_up, s_rows, d, (T *)act + act_end, nullptr)
+#define DOWN_SLOTS(T, PACKED, MODE) moe_gemm_slots_kernel<T, MODE, PACKED><<<sd, dim3(512), 0, stream>>>((const T *)act, ff, (const T *)w_down, down_stride, d, ff, \
+                                                ids, total, wts, nullptr, down_to, d, top, add, 0.f, 0.f, experts, slots, \
+                                                (const T *)act + act_end, (const T *)shared_down, d, shared_ff, nullptr, y + (size_t)total * d)
 #define UP(T, PACKED, MODE) moe_gemm_few_kernel<T, MODE, PACKED><<<gu, block, 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \
                                                 ids, total, wts, (T *)act, nullptr, ff, top, 0, alpha, limit, experts, \
                                                 (const T *)h, (const T *)shared_up, s_rows, d, (T *)act + act_end, nullptr, sorted, t_exp, t_beg, t_rows, n_tiles, max_tiles)
@@ -915,9 +1029,15 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
                                                 ids, total, wts, nullptr, down_to, d, top, add, 0.f, 0.f, experts, \
                                                 (const T *)act + act_end, (const T *)shared_down, d, shared_ff, nullptr, y + (size_t)total * d, sorted, t_exp, t_beg, t_rows, n_tiles, max_tiles)
         int packed = packed_up;
-        if (gated) { TYPED(UP, MOE_UP_GATED); } else { TYPED(UP, MOE_UP); }
+        if (up_slots) {
+            if (gated) { TYPED(UP_SLOTS, MOE_UP_GATED); } else { TYPED(UP_SLOTS, MOE_UP); }
+        } else {
+            if (gated) { TYPED(UP, MOE_UP_GATED); } else { TYPED(UP, MOE_UP); }
+        }
         packed = packed_down;
-        TYPED(DOWN, MOE_DOWN);
+        if (down_slots) { TYPED(DOWN_SLOTS, MOE_DOWN); } else { TYPED(DOWN, MOE_DOWN); }
+#undef UP_SLOTS
+#undef DOWN_SLOTS
 #undef UP
 #undef DOWN
     } else {

@@ -260,3 +260,32 @@ def test_memory_that_nobody_reads_is_not_asked_for(gated):
     assert more <= 4 * n * d * gated + 2 * n * ff + (1 << 16), more            # (the pairs' rows, the activations, the lists)
     if gated:
         assert torch.equal(kept.rows(), torch.zeros(n, d, device="cuda"))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("n,top,experts,identity", [(1, 1, 3, 0), (1, 4, 8, 2), (3, 2, 2, 0), (16, 4, 5, 3), (16, 2, 40, 0), (17, 1, 4, 0)])
+@pytest.mark.parametrize("d,ff", [(72, 32), (520, 144)])
+def test_the_experts_that_any_pair_names(dtype, n, top, experts, identity, d, ff):
+    """The kernel of the least pairs at its edges (one pair; every expert named; 64 pairs; 16 tokens, and 17 of which it takes none): the same bits as from tiles of 16
+    sorted rows, with and without identity experts and a shared one."""
+    from llama_cu_amd.kernels import build, ops
+    tdt = TYPES[dtype]
+    h = rnd(n, d, seed=1).to(tdt).cuda()
+    gen = torch.Generator().manual_seed(2)
+    ids = torch.stack([torch.randperm(experts + identity, generator=gen)[:top] for _ in range(n)]).to(torch.int32).cuda()
+    wts = torch.rand(n, top, generator=gen).cuda()
+    rows = ops.gated_rows(*(rnd(experts, ff, d, seed=k, std=d ** -0.5).to(tdt).cuda() for k in (3, 4)))
+    up, down = ops.pack_experts(rows), ops.pack_experts(rnd(experts, d, ff, seed=5, std=ff ** -0.5).to(tdt).cuda())
+    sff = 48
+    shared = (ops.pack_experts(ops.gated_rows(*(rnd(1, sff, d, seed=k, std=d ** -0.5).to(tdt).cuda() for k in (6, 7)))),
+              ops.pack_experts(rnd(1, d, sff, seed=8, std=sff ** -0.5).to(tdt).cuda()))
+    kw = dict(gated=True, fresh=True, identity=identity, shared_expert=shared if ops.moe_shared_beside(n, top, experts, up, down) else None)
+    got, want = torch.empty(n, d, device="cuda"), torch.empty(n, d, device="cuda")
+    ops.moe_experts(h, ids, wts, up, down, got, **kw)
+    lib = build.load("moe")
+    real, lib.lcu_moe_tile_rows = lib.lcu_moe_tile_rows, lambda *a: 16
+    try:
+        ops.moe_experts(h, ids, wts, up, down, want, **kw)
+    finally:
+        lib.lcu_moe_tile_rows = real
+    assert torch.equal(got, want)
