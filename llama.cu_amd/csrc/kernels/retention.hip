@@ -57,6 +57,12 @@ retention_prep_kernel(const TI *__restrict__ rows, int row_stride, int q_off, in
         qk[((size_t)(w / dv) * n + t) * (2 * d + dv) + 2 * d + w % dv] = to_f32(row[v_off + w]);
 }
 
+// One element of S and its share of an output, rounded the same way in every kernel: the decayed element is rounded, the new term fused into the sum.
+__device__ __forceinline__ void retention_step(float &s, float &o, float g, float k, float v, float q) {
+    s = __builtin_fmaf(k, v, g * s);
+    o = __builtin_fmaf(s, q, o);
+}
+
 // The scan.  DPL: key channels per lane (d <= 16 * DPL), a lane's channels neighbours; TOK: tokens staged at a time.  Two
 // buffers in LDS: while the waves work through one, every thread holds the next tokens' share in registers (loaded
 // before the work began) and writes it into the other afterwards: one barrier a stage.
@@ -158,10 +164,10 @@ retention_scan_kernel(const float *__restrict__ qk,
 #pragma unroll
             for (int e4 = 0; e4 < DPL / 4; ++e4) {
                 const float4 k4 = *(const float4 *)(ks + sub * DPL + 4 * e4), q4 = *(const float4 *)(qs + sub * DPL + 4 * e4);
-                s[4 * e4 + 0] = gt * s[4 * e4 + 0] + k4.x * v; acc[tt] += s[4 * e4 + 0] * q4.x;
-                s[4 * e4 + 1] = gt * s[4 * e4 + 1] + k4.y * v; acc[tt] += s[4 * e4 + 1] * q4.y;
-                s[4 * e4 + 2] = gt * s[4 * e4 + 2] + k4.z * v; acc[tt] += s[4 * e4 + 2] * q4.z;
-                s[4 * e4 + 3] = gt * s[4 * e4 + 3] + k4.w * v; acc[tt] += s[4 * e4 + 3] * q4.w;
+                retention_step(s[4 * e4 + 0], acc[tt], gt, k4.x, v, q4.x);
+                retention_step(s[4 * e4 + 1], acc[tt], gt, k4.y, v, q4.y);
+                retention_step(s[4 * e4 + 2], acc[tt], gt, k4.z, v, q4.z);
+                retention_step(s[4 * e4 + 3], acc[tt], gt, k4.w, v, q4.w);
             }
         }
         // after the moves every lane of a column's sixteen holds the token's sum: lane `tt` of them keeps token tt's, and
@@ -245,6 +251,134 @@ retention_out_kernel(const float *__restrict__ o, const TG *__restrict__ gate, i
         const float z = to_f32(gate[(size_t)t * gate_stride + g_off + h * dv + c]);
         out[(size_t)t * nh * dv + (size_t)h * dv + c] = from_f32<T>(at(c) * f * (z / (1.0f + expf(-z))));
     }
+}
+
+// ---------------------------------------------------------------- one token a request
+// A step in which every request feeds one token (row r is request r's): all of the above in one kernel, a workgroup per (request, head).  A wave takes 32
+// columns of S at a time, a lane four neighbouring ones (16-byte loads) of 2 DPL key channels; the matrix is on its way while q and k are turned.  Every sum
+// is made in the scan's and the output's order (a lane's two shares of DPL channels are two of the scan's sixteen lanes, the groups of eight lanes the rest
+// of their tree), so a token has the same bits either way.  The three kernels read and wrote the token's vectors through memory, and the scan staged
+// sixteen tokens where there is one.  What bounds it are the matrices and, for few, the way from a load to the next.  One MI355X, 8 heads of 128 x 128, us: 1 request 12.9 -> 4.8, 8
+// 16.4 -> 5.3, 64 55 -> 11.0; 16 of 64 x 64, 256 requests 78 -> 24; 4 of 32 x 16, 1 request 7.8 -> 3.5; 4 of 128 x 512, 8 requests 26.8 -> 11.6.
+constexpr int RS_MAX_DV = 512;
+__device__ __forceinline__ float sum_over_eighths(float v) {
+    v += __shfl_xor(v, 8, WAVE);
+    v += __shfl_xor(v, 16, WAVE);
+    return v + __shfl_xor(v, 32, WAVE);
+}
+template <int DPL, class TI, class T>
+__global__ void __launch_bounds__(256)
+retention_single_kernel(const TI *__restrict__ rows, int row_stride, int q_off, int k_off, int v_off, int g_off, const float *__restrict__ cos_t,
+                        const float *__restrict__ sin_t, int max_pos, int rot_dim, int pairing, float k_scale, const float *__restrict__ decay,
+                        float *__restrict__ state, T *__restrict__ out, const int *__restrict__ ctx_len, const int *__restrict__ state_slot, int nh, int d,
+                        int dv, float eps) {
+    typedef __attribute__((ext_vector_type(4))) float f32x4;
+    constexpr int D = RT_LANES * DPL, SL = 2 * DPL, VEC = 8 * (SL + 4);                      // a vector in LDS: the groups' shares, four floats of padding behind each
+    __shared__ __attribute__((aligned(16))) float qs[VEC], ks[VEC], os[RS_MAX_DV];
+    const int r = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = lane / 8;
+    const TI *row = rows + (size_t)r * row_stride;
+    const int ctx = ctx_len[r];
+    float *S = state + ((size_t)state_slot[r] * nh + h) * (size_t)d * dv;
+    f32x4 s[SL];
+    auto load = [&](int col) {
+#pragma unroll
+        for (int i = 0; i < SL; ++i) {
+            s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (ctx > 1 && grp * SL + i < d && col < dv) s[i] = *(const f32x4 *)(S + (size_t)(grp * SL + i) * dv + col);
+        }
+    };
+    int col = 32 * wave + lane % 8 * 4;
+    load(col);
+    if (tid < D) {
+        float qv = 0.f, kv = 0.f;
+        const int i = tid;
+        if (i < d) {
+            qv = to_f32(row[q_off + h * d + i]);
+            kv = to_f32(row[k_off + h * d + i]);
+            if (cos_t && i < rot_dim) {
+                const int half = rot_dim / 2, pos = ctx - 1;
+                const bool first = pairing == 0 ? i < half : (i & 1) == 0;
+                const int pi = pairing == 0 ? (first ? i : i - half) : i >> 1, partner = pairing == 0 ? (first ? i + half : i - half) : i ^ 1;
+                const float qp = to_f32(row[q_off + h * d + partner]), kp = to_f32(row[k_off + h * d + partner]);
+                float c = __uint_as_float(0x7fc00000u), sn = c, ra, rb;               // a position outside the table gives NaN
+                if (pos >= 0 && pos < max_pos) { c = cos_t[(size_t)pos * half + pi]; sn = sin_t[(size_t)pos * half + pi]; }
+                if (first) { rotate_pair(qv, qp, c, sn, ra, rb); qv = ra; rotate_pair(kv, kp, c, sn, ra, rb); kv = ra; }
+                else { rotate_pair(qp, qv, c, sn, ra, rb); qv = rb; rotate_pair(kp, kv, c, sn, ra, rb); kv = rb; }
+            }
+        }
+        qs[i / SL * (SL + 4) + i % SL] = qv;
+        ks[i / SL * (SL + 4) + i % SL] = kv * k_scale;
+    }
+    const float g = decay[h];
+    lds_barrier();
+    for (;;) {
+        const bool live = col < dv;
+        f32x4 v = {0.f, 0.f, 0.f, 0.f}, acc[2] = {};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = live ? to_f32(row[v_off + h * dv + col + e]) : 0.f;
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int i4 = 0; i4 < DPL; i4 += 4) {
+                const int at = grp * (SL + 4) + half * DPL + i4;
+                const f32x4 k4 = *(const f32x4 *)(ks + at), q4 = *(const f32x4 *)(qs + at);
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    f32x4 &sx = s[half * DPL + i4 + x];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float t = sx[e], sum = acc[half][e];
+                        retention_step(t, sum, g, k4[x], v[e], q4[x]);
+                        sx[e] = t;
+                        acc[half][e] = sum;
+                    }
+                }
+            }
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = sum_over_eighths(acc[0][e] + acc[1][e]);
+        if (live) {
+#pragma unroll
+            for (int i = 0; i < SL; ++i)
+                if (grp * SL + i < d) *(f32x4 *)(S + (size_t)(grp * SL + i) * dv + col) = s[i];
+            if (grp == 0) *(f32x4 *)(os + col) = o;
+        }
+        col += 128;
+        if (col - lane % 8 * 4 >= dv) break;
+        load(col);
+    }
+    lds_barrier();
+    float sq = 0.f;
+    for (int c = lane; c < dv; c += WAVE) sq += os[c] * os[c];
+    const float f = rsqrtf(wave_sum(sq) / (float)dv + eps);
+    for (int c = tid; c < dv; c += 256) {
+        const float z = to_f32(row[g_off + h * dv + c]);
+        out[((size_t)r * nh + h) * dv + c] = from_f32<T>(os[c] * f * (z / (1.0f + expf(-z))));
+    }
+}
+
+// Whether lcu_retention_single takes heads of these sizes.
+LCU_API int lcu_retention_single_takes(int d, int dv) { return d > 0 && d <= 128 && dv > 0 && dv % 4 == 0 && dv <= RS_MAX_DV; }
+
+// lcu_retention for a step in which every request feeds one token, where lcu_retention_single_takes says so; state 16-byte aligned.
+LCU_API int lcu_retention_single(const void *rows, int in_type, int row_stride, int q_off, int k_off, int v_off, int g_off, const float *cos_t,
+                                 const float *sin_t, int max_pos, int rot_dim, int pairing, float k_scale, const float *decay, float *state, void *out,
+                                 int out_type, const int *ctx_len, const int *state_slot, int n_req, int nh, int d, int dv, float eps, hipStream_t stream) {
+    if (n_req <= 0) return LCU_OK;
+    if (!lcu_retention_single_takes(d, dv) || nh <= 0 || nh > 65535 || rot_dim < 0 || rot_dim % 2 || rot_dim > d || (pairing != 0 && pairing != 1) || !rows || !decay ||
+        !state || (uintptr_t)state % 16 || !out || (cos_t && !sin_t))
+        return LCU_BAD_ARGUMENT;
+#define GO(DPL, TI, T) retention_single_kernel<DPL, TI, T><<<dim3(n_req, nh), dim3(256), 0, stream>>>((const TI *)rows, row_stride, q_off, k_off, v_off, g_off, cos_t, sin_t, \
+                                                max_pos, rot_dim, pairing, k_scale, decay, state, (T *)out, ctx_len, state_slot, nh, d, dv, eps)
+#define SIZES(TI, T) do { if (d <= 64) GO(4, TI, T); else GO(8, TI, T); } while (0)
+    if (in_type == LCU_F32 && out_type == LCU_F32) SIZES(float, float);
+    else if (in_type == LCU_F32 && out_type == LCU_BF16) SIZES(float, bf16_t);
+    else if (in_type == LCU_BF16 && out_type == LCU_BF16) SIZES(bf16_t, bf16_t);
+    else return LCU_BAD_ARGUMENT;
+#undef SIZES
+#undef GO
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
 }
 
 // rows: [n, row_stride] of in_type with q (nh * d) at q_off, k at k_off, v (nh * dv) at v_off and the gate (nh * dv)
