@@ -320,10 +320,12 @@ __device__ __forceinline__ void load_q(const bf16_t *__restrict__ qrow, bool val
 }
 
 // ============================================================================ decode
-// WAVES: 8, or 4 where the rows of a workgroup are sixteen (their sums of eight waves would be more LDS than a launch gets unasked).  What bounds it over few
+// WAVES: 8, or 4 where no request has more keys than four waves take in one step each, or where the rows of a workgroup are sixteen (their sums of eight waves would be more LDS than a
+// launch gets unasked).  What bounds it over few
 // requests is how much one compute unit asks for at a time: with 4 waves everywhere a wave walked twice the steps, 2.5 us each: 8 requests of 1,024
-// keys, 16 heads of 128 over 4, 18.1 us and 14.9 with 8, 64 requests of 150 to 1,500, 32 heads over 8, 40.8 and 37.0; 32 requests of 20 to 100 keys 5.1 and 5.2
+// keys, 16 heads of 128 over 4, 18.1 us and 14.9 with 8, 64 requests of 150 to 1,500, 32 heads over 8, 40.8 and 37.0; 60 requests of 8 to 19 keys, 2.3 us less with 4, 8 of 32 keys 3.7 and 3.9
 // (16 waves want more than their 128 registers each).
+constexpr int DEC_FEW_KEYS = 128;
 template <int DH, int WAVES>
 __global__ void __launch_bounds__(WAVES *WAVE, 2)
 attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__restrict__ out, int out_stride,
@@ -331,7 +333,7 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
                         const int *__restrict__ q_start, const int *__restrict__ ctx_len,
                         const int *__restrict__ req_list, int nh, int nkvh, int page, float scale_log2, int window,
                         int n_splits, float *__restrict__ part_o, float *__restrict__ part_ml SCORE_KPARAMS) {
-    // [waves][held][DH + 4] outputs, then [waves][held][2] (m, l), held the most rows of a workgroup.  The four words more a row spread the sixteen rows over the banks
+    // [waves][held][DH + 4] outputs, then [held][2][waves] (m, then l), held the most rows of a workgroup.  The four words more a row spread the sixteen rows over the banks
     extern __shared__ __attribute__((aligned(16))) float lds[];
     constexpr int PITCH = DH + 4;
     const int g = nh / nkvh;
@@ -388,8 +390,10 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     for (; blk < b1; blk += 2 * WAVES) {
         const int nb = blk + WAVES, nb2 = blk + 2 * WAVES;
         if (nb < b1) load_kv<DH>(fb, cache, idb, page, page_elems, nkvh, kvh, l16, grp);
-        ida = kv_pages(bt, max_pages, page, nb2 * 32);
-        idb = kv_pages(bt, max_pages, page, (nb2 + WAVES) * 32);
+        if (nb2 < b1) {                                // (numbers that nobody wants would be waited for at the merge all the same)
+            ida = kv_pages(bt, max_pages, page, nb2 * 32);
+            idb = kv_pages(bt, max_pages, page, (nb2 + WAVES) * 32);
+        }
         attn_block<DH, 1>(fa, blk * 32, blk * 32 + 31 > p || blk * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
         if (nb2 < b1) load_kv<DH>(fa, cache, ida, page, page_elems, nkvh, kvh, l16, grp);
         if (nb < b1)
@@ -407,24 +411,27 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
 #pragma unroll
         for (int dt = 0; dt < DH / 16; ++dt) *(f32x4 *)(lds_o + (wave * held + l16) * PITCH + 16 * dt + 4 * grp) = st.o[0][dt];
         if (grp == 0) {
-            lds_ml[(wave * held + l16) * 2 + 0] = st.m[0];
-            lds_ml[(wave * held + l16) * 2 + 1] = l_all;
+            lds_ml[l16 * 2 * WAVES + wave] = st.m[0];
+            lds_ml[l16 * 2 * WAVES + WAVES + wave] = l_all;
         }
     }
     __syncthreads();
     const bool four = ((uintptr_t)out & 7) == 0;       // (out_stride is a multiple of four)
     for (int idx = threadIdx.x; idx < rows * (DH / 4); idx += WAVES * WAVE) {
         const int row = idx / (DH / 4), d = idx % (DH / 4) * 4;
+        f32x4 ml[2][WAVES / 4];
+#pragma unroll
+        for (int w = 0; w < WAVES / 2; ++w) ml[w / (WAVES / 4)][w % (WAVES / 4)] = *(const f32x4 *)(lds_ml + row * 2 * WAVES + 4 * w);
         float M = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, lds_ml[(w * held + row) * 2]);
+        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, ml[0][w / 4][w % 4]);
         const float M_safe = M == -INFINITY ? 0.f : M;
         float L = 0.f;
         f32x4 val = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) {
-            const float f = exp2f(lds_ml[(w * held + row) * 2] - M_safe);
-            L += lds_ml[(w * held + row) * 2 + 1] * f;
+            const float f = exp2f(ml[0][w / 4][w % 4] - M_safe);
+            L += ml[1][w / 4][w % 4] * f;
             val += *(const f32x4 *)(lds_o + (w * held + row) * PITCH + d) * f;
         }
         const int head = head0 + row;
@@ -509,10 +516,10 @@ template <int DH>
 static int launch_decode(const void *q, int q_stride, void *out, int out_stride, const void *cache,
                          const int *block_table, int max_pages, const int *q_start, const int *ctx_len,
                          const int *req_list, int n_req, int nh, int nkvh, int page, float scale, int window,
-                         int n_splits, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
+                         int n_splits, int few_keys, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
     const int g = nh / nkvh, chunks = (g + 15) / 16;
     const float scale_log2 = SCORE_LOG2(scale);
-    const int held = g < 16 ? g : 16, waves = held < 16 ? 8 : 4;
+    const int held = g < 16 ? g : 16, waves = held < 16 && !few_keys ? 8 : 4;
     const size_t lds_bytes = (size_t)waves * held * (DH + 4 + 2) * sizeof(float);
     static_assert(8 * 15 * (128 + 4 + 2) * sizeof(float) <= 65536, "what a launch gets unasked");
     dim3 grid(n_req * nkvh * chunks, n_splits), block(waves * WAVE);
@@ -543,10 +550,11 @@ static int decode_arguments(int q_stride, int out_stride, int max_pages, int nh,
     return LCU_OK;
 }
 
-LCU_API int lcu_attention_decode_bf16(const void *q, int q_stride, void *out, int out_stride, const void *cache,
+// few_keys: no request has more than DEC_FEW_KEYS keys (a matter of speed alone).
+LCU_API int lcu_attention_decode_lengths_bf16(const void *q, int q_stride, void *out, int out_stride, const void *cache,
                                       const int *block_table, int max_pages, const int *q_start, const int *ctx_len,
                                       const int *req_list, int n_req, int nh, int nkvh, int dh, int page, float scale,
-                                      int window, int n_splits, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
+                                      int window, int n_splits, int few_keys, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
     if (n_req <= 0) return LCU_OK;
 #ifdef LCU_SCORE_BIAS
     if (!head_slopes || !(scale > 0.f)) return LCU_BAD_ARGUMENT;
@@ -557,13 +565,21 @@ LCU_API int lcu_attention_decode_bf16(const void *q, int q_stride, void *out, in
     const int args = decode_arguments(q_stride, out_stride, max_pages, nh, nkvh, dh, page, window, n_splits);
     if (args != LCU_OK) return args;
     if (n_splits > 1 && (!part_o || !part_ml)) return LCU_BAD_ARGUMENT;
-#define GO(D) return launch_decode<D>(q, q_stride, out, out_stride, cache, block_table, max_pages, q_start, ctx_len, req_list, n_req, nh, nkvh, page, scale, window, n_splits, part_o, part_ml, stream SCORE_ARGS)
+#define GO(D) return launch_decode<D>(q, q_stride, out, out_stride, cache, block_table, max_pages, q_start, ctx_len, req_list, n_req, nh, nkvh, page, scale, window, n_splits, few_keys, part_o, part_ml, stream SCORE_ARGS)
     if (dh == 128) GO(128);
     if (dh == 64) GO(64);
     if (dh == 96) GO(96);
     if (dh == 32) GO(32);
 #undef GO
     return LCU_UNSUPPORTED;
+}
+
+LCU_API int lcu_attention_decode_bf16(const void *q, int q_stride, void *out, int out_stride, const void *cache,
+                                      const int *block_table, int max_pages, const int *q_start, const int *ctx_len,
+                                      const int *req_list, int n_req, int nh, int nkvh, int dh, int page, float scale,
+                                      int window, int n_splits, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
+    return lcu_attention_decode_lengths_bf16(q, q_stride, out, out_stride, cache, block_table, max_pages, q_start, ctx_len, req_list, n_req, nh, nkvh, dh, page,
+                                             scale, window, n_splits, 0, part_o, part_ml, stream SCORE_ARGS);
 }
 
 // ---------------------------------------------------------------------------- no allocation

@@ -36,7 +36,7 @@ HOST_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-pthread", "-ff
 HIP_FLAGS += os.environ.get("LCU_HIP_FLAGS", "").split()
 
 KERNEL_LIBRARIES = ["elementwise", "rope_kv", "attention_generic", "attention_mfma", "attention_mfma_bias", "attention_mfma_cap", "gemm_generic", "gemm_skinny",
-                    "gemm_mid", "gemm_wavek", "sampling", "random_fill", "norm_conv", "qk_norm", "delta_rule", "moe", "norm_post", "qkv_prepare",
+                    "gemm_mid", "gemm_wavek", "gemm_tiles", "sampling", "random_fill", "norm_conv", "qk_norm", "delta_rule", "moe", "norm_post", "qkv_prepare",
                     "retention", "rglru", "latent", "causal_conv", "selective_scan", "wkv", "head_mix", "streams", "decay_scan", "step_arrays"]
 HOST_LIBRARY = "host"
 

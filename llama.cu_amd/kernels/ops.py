@@ -492,11 +492,12 @@ def _attention_library(head_slopes=None, softcap: float = 0.0):
 
 def attention_decode(q, out, cache, block_table, q_start, ctx_len, n_req, n_heads, n_kv_heads, head_dim, page_size,
                      scale, window, n_splits, req_list: Optional[torch.Tensor] = None,
-                     head_slopes: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, softcap: float = 0.0) -> torch.Tensor:
+                     head_slopes: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, softcap: float = 0.0,
+                     few_keys: bool = False) -> torch.Tensor:
     """Matrix-core attention for requests that feed one token each: all ``n_req`` requests of
     the batch, or the ``n_req`` whose indices ``req_list`` holds.  ``head_slopes``: the bias on the distance inside
     the scores (the kernels of the second library, ``attention_mfma_bias``); ``softcap``: a cap on them (the third,
-    ``attention_mfma_cap``)."""
+    ``attention_mfma_cap``).  ``few_keys``: no request has many (``decode_few_keys``)."""
     if req_list is not None:
         _i32(req_list, "req_list", n_req)
     part_o = part_ml = None
@@ -505,10 +506,10 @@ def attention_decode(q, out, cache, block_table, q_start, ctx_len, n_req, n_head
         part_ml = torch.empty(n_req * n_heads * n_splits * 2, dtype=torch.float32, device=q.device)
     lib = build.load(_attention_library(head_slopes, softcap))
     more = (_ptr(head_slopes), _ptr(sinks)) if head_slopes is not None else (ctypes.c_float(softcap),) if softcap else ()
-    _check(lib.lcu_attention_decode_bf16(_ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(cache), _ptr(block_table),
+    _check(lib.lcu_attention_decode_lengths_bf16(_ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(cache), _ptr(block_table),
                                          block_table.shape[1], _ptr(q_start), _ptr(ctx_len), _ptr(req_list), n_req, n_heads,
                                          n_kv_heads,
-                                         head_dim, page_size, ctypes.c_float(scale), int(window), int(n_splits),
+                                         head_dim, page_size, ctypes.c_float(scale), int(window), int(n_splits), int(bool(few_keys)),
                                          _ptr(part_o), _ptr(part_ml), _stream(), *more), "attention_decode")
     return out
 
@@ -576,13 +577,13 @@ class AttentionPlan:
     prefill kernel's tasks (``task_req``, ``task_tok0``; ``n_tasks`` on the device says how many).  The launches' sizes
     (``max_tasks``, ``n_single``, ``single_splits``) follow from the step's sizes and the longest context rounded up to
     a power of two; what the lists hold is data."""
-    __slots__ = ("task_req", "task_tok0", "n_tasks_dev", "max_tasks", "per_wg", "singles", "n_single", "single_splits")
+    __slots__ = ("task_req", "task_tok0", "n_tasks_dev", "max_tasks", "per_wg", "singles", "n_single", "single_splits", "single_few_keys")
 
     @property
     def signature(self):
         """What fixes the launches that ``paged_attention`` makes with this plan: two steps with equal signatures are
         served by the same recorded launches."""
-        return (self.max_tasks, self.per_wg, self.n_single, self.single_splits)
+        return (self.max_tasks, self.per_wg, self.n_single, self.single_splits, self.single_few_keys)
 
 
 def plan_attention(step, n_heads: int, n_kv_heads: int, window: int = 0, biased: bool = False, capped: bool = False) -> Optional[AttentionPlan]:
@@ -610,6 +611,7 @@ def plan_attention(step, n_heads: int, n_kv_heads: int, window: int = 0, biased:
     # the most tasks that a step of these sizes can have: a request of q tokens has at most q / tpt + 1
     plan.max_tasks = (step.n - len(singles)) // tpt + (step.n_req - len(singles))
     plan.single_splits = decode_splits(len(singles), n_heads, n_kv_heads, max([step.ctx_lens[r] for r in singles], default=0)) if singles else 1
+    plan.single_few_keys = decode_few_keys(max([step.ctx_lens[r] for r in singles], default=0))
     builder = getattr(step, "builder", None)
     if builder is not None:
         cap_tasks = builder.max_tokens // tpt + builder.max_reqs
@@ -663,6 +665,11 @@ def decode_splits(n_req: int, n_heads: int, n_kv_heads: int, max_ctx_len: int) -
     return 1 + next(i for i, f in enumerate(fill) if f >= max(fill) - t.decode_fill_slack)
 
 
+def decode_few_keys(max_ctx_len: int) -> bool:
+    """Whether a step's requests have so few keys that the decode kernel's workgroups are as fast or faster with half the waves: up to ``TUNING.decode_few_keys``."""
+    return int(max_ctx_len) <= TUNING.decode_few_keys
+
+
 _zeros: Dict = {}
 
 
@@ -713,13 +720,14 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, cache: torch.Tensor, ste
         # batch says which they are (64 requests of 150 to 2,200 keys: the step 11.2 -> 11.0 ms)
         return attention_decode(q, out, cache, bt, step.q_start, step.ctx_len, step.n_req, n_heads, n_kv_heads, head_dim,
                                 page_size, scale, window, splits, req_list=step.decode_order, head_slopes=head_slopes, sinks=sinks,
-                                softcap=softcap)
+                                softcap=softcap, few_keys=decode_few_keys(step.max_ctx_len) if step.attn_few_keys is None else step.attn_few_keys)
     # a mixed batch: the requests that decode one token go to the decode kernel, the portions
     # to the prefill kernel (each would be slow at the other's work)
     plan = plan_attention(step, n_heads, n_kv_heads, window, biased=second, capped=bool(softcap))
     if plan.n_single:
         attention_decode(q, out, cache, bt, step.q_start, step.ctx_len, plan.n_single, n_heads, n_kv_heads, head_dim, page_size,
-                         scale, window, plan.single_splits, req_list=plan.singles, head_slopes=head_slopes, sinks=sinks, softcap=softcap)
+                         scale, window, plan.single_splits, req_list=plan.singles, head_slopes=head_slopes, sinks=sinks, softcap=softcap,
+                         few_keys=plan.single_few_keys)
     if plan.max_tasks:
         attention_prefill(q, out, cache, bt, step.q_start, step.ctx_len, plan.task_req, plan.task_tok0, plan.max_tasks,
                           plan.per_wg, n_heads, n_kv_heads, head_dim, page_size, scale, window, n_tasks_dev=plan.n_tasks_dev,
@@ -989,6 +997,55 @@ def gemm_wavek(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = N
                               _ptr(gate), gate.stride(0) if gate is not None else 0, m, n, k, epi, int(wavek_wide(n)),
                               _ptr(row_sumsq), row_sumsq.shape[1] if row_sumsq is not None else 0, int(norm_width), ctypes.c_float(eps),
                               ctypes.c_float(act_alpha), ctypes.c_float(act_limit), _stream()), "gemm_wavek")
+    return out
+
+
+TILES = ((128, 128), (128, 256), (256, 256))      # features x tokens of the shapes of gemm_tiles
+
+
+def tiles_choice(m: int, n: int, k: int, swiglu: bool = False) -> int:
+    """The shape of ``gemm_tiles`` for a product of many bfloat16 rows where it is faster than the library's (and, with SwiGLU, than that and the activation kernel),
+    else -1.  It is where its workgroups fill more than half of a round and, mostly, no more than one (measured from 200 to 4,000 rows, 1024 x 1024 to 28672 x 4096;
+    the numbers are ``TUNING``'s)."""
+    t = TUNING
+    if m <= t.tiles_rows or k % 64 or n % 64 or (swiglu and k > t.tiles_swiglu_k):
+        return -1
+    cu, columns = t.compute_units, (n + 127) // 128
+    square = (m + 127) // 128 * columns
+    if square <= cu:
+        return 0 if 2 * square > cu else -1
+    wide = (m + 255) // 256 * columns
+    if swiglu:
+        return 1 if wide <= cu else 2 if (m + 255) // 256 * ((n + 255) // 256) <= cu else -1
+    return 1 if 8 * wide <= 5 * cu and k <= t.tiles_short_k else -1
+
+
+def tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_tiles`` takes these rows and this plain weight."""
+    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.stride(1) == 1 and w.is_contiguous()
+            and x.shape[1] % 64 == 0 and w.shape[0] % 16 == 0 and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (x.shape[0] + 256) * x.stride(0) < 1 << 31 and (w.shape[0] + 256) * w.shape[1] < 1 << 31)
+
+
+def gemm_tiles(x: torch.Tensor, w: torch.Tensor, shape: int, out: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None, swiglu: bool = False,
+               act_alpha: float = 1.0, act_limit: float = 0.0, known: bool = False) -> torch.Tensor:
+    """``x @ w.T`` for many bfloat16 rows, ``w [n, k]`` plain; ``shape``: see ``TILES``.  ``out [m, n]`` bfloat16 or float32; ``swiglu``: ``w`` holds gate rows, then up rows,
+    ``out [m, n / 2]`` bfloat16 (the limited activation with ``act_limit`` > 0).  ``known``: the caller has asked ``tiles_supported``."""
+    if not known:
+        _gpu(x, w, out)
+    if not 0 <= shape < len(TILES) or not (known or tiles_supported(x, w)):
+        raise KernelError(f"gemm_tiles: x {tuple(x.shape)} {x.dtype} with w {tuple(w.shape)} {w.dtype} is not supported")
+    m, k = x.shape
+    n = w.shape[0]
+    dtype, cols = out.dtype if out is not None else (out_dtype or torch.bfloat16), n // 2 if swiglu else n
+    fresh = out is None
+    if fresh:
+        out = torch.empty((m, cols), dtype=dtype, device=x.device)
+    if dtype not in (torch.bfloat16, torch.float32) or (swiglu and dtype != torch.bfloat16) \
+            or (fresh and cols % 8) or (not fresh and (out.shape != (m, cols) or out.stride(1) != 1 or out.stride(0) * out.element_size() % 16 or out.data_ptr() % 16)):
+        raise KernelError(f"gemm_tiles out: {out.dtype} {tuple(out.shape)} with strides {out.stride()} is not supported")
+    _check(build.load("gemm_tiles").lcu_gemm_tiles(_ptr(x), x.stride(0), _ptr(w), _ptr(out), out.stride(0), m, n, k, 2 if swiglu else 1 if dtype == torch.float32 else 0,
+                                                   int(shape), ctypes.c_float(act_alpha), ctypes.c_float(act_limit), _stream()), "gemm_tiles")
     return out
 
 

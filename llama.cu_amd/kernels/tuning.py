@@ -96,6 +96,14 @@ class Tuning:
                                         # 28.2, 30.2, 32.0 against 32.6, 31.0, 35.1; 24 heads, K = 512: 6.1, 6.4, 7.2 against 6.2, 6.3, 7.5, K = 2048: 10.5, 10.9, 12.3
                                         # against 10.7, 10.5, 12.6; 8 heads of 64, K = 8192: 21.8, 23.4, 26.6 against 27.8, 27.8, 31.2; measured for 8 to 64 heads); 15.5
                                         # against 14.8 at 24 rows, 48 heads, K = 4096
+    # ---- the product of many rows in tiles (gemm_tiles.hip), us of the library's and of it
+    tiles_rows: int = 256               # above so many rows (fewer have kernels of their own)
+    tiles_swiglu_k: int = 2048          # SwiGLU with a longer K stays with the library (28672 x 4096: 83 and 95 at 300 rows, 290 and 306 at 1,500; 5632 x 2048 51.8 and 49.3
+                                        # there, 59.7 and 52.4 at 2,014; 2816 x 1024 26.3 and 18.8)
+    tiles_short_k: int = 2048           # a round of 128 x 256 up to five eighths full only with a K up to this (4096 x 2048, 1,100 rows: 27.0 and 24.3; 2560 x 2048, 2,014: 27.8 and
+                                        # 25.0; 4096 x 4096, 1,100: 42.6 and 42.8)
+                                        # (a fuller round, with any K, is no gain in a whole prompt, where the card's power limit lets every kernel pay for another's work: 4096 x
+                                        # 14336, 2,048 rows, 210 and 196 alone, 225 and 204 inside an 8-layer prompt of the 8B shape, which takes 6.79 and 6.85 ms)
     # ---- the library's product of many rows (parts/linear.library_friendly_rows)
     library_rows: int = -1              # rows of zeros behind each half of a plain gate/up matrix: -1 times the library once per
                                         # shape at load and fills up where that is 15 % faster (the outcome can differ from box
@@ -103,6 +111,7 @@ class Tuning:
     # ---- the decode attention's cut of a request's keys into parts (attention_mfma.hip)
     decode_min_part_keys: int = 512     # a part of so many keys; up to 512 keys one part
     decode_max_parts: int = 32
+    decode_few_keys: int = 128          # up to so many keys, which four waves take in one step each, a workgroup has four waves, beyond eight (attention_mfma.hip)
     decode_few_parts: int = 8           # ... beyond them up to so many parts, however short (of at least 64 keys: 513 are taken for 1,024).  One MI355X, us with its second
                                         # kernel, 16 heads over 4, 1 / 2 / 4 / 8 parts: 4 requests of 1,000 keys 12.6, 10.9, 8.9, 7.5, 8 of 1,000 13.8, 11.6, 9.3, 8.3, 1 of 2,000
                                         # 18.6, 11.1, 9.2, 7.7; 500 keys 4 requests 6.6, 7.8, 6.8, 6.7, 8 requests 8.7, 8.9, 7.7, 7.3, of 300 6.6, 7.7, 7.1

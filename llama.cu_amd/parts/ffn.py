@@ -16,7 +16,7 @@ from ..kernels import ops
 from .base import BuildContext, Part, ScaledRows, TensorSpec, register_part
 from ..weights.loader import fused_rows
 from .linear import (Weight, end_in_norm, f32_takes_scaled_rows, library_friendly_rows, linear, linear_planes, linear_swiglu,
-                     linear_swiglu_mid, mid_swiglu_takes, mid_takes, skinny_row_limit, skinny_takes, wavek_swiglu_takes)
+                     linear_swiglu_mid, mid_swiglu_takes, mid_takes, skinny_row_limit, skinny_takes, tiles_swiglu_shape, wavek_swiglu_takes)
 
 
 class SwiGLU(Part):
@@ -126,6 +126,8 @@ class SwiGLU(Part):
               and ops.skinny_supported(h, self.w_gate_up.plain, self.dtype)):
             # few rows: one pass over the weights, the activation in the product's epilogue
             act = linear_swiglu(h, self.w_gate_up, **self.act)
+        elif (shape := tiles_swiglu_shape(h, self.w_gate_up)) >= 0:
+            act = ops.gemm_tiles(h, self.w_gate_up.plain, shape, swiglu=True, known=True, **self.act)
         else:
             gu = linear(h, self.w_gate_up, out_dtype=self.dtype)
             act = ops.swiglu(gu, activation=self.activation, alpha=self.alpha, limit=self.limit)

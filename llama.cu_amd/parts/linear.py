@@ -3,7 +3,8 @@
 Which routine multiplies is decided here and nowhere else:
 
 * bfloat16 activations and weights: few rows (decoding) go to the hand-written
-  weight-streaming kernel, many rows to the library's matrix product (hipBLASLt through
+  weight-streaming kernel, many rows to the hand-written product in tiles where that is the faster one
+  (``ops.tiles_choice``), else to the library's matrix product (hipBLASLt through
   torch, with bfloat16 or, for logits, float32 output), as the reference's engine calls
   its vendor library (llama.cu/src/op/linear.rs:91-118);
 * all float32 (the true 32-bit path): the hand-written weight-streaming kernel on the
@@ -83,6 +84,10 @@ def linear(x: torch.Tensor, weight: Union[torch.Tensor, Weight], out_dtype: Opti
         if packed is not None:
             return ops.gemm_skinny(x, packed, out=out, out_dtype=out_dtype, accumulate=accumulate, packed=True)
         return ops.gemm_skinny(x, weight, out=out, out_dtype=out_dtype, accumulate=accumulate)
+    if all_bf16 and x.shape[0] > ops.TUNING.tiles_rows and not accumulate and x.dim() == 2 and out_dtype in (torch.bfloat16, torch.float32):
+        shape = ops.tiles_choice(x.shape[0], weight.shape[0], weight.shape[1])
+        if shape >= 0 and ops.tiles_supported(x, weight) and (out is None or _plain_rows(out) and out.stride(0) * out.element_size() % 16 == 0):
+            return ops.gemm_tiles(x, weight, shape, out=out, out_dtype=out_dtype, known=True)
     if all_bf16 and out_dtype == torch.bfloat16 and not accumulate:
         if out is None:
             return torch.matmul(x, weight.t())
@@ -109,6 +114,15 @@ def linear_swiglu(h, weight: Union[torch.Tensor, Weight], row_sumsq=None, norm_w
     if packed is not None:
         return ops.gemm_skinny(h, packed, swiglu=True, packed=True, **kw)
     return ops.gemm_skinny(h, weight, swiglu=True, **kw)
+
+
+def tiles_swiglu_shape(h: torch.Tensor, weight: Union[torch.Tensor, Weight]) -> int:
+    """The shape of the product in tiles that takes these rows with SwiGLU in its epilogue, or -1 (``ops.tiles_choice``)."""
+    if h.shape[0] <= ops.TUNING.tiles_rows or h.dim() != 2:
+        return -1
+    w = _split(weight)[0]
+    shape = ops.tiles_choice(h.shape[0], w.shape[0], w.shape[1], swiglu=True)
+    return shape if shape >= 0 and ops.tiles_supported(h, w) else -1
 
 
 def wavek_swiglu_takes(h: torch.Tensor, weight: Union[torch.Tensor, Weight]) -> bool:

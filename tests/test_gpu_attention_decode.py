@@ -50,3 +50,5 @@ def test_rows_waves_and_pages(nh, nkv, dh, page, splits):
     ops.paged_attention_generic(q, wanted, cache, table, starts, lens, of, nh, nkv, dh, page, dh ** -0.5, 0)
     ops.attention_decode(q, got, cache, table, starts, lens, n, nh, nkv, dh, page, dh ** -0.5, 0, splits)
     assert_close(got, wanted, 3 * 2.0 ** -8, "against the generic kernel")        # the weights and both outputs rounded to bfloat16
+    ops.attention_decode(q, got.fill_(float("nan")), cache, table, starts, lens, n, nh, nkv, dh, page, dh ** -0.5, 0, splits, few_keys=True)
+    assert_close(got, wanted, 3 * 2.0 ** -8, "four waves, however many keys")

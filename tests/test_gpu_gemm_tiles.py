@@ -1,0 +1,79 @@
+"""The product of many rows in tiles, against 64 bits: every shape of tile at edges of tiles, of the rings and of the rows, with each epilogue."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from divasun_common import assert_close
+from test_gpu_divasun import rnd
+
+pytestmark = pytest.mark.gpu
+
+BF16_REL = 2.0 ** -8            # one rounding of the result, and the largest of the 32-bit sums' errors far below it
+
+
+# fewer steps of K than a ring holds, as many, and more; one row, a tile less one and more, several tiles; features that end within a tile
+@pytest.mark.parametrize("shape", [0, 1, 2])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (127, 80, 128), (129, 208, 192), (257, 400, 256), (300, 1040, 320), (511, 16, 1088), (33, 2112, 704)])
+def test_tiles(shape, m, n, k):
+    from llama_cu_amd.kernels import ops
+    x, w = rnd(m, k + 24, seed=1).bfloat16().cuda()[:, 8:8 + k], rnd(n, k, seed=2, std=k ** -0.5).bfloat16().cuda()
+    want = x.double() @ w.double().T
+    assert_close(ops.gemm_tiles(x, w, shape), want, BF16_REL, "bfloat16")
+    assert_close(ops.gemm_tiles(x, w, shape, out_dtype=torch.float32), want, 1e-5, "float32")
+    room = torch.full((m + 1, n + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.gemm_tiles(x, w, shape, out=room[:m, :n])
+    assert torch.equal(room[:m, :n], ops.gemm_tiles(x, w, shape)) and (room[m:] == 7).all() and (room[:, n:] == 7).all()
+    for limit in (0.0, 0.8):
+        g, u = want.chunk(2, 1)
+        act = g * torch.sigmoid(g) * u
+        if limit:
+            g, u = torch.clamp(g, max=limit), torch.clamp(u, -limit, limit)
+            act = g * torch.sigmoid(1.7 * g) * (u + 1.0)
+        got = ops.gemm_tiles(x, w, shape, swiglu=True, **(dict(act_alpha=1.7, act_limit=limit) if limit else {}))
+        assert_close(got, act, BF16_REL, f"swiglu, limit {limit}")
+
+
+def test_rows_and_features_know_nothing_of_each_other():
+    """A row of NaN and a feature of infinities reach their own row and column only; rows that hold more than the operands' K, and what lies behind the last row, are not
+    looked at."""
+    from llama_cu_amd.kernels import ops
+    m, n, k = 200, 144, 128
+    wide = rnd(m, 2 * k, seed=1).bfloat16()
+    wide[:, k:] = float("nan")
+    wide[70, :k] = float("nan")
+    w = rnd(n, k, seed=2).bfloat16()
+    w[9] = float("inf")
+    for shape in range(3):
+        y = ops.gemm_tiles(wide.cuda()[:, :k], w.cuda(), shape).float().cpu()
+        good = torch.ones(m, n, dtype=torch.bool)
+        good[70] = False
+        good[:, 9] = False
+        assert torch.isfinite(y[good]).all() and torch.isnan(y[70]).all() and not torch.isfinite(y[:, 9]).any()
+
+
+@pytest.mark.parametrize("m,n,k", [(2014, 2560, 2048), (1100, 2048, 2048), (2014, 5632, 2048)])
+def test_the_products_that_the_rule_names(m, n, k):
+    """What ``linear`` computes where ``tiles_choice`` names a shape, and the choice itself at its edges."""
+    from llama_cu_amd.kernels import ops
+    from llama_cu_amd.parts.linear import linear
+    swiglu = n == 5632
+    shape = ops.tiles_choice(m, n, k, swiglu)
+    assert shape >= 0 and ops.tiles_choice(ops.TUNING.tiles_rows, n, k, swiglu) == -1 and ops.tiles_choice(m, n, k + 8, swiglu) == -1
+    x, w = rnd(m, k, seed=1).bfloat16().cuda(), rnd(n, k, seed=2, std=k ** -0.5).bfloat16().cuda()
+    if swiglu:
+        g, u = (x.double() @ w.double().T).chunk(2, 1)
+        assert_close(ops.gemm_tiles(x, w, shape, swiglu=True), g * torch.sigmoid(g) * u, BF16_REL, "swiglu")
+        return
+    assert torch.equal(linear(x, w), ops.gemm_tiles(x, w, shape))
+    assert_close(linear(x, w), x.double() @ w.double().T, BF16_REL, "linear")
+
+
+def test_what_is_refused():
+    from llama_cu_amd.kernels import ops
+    x, w = rnd(40, 128, seed=1).bfloat16().cuda(), rnd(64, 128, seed=2).bfloat16().cuda()
+    for bad in (lambda: ops.gemm_tiles(x, w, 3), lambda: ops.gemm_tiles(x.float(), w, 0), lambda: ops.gemm_tiles(x[:, :96], w[:, :96].contiguous(), 0),
+                lambda: ops.gemm_tiles(x, w[:40], 0), lambda: ops.gemm_tiles(x[:, 1:65], w[:, :64].contiguous(), 0),
+                lambda: ops.gemm_tiles(x, w, 0, out=torch.empty(40, 66, dtype=torch.bfloat16, device="cuda")[:, 1:65])):
+        with pytest.raises(ops.KernelError):
+            bad()

@@ -19,7 +19,7 @@ OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 # instruction: wait states before its result may be read or overwritten by anything but the next sum in the same registers; what the
 # compiler leaves where no branch lies between, 4 and 8 passes of bfloat16, 8 of 32-bit and 16 of 64-bit
 WAITS = {"v_mfma_f32_16x16x32_bf16": 8, "v_mfma_f32_32x32x16_bf16": 12, "v_mfma_f32_16x16x4_f32": 10, "v_mfma_f64_16x16x4_f64": 19}
-LIBRARIES = ["attention_mfma", "attention_mfma_bias", "attention_mfma_cap", "decay_scan", "delta_rule", "gemm_mid", "gemm_skinny", "gemm_wavek", "moe", "rglru"]
+LIBRARIES = ["attention_mfma", "attention_mfma_bias", "attention_mfma_cap", "decay_scan", "delta_rule", "gemm_mid", "gemm_skinny", "gemm_tiles", "gemm_wavek", "moe", "rglru"]
 
 _REG = re.compile(r"\b([va])(?:\[(\d+):(\d+)\]|(\d+))")
 _LINE = re.compile(r"^\s+(\w+)\s*(.*?)\s*//\s*([0-9A-Fa-f]+):")
