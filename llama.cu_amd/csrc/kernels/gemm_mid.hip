@@ -21,7 +21,8 @@
 //     output, [slice][M][N], and the kernel that follows (residual sum and norm) adds the planes
 //     in a fixed order.  Nothing is added atomically: results do not depend on timing.
 //
-// A second kernel (gemm_mid_qkv_kernel, below) is the q, k, v product with the rotation and the cache write
+// Packed weights that are cut over K, and gate/up beyond 64 rows, have a kernel without producers up to 128 rows (gemm_mid_ring_kernel, below).
+// A further kernel (gemm_mid_qkv_kernel, below) is the q, k, v product with the rotation and the cache write
 // in its epilogue: there the consumer waves share each macro-step of K instead of the features.
 //
 // W is plain rows or packed as gemm_skinny.hip describes it (16 x 128 blocks of 4 KB).  (The reference
@@ -312,6 +313,183 @@ gemm_mid_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict_
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// Packed weights with up to 128 rows: the products that are cut over K (and the uncut one with 32-bit output), and gate/up beyond 64 rows.  The kernel above
+// keeps eight tiles of W in flight a wave, but X comes to LDS through the registers of one producer for 64 rows, and it is this wave's round trips
+// (load, store, barrier) that the others wait for: at 64 rows of the 4096 x 14336 down projection 28.5 us, 4.1 TB/s.  Here X comes by loads that go straight
+// to LDS, each wave asks for a quarter of it, and nobody produces:
+//   * four waves a workgroup, each with its own tile of 16 features (SwiGLU: a gate and an up tile).  Macro-step s of K (128 k): W in registers, asked for D
+//     steps ahead; X in slot s % D of a ring in LDS, asked for D - 1 steps ahead, one step after its W (a slot is free only once every wave has passed
+//     the barrier after its last read).  A wave's loads come back in order, so each step waits for a count: all but the younger steps' loads;
+//   * a slot holds, for each 16 rows, four KB pieces: piece i has rows 4 i .. 4 i + 3 (wave i asks for it), lane 16 g + 4 a + p of the load k = 32 g + 8 (p ^ swizzle) of
+//     row 4 i + a.  A load writes its lanes' 16 bytes one after the other, so the lane chooses what it asks for: the swizzle spreads the 16 rows that an
+//     operand's read takes over all banks, and the four lanes of a row and group still read one 64-byte piece;
+//   * the order of the sums is the one of the kernel above: the same bits.
+// D = 3; with more workgroups than compute units D = 2 (from 33 rows on), which leaves LDS for several on each: 50,304 x 2048 at 121 rows 57 against 64 us.  With
+// up to 32 rows D = 3 fits several times (128,256 x 4096 at 24 rows 182 against 193 us).
+// What bounds it: at 64 rows a unit's share of 14336 x 4096 in four slices is 459 KB of W and 459 of X, in 24.0 us 38 bytes a ns: the rate at which
+// a compute unit reads.  Measured, weights out of memory, this kernel and the one above: 4096 x 14336, four slices, 32 / 64 / 121 rows: 21.2 / 24.0 / 31.0 us against
+// 22.4 / 28.5 / 36.4; 4096 x 4096 9.7 / 10.7 / 13.5 against 10.6 / 13.4 / 17.2; 2048 x 2816 at 64 / 121 rows 6.8 / 9.0 against 8.4 / 11.5; the uncut 128,256 x 4096
+// at 48 / 64 rows 201 / 211 against 210 / 233.  SwiGLU, 28,672 x 4096 at 121 rows: 48.6 against 51.9; 16,384 x 2048 22.3 against 26.1; up to 64 rows it is no faster
+// (43.7 against 43.2) and stays there.
+constexpr int RING_WAVES = 4;
+
+template <int LEFT>
+__device__ __forceinline__ void ring_wait_loads() {
+    static_assert(LEFT >= 0 && LEFT < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((LEFT & 15) | ((LEFT >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// One macro-step: asks for a later one's X (into `free_slot`, which every wave has read) and multiplies this one's.  A function of its own with both slots
+// restrict: otherwise the compiler takes the loads to LDS for writes that the reads after them must wait for.
+template <int NT, int MT>
+__device__ __forceinline__ void ring_step(const u32x4 *__restrict__ slot, u32x4 *__restrict__ free_slot, const __amdgpu_buffer_rsrc_t xb, const uint32_t (&src)[MT],
+                                          uint32_t step_bytes, uint32_t none, int wave, const int (&at)[4], const u32x4 (&w)[NT][4], f32x4 (&acc)[NT][MT]) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        auto *to = (__attribute__((address_space(3))) void *)(free_slot + (m * RING_WAVES + wave) * WAVE);
+        const uint32_t from = (src[m] + step_bytes) | none;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xb, to, 16, from, 0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        u32x4 x[MT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) x[m] = slot[at[j] + m * RING_WAVES * WAVE];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[t][m] = mid_mfma(w[t][j], x[m], acc[t][m]);
+    }
+}
+
+template <int MT, int EPI, int D>
+__global__ void __launch_bounds__(RING_WAVES * WAVE, 1)
+gemm_mid_ring_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict__ W, void *__restrict__ Y, int ldy, int M, int N, int K, int steps_per_slice,
+                     const float *__restrict__ sumsq_in, int n_in, int norm_width, float eps, float act_alpha, float act_limit) {
+    static_assert(EPI == MID_EPI_SWIGLU || EPI == MID_EPI_PARTIAL_F32, "what the kernel is chosen for");
+    extern __shared__ __attribute__((aligned(16))) char xs[];      // the ring of X, then the rows' factors
+    constexpr int NT = EPI == MID_EPI_SWIGLU ? 2 : 1, SLOT = MT * RING_WAVES * WAVE, W_LOADS = 4 * NT;
+    u32x4 *ring = (u32x4 *)xs;
+    float *row_scale = (float *)(ring + D * SLOT);
+    const int lane = threadIdx.x & (WAVE - 1), l16 = lane & 15, grp = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int steps_total = K / 128, s_begin = blockIdx.y * steps_per_slice, nst = min(steps_total, s_begin + steps_per_slice) - s_begin;
+    const int n_tiles = (EPI == MID_EPI_SWIGLU ? N / 2 : N) / 16;
+    const int tile0 = (int)((long long)blockIdx.x * n_tiles / gridDim.x) + wave;
+    const bool live = tile0 < (int)((long long)(blockIdx.x + 1) * n_tiles / gridDim.x);   // a wave without a tile asks for its quarter of X and stores nothing
+    // buffer resources that end with the slice: what lies beyond reads zeros
+    __amdgpu_buffer_rsrc_t wb[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int tile = (live ? tile0 : n_tiles - 1) + t * n_tiles;
+        wb[t] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(W + ((size_t)tile * steps_total + s_begin) * 2048), 0, live ? (uint32_t)nst * 4096u : 0u, 0x00020000);
+    }
+    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t *>(X + (size_t)128 * s_begin), 0, (uint32_t)(((size_t)(M - 1) * ldx + 128 * nst) * 2), 0x00020000);
+    uint32_t src[MT];                                  // rows from M on lie beyond the end
+    {
+        const int a = (lane >> 2) & 3, p = lane & 3, swizzle = (a >> 1) + 2 * (wave & 1);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int row = 16 * m + 4 * wave + a;
+            src[m] = row < M ? (uint32_t)(row * ldx + 32 * grp + 8 * (p ^ swizzle)) * 2u : 0x80000000u;
+        }
+    }
+    int at[4];                                         // where the operand of row l16, instruction j, lies in a slot's 16 rows
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int i = l16 >> 2, a = l16 & 3;
+        at[j] = i * WAVE + grp * 16 + a * 4 + (j ^ ((a >> 1) + 2 * (i & 1)));
+    }
+    // the rows' factors, as in the kernel above (these loads are the oldest: the counts below hold with them)
+    const bool scales = sumsq_in != nullptr && wave < MT;
+    float scale_ss = 0.f;
+    if (scales) {
+        const int tok = 16 * wave + l16;
+        const float *sh = sumsq_in + (size_t)(tok < M ? tok : 0) * n_in;
+        if ((n_in & 15) == 0) {
+            const int q4 = n_in / 16;
+            const f32x4 *p4 = (const f32x4 *)sh + grp * q4;
+            for (int i = 0; i < q4; i += 16) {
+                f32x4 v[16];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) v[e] = p4[i + e < q4 ? i + e : q4 - 1];
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (i + e < q4) scale_ss += (v[e][0] + v[e][1]) + (v[e][2] + v[e][3]);
+            }
+        } else {
+            for (int i = grp; i < n_in; i += 4) scale_ss += sh[i];
+        }
+    }
+    u32x4 w[D][NT][4];
+    f32x4 acc[NT][MT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#define RING_LOAD_W(i, step)                                                                                    \
+    _Pragma("unroll") for (int t = 0; t < NT; ++t) _Pragma("unroll") for (int j = 0; j < 4; ++j) w[i][t][j] =  \
+        __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wb[t], (uint32_t)lane * 16u + (uint32_t)(step) * 4096u + 1024u * j, 0, MID_STREAM))
+#pragma unroll
+    for (int s = 0; s < D; ++s) {
+        if (s > 0) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                auto *to = (__attribute__((address_space(3))) void *)(ring + (s - 1) * SLOT + (m * RING_WAVES + wave) * WAVE);
+                const uint32_t from = (src[m] + (uint32_t)(s - 1) * 256u) | (s - 1 < nst ? 0u : 0x80000000u);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xb, to, 16, from, 0, 0, 0);
+            }
+        }
+        RING_LOAD_W(s, s);
+    }
+    if (scales) {
+        scale_ss += __shfl_xor(scale_ss, 16, WAVE);
+        scale_ss += __shfl_xor(scale_ss, 32, WAVE);
+        if (grp == 0) row_scale[16 * wave + l16] = rsqrtf(scale_ss / (float)norm_width + eps);
+    }
+    for (int s0 = 0; s0 < nst; s0 += D) {
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            const int s = s0 + i;
+            if (s >= nst) break;
+            // younger than this step's X: the W of D - 1 steps and the X of D - 2
+            ring_wait_loads<(D - 1) * W_LOADS + (D - 2) * MT>();
+            lds_barrier();
+            ring_step<NT, MT>(ring + i * SLOT, ring + (i == 0 ? D - 1 : i - 1) * SLOT, xb, src, (uint32_t)(s + D - 1) * 256u, s + D - 1 < nst ? 0u : 0x80000000u, wave, at, w[i], acc);
+            RING_LOAD_W(i, s + D);
+        }
+    }
+#undef RING_LOAD_W
+    ring_wait_loads<0>();                              // nothing of this workgroup is on its way to LDS when it ends
+    if (!live) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        // the lane holds, per tile, features 4 grp + r of token 16 m + l16
+        const int tok = 16 * m + l16;
+        if (tok >= M) continue;
+        if (sumsq_in != nullptr) {                     // (the factors were written before the loop's barriers)
+            const float rs = row_scale[tok];
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[t][m][r] *= rs;
+        }
+        const int n = 16 * tile0 + 4 * grp;
+        if (EPI == MID_EPI_SWIGLU) {
+            float o[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = gate_up_of(acc[0][m][r], acc[NT - 1][m][r], act_alpha, act_limit);
+            uint2 pk = {pack2_bf16(o[0], o[1]), pack2_bf16(o[2], o[3])};
+            *(uint2 *)((bf16_t *)Y + (size_t)tok * ldy + n) = pk;
+        } else {
+            float *plane = (float *)Y + (size_t)blockIdx.y * M * ldy;
+            *(f32x4 *)(plane + (size_t)tok * ldy + n) = acc[0][m];
+        }
+    }
+}
+
 // The number of compute units of the current device (asked once per device).
 static int mid_compute_units() {
     static int units[64] = {};
@@ -366,10 +544,15 @@ static int mid_launch_c(const void *X, int ldx, const void *W, int ldw, void *Y,
             (const bf16_t *)X, ldx, (const bf16_t *)W, ldw, Y, ldy, M, N, K, per, sc.sumsq_in, sc.n_in, sc.norm_width, sc.eps,   \
             sc.act_alpha, sc.act_limit); \
     } while (0)
-#define GO_MT(MT_)                 \
-    do {                           \
-        if (packed) GO(MT_, true); \
-        else GO(MT_, false);       \
+    // packed rows that the ring kernel takes never come here
+#define GO_MT(MT_)                                                                          \
+    do {                                                                                    \
+        if constexpr (EPI == MID_EPI_BF16 || MT_ > 8 || (EPI == MID_EPI_SWIGLU && MT_ <= 4)) { \
+            if (packed) GO(MT_, true);                                                      \
+            else GO(MT_, false);                                                            \
+        } else {                                                                            \
+            GO(MT_, false);                                                                 \
+        }                                                                                   \
     } while (0)
     if constexpr (C < MID_CONSUMERS) {
         GO_MT(2);                                   // (chosen for up to 32 rows only)
@@ -397,6 +580,56 @@ static int mid_launch(const void *X, int ldx, const void *W, int ldw, void *Y, i
     return mid_launch_c<NT, EPI, MID_CONSUMERS>(X, ldx, W, ldw, Y, ldy, M, N, K, packed, slices, sc, stream);
 }
 
+// The ring kernel's rows (above): packed weights, up to 128 rows, SwiGLU beyond 64 of them.
+static bool mid_ring_takes(int M, int epi, int packed) {
+    return packed && M <= 128 && (epi == MID_EPI_PARTIAL_F32 || (epi == MID_EPI_SWIGLU && M > 64));
+}
+
+template <int EPI>
+static int mid_ring_launch(const void *X, int ldx, const void *W, void *Y, int ldy, int M, int N, int K, int slices, const MidScale &sc, hipStream_t stream) {
+    const int n_tiles = (EPI == MID_EPI_SWIGLU ? N / 2 : N) / 16, units = mid_compute_units();
+    const int steps = K / 128, per = (steps + slices - 1) / slices, planes = (steps + per - 1) / per;
+    int groups = (n_tiles + RING_WAVES - 1) / RING_WAVES;
+    // gate/up: the next multiple of the number of compute units (28,672 x 4096 at 96 rows as 256 workgroups 48.4, as 224 49.2 us; 22,016 x 4096 41.9 and 45.0)
+    if (EPI == MID_EPI_SWIGLU && units > 0) groups = min(n_tiles, (groups + units - 1) / units * units);
+    const dim3 grid(groups, planes);
+    const bool several = EPI == MID_EPI_PARTIAL_F32 && units > 0 && (long long)groups * planes > units;      // several workgroups for a unit: a ring of two
+#define GO(MT_, D_)                                                                                                            \
+    do {                                                                                                                       \
+        auto kernel = gemm_mid_ring_kernel<MT_, EPI, D_>;                                                                      \
+        constexpr int lds = D_ * MT_ * RING_WAVES * WAVE * 16 + 16 * MT_ * (int)sizeof(float);                                 \
+        if (lds > 64 * 1024) {                                                                                                 \
+            static bool asked = false;                                                                                         \
+            if (!asked) {                                                                                                      \
+                hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);    \
+                if (e != hipSuccess) return (int)e;                                                                            \
+                asked = true;                                                                                                  \
+            }                                                                                                                  \
+        }                                                                                                                      \
+        kernel<<<grid, dim3(RING_WAVES * WAVE), lds, stream>>>((const bf16_t *)X, ldx, (const bf16_t *)W, Y, ldy, M, N, K, per, \
+                                                               sc.sumsq_in, sc.n_in, sc.norm_width, sc.eps, sc.act_alpha, sc.act_limit); \
+    } while (0)
+#define GO_D(MT_)                   \
+    do {                            \
+        if (several) GO(MT_, 2);    \
+        else GO(MT_, 3);            \
+    } while (0)
+    if constexpr (EPI == MID_EPI_SWIGLU) {
+        if (M <= 96) GO(6, 3);
+        else GO(8, 3);
+    } else {
+        if (M <= 32) GO(2, 3);
+        else if (M <= 48) GO_D(3);
+        else if (M <= 64) GO_D(4);
+        else if (M <= 96) GO_D(6);
+        else GO_D(8);
+    }
+#undef GO_D
+#undef GO
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
+}
+
 // X: [M, K] bfloat16 rows ldx apart, M <= 256 (rows that wait for their normalisation: M <= 64); W: [N, K] bfloat16, rows ldw apart or packed; K a
 // multiple of 128, N of 16 (SwiGLU: of 32; W holds N/2 gate rows, then N/2 up rows).
 // epilogue MID_EPI_BF16: Y [M, N] bfloat16 rows ldy apart (slices must be 1);
@@ -422,9 +655,11 @@ static int mid_bf16(const void *X, int ldx, const void *W, int ldw, void *Y, int
         return mid_launch<1, MID_EPI_BF16>(X, ldx, W, ldw, Y, ldy, M, N, K, w_packed, 1, sc, stream);
     case MID_EPI_PARTIAL_F32:
         if (ldy < N || ldy % 4) return LCU_BAD_ARGUMENT;
+        if (mid_ring_takes(M, epilogue, w_packed)) return mid_ring_launch<MID_EPI_PARTIAL_F32>(X, ldx, W, Y, ldy, M, N, K, slices, sc, stream);
         return mid_launch<1, MID_EPI_PARTIAL_F32>(X, ldx, W, ldw, Y, ldy, M, N, K, w_packed, slices, sc, stream);
     case MID_EPI_SWIGLU:
         if (slices != 1 || N % 32 || ldy < N / 2 || ldy % 4) return LCU_BAD_ARGUMENT;
+        if (mid_ring_takes(M, epilogue, w_packed)) return mid_ring_launch<MID_EPI_SWIGLU>(X, ldx, W, Y, ldy, M, N, K, 1, sc, stream);
         return mid_launch<2, MID_EPI_SWIGLU>(X, ldx, W, ldw, Y, ldy, M, N, K, w_packed, 1, sc, stream);
     default: return LCU_BAD_ARGUMENT;
     }

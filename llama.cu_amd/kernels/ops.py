@@ -1060,7 +1060,7 @@ def gemm_mid(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
              slices: Optional[int] = None, packed: bool = False, row_sumsq: Optional[torch.Tensor] = None,
              norm_width: int = 0, eps: float = 0.0, act_alpha: float = 1.0, act_limit: float = 0.0) -> torch.Tensor:
     """``x @ w.T`` for up to 256 rows of bfloat16 ``x`` (chosen from 12 to 33 rows on, by the product), streaming ``w`` once while
-    the waves of a workgroup share ``x`` through LDS.  ``slices=None``: ``out [m, n]`` bfloat16
+    the waves of a workgroup share ``x`` through LDS (packed, up to 128 rows: loaded straight into it).  ``slices=None``: ``out [m, n]`` bfloat16
     (``swiglu``: ``w`` holds gate rows, then up rows, ``out [m, n/2] = silu(gate) * up``, or the limited activation with
     ``act_limit`` > 0).
     ``slices=s``: K is cut into (at most) ``s`` slices and ``out [planes, m, n]`` float32 holds

@@ -39,7 +39,7 @@ class Tuning:
     mid_swiglu_max_rows: int = 192      # ... up to this many (at 160 and 192 rows 57 and 61 us against the library's 62 and 66 with
                                         # the activation kernel: whole steps 4 and 6 % faster; at 256 rows 78 against 73)
     mid_long_k_max_rows: int = 256      # the products cut over K go to it up to this many rows with a long K (the down
-                                        # projection: 42 us against the library's 85 at 160 rows, 55 against 65 at 256)
+                                        # projection: 31 us at 121 rows, 42 against the library's 85 at 160, 55 against 65 at 256)
     mid_short_k_max_rows: int = 192     # ... and up to this many with a shorter one (the output projection: 19 us against 25 to
                                         # 28 at 160 to 192 rows, no gain beyond)
     mid_qkv_rows: int = 16              # q/k/v with the rotation and the cache write in its epilogue goes to it above this
@@ -55,8 +55,8 @@ class Tuning:
                                         # faster at 20 rows, 1.7 % at 32; 2 % slower at 16 and at 40 to 48, where the first product
                                         # of the feed-forward pays more for the rows' factors than the norm kernel cost
     mid_f32_rows: int = 32              # a product with 32-bit output (the output matrix, 1.05 GB) goes to it, uncut, above this many
-    mid_f32_max_rows: int = 64          # rows and up to this many (whole steps 1.3 % faster at 40 rows, 1.9 % at 48, 0.7 % at 64;
-                                        # nothing at 25 to 32)
+    mid_f32_max_rows: int = 64          # rows and up to this many (193 / 203 / 214 us against the library's 207 / 215 / 217 at 33 / 48 / 64 rows; beyond,
+                                        # 232 and 234 at 96, 246 and 243 at 128; whole steps at 25 to 32 rows: nothing)
     mid_min_slice_steps: int = 4        # a slice of K keeps at least this many macro-steps of 128
     mid_max_slices: int = 8
     # ---- the product whose waves share out K (gemm_wavek.hip, up to 64 rows)

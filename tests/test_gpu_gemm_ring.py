@@ -1,0 +1,48 @@
+"""Products of packed weights with up to 128 rows whose rows reach LDS by themselves: the bits of the kernel with producer waves, at edges of the ring and of the tiles."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_gpu_divasun import rnd
+
+pytestmark = pytest.mark.gpu
+
+
+# fewer macro-steps of K than the ring holds, as many, one more and several turns; features that end within a workgroup; slices of unequal length; with
+# 16,512 features more workgroups than compute units (the shorter ring).  The kernel that takes plain weights adds in the same order, so the bits are the same
+@pytest.mark.parametrize("m", [1, 17, 32, 33, 48, 49, 64, 65, 96, 97, 127, 128])
+@pytest.mark.parametrize("n,k,slices", [(16, 128, 1), (80, 256, 1), (208, 384, 1), (64, 512, 1), (208, 1408, 1), (144, 1408, 3), (80, 1152, 8), (16512, 384, 1), (4160, 640, 5)])
+def test_planes_are_those_of_plain_weights(m, n, k, slices):
+    from llama_cu_amd.kernels import ops
+    wide = rnd(m + 1, k + 16, seed=1).bfloat16()
+    wide[m:] = float("nan")
+    wide[:, k + 8:] = float("nan")
+    wide[:, :8] = float("nan")                             # what lies around the rows counts for nothing
+    if m > 20:
+        wide[20] = float("nan")                            # and a row of NaN for its own results only
+    x, w = wide.cuda()[:m, 8:8 + k], rnd(n, k, seed=2, std=k ** -0.5).bfloat16().cuda()
+    room = torch.full((ops.mid_planes(k, slices), m, n + 4), 7.0, device="cuda")
+    got = ops.gemm_mid(x, ops.pack_weight(w), out=room[:, :, :n], slices=slices, packed=True)
+    want = ops.gemm_mid(x, w, slices=slices)
+    good = torch.arange(m) != 20
+    assert torch.equal(got[:, good], want[:, good]) and torch.isfinite(got[:, good]).all() and (room[:, :, n:] == 7).all()
+    assert m <= 20 or torch.isnan(got[:, 20]).all()
+
+
+@pytest.mark.parametrize("m", [65, 96, 97, 128])
+@pytest.mark.parametrize("di,k", [(16, 128), (80, 384), (8256, 256), (208, 1408)])
+@pytest.mark.parametrize("act", [{}, dict(act_alpha=1.7, act_limit=0.8)])
+def test_swiglu_is_that_of_plain_weights(m, di, k, act):
+    from llama_cu_amd.kernels import ops
+    x, w = rnd(m, k, seed=1).bfloat16().cuda(), rnd(2 * di, k, seed=2, std=k ** -0.5).bfloat16().cuda()
+    assert torch.equal(ops.gemm_mid(x, ops.pack_weight(w), swiglu=True, packed=True, **act), ops.gemm_mid(x, w, swiglu=True, **act))
+
+
+@pytest.mark.parametrize("m,parts", [(17, 1), (33, 48), (49, 100), (64, 256)])
+def test_rows_that_wait_for_their_normalisation(m, parts):
+    from llama_cu_amd.kernels import ops
+    n, k = 208, 1408
+    x, w, shares = rnd(m, k, seed=1).bfloat16().cuda(), rnd(n, k, seed=2, std=k ** -0.5).bfloat16().cuda(), rnd(m, parts, seed=3).abs().cuda()
+    kw = dict(slices=4, row_sumsq=shares, norm_width=k, eps=1e-3)
+    assert torch.equal(ops.gemm_mid(x, ops.pack_weight(w), packed=True, **kw), ops.gemm_mid(x, w, **kw))
