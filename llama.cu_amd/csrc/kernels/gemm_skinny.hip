@@ -40,6 +40,7 @@
 #include "kv_layout.h"
 #include "qkv_store.h"
 #include "quad_rows.h"
+#include "stream_steps.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -110,13 +111,13 @@ struct Frag {
 __device__ __forceinline__ u32x4 stream_load(const u32x4 *p) { return __builtin_nontemporal_load(p); }
 
 // The lane's loads of macro-step s: W's k = 128 s + 32 grp + 8 j .. + 7 for j = 0..3; X as quad_rows.h says, through a buffer that ends with the
-// last row's k (rows beyond it read zeros), x_place the lane's place in its first four rows and x_four the bytes of four rows.
-template <int NT, int MT, bool PACKED, int LOADS>
+// last row's k (rows beyond it read zeros; WHOLE: K has no partial step), x_place the lane's place in its first four rows and x_four the bytes of four rows.
+template <int NT, int MT, bool PACKED, int LOADS, bool WHOLE>
 __device__ __forceinline__ void load_frag(Frag<NT, MT, LOADS> &f, const bf16_t *const (&wrow)[NT], __amdgpu_buffer_rsrc_t xb, uint32_t x_place,
                                           uint32_t x_four, int s, int lane, int K) {
     const int grp = lane >> 4, kb = 128 * s + 32 * grp;
     const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
-    if (128 * (s + 1) <= K) {
+    if (WHOLE || 128 * (s + 1) <= K) {
         // packed: wrow is the lane's place in the tile's first block; blocks are 2048 elements,
         // the four loads of a block 512 apart
         const int w0 = PACKED ? 2048 * s : kb, wj = PACKED ? 512 : 8;
@@ -164,7 +165,7 @@ __device__ __forceinline__ void mul_frag(const Frag<NT, MT, LOADS> &f, f32x4 (&a
 }
 
 template <int NT, int MT, int EPI, int SK_WAVES, bool PACKED, int LOADS>
-__global__ void __launch_bounds__(SK_WAVES *WAVE)
+__global__ void __launch_bounds__(SK_WAVES *WAVE, SK_WAVES == 8 && NT * MT == 1 && LOADS <= 2 ? 4 : 1)
 gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict__ W, int ldw, void *__restrict__ Y,
                    int ldy, int M, int N, int K, SkinnyExtra ex) {
     __shared__ float red[SK_WAVES][NT * MT * 4][WAVE];
@@ -232,24 +233,33 @@ gemm_skinny_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restri
     }
 
     // A ring of STAGES macro-steps in flight per wave: with few workgroups per compute unit
-    // (small N) this is what keeps enough bytes on their way from HBM.
+    // (small N) this is what keeps enough bytes on their way from HBM.  Packed rows go through it without a condition (stream_steps.h; with one the wave waited for the whole
+    // ring once in STAGES steps): passes of the 8B shape, one request 7.10 -> 6.99 ms, eight 7.80 -> 7.68.  Four waves a SIMD, as before, for one tile of few rows (129 registers
+    // otherwise).
     // Two tiles of rows with four of features: two as well while the second tile has up to eight rows (25 to 32 rows want the registers).  SwiGLU, us, 17 to 24 rows with two stages (with
     // one, and all eight loads of rows): 7168 x 8192 33.0 to 34.1 (37.2 to 38.1), 2048 x 6144 23.3 to 24.3 (27.0 to 27.4), 7680 x 16384 65.8 to 67.9 (74.8 to 75.2).
     constexpr int STAGES = NT * MT == 1 ? 4 : NT * MT == 2 ? 3 : NT * MT == 8 && SK_WAVES == 8 && LOADS == 4 ? 1 : 2;
     const int nsteps = (K + 127) / 128;
     Frag<NT, MT, LOADS> f[STAGES];
-    int s = wave;
+    if constexpr (PACKED) {                                            // (K is a multiple of 128)
+        stream_steps<STAGES>(
+            wave < nsteps ? (nsteps - 1 - wave) / SK_WAVES + 1 : 0,
+            [&](int u, int i) { load_frag<NT, MT, true, LOADS, true>(f[u], wrow, xb, x_place, x_four, wave + i * SK_WAVES, lane, K); },
+            [&](int u, int) { mul_frag<NT, MT, LOADS>(f[u], acc); });
+    } else {
+        int s = wave;
 #pragma unroll
-    for (int i = 0; i < STAGES; ++i)
-        if (s + i * SK_WAVES < nsteps) load_frag<NT, MT, PACKED, LOADS>(f[i], wrow, xb, x_place, x_four, s + i * SK_WAVES, lane, K);
-    for (; s < nsteps; s += STAGES * SK_WAVES) {
+        for (int i = 0; i < STAGES; ++i)
+            if (s + i * SK_WAVES < nsteps) load_frag<NT, MT, false, LOADS, false>(f[i], wrow, xb, x_place, x_four, s + i * SK_WAVES, lane, K);
+        for (; s < nsteps; s += STAGES * SK_WAVES) {
 #pragma unroll
-        for (int i = 0; i < STAGES; ++i) {
-            const int cur = s + i * SK_WAVES;
-            if (cur < nsteps) {
-                mul_frag<NT, MT, LOADS>(f[i], acc);
-                if (cur + STAGES * SK_WAVES < nsteps)
-                    load_frag<NT, MT, PACKED, LOADS>(f[i], wrow, xb, x_place, x_four, cur + STAGES * SK_WAVES, lane, K);
+            for (int i = 0; i < STAGES; ++i) {
+                const int cur = s + i * SK_WAVES;
+                if (cur < nsteps) {
+                    mul_frag<NT, MT, LOADS>(f[i], acc);
+                    if (cur + STAGES * SK_WAVES < nsteps)
+                        load_frag<NT, MT, false, LOADS, false>(f[i], wrow, xb, x_place, x_four, cur + STAGES * SK_WAVES, lane, K);
+                }
             }
         }
     }
