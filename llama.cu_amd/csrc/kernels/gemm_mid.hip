@@ -33,6 +33,7 @@
 // rsqrt(sum of the row's shares / norm_width + eps), which commutes with the product): consumer
 // wave w loads the shares of rows 16 w .. 16 w + 15 before its first loads of W, so they are back
 // first, adds them in a fixed order and leaves the factors in LDS for the epilogue.
+#include <type_traits>
 #include "common.h"
 #include "gate_act.h"
 #include "qkv_store.h"
@@ -318,7 +319,7 @@ gemm_mid_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict_
 // keeps eight tiles of W in flight a wave, but X comes to LDS through the registers of one producer for 64 rows, and it is this wave's round trips
 // (load, store, barrier) that the others wait for: at 64 rows of the 4096 x 14336 down projection 28.5 us, 4.1 TB/s.  Here X comes by loads that go straight
 // to LDS, each wave asks for a quarter of it, and nobody produces:
-//   * four waves a workgroup, each with its own tile of 16 features (SwiGLU: a gate and an up tile).  Macro-step s of K (128 k): W in registers, asked for D
+//   * four waves a workgroup, each with its own tile of 16 features (SwiGLU: a gate and an up tile; many features, uncut: eight waves of two tiles, mid_ring_wide).  Macro-step s of K (128 k): W in registers, asked for D
 //     steps ahead; X in slot s % D of a ring in LDS, asked for D - 1 steps ahead, one step after its W (a slot is free only once every wave has passed
 //     the barrier after its last read).  A wave's loads come back in order, so each step waits for a count: all but the younger steps' loads;
 //   * a slot holds, for each 16 rows, four KB pieces: piece i has rows 4 i .. 4 i + 3 (wave i asks for it), lane 16 g + 4 a + p of the load k = 32 g + 8 (p ^ swizzle) of
@@ -328,11 +329,11 @@ gemm_mid_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict_
 // D = 3; with more workgroups than compute units D = 2 (from 33 rows on), which leaves LDS for several on each: 50,304 x 2048 at 121 rows 57 against 64 us.  With
 // up to 32 rows D = 3 fits several times (128,256 x 4096 at 24 rows 182 against 193 us).
 // What bounds it: at 64 rows a unit's share of 14336 x 4096 in four slices is 459 KB of W and 459 of X, in 24.0 us 38 bytes a ns: the rate at which
-// a compute unit reads.  Measured, weights out of memory, this kernel and the one above: 4096 x 14336, four slices, 32 / 64 / 121 rows: 21.2 / 24.0 / 31.0 us against
-// 22.4 / 28.5 / 36.4; 4096 x 4096 9.7 / 10.7 / 13.5 against 10.6 / 13.4 / 17.2; 2048 x 2816 at 64 / 121 rows 6.8 / 9.0 against 8.4 / 11.5; the uncut 128,256 x 4096
-// at 48 / 64 rows 201 / 211 against 210 / 233.  SwiGLU, 28,672 x 4096 at 121 rows: 48.6 against 51.9; 16,384 x 2048 22.3 against 26.1; up to 64 rows it is no faster
+// a compute unit reads.  Measured, weights out of memory, this kernel and the one above: 4096 x 14336, four slices, 32 / 64 / 121 rows: 20.5 / 23.7 / 29.1 us against
+// 22.4 / 28.5 / 36.4 (21.8 / 25.5 / 32.6 while each third step waited for all but three loads, see the loop); 4096 x 4096 9.6 / 10.7 / 13.2 against 10.6 / 13.4 / 17.2;
+// 2048 x 2816 at 64 / 121 rows 6.9 / 8.9 against 8.4 / 11.5; the uncut 128,256 x 4096 at 48 / 64 rows 202 / 211 (193 / 195 with eight waves) against 210 / 233.  SwiGLU, 28,672 x 4096 at 121 rows: 48.6 against 51.9; 16,384 x 2048 22.3 against 26.1; up to 64 rows it is no faster
 // (43.7 against 43.2) and stays there.
-constexpr int RING_WAVES = 4;
+constexpr int RING_PIECES = 4;
 
 template <int LEFT>
 __device__ __forceinline__ void ring_wait_loads() {
@@ -340,22 +341,25 @@ __device__ __forceinline__ void ring_wait_loads() {
     __builtin_amdgcn_s_waitcnt((LEFT & 15) | ((LEFT >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
-// One macro-step: asks for a later one's X (into `free_slot`, which every wave has read) and multiplies this one's.  A function of its own with both slots
-// restrict: otherwise the compiler takes the loads to LDS for writes that the reads after them must wait for.
-template <int NT, int MT>
-__device__ __forceinline__ void ring_step(const u32x4 *__restrict__ slot, u32x4 *__restrict__ free_slot, const __amdgpu_buffer_rsrc_t xb, const uint32_t (&src)[MT],
-                                          uint32_t step_bytes, uint32_t none, int wave, const int (&at)[4], const u32x4 (&w)[NT][4], f32x4 (&acc)[NT][MT]) {
+// One macro-step: asks for a later one's X (into `free_slot`, which every wave has read; the last steps, without ASK, ask for none) and multiplies this one's.  A
+// function of its own with both slots restrict: otherwise the compiler takes the loads to LDS for writes that the reads after them must wait for.
+template <bool ASK, int NT, int MT, int PIECES>
+__device__ __forceinline__ void ring_step(const u32x4 *__restrict__ slot, u32x4 *__restrict__ free_slot, const __amdgpu_buffer_rsrc_t xb, const uint32_t (&src)[PIECES],
+                                          const int (&dst)[PIECES], uint32_t step_bytes, uint32_t none, const int (&at)[4], const u32x4 (&w)[NT][4],
+                                          f32x4 (&acc)[NT][MT]) {
+    if (ASK) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        auto *to = (__attribute__((address_space(3))) void *)(free_slot + (m * RING_WAVES + wave) * WAVE);
-        const uint32_t from = (src[m] + step_bytes) | none;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xb, to, 16, from, 0, 0, 0);
+        for (int m = 0; m < PIECES; ++m) {
+            auto *to = (__attribute__((address_space(3))) void *)(free_slot + dst[m]);
+            const uint32_t from = (src[m] + step_bytes) | none;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xb, to, 16, from, 0, 0, 0);
+        }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         u32x4 x[MT];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) x[m] = slot[at[j] + m * RING_WAVES * WAVE];
+        for (int m = 0; m < MT; ++m) x[m] = slot[at[j] + m * RING_PIECES * WAVE];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -363,37 +367,43 @@ __device__ __forceinline__ void ring_step(const u32x4 *__restrict__ slot, u32x4 
     }
 }
 
-template <int MT, int EPI, int D>
-__global__ void __launch_bounds__(RING_WAVES * WAVE, 1)
+template <int MT, int EPI, int D, int WAVES, int TILES>
+__global__ void __launch_bounds__(WAVES * WAVE, 1)
 gemm_mid_ring_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict__ W, void *__restrict__ Y, int ldy, int M, int N, int K, int steps_per_slice,
                      const float *__restrict__ sumsq_in, int n_in, int norm_width, float eps, float act_alpha, float act_limit) {
     static_assert(EPI == MID_EPI_SWIGLU || EPI == MID_EPI_PARTIAL_F32, "what the kernel is chosen for");
     extern __shared__ __attribute__((aligned(16))) char xs[];      // the ring of X, then the rows' factors
-    constexpr int NT = EPI == MID_EPI_SWIGLU ? 2 : 1, SLOT = MT * RING_WAVES * WAVE, W_LOADS = 4 * NT;
+    constexpr bool SWIGLU = EPI == MID_EPI_SWIGLU;
+    static_assert((WAVES == 4 || WAVES == 8) && (!SWIGLU || TILES == 1), "a wave asks for MT or half as many pieces of X");
+    constexpr int NT = SWIGLU ? 2 : TILES, SLOT = MT * RING_PIECES * WAVE, W_LOADS = 4 * NT, PIECES = WAVES == 8 ? (MT + 1) / 2 : MT;
     u32x4 *ring = (u32x4 *)xs;
     float *row_scale = (float *)(ring + D * SLOT);
     const int lane = threadIdx.x & (WAVE - 1), l16 = lane & 15, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int steps_total = K / 128, s_begin = blockIdx.y * steps_per_slice, nst = min(steps_total, s_begin + steps_per_slice) - s_begin;
     const int n_tiles = (EPI == MID_EPI_SWIGLU ? N / 2 : N) / 16;
-    const int tile0 = (int)((long long)blockIdx.x * n_tiles / gridDim.x) + wave;
-    const bool live = tile0 < (int)((long long)(blockIdx.x + 1) * n_tiles / gridDim.x);   // a wave without a tile asks for its quarter of X and stores nothing
+    const int tile0 = (int)((long long)blockIdx.x * n_tiles / gridDim.x) + TILES * wave, tile_end = (int)((long long)(blockIdx.x + 1) * n_tiles / gridDim.x);
+    const bool live = tile0 < tile_end;                // a wave without a tile asks for its share of X and stores nothing
     // buffer resources that end with the slice: what lies beyond reads zeros
     __amdgpu_buffer_rsrc_t wb[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-        const int tile = (live ? tile0 : n_tiles - 1) + t * n_tiles;
-        wb[t] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(W + ((size_t)tile * steps_total + s_begin) * 2048), 0, live ? (uint32_t)nst * 4096u : 0u, 0x00020000);
+        const bool has = SWIGLU ? live : tile0 + t < tile_end;
+        const int tile = (has ? tile0 : n_tiles - 1) + (SWIGLU ? t * n_tiles : has ? t : 0);
+        wb[t] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(W + ((size_t)tile * steps_total + s_begin) * 2048), 0, has ? (uint32_t)nst * 4096u : 0u, 0x00020000);
     }
     const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<bf16_t *>(X + (size_t)128 * s_begin), 0, (uint32_t)(((size_t)(M - 1) * ldx + 128 * nst) * 2), 0x00020000);
-    uint32_t src[MT];                                  // rows from M on lie beyond the end
+    uint32_t src[PIECES];                              // rows from M on lie beyond the end
+    int dst[PIECES];
     {
-        const int a = (lane >> 2) & 3, p = lane & 3, swizzle = (a >> 1) + 2 * (wave & 1);
+        const int a = (lane >> 2) & 3, p = lane & 3, piece = wave & 3, swizzle = (a >> 1) + 2 * (piece & 1);
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const int row = 16 * m + 4 * wave + a;
-            src[m] = row < M ? (uint32_t)(row * ldx + 32 * grp + 8 * (p ^ swizzle)) * 2u : 0x80000000u;
+        for (int k = 0; k < PIECES; ++k) {
+            const int m = WAVES == 8 ? min(2 * k + (wave >> 2), MT - 1) : k;    // (an odd MT's last pieces come twice, the same bytes to the same place)
+            const int row = 16 * m + 4 * piece + a;
+            src[k] = row < M ? (uint32_t)(row * ldx + 32 * grp + 8 * (p ^ swizzle)) * 2u : 0x80000000u;
+            dst[k] = (m * RING_PIECES + piece) * WAVE;
         }
     }
     int at[4];                                         // where the operand of row l16, instruction j, lies in a slot's 16 rows
@@ -436,31 +446,53 @@ gemm_mid_ring_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__rest
     for (int s = 0; s < D; ++s) {
         if (s > 0) {
 #pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                auto *to = (__attribute__((address_space(3))) void *)(ring + (s - 1) * SLOT + (m * RING_WAVES + wave) * WAVE);
+            for (int m = 0; m < PIECES; ++m) {
+                auto *to = (__attribute__((address_space(3))) void *)(ring + (s - 1) * SLOT + dst[m]);
                 const uint32_t from = (src[m] + (uint32_t)(s - 1) * 256u) | (s - 1 < nst ? 0u : 0x80000000u);
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(xb, to, 16, from, 0, 0, 0);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
         RING_LOAD_W(s, s);
+        __builtin_amdgcn_sched_barrier(0);
     }
     if (scales) {
         scale_ss += __shfl_xor(scale_ss, 16, WAVE);
         scale_ss += __shfl_xor(scale_ss, 32, WAVE);
         if (grp == 0) row_scale[16 * wave + l16] = rsqrtf(scale_ss / (float)norm_width + eps);
     }
-    for (int s0 = 0; s0 < nst; s0 += D) {
+    // Whole rounds of D steps, then what is left of them, for which everything has been asked for.  (A way out between the steps would make the compiler take the
+    // W that a round begins with for just asked for, and wait for all loads but the last three.)
+    const int whole = nst / D * D, rest = nst - whole;
+    for (int s0 = 0; s0 < whole; s0 += D) {
 #pragma unroll
         for (int i = 0; i < D; ++i) {
             const int s = s0 + i;
-            if (s >= nst) break;
             // younger than this step's X: the W of D - 1 steps and the X of D - 2
-            ring_wait_loads<(D - 1) * W_LOADS + (D - 2) * MT>();
+            ring_wait_loads<(D - 1) * W_LOADS + (D - 2) * PIECES>();
             lds_barrier();
-            ring_step<NT, MT>(ring + i * SLOT, ring + (i == 0 ? D - 1 : i - 1) * SLOT, xb, src, (uint32_t)(s + D - 1) * 256u, s + D - 1 < nst ? 0u : 0x80000000u, wave, at, w[i], acc);
+            ring_step<true, NT, MT, PIECES>(ring + i * SLOT, ring + (i == 0 ? D - 1 : i - 1) * SLOT, xb, src, dst, (uint32_t)(s + D - 1) * 256u,
+                                            s + D - 1 < nst ? 0u : 0x80000000u, at, w[i], acc);
+            // W's registers are read now: the products stay in front of the loads (behind them, W would come to other registers, and be copied, all of it awaited)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) asm volatile("" : "+a"(acc[t][m]));
+            __builtin_amdgcn_sched_barrier(0);         // (the counts rest on the loads' order: X before W)
             RING_LOAD_W(i, s + D);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
+    auto last = [&](auto place) {
+        constexpr int I = decltype(place)::value;
+        if (I >= rest) return;
+        ring_wait_loads<(D - 1 - I) * W_LOADS + (D - 2 - I) * PIECES>();
+        lds_barrier();
+        ring_step<false, NT, MT, PIECES>(ring + I * SLOT, ring + I * SLOT, xb, src, dst, 0, 0, at, w[I], acc);
+    };
+    last(std::integral_constant<int, 0>());
+    if constexpr (D > 2) last(std::integral_constant<int, 1>());
+    static_assert(D <= 3, "the steps that may be left");
 #undef RING_LOAD_W
     ring_wait_loads<0>();                              // nothing of this workgroup is on its way to LDS when it ends
     if (!live) return;
@@ -485,7 +517,9 @@ gemm_mid_ring_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__rest
             *(uint2 *)((bf16_t *)Y + (size_t)tok * ldy + n) = pk;
         } else {
             float *plane = (float *)Y + (size_t)blockIdx.y * M * ldy;
-            *(f32x4 *)(plane + (size_t)tok * ldy + n) = acc[0][m];
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                if (tile0 + t < tile_end) *(f32x4 *)(plane + (size_t)tok * ldy + n + 16 * t) = acc[t][m];
         }
     }
 }
@@ -585,19 +619,31 @@ static bool mid_ring_takes(int M, int epi, int packed) {
     return packed && M <= 128 && (epi == MID_EPI_PARTIAL_F32 || (epi == MID_EPI_SWIGLU && M > 64));
 }
 
+// Eight waves of two tiles each, a workgroup for 256 features: it reads the rows of X a quarter as often, but there is one of it on a compute unit, so its
+// workgroups have to fill their rounds: three quarters of a single one, nine tenths of several.  Uncut, 32-bit sums, us with four waves of a tile and with this
+// (the library's) at 48 / 64 / 96 / 121 rows: 128,256 x 4096 (501 workgroups) 202 / 211 / 227 / 247 and 193 / 195 / 198 / 202 (215 / 219 / 235 / 246); x 2048 103 / 107 / 120 / 129
+// and 98 / 99 / 105 / 107 (116 / 121 / 129 / 133); 65,536 x 4096 (256) 98 / 104 / 113 / 124 and 92 / 93 / 98 / 99 (128 / 131 / 134 / 135); 50,304 x 2048 (197) 45 / 46 / 54 / 59 and
+// 39 / 38 / 41 / 45 (52 / 54 / 56 / 57).  Where rounds are not full, at 64 rows: 98,304 x 2048 (384) 80 and 88, 65,792 x 2048 (257) 61 and 79, 40,960 x 2048 (160) 36 and 38,
+// 32,000 x 4096 (125) 49 and 57.  Up to 32 rows: 128,256 x 4096 188 and 187.
+static bool mid_ring_wide(int M, int n_tiles, int K, int units) {
+    const int groups = (n_tiles + 15) / 16, rounds = units > 0 ? (groups + units - 1) / units : 0;
+    return M > 32 && K >= 2048 && (rounds == 1 ? 4 * groups >= 3 * units : rounds > 1 && 10 * groups >= 9 * rounds * units);
+}
+
 template <int EPI>
 static int mid_ring_launch(const void *X, int ldx, const void *W, void *Y, int ldy, int M, int N, int K, int slices, const MidScale &sc, hipStream_t stream) {
     const int n_tiles = (EPI == MID_EPI_SWIGLU ? N / 2 : N) / 16, units = mid_compute_units();
     const int steps = K / 128, per = (steps + slices - 1) / slices, planes = (steps + per - 1) / per;
-    int groups = (n_tiles + RING_WAVES - 1) / RING_WAVES;
+    const bool wide = EPI == MID_EPI_PARTIAL_F32 && planes == 1 && mid_ring_wide(M, n_tiles, K, units);
+    int groups = wide ? (n_tiles + 15) / 16 : (n_tiles + 3) / 4;
     // gate/up: the next multiple of the number of compute units (28,672 x 4096 at 96 rows as 256 workgroups 48.4, as 224 49.2 us; 22,016 x 4096 41.9 and 45.0)
     if (EPI == MID_EPI_SWIGLU && units > 0) groups = min(n_tiles, (groups + units - 1) / units * units);
     const dim3 grid(groups, planes);
     const bool several = EPI == MID_EPI_PARTIAL_F32 && units > 0 && (long long)groups * planes > units;      // several workgroups for a unit: a ring of two
-#define GO(MT_, D_)                                                                                                            \
+#define GO(MT_, D_, WAVES_, TILES_)                                                                                            \
     do {                                                                                                                       \
-        auto kernel = gemm_mid_ring_kernel<MT_, EPI, D_>;                                                                      \
-        constexpr int lds = D_ * MT_ * RING_WAVES * WAVE * 16 + 16 * MT_ * (int)sizeof(float);                                 \
+        auto kernel = gemm_mid_ring_kernel<MT_, EPI, D_, WAVES_, TILES_>;                                                      \
+        constexpr int lds = D_ * MT_ * RING_PIECES * WAVE * 16 + 16 * MT_ * (int)sizeof(float);                                 \
         if (lds > 64 * 1024) {                                                                                                 \
             static bool asked = false;                                                                                         \
             if (!asked) {                                                                                                      \
@@ -606,19 +652,22 @@ static int mid_ring_launch(const void *X, int ldx, const void *W, void *Y, int l
                 asked = true;                                                                                                  \
             }                                                                                                                  \
         }                                                                                                                      \
-        kernel<<<grid, dim3(RING_WAVES * WAVE), lds, stream>>>((const bf16_t *)X, ldx, (const bf16_t *)W, Y, ldy, M, N, K, per, \
+        kernel<<<grid, dim3(WAVES_ * WAVE), lds, stream>>>((const bf16_t *)X, ldx, (const bf16_t *)W, Y, ldy, M, N, K, per,   \
                                                                sc.sumsq_in, sc.n_in, sc.norm_width, sc.eps, sc.act_alpha, sc.act_limit); \
     } while (0)
-#define GO_D(MT_)                   \
-    do {                            \
-        if (several) GO(MT_, 2);    \
-        else GO(MT_, 3);            \
+#define GO_D(MT_)                                          \
+    do {                                                   \
+        if constexpr (EPI == MID_EPI_PARTIAL_F32) {        \
+            if (wide) GO(MT_, 3, 8, 2);                    \
+            else if (several) GO(MT_, 2, 4, 1);            \
+            else GO(MT_, 3, 4, 1);                         \
+        }                                                  \
     } while (0)
     if constexpr (EPI == MID_EPI_SWIGLU) {
-        if (M <= 96) GO(6, 3);
-        else GO(8, 3);
+        if (M <= 96) GO(6, 3, 4, 1);
+        else GO(8, 3, 4, 1);
     } else {
-        if (M <= 32) GO(2, 3);
+        if (M <= 32) GO(2, 3, 4, 1);
         else if (M <= 48) GO_D(3);
         else if (M <= 64) GO_D(4);
         else if (M <= 96) GO_D(6);

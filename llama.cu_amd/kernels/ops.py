@@ -918,6 +918,17 @@ def mid_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
             and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def mid_f32_preferred(m: int, n: int, k: int) -> bool:
+    """Whether a product ``[m, k] x [n, k]`` with 32-bit output and a packed weight is faster uncut in ``gemm_mid`` than in the library."""
+    t = TUNING
+    if t.mid_f32_rows < m <= t.mid_f32_max_rows:
+        return True
+    groups = (n + 255) // 256                 # as mid_ring_wide in gemm_mid.hip chooses its eight waves
+    rounds = (groups + t.compute_units - 1) // t.compute_units
+    return t.mid_f32_max_rows < m <= t.mid_f32_wide_max_rows and k >= 2048 and \
+        (4 * groups >= 3 * t.compute_units if rounds == 1 else 10 * groups >= 9 * rounds * t.compute_units)
+
+
 WAVEK_MAX_ROWS = 64       # what gemm_wavek takes
 
 

@@ -55,8 +55,9 @@ class Tuning:
                                         # faster at 20 rows, 1.7 % at 32; 2 % slower at 16 and at 40 to 48, where the first product
                                         # of the feed-forward pays more for the rows' factors than the norm kernel cost
     mid_f32_rows: int = 32              # a product with 32-bit output (the output matrix, 1.05 GB) goes to it, uncut, above this many
-    mid_f32_max_rows: int = 64          # rows and up to this many (193 / 203 / 214 us against the library's 207 / 215 / 217 at 33 / 48 / 64 rows; beyond,
-                                        # 232 and 234 at 96, 246 and 243 at 128; whole steps at 25 to 32 rows: nothing)
+    mid_f32_max_rows: int = 64          # rows and up to this many (193 / 195 us against the library's 215 / 219 at 48 / 64 rows; whole steps at 25 to 32 rows: nothing) ...
+    mid_f32_wide_max_rows: int = 128    # ... and where its workgroups of 256 features fill their rounds (mid_ring_wide in gemm_mid.hip) up to so many (198 and 202 us
+                                        # against 235 and 246 at 96 and 121 rows)
     mid_min_slice_steps: int = 4        # a slice of K keeps at least this many macro-steps of 128
     mid_max_slices: int = 8
     # ---- the product whose waves share out K (gemm_wavek.hip, up to 64 rows)

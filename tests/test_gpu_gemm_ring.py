@@ -46,3 +46,14 @@ def test_rows_that_wait_for_their_normalisation(m, parts):
     x, w, shares = rnd(m, k, seed=1).bfloat16().cuda(), rnd(n, k, seed=2, std=k ** -0.5).bfloat16().cuda(), rnd(m, parts, seed=3).abs().cuda()
     kw = dict(slices=4, row_sumsq=shares, norm_width=k, eps=1e-3)
     assert torch.equal(ops.gemm_mid(x, ops.pack_weight(w), packed=True, **kw), ops.gemm_mid(x, w, **kw))
+
+
+# features that leave the last workgroup of 256 a tile; one round of workgroups, and two; K that leaves none, one and two steps behind the ring's turns
+@pytest.mark.parametrize("m", [33, 48, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("n,k", [(49168, 2048), (49152, 2176), (120064, 2304)])
+def test_many_features_uncut(m, n, k):
+    from llama_cu_amd.kernels import ops
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w = torch.randn(m, k, device="cuda", generator=g).bfloat16(), (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).bfloat16()
+    assert ops.mid_f32_preferred(m, n, k)
+    assert torch.equal(ops.gemm_mid(x, ops.pack_weight(w), slices=1, packed=True), ops.gemm_mid(x, w, slices=1))
