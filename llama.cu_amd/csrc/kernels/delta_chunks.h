@@ -15,7 +15,8 @@
 // below).
 //
 // What bounds them: `maps` runs 4,300 (channel-wise 6,300) matrix instructions of 64 cycles a chunk and head, 28 (42) us on a compute
-// unit's four SIMDs; one workgroup of 8 waves fits a compute unit beside its LDS.  `chain` is its 96 matrix
+// unit's four SIMDs; one workgroup of 8 waves fits a compute unit beside its LDS (560 of them, 2,014 tokens of four requests, channel-wise, are three rounds: 220 us, and 241
+// while the vectors and values were asked for a few at a time, each under a condition, and so awaited in turn).  `chain` is its 96 matrix
 // instructions a SIMD and chunk (2.6 us) and the round through LDS; the affine form costs `maps` a third more products than c, o and S
 // in turn would, but leaves one product instead of two, one after the other, on the chain.
 //
@@ -247,12 +248,21 @@ delta_maps_kernel(DeltaChunkArgs p) {
         static_assert(2 * GROUPS * DK <= L::DINV, "room for the groups' products");
         const int c = tid % DK, grp = tid / DK, row = 5 * dk;
         const float *s = p.prep + ((size_t)t0 * heads + head) * row + min(c, dk - 1);
-        float w[PER];
+        float w[PER], al[PER], u[PER], k[PER], r[PER];                        // (all asked for before the first is used, and under no condition)
+#pragma unroll
+        for (int e = 0; e < PER; ++e) w[e] = s[(size_t)min(grp * PER + e, nt - 1) * heads * row];
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+            const float *x = s + (size_t)min(grp * PER + e, nt - 1) * heads * row;
+            al[e] = x[dk];
+            u[e] = x[2 * dk];
+            k[e] = x[3 * dk];
+            r[e] = x[4 * dk];
+        }
         double own = 1.0;
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
             const int t = grp * PER + e;
-            w[e] = s[(size_t)min(t, nt - 1) * heads * row];
             if (t >= nt || c >= dk) w[e] = 1.f;
             wild |= !(w[e] >= 0.5f && w[e] <= 1.f);
             own *= (double)w[e];
@@ -264,16 +274,14 @@ delta_maps_kernel(DeltaChunkArgs p) {
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
             const int t = grp * PER + e;
-            const float *x = s + (size_t)min(t, nt - 1) * heads * row;
-            const bool in = t < nt && c < dk;
-            const float al = in ? x[dk] : 0.f, u = in ? x[2 * dk] : 0.f, k = in ? x[3 * dk] : 0.f, r = in ? x[4 * dk] : 0.f;
-            wild |= dc_wild(make_float4(al, u, k, r));
-            us[t * LD + c] = (float)(u * before);
+            if (t >= nt || c >= dk) al[e] = u[e] = k[e] = r[e] = 0.f;
+            wild |= dc_wild(make_float4(al[e], u[e], k[e], r[e]));
+            us[t * LD + c] = (float)(u[e] * before);
             before *= (double)w[e];
             const double inv = 1.0 / before;
-            rs[t * LD + c] = (float)(r * before);
-            ks[t * LD + c] = (float)(k * inv);
-            as[t * LD + c] = (float)(al * inv);
+            rs[t * LD + c] = (float)(r[e] * before);
+            ks[t * LD + c] = (float)(k[e] * inv);
+            as[t * LD + c] = (float)(al[e] * inv);
         }
         if (grp == GROUPS - 1) g_all[dc_place(c)] = before;
     }
@@ -424,16 +432,25 @@ delta_maps_kernel(DeltaChunkArgs p) {
             const int col = tile * 16 + l16;
             dc_f64x4 v[4], x[4];
             dc_forget();
+            const int cc = head * dv + min(col, dv - 1);
+            float value[16];                                                  // all asked for before the first is used: the choice of where from stands outside
+            if (p.vf) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) value[e] = p.vf[(size_t)(t0 + min(4 * e + g, nt - 1)) * heads * dv + cc];
+            } else {
+                T raw[16];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) raw[e] = ((const T *)p.proj)[(size_t)(t0 + min(4 * e + g, nt - 1)) * p.row_stride + p.off_v + cc];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) value[e] = to_f32(raw[e]);
+            }
 #pragma unroll
             for (int b = 0; b < 4; ++b)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int s = 16 * b + 4 * i + g;
-                    const size_t tok = t0 + min(s, nt - 1);
-                    const int cc = head * dv + min(col, dv - 1);
-                    const float e = p.vf ? p.vf[tok * heads * dv + cc] : to_f32(((const T *)p.proj)[tok * p.row_stride + p.off_v + cc]);
-                    v[b][i] = s < nt && col < dv ? (double)e : 0.0;
-                    wild |= s < nt && col < dv && dc_wild(e);
+                    const bool in = 16 * b + 4 * i + g < nt && col < dv;
+                    v[b][i] = in ? (double)value[4 * b + i] : 0.0;
+                    wild |= in && dc_wild(value[4 * b + i]);
                 }
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
