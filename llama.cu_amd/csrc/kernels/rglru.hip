@@ -444,7 +444,8 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
 // which with the lanes that hold the sums were four one after the other, most of them of tokens that are not there.  The sums are
 // those of `slices` equal parts of the input channels, added in their order: RG_SLICES up to RG_FEW_ROWS tokens, one beyond, as the kernels above have them, so
 // that a token's bits do not depend on what else a step of so many tokens holds.  32-bit rows whose fours are aligned (the layer's), up to four taps, slices of whole matrix
-// instructions.  Latency bounds it: four trips to memory, 1.7 us of matrix instructions.  One MI355X, 4 taps, us beside the sliced kernel and the scan: width 2048
+// instructions.  Latency bounds it: two trips to memory (four while the states' numbers were asked for behind the matrices: 8.6 us of a launch in a model of width 2048 with 8 requests,
+// now 8.0), 1.7 us of matrix instructions.  One MI355X, 4 taps, us alone beside the sliced kernel and the scan, with four trips: width 2048
 // in 16 blocks 8.0 / 10.9 with 8 requests, 8.8 / 14.0 with 64; width 1024 in 16 blocks 5.8 / 8.5 with 8.  (Blocks of 192 channels, whose twelve sixteens do not fit the
 // registers: 24 / 10.4.)
 constexpr int RG_ONE_TOK = 4, RG_ONE_THREADS = 512, RG_ONE_BS = 128;
@@ -460,44 +461,57 @@ rglru_single_kernel(const float *__restrict__ rows, int row_stride, int y_off, i
     const int ld = bs + 4, b = blockIdx.y, tok0 = blockIdx.x * RG_ONE_TOK, nt = min(RG_ONE_TOK, n - tok0);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
     const int tiles = bs / 16, each = bs / 4 / slices;                    // matrix instructions a slice
-    rg_f32x4 w[2][MOST];
-    if (wave < tiles) {
-        const float *at = gates + (size_t)(b * tiles + wave) * tiles * 512 + 4 * lane;
-#pragma unroll
-        for (int j = 0; j < MOST; ++j) {
-            if (j >= tiles) break;
-#pragma unroll
-            for (int q = 0; q < 2; ++q) w[q][j] = *(const rg_f32x4 *)(at + 512 * j + 256 * q);
-        }
-    }
-    // ---- u, four neighbouring channels of a token a thread
+    // ---- what a thread asks for: under no condition (threads without work ask for a neighbour's), as loads come back in order: the numbers of the states first, what hangs on
+    // nothing, the matrices, and behind them what lies in the states
     auto load = [](const float *q) { return *(const rg_f32x4 *)q; };
-    for (int x = threadIdx.x; x < nt * (bs / 4); x += RG_ONE_THREADS) {
-        const int tt = x / (bs / 4), i = x % (bs / 4) * 4, c = b * bs + i, t = tok0 + tt;
-        const int before = ctx_len[t] - 1;                                // how many tokens the request has behind it
-        float *st = state + (size_t)state_slot[t] * taps * width + c;
-        rg_f32x4 here = load(rows + (size_t)t * row_stride + x_off + c), old[RG_MFMA_TAPS - 1], acc = {}, zero = {};
-        float cw[4 * RG_MFMA_TAPS];
-        if (taps == 4) {
+    static_assert(RG_ONE_TOK * RG_ONE_BS <= RG_ONE_THREADS && RG_ONE_BS / 16 <= RG_ONE_THREADS / WAVE, "an element a thread, sixteen output channels a wave");
+    const int x = min((int)threadIdx.x, nt * (bs / 4) - 1), tt = x / (bs / 4), i = x % (bs / 4) * 4, c = b * bs + i, t = tok0 + tt;      // u: four neighbouring channels of a token
+    const int e_tt = min((int)threadIdx.x / bs, nt - 1), e_o = threadIdx.x % bs, e_t = tok0 + e_tt, e_c = b * bs + e_o;                // the recurrence: an element
+    const bool e_in = (int)threadIdx.x / bs < nt;
+    const int ctx = ctx_len[t], slot = state_slot[t], e_ctx = ctx_len[e_t], e_slot = state_slot[e_t];
+    rg_f32x4 here = load(rows + (size_t)t * row_stride + x_off + c), old[RG_MFMA_TAPS - 1], acc = {}, zero = {};
+    float cw[4 * RG_MFMA_TAPS];
+    if (taps == 4) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const rg_f32x4 four = load(conv_w + (size_t)c * 4 + 4 * k);
+        for (int k = 0; k < 4; ++k) {
+            const rg_f32x4 four = load(conv_w + (size_t)c * 4 + 4 * k);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) cw[4 * k + j] = four[j];
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-#pragma unroll
-                for (int j = 0; j < RG_MFMA_TAPS; ++j) cw[4 * k + j] = conv_w[(size_t)(c + k) * taps + min(j, taps - 1)];
+            for (int j = 0; j < 4; ++j) cw[4 * k + j] = four[j];
         }
+    } else {
 #pragma unroll
-        for (int j = 0; j < RG_MFMA_TAPS - 1; ++j) old[j] = load(st + (size_t)min(j, taps - 1) * width);
-        if (bias) {
+        for (int k = 0; k < 4; ++k)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) here[k] += bias[x_off + c + k];
-        }
-        if (conv_b) acc = load(conv_b + c);
+            for (int j = 0; j < RG_MFMA_TAPS; ++j) cw[4 * k + j] = conv_w[(size_t)(c + k) * taps + min(j, taps - 1)];
+    }
+    if (conv_b) acc = load(conv_b + c);
+    float x_bias[4] = {}, y_bias = 0.f;
+    if (bias) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x_bias[k] = bias[x_off + c + k];
+        y_bias = bias[y_off + e_c];
+    }
+    const float e_lam = lam[e_c], e_ba = ba[e_c], e_bi = bi[e_c], y_in = rows[(size_t)e_t * row_stride + y_off + e_c];
+    __builtin_amdgcn_sched_barrier(0);
+    rg_f32x4 w[2][MOST];
+    {
+        const float *at = gates + (size_t)(b * tiles + min(wave, tiles - 1)) * tiles * 512 + 4 * lane;
+#pragma unroll
+        for (int j = 0; j < MOST; ++j)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) w[q][j] = *(const rg_f32x4 *)(at + 512 * min(j, tiles - 1) + 256 * q);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float *st = state + (size_t)slot * taps * width + c;
+#pragma unroll
+    for (int j = 0; j < RG_MFMA_TAPS - 1; ++j) old[j] = load(st + (size_t)min(j, taps - 1) * width);
+    float *e_at = state + ((size_t)e_slot * taps + taps - 1) * width + e_c;
+    const float e_old = *e_at, e_s = e_ctx > 1 ? e_old : 0.f, e_y = y_in + y_bias;
+    // ---- u
+    if ((int)threadIdx.x < nt * (bs / 4)) {
+        const int before = ctx - 1;                                       // how many tokens the request has behind it
+#pragma unroll
+        for (int k = 0; k < 4; ++k) here[k] += x_bias[k];
 #pragma unroll
         for (int j = 0; j < RG_MFMA_TAPS; ++j) {
             const int back = taps - 1 - j;
@@ -510,18 +524,6 @@ rglru_single_kernel(const float *__restrict__ rows, int row_stride, int y_off, i
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) us_tile[tt * ld + rg_place(i + k)] = acc[k];
-    }
-    // what a thread needs in the end for its element
-    static_assert(RG_ONE_TOK * RG_ONE_BS <= RG_ONE_THREADS && RG_ONE_BS / 16 <= RG_ONE_THREADS / WAVE, "an element a thread, sixteen output channels a wave");
-    const int e_tt = threadIdx.x / bs, e_o = threadIdx.x % bs, e_t = tok0 + e_tt, e_c = b * bs + e_o;
-    const bool e_in = e_tt < nt;
-    float e_lam = 0.f, e_ba = 0.f, e_bi = 0.f, e_y = 0.f, e_s = 0.f;
-    if (e_in) {
-        e_lam = lam[e_c];
-        e_ba = ba[e_c];
-        e_bi = bi[e_c];
-        e_y = to_f32(rows[(size_t)e_t * row_stride + y_off + e_c]) + (bias ? bias[y_off + e_c] : 0.f);
-        e_s = ctx_len[e_t] > 1 ? state[((size_t)state_slot[e_t] * taps + taps - 1) * width + e_c] : 0.f;
     }
     __syncthreads();
     // ---- the gates (the instruction's other rows are the last token's again)
@@ -562,7 +564,7 @@ rglru_single_kernel(const float *__restrict__ rows, int row_stride, int y_off, i
         const float log_a = -c_exp * gr * (e_lam > 20.f ? e_lam : log1pf(expf(e_lam)));
         const float mult = sqrtf(-expm1f(2.0f * log_a));
         const float S = fmaf(expf(log_a), e_s, mult * gate * us_tile[e_tt * ld + rg_place(e_o)]);
-        state[((size_t)state_slot[e_t] * taps + taps - 1) * width + e_c] = S;
+        *e_at = S;
         out[(size_t)e_t * width + e_c] = from_f32<T>(S * gelu_tanh(e_y));
     }
 }
