@@ -21,7 +21,7 @@
 //     output, [slice][M][N], and the kernel that follows (residual sum and norm) adds the planes
 //     in a fixed order.  Nothing is added atomically: results do not depend on timing.
 //
-// Packed weights that are cut over K, and gate/up beyond 64 rows, have a kernel without producers up to 128 rows (gemm_mid_ring_kernel, below).
+// Packed weights that are cut over K, and gate/up beyond 32 rows, have a kernel without producers up to 128 rows (gemm_mid_ring_kernel, below).
 // A further kernel (gemm_mid_qkv_kernel, below) is the q, k, v product with the rotation and the cache write
 // in its epilogue: there the consumer waves share each macro-step of K instead of the features.
 //
@@ -315,7 +315,7 @@ gemm_mid_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict_
 }
 
 // ------------------------------------------------------------------------------------------------
-// Packed weights with up to 128 rows: the products that are cut over K (and the uncut one with 32-bit output), and gate/up beyond 64 rows.  The kernel above
+// Packed weights with up to 128 rows: the products that are cut over K (and the uncut one with 32-bit output), and gate/up beyond 32 rows.  The kernel above
 // keeps eight tiles of W in flight a wave, but X comes to LDS through the registers of one producer for 64 rows, and it is this wave's round trips
 // (load, store, barrier) that the others wait for: at 64 rows of the 4096 x 14336 down projection 28.5 us, 4.1 TB/s.  Here X comes by loads that go straight
 // to LDS, each wave asks for a quarter of it, and nobody produces:
@@ -331,8 +331,9 @@ gemm_mid_kernel(const bf16_t *__restrict__ X, int ldx, const bf16_t *__restrict_
 // What bounds it: at 64 rows a unit's share of 14336 x 4096 in four slices is 459 KB of W and 459 of X, in 24.0 us 38 bytes a ns: the rate at which
 // a compute unit reads.  Measured, weights out of memory, this kernel and the one above: 4096 x 14336, four slices, 32 / 64 / 121 rows: 20.5 / 23.7 / 29.1 us against
 // 22.4 / 28.5 / 36.4 (21.8 / 25.5 / 32.6 while each third step waited for all but three loads, see the loop); 4096 x 4096 9.6 / 10.7 / 13.2 against 10.6 / 13.4 / 17.2;
-// 2048 x 2816 at 64 / 121 rows 6.9 / 8.9 against 8.4 / 11.5; the uncut 128,256 x 4096 at 48 / 64 rows 202 / 211 (193 / 195 with eight waves) against 210 / 233.  SwiGLU, 28,672 x 4096 at 121 rows: 48.6 against 51.9; 16,384 x 2048 22.3 against 26.1; up to 64 rows it is no faster
-// (43.7 against 43.2) and stays there.
+// 2048 x 2816 at 64 / 121 rows 6.9 / 8.9 against 8.4 / 11.5; the uncut 128,256 x 4096 at 48 / 64 rows 202 / 211 (193 / 195 with eight waves) against 210 / 233.  SwiGLU, 28,672 x 4096 at 48 / 64 / 121 rows: 41.2 / 42.4 / 48.6 against 42.6 / 44.2 /
+// 51.9; 16,384 x 2048 15.4 / 17.4 / 22.3 against 17.2 / 19.0 / 26.1; 22,016 x 4096 at 64 33.0 against 35.3, 57,344 x 8192 155 against 164, 8192 x 4096 24.9 against 27.6.  Up to 32 rows,
+// where that kernel has workgroups of two tiles, it is faster in places (8192 x 4096 at 24 rows 15.7 against 21.6, 12,288 x 2048 13.1 and 13.6, 32,768 x 4096 44.7 and 50) and keeps them all.
 constexpr int RING_PIECES = 4;
 
 template <int LEFT>
@@ -581,7 +582,7 @@ static int mid_launch_c(const void *X, int ldx, const void *W, int ldw, void *Y,
     // packed rows that the ring kernel takes never come here
 #define GO_MT(MT_)                                                                          \
     do {                                                                                    \
-        if constexpr (EPI == MID_EPI_BF16 || MT_ > 8 || (EPI == MID_EPI_SWIGLU && MT_ <= 4)) { \
+        if constexpr (EPI == MID_EPI_BF16 || MT_ > 8 || (EPI == MID_EPI_SWIGLU && MT_ <= 2)) { \
             if (packed) GO(MT_, true);                                                      \
             else GO(MT_, false);                                                            \
         } else {                                                                            \
@@ -614,9 +615,9 @@ static int mid_launch(const void *X, int ldx, const void *W, int ldw, void *Y, i
     return mid_launch_c<NT, EPI, MID_CONSUMERS>(X, ldx, W, ldw, Y, ldy, M, N, K, packed, slices, sc, stream);
 }
 
-// The ring kernel's rows (above): packed weights, up to 128 rows, SwiGLU beyond 64 of them.
+// The ring kernel's rows (above): packed weights, up to 128 rows, SwiGLU beyond 32 of them.
 static bool mid_ring_takes(int M, int epi, int packed) {
-    return packed && M <= 128 && (epi == MID_EPI_PARTIAL_F32 || (epi == MID_EPI_SWIGLU && M > 64));
+    return packed && M <= 128 && (epi == MID_EPI_PARTIAL_F32 || (epi == MID_EPI_SWIGLU && M > 32));
 }
 
 // Eight waves of two tiles each, a workgroup for 256 features: it reads the rows of X a quarter as often, but there is one of it on a compute unit, so its
@@ -664,7 +665,9 @@ static int mid_ring_launch(const void *X, int ldx, const void *W, void *Y, int l
         }                                                  \
     } while (0)
     if constexpr (EPI == MID_EPI_SWIGLU) {
-        if (M <= 96) GO(6, 3, 4, 1);
+        if (M <= 48) GO(3, 3, 4, 1);
+        else if (M <= 64) GO(4, 3, 4, 1);
+        else if (M <= 96) GO(6, 3, 4, 1);
         else GO(8, 3, 4, 1);
     } else {
         if (M <= 32) GO(2, 3, 4, 1);

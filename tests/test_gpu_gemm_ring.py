@@ -30,7 +30,7 @@ def test_planes_are_those_of_plain_weights(m, n, k, slices):
     assert m <= 20 or torch.isnan(got[:, 20]).all()
 
 
-@pytest.mark.parametrize("m", [65, 96, 97, 128])
+@pytest.mark.parametrize("m", [32, 33, 48, 49, 64, 65, 96, 97, 128])
 @pytest.mark.parametrize("di,k", [(16, 128), (80, 384), (8256, 256), (208, 1408)])
 @pytest.mark.parametrize("act", [{}, dict(act_alpha=1.7, act_limit=0.8)])
 def test_swiglu_is_that_of_plain_weights(m, di, k, act):
