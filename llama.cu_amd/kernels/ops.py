@@ -1024,6 +1024,9 @@ def tiles_choice(m: int, n: int, k: int, swiglu: bool = False) -> int:
     cu, columns = t.compute_units, (n + 127) // 128
     square = (m + 127) // 128 * columns
     if square <= cu:
+        finer = (m + t.tiles_library_tile - 1) // t.tiles_library_tile * columns      # the library's workgroups where it takes tiles of fewer rows
+        if not swiglu and k >= t.tiles_library_k and 8 * finer >= 7 * cu and finer <= cu:
+            return -1
         return 0 if 2 * square > cu else -1
     wide = (m + 255) // 256 * columns
     if swiglu:

@@ -101,6 +101,10 @@ class Tuning:
     tiles_rows: int = 256               # above so many rows (fewer have kernels of their own)
     tiles_swiglu_k: int = 2048          # SwiGLU with a longer K stays with the library (28672 x 4096: 83 and 95 at 300 rows, 290 and 306 at 1,500; 5632 x 2048 51.8 and 49.3
                                         # there, 59.7 and 52.4 at 2,014; 2816 x 1024 26.3 and 18.8)
+    tiles_library_tile: int = 96        # with a K from tiles_library_k on the library's tiles of 96 x 128, where they fill a round to seven eighths or more, are faster than one of
+    tiles_library_k: int = 4096         # 128 x 128 that is less full (4096 x 4096 at 640 / 700 / 765 rows 36.5 / 32.6 / 34.1 and 37.8 / 33.2 / 38.2; 4096 x 14336 112 / 100 / 106 and 130 / 113 / 129;
+                                        # 5120 x 4096 at 512 and 576 36.5 / 32.9 and 38.1 / 33.5), below and beyond not (4096 x 4096 at 576 / 800 36.6 / 39.8 and 33.5 / 31.7, 5120 x 4096 at 450 / 640 35.1 / 39.6 and
+                                        # 33.1 / 38.1), and with a shorter K neither (3072 x 2048 at 765 19.4 and 15.9, 2048 x 2816 at 1,280 22.6 and 20.6, at 1,400 21.1 and 21.7)
     tiles_short_k: int = 2048           # a round of 128 x 256 up to five eighths full only with a K up to this (4096 x 2048, 1,100 rows: 27.0 and 24.3; 2560 x 2048, 2,014: 27.8 and
                                         # 25.0; 4096 x 4096, 1,100: 42.6 and 42.8)
                                         # (a fuller round, with any K, is no gain in a whole prompt, where the card's power limit lets every kernel pay for another's work: 4096 x

@@ -77,3 +77,12 @@ def test_what_is_refused():
                 lambda: ops.gemm_tiles(x, w, 0, out=torch.empty(40, 66, dtype=torch.bfloat16, device="cuda")[:, 1:65])):
         with pytest.raises(ops.KernelError):
             bad()
+
+
+@pytest.mark.parametrize("m,n,k,shape", [(576, 4096, 4096, 0), (577, 4096, 4096, -1), (768, 4096, 4096, -1), (769, 4096, 4096, 0), (768, 4096, 4032, 0), (480, 5120, 4096, 0), (576, 5120, 4096, -1), (577, 5120, 4096, 0)])
+def test_where_finer_tiles_fill_a_round(m, n, k, shape):
+    """On a card of 256 compute units; on both sides of the lines between which the library's finer tiles are taken."""
+    from llama_cu_amd.kernels import ops
+    if ops.TUNING.compute_units != 256:
+        pytest.skip("the lines are those of 256 compute units")
+    assert ops.tiles_choice(m, n, k) == shape
