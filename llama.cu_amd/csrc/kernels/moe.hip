@@ -556,7 +556,8 @@ moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__
 
 // The least pairs (one to eight tokens of two, say): a workgroup looks for the blockIdx.y-th expert that any of them names, so the launch holds no
 // workgroups of experts without a pair, and has eight waves, a quarter of K and one of the two tiles each, with eight steps on their way: few workgroups then
-// ask for as much at a time as many would.  The sums are added up as in the kernel for few rows: the same bits.  What bounds it is the way of the numbers of the experts
+// ask for as much at a time as many would.  An expert's pairs go sixteen at a time; a token may name an expert more than once, so they may be more than the tokens, and what is beyond the
+// first sixteen goes through a loop of its own (one loop for all takes more registers: 14.8 us in the place of 10.8 for a token of two).  The sums are added up as in the kernel for few rows: the same bits.  What bounds it is the way of the numbers of the experts
 // and of their matrices' first lines through memory, one after the other.  One MI355X, both products, us, with the kernel for few rows everywhere and now: a token of two experts of
 // 2 x 1024 x 2048 with a shared one of 704 13.6 and 11.9, two tokens 19.5 and 17.5; a token of two of 2 x 1408 x 2048 14.4 and 11.9, of four of 2 x 512 x 2048 13.1 and 10.9, of one of
 // 2 x 3584 x 1024 16.5 and 13.1.  From some 400 workgroups on four waves with two tiles each read the rows half as often: four tokens of two of 2 x 1408 x 2048 23.7 and 25.4, eight of
@@ -572,15 +573,15 @@ moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict
     typedef Mma<T> M;
     typedef typename M::frag frag;
     constexpr bool GATED = MODE == MOE_UP_GATED, UP = MODE != MOE_DOWN;
-    constexpr int AHEAD = 8;
     __shared__ f32x4 red[4][2][WAVE];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, g = lane / 16, l16 = lane % 16;
     const int part = wave & 3, side = wave >> 2;
     const bool shared = (int)blockIdx.y == slots;
     const T *we = sw;
-    int count = total, flat = l16;                   // of row l16
+    int count = total;
+    unsigned long long pairs = 0;                    // the expert's, a bit each
     if (shared) {                                    // every token's rows [n, s_k] and a matrix of its own size
-        count /= top;
+        count /= top;                                // (at most MOE_SLOT_ROWS)
         top = 1;
         x = sx;
         N = s_n;
@@ -591,7 +592,7 @@ moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict
         out_stride = GATED ? s_n / 2 : out_stride;
         alpha = 1.f;
         limit = 0.f;
-        flat = min(l16, count - 1);
+        pairs = (1ull << count) - 1;
     } else {
         const int mine = lane < total ? ids[lane] : -1;
         bool first = mine >= 0 && mine < experts;    // (identity experts have no matrices)
@@ -600,61 +601,71 @@ moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict
         if ((int)blockIdx.y >= __popcll(which)) return;
         for (int y = 0; y < (int)blockIdx.y; ++y) which &= which - 1;
         const int e = __builtin_amdgcn_readlane(mine, __builtin_ctzll(which));
-        unsigned long long pairs = __ballot(mine == e);
+        pairs = __ballot(mine == e);
         count = __popcll(pairs);
-        for (int r = 0; r < min(l16, count - 1); ++r) pairs &= pairs - 1;
-        flat = __builtin_ctzll(pairs);
         we = w + (size_t)e * w_expert_stride;
     }
     if ((int)blockIdx.x * 32 >= N) return;
     const int tile0 = 2 * blockIdx.x, steps = (K + M::KSTEP - 1) / M::KSTEP, per = quarter_steps(steps);
     const int s0 = min(steps, part * per), s1 = min(steps, s0 + per);
-    const Unit<T, PACKED> wu(we, tile0 + side, N, K, steps, lane);
-    const T *xr = x + (size_t)(UP ? flat / top : flat) * x_stride + g * M::PER_LANE;
-    const float sc = MODE == MOE_UP ? wts[flat] : 1.f;
-    const int x_left = K - g * M::PER_LANE;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    frag a[AHEAD], b[AHEAD];
-    auto fetch = [&](int u, int s) {
-        a[u] = wu.load(s);
-        b[u] = s * M::KSTEP < x_left ? M::load(xr + s * M::KSTEP) : M::zero();
-    };
+    // sixteen of the pairs, of which `left` are left
+    auto pass = [&](auto ahead, int left) {
+        constexpr int AHEAD = decltype(ahead)::value;
+        const Unit<T, PACKED> wu(we, tile0 + side, N, K, steps, lane);
+        unsigned long long own = pairs;
+        for (int r = 0; r < min(l16, left - 1); ++r) own &= own - 1;
+        const int flat = __builtin_ctzll(own);       // of row l16
+        const T *xr = x + (size_t)(UP ? flat / top : flat) * x_stride + g * M::PER_LANE;
+        const float sc = MODE == MOE_UP ? wts[flat] : 1.f;
+        const int x_left = K - g * M::PER_LANE;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        frag a[AHEAD], b[AHEAD];
+        auto fetch = [&](int u, int s) {
+            a[u] = wu.load(s);
+            b[u] = s * M::KSTEP < x_left ? M::load(xr + s * M::KSTEP) : M::zero();
+        };
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u)
-        if (s0 + u < s1) fetch(u, s0 + u);
-    for (int s = s0; s < s1; s += AHEAD) {
+        for (int u = 0; u < AHEAD; ++u)
+            if (s0 + u < s1) fetch(u, s0 + u);
+        for (int s = s0; s < s1; s += AHEAD) {
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-            if (s + u >= s1) break;
-            acc = M::mma(a[u], MODE == MOE_UP ? M::scaled(b[u], sc) : b[u], acc);
-            if (s + u + AHEAD < s1) fetch(u, s + u + AHEAD);
+            for (int u = 0; u < AHEAD; ++u) {
+                if (s + u >= s1) break;
+                acc = M::mma(a[u], MODE == MOE_UP ? M::scaled(b[u], sc) : b[u], acc);
+                if (s + u + AHEAD < s1) fetch(u, s + u + AHEAD);
+            }
         }
-    }
-    red[part][side][lane] = acc;
-    __syncthreads();
-    // the first wave stores (with two products' sums the first two, one each): four neighbouring features of a row a lane
-    if (wave >= (GATED ? 1 : 2)) return;
-    const f32x4 v = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
-    const int dst = !UP && add ? flat / top : flat;
-    if (l16 >= count) return;
-    if constexpr (GATED) {
-        const f32x4 up = ((red[0][1][lane] + red[1][1][lane]) + red[2][1][lane]) + red[3][1][lane];
-        Quad<T> q;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gate_up_of(v[i], up[i], alpha, limit));
-        *(Quad<T> *)(out_t + (size_t)dst * out_stride + tile0 * 8 + 4 * g) = q;
-    } else {
-        const int col = (tile0 + wave) * 16 + 4 * g; // (N is a multiple of 4)
-        if (col >= N) return;
-        if constexpr (MODE == MOE_UP) {
+        if (left < count) __syncthreads();           // the sums of the rows before have been read
+        red[part][side][lane] = acc;
+        __syncthreads();
+        // the first wave stores (with two products' sums the first two, one each): four neighbouring features of a row a lane
+        if (wave >= (GATED ? 1 : 2) || l16 >= left) return;
+        const f32x4 v = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
+        const int dst = !UP && add ? flat / top : flat;
+        if constexpr (GATED) {
+            const f32x4 up = ((red[0][1][lane] + red[1][1][lane]) + red[2][1][lane]) + red[3][1][lane];
             Quad<T> q;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gelu_erf(v[i]));
-            *(Quad<T> *)(out_t + (size_t)dst * out_stride + col) = q;
+            for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gate_up_of(v[i], up[i], alpha, limit));
+            *(Quad<T> *)(out_t + (size_t)dst * out_stride + tile0 * 8 + 4 * g) = q;
         } else {
-            f32x4 *o = (f32x4 *)(out_f + (size_t)dst * out_stride + col);
-            *o = add ? *o + v : v;
+            const int col = (tile0 + wave) * 16 + 4 * g; // (N is a multiple of 4)
+            if (col >= N) return;
+            if constexpr (MODE == MOE_UP) {
+                Quad<T> q;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q.v[i] = from_f32<T>(gelu_erf(v[i]));
+                *(Quad<T> *)(out_t + (size_t)dst * out_stride + col) = q;
+            } else {
+                f32x4 *o = (f32x4 *)(out_f + (size_t)dst * out_stride + col);
+                *o = add ? *o + v : v;
+            }
         }
+    };
+    pass(Int<8>(), count);
+    for (int left = count - 16; left > 0; left -= 16) {
+        for (int r = 0; r < 16; ++r) pairs &= pairs - 1;
+        pass(Int<2>(), left);
     }
 }
 

@@ -289,3 +289,67 @@ def test_the_experts_that_any_pair_names(dtype, n, top, experts, identity, d, ff
     finally:
         lib.lcu_moe_tile_rows = real
     assert torch.equal(got, want)
+
+
+def experts_of(experts, d, ff, tdt, gated):
+    """Packed matrices of ``experts`` experts, and those of a shared one."""
+    from llama_cu_amd.kernels import ops
+    sff = 48
+    rows = lambda e, f, seed: rnd(e, f, d, seed=seed, std=d ** -0.5).to(tdt).cuda()
+    first = ops.gated_rows(rows(experts, ff, 3), rows(experts, ff, 4)) if gated else rows(experts, ff, 3)
+    up, down = ops.pack_experts(first), ops.pack_experts(rnd(experts, d, ff, seed=5, std=ff ** -0.5).to(tdt).cuda())
+    return up, down, (ops.pack_experts(ops.gated_rows(rows(1, sff, 6), rows(1, sff, 7))), ops.pack_experts(rnd(1, d, sff, seed=8, std=sff ** -0.5).to(tdt).cuda()))
+
+
+def beside_tiles(h, ids, wts, up, down, monkeypatch, **kw):
+    """``moe_experts`` as it chooses and from tiles of 16 sorted rows, whatever memory they are given full of NaN beforehand."""
+    from llama_cu_amd.kernels import build, ops
+    empty = torch.empty
+
+    def poisoned(*a, **k):
+        t = empty(*a, **k)
+        return t.fill_(float("nan")) if t.is_floating_point() else t
+    lib = build.load("moe")
+    outs = []
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", poisoned)
+        for tiles in (lib.lcu_moe_tile_rows, lambda *a: 16):
+            m.setattr(lib, "lcu_moe_tile_rows", tiles)
+            outs.append(torch.zeros(h.shape, device="cuda"))
+            ops.moe_experts(h, ids, wts, up, down, outs[-1], **kw)
+    return outs
+
+
+# 9 tokens of two, all on one expert (18 pairs); 16 of four on two experts (32 each), on one (64) and with a last turn of a single pair (17)
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("n,top,experts,named", [(9, 2, 2, [[0, 0]] * 9), (16, 4, 8, [[3, 5, 5, 3]] * 16), (16, 4, 4, [[1] * 4] * 16),
+                                                 (16, 2, 40, [[7, 7]] + [[7, 8]] * 15)])
+@pytest.mark.parametrize("d,ff", [(72, 32), (520, 144)])
+def test_an_expert_that_a_token_names_more_than_once(dtype, gated, n, top, experts, named, d, ff, monkeypatch):
+    """An expert's pairs may be more than the step's tokens: every one of them is multiplied, with the bits of tiles of 16 sorted rows."""
+    from llama_cu_amd.kernels import ops
+    tdt = TYPES[dtype]
+    up, down, shared = experts_of(experts, d, ff, tdt, gated)
+    h, wts = rnd(n, d, seed=1).to(tdt).cuda(), torch.rand(n, top, generator=torch.Generator().manual_seed(2)).cuda()
+    kw = dict(gated=True, fresh=True, shared_expert=shared if ops.moe_shared_beside(n, top, experts, up, down) else None) if gated else {}
+    assert ops.moe_tile_rows(ops._type(h, "rows"), n * top, experts, up.shape[1], d, ff) == 0
+    got, want = beside_tiles(h, torch.tensor(named, dtype=torch.int32).cuda(), wts, up, down, monkeypatch, **kw)
+    assert torch.isfinite(want).all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_row_of_nan_among_rows_that_share_an_expert(dtype, monkeypatch):
+    """The router gives a row of NaN its first expert in every place; what the other rows, which name that expert too, get from it does not change."""
+    from llama_cu_amd.kernels import ops
+    tdt, n, top, experts, d, ff = TYPES[dtype], 16, 4, 8, 72, 32
+    up, down, shared = experts_of(experts, d, ff, tdt, True)
+    h, router = rnd(n, d, seed=1).to(tdt).cuda(), rnd(experts, d, seed=2).cuda()
+    bias = torch.zeros(experts, device="cuda")
+    bias[0] = 100.0                                          # every row names expert 0
+    healthy = ops.moe_route(h, router, top, bias)
+    h[0] = float("nan")
+    ids, wts = ops.moe_route(h, router, top, bias)
+    assert (ids[1:] == healthy[0][1:]).all() and (ids == 0).sum() == n + top - 1
+    got, want = beside_tiles(h, ids, wts, up, down, monkeypatch, gated=True, fresh=True, shared_expert=shared)
+    assert torch.isnan(got[0]).all() and torch.isfinite(got[1:]).all() and torch.equal(got[1:], want[1:])
