@@ -1036,7 +1036,7 @@ def tiles_choice(m: int, n: int, k: int, swiglu: bool = False) -> int:
 
 def tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gemm_tiles`` takes these rows and this plain weight."""
-    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.stride(1) == 1 and w.is_contiguous()
+    return (x.is_cuda and x.device == w.device and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.stride(1) == 1 and w.is_contiguous()
             and x.shape[1] % 64 == 0 and w.shape[0] % 16 == 0 and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and (x.shape[0] + 256) * x.stride(0) < 1 << 31 and (w.shape[0] + 256) * w.shape[1] < 1 << 31)
 
@@ -1045,8 +1045,7 @@ def gemm_tiles(x: torch.Tensor, w: torch.Tensor, shape: int, out: Optional[torch
                act_alpha: float = 1.0, act_limit: float = 0.0, known: bool = False) -> torch.Tensor:
     """``x @ w.T`` for many bfloat16 rows, ``w [n, k]`` plain; ``shape``: see ``TILES``.  ``out [m, n]`` bfloat16 or float32; ``swiglu``: ``w`` holds gate rows, then up rows,
     ``out [m, n / 2]`` bfloat16 (the limited activation with ``act_limit`` > 0).  ``known``: the caller has asked ``tiles_supported``."""
-    if not known:
-        _gpu(x, w, out)
+    _gpu(x, w, out)
     if not 0 <= shape < len(TILES) or not (known or tiles_supported(x, w)):
         raise KernelError(f"gemm_tiles: x {tuple(x.shape)} {x.dtype} with w {tuple(w.shape)} {w.dtype} is not supported")
     m, k = x.shape

@@ -86,3 +86,19 @@ def test_where_finer_tiles_fill_a_round(m, n, k, shape):
     if ops.TUNING.compute_units != 256:
         pytest.skip("the lines are those of 256 compute units")
     assert ops.tiles_choice(m, n, k) == shape
+
+
+def test_operands_on_other_devices_are_refused():
+    """A weight, or an output, in host memory: the library's error from ``linear``, the kernel's own from ``gemm_tiles``, and no launch."""
+    from llama_cu_amd.kernels import ops
+    from llama_cu_amd.parts.linear import linear, tiles_swiglu_shape
+    x, w = rnd(1100, 2048, seed=1).bfloat16().cuda(), rnd(2048, 2048, seed=2).bfloat16().cuda()
+    assert ops.tiles_choice(1100, 2048, 2048) >= 0 and tiles_swiglu_shape(x, w) >= 0 and tiles_swiglu_shape(x, w.cpu()) == -1
+    out = torch.empty(1100, 2048, dtype=torch.bfloat16)
+    for bad in (lambda: linear(x, w.cpu()), lambda: linear(x, w, out=out), lambda: linear(x, w.cpu(), out_dtype=torch.float32)):
+        with pytest.raises(RuntimeError):
+            bad()
+    for known in (False, True):
+        for bad in (lambda: ops.gemm_tiles(x, w.cpu(), 0, known=known), lambda: ops.gemm_tiles(x, w, 0, out=out, known=known)):
+            with pytest.raises(ops.KernelError):
+                bad()

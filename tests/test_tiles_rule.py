@@ -1,0 +1,16 @@
+"""Which products go to the kernel in tiles: the rule alone, which needs no GPU."""
+from __future__ import annotations
+
+import torch
+
+from llama_cu_amd.kernels import ops
+
+
+def rows(m, k, device="cpu"):
+    return torch.empty(m, k, dtype=torch.bfloat16, device=device)
+
+
+def test_operands_that_are_not_on_one_gpu():
+    """The kernel takes addresses, so operands in host memory, or on two devices, are left to the library, which refuses them."""
+    for x, w in ((rows(300, 2048), rows(2048, 2048)), (rows(300, 2048, "meta"), rows(2048, 2048)), (rows(300, 2048), rows(2048, 2048, "meta"))):
+        assert not ops.tiles_supported(x, w)
