@@ -1019,7 +1019,7 @@ def tiles_choice(m: int, n: int, k: int, swiglu: bool = False) -> int:
     else -1.  It is where its workgroups fill more than half of a round and, mostly, no more than one (measured from 200 to 4,000 rows, 1024 x 1024 to 28672 x 4096;
     the numbers are ``TUNING``'s)."""
     t = TUNING
-    if m <= t.tiles_rows or k % 64 or n % 64 or (swiglu and k > t.tiles_swiglu_k):
+    if m <= t.tiles_rows or k <= 0 or k % 64 or n % 64 or (swiglu and k > t.tiles_swiglu_k):
         return -1
     cu, columns = t.compute_units, (n + 127) // 128
     square = (m + 127) // 128 * columns

@@ -102,3 +102,11 @@ def test_operands_on_other_devices_are_refused():
         for bad in (lambda: ops.gemm_tiles(x, w.cpu(), 0, known=known), lambda: ops.gemm_tiles(x, w, 0, out=out, known=known)):
             with pytest.raises(ops.KernelError):
                 bad()
+
+
+def test_rows_of_no_width():
+    from llama_cu_amd.parts.linear import linear
+    x, w = torch.empty(1100, 0, dtype=torch.bfloat16, device="cuda"), torch.empty(2048, 0, dtype=torch.bfloat16, device="cuda")
+    for dtype in (torch.bfloat16, torch.float32):
+        y = linear(x, w, out_dtype=dtype)
+        assert y.shape == (1100, 2048) and y.dtype == dtype and (y == 0).all()

@@ -14,3 +14,9 @@ def test_operands_that_are_not_on_one_gpu():
     """The kernel takes addresses, so operands in host memory, or on two devices, are left to the library, which refuses them."""
     for x, w in ((rows(300, 2048), rows(2048, 2048)), (rows(300, 2048, "meta"), rows(2048, 2048)), (rows(300, 2048), rows(2048, 2048, "meta"))):
         assert not ops.tiles_supported(x, w)
+
+
+def test_products_over_nothing():
+    """A sum of no terms is zeros, which the library gives; the kernel refuses it."""
+    for swiglu in (False, True):
+        assert ops.tiles_choice(1100, 2048, 0, swiglu) == -1 and ops.tiles_choice(1100, 0, 2048, swiglu) == -1
