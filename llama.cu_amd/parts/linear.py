@@ -67,6 +67,12 @@ def _plain_rows(out: torch.Tensor) -> bool:
     return out.dtype in (torch.bfloat16, torch.float32) and out.dim() == 2 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0
 
 
+def _tiles_out(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether the product in tiles writes into ``out`` (the library makes one of another shape fit, and refuses one on another device)."""
+    return (out.device == x.device and out.shape == (x.shape[0], weight.shape[0]) and _plain_rows(out)
+            and out.stride(0) * out.element_size() % 16 == 0)
+
+
 def linear(x: torch.Tensor, weight: Union[torch.Tensor, Weight], out_dtype: Optional[torch.dtype] = None,
            out: Optional[torch.Tensor] = None, accumulate: bool = False) -> torch.Tensor:
     """``out (+)= x @ weight.T``.  ``accumulate`` adds into a float32 ``out`` in 32-bit."""
@@ -86,7 +92,7 @@ def linear(x: torch.Tensor, weight: Union[torch.Tensor, Weight], out_dtype: Opti
         return ops.gemm_skinny(x, weight, out=out, out_dtype=out_dtype, accumulate=accumulate)
     if all_bf16 and x.shape[0] > ops.TUNING.tiles_rows and not accumulate and x.dim() == 2 and out_dtype in (torch.bfloat16, torch.float32):
         shape = ops.tiles_choice(x.shape[0], weight.shape[0], weight.shape[1])
-        if shape >= 0 and ops.tiles_supported(x, weight) and (out is None or out.device == x.device and _plain_rows(out) and out.stride(0) * out.element_size() % 16 == 0):
+        if shape >= 0 and ops.tiles_supported(x, weight) and (out is None or _tiles_out(out, x, weight)):
             return ops.gemm_tiles(x, weight, shape, out=out, out_dtype=out_dtype, known=True)
     if all_bf16 and out_dtype == torch.bfloat16 and not accumulate:
         if out is None:

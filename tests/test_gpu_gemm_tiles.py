@@ -110,3 +110,15 @@ def test_rows_of_no_width():
     for dtype in (torch.bfloat16, torch.float32):
         y = linear(x, w, out_dtype=dtype)
         assert y.shape == (1100, 2048) and y.dtype == dtype and (y == 0).all()
+
+
+def test_an_output_of_another_shape():
+    """The library makes it fit, with a warning; the kernel in tiles would refuse it."""
+    from llama_cu_amd.parts.linear import linear
+    x, w = rnd(1100, 128, seed=1).bfloat16().cuda(), rnd(2048, 128, seed=2).bfloat16().cuda()
+    for shape in ((1100, 2056), (1104, 2048)):
+        out = torch.empty(shape, dtype=torch.bfloat16, device="cuda")
+        with pytest.warns(UserWarning, match="resized"):
+            assert linear(x, w, out=out) is out
+        assert out.shape == (1100, 2048)
+        assert_close(out, x.double() @ w.double().T, BF16_REL, "resized")
