@@ -92,7 +92,8 @@ def linear(x: torch.Tensor, weight: Union[torch.Tensor, Weight], out_dtype: Opti
         return ops.gemm_skinny(x, weight, out=out, out_dtype=out_dtype, accumulate=accumulate)
     if all_bf16 and x.shape[0] > ops.TUNING.tiles_rows and not accumulate and x.dim() == 2 and out_dtype in (torch.bfloat16, torch.float32):
         shape = ops.tiles_choice(x.shape[0], weight.shape[0], weight.shape[1])
-        if shape >= 0 and ops.tiles_supported(x, weight) and (out is None or _tiles_out(out, x, weight)):
+        asked = torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)        # (the kernel has no gradient)
+        if shape >= 0 and not asked and ops.tiles_supported(x, weight) and (out is None or _tiles_out(out, x, weight)):
             return ops.gemm_tiles(x, weight, shape, out=out, out_dtype=out_dtype, known=True)
     if all_bf16 and out_dtype == torch.bfloat16 and not accumulate:
         if out is None:

@@ -122,3 +122,15 @@ def test_an_output_of_another_shape():
             assert linear(x, w, out=out) is out
         assert out.shape == (1100, 2048)
         assert_close(out, x.double() @ w.double().T, BF16_REL, "resized")
+
+
+def test_a_product_that_is_differentiated():
+    """Where a gradient is asked for, ``linear`` of many bfloat16 rows stays the library's, which has one."""
+    from llama_cu_amd.parts.linear import linear
+    x, w = rnd(1100, 128, seed=1).bfloat16().cuda(), rnd(2048, 128, seed=2).bfloat16().cuda()
+    g = rnd(1100, 2048, seed=3).bfloat16().cuda()
+    grads = torch.autograd.grad(linear(x.requires_grad_(), w.requires_grad_()), (x, w), g)
+    assert_close(grads[0], g.double() @ w.double(), BF16_REL, "x")
+    assert_close(grads[1], g.double().T @ x.double(), BF16_REL, "w")
+    with torch.no_grad():
+        assert not linear(x, w).requires_grad
