@@ -210,6 +210,13 @@ static int gt_go(const void *X, int ldx, const void *W, void *Y, int ldy, int M,
     const int up_rows = N / 2;
     const int tiles = ((M + S::T - 1) / S::T) * ((N + S::F - 1) / S::F);
     constexpr int bytes = S::LDS * 16;
+    static_assert(bytes > 64 * 1024, "more LDS than a launch gets unasked");
+    static bool asked = false;
+    if (!asked) {
+        const hipError_t e = hipFuncSetAttribute((const void *)gemm_tiles_kernel<S, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        if (e != hipSuccess) return (int)e;
+        asked = true;
+    }
     gemm_tiles_kernel<S, EPI><<<dim3((tiles + 7) / 8 * 8), dim3(S::THREADS), bytes, stream>>>((const bf16_t *)X, ldx, (const bf16_t *)W, Y, ldy, M, N, K, up_rows, alpha, limit);
     LCU_LAUNCH_CHECK();
     return LCU_OK;

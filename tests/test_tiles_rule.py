@@ -1,9 +1,13 @@
 """Which products go to the kernel in tiles: the rule alone, which needs no GPU."""
 from __future__ import annotations
 
+import shutil
+import subprocess
+
+import pytest
 import torch
 
-from llama_cu_amd.kernels import ops
+from llama_cu_amd.kernels import build, ops
 
 
 def rows(m, k, device="cpu"):
@@ -20,3 +24,12 @@ def test_products_over_nothing():
     """A sum of no terms is zeros, which the library gives; the kernel refuses it."""
     for swiglu in (False, True):
         assert ops.tiles_choice(1100, 2048, 0, swiglu) == -1 and ops.tiles_choice(1100, 0, 2048, swiglu) == -1
+
+
+def test_the_kernel_asks_for_its_lds():
+    """Its tiles take 128 to 160 KB of LDS, and a launch is promised 64 KB unless it asks: the library calls what asks (a runtime that does not hold launches to the
+    promise runs the kernel either way)."""
+    if not shutil.which("nm"):
+        pytest.skip("no nm")
+    names = subprocess.run(["nm", "-D", "--undefined-only", build.build("gemm_tiles")], check=True, capture_output=True, text=True).stdout
+    assert "hipFuncSetAttribute" in names
