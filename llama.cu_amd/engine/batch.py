@@ -83,7 +83,8 @@ class StepContext:
 
     @property
     def decode_only(self) -> bool:
-        return self.max_q_len == 1
+        """Every request feeds one token: row r is request r's (a request that feeds none would move the rows behind it)."""
+        return self.max_q_len == 1 and self.n == self.n_req
 
 
 class BatchBuilder:

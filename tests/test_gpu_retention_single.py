@@ -37,3 +37,17 @@ def test_the_same_bits_as_beside_a_longer_request(dtype, heads, d, dv, rot, inte
     assert torch.equal(got, want[:n]) and torch.isfinite(got.float()).all()
     assert torch.equal(one[:7], two[:7]) and torch.equal(one[7], start[7]) and torch.equal(one[3], start[3]) and torch.equal(one[5], start[5])
     assert not torch.equal(one[4], start[4])
+
+
+def test_a_request_that_feeds_nothing():
+    """A step of single tokens in which a request has none: its rows are not the requests' in order, so it goes through the kernels for any step; the others' outputs and states are
+    those of a step without it, its own state stays."""
+    from llama_cu_amd.kernels import ops
+    heads, d, dv = 2, 64, 64
+    hk, hv = heads * d, heads * dv
+    off = {"q": 0, "k": hk, "v": 2 * hk, "g": 2 * hk + hv}
+    rows, decay, start = rnd(2, 2 * hk + 2 * hv, seed=1).cuda(), torch.tensor([0.9, 0.999]).cuda(), rnd(3, heads, d, dv, seed=2).cuda()
+    one, two = start.clone(), start.clone()
+    got = ops.retention(rows, off, decay, one, hand_step([1, 0, 1], [5, 4, 1], [2, 0, 1]), heads, d, dv, 0.3, 1e-5, torch.float32)
+    want = ops.retention(rows, off, decay, two, hand_step([1, 1], [5, 1], [2, 1]), heads, d, dv, 0.3, 1e-5, torch.float32)
+    assert torch.equal(got, want) and torch.equal(one, two) and torch.equal(one[0], start[0])
