@@ -695,10 +695,13 @@ LCU_API int lcu_gemm_mid_planes(int K, int slices) {
     return (steps + per - 1) / per;
 }
 
+// Whether the rows of X span less than 2^32 bytes: a load's place in them is 32 bits.
+static bool mid_rows_fit(int M, int ldx, int K) { return (long long)(M - 1) * ldx + K < 1ll << 31; }
+
 static int mid_bf16(const void *X, int ldx, const void *W, int ldw, void *Y, int ldy, int M, int N, int K, int epilogue,
                     int slices, int w_packed, const MidScale &sc, hipStream_t stream) {
     if (M <= 0 || N <= 0) return LCU_OK;
-    if (M > 256 || (sc.sumsq_in && M > 64) || K <= 0 || K % 128 || N % 16 || ldx % 8 || ldx < K || slices <= 0 || slices > 64) return LCU_BAD_ARGUMENT;
+    if (M > 256 || (sc.sumsq_in && M > 64) || K <= 0 || K % 128 || N % 16 || ldx % 8 || ldx < K || !mid_rows_fit(M, ldx, K) || slices <= 0 || slices > 64) return LCU_BAD_ARGUMENT;
     if (!w_packed && (ldw % 8 || ldw < K)) return LCU_BAD_ARGUMENT;
     if ((uintptr_t)X % 16 || (uintptr_t)W % 16 || (uintptr_t)Y % 16 || (uintptr_t)sc.sumsq_in % 16) return LCU_BAD_ARGUMENT;
     switch (epilogue) {
@@ -883,7 +886,7 @@ LCU_API int lcu_gemm_mid_bf16_qkv_rope(const void *X, int ldx, const void *W, in
                                        int w_packed, hipStream_t stream) {
     if (M <= 0) return LCU_OK;
     if (M > 256 || K <= 0 || K % 128 || heads <= 0 || kv_heads <= 0 || head_dim <= 0 || head_dim % 32 || page <= 0 || page % 8 ||
-        !q_out || !positions || !cos_t || !sin_t || max_pos <= 0 || !cache || ldq < heads * head_dim || ldx % 8 || ldx < K)
+        !q_out || !positions || !cos_t || !sin_t || max_pos <= 0 || !cache || ldq < heads * head_dim || ldx % 8 || ldx < K || !mid_rows_fit(M, ldx, K))
         return LCU_BAD_ARGUMENT;
     if (!w_packed && (ldw % 8 || ldw < K)) return LCU_BAD_ARGUMENT;
     if ((uintptr_t)X % 16 || (uintptr_t)W % 16) return LCU_BAD_ARGUMENT;
@@ -1041,7 +1044,7 @@ LCU_API int lcu_gemm_mid_bf16_add_norm(const void *X, int ldx, const void *W, in
                                        const void *norm_w, int norm_w_type, void *h_out, int ldh, float *sumsq_out, int w_packed,
                                        float res_scale, hipStream_t stream) {
     if (M <= 0 || N <= 0) return LCU_OK;
-    if (M > 64 || K <= 0 || K % 128 || N % 16 || ldx % 8 || ldx < K || ldr < N || ldr % 4 || ldh < N || ldh % 4 || !residual || !norm_w ||
+    if (M > 64 || K <= 0 || K % 128 || N % 16 || ldx % 8 || ldx < K || !mid_rows_fit(M, ldx, K) || ldr < N || ldr % 4 || ldh < N || ldh % 4 || !residual || !norm_w ||
         !h_out || !sumsq_out || (norm_w_type != LCU_F32 && norm_w_type != LCU_BF16))
         return LCU_BAD_ARGUMENT;
     if (!w_packed && (ldw % 8 || ldw < K)) return LCU_BAD_ARGUMENT;

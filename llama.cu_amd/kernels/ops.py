@@ -911,11 +911,12 @@ MID_MAX_SCALED_ROWS = 64
 
 def mid_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gemm_mid`` takes these operands: up to 256 bfloat16 rows with K a multiple of 128
-    and a bfloat16 weight of a multiple of 16 rows."""
+    and a bfloat16 weight of a multiple of 16 rows.  (A load's place in the rows is 32 bits.)"""
     return (x.is_cuda and w.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
             and w.dim() == 2 and 0 < x.shape[0] <= MID_MAX_ROWS and x.shape[1] == w.shape[1] and w.shape[1] % 128 == 0
             and w.shape[0] % 16 == 0 and x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0
-            and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+            and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (x.shape[0] - 1) * x.stride(0) + x.shape[1] < 1 << 31)
 
 
 def mid_f32_preferred(m: int, n: int, k: int) -> bool:

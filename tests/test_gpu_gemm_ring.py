@@ -57,3 +57,20 @@ def test_many_features_uncut(m, n, k):
     x, w = torch.randn(m, k, device="cuda", generator=g).bfloat16(), (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).bfloat16()
     assert ops.mid_f32_preferred(m, n, k)
     assert torch.equal(ops.gemm_mid(x, ops.pack_weight(w), slices=1, packed=True), ops.gemm_mid(x, w, slices=1))
+
+
+def test_rows_that_span_more_than_a_load_reaches():
+    """65 to 128 rows of 32-bit logits taken out of longer sequences, 4 GiB and more from the first to the last: ``linear`` leaves them to the library, and the kernel refuses
+    them.  (A load's place in the rows is 32 bits.)"""
+    from llama_cu_amd.kernels import ops
+    from llama_cu_amd.parts.linear import Weight, linear
+    m, k, n, apart = 100, 2048, 49152, (1 << 31) // 99 + 8 & ~7
+    room = torch.empty((m - 1) * apart + k, dtype=torch.bfloat16, device="cuda")
+    x = room.as_strided((m, k), (apart, 1))
+    x.copy_(rnd(m, k, seed=1))
+    w = Weight(rnd(n, k, seed=2, std=k ** -0.5).bfloat16().cuda())
+    assert ops.mid_f32_preferred(m, n, k) and not ops.mid_supported(x, w.plain) and ops.mid_supported(room.as_strided((m, k), (apart - 32, 1)), w.plain)
+    want = x.double() @ w.plain.double().T
+    assert (linear(x, w, out_dtype=torch.float32) - want).abs().max() < 1e-4
+    with pytest.raises(ops.KernelError):
+        ops.gemm_mid(x, w.packed, slices=1, packed=True)

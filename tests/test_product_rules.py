@@ -1,6 +1,7 @@
-"""Which products go to the kernel in tiles: the rule alone, which needs no GPU."""
+"""What the products' rules and entries take and refuse, which needs no GPU."""
 from __future__ import annotations
 
+import ctypes
 import shutil
 import subprocess
 
@@ -33,3 +34,11 @@ def test_the_kernel_asks_for_its_lds():
         pytest.skip("no nm")
     names = subprocess.run(["nm", "-D", "--undefined-only", build.build("gemm_tiles")], check=True, capture_output=True, text=True).stdout
     assert "hipFuncSetAttribute" in names
+
+
+def test_rows_that_span_more_than_a_load_reaches():
+    """The product that shares rows through LDS refuses rows of 4 GiB and more from the first to the last before it launches anything (the addresses are none)."""
+    lib, p, f = build.load("gemm_mid"), ctypes.c_void_p(4096), ctypes.c_float
+    apart = (1 << 31) // 99 + 8 & ~7
+    for packed, epilogue in ((1, 1), (0, 1), (1, 2), (1, 0)):
+        assert lib.lcu_gemm_mid_bf16(p, apart, p, 128, p, 64, 100, 64, 128, epilogue, 1, packed, f(1), f(0), None) == -1
