@@ -17,7 +17,7 @@
 //
 //   decode kernel   one token per request, v_mfma_f32_16x16x32_bf16 (blocks of 16 rows; a lane
 //                   owns row lane % 16 and 8 of each 32 keys, neighbours in memory).  A
-//                   workgroup of 8 waves (4 with sixteen rows) takes one request and
+//                   workgroup of 8 or 4 waves (decode_waves) takes one request and
 //                   key/value head and one of `n_splits` equal parts of its keys; the
 //                   waves take 32-key steps in turn and merge through LDS; parts are
 //                   merged by a second kernel.
@@ -27,6 +27,7 @@
 //                   step are copied to LDS once and shared by the waves.
 #include <mutex>
 
+#include <type_traits>
 #include <utility>
 
 #include "attention_static.h"
@@ -145,17 +146,18 @@ struct KVFrag {
 __device__ __forceinline__ int mix_key(int grp) { return 16 * (grp & 1) + 8 * (grp >> 1); }
 
 // The two pages that hold the keys k0 .. k0+15 and k0+16 .. k0+31 and the places of these in them, asked for a step before the loads that want them.
-// (Pages of 16 tokens need no division, which would stand between a workgroup's start and its first load: 0.4 us.)
+// PAGE16: pages of 16 tokens, which need no division: 0.4 us between a workgroup's start and its first load, 0.2 us of a few keys even where a branch leads past it.
 struct KVPages {
     int page[2], tok[2];
 };
+template <bool PAGE16>
 __device__ __forceinline__ KVPages kv_pages(const int *__restrict__ bt, int max_pages, int page, int k0) {
     KVPages at;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         int i = (k0 + 16 * t) / 16;
         at.tok[t] = 0;
-        if (page != 16) {
+        if (!PAGE16) {
             const int tile = i, tiles = page / 16;
             i = tile / tiles;
             at.tok[t] = 16 * (tile - i * tiles);
@@ -320,13 +322,9 @@ __device__ __forceinline__ void load_q(const bf16_t *__restrict__ qrow, bool val
 }
 
 // ============================================================================ decode
-// WAVES: 8, or 4 where no request has more keys than four waves take in one step each, or where the rows of a workgroup are sixteen (their sums of eight waves would be more LDS than a
-// launch gets unasked).  What bounds it over few
-// requests is how much one compute unit asks for at a time: with 4 waves everywhere a wave walked twice the steps, 2.5 us each: 8 requests of 1,024
-// keys, 16 heads of 128 over 4, 18.1 us and 14.9 with 8, 64 requests of 150 to 1,500, 32 heads over 8, 40.8 and 37.0; 60 requests of 8 to 19 keys, 2.3 us less with 4, 8 of 32 keys 3.7 and 3.9
-// (16 waves want more than their 128 registers each).
-constexpr int DEC_FEW_KEYS = 128;
-template <int DH, int WAVES>
+// WAVES: 8 or 4 (decode_waves, below).  What bounds the kernel over few requests is how much one compute unit asks for at a time: 8 requests of 1,024 keys, 16 heads of 128 over 4,
+// 18.1 us with 4 waves and 14.9 with 8 (16 waves want more than their 128 registers each).
+template <int DH, int WAVES, bool PAGE16>
 __global__ void __launch_bounds__(WAVES *WAVE, 2)
 attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__restrict__ out, int out_stride,
                         const bf16_t *__restrict__ cache, const int *__restrict__ block_table, int max_pages,
@@ -351,10 +349,7 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     // without a window a request's one part begins with its first key: its first pages are asked for together with its length
     const bool known = window == 0 && n_splits == 1;
     KVPages ida, idb;
-    if (known) {
-        ida = kv_pages(bt, max_pages, page, wave * 32);
-        idb = kv_pages(bt, max_pages, page, (wave + WAVES) * 32);
-    }
+    if (known) ida = kv_pages<PAGE16>(bt, max_pages, page, wave * 32);
     const int token = q_start[r];
     const int p = ctx_len[r] - 1;
     const int lo = first_key(p, window);
@@ -382,17 +377,21 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     // step after it are known
     KVFrag<DH> fa, fb;
     int blk = b0 + wave;
+    // up to four steps the other waves have none, and go: nobody waits for them, and the merge leaves them out
+    const int live = WAVES > 4 && b1 - b0 <= 4 ? 4 : WAVES;
+    if (wave >= live) return;
     if (!known) {
-        ida = kv_pages(bt, max_pages, page, blk * 32);
-        idb = kv_pages(bt, max_pages, page, (blk + WAVES) * 32);
+        ida = kv_pages<PAGE16>(bt, max_pages, page, blk * 32);
+        idb = kv_pages<PAGE16>(bt, max_pages, page, (blk + WAVES) * 32);
     }
     if (blk < b1) load_kv<DH>(fa, cache, ida, page, page_elems, nkvh, kvh, l16, grp);
+    if (known && blk + WAVES < b1) idb = kv_pages<PAGE16>(bt, max_pages, page, (wave + WAVES) * 32);
     for (; blk < b1; blk += 2 * WAVES) {
         const int nb = blk + WAVES, nb2 = blk + 2 * WAVES;
         if (nb < b1) load_kv<DH>(fb, cache, idb, page, page_elems, nkvh, kvh, l16, grp);
         if (nb2 < b1) {                                // (numbers that nobody wants would be waited for at the merge all the same)
-            ida = kv_pages(bt, max_pages, page, nb2 * 32);
-            idb = kv_pages(bt, max_pages, page, (nb2 + WAVES) * 32);
+            ida = kv_pages<PAGE16>(bt, max_pages, page, nb2 * 32);
+            idb = kv_pages<PAGE16>(bt, max_pages, page, (nb2 + WAVES) * 32);
         }
         attn_block<DH, 1>(fa, blk * 32, blk * 32 + 31 > p || blk * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
         if (nb2 < b1) load_kv<DH>(fa, cache, ida, page, page_elems, nkvh, kvh, l16, grp);
@@ -417,47 +416,52 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
     }
     __syncthreads();
     const bool four = ((uintptr_t)out & 7) == 0;       // (out_stride is a multiple of four)
-    for (int idx = threadIdx.x; idx < rows * (DH / 4); idx += WAVES * WAVE) {
-        const int row = idx / (DH / 4), d = idx % (DH / 4) * 4;
-        f32x4 ml[2][WAVES / 4];
+    auto merge = [&](auto waves) {
+        constexpr int N = decltype(waves)::value;
+        for (int idx = threadIdx.x; idx < rows * (DH / 4); idx += N * WAVE) {
+            const int row = idx / (DH / 4), d = idx % (DH / 4) * 4;
+            f32x4 ml[2][N / 4];
 #pragma unroll
-        for (int w = 0; w < WAVES / 2; ++w) ml[w / (WAVES / 4)][w % (WAVES / 4)] = *(const f32x4 *)(lds_ml + row * 2 * WAVES + 4 * w);
-        float M = -INFINITY;
+            for (int w = 0; w < N / 2; ++w) ml[w / (N / 4)][w % (N / 4)] = *(const f32x4 *)(lds_ml + row * 2 * WAVES + w / (N / 4) * WAVES + 4 * (w % (N / 4)));
+            float M = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, ml[0][w / 4][w % 4]);
-        const float M_safe = M == -INFINITY ? 0.f : M;
-        float L = 0.f;
-        f32x4 val = {0.f, 0.f, 0.f, 0.f};
+            for (int w = 0; w < N; ++w) M = fmaxf(M, ml[0][w / 4][w % 4]);
+            const float M_safe = M == -INFINITY ? 0.f : M;
+            float L = 0.f;
+            f32x4 val = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const float f = exp2f(ml[0][w / 4][w % 4] - M_safe);
-            L += ml[1][w / 4][w % 4] * f;
-            val += *(const f32x4 *)(lds_o + (w * held + row) * PITCH + d) * f;
-        }
-        const int head = head0 + row;
-        if (n_splits == 1) {
-            bf16_t *to = out + (size_t)token * out_stride + (size_t)head * DH + d;
-            f32x4 o;
+            for (int w = 0; w < N; ++w) {
+                const float f = exp2f(ml[0][w / 4][w % 4] - M_safe);
+                L += ml[1][w / 4][w % 4] * f;
+                val += *(const f32x4 *)(lds_o + (w * held + row) * PITCH + d) * f;
+            }
+            const int head = head0 + row;
+            if (n_splits == 1) {
+                bf16_t *to = out + (size_t)token * out_stride + (size_t)head * DH + d;
+                f32x4 o;
 #ifdef LCU_SCORE_BIAS
-            const float share = sinks ? sink_share(M_safe, L, sinks[head]) : 0.f;
+                const float share = sinks ? sink_share(M_safe, L, sinks[head]) : 0.f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = sinks ? val[e] * share : val[e] / L;
+                for (int e = 0; e < 4; ++e) o[e] = sinks ? val[e] * share : val[e] / L;
 #else
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = val[e] / L;
+                for (int e = 0; e < 4; ++e) o[e] = val[e] / L;
 #endif
-            if (four) {
-                *(u32x2 *)to = u32x2{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
-            } else {
+                if (four) {
+                    *(u32x2 *)to = u32x2{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
+                } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) to[e] = from_f32<bf16_t>(o[e]);
+                    for (int e = 0; e < 4; ++e) to[e] = from_f32<bf16_t>(o[e]);
+                }
+            } else {
+                const size_t slot = ((size_t)ri * nh + head) * n_splits + split;
+                *(f32x4 *)(part_o + slot * DH + d) = val;
+                if (d == 0) { part_ml[slot * 2] = M; part_ml[slot * 2 + 1] = L; }
             }
-        } else {
-            const size_t slot = ((size_t)ri * nh + head) * n_splits + split;
-            *(f32x4 *)(part_o + slot * DH + d) = val;
-            if (d == 0) { part_ml[slot * 2] = M; part_ml[slot * 2 + 1] = L; }
         }
-    }
+    };
+    if (live < WAVES) merge(std::integral_constant<int, 4>());
+    else merge(std::integral_constant<int, WAVES>());
 }
 
 // Merges the parts of every (token, head): out = sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).
@@ -512,6 +516,36 @@ attention_merge_kernel(bf16_t *__restrict__ out, int out_stride, const float *__
     *(u32x2 *)(out + (size_t)token * out_stride + (size_t)head * DH + d0) = w;
 }
 
+// The number of compute units of the current device (asked once per device; 0: unknown).
+static int decode_compute_units() {
+    static int units[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+    if (units[dev] == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
+        units[dev] = n > 0 ? n : -1;
+    }
+    return units[dev] > 0 ? units[dev] : 0;
+}
+
+// The waves of a workgroup.  Eight where every workgroup finds a compute unit of its own; beyond that eight leave room for one workgroup at a time on a compute unit, whose first
+// loads and merge nothing then covers.  One MI355X, us, 8 waves and 4: 16 requests of 1,000 keys, 12 heads of 64, 10.3 and 12.1; 64 of 1,000, 24 heads of 32 over 4, 8.4 and 10.8; 24 of 500, 32 heads of
+// 128 over 8, 11.0 and 11.3; but 256 requests of up to 129 keys, 16 heads of 64, 45.6 and 22.7, of 200 50.9 and 29, 32 heads of 128 over 8 37.8 and 24.4; 64 of 150 to 1,500 36.5 and 37.0.
+// Heads of 128 in parts are long, and where they fill more than half of the chip four waves ask for all that memory gives: 8 requests of 4,000 keys, 32 heads over 8, in four
+// parts, 22.3 and 21.2, of 2,000 14.1 and 14.5.  Sixteen rows: their sums of eight waves would be more LDS than a launch gets unasked.
+static int decode_waves(long long workgroups, int rows, int dh, int n_splits, int units) {
+    if (rows >= 16 || workgroups > units) return 4;
+    return dh == 128 && n_splits > 1 && 2 * workgroups > units ? 4 : 8;
+}
+
+// The same for whoever wants to know (units: the device's compute units).
+LCU_API int lcu_attention_decode_waves(int n_req, int nh, int nkvh, int dh, int n_splits, int units) {
+    if (n_req <= 0 || nh <= 0 || nkvh <= 0 || nh % nkvh || n_splits <= 0) return LCU_BAD_ARGUMENT;
+    const int g = nh / nkvh;
+    return decode_waves((long long)n_req * nkvh * ((g + 15) / 16) * n_splits, g < 16 ? g : 16, dh, n_splits, units);
+}
+
 template <int DH>
 static int launch_decode(const void *q, int q_stride, void *out, int out_stride, const void *cache,
                          const int *block_table, int max_pages, const int *q_start, const int *ctx_len,
@@ -519,11 +553,14 @@ static int launch_decode(const void *q, int q_stride, void *out, int out_stride,
                          int n_splits, int few_keys, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
     const int g = nh / nkvh, chunks = (g + 15) / 16;
     const float scale_log2 = SCORE_LOG2(scale);
-    const int held = g < 16 ? g : 16, waves = held < 16 && !few_keys ? 8 : 4;
+    const int held = g < 16 ? g : 16;
+    dim3 grid(n_req * nkvh * chunks, n_splits);
+    const int waves = few_keys ? 4 : decode_waves((long long)grid.x * n_splits, held, DH, n_splits, decode_compute_units());
     const size_t lds_bytes = (size_t)waves * held * (DH + 4 + 2) * sizeof(float);
     static_assert(8 * 15 * (128 + 4 + 2) * sizeof(float) <= 65536, "what a launch gets unasked");
-    dim3 grid(n_req * nkvh * chunks, n_splits), block(waves * WAVE);
-    (waves == 8 ? attention_decode_kernel<DH, 8> : attention_decode_kernel<DH, 4>)<<<grid, block, lds_bytes, stream>>>(
+    dim3 block(waves * WAVE);
+    (page == 16 ? waves == 8 ? attention_decode_kernel<DH, 8, true> : attention_decode_kernel<DH, 4, true>
+                : waves == 8 ? attention_decode_kernel<DH, 8, false> : attention_decode_kernel<DH, 4, false>)<<<grid, block, lds_bytes, stream>>>(
         (const bf16_t *)q, q_stride, (bf16_t *)out, out_stride, (const bf16_t *)cache, block_table, max_pages, q_start,
         ctx_len, req_list, nh, nkvh, page, scale_log2, window, n_splits, part_o, part_ml SCORE_KARGS(scale));
     LCU_LAUNCH_CHECK();
@@ -550,7 +587,7 @@ static int decode_arguments(int q_stride, int out_stride, int max_pages, int nh,
     return LCU_OK;
 }
 
-// few_keys: no request has more than DEC_FEW_KEYS keys (a matter of speed alone).
+// few_keys: four waves a workgroup, however few the workgroups (a matter of speed alone).
 LCU_API int lcu_attention_decode_lengths_bf16(const void *q, int q_stride, void *out, int out_stride, const void *cache,
                                       const int *block_table, int max_pages, const int *q_start, const int *ctx_len,
                                       const int *req_list, int n_req, int nh, int nkvh, int dh, int page, float scale,

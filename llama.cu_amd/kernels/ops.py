@@ -497,7 +497,7 @@ def attention_decode(q, out, cache, block_table, q_start, ctx_len, n_req, n_head
     """Matrix-core attention for requests that feed one token each: all ``n_req`` requests of
     the batch, or the ``n_req`` whose indices ``req_list`` holds.  ``head_slopes``: the bias on the distance inside
     the scores (the kernels of the second library, ``attention_mfma_bias``); ``softcap``: a cap on them (the third,
-    ``attention_mfma_cap``).  ``few_keys``: no request has many (``decode_few_keys``)."""
+    ``attention_mfma_cap``).  ``few_keys``: no request has many, so four waves a workgroup do, however few the workgroups (a matter of speed alone)."""
     if req_list is not None:
         _i32(req_list, "req_list", n_req)
     part_o = part_ml = None
@@ -577,13 +577,13 @@ class AttentionPlan:
     prefill kernel's tasks (``task_req``, ``task_tok0``; ``n_tasks`` on the device says how many).  The launches' sizes
     (``max_tasks``, ``n_single``, ``single_splits``) follow from the step's sizes and the longest context rounded up to
     a power of two; what the lists hold is data."""
-    __slots__ = ("task_req", "task_tok0", "n_tasks_dev", "max_tasks", "per_wg", "singles", "n_single", "single_splits", "single_few_keys")
+    __slots__ = ("task_req", "task_tok0", "n_tasks_dev", "max_tasks", "per_wg", "singles", "n_single", "single_splits")
 
     @property
     def signature(self):
         """What fixes the launches that ``paged_attention`` makes with this plan: two steps with equal signatures are
         served by the same recorded launches."""
-        return (self.max_tasks, self.per_wg, self.n_single, self.single_splits, self.single_few_keys)
+        return (self.max_tasks, self.per_wg, self.n_single, self.single_splits)
 
 
 def plan_attention(step, n_heads: int, n_kv_heads: int, window: int = 0, biased: bool = False, capped: bool = False) -> Optional[AttentionPlan]:
@@ -611,7 +611,6 @@ def plan_attention(step, n_heads: int, n_kv_heads: int, window: int = 0, biased:
     # the most tasks that a step of these sizes can have: a request of q tokens has at most q / tpt + 1
     plan.max_tasks = (step.n - len(singles)) // tpt + (step.n_req - len(singles))
     plan.single_splits = decode_splits(len(singles), n_heads, n_kv_heads, max([step.ctx_lens[r] for r in singles], default=0)) if singles else 1
-    plan.single_few_keys = decode_few_keys(max([step.ctx_lens[r] for r in singles], default=0))
     builder = getattr(step, "builder", None)
     if builder is not None:
         cap_tasks = builder.max_tokens // tpt + builder.max_reqs
@@ -665,11 +664,6 @@ def decode_splits(n_req: int, n_heads: int, n_kv_heads: int, max_ctx_len: int) -
     return 1 + next(i for i, f in enumerate(fill) if f >= max(fill) - t.decode_fill_slack)
 
 
-def decode_few_keys(max_ctx_len: int) -> bool:
-    """Whether a step's requests have so few keys that the decode kernel's workgroups are as fast or faster with half the waves: up to ``TUNING.decode_few_keys``."""
-    return int(max_ctx_len) <= TUNING.decode_few_keys
-
-
 _zeros: Dict = {}
 
 
@@ -720,14 +714,13 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, cache: torch.Tensor, ste
         # batch says which they are (64 requests of 150 to 2,200 keys: the step 11.2 -> 11.0 ms)
         return attention_decode(q, out, cache, bt, step.q_start, step.ctx_len, step.n_req, n_heads, n_kv_heads, head_dim,
                                 page_size, scale, window, splits, req_list=step.decode_order, head_slopes=head_slopes, sinks=sinks,
-                                softcap=softcap, few_keys=decode_few_keys(step.max_ctx_len) if step.attn_few_keys is None else step.attn_few_keys)
+                                softcap=softcap)
     # a mixed batch: the requests that decode one token go to the decode kernel, the portions
     # to the prefill kernel (each would be slow at the other's work)
     plan = plan_attention(step, n_heads, n_kv_heads, window, biased=second, capped=bool(softcap))
     if plan.n_single:
         attention_decode(q, out, cache, bt, step.q_start, step.ctx_len, plan.n_single, n_heads, n_kv_heads, head_dim, page_size,
-                         scale, window, plan.single_splits, req_list=plan.singles, head_slopes=head_slopes, sinks=sinks, softcap=softcap,
-                         few_keys=plan.single_few_keys)
+                         scale, window, plan.single_splits, req_list=plan.singles, head_slopes=head_slopes, sinks=sinks, softcap=softcap)
     if plan.max_tasks:
         attention_prefill(q, out, cache, bt, step.q_start, step.ctx_len, plan.task_req, plan.task_tok0, plan.max_tasks,
                           plan.per_wg, n_heads, n_kv_heads, head_dim, page_size, scale, window, n_tasks_dev=plan.n_tasks_dev,

@@ -114,12 +114,11 @@ class Tuning:
                                         # shape at load and fills up where that is 15 % faster (the outcome can differ from box
                                         # to box near that mark); 0 never fills up; n > 0 fills each half up to a multiple of n
     # ---- the decode attention's cut of a request's keys into parts (attention_mfma.hip)
-    decode_min_part_keys: int = 512     # a part of so many keys; up to 512 keys one part
+    decode_min_part_keys: int = 512     # a part of so many keys; up to 512 keys one part (the longest context rounded up to a power of two).  One MI355X, us, 16 heads over 4, 1 / 2 / 4 / 8
+                                        # parts with their second kernel: 4 requests of 500 keys 6.6, 7.8, 6.8, 6.7, 8 of 300 6.6, 7.7, -, 7.1, of 500 8.7, 8.9, 7.7, 7.3 (the one case in which parts gain)
     decode_max_parts: int = 32
-    decode_few_keys: int = 128          # up to so many keys, which four waves take in one step each, a workgroup has four waves, beyond eight (attention_mfma.hip)
-    decode_few_parts: int = 8           # ... beyond them up to so many parts, however short (of at least 64 keys: 513 are taken for 1,024).  One MI355X, us with its second
-                                        # kernel, 16 heads over 4, 1 / 2 / 4 / 8 parts: 4 requests of 1,000 keys 12.6, 10.9, 8.9, 7.5, 8 of 1,000 13.8, 11.6, 9.3, 8.3, 1 of 2,000
-                                        # 18.6, 11.1, 9.2, 7.7; 500 keys 4 requests 6.6, 7.8, 6.8, 6.7, 8 requests 8.7, 8.9, 7.7, 7.3, of 300 6.6, 7.7, 7.1
+    decode_few_parts: int = 8           # beyond 512 keys up to so many parts, however short (of at least 64 keys: 513 are taken for 1,024).  4 requests of 1,000 keys 12.6, 10.9, 8.9, 7.5,
+                                        # 8 of 1,000 13.8, 11.6, 9.3, 8.3, 1 of 2,000 18.6, 11.1, 9.2, 7.7
     decode_few_workgroups: int = 128    # up to this many workgroups without parts: about one workgroup per compute unit
     decode_long_context: int = 2048     # between half the chip's worth of workgroups and all of it: parts only from here on
                                         # (rounded up to a power of two: from 1,025 keys),

@@ -315,6 +315,30 @@ def test_captured_decode_steps_equal_eager_ones():
         assert torch.equal(a, b), f"decode step {i} differs between eager and captured"
 
 
+@pytest.mark.parametrize("prompt,graphs", [(122, 1), (504, 2)])
+def test_captured_decode_steps_as_their_contexts_grow(prompt, graphs):
+    """Contexts that grow past what the waves of the decode attention take in a step each need no other graph; past 512 keys, where the keys are cut into parts, one more is
+    captured.  Every step gives the logits of the eager one."""
+    from llama_cu_amd.engine.runner import ModelRunner
+    folder = common.make_folder(dict(common.TINY_B, max_position_embeddings=1024), seed=31, dtype=torch.bfloat16, std=common.BF16_STD)
+    reqs = list(common.random_requests(384, [prompt, 40], seed=8).values())
+
+    def decode(use_graphs):
+        runner = ModelRunner.from_folder(folder, dtype="bfloat16", max_tokens=1200, max_seqs=4, use_graphs=use_graphs)
+        runner.step([0, 1], reqs)
+        rng = np.random.default_rng(0)
+        outs = []
+        for _ in range(18):
+            outs.append(runner.step([0, 1], [[int(rng.integers(384))] for _ in range(2)]).float().cpu())
+        return outs, runner
+
+    eager, _ = decode(False)
+    graphed, runner = decode(True)
+    assert len([key for key in runner._graphs if key[0] == 2]) == graphs, runner._graphs.keys()
+    for i, (a, b) in enumerate(zip(eager, graphed)):
+        assert torch.equal(a, b), f"decode step {i} differs between eager and captured"
+
+
 @pytest.mark.parametrize("name", ["B", "D"])
 def test_captured_steps_with_a_prompt_portion_beside_decoding_requests_equal_eager_ones(name):
     """Steps that are not all single tokens are captured too, by their sizes: three requests decode while a fourth

@@ -1,4 +1,4 @@
-"""What the products' rules and entries take and refuse, which needs no GPU."""
+"""What kernels' rules and entries take and refuse, which needs no GPU."""
 from __future__ import annotations
 
 import ctypes
@@ -42,3 +42,23 @@ def test_rows_that_span_more_than_a_load_reaches():
     apart = (1 << 31) // 99 + 8 & ~7
     for packed, epilogue in ((1, 1), (0, 1), (1, 2), (1, 0)):
         assert lib.lcu_gemm_mid_bf16(p, apart, p, 128, p, 64, 100, 64, 128, epilogue, 1, packed, f(1), f(0), None) == -1
+
+
+@pytest.mark.parametrize("name", ["attention_mfma", "attention_mfma_bias", "attention_mfma_cap"])
+def test_waves_of_the_decode_attention(name):
+    """Eight waves a workgroup where every workgroup has a compute unit of its own, four beyond (256 requests of some 129 keys took twice as long with eight), for sixteen
+    rows, and for parts of heads of 128 that fill more than half of the chip."""
+    waves = build.load(name).lcu_attention_decode_waves
+    for dh in (32, 64, 96, 128):
+        assert [waves(n, 16, 16, dh, 1, 256) for n in (1, 16, 17, 256)] == [8, 8, 4, 4]
+        assert [waves(n, 32, 8, dh, 1, 256) for n in (32, 33)] == [8, 4] and waves(33, 32, 8, dh, 1, 304) == 8
+        assert [waves(1, g, 1, dh, 1, 256) for g in (15, 16, 17, 32)] == [8, 4, 4, 4]
+        assert [waves(n, 32, 8, dh, 4, 256) for n in (4, 5, 8, 9)] == [8, 4 if dh == 128 else 8, 4 if dh == 128 else 8, 4]
+        assert waves(1, 32, 8, dh, 1, 0) == 4                  # (a device that does not say how many units it has)
+
+
+def test_parts_of_few_requests():
+    """One part up to 512 keys, eight beyond as far as the chip has compute units for them, longer ones from 4,097 keys on."""
+    splits = ops.decode_splits
+    assert [splits(1, 16, 4, c) for c in (1, 512, 513, 1024, 1025, 4096, 4097)] == [1, 1, 8, 8, 8, 8, 16]
+    assert [splits(n, 16, 4, 513) for n in (8, 9, 16, 32, 33)] == [8, 7, 4, 2, 1] and splits(32, 16, 4, 512) == 1
