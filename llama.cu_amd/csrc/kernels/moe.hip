@@ -558,12 +558,22 @@ moe_gemm_few_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__
 // workgroups of experts without a pair, and has eight waves, a quarter of K and one of the two tiles each, with eight steps on their way: few workgroups then
 // ask for as much at a time as many would.  An expert's pairs go sixteen at a time; a token may name an expert more than once, so they may be more than the tokens, and what is beyond the
 // first sixteen goes through a loop of its own (one loop for all takes more registers: 14.8 us in the place of 10.8 for a token of two).  The sums are added up as in the kernel for few rows: the same bits.  What bounds it is the way of the numbers of the experts
-// and of their matrices' first lines through memory, one after the other.  One MI355X, both products, us, with the kernel for few rows everywhere and now: a token of two experts of
-// 2 x 1024 x 2048 with a shared one of 704 13.6 and 11.9, two tokens 19.5 and 17.5; a token of two of 2 x 1408 x 2048 14.4 and 11.9, of four of 2 x 512 x 2048 13.1 and 10.9, of one of
-// 2 x 3584 x 1024 16.5 and 13.1.  From some 400 workgroups on four waves with two tiles each read the rows half as often: four tokens of two of 2 x 1408 x 2048 23.7 and 25.4, eight of
-// four of 2 x 512 x 2048 29.3 and 46.6.
+// and of their matrices' first lines through memory, one after the other, and what a workgroup does to find its pairs: a turn an expert, and one permutation of the lanes (a
+// turn a pair and fifteen for the rows took 8 us of 64 pairs, 4 experts of 2 x 1024 x 1024: 20.5, now 12.7).  One MI355X, both products, us, with the kernel for few rows everywhere and now: a token of two experts of
+// 2 x 1024 x 2048 with a shared one of 704 13.6 and 11.9, two tokens 19.5 and 17.5; a token of two of 2 x 1408 x 2048 14.4 and 11.9, of four of 2 x 512 x 2048 11.9 and 10.5, of one of
+// 2 x 3584 x 1024 16.4 and 13.1; four tokens of two of 64 of 2 x 512 x 1024 13.8 and 10.2.
 constexpr int MOE_SLOTS = 64, MOE_SLOT_ROWS = 16;      // pairs, a lane each; tokens
-constexpr int MOE_SLOT_WORKGROUPS = 384;               // of the experts that pairs name, at most
+// Whether the kernel takes a product of `rows` features.  From some 400 workgroups on four waves with two tiles each read the rows half as often: four tokens of two of 2 x 1408 x 2048 23.7 and 25.4, eight of
+// four of 2 x 512 x 2048 29.3 and 46.6.  From 256 on it is so where half of the experts or more are named, so that the other kernel holds few workgroups for nothing: 12 tokens of two of 32 of 2 x 256 x 512 9.0
+// and 9.8, 3 of four of 16 of 2 x 512 x 2048 15.8 and 16.4; but 3 of four of 64 of 2 x 512 x 1024 15.0 and 11.9.  With more than a dozen pairs an expert the turns of the two kernels are equally full: 16 tokens of
+// four, all of 4 experts of 2 x 1024 x 1024, 32 bits 19.0 and 20.0, 12 tokens 18.4 and 18.3.
+static bool moe_slots_take(int n, int top, int experts, int rows) {
+    const int total = n * top, slots = total < experts ? total : experts;
+    return total <= MOE_SLOTS && n <= MOE_SLOT_ROWS && total <= 12 * slots && (rows + 31) / 32 * slots <= (experts >= 2 * slots ? 384 : 256);
+}
+// The same for whoever wants to know.
+LCU_API int lcu_moe_slots_take(int n, int top, int experts, int rows) { return n > 0 && top > 0 && experts > 0 && rows > 0 && moe_slots_take(n, top, experts, rows); }
+
 template <class T, int MODE, bool PACKED>
 __global__ void __launch_bounds__(512)
 moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict__ w, size_t w_expert_stride, int N, int K,
@@ -578,8 +588,7 @@ moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict
     const int part = wave & 3, side = wave >> 2;
     const bool shared = (int)blockIdx.y == slots;
     const T *we = sw;
-    int count = total;
-    unsigned long long pairs = 0;                    // the expert's, a bit each
+    int count = total, sorted = lane;                // lane r: the expert's r-th pair
     if (shared) {                                    // every token's rows [n, s_k] and a matrix of its own size
         count /= top;                                // (at most MOE_SLOT_ROWS)
         top = 1;
@@ -592,29 +601,29 @@ moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict
         out_stride = GATED ? s_n / 2 : out_stride;
         alpha = 1.f;
         limit = 0.f;
-        pairs = (1ull << count) - 1;
     } else {
         const int mine = lane < total ? ids[lane] : -1;
-        bool first = mine >= 0 && mine < experts;    // (identity experts have no matrices)
-        for (int j = 0; j < total - 1; ++j) first = first && !(j < lane && __builtin_amdgcn_readlane(mine, j) == mine);
-        unsigned long long which = __ballot(first);
-        if ((int)blockIdx.y >= __popcll(which)) return;
-        for (int y = 0; y < (int)blockIdx.y; ++y) which &= which - 1;
-        const int e = __builtin_amdgcn_readlane(mine, __builtin_ctzll(which));
-        pairs = __ballot(mine == e);
+        unsigned long long left = __ballot(mine >= 0 && mine < experts), pairs = 0;      // (identity experts have no matrices)
+        int e = 0;
+        for (int y = 0; y <= (int)blockIdx.y; ++y) { // an expert a turn, in the order of their first pairs
+            left &= ~pairs;
+            if (!left) return;
+            e = __builtin_amdgcn_readlane(mine, __builtin_ctzll(left));
+            pairs = __ballot(mine == e);
+        }
         count = __popcll(pairs);
+        const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(pairs >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)pairs, 0));
+        sorted = __builtin_amdgcn_ds_permute(4 * (mine == e ? before : count + lane - before), lane);
         we = w + (size_t)e * w_expert_stride;
     }
     if ((int)blockIdx.x * 32 >= N) return;
     const int tile0 = 2 * blockIdx.x, steps = (K + M::KSTEP - 1) / M::KSTEP, per = quarter_steps(steps);
     const int s0 = min(steps, part * per), s1 = min(steps, s0 + per);
-    // sixteen of the pairs, of which `left` are left
-    auto pass = [&](auto ahead, int left) {
+    // sixteen of the pairs, from the r0-th on
+    auto pass = [&](auto ahead, int r0) {
         constexpr int AHEAD = decltype(ahead)::value;
         const Unit<T, PACKED> wu(we, tile0 + side, N, K, steps, lane);
-        unsigned long long own = pairs;
-        for (int r = 0; r < min(l16, left - 1); ++r) own &= own - 1;
-        const int flat = __builtin_ctzll(own);       // of row l16
+        const int flat = __builtin_amdgcn_ds_bpermute(4 * min(r0 + l16, count - 1), sorted);      // of row l16
         const T *xr = x + (size_t)(UP ? flat / top : flat) * x_stride + g * M::PER_LANE;
         const float sc = MODE == MOE_UP ? wts[flat] : 1.f;
         const int x_left = K - g * M::PER_LANE;
@@ -635,11 +644,11 @@ moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict
                 if (s + u + AHEAD < s1) fetch(u, s + u + AHEAD);
             }
         }
-        if (left < count) __syncthreads();           // the sums of the rows before have been read
+        if (r0 > 0) __syncthreads();                 // the sums of the rows before have been read
         red[part][side][lane] = acc;
         __syncthreads();
         // the first wave stores (with two products' sums the first two, one each): four neighbouring features of a row a lane
-        if (wave >= (GATED ? 1 : 2) || l16 >= left) return;
+        if (wave >= (GATED ? 1 : 2) || r0 + l16 >= count) return;
         const f32x4 v = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
         const int dst = !UP && add ? flat / top : flat;
         if constexpr (GATED) {
@@ -662,11 +671,8 @@ moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict
             }
         }
     };
-    pass(Int<8>(), count);
-    for (int left = count - 16; left > 0; left -= 16) {
-        for (int r = 0; r < 16; ++r) pairs &= pairs - 1;
-        pass(Int<2>(), left);
-    }
+    pass(Int<8>(), 0);
+    for (int r0 = 16; r0 < count; r0 += 16) pass(Int<2>(), r0);
 }
 
 // Many rows an expert (prompts): tiles of up to 32, 64, 96 or 128 rows; a block of four waves takes a tile and 128 features, a wave 32 of them with all
@@ -1024,9 +1030,8 @@ LCU_API int lcu_moe_experts(const void *h, int type, const int *ids, const float
         const size_t act_end = (size_t)total * ff;
         const dim3 block(256), gu((wider + 31) / 32, with), gd((d + 31) / 32, with);
         const int slots = total < experts ? total : experts;
-        const bool least = !tile_rows && total <= MOE_SLOTS && n <= MOE_SLOT_ROWS;
         const dim3 su(gu.x, slots + (shared_up ? 1 : 0)), sd(gd.x, su.y);
-        const bool up_slots = least && (up_rows + 31) / 32 * slots <= MOE_SLOT_WORKGROUPS, down_slots = least && (d + 31) / 32 * slots <= MOE_SLOT_WORKGROUPS;
+        const bool up_slots = !tile_rows && moe_slots_take(n, top, experts, up_rows), down_slots = !tile_rows && moe_slots_take(n, top, experts, d);
 #define UP_SLOTS(T, PACKED, MODE) moe_gemm_slots_kernel<T, MODE, PACKED><<<su, dim3(512), 0, stream>>>((const T *)h, d, (const T *)w_up, up_stride, up_rows, d, \
                                                 ids, total, wts, (T *)act, nullptr, ff, top, 0, alpha, limit, experts, slots, \
                                                 (const T *)h, (const T *)shared_up, s_rows, d, (T *)act + act_end, nullptr)

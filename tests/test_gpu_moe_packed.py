@@ -320,10 +320,10 @@ def beside_tiles(h, ids, wts, up, down, monkeypatch, **kw):
     return outs
 
 
-# 9 tokens of two, all on one expert (18 pairs); 16 of four on two experts (32 each), on one (64) and with a last turn of a single pair (17)
+# 9 tokens of two, all on one expert (18 pairs); 16 of four on two experts (32 each), on one (64; of 4 experts they go to the other kernel) and with a last turn of a single pair (17)
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("gated", [True, False])
-@pytest.mark.parametrize("n,top,experts,named", [(9, 2, 2, [[0, 0]] * 9), (16, 4, 8, [[3, 5, 5, 3]] * 16), (16, 4, 4, [[1] * 4] * 16),
+@pytest.mark.parametrize("n,top,experts,named", [(9, 2, 2, [[0, 0]] * 9), (16, 4, 8, [[3, 5, 5, 3]] * 16), (16, 4, 4, [[1] * 4] * 16), (16, 4, 6, [[1] * 4] * 16),
                                                  (16, 2, 40, [[7, 7]] + [[7, 8]] * 15)])
 @pytest.mark.parametrize("d,ff", [(72, 32), (520, 144)])
 def test_an_expert_that_a_token_names_more_than_once(dtype, gated, n, top, experts, named, d, ff, monkeypatch):

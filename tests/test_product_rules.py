@@ -62,3 +62,12 @@ def test_parts_of_few_requests():
     splits = ops.decode_splits
     assert [splits(1, 16, 4, c) for c in (1, 512, 513, 1024, 1025, 4096, 4097)] == [1, 1, 8, 8, 8, 8, 16]
     assert [splits(n, 16, 4, 513) for n in (8, 9, 16, 32, 33)] == [8, 7, 4, 2, 1] and splits(32, 16, 4, 512) == 1
+
+
+def test_experts_of_few_pairs():
+    """Which products of a step's first pairs go to the kernel that holds the named experts' workgroups alone: at its edges (16 tokens, 64 pairs, 256 workgroups, or 384 where most experts
+    have no pair, a dozen pairs an expert)."""
+    takes = build.load("moe").lcu_moe_slots_take
+    assert takes(1, 2, 16, 2048) and takes(16, 2, 40, 64) and not takes(17, 1, 40, 64) and takes(16, 4, 64, 64) and not takes(16, 5, 80, 64)
+    assert takes(12, 1, 24, 1024) and not takes(12, 1, 24, 1025) and takes(12, 1, 23, 672) and not takes(12, 1, 23, 1024)
+    assert takes(12, 4, 4, 1024) and not takes(13, 4, 4, 1024) and not takes(16, 4, 4, 1024) and takes(12, 1, 1, 1024) and not takes(13, 1, 1, 1024)
