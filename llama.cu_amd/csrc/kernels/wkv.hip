@@ -378,8 +378,9 @@ wkv_out_kernel(const float *__restrict__ o, int DV, const TG *__restrict__ rows,
 // A workgroup per (request, head).  Wave w walks the key channels w, w + 4, ..: a lane holds the columns lane, lane + 64, .. of a
 // row, so a row of the state is read and written in whole lines.  The first rows are on their way while the decay is made, and so is all that hangs on nothing: the
 // trips to memory one after the other are what bounds it (32 requests, 32 heads of 64, a launch inside a model 13.2 us with the decay's matrix, its base, the gate and the weight
-// each asked for where it is used, 12.4 with all of them in front; 33 MB of states would take 6).
-template <int D, class TG, class T>
+// each asked for where it is used, 12.4 with all of them in front; 33 MB of states would take 6).  FRONT: all of them in front, which takes 15 registers: with heads of up to 64 a compute unit
+// then holds five workgroups and not six (wkv_front).
+template <int D, bool FRONT, class TG, class T>
 __global__ void __launch_bounds__(WK_THREADS)
 wkv_single_kernel(const TG *__restrict__ rows, int row_stride, int r_off, int k_off, int v_off, int g_off, const float *__restrict__ low,
                   int ld_low, const float *__restrict__ w2t, const float *__restrict__ w0, const float *__restrict__ u,
@@ -406,14 +407,23 @@ wkv_single_kernel(const TG *__restrict__ rows, int row_stride, int r_off, int k_
     };
     load(0);
     // what the decay's second product and the end want: on their way as well, the first rows of the matrix that a thread takes
-    constexpr int EARLY = 16;
+    constexpr int EARLY = FRONT ? 16 : 0;
     const int c = tid % D, p = tid / D, per = (rank + PARTS - 1) / PARTS, j0 = p * per, j1 = min(rank, j0 + per);
     const float *w2 = w2t + h * d + min(c, d - 1);
-    float early[EARLY];
+    float early[EARLY + 1];
 #pragma unroll
     for (int e = 0; e < EARLY; ++e) early[e] = w2[(size_t)min(j0 + e, rank - 1) * nh * d];
-    const float base = w0[h * d + min(tid, d - 1)], scale = weight[h * dv + min(tid, dv - 1)];
-    const float value = to_f32(row[v_off + h * dv + min(tid, dv - 1)]), gate = to_f32(row[g_off + h * dv + min(tid, dv - 1)]);
+    float base = 0.f, scale = 0.f, value = 0.f, gate = 0.f;
+    auto ask_base = [&] { base = w0[h * d + min(tid, d - 1)]; };
+    auto ask_end = [&] {
+        scale = weight[h * dv + min(tid, dv - 1)];
+        value = to_f32(row[v_off + h * dv + min(tid, dv - 1)]);
+        gate = to_f32(row[g_off + h * dv + min(tid, dv - 1)]);
+    };
+    if (FRONT) {
+        ask_base();
+        ask_end();
+    }
     float v[NV];
 #pragma unroll
     for (int e = 0; e < NV; ++e) v[e] = lane + 64 * e < dv ? to_f32(row[v_off + h * dv + lane + 64 * e]) : 0.f;
@@ -440,6 +450,7 @@ wkv_single_kernel(const TG *__restrict__ rows, int row_stride, int r_off, int k_
     }
     __syncthreads();
     if (tid < D) {
+        if (!FRONT) ask_base();
         float z = tid < d ? base : 0.f;
 #pragma unroll
         for (int p = 0; p < PARTS; ++p) z += zs[p][tid];
@@ -467,6 +478,7 @@ wkv_single_kernel(const TG *__restrict__ rows, int row_stride, int r_off, int k_
     for (int e = 0; e < NV; ++e) red[wave][lane + 64 * e] = acc[e];
     __syncthreads();
     float o = 0.f;
+    if (!FRONT) ask_end();
     if (tid < dv) {
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) o += red[w][tid];
@@ -553,7 +565,31 @@ LCU_API int lcu_wkv(const void *rows, int rows_type, int row_stride, int r_off, 
     return LCU_OK;
 }
 
-// The same for a step in which every request feeds one token (n == n_req), in one kernel without scratch.
+// Whether a step of single tokens asks for all in front: not where that takes another round of workgroups, of which a compute unit holds five then and six otherwise (heads of up to 64; of
+// larger ones as many either way).  One MI355X, us, in front and not: 128 requests of 12 heads (1,536 workgroups) 15.3 and 11.9, 64 of 24 18.9 and 16.6, but 64 of 32 22.5 and 23.1, 32 of 32 with a
+// rank of 256 17.0 and 17.8, 1 of 32 8.8 and 9.1.
+static bool wkv_front(int n_req, int heads, int D, int units) {
+    if (D > 64 || units <= 0) return true;
+    const long long all = (long long)n_req * heads;
+    return (all + 5ll * units - 1) / (5ll * units) <= (all + 6ll * units - 1) / (6ll * units);
+}
+// The same for whoever wants to know.
+LCU_API int lcu_wkv_front(int n_req, int heads, int d, int units) { return wkv_front(n_req, heads, wk_pad_keys(d), units); }
+
+// The number of compute units of the current device (asked once per device; 0: unknown).
+static int wkv_compute_units() {
+    static int units[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+    if (units[dev] == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
+        units[dev] = n > 0 ? n : -1;
+    }
+    return units[dev] > 0 ? units[dev] : 0;
+}
+
+// lcu_wkv for a step in which every request feeds one token (n == n_req), in one kernel without scratch.
 LCU_API int lcu_wkv_single(const void *rows, int rows_type, int row_stride, int r_off, int k_off, int v_off, int g_off, const float *low,
                            int ld_low, const float *w2t, const float *w0, const float *u, const float *weight, float *state,
                            long long slot_stride, void *out, int out_type, const int *q_start, const int *ctx_len, const int *state_slot,
@@ -561,12 +597,14 @@ LCU_API int lcu_wkv_single(const void *rows, int rows_type, int row_stride, int 
     if (n_req <= 0) return LCU_OK;
     if (!wkv_sizes_ok(heads, d, dv, rank, slot_stride)) return LCU_BAD_ARGUMENT;
     const int D = wk_pad_keys(d);
-#define GO(D_, TG, T) wkv_single_kernel<D_, TG, T><<<dim3(n_req, heads), dim3(WK_THREADS), 0, stream>>>((const TG *)rows, row_stride, r_off, k_off, v_off, g_off, low, ld_low, w2t, w0, u, weight, state, (size_t)slot_stride, (T *)out, ctx_len, q_start, state_slot, heads, d, dv, rank, eps)
+    const bool front = wkv_front(n_req, heads, D, wkv_compute_units());
+#define GO(D_, FRONT, TG, T) wkv_single_kernel<D_, FRONT, TG, T><<<dim3(n_req, heads), dim3(WK_THREADS), 0, stream>>>((const TG *)rows, row_stride, r_off, k_off, v_off, g_off, low, ld_low, w2t, w0, u, weight, state, (size_t)slot_stride, (T *)out, ctx_len, q_start, state_slot, heads, d, dv, rank, eps)
 #define SIZES(TG, T)                  \
     do {                              \
-        if (D == 64) GO(64, TG, T);   \
-        else if (D == 128) GO(128, TG, T); \
-        else GO(256, TG, T);          \
+        if (D == 64 && !front) GO(64, false, TG, T); \
+        else if (D == 64) GO(64, true, TG, T); \
+        else if (D == 128) GO(128, true, TG, T); \
+        else GO(256, true, TG, T);    \
     } while (0)
     if (rows_type == LCU_F32 && out_type == LCU_F32) SIZES(float, float);
     else if (rows_type == LCU_F32 && out_type == LCU_BF16) SIZES(float, bf16_t);

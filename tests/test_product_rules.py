@@ -71,3 +71,10 @@ def test_experts_of_few_pairs():
     assert takes(1, 2, 16, 2048) and takes(16, 2, 40, 64) and not takes(17, 1, 40, 64) and takes(16, 4, 64, 64) and not takes(16, 5, 80, 64)
     assert takes(12, 1, 24, 1024) and not takes(12, 1, 24, 1025) and takes(12, 1, 23, 672) and not takes(12, 1, 23, 1024)
     assert takes(12, 4, 4, 1024) and not takes(13, 4, 4, 1024) and not takes(16, 4, 4, 1024) and takes(12, 1, 1, 1024) and not takes(13, 1, 1, 1024)
+
+
+def test_what_the_recurrence_with_a_bonus_asks_for_in_front():
+    """All of it, unless that takes another round of workgroups: heads of up to 64, of which a compute unit holds five then and six otherwise."""
+    front = lambda *a: bool(build.load("wkv").lcu_wkv_front(*a))
+    assert [front(n, 1, 64, 256) for n in (1, 1280, 1281, 1536, 1537, 2560, 2561, 3072, 3073)] == [True, True, False, False, True, True, False, False, True]
+    assert not front(128, 12, 48, 256) and front(128, 12, 65, 256) and front(128, 12, 48, 0)
