@@ -448,11 +448,14 @@ rglru_gates_mfma_kernel(const TI *__restrict__ rows, int row_stride, int x_off, 
 // now 8.0), 1.7 us of matrix instructions.  One MI355X, 4 taps, us alone beside the sliced kernel and the scan, with four trips: width 2048
 // in 16 blocks 8.0 / 10.9 with 8 requests, 8.8 / 14.0 with 64; width 1024 in 16 blocks 5.8 / 8.5 with 8.  (Blocks of 192 channels, whose twelve sixteens do not fit the
 // registers: 24 / 10.4.)
-constexpr int RG_ONE_TOK = 4, RG_ONE_THREADS = 512, RG_ONE_BS = 128;
+constexpr int RG_ONE_TOK = 4, RG_ONE_BS = 128;
 
-// MOST: sixteens of input channels at most
+// MOST: sixteens of channels at most.  Up to 64 channels a workgroup has a wave for each sixteen, and so a thread for each element of its four tokens (with eight waves always, those without a
+// matrix, which ask for a neighbour's, made blocks of 32 channels slower than four trips: width 2048 in 64 blocks, 64 requests, 10.2 us and 9.2; now 5.9), beyond it eight (96 channels, 256 requests:
+// 17.3 us, with six waves, of which two SIMDs hold two, 20.1).
+constexpr int rg_one_threads(int bs) { return bs <= 64 ? RG_ONE_TOK * bs : RG_ONE_TOK * RG_ONE_BS; }
 template <class T, int MOST>
-__global__ void __launch_bounds__(RG_ONE_THREADS)
+__global__ void __launch_bounds__(rg_one_threads(16 * MOST))
 rglru_single_kernel(const float *__restrict__ rows, int row_stride, int y_off, int x_off, const float *__restrict__ bias,
                     const float *__restrict__ conv_w, const float *__restrict__ conv_b, float *__restrict__ state,
                     const float *__restrict__ gates, const float *__restrict__ ba, const float *__restrict__ bi, const float *__restrict__ lam, float c_exp,
@@ -464,7 +467,7 @@ rglru_single_kernel(const float *__restrict__ rows, int row_stride, int y_off, i
     // ---- what a thread asks for: under no condition (threads without work ask for a neighbour's), as loads come back in order: the numbers of the states first, what hangs on
     // nothing, the matrices, and behind them what lies in the states
     auto load = [](const float *q) { return *(const rg_f32x4 *)q; };
-    static_assert(RG_ONE_TOK * RG_ONE_BS <= RG_ONE_THREADS && RG_ONE_BS / 16 <= RG_ONE_THREADS / WAVE, "an element a thread, sixteen output channels a wave");
+    static_assert(RG_ONE_TOK * 16 == WAVE, "an element a thread, sixteen output channels a wave");
     const int x = min((int)threadIdx.x, nt * (bs / 4) - 1), tt = x / (bs / 4), i = x % (bs / 4) * 4, c = b * bs + i, t = tok0 + tt;      // u: four neighbouring channels of a token
     const int e_tt = min((int)threadIdx.x / bs, nt - 1), e_o = threadIdx.x % bs, e_t = tok0 + e_tt, e_c = b * bs + e_o;                // the recurrence: an element
     const bool e_in = (int)threadIdx.x / bs < nt;
@@ -681,9 +684,9 @@ LCU_API int lcu_rglru(const void *rows, int in_type, int row_stride, int y_off, 
     if (matrix && single && n == n_req && taps <= RG_MFMA_TAPS && bs <= RG_ONE_BS && in_type == LCU_F32 && bs % (4 * slices) == 0 && x_off % 4 == 0 && row_stride % 4 == 0 &&
         ((uintptr_t)rows | (uintptr_t)conv_w | (uintptr_t)conv_b | (uintptr_t)state) % 16 == 0) {
 #define ONE(T, MOST)                                                                                                                                                      \
-    rglru_single_kernel<T, MOST><<<dim3((n + RG_ONE_TOK - 1) / RG_ONE_TOK, blocks), dim3(RG_ONE_THREADS), 0, stream>>>((const float *)rows, row_stride, y_off, x_off, bias, conv_w, \
+    rglru_single_kernel<T, MOST><<<dim3((n + RG_ONE_TOK - 1) / RG_ONE_TOK, blocks), dim3(rg_one_threads(bs)), 0, stream>>>((const float *)rows, row_stride, y_off, x_off, bias, conv_w, \
                                                                               conv_b, state, gates, ba, bi, lam, c_exp, (T *)out, ctx_len, state_slot, n, width, bs, taps, slices)
-#define STEP(T) do { if (bs <= 64) ONE(T, 4); else ONE(T, RG_ONE_BS / 16); } while (0)
+#define STEP(T) do { if (bs <= 32) ONE(T, 2); else if (bs <= 64) ONE(T, 4); else if (bs <= 96) ONE(T, 6); else ONE(T, RG_ONE_BS / 16); } while (0)
         if (out_type == LCU_BF16) STEP(bf16_t);
         else STEP(float);
 #undef STEP

@@ -141,3 +141,14 @@ def test_bits_of_many_tokens(width, blocks, taps, types):
     rows, old = rnd(sum(lens), 2 * width + 8, seed=64).to(ti).cuda(), rnd(5, taps, width, seed=65).cuda()
     (a, sa), (b, sb) = both_ways(unit, unit.args(), rows, old, lens, [700, 2, 40, 66, 560], [0, 3, 1, 4, 2], to)
     assert torch.equal(a, b) and torch.equal(sa, sb)
+
+
+@pytest.mark.parametrize("width,blocks", [(32, 2), (96, 2), (160, 2), (224, 2), (64, 2), (128, 2), (192, 2), (256, 2)])
+@pytest.mark.parametrize("n", [1, 32, 33, 130])
+@pytest.mark.parametrize("taps", [1, 4])
+def test_single_tokens_by_the_size_of_a_block(width, blocks, n, taps):
+    """Blocks of every number of sixteens up to eight, for which a workgroup has one, two, three, four or eight waves: the bits of the kernels without packed gates."""
+    unit = Unit(width, blocks, taps, offsets=(0, 0))
+    args, rows, state = unit.args(), rnd(n, 2 * width + 8, seed=20).cuda(), rnd(n + 1, taps, width, seed=22).cuda()
+    (got, after), (want, kept) = both_ways(unit, args, rows, state, [1] * n, [1 + (3 * i) % 7 for i in range(n)], list(range(n)), torch.float32)
+    assert torch.isfinite(got).all() and torch.equal(got, want) and torch.equal(after, kept)
