@@ -1010,22 +1010,30 @@ TILES = ((128, 128), (128, 256), (256, 256))      # features x tokens of the sha
 
 def tiles_choice(m: int, n: int, k: int, swiglu: bool = False) -> int:
     """The shape of ``gemm_tiles`` for a product of many bfloat16 rows where it is faster than the library's (and, with SwiGLU, than that and the activation kernel),
-    else -1.  It is where its workgroups fill more than half of a round and, mostly, no more than one (measured from 200 to 4,000 rows, 1024 x 1024 to 28672 x 4096;
-    the numbers are ``TUNING``'s)."""
+    else -1.  It is where its workgroups, and with them the rows and features that are there, fill more than half of a round and, mostly, no more than one, unless the library has tiles that
+    fit better: few features, long sums (measured over 3,300 sizes of 257 to 4,096 rows, 512 to 28,672 features and a K of 256 to 14,336; the numbers are ``TUNING``'s)."""
     t = TUNING
     if m <= t.tiles_rows or k <= 0 or k % 64 or n % 64 or (swiglu and k > t.tiles_swiglu_k):
         return -1
     cu, columns = t.compute_units, (n + 127) // 128
+    full = 128 * 128 * cu                     # elements of a round of square tiles
     square = (m + 127) // 128 * columns
     if square <= cu:
+        if k > t.tiles_any_k and (5 * m * n <= 2 * full if swiglu else 2 * m * n <= full):
+            return -1
+        if not swiglu and (10 * m > 9 * n and k > t.tiles_long_k or 2 * m > 3 * n and k > t.tiles_tall_k or 5 * m > 6 * n and 10 * square > 9 * cu
+                           or k > t.tiles_long_k and (8 * square < 5 * cu or 8 * square == 5 * cu and 3 * m > n)):
+            return -1
         finer = (m + t.tiles_library_tile - 1) // t.tiles_library_tile * columns      # the library's workgroups where it takes tiles of fewer rows
         if not swiglu and k >= t.tiles_library_k and 8 * finer >= 7 * cu and finer <= cu:
             return -1
         return 0 if 2 * square > cu else -1
     wide = (m + 255) // 256 * columns
     if swiglu:
-        return 1 if wide <= cu else 2 if (m + 255) // 256 * ((n + 255) // 256) <= cu else -1
-    return 1 if 8 * wide <= 5 * cu and k <= t.tiles_short_k else -1
+        if wide <= cu:
+            return 1
+        return 2 if (m + 255) // 256 * ((n + 255) // 256) <= cu and (k < t.tiles_any_k or 2 * m * n > 5 * full) else -1
+    return 1 if 8 * wide <= 5 * cu and k <= t.tiles_short_k and (k < t.tiles_short_k or 5 * wide >= 3 * cu) else -1
 
 
 def tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:

@@ -106,9 +106,16 @@ class Tuning:
                                         # 5120 x 4096 at 512 and 576 36.5 / 32.9 and 38.1 / 33.5), below and beyond not (4096 x 4096 at 576 / 800 36.6 / 39.8 and 33.5 / 31.7, 5120 x 4096 at 450 / 640 35.1 / 39.6 and
                                         # 33.1 / 38.1), and with a shorter K neither (3072 x 2048 at 765 19.4 and 15.9, 2048 x 2816 at 1,280 22.6 and 20.6, at 1,400 21.1 and 21.7)
     tiles_short_k: int = 2048           # a round of 128 x 256 up to five eighths full only with a K up to this (4096 x 2048, 1,100 rows: 27.0 and 24.3; 2560 x 2048, 2,014: 27.8 and
-                                        # 25.0; 4096 x 4096, 1,100: 42.6 and 42.8)
+                                        # 25.0; 4096 x 4096, 1,100: 42.6 and 42.8), and with this K not one less than three fifths full (3072 x 2048 at 1,400 23.6 and 24.7, 5632 x 2048 at 661 23.3 and 25.9)
                                         # (a fuller round, with any K, is no gain in a whole prompt, where the card's power limit lets every kernel pay for another's work: 4096 x
                                         # 14336, 2,048 rows, 210 and 196 alone, 225 and 204 inside an 8-layer prompt of the 8B shape, which takes 6.79 and 6.85 ms)
+    tiles_any_k: int = 1024             # with a longer K a round that the rows and features that are there fill to less than half (SwiGLU: two fifths) is the library's: 6144 x 2048 at 300 rows 15.5 and 16.2 (32-bit
+                                        # sums 16.0 and 19.4), 3584 x 3584 at 513 / 576 / 640 23.1 / 23.0 / 26.0 and 25.1 / 25.0 / 24.0; 2816 x 1024 at 700 11.6 and 11.0.  SwiGLU in tiles of 256 x 256 from this K on has
+                                        # to fill more than two and a half rounds of square tiles: 11264 x 2048 at 576 / 800 / 1,000 36.3 / 43.0 / 58 and 44.9 / 46.3 / 49, 5632 x 2048 at 1,400 / 2,014 39.6 / 59.7 and 48.8 / 50
+    tiles_tall_k: int = 2048            # a longer K with half as many rows again as features is the library's (768 x 3072 at 3,471 22.9 and 25.6, 1024 x 2816 at 2,841 22.9 and 24.2; 960 x 1536 at 3,552 1.08 times as fast
+                                        # in tiles), with any K once a round is nine tenths full and a fifth more rows than features (1536 x 1536 at 2,300 / 2,547 rows 1.09 and 0.82 times as fast, 1792 x 3072 at 2,249 0.86)
+    tiles_long_k: int = 4096            # a longer one with nine tenths as many rows as features (2048 x 8192 at 2,048 66.8 and 70.5, 1024 x 8192 at 4,000 68.1 and 78.5), or a round less than five eighths full, or so full with a third as many rows as features (2048 x 14336
+                                        # at 1,117 107 and 121, 2944 x 5632 at 688 34.2 and 37.4, 2560 x 11008 at 1,004 86 and 93; 4096 x 14336 at 513 1.14 times as fast in tiles)
     # ---- the library's product of many rows (parts/linear.library_friendly_rows)
     library_rows: int = -1              # rows of zeros behind each half of a plain gate/up matrix: -1 times the library once per
                                         # shape at load and fills up where that is 15 % faster (the outcome can differ from box

@@ -78,3 +78,16 @@ def test_what_the_recurrence_with_a_bonus_asks_for_in_front():
     front = lambda *a: bool(build.load("wkv").lcu_wkv_front(*a))
     assert [front(n, 1, 64, 256) for n in (1, 1280, 1281, 1536, 1537, 2560, 2561, 3072, 3073)] == [True, True, False, False, True, True, False, False, True]
     assert not front(128, 12, 48, 256) and front(128, 12, 65, 256) and front(128, 12, 48, 0)
+
+
+@pytest.mark.parametrize("m,n,k,swiglu,shape", [
+    (341, 6144, 2048, False, -1), (342, 6144, 2048, False, 0), (300, 6144, 1024, False, 0), (363, 5632, 2048, True, 0), (297, 5632, 2048, True, -1), (299, 5632, 2048, True, 0),      # rows that fill half, or two fifths
+    (3073, 768, 2112, False, -1), (3073, 768, 2048, False, 0), (1536, 1024, 2112, False, -1), (2304, 1536, 2048, False, 0), (2433, 1536, 2048, False, -1),                       # few features
+    (1843, 2048, 4096, False, 0), (1844, 2048, 4160, False, -1), (1843, 2048, 4160, False, 0), (800, 4096, 4160, False, 0), (1117, 2048, 14336, False, -1), (513, 4096, 14336, False, 0), (1004, 2560, 11008, False, -1),     # long sums
+    (2049, 2048, 1984, False, 1), (2049, 2048, 2048, False, -1), (2305, 2048, 2048, False, 1), (1400, 3072, 2048, False, -1), (1400, 3072, 1984, False, 1),                                                    # 128 x 256
+    (1861, 5632, 2048, True, -1), (1862, 5632, 2048, True, 2), (1400, 5632, 960, True, 2), (1400, 5632, 1024, True, -1)])                                                        # 256 x 256
+def test_where_the_library_s_tiles_fit_better(m, n, k, swiglu, shape):
+    """On both sides of the lines behind which many rows in tiles stay with the library, on a card of 256 compute units."""
+    if ops.TUNING.compute_units != 256:
+        pytest.skip("the lines are those of 256 compute units")
+    assert ops.tiles_choice(m, n, k, swiglu) == shape
