@@ -531,31 +531,33 @@ static int decode_compute_units() {
 
 // The waves of a workgroup.  Eight where every workgroup finds a compute unit of its own; beyond that eight leave room for one workgroup at a time on a compute unit, whose first
 // loads and merge nothing then covers.  One MI355X, us, 8 waves and 4: 16 requests of 1,000 keys, 12 heads of 64, 10.3 and 12.1; 64 of 1,000, 24 heads of 32 over 4, 8.4 and 10.8; 24 of 500, 32 heads of
-// 128 over 8, 11.0 and 11.3; but 256 requests of up to 129 keys, 16 heads of 64, 45.6 and 22.7, of 200 50.9 and 29, 32 heads of 128 over 8 37.8 and 24.4; 64 of 150 to 1,500 36.5 and 37.0.
-// Heads of 128 in parts are long, and where they fill more than half of the chip four waves ask for all that memory gives: 8 requests of 4,000 keys, 32 heads over 8, in four
+// 128 over 8, 11.0 and 11.3; also up to twice as many workgroups whose longest request has many keys, for which the others wait (64 of 150 to 1,500, 32 heads over 8, 36.5 and 37.7; the caller says so); but 256 requests of up to 129 keys, 16 heads of 64, 45.6 and 22.7, of 200 50.9 and 29, 32 heads of 128 over 8 37.8 and 24.4.
+// Where parts of heads of 128 fill more than half of the chip and are long (the caller says so) four waves ask for all that memory gives: 8 requests of 4,000 keys, 40 heads over 8, in four
 // parts, 22.3 and 21.2, of 2,000 14.1 and 14.5.  Sixteen rows: their sums of eight waves would be more LDS than a launch gets unasked.
-static int decode_waves(long long workgroups, int rows, int dh, int n_splits, int units) {
-    if (rows >= 16 || workgroups > units) return 4;
-    return dh == 128 && n_splits > 1 && 2 * workgroups > units ? 4 : 8;
+enum { DEC_FEW_KEYS = 1, DEC_MANY_KEYS = 2 };      // what a caller may know of the requests' lengths: none has many keys (four waves then); the longest has
+static int decode_waves(long long workgroups, int rows, int dh, int n_splits, int units, int lengths) {
+    if (rows >= 16 || lengths == DEC_FEW_KEYS) return 4;
+    if (workgroups > units) return lengths == DEC_MANY_KEYS && n_splits == 1 && workgroups <= 2 * units ? 8 : 4;
+    return lengths == DEC_MANY_KEYS && dh == 128 && n_splits > 1 && 2 * workgroups > units ? 4 : 8;
 }
 
 // The same for whoever wants to know (units: the device's compute units).
-LCU_API int lcu_attention_decode_waves(int n_req, int nh, int nkvh, int dh, int n_splits, int units) {
+LCU_API int lcu_attention_decode_waves(int n_req, int nh, int nkvh, int dh, int n_splits, int units, int lengths) {
     if (n_req <= 0 || nh <= 0 || nkvh <= 0 || nh % nkvh || n_splits <= 0) return LCU_BAD_ARGUMENT;
     const int g = nh / nkvh;
-    return decode_waves((long long)n_req * nkvh * ((g + 15) / 16) * n_splits, g < 16 ? g : 16, dh, n_splits, units);
+    return decode_waves((long long)n_req * nkvh * ((g + 15) / 16) * n_splits, g < 16 ? g : 16, dh, n_splits, units, lengths);
 }
 
 template <int DH>
 static int launch_decode(const void *q, int q_stride, void *out, int out_stride, const void *cache,
                          const int *block_table, int max_pages, const int *q_start, const int *ctx_len,
                          const int *req_list, int n_req, int nh, int nkvh, int page, float scale, int window,
-                         int n_splits, int few_keys, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
+                         int n_splits, int lengths, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
     const int g = nh / nkvh, chunks = (g + 15) / 16;
     const float scale_log2 = SCORE_LOG2(scale);
     const int held = g < 16 ? g : 16;
     dim3 grid(n_req * nkvh * chunks, n_splits);
-    const int waves = few_keys ? 4 : decode_waves((long long)grid.x * n_splits, held, DH, n_splits, decode_compute_units());
+    const int waves = decode_waves((long long)grid.x * n_splits, held, DH, n_splits, decode_compute_units(), lengths);
     const size_t lds_bytes = (size_t)waves * held * (DH + 4 + 2) * sizeof(float);
     static_assert(8 * 15 * (128 + 4 + 2) * sizeof(float) <= 65536, "what a launch gets unasked");
     dim3 block(waves * WAVE);
@@ -587,11 +589,11 @@ static int decode_arguments(int q_stride, int out_stride, int max_pages, int nh,
     return LCU_OK;
 }
 
-// few_keys: four waves a workgroup, however few the workgroups (a matter of speed alone).
+// lengths: 0, DEC_FEW_KEYS or DEC_MANY_KEYS (a matter of speed alone).
 LCU_API int lcu_attention_decode_lengths_bf16(const void *q, int q_stride, void *out, int out_stride, const void *cache,
                                       const int *block_table, int max_pages, const int *q_start, const int *ctx_len,
                                       const int *req_list, int n_req, int nh, int nkvh, int dh, int page, float scale,
-                                      int window, int n_splits, int few_keys, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
+                                      int window, int n_splits, int lengths, float *part_o, float *part_ml, hipStream_t stream SCORE_PARAMS) {
     if (n_req <= 0) return LCU_OK;
 #ifdef LCU_SCORE_BIAS
     if (!head_slopes || !(scale > 0.f)) return LCU_BAD_ARGUMENT;
@@ -602,7 +604,7 @@ LCU_API int lcu_attention_decode_lengths_bf16(const void *q, int q_stride, void 
     const int args = decode_arguments(q_stride, out_stride, max_pages, nh, nkvh, dh, page, window, n_splits);
     if (args != LCU_OK) return args;
     if (n_splits > 1 && (!part_o || !part_ml)) return LCU_BAD_ARGUMENT;
-#define GO(D) return launch_decode<D>(q, q_stride, out, out_stride, cache, block_table, max_pages, q_start, ctx_len, req_list, n_req, nh, nkvh, page, scale, window, n_splits, few_keys, part_o, part_ml, stream SCORE_ARGS)
+#define GO(D) return launch_decode<D>(q, q_stride, out, out_stride, cache, block_table, max_pages, q_start, ctx_len, req_list, n_req, nh, nkvh, page, scale, window, n_splits, lengths, part_o, part_ml, stream SCORE_ARGS)
     if (dh == 128) GO(128);
     if (dh == 64) GO(64);
     if (dh == 96) GO(96);

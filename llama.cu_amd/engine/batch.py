@@ -47,7 +47,8 @@ class StepContext:
     req_ids: List[int] = field(default_factory=list)
     state_slots: List[int] = field(default_factory=list)    # ``state_slot`` on the host
     logits_all: bool = False                    # the logits of every token are wanted, in order (logit_rows is 0, 1, ...)
-    attn_splits: Optional[int] = None           # fixed number of key parts for the decode kernel (captured graphs)
+    attn_splits: Optional[int] = None           # fixed number of key parts for the decode kernel (captured graphs) ...
+    attn_long: Optional[bool] = None            # ... and whether it counts on many keys (ops.decode_long)
     scratch: dict = field(default_factory=dict)  # what kernels' wrappers derive from the batch once per step
     # tokens that the step before sampled and the host does not know yet: tokens[feed_dst[i]] is
     # to be taken from row feed_src[i] of that step's sampled ids, on the device

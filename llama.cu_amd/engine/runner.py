@@ -174,7 +174,7 @@ class ModelRunner:
         # captured steps: for steps of single tokens by batch size and key parts: (graph, its logits tensor)
         self.use_graphs = bool(use_graphs) and self.model.graph_safe
         self.tensors: Dict[str, torch.Tensor] = tensors      # by the names that files use (views of the load's one allocation)
-        self._graphs: Dict[tuple, Any] = {}        # (batch size, key parts) -> (graph, its logits)
+        self._graphs: Dict[tuple, Any] = {}        # (batch size, key parts[, "long"]) -> (graph, its logits)
         self._seen: Dict[tuple, int] = {}
         self.graph_replays: Dict[tuple, int] = {}  # how often each was replayed
         self._step_graphs: Dict[tuple, Any] = {}   # the same for steps that are not all single tokens, by their sizes
@@ -295,8 +295,8 @@ class ModelRunner:
         four hundred launches), so they are captured into HIP graphs and replayed: the batch arrays, and what
         the parts derive from them on the host (``Part.prepare``), live at fixed device addresses, so a replay
         reads the new step's tokens, positions, block tables and task lists.  A graph fits every step with the same
-        sizes: for steps in which every request decodes one token the number of requests and the number of parts
-        into which the decode attention cuts the keys; for any other step (a prompt portion beside decoding
+        sizes: for steps in which every request decodes one token the number of requests, the number of parts
+        into which the decode attention cuts the keys and whether a layer counts on many of them (``Part.decode_long``); for any other step (a prompt portion beside decoding
         requests, say) the numbers of tokens, requests, single tokens and wanted rows, and what the parts' plans
         say fixes their launches (``signature``).  (The reference captures everything between two attentions per
         token-count bucket, llama.cu/src/exec/step.rs:82-96; here the whole step is one graph.)"""
@@ -311,7 +311,9 @@ class ModelRunner:
             # graph is made for a batch size and a number of parts (which follows the longest
             # context rounded up to a power of two, so it changes rarely)
             step.attn_splits = self._decode_splits(b, step.max_ctx_len)
-            return self._run_captured(self._graphs, (b, step.attn_splits), step, self.graph_replays)
+            step.attn_long = any(layer.decode_long(b, step.max_ctx_len) for layer in self.model.layers)
+            key = (b, step.attn_splits, "long") if step.attn_long else (b, step.attn_splits)
+            return self._run_captured(self._graphs, key, step, self.graph_replays)
         if step.n > self.GRAPH_MAX_TOKENS:
             return self.model.forward(step, self.caches)
         plans = tuple(sorted((k, v.signature) for k, v in step.scratch.items() if hasattr(v, "signature")))

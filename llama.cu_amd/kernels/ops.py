@@ -493,11 +493,12 @@ def _attention_library(head_slopes=None, softcap: float = 0.0):
 def attention_decode(q, out, cache, block_table, q_start, ctx_len, n_req, n_heads, n_kv_heads, head_dim, page_size,
                      scale, window, n_splits, req_list: Optional[torch.Tensor] = None,
                      head_slopes: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None, softcap: float = 0.0,
-                     few_keys: bool = False) -> torch.Tensor:
+                     few_keys: bool = False, many_keys: bool = False) -> torch.Tensor:
     """Matrix-core attention for requests that feed one token each: all ``n_req`` requests of
     the batch, or the ``n_req`` whose indices ``req_list`` holds.  ``head_slopes``: the bias on the distance inside
     the scores (the kernels of the second library, ``attention_mfma_bias``); ``softcap``: a cap on them (the third,
-    ``attention_mfma_cap``).  ``few_keys``: no request has many, so four waves a workgroup do, however few the workgroups (a matter of speed alone)."""
+    ``attention_mfma_cap``).  ``few_keys``: no request has many, so four waves a workgroup do, however few the workgroups; ``many_keys``: the longest has
+    (``decode_long``).  (Matters of speed alone.)"""
     if req_list is not None:
         _i32(req_list, "req_list", n_req)
     part_o = part_ml = None
@@ -509,7 +510,7 @@ def attention_decode(q, out, cache, block_table, q_start, ctx_len, n_req, n_head
     _check(lib.lcu_attention_decode_lengths_bf16(_ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(cache), _ptr(block_table),
                                          block_table.shape[1], _ptr(q_start), _ptr(ctx_len), _ptr(req_list), n_req, n_heads,
                                          n_kv_heads,
-                                         head_dim, page_size, ctypes.c_float(scale), int(window), int(n_splits), int(bool(few_keys)),
+                                         head_dim, page_size, ctypes.c_float(scale), int(window), int(n_splits), 1 if few_keys else 2 if many_keys else 0,
                                          _ptr(part_o), _ptr(part_ml), _stream(), *more), "attention_decode")
     return out
 
@@ -577,13 +578,13 @@ class AttentionPlan:
     prefill kernel's tasks (``task_req``, ``task_tok0``; ``n_tasks`` on the device says how many).  The launches' sizes
     (``max_tasks``, ``n_single``, ``single_splits``) follow from the step's sizes and the longest context rounded up to
     a power of two; what the lists hold is data."""
-    __slots__ = ("task_req", "task_tok0", "n_tasks_dev", "max_tasks", "per_wg", "singles", "n_single", "single_splits")
+    __slots__ = ("task_req", "task_tok0", "n_tasks_dev", "max_tasks", "per_wg", "singles", "n_single", "single_splits", "single_long")
 
     @property
     def signature(self):
         """What fixes the launches that ``paged_attention`` makes with this plan: two steps with equal signatures are
         served by the same recorded launches."""
-        return (self.max_tasks, self.per_wg, self.n_single, self.single_splits)
+        return (self.max_tasks, self.per_wg, self.n_single, self.single_splits, self.single_long)
 
 
 def plan_attention(step, n_heads: int, n_kv_heads: int, window: int = 0, biased: bool = False, capped: bool = False) -> Optional[AttentionPlan]:
@@ -611,6 +612,8 @@ def plan_attention(step, n_heads: int, n_kv_heads: int, window: int = 0, biased:
     # the most tasks that a step of these sizes can have: a request of q tokens has at most q / tpt + 1
     plan.max_tasks = (step.n - len(singles)) // tpt + (step.n_req - len(singles))
     plan.single_splits = decode_splits(len(singles), n_heads, n_kv_heads, max([step.ctx_lens[r] for r in singles], default=0)) if singles else 1
+    # (with heads of 128, which count on it in more steps than others, as the plan serves layers with heads of any size)
+    plan.single_long = decode_long(len(singles), n_heads, n_kv_heads, 128, max([step.ctx_lens[r] for r in singles], default=0), window) if singles else False
     builder = getattr(step, "builder", None)
     if builder is not None:
         cap_tasks = builder.max_tokens // tpt + builder.max_reqs
@@ -664,6 +667,20 @@ def decode_splits(n_req: int, n_heads: int, n_kv_heads: int, max_ctx_len: int) -
     return 1 + next(i for i, f in enumerate(fill) if f >= max(fill) - t.decode_fill_slack)
 
 
+def decode_long(n_req: int, n_heads: int, n_kv_heads: int, head_dim: int, max_ctx_len: int, window: int = 0, splits: Optional[int] = None) -> bool:
+    """Whether the longest request has so many keys (in a window or chunk) that the decode kernel's workgroups have another number of waves (``decode_waves`` in attention_mfma.hip, which asks
+    for it where it matters): eight where they outnumber the compute units up to twice, as the others wait for it, from ``TUNING.decode_long_keys`` on; four where parts of heads of 128
+    fill more than half of the chip, from ``TUNING.decode_long_part`` keys a part on.  ``splits``: the number of parts, if it is fixed."""
+    t, base = TUNING, n_req * n_kv_heads
+    if n_heads // n_kv_heads >= 16:
+        return False
+    keys = min(int(max_ctx_len), abs(int(window)) or int(max_ctx_len))
+    if base > t.compute_units:
+        return base <= 2 * t.compute_units and keys > t.decode_long_keys
+    splits = splits or decode_splits(n_req, n_heads, n_kv_heads, max_ctx_len)
+    return head_dim == 128 and splits > 1 and 2 * base * splits > t.compute_units and keys > t.decode_long_part * splits
+
+
 _zeros: Dict = {}
 
 
@@ -714,13 +731,15 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, cache: torch.Tensor, ste
         # batch says which they are (64 requests of 150 to 2,200 keys: the step 11.2 -> 11.0 ms)
         return attention_decode(q, out, cache, bt, step.q_start, step.ctx_len, step.n_req, n_heads, n_kv_heads, head_dim,
                                 page_size, scale, window, splits, req_list=step.decode_order, head_slopes=head_slopes, sinks=sinks,
-                                softcap=softcap)
+                                softcap=softcap, many_keys=step.attn_long is not False and
+                                decode_long(step.n_req, n_heads, n_kv_heads, head_dim, step.max_ctx_len if step.attn_long is None else 1 << 30, window, splits))
     # a mixed batch: the requests that decode one token go to the decode kernel, the portions
     # to the prefill kernel (each would be slow at the other's work)
     plan = plan_attention(step, n_heads, n_kv_heads, window, biased=second, capped=bool(softcap))
     if plan.n_single:
         attention_decode(q, out, cache, bt, step.q_start, step.ctx_len, plan.n_single, n_heads, n_kv_heads, head_dim, page_size,
-                         scale, window, plan.single_splits, req_list=plan.singles, head_slopes=head_slopes, sinks=sinks, softcap=softcap)
+                         scale, window, plan.single_splits, req_list=plan.singles, head_slopes=head_slopes, sinks=sinks, softcap=softcap,
+                         many_keys=plan.single_long)
     if plan.max_tasks:
         attention_prefill(q, out, cache, bt, step.q_start, step.ctx_len, plan.task_req, plan.task_tok0, plan.max_tasks,
                           plan.per_wg, n_heads, n_kv_heads, head_dim, page_size, scale, window, n_tasks_dev=plan.n_tasks_dev,

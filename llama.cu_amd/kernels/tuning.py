@@ -126,6 +126,11 @@ class Tuning:
     decode_max_parts: int = 32
     decode_few_parts: int = 8           # beyond 512 keys up to so many parts, however short (of at least 64 keys: 513 are taken for 1,024).  4 requests of 1,000 keys 12.6, 10.9, 8.9, 7.5,
                                         # 8 of 1,000 13.8, 11.6, 9.3, 8.3, 1 of 2,000 18.6, 11.1, 9.2, 7.7
+    decode_long_keys: int = 1024        # beyond so many keys of the longest request eight waves a workgroup for one to two workgroups a compute unit (attention_mfma.hip).  Lengths of 10 to 100 % and of 50
+                                        # to 100 % of it, 8 waves' time over 4's: 512 workgroups of heads of 128 at 500 / 1,000 / 1,500 / 3,000 keys 1.05 / 0.98 / 0.95 / 0.96 and 1.08 / 1.01 / 1.00 / 0.95, 384 of heads of
+                                        # 64 1.10 / 0.99 / 0.83 / 0.82 and 1.21 / 1.06 / 1.01 / 0.95; 768 and more 1.02 to 1.14 from 1,000 to 1,500 keys on
+    decode_long_part: int = 768         # from so many keys a part on four waves for parts of heads of 128 that fill more than half of the chip: eight parts of 32 to 256 workgroups, 8 waves' time over 4's at 250 / 500 /
+                                        # 1,000 / 2,000 keys a part 0.93 to 1.01, 0.93 to 1.01, 1.01 to 1.07, 1.02 to 1.05
     decode_few_workgroups: int = 128    # up to this many workgroups without parts: about one workgroup per compute unit
     decode_long_context: int = 2048     # between half the chip's worth of workgroups and all of it: parts only from here on
                                         # (rounded up to a power of two: from 1,025 keys),

@@ -166,6 +166,9 @@ class Attention(Part):
         requests decode over at most ``max_ctx_len`` keys (a captured graph fixes the number)."""
         return ops.decode_splits(batch, self.heads, self.kv_heads, max_ctx_len)
 
+    def decode_long(self, batch: int, max_ctx_len: int) -> bool:
+        return ops.decode_long(batch, self.heads, self.kv_heads, self.stored_dim if self.general else self.padded_dim, max_ctx_len, self.window or self.chunk)
+
     def _load_general(self, tensors, build: BuildContext) -> None:
         nm, nh, nkv, dh, dv = self.names, self.heads, self.kv_heads, self.head_dim, self.value_dim
         self.w_in = Weight(fused_rows([tensors[nm[k]] for k in self._in_keys()]), build)

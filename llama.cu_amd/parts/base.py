@@ -317,6 +317,11 @@ class Part:
         ``batch`` requests decode over at most ``max_ctx_len`` keys; a captured graph fixes the number."""
         return 1
 
+    def decode_long(self, batch: int, max_ctx_len: int) -> bool:
+        """Whether a mixer (or a block, for its mixer) decodes ``batch`` requests another way where the longest has so many keys
+        (``ops.decode_long``); a captured graph fixes that too."""
+        return False
+
     # position: what a position encoding may be, each optional (``parts/position.py`` describes them): tables of
     # a rotation, any other change of queries and keys in place, a bias inside the scores.
     def rotary_tables(self):

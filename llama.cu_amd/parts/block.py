@@ -66,6 +66,9 @@ class PreNormBlock(Part):
     def decode_splits(self, batch: int, max_ctx_len: int) -> int:
         return int(self.mixer.decode_splits(batch, max_ctx_len))
 
+    def decode_long(self, batch: int, max_ctx_len: int) -> bool:
+        return bool(self.mixer.decode_long(batch, max_ctx_len))
+
     @property
     def first_norm(self):
         return self.norm1
@@ -197,6 +200,9 @@ class ParallelBlock(Part):
     def decode_splits(self, batch: int, max_ctx_len: int) -> int:
         return int(self.mixer.decode_splits(batch, max_ctx_len))
 
+    def decode_long(self, batch: int, max_ctx_len: int) -> bool:
+        return bool(self.mixer.decode_long(batch, max_ctx_len))
+
     @property
     def takes_planes(self) -> bool:
         return bool(self.norm1.takes_planes)
@@ -290,6 +296,9 @@ class _SublayersInTurn(Part):
 
     def decode_splits(self, batch: int, max_ctx_len: int) -> int:
         return int(self.mixer.decode_splits(batch, max_ctx_len))
+
+    def decode_long(self, batch: int, max_ctx_len: int) -> bool:
+        return bool(self.mixer.decode_long(batch, max_ctx_len))
 
 
 class SandwichBlock(_SublayersInTurn):

@@ -90,6 +90,9 @@ class DifferentialAttention(Part):
     def decode_splits(self, batch: int, max_ctx_len: int) -> int:
         return ops.decode_splits(batch, self.map_heads, self.stored_heads, max_ctx_len)
 
+    def decode_long(self, batch: int, max_ctx_len: int) -> bool:
+        return ops.decode_long(batch, self.map_heads, self.stored_heads, self.stored_dim, max_ctx_len, self.window)
+
     def load(self, tensors, build: BuildContext) -> None:
         nm, nh, nkv, dh, dv = self.names, self.heads, self.kv_heads, self.head_dim, self.value_dim
         self.w_in = Weight(fused_rows([tensors[nm[k]] for k in self._in_keys()]), build)

@@ -106,6 +106,9 @@ class LatentAttention(Part):
     def decode_splits(self, batch: int, max_ctx_len: int) -> int:
         return ops.decode_splits(batch, self.heads, 1, max_ctx_len)
 
+    def decode_long(self, batch: int, max_ctx_len: int) -> bool:
+        return ops.decode_long(batch, self.heads, 1, self.stored_dim, max_ctx_len, self.window)
+
     def load(self, tensors, build: BuildContext) -> None:
         nm, nh, dn, dr, dv, rank = self.names, self.heads, self.head_dim, self.rot_dim, self.value_dim, self.kv_rank
         self.dtype, self.page_size = build.dtype, build.page_size

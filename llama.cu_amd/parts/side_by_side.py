@@ -68,6 +68,9 @@ class SideBySide(Part):
     def decode_splits(self, batch: int, max_ctx_len: int) -> int:
         return max(int(m.decode_splits(batch, max_ctx_len)) for m in self.mixers)
 
+    def decode_long(self, batch: int, max_ctx_len: int) -> bool:
+        return any(m.decode_long(batch, max_ctx_len) for m in self.mixers)
+
     # (with one product for all: it ends as a single mixer's would)
     @property
     def ends_in_planes(self):

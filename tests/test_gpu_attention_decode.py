@@ -52,3 +52,23 @@ def test_rows_waves_and_pages(nh, nkv, dh, page, splits):
     assert_close(got, wanted, 3 * 2.0 ** -8, "against the generic kernel")        # the weights and both outputs rounded to bfloat16
     ops.attention_decode(q, got.fill_(float("nan")), cache, table, starts, lens, n, nh, nkv, dh, page, dh ** -0.5, 0, splits, few_keys=True)
     assert_close(got, wanted, 3 * 2.0 ** -8, "four waves, however many keys")
+
+
+@pytest.mark.parametrize("nh,nkv,dh,n,splits", [(4, 4, 64, 80, 1), (2, 2, 128, 30, 4)])
+def test_requests_whose_longest_has_many_keys(nh, nkv, dh, n, splits):
+    """More workgroups than compute units with eight waves, and parts of heads of 128 with four: what the caller's word for many keys changes is the number of waves."""
+    from llama_cu_amd.kernels import build, ops
+    units, waves = torch.cuda.get_device_properties(0).multi_processor_count, build.load("attention_mfma").lcu_attention_decode_waves
+    if units == 256:
+        assert waves(n, nh, nkv, dh, splits, units, 0) != waves(n, nh, nkv, dh, splits, units, 2)
+    page, ctx = 16, [1 + (37 * i) % 300 for i in range(n - 1)] + [1100]
+    most = -(-max(ctx) // page)
+    cache = rnd(n * most + 1, 2, nkv * dh * page, seed=4).bfloat16().cuda()
+    table = (torch.randperm(n * most, generator=torch.Generator().manual_seed(5)) + 1).to(torch.int32).view(n, most).contiguous().cuda()
+    q = rnd(n, nh * dh, seed=6).bfloat16().cuda()
+    starts, of, lens = torch.arange(n + 1, dtype=torch.int32).cuda(), torch.arange(n, dtype=torch.int32).cuda(), torch.tensor(ctx, dtype=torch.int32).cuda()
+    got, wanted = torch.empty(n, nh * dh, dtype=torch.bfloat16, device="cuda"), torch.empty(n, nh * dh, dtype=torch.bfloat16, device="cuda")
+    ops.paged_attention_generic(q, wanted, cache, table, starts, lens, of, nh, nkv, dh, page, dh ** -0.5, 0)
+    for many in (False, True):
+        ops.attention_decode(q, got.fill_(float("nan")), cache, table, starts, lens, n, nh, nkv, dh, page, dh ** -0.5, 0, splits, many_keys=many)
+        assert_close(got, wanted, 3 * 2.0 ** -8, f"many keys: {many}")        # the weights and both outputs rounded to bfloat16

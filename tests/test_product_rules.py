@@ -48,13 +48,27 @@ def test_rows_that_span_more_than_a_load_reaches():
 def test_waves_of_the_decode_attention(name):
     """Eight waves a workgroup where every workgroup has a compute unit of its own, four beyond (256 requests of some 129 keys took twice as long with eight), for sixteen
     rows, and for parts of heads of 128 that fill more than half of the chip."""
-    waves = build.load(name).lcu_attention_decode_waves
+    waves = lambda *a, lengths=0: build.load(name).lcu_attention_decode_waves(*a, lengths)
     for dh in (32, 64, 96, 128):
         assert [waves(n, 16, 16, dh, 1, 256) for n in (1, 16, 17, 256)] == [8, 8, 4, 4]
         assert [waves(n, 32, 8, dh, 1, 256) for n in (32, 33)] == [8, 4] and waves(33, 32, 8, dh, 1, 304) == 8
         assert [waves(1, g, 1, dh, 1, 256) for g in (15, 16, 17, 32)] == [8, 4, 4, 4]
-        assert [waves(n, 32, 8, dh, 4, 256) for n in (4, 5, 8, 9)] == [8, 4 if dh == 128 else 8, 4 if dh == 128 else 8, 4]
+        assert [waves(n, 32, 8, dh, 4, 256) for n in (4, 5, 8, 9)] == [8, 8, 8, 4]
+        assert [waves(n, 32, 8, dh, 4, 256, lengths=2) for n in (4, 5, 8, 9)] == [8, 4 if dh == 128 else 8, 4 if dh == 128 else 8, 4]
         assert waves(1, 32, 8, dh, 1, 0) == 4                  # (a device that does not say how many units it has)
+        assert [waves(n, 32, 8, dh, 1, 256, lengths=2) for n in (32, 33, 64, 65)] == [8, 8, 8, 4] and waves(33, 32, 8, dh, 2, 256, lengths=2) == 4
+        assert waves(1, 32, 8, dh, 1, 256, lengths=1) == 4 and waves(40, 16, 1, dh, 1, 256, lengths=2) == 4
+
+
+def test_requests_whose_longest_has_many_keys():
+    """Where the decode attention's workgroups are one to two a compute unit, and where parts of heads of 128 fill more than half of the chip; not for layers that see a window of fewer keys."""
+    long = ops.decode_long
+    if ops.TUNING.compute_units != 256:
+        pytest.skip("the lines are those of 256 compute units")
+    assert [long(n, 32, 8, 64, 1025) for n in (32, 33, 64, 65)] == [False, True, True, False] and not long(64, 32, 8, 64, 1024)
+    assert not long(64, 32, 8, 128, 4000, 1024) and not long(64, 32, 8, 128, 4000, -128) and long(64, 32, 8, 128, 4000, 1025) and not long(300, 16, 1, 64, 4000) and long(300, 15, 1, 64, 4000)
+    assert not long(8, 32, 8, 128, 3072) and long(8, 32, 8, 128, 3073) and not long(8, 32, 8, 96, 3073) and long(16, 32, 8, 128, 1537) and not long(16, 32, 8, 128, 1537, 1536)
+    assert not long(4, 32, 8, 128, 3073) and long(4, 32, 8, 128, 6145) and not long(1, 32, 8, 128, 24576) and long(1, 32, 8, 128, 24577) and not long(8, 32, 8, 128, 1537, 0, 4) and long(8, 32, 8, 128, 1537, 0, 2) == False
 
 
 def test_parts_of_few_requests():
