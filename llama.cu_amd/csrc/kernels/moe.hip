@@ -644,6 +644,7 @@ moe_gemm_slots_kernel(const T *__restrict__ x, int x_stride, const T *__restrict
                 if (s + u + AHEAD < s1) fetch(u, s + u + AHEAD);
             }
         }
+        asm volatile("s_nop 3" : "+v"(acc));         // the last matrix instruction's wait, which the compiler leaves a state short behind the branches
         if (r0 > 0) __syncthreads();                 // the sums of the rows before have been read
         red[part][side][lane] = acc;
         __syncthreads();
