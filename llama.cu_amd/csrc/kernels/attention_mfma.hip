@@ -394,7 +394,7 @@ attention_decode_kernel(const bf16_t *__restrict__ q, int q_stride, bf16_t *__re
             idb = kv_pages<PAGE16>(bt, max_pages, page, (nb2 + WAVES) * 32);
         }
         attn_block<DH, 1>(fa, blk * 32, blk * 32 + 31 > p || blk * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
-        asm volatile("s_nop 3" : "+v"(st.o[0][DH / 16 - 1]));        // the last matrix instruction's wait, which the compiler leaves a state short behind the branches
+        asm("s_nop 3" : "+v"(st.o[0][DH / 16 - 1]));                 // the last matrix instruction's wait, which the compiler leaves a state short behind the branches
         if (nb2 < b1) load_kv<DH>(fa, cache, ida, page, page_elems, nkvh, kvh, l16, grp);
         if (nb < b1)
             attn_block<DH, 1>(fb, nb * 32, nb * 32 + 31 > p || nb * 32 < lo, qv, st, p_row, lo_row, p, lo, scale_log2, grp);
