@@ -677,8 +677,10 @@ def decode_long(n_req: int, n_heads: int, n_kv_heads: int, head_dim: int, max_ct
     keys = min(int(max_ctx_len), abs(int(window)) or int(max_ctx_len))
     if base > t.compute_units:
         return base <= 2 * t.compute_units and keys > t.decode_long_keys
+    if head_dim != 128 or keys <= 2 * t.decode_long_part:        # (two parts at least)
+        return False
     splits = splits or decode_splits(n_req, n_heads, n_kv_heads, max_ctx_len)
-    return head_dim == 128 and splits > 1 and 2 * base * splits > t.compute_units and keys > t.decode_long_part * splits
+    return splits > 1 and 2 * base * splits > t.compute_units and keys > t.decode_long_part * splits
 
 
 _zeros: Dict = {}
