@@ -1,6 +1,7 @@
 """Generation through the entry points: greedy tokens equal the plain implementation's;
 seeded temperature sampling equals the plain sampler drawing from the plain logits;
 scheduling decisions (portions, few pages, preemption) change no token."""
+import dataclasses
 import os
 import subprocess
 import sys
@@ -547,3 +548,26 @@ def test_a_random_serving_session_changes_no_token(folder_b):
         eng.drop(i)
     eng.runner.cache.check()
     assert eng.runner.cache.free_pages(0) == eng.runner.num_pages and eng.runner.cache.free_slots() == 4
+
+
+def test_captured_decode_steps_whose_attention_counts_on_many_keys(monkeypatch):
+    """Where the decode attention's workgroups are more than the compute units a second graph is captured once the longest request has many keys (here: more than 24); every step gives the
+    logits of the eager one."""
+    from llama_cu_amd.engine.runner import ModelRunner
+    from llama_cu_amd.kernels import ops
+    monkeypatch.setattr(ops, "TUNING", dataclasses.replace(ops.TUNING, decode_long_keys=24))
+    folder = common.make_folder(dict(common.TINY_B, num_key_value_heads=4), seed=31, dtype=torch.bfloat16, std=common.BF16_STD)
+    n = ops.TUNING.compute_units // 4 + 3
+    reqs = list(common.random_requests(384, [3 + i % 17 for i in range(n)], seed=8).values())
+
+    def decode(use_graphs):
+        runner = ModelRunner.from_folder(folder, dtype="bfloat16", max_tokens=64 * n, max_seqs=n, use_graphs=use_graphs)
+        runner.step(list(range(n)), reqs)
+        rng = np.random.default_rng(0)
+        return [runner.step(list(range(n)), [[int(t)] for t in rng.integers(384, size=n)]).float().cpu() for _ in range(11)], runner
+
+    eager, _ = decode(False)
+    graphed, runner = decode(True)
+    assert sorted(runner._graphs) == [(n, 1), (n, 1, "long")]
+    for i, (a, b) in enumerate(zip(eager, graphed)):
+        assert torch.equal(a, b), f"decode step {i} differs between eager and captured"
