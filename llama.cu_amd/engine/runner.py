@@ -311,7 +311,7 @@ class ModelRunner:
             # graph is made for a batch size and a number of parts (which follows the longest
             # context rounded up to a power of two, so it changes rarely)
             step.attn_splits = self._decode_splits(b, step.max_ctx_len)
-            step.attn_long = any(layer.decode_long(b, step.max_ctx_len) for layer in self.model.layers)
+            step.attn_long = step.max_ctx_len > ops.decode_long_from() and any(layer.decode_long(b, step.max_ctx_len) for layer in self.model.layers)
             key = (b, step.attn_splits, "long") if step.attn_long else (b, step.attn_splits)
             return self._run_captured(self._graphs, key, step, self.graph_replays)
         if step.n > self.GRAPH_MAX_TOKENS:

@@ -667,12 +667,17 @@ def decode_splits(n_req: int, n_heads: int, n_kv_heads: int, max_ctx_len: int) -
     return 1 + next(i for i, f in enumerate(fill) if f >= max(fill) - t.decode_fill_slack)
 
 
+def decode_long_from() -> int:
+    """Up to so many keys of the longest request ``decode_long`` says no whatever the sizes: a step need not ask its layers."""
+    return min(TUNING.decode_long_keys, 2 * TUNING.decode_long_part)
+
+
 def decode_long(n_req: int, n_heads: int, n_kv_heads: int, head_dim: int, max_ctx_len: int, window: int = 0, splits: Optional[int] = None) -> bool:
     """Whether the longest request has so many keys (in a window or chunk) that the decode kernel's workgroups have another number of waves (``decode_waves`` in attention_mfma.hip, which asks
     for it where it matters): eight where they outnumber the compute units up to twice, as the others wait for it, from ``TUNING.decode_long_keys`` on; four where parts of heads of 128
     fill more than half of the chip, from ``TUNING.decode_long_part`` keys a part on.  ``splits``: the number of parts, if it is fixed."""
     t, base = TUNING, n_req * n_kv_heads
-    if n_heads // n_kv_heads >= 16:
+    if max_ctx_len <= decode_long_from() or n_heads // n_kv_heads >= 16:
         return False
     keys = min(int(max_ctx_len), abs(int(window)) or int(max_ctx_len))
     if base > t.compute_units:

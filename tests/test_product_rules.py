@@ -71,6 +71,13 @@ def test_requests_whose_longest_has_many_keys():
     assert not long(4, 32, 8, 128, 3073) and long(4, 32, 8, 128, 6145) and not long(1, 32, 8, 128, 24576) and long(1, 32, 8, 128, 24577) and not long(8, 32, 8, 128, 1537, 0, 4) and long(8, 32, 8, 128, 1537, 0, 2) == False
 
 
+def test_short_steps_do_not_ask_for_many_keys():
+    """Up to the number of keys that a step looks at first no sizes count on many; behind it some do."""
+    least = ops.decode_long_from()
+    sizes = [(n, nh, nkv, dh) for n in (1, 7, 8, 33, 64, 300) for nh, nkv in ((32, 8), (16, 4), (40, 8), (15, 1)) for dh in (64, 128)]
+    assert not any(ops.decode_long(*z, least) for z in sizes) and any(ops.decode_long(*z, least + 1) for z in sizes)
+
+
 def test_parts_of_few_requests():
     """One part up to 512 keys, eight beyond as far as the chip has compute units for them, longer ones from 4,097 keys on."""
     splits = ops.decode_splits
